@@ -77,6 +77,8 @@ public:
   void assign_i8(const int8_t *first, size_t num, int32_t bidx);
   // slot bidx as float-stored NCHW host data
   std::shared_ptr<std::vector<float>> tensor(int32_t bidx) const;
+  // the same into the caller's buffer
+  void read(float *dst, size_t num, int32_t bidx) const;
   // slot bidx as int8 NCHW host data (no float detour)
   void read_i8(int8_t *dst, size_t num, int32_t bidx) const;
   // lays the tensor out again with another channel stride (4 for a tensor of at most 4 channels whose
@@ -95,9 +97,8 @@ public:
 private:
   tpuhip_ctx *ctx_;
   size_t size_;
+  void *slot(int32_t bidx) const { return (char *)base_ + slot_bytes() * (size_t)bidx; }
   void *base_ = nullptr;
-  // staging for assign(): a pinned host copy and its fp32 image on the device, made on first use
-  void *stage_host_ = nullptr, *stage_dev_ = nullptr;
   void *ptr_ = nullptr;
   int32_t cur_ = 0;
 };
@@ -620,6 +621,7 @@ public:
   // the same from int8 NCHW data (no counterpart in the reference, whose tensors are float-stored)
   void setTensorI8(const std::string &name, const int8_t *data, size_t count, int32_t bidx);
   std::shared_ptr<std::vector<float>> getTensor(std::string &name, int32_t bidx);
+  void getTensor(const std::string &name, float *dst, size_t num, int32_t bidx);
   void getTensorI8(const std::string &name, int8_t *dst, size_t num, int32_t bidx);
   std::vector<int64_t> getTensorShape(std::string &name);
   std::string getDataType(std::string &name);

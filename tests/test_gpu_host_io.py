@@ -1,0 +1,95 @@
+"""Tensors between host memory and the device: the layout kernels at the edges of their tiles, and set_tensor /
+get_tensor in one piece, in several, and through more than the staging buffer holds."""
+import numpy as np
+import pytest
+
+from tpu_compiler_amd import capi, graphs, module
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("shape,cs", [
+    ((2, 3, 5, 7), 16), ((2, 3, 5, 7), 4), ((3, 4, 1, 127), 4), ((1, 1, 32, 32), 16), ((2, 2, 33, 31), 4),   # images
+    ((5, 1000, 1, 1), None), ((3, 13, 1, 1), None), ((1, 16, 1, 1), 48), ((70, 255, 1, 1), None),            # vectors
+    ((2, 64, 16, 8), None), ((2, 65, 1, 129), None), ((1, 17, 3, 43), 64), ((3, 255, 13, 13), None),         # tiles
+    ((2, 128, 2, 1), None), ((1, 5, 300, 1), None)])
+def test_layout_conversions(ctx, shape, cs):
+    rng = np.random.default_rng(sum(shape))
+    x = rng.integers(-128, 128, shape).astype(np.int8)
+    t = ctx.tensor(shape, cs)
+    ctx._ck(ctx.lib.tpuhip_memset(ctx.h, t.ptr, 0x55, t.nbytes))
+    t2 = ctx.from_nchw(x, cs)
+    raw = ctx.raw(t2)
+    assert np.array_equal(raw[..., :shape[1]], x.transpose(0, 2, 3, 1)) and not raw[..., shape[1]:].any()
+    assert np.array_equal(ctx.to_nchw(t2), x)
+    t.free()
+    t2.free()
+
+
+def _relu_module(shape, quant="INT8"):
+    g = graphs.Graph("io", 1)
+    op = g.add(graphs.Op("tpu.input", "x", [], shape))
+    if quant == "NONE":
+        op.quant = "NONE"
+        g.add(graphs.Op("tpu.quant", "q", ["x"], shape, dict(scale=1.0)))
+        y = g.add(graphs.Op("tpu.quant", "y", ["q"], shape, dict(scale=1.0)))
+        y.quant = "NONE"
+    else:
+        g.add(graphs.Op("tpu.relu", "y", ["x"], shape))
+    g.outputs = ["y"]
+    m = module()
+    m.load(g)
+    return m
+
+
+# one piece; several pieces; spans with a ragged end; more than the staging buffer holds
+SHAPES = [(1, 3, 20, 31), (2, 3, 181, 182), (4, 70, 61, 67), (3, 129, 130, 131), (5, 64, 331, 333)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_round_trip_of_float_and_int8_tensors(shape):
+    m = _relu_module(shape)
+    rng = np.random.default_rng(shape[3])
+    for k in range(2):      # a second tensor behind the first: the staging buffer is in use again
+        x = rng.integers(-128, 128, shape).astype(np.int8)
+        want = np.maximum(x, 0)
+        if k:
+            m.set_tensor_i8("x", x)
+        else:
+            m.set_tensor("x", x.astype(np.float32))
+        m.invoke()
+        assert np.array_equal(m.get_tensor_i8("y"), want)
+        assert np.array_equal(m.get_tensor("y"), want.astype(np.float32))
+        assert np.array_equal(m.get_tensor("x"), x.astype(np.float32))
+    m.close()
+
+
+@pytest.mark.parametrize("shape", SHAPES[:4])
+@pytest.mark.parametrize("value", [0.5, 128.0, -129.0, np.nan, np.inf])
+def test_a_float_that_is_no_int8_is_refused_and_changes_nothing(shape, value):
+    m = _relu_module(shape)
+    x = np.random.default_rng(3).integers(-128, 128, shape).astype(np.float32)
+    m.set_tensor("x", x)
+    bad = np.zeros(shape, np.float32)
+    bad.reshape(-1)[-2] = value
+    with pytest.raises(capi.TpuHipError, match="element %d" % (bad.size - 2)):
+        m.set_tensor("x", bad)
+    assert np.array_equal(m.get_tensor("x"), x)
+    m.close()
+
+
+@pytest.mark.parametrize("shape", SHAPES[:3])
+def test_round_trip_of_fp32_edges(shape):
+    m = _relu_module(shape, "NONE")
+    x = np.random.default_rng(5).integers(-128, 128, shape).astype(np.float32)
+    m.set_tensor("x", x)
+    m.invoke()
+    assert np.array_equal(m.get_tensor("x"), x) and np.array_equal(m.get_tensor("y"), x)
+    m.close()

@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "tpuhip.h"
 
@@ -24,6 +25,12 @@ struct tpuhip_ctx {
   // device memory kernels use beyond their operands (split-K partial sums): allocated on first need, grown when a larger layer comes, freed with the context
   void *workspace = nullptr;
   size_t workspace_bytes = 0;
+  // host tensors on their way to and from the device (host/host_io.cpp): a pinned buffer of at most 32 MiB, device memory
+  // for the dense form of a tensor that takes more than one piece, events behind the pieces; made on first use
+  void *stage = nullptr, *landing = nullptr;
+  size_t stage_bytes = 0, landing_bytes = 0;
+  bool stage_busy = false;   // kernels that read or write the pinned buffer may still be in flight
+  std::vector<hipEvent_t> stage_events;
 };
 
 // conv.hip: looks up this device's copy of the library's static scratch array (the one the
@@ -33,6 +40,9 @@ extern "C" int tpuhip_static_scratch_init(int device);
 extern "C" void tpuhip_static_scratch_forget(const tpuhip_ctx *ctx);
 
 namespace tpuhip {
+
+// host/host_io.cpp: frees a context's staging buffers
+void host_io_release(tpuhip_ctx *ctx);
 
 int set_error(int status, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 

@@ -301,6 +301,145 @@ __global__ __launch_bounds__(kThreads) void nhwc_to_nchw_kernel(const int8_t *sr
   }
 }
 
+// The int8 conversions move dwords: four pixels of four channels at a time, transposed in registers.  NCHW rows start at
+// any byte, so that side is accessed unaligned; where it lies in pinned host memory the bus sees whole runs of 128 bytes
+// (byte accesses: 64).  hw pixels, tile of 64 channels x 128 pixels, LDS rows of one pixel's 16 dwords + 1.
+__device__ __forceinline__ void transpose4x4(const uint32_t (&r)[4], uint32_t (&t)[4]) {
+  const uint32_t lo01 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
+  const uint32_t lo23 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+  t[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+  t[1] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+  t[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+  t[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+}
+// up to `left` bytes at p (any alignment); the rest of the dword is zero
+__device__ __forceinline__ uint32_t load_run(const int8_t *p, int64_t left) {
+  uint32_t v = 0;
+  if (left >= 4) {
+    __builtin_memcpy(&v, p, 4);
+  } else {
+    for (int k = 0; k < 4; ++k)
+      if (k < left) v |= (uint32_t)(uint8_t)p[k] << (8 * k);
+  }
+  return v;
+}
+__device__ __forceinline__ void store_run(int8_t *p, uint32_t v, int64_t left) {
+  if (left >= 4) {
+    __builtin_memcpy(p, &v, 4);
+  } else {
+    for (int k = 0; k < 4; ++k)
+      if (k < left) p[k] = (int8_t)(v >> (8 * k));
+  }
+}
+constexpr int kTransPix = 128, kTransRow = 17;
+
+__global__ __launch_bounds__(kThreads) void nchw_to_nhwc_i8_kernel(const int8_t *src, int8_t *dst, int c, int64_t hw, int cs) {
+  __shared__ uint32_t tile[kTransPix * kTransRow];
+  const int64_t s0 = (int64_t)blockIdx.x * kTransPix;
+  const int c0 = blockIdx.y * 64, n = blockIdx.z;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int pq = threadIdx.x & 31, cq = (threadIdx.x >> 5) + u * 8;
+    const int64_t s = s0 + pq * 4;
+    uint32_t r[4], t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ch = c0 + cq * 4 + i;
+      r[i] = ch < c && s < hw ? load_run(src + ((int64_t)n * c + ch) * hw + s, hw - s) : 0u;
+    }
+    transpose4x4(r, t);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tile[(pq * 4 + j) * kTransRow + cq] = t[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kTransPix / 16; ++u) {
+    const int cq = threadIdx.x & 15, p = (threadIdx.x >> 4) + u * 16;
+    if (s0 + p < hw && c0 + cq * 4 < cs)
+      *reinterpret_cast<uint32_t *>(dst + ((int64_t)n * hw + s0 + p) * cs + c0 + cq * 4) = tile[p * kTransRow + cq];
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void nhwc_to_nchw_i8_kernel(const int8_t *src, int8_t *dst, int c, int64_t hw, int cs) {
+  __shared__ uint32_t tile[kTransPix * kTransRow];
+  const int64_t s0 = (int64_t)blockIdx.x * kTransPix;
+  const int c0 = blockIdx.y * 64, n = blockIdx.z;
+#pragma unroll
+  for (int u = 0; u < kTransPix / 16; ++u) {
+    const int cq = threadIdx.x & 15, p = (threadIdx.x >> 4) + u * 16;
+    uint32_t v = 0;
+    if (s0 + p < hw && c0 + cq * 4 < cs)
+      v = *reinterpret_cast<const uint32_t *>(src + ((int64_t)n * hw + s0 + p) * cs + c0 + cq * 4);
+    tile[p * kTransRow + cq] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int pq = threadIdx.x & 31, cq = (threadIdx.x >> 5) + u * 8;
+    const int64_t s = s0 + pq * 4;
+    uint32_t r[4], t[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = tile[(pq * 4 + j) * kTransRow + cq];
+    transpose4x4(r, t);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ch = c0 + cq * 4 + i;
+      if (ch < c && s < hw) store_run(dst + ((int64_t)n * c + ch) * hw + s, t[i], hw - s);
+    }
+  }
+}
+
+// at most four channels (images): a lane makes four pixels from one dword of each plane and writes their channel rows,
+// one dword (cs 4) or 16 bytes (cs 16) each.  64 images of 3 x 224 x 224 from a 64-channel tile: 61 of 64 rows idle
+__global__ __launch_bounds__(kThreads) void image_to_nhwc_i8_kernel(const int8_t *src, int8_t *dst, int c, int64_t hw, int cs) {
+  const int64_t s = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 4;
+  const int n = blockIdx.z;
+  if (s >= hw) return;
+  uint32_t r[4], t[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = i < c ? load_run(src + ((int64_t)n * c + i) * hw + s, hw - s) : 0u;
+  transpose4x4(r, t);
+  int8_t *to = dst + ((int64_t)n * hw + s) * cs;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (s + j < hw) {
+      if (cs == 4) *reinterpret_cast<uint32_t *>(to + j * 4) = t[j];
+      else *reinterpret_cast<v4i *>(to + j * 16) = v4i{(int)t[j], 0, 0, 0};
+    }
+}
+
+// one pixel per image (vectors): both sides are rows of channels, only their pitch differs; 16 bytes per lane, the
+// dense side unaligned
+template <bool TO_DENSE>
+__global__ __launch_bounds__(kThreads) void vector_rows_i8_kernel(const int8_t *src, int8_t *dst, int64_t rows, int c, int cs) {
+  const int groups = TO_DENSE ? (c + 15) >> 4 : cs >> 4;
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const int64_t row = i / groups;
+  if (row >= rows) return;
+  const int c0 = (int)(i - row * groups) * 16;
+  if (TO_DENSE) {
+    const v4i v = *reinterpret_cast<const v4i *>(src + row * cs + c0);
+    int8_t *to = dst + row * c + c0;
+    if (c0 + 16 <= c) {
+      __builtin_memcpy(to, &v, 16);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) store_run(to + q * 4, (uint32_t)v[q], (int64_t)c - c0 - q * 4);
+    }
+  } else {
+    const int8_t *from = src + row * c + c0;
+    v4i v = {0, 0, 0, 0};
+    if (c0 + 16 <= c) {
+      __builtin_memcpy(&v, from, 16);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (c0 + q * 4 < c) v[q] = (int)load_run(from + q * 4, (int64_t)c - c0 - q * 4);
+    }
+    *reinterpret_cast<v4i *>(dst + row * cs + c0) = v;
+  }
+}
+
 int check_layout_args(const void *a, const void *b, int n, int c, int h, int w, int cs) {
   TPUHIP_REQUIRE(a && b, "layout: NULL pointer");
   TPUHIP_REQUIRE(n > 0 && c > 0 && h > 0 && w > 0, "layout: non-positive dimension");
@@ -315,8 +454,22 @@ int to_nhwc(tpuhip_ctx *ctx, const void *src, void *dst, int n, int c, int h, in
   TPUHIP_REQUIRE(ctx, "layout: NULL context");
   if (int rc = check_layout_args(src, dst, n, c, h, w, cs)) return rc;
   const int64_t hw = (int64_t)h * w;
-  dim3 grid((unsigned)ceil_div64(hw, 64), (unsigned)((cs + 63) / 64), (unsigned)n);
-  launch(ctx, (nchw_to_nhwc_kernel<SRC>), grid, dim3(kThreads), (const SRC *)src, (int8_t *)dst, c, hw, cs);
+  if constexpr (sizeof(SRC) == 1) {
+    // vectors, images, everything else
+    const auto *from = (const int8_t *)src;
+    if (hw == 1 && cs % 16 == 0)
+      launch(ctx, (vector_rows_i8_kernel<false>), dim3((unsigned)ceil_div64((int64_t)n * (cs / 16), kThreads)), dim3(kThreads), from,
+             (int8_t *)dst, (int64_t)n, c, cs);
+    else if (c <= 4 && cs <= 16)
+      launch(ctx, image_to_nhwc_i8_kernel, dim3((unsigned)ceil_div64(hw, kThreads * 4), 1, (unsigned)n), dim3(kThreads), from,
+             (int8_t *)dst, c, hw, cs);
+    else
+      launch(ctx, nchw_to_nhwc_i8_kernel, dim3((unsigned)ceil_div64(hw, kTransPix), (unsigned)((cs + 63) / 64), (unsigned)n),
+             dim3(kThreads), from, (int8_t *)dst, c, hw, cs);
+  } else {
+    dim3 grid((unsigned)ceil_div64(hw, 64), (unsigned)((cs + 63) / 64), (unsigned)n);
+    launch(ctx, (nchw_to_nhwc_kernel<SRC>), grid, dim3(kThreads), (const SRC *)src, (int8_t *)dst, c, hw, cs);
+  }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }
@@ -326,8 +479,17 @@ int to_nchw(tpuhip_ctx *ctx, const void *src, void *dst, int n, int c, int h, in
   TPUHIP_REQUIRE(ctx, "layout: NULL context");
   if (int rc = check_layout_args(src, dst, n, c, h, w, cs)) return rc;
   const int64_t hw = (int64_t)h * w;
-  dim3 grid((unsigned)ceil_div64(hw, 64), (unsigned)((c + 63) / 64), (unsigned)n);
-  launch(ctx, (nhwc_to_nchw_kernel<DST>), grid, dim3(kThreads), (const int8_t *)src, (DST *)dst, c, hw, cs);
+  if constexpr (sizeof(DST) == 1) {
+    if (hw == 1 && cs % 16 == 0)
+      launch(ctx, (vector_rows_i8_kernel<true>), dim3((unsigned)ceil_div64((int64_t)n * ((c + 15) / 16), kThreads)), dim3(kThreads),
+             (const int8_t *)src, (int8_t *)dst, (int64_t)n, c, cs);
+    else
+      launch(ctx, nhwc_to_nchw_i8_kernel, dim3((unsigned)ceil_div64(hw, kTransPix), (unsigned)((c + 63) / 64), (unsigned)n),
+             dim3(kThreads), (const int8_t *)src, (int8_t *)dst, c, hw, cs);
+  } else {
+    dim3 grid((unsigned)ceil_div64(hw, 64), (unsigned)((c + 63) / 64), (unsigned)n);
+    launch(ctx, (nhwc_to_nchw_kernel<DST>), grid, dim3(kThreads), (const int8_t *)src, (DST *)dst, c, hw, cs);
+  }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }

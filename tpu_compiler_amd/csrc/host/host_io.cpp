@@ -1,0 +1,445 @@
+#include "host_io.hpp"
+
+#include <sched.h>
+#include <unistd.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <condition_variable>
+#include <cstring>
+#include <functional>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#if !defined(__HIP_DEVICE_COMPILE__) && defined(__x86_64__)
+#include <immintrin.h>
+#define TPUHIP_X86 1
+#endif
+
+namespace tpuhip {
+
+// ---------------------------------------------------------------------------
+// float <-> int8.  A float is an integer of the range when it equals its own rounding and lies between the bounds; a
+// NaN fails the comparisons, which are all written so that an unordered result counts as bad.
+// ---------------------------------------------------------------------------
+namespace {
+
+bool to_bytes_plain(const float *src, int8_t *dst, size_t n, float lo, float hi) {
+  unsigned bad = 0;
+  const float magic = 12582912.0f;   // 1.5 * 2^23: adding and subtracting it rounds below 2^22
+  for (size_t i = 0; i < n; ++i) {
+    const float v = src[i];
+    bad |= (unsigned)!(v >= lo && v <= hi) | (unsigned)((v + magic) - magic != v);
+    const float in_range = v >= lo && v <= hi ? v : 0.0f;
+    dst[i] = (int8_t)(int32_t)in_range;
+  }
+  return bad != 0;
+}
+
+#ifdef TPUHIP_X86
+__attribute__((target("avx512f,avx512bw"))) bool to_bytes_avx512(const float *src, int8_t *dst, size_t n, float lo, float hi) {
+  const __m512 vlo = _mm512_set1_ps(lo), vhi = _mm512_set1_ps(hi);
+  __mmask16 bad = 0;
+  size_t i = 0;
+  for (; i + 16 <= n; i += 16) {
+    const __m512 v = _mm512_loadu_ps(src + i);
+    const __m512i q = _mm512_cvtps_epi32(v);   // rounds to nearest even
+    bad |= _mm512_cmp_ps_mask(v, vlo, _CMP_NGE_UQ) | _mm512_cmp_ps_mask(v, vhi, _CMP_NLE_UQ) |
+           _mm512_cmp_ps_mask(v, _mm512_cvtepi32_ps(q), _CMP_NEQ_UQ);
+    _mm_storeu_si128((__m128i *)(dst + i), _mm512_cvtepi32_epi8(q));   // keeps the low byte
+  }
+  const bool tail = to_bytes_plain(src + i, dst + i, n - i, lo, hi);
+  return bad != 0 || tail;
+}
+
+__attribute__((target("avx2"))) bool to_bytes_avx2(const float *src, int8_t *dst, size_t n, float lo, float hi) {
+  const __m256 vlo = _mm256_set1_ps(lo), vhi = _mm256_set1_ps(hi);
+  const __m256i low = _mm256_set1_epi32(0xff);
+  const __m256i order = _mm256_setr_epi32(0, 4, 1, 5, 2, 6, 3, 7);
+  __m256 bad = _mm256_setzero_ps();
+  size_t i = 0;
+  for (; i + 32 <= n; i += 32) {
+    __m256i q[4];
+    for (int k = 0; k < 4; ++k) {
+      const __m256 v = _mm256_loadu_ps(src + i + 8 * k);
+      q[k] = _mm256_cvtps_epi32(v);
+      bad = _mm256_or_ps(bad, _mm256_or_ps(_mm256_or_ps(_mm256_cmp_ps(v, vlo, _CMP_NGE_UQ), _mm256_cmp_ps(v, vhi, _CMP_NLE_UQ)),
+                                           _mm256_cmp_ps(v, _mm256_cvtepi32_ps(q[k]), _CMP_NEQ_UQ)));
+      q[k] = _mm256_and_si256(q[k], low);
+    }
+    const __m256i a = _mm256_packus_epi32(q[0], q[1]), b = _mm256_packus_epi32(q[2], q[3]);
+    _mm256_storeu_si256((__m256i *)(dst + i), _mm256_permutevar8x32_epi32(_mm256_packus_epi16(a, b), order));
+  }
+  const bool tail = to_bytes_plain(src + i, dst + i, n - i, lo, hi);
+  return _mm256_movemask_ps(bad) != 0 || tail;
+}
+
+__attribute__((target("avx512f"))) void to_floats_avx512(const int8_t *src, float *dst, size_t n, bool is_unsigned) {
+  size_t i = 0;
+  for (; i + 16 <= n; i += 16) {
+    const __m128i b = _mm_loadu_si128((const __m128i *)(src + i));
+    _mm512_storeu_ps(dst + i, _mm512_cvtepi32_ps(is_unsigned ? _mm512_cvtepu8_epi32(b) : _mm512_cvtepi8_epi32(b)));
+  }
+  for (; i < n; ++i) dst[i] = is_unsigned ? (float)(uint8_t)src[i] : (float)src[i];
+}
+
+__attribute__((target("avx2"))) void to_floats_avx2(const int8_t *src, float *dst, size_t n, bool is_unsigned) {
+  size_t i = 0;
+  for (; i + 8 <= n; i += 8) {
+    const __m128i b = _mm_loadl_epi64((const __m128i *)(src + i));
+    _mm256_storeu_ps(dst + i, _mm256_cvtepi32_ps(is_unsigned ? _mm256_cvtepu8_epi32(b) : _mm256_cvtepi8_epi32(b)));
+  }
+  for (; i < n; ++i) dst[i] = is_unsigned ? (float)(uint8_t)src[i] : (float)src[i];
+}
+
+int simd_level() {
+  static const int level = __builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512bw") ? 2
+                           : __builtin_cpu_supports("avx2")                                        ? 1
+                                                                                                   : 0;
+  return level;
+}
+#endif
+
+}  // namespace
+
+bool floats_to_bytes(const float *src, int8_t *dst, size_t n, bool is_unsigned) {
+  const float lo = is_unsigned ? 0.0f : -128.0f, hi = is_unsigned ? 255.0f : 127.0f;
+#ifdef TPUHIP_X86
+  if (simd_level() == 2) return to_bytes_avx512(src, dst, n, lo, hi);
+  if (simd_level() == 1) return to_bytes_avx2(src, dst, n, lo, hi);
+#endif
+  return to_bytes_plain(src, dst, n, lo, hi);
+}
+
+void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned) {
+#ifdef TPUHIP_X86
+  if (simd_level() == 2) return to_floats_avx512(src, dst, n, is_unsigned);
+  if (simd_level() == 1) return to_floats_avx2(src, dst, n, is_unsigned);
+#endif
+  for (size_t i = 0; i < n; ++i) dst[i] = is_unsigned ? (float)(uint8_t)src[i] : (float)src[i];
+}
+
+// ---------------------------------------------------------------------------
+// A few threads for the host passes, shared by all contexts of the process and started with the first tensor that is
+// worth them.  One caller has them at a time; another one that comes meanwhile does its pieces alone.  The caller takes
+// pieces like any worker and waits only for pieces that a worker has taken, so a process without them (a fork's child)
+// works the same, only slower.  They end with the process.
+// ---------------------------------------------------------------------------
+namespace {
+
+struct HostJob {
+  std::function<void(size_t)> piece;
+  size_t pieces = 0;
+  std::atomic<size_t> next{0}, finished{0};
+  bool step() {
+    const size_t i = next.fetch_add(1, std::memory_order_relaxed);
+    if (i >= pieces) return false;
+    piece(i);
+    finished.fetch_add(1, std::memory_order_release);
+    return true;
+  }
+};
+
+class HostWorkers {
+ public:
+  static HostWorkers &get() {
+    static HostWorkers w;
+    return w;
+  }
+
+  // offers the job to the workers; false: they are busy with another caller's.  Ends with leave().
+  bool enter(const std::shared_ptr<HostJob> &job) {
+    if (!users_.try_lock()) return false;
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      if (threads_.empty()) start();
+      job_ = job;
+      ++serial_;
+    }
+    wake_.notify_all();
+    return true;
+  }
+  void leave() {
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      job_.reset();
+    }
+    users_.unlock();
+  }
+
+ private:
+  HostWorkers() = default;
+  ~HostWorkers() {
+    if (getpid() != pid_) {   // a fork's child: the threads are the parent's
+      for (auto &t : threads_) t.detach();
+      return;
+    }
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      stop_ = true;
+    }
+    wake_.notify_all();
+    for (auto &t : threads_) t.join();
+  }
+
+  void start() {
+    pid_ = getpid();
+    cpu_set_t set;
+    int cpus = 1;
+    if (sched_getaffinity(0, sizeof(set), &set) == 0) cpus = CPU_COUNT(&set);
+    // seven beside the caller reach the memory bandwidth of a socket's share; never more than the CPUs there are
+    const int count = std::max(0, std::min(7, cpus - 1));
+    for (int i = 0; i < count; ++i) threads_.emplace_back([this] { work(); });
+  }
+
+  void work() {
+    uint64_t seen = 0;
+    for (;;) {
+      std::shared_ptr<HostJob> job;
+      {
+        std::unique_lock<std::mutex> l(mu_);
+        wake_.wait(l, [&] { return stop_ || (job_ && serial_ != seen); });
+        if (stop_) return;
+        seen = serial_;
+        job = job_;
+      }
+      while (job->step()) {
+      }
+    }
+  }
+
+  std::mutex users_, mu_;
+  std::condition_variable wake_;
+  std::shared_ptr<HostJob> job_;
+  uint64_t serial_ = 0;
+  bool stop_ = false;
+  pid_t pid_ = 0;
+  std::vector<std::thread> threads_;
+};
+
+constexpr size_t kPiece = 256 << 10;        // bytes of the staging buffer per piece of a host pass
+constexpr size_t kAlone = 192 << 10;        // up to here one thread is done before a worker has woken
+constexpr size_t kStageMax = 32 << 20;      // the staging buffer grows to this; larger tensors go through it in parts
+
+// the pinned buffer, free to be written: transfers out of it that are still in flight have ended
+int stage_ready(tpuhip_ctx *ctx, size_t bytes) {
+  TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
+  if (ctx->stage_busy) {
+    TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->stage_busy = false;
+  }
+  bytes = std::min(bytes, kStageMax);
+  if (bytes <= ctx->stage_bytes) return TPUHIP_OK;
+  size_t want = 64 << 10;
+  while (want < bytes) want *= 2;
+  if (ctx->stage) TPUHIP_CHECK_HIP(hipHostFree(ctx->stage));
+  ctx->stage = nullptr;
+  ctx->stage_bytes = 0;
+  TPUHIP_CHECK_HIP(hipHostMalloc(&ctx->stage, want, hipHostMallocDefault));
+  ctx->stage_bytes = want;
+  return TPUHIP_OK;
+}
+
+// device memory for a tensor that arrives in more than one piece
+int landing_ready(tpuhip_ctx *ctx, size_t bytes) {
+  if (bytes <= ctx->landing_bytes) return TPUHIP_OK;
+  if (ctx->landing) {
+    TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    TPUHIP_CHECK_HIP(hipFree(ctx->landing));
+  }
+  ctx->landing = nullptr;
+  ctx->landing_bytes = 0;
+  TPUHIP_CHECK_HIP(hipMalloc(&ctx->landing, bytes + 256));
+  ctx->landing_bytes = bytes;
+  return TPUHIP_OK;
+}
+
+// dwords between pinned and device memory (bus-bound: 57 GB/s from 256 workgroups on, wider accesses no faster); int8
+// data may be rounded up to a dword, the staging and landing buffers have the room, floats are whole dwords
+__global__ __launch_bounds__(256) void stage_copy_kernel(const uint32_t *src, uint32_t *dst, size_t n) {
+  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  for (; i < n; i += stride) dst[i] = src[i];
+}
+
+int stage_copy(tpuhip_ctx *ctx, const void *src, void *dst, size_t bytes) {
+  const size_t n = (bytes + 3) / 4;
+  const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 256);
+  hipLaunchKernelGGL(stage_copy_kernel, dim3(blocks), dim3(256), 0, ctx->stream, (const uint32_t *)src, (uint32_t *)dst, n);
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
+}
+
+// element -> bytes on the host side and in the staging buffer
+size_t host_size(HostKind k) { return k == HostKind::kBytes ? 1 : sizeof(float); }
+size_t stage_size(HostKind k) { return k == HostKind::kFloats ? sizeof(float) : 1; }
+
+}  // namespace
+
+int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst, bool *bad) {
+  *bad = false;
+  const size_t count = (size_t)t.n * t.c * t.h * t.w;
+  const size_t per = stage_size(kind), total = count * per;
+  if (int rc = stage_ready(ctx, total)) return rc;
+  auto pass = [&](size_t first, size_t elements, int8_t *to) {
+    const char *from = (const char *)src + first * host_size(kind);
+    if (kind == HostKind::kFloatStored) return floats_to_bytes((const float *)from, to, elements, t.is_unsigned);
+    memcpy(to, from, elements * per);
+    return false;
+  };
+  int8_t *stage = (int8_t *)ctx->stage;
+  if (total <= kAlone) {
+    *bad = pass(0, count, stage);
+    if (*bad) return TPUHIP_OK;
+    ctx->stage_busy = true;
+    if (kind == HostKind::kFloats) return stage_copy(ctx, stage, dst, total);
+    return tpuhip_nchw_to_nhwc_i8(ctx, stage, dst, t.n, t.c, t.h, t.w, t.cs);
+  }
+  // several pieces: each goes to a landing buffer on the device as soon as it and those before it are there; the tensor
+  // itself is written once all of them have passed the check
+  void *land = dst;
+  if (kind != HostKind::kFloats) {
+    if (int rc = landing_ready(ctx, total)) return rc;
+    land = ctx->landing;
+  }
+  std::atomic<bool> any_bad{false};
+  for (size_t part = 0; part < total; part += ctx->stage_bytes) {
+    const size_t bytes = std::min(total - part, ctx->stage_bytes);
+    if (part) TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));   // the buffer is written anew
+    auto job = std::make_shared<HostJob>();
+    job->pieces = (bytes + kPiece - 1) / kPiece;
+    std::unique_ptr<std::atomic<uint8_t>[]> there(new std::atomic<uint8_t>[job->pieces]);
+    for (size_t i = 0; i < job->pieces; ++i) there[i].store(0, std::memory_order_relaxed);
+    job->piece = [&, part, bytes](size_t i) {
+      const size_t at = i * kPiece, len = std::min(kPiece, bytes - at);
+      if (pass((part + at) / per, len / per, stage + at)) any_bad.store(true, std::memory_order_relaxed);
+      there[i].store(1, std::memory_order_release);
+    };
+    HostWorkers &workers = HostWorkers::get();
+    const bool shared = workers.enter(job);
+    int rc = TPUHIP_OK;
+    size_t sent = 0;   // pieces handed to the device
+    ctx->stage_busy = true;
+    for (bool more = true; sent < job->pieces;) {
+      if (more) more = job->step();
+      size_t run = sent;
+      while (run < job->pieces && there[run].load(std::memory_order_acquire)) ++run;
+      // one launch moves what is there: at least four pieces while there is still something to do meanwhile
+      if (run == sent || (more && run - sent < 4)) {
+        if (!more) std::this_thread::yield();
+        continue;
+      }
+      const size_t at = sent * kPiece, end = std::min(run * kPiece, bytes);
+      if (!rc && !any_bad.load(std::memory_order_relaxed)) rc = stage_copy(ctx, stage + at, (char *)land + part + at, end - at);
+      sent = run;
+    }
+    while (job->finished.load(std::memory_order_acquire) < job->pieces) std::this_thread::yield();
+    if (shared) workers.leave();
+    if (rc) return rc;
+    if (any_bad.load()) {
+      *bad = true;
+      return TPUHIP_OK;
+    }
+  }
+  if (kind == HostKind::kFloats) return TPUHIP_OK;
+  return tpuhip_nchw_to_nhwc_i8(ctx, land, dst, t.n, t.c, t.h, t.w, t.cs);
+}
+
+int device_to_host(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst) {
+  const size_t count = (size_t)t.n * t.c * t.h * t.w;
+  const size_t per = stage_size(kind), total = count * per;
+  if (int rc = stage_ready(ctx, total)) return rc;
+  int8_t *stage = (int8_t *)ctx->stage;
+  auto pass = [&](size_t first, size_t elements, const int8_t *from) {
+    char *to = (char *)dst + first * host_size(kind);
+    if (kind == HostKind::kFloatStored)
+      bytes_to_floats(from, (float *)to, elements, t.is_unsigned);
+    else
+      memcpy(to, from, elements * per);
+  };
+  // the host bytes are what the caller's memory costs (fresh pages above all), so they decide on the threads
+  const bool alone = count * host_size(kind) <= kAlone;
+  if (total <= ctx->stage_bytes && (alone || total <= 2 * kPiece)) {
+    const int rc = kind == HostKind::kFloats ? stage_copy(ctx, src, stage, total)
+                                             : tpuhip_nhwc_to_nchw_i8(ctx, src, stage, t.n, t.c, t.h, t.w, t.cs);
+    if (rc) return rc;
+    TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    if (alone) {
+      pass(0, count, stage);
+      return TPUHIP_OK;
+    }
+    auto job = std::make_shared<HostJob>();
+    const size_t grain = kPiece / host_size(kind);
+    job->pieces = (count + grain - 1) / grain;
+    job->piece = [&](size_t i) { pass(i * grain, std::min(grain, count - i * grain), stage + i * grain * per); };
+    const bool shared = HostWorkers::get().enter(job);
+    while (job->step()) {
+    }
+    while (job->finished.load(std::memory_order_acquire) < job->pieces) std::this_thread::yield();
+    if (shared) HostWorkers::get().leave();
+    return TPUHIP_OK;
+  }
+  // The dense form is made on the device and comes over in spans of eight pieces, an event behind each; the host pass
+  // of a span runs while the next ones are on the bus.
+  const void *dense = src;
+  if (kind != HostKind::kFloats) {
+    if (int rc = landing_ready(ctx, total)) return rc;
+    if (int rc = tpuhip_nhwc_to_nchw_i8(ctx, src, ctx->landing, t.n, t.c, t.h, t.w, t.cs)) return rc;
+    dense = ctx->landing;
+  }
+  constexpr size_t kSpan = 8 * kPiece;
+  for (size_t part = 0; part < total; part += ctx->stage_bytes) {
+    const size_t bytes = std::min(total - part, ctx->stage_bytes);
+    const size_t spans = (bytes + kSpan - 1) / kSpan;
+    while (ctx->stage_events.size() < spans) {
+      hipEvent_t e;
+      TPUHIP_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      ctx->stage_events.push_back(e);
+    }
+    for (size_t s = 0; s < spans; ++s) {
+      const size_t at = s * kSpan;
+      if (int rc = stage_copy(ctx, (const char *)dense + part + at, stage + at, std::min(kSpan, bytes - at))) return rc;
+      TPUHIP_CHECK_HIP(hipEventRecord(ctx->stage_events[s], ctx->stream));
+    }
+    auto job = std::make_shared<HostJob>();
+    job->pieces = (bytes + kPiece - 1) / kPiece;
+    std::atomic<size_t> arrived{0};     // spans that are in the buffer
+    std::atomic<bool> lost{false};      // the device failed: nothing more arrives
+    job->piece = [&, part, bytes](size_t i) {
+      const size_t at = i * kPiece, len = std::min(kPiece, bytes - at);
+      while (arrived.load(std::memory_order_acquire) <= at / kSpan) {
+        if (lost.load(std::memory_order_relaxed)) return;
+        std::this_thread::yield();
+      }
+      pass((part + at) / per, len / per, stage + at);
+    };
+    HostWorkers &workers = HostWorkers::get();
+    const bool shared = workers.enter(job);
+    hipError_t e = hipSuccess;
+    for (size_t s = 0; s < spans && e == hipSuccess; ++s) {
+      e = hipEventSynchronize(ctx->stage_events[s]);
+      if (e == hipSuccess) arrived.store(s + 1, std::memory_order_release);
+    }
+    if (e != hipSuccess) lost.store(true);
+    while (job->step()) {
+    }
+    while (job->finished.load(std::memory_order_acquire) < job->pieces) std::this_thread::yield();
+    if (shared) workers.leave();
+    TPUHIP_CHECK_HIP(e);
+  }
+  return TPUHIP_OK;
+}
+
+void host_io_release(tpuhip_ctx *ctx) {
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
+  if (ctx->landing) (void)hipFree(ctx->landing);
+  for (hipEvent_t e : ctx->stage_events) (void)hipEventDestroy(e);
+  ctx->stage = ctx->landing = nullptr;
+  ctx->stage_bytes = ctx->landing_bytes = 0;
+  ctx->stage_events.clear();
+}
+
+}  // namespace tpuhip

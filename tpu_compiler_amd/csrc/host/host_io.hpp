@@ -1,0 +1,36 @@
+// Tensors between a caller's host memory and the device: pageable buffers on one side, channels-last int8 on the
+// other, a pinned staging buffer of the context in between.
+//
+// Only int8 crosses the bus, whatever type the caller holds, and no DMA is involved: the layout kernels read and write
+// the pinned buffer themselves (a kernel moves it at the bus rate, 57 GB/s, and a copy engine in front of a kernel
+// costs another 8 us).  The host pass (float <-> int8 with its check, or a plain copy) runs in pieces on a few threads,
+// and the pieces overlap with the transfer of those before them.
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+#include "common.hpp"
+
+namespace tpuhip {
+
+// n floats -> int8; the return value tells whether one of them is no integer in [-128, 127] (is_unsigned: [0, 255],
+// stored as the byte)
+bool floats_to_bytes(const float *src, int8_t *dst, size_t n, bool is_unsigned);
+// n int8 (is_unsigned: uint8) -> floats
+void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned);
+
+// What the host side holds: float-stored integers (converted and checked), int8 bytes, or floats that stay floats.
+enum class HostKind { kFloatStored, kBytes, kFloats };
+
+struct HostTensor {
+  int n, c, h, w, cs;   // channels-last int8 on the device; for kFloats the device side is dense NCHW floats
+  bool is_unsigned;
+};
+
+// host -> device, issued to the context's stream; the caller's buffer may be reused on return.  *bad: an element of a
+// float-stored tensor is no integer of the byte range (nothing has been written to dst then).
+int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst, bool *bad);
+// device -> host; waits for the work in front of it
+int device_to_host(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst);
+}  // namespace tpuhip

@@ -466,6 +466,12 @@ std::shared_ptr<std::vector<float>> ModuleInterpreter::getTensor(std::string &na
   return it->second->tensor(bidx);
 }
 
+void ModuleInterpreter::getTensor(const std::string &name, float *dst, size_t num, int32_t bidx) {
+  auto it = activationMapping.find(name);
+  if (it == activationMapping.end()) fail(" Not Find Op name: " + name + " tensor");
+  it->second->read(dst, num, bidx);
+}
+
 void ModuleInterpreter::getTensorI8(const std::string &name, int8_t *dst, size_t num, int32_t bidx) {
   auto it = activationMapping.find(name);
   if (it == activationMapping.end()) fail(" Not Find Op name: " + name + " tensor");

@@ -5,6 +5,8 @@
 // through the C ABI.
 #include "tpuhip/interpreter.hpp"
 
+#include "host_io.hpp"
+
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -101,8 +103,6 @@ TensorData::TensorData(tpuhip_ctx *ctx, int32_t batch_, const SyncedDataShape &s
 }
 
 TensorData::~TensorData() {
-  if (stage_dev_) tpuhip_free(ctx_, stage_dev_);
-  if (stage_host_) tpuhip_host_free(ctx_, stage_host_);
   if (base_) tpuhip_free(ctx_, base_);
 }
 
@@ -126,73 +126,42 @@ void TensorData::set_batch_idx(int32_t bidx) {
 void TensorData::assign(const float *first, size_t num, int32_t bidx) {
   if (num != size_) fail("TensorData::assign: size mismatch");
   if (bidx < 0 || bidx >= batch) fail("TensorData::assign: slot out of range");
-  if (f32) {
-    ck(tpuhip_upload(ctx_, (char *)base_ + slot_bytes() * (size_t)bidx, first, num * sizeof(float)),
-       "TensorData::assign");
-    return;
-  }
-  const float lo = is_unsigned ? 0.0f : -128.0f, hi = is_unsigned ? 255.0f : 127.0f;
-  if (!stage_host_) ck(tpuhip_host_malloc(ctx_, num * sizeof(float), &stage_host_), "TensorData::assign");
-  if (!stage_dev_) ck(tpuhip_malloc(ctx_, num * sizeof(float), &stage_dev_), "TensorData::assign");
-  // One pass: copy into the pinned buffer, check that every element is an integer of the
-  // tensor's byte range, and let 128..255 travel as the int8 value with the same byte.  No
-  // early exit and no library call in the loop, so it vectorises; adding and subtracting
-  // 1.5 * 2^23 rounds a float of magnitude below 2^22 to an integer.
-  float *stage = static_cast<float *>(stage_host_);
-  const float magic = 12582912.0f, wrap_from = is_unsigned ? 128.0f : 1e9f;
-  unsigned bad = 0;
-  for (size_t i = 0; i < num; ++i) {
-    const float v = first[i];
-    const float r = (v + magic) - magic;
-    bad |= (unsigned)!(v >= lo && v <= hi) | (unsigned)(r != v);
-    stage[i] = v >= wrap_from ? v - 256.0f : v;
-  }
-  if (bad)
-    for (size_t i = 0; i < num; ++i)
-      if (!(first[i] >= lo && first[i] <= hi) || first[i] != std::nearbyint(first[i]))
-        fail("TensorData::assign: element " + std::to_string(i) + " = " + std::to_string(first[i]) +
-             (is_unsigned ? " is not a uint8 value" : " is not an int8 value"));
-  ck(tpuhip_upload(ctx_, stage_dev_, stage, num * sizeof(float)), "TensorData::assign");
-  ck(tpuhip_nchw_f32_to_nhwc_i8(ctx_, stage_dev_, (char *)base_ + slot_bytes() * (size_t)bidx, n, c, h, w,
-                                cs),
+  bool bad = false;
+  ck(host_to_device(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, f32 ? HostKind::kFloats : HostKind::kFloatStored, first,
+                    slot(bidx), &bad),
      "TensorData::assign");
+  if (!bad) return;
+  const float lo = is_unsigned ? 0.0f : -128.0f, hi = is_unsigned ? 255.0f : 127.0f;
+  for (size_t i = 0; i < num; ++i)
+    if (!(first[i] >= lo && first[i] <= hi) || first[i] != std::nearbyint(first[i]))
+      fail("TensorData::assign: element " + std::to_string(i) + " = " + std::to_string(first[i]) +
+           (is_unsigned ? " is not a uint8 value" : " is not an int8 value"));
+  fail("TensorData::assign: the data changed while it was read");
 }
 
 void TensorData::assign_i8(const int8_t *first, size_t num, int32_t bidx) {
   if (num != size_) fail("TensorData::assign_i8: size mismatch");
   if (bidx < 0 || bidx >= batch) fail("TensorData::assign_i8: slot out of range");
   if (f32) fail("TensorData::assign_i8: this tensor holds fp32 data");
-  // the staging buffers of assign() serve here too (a quarter of them is used)
-  if (!stage_host_) ck(tpuhip_host_malloc(ctx_, num * sizeof(float), &stage_host_), "TensorData::assign_i8");
-  if (!stage_dev_) ck(tpuhip_malloc(ctx_, num * sizeof(float), &stage_dev_), "TensorData::assign_i8");
-  std::memcpy(stage_host_, first, num);
-  ck(tpuhip_upload(ctx_, stage_dev_, stage_host_, num), "TensorData::assign_i8");
-  ck(tpuhip_nchw_to_nhwc_i8(ctx_, stage_dev_, (char *)base_ + slot_bytes() * (size_t)bidx, n, c, h, w, cs),
+  bool bad = false;
+  ck(host_to_device(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, HostKind::kBytes, first, slot(bidx), &bad),
      "TensorData::assign_i8");
 }
 
-std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
+void TensorData::read(float *dst, size_t num, int32_t bidx) const {
   if (!materialized)
     fail("TensorData::tensor: this tensor is fused into its consumer and never written "
          "(load the module with keep_all_tensors to read it)");
+  if (num != size_) fail("TensorData::tensor: size mismatch");
   if (bidx < 0 || bidx >= batch) fail("TensorData::tensor: slot out of range");
+  ck(device_to_host(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, f32 ? HostKind::kFloats : HostKind::kFloatStored,
+                    slot(bidx), dst),
+     "TensorData::tensor");
+}
+
+std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
   auto out = std::make_shared<std::vector<float>>(size_);
-  if (f32) {
-    ck(tpuhip_download(ctx_, out->data(), (char *)base_ + slot_bytes() * (size_t)bidx,
-                       size_ * sizeof(float)),
-       "TensorData::tensor");
-    return out;
-  }
-  void *tmp = nullptr;
-  ck(tpuhip_malloc(ctx_, size_ * sizeof(float), &tmp), "TensorData::tensor");
-  int rc = tpuhip_nhwc_i8_to_nchw_f32(ctx_, (char *)base_ + slot_bytes() * (size_t)bidx, tmp, n, c,
-                                      h, w, cs);
-  if (!rc) rc = tpuhip_download(ctx_, out->data(), tmp, size_ * sizeof(float));
-  tpuhip_free(ctx_, tmp);
-  ck(rc, "TensorData::tensor");
-  if (is_unsigned)
-    for (auto &v : *out)
-      if (v < 0.0f) v += 256.0f;
+  read(out->data(), out->size(), bidx);
   return out;
 }
 
@@ -203,13 +172,7 @@ void TensorData::read_i8(int8_t *dst, size_t num, int32_t bidx) const {
   if (f32) fail("TensorData::read_i8: this tensor holds fp32 data");
   if (num != size_) fail("TensorData::read_i8: size mismatch");
   if (bidx < 0 || bidx >= batch) fail("TensorData::read_i8: slot out of range");
-  void *tmp = nullptr;
-  ck(tpuhip_malloc(ctx_, size_, &tmp), "TensorData::read_i8");
-  int rc = tpuhip_nhwc_to_nchw_i8(ctx_, (char *)base_ + slot_bytes() * (size_t)bidx, tmp, n, c, h, w,
-                                  cs);
-  if (!rc) rc = tpuhip_download(ctx_, dst, tmp, size_);
-  tpuhip_free(ctx_, tmp);
-  ck(rc, "TensorData::read_i8");
+  ck(device_to_host(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, HostKind::kBytes, slot(bidx), dst), "TensorData::read_i8");
 }
 
 // ---------------------------------------------------------------------------

@@ -135,10 +135,7 @@ int tpuhip_module_get_tensor(tpuhip_module *m, const char *name, float *dst, siz
                              int bidx) {
   GUARD(m, {
     if (!name || !dst) throw std::runtime_error("get_tensor: NULL argument");
-    std::string n(name);
-    auto t = m->interp->getTensor(n, bidx);
-    if (t->size() != count) throw std::runtime_error("get_tensor: size mismatch");
-    memcpy(dst, t->data(), count * sizeof(float));
+    m->interp->getTensor(name, dst, count, bidx);
   })
 }
 

@@ -62,6 +62,7 @@ class module:
         self.op_info = []
         self.graph = None
         self._mlir_path = None
+        self._known = {}      # names and shapes of the loaded graph, asked for once (a ctypes call each)
 
     def close(self):
         if self.h:
@@ -81,6 +82,7 @@ class module:
     def load(self, graph, target_op=""):
         """updateWeightMap + loadModule (pymlir.cpp:99-122) for a TPU-dialect .mlir file given by
         name, like pymlir, or for a graph object built in Python."""
+        self._known = {}
         if isinstance(graph, (str, os.PathLike)):
             self.graph = None
             self._mlir_path = os.fspath(graph)
@@ -149,6 +151,7 @@ class module:
         """the tpuc-interpreter tool: <mlir> --tensor-in <npz> [--tensor-out <npz>]
         [--dump-all-tensor <npz>]"""
         enc = lambda p: os.fspath(p).encode() if p else None
+        self._known = {}
         self._ck(self.lib.tpuhip_module_interpret_files(self.h, enc(mlir_path), enc(tensor_in),
                                                         enc(tensor_out), enc(dump_all_tensor)))
 
@@ -158,6 +161,9 @@ class module:
 
     # -- details ------------------------------------------------------------
     def get_input_details(self):
+        return dict(self._once("inputs", self._ask_inputs))
+
+    def _ask_inputs(self):
         out = {}
         for i in range(self.lib.tpuhip_module_num_inputs(self.h)):
             name = self.lib.tpuhip_module_input_name(self.h, i).decode()
@@ -165,14 +171,22 @@ class module:
         return out
 
     def get_output_details(self):
-        return [self.lib.tpuhip_module_output_name(self.h, i).decode()
-                for i in range(self.lib.tpuhip_module_num_outputs(self.h))]
+        return list(self._once("outputs", lambda: [self.lib.tpuhip_module_output_name(self.h, i).decode()
+                                                   for i in range(self.lib.tpuhip_module_num_outputs(self.h))]))
+
+    def _once(self, key, ask):
+        if key not in self._known:
+            self._known[key] = ask()
+        return self._known[key]
 
     def tensor_names(self):
         return [self.lib.tpuhip_module_tensor_name(self.h, i).decode()
                 for i in range(self.lib.tpuhip_module_num_tensors(self.h))]
 
     def tensor_shape(self, name):
+        return self._once(("shape", name), lambda: self._ask_shape(name))
+
+    def _ask_shape(self, name):
         dims = (C.c_int64 * 8)()
         nd = C.c_int()
         self._ck(self.lib.tpuhip_module_tensor_shape(self.h, name.encode(), dims, C.byref(nd)))
