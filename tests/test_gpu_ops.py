@@ -1514,3 +1514,34 @@ def test_random_pool_add_table_upsample_concat_sweep(ctx):
             for t in tmp:
                 t.free()
     assert len(seen) == 7 and min(seen.values()) > 50, seen
+
+
+# n, g, ic, oc, ih, iw, k, stride, pads, dil, ins, relu: grouped convs and convs over inserted zeros
+GATHER_CASES = [
+    (2, 32, 128, 128, 13, 11, 3, (1, 1), (1, 1, 1, 1), (1, 1), (0, 0), True),      # 4 x 4 channels per group
+    (1, 2, 96, 64, 9, 10, 3, (2, 1), (1, 1, 1, 1), (1, 1), (0, 0), False),         # wide groups, stride
+    (3, 3, 30, 99, 6, 7, 1, (1, 1), (0, 0, 0, 0), (1, 1), (0, 0), True),           # group borders off the 16s and 32s
+    (1, 4, 48, 8, 8, 8, 3, (1, 1), (2, 2, 2, 2), (2, 2), (0, 0), False),           # few output channels, dilation
+    (2, 1, 64, 40, 9, 7, 4, (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True),           # transposed 4x4 stride 2
+    (1, 1, 20, 33, 6, 5, 3, (1, 1), (2, 2, 2, 2), (1, 1), (2, 1), False),          # zeros 2 by 1, odd kernel
+    (1, 1, 16, 16, 5, 6, 2, (1, 1), (0, 1, 0, 1), (1, 1), (3, 3), False),          # phases without a tap
+    (1, 1, 24, 16, 7, 7, 3, (2, 2), (1, 1, 1, 1), (1, 2), (1, 2), True),           # stride against the zeros
+    (1, 5, 40, 20, 6, 9, 4, (1, 1), (2, 3, 1, 2), (1, 1), (1, 1), False),          # groups and zeros
+    (1, 1, 1, 1, 1, 1, 2, (1, 1), (1, 1, 1, 1), (1, 1), (1, 1), False),            # one pixel
+    (9, 8, 256, 256, 40, 44, 3, (1, 1), (1, 1, 1, 1), (1, 1), (0, 0), True),       # 64 pixels per wave
+    (6, 1, 96, 96, 40, 37, 4, (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True),
+]
+
+
+@pytest.mark.parametrize("case", GATHER_CASES)
+@pytest.mark.parametrize("smallest_shift", [0, 1])
+def test_conv_grouped_and_transposed(ctx, case, smallest_shift):
+    n, g, ic, oc, ih, iw, k, stride, pads, dil, ins, relu = case
+    rng = np.random.default_rng(ic * 7 + oc + k + ih)
+    x = rnd_i8(rng, (n, ic, ih, iw))
+    w = rnd_w(rng, (oc, ic // g, k, k), sigma=20)
+    bias, rsh, mult = rnd_params(rng, oc, 5, 11)
+    rsh[::7] = smallest_shift                       # 0: the form of the requantisation that may overflow
+    want = oracle_conv(x, w, bias, rsh, mult, g, stride, pads, dil, ins, relu)
+    got, _ = run_conv(ctx, x, w, bias, rsh, mult, g=g, stride=stride, pads=pads, dil=dil, ins=ins, do_relu=relu)
+    assert np.array_equal(got, want), "%d mismatches" % (got != want).sum()

@@ -5,13 +5,14 @@
 //     output channels), im2col'ed channels-last activations as the B operand
 //     (columns = output pixels), both staged through LDS in 64-byte K slices;
 //   * depthwise (g == ic == oc): channels-last direct kernel, no MFMA;
-//   * anything else (grouped, input dilation): one thread per output.
+//   * anything else (grouped, inserted zeros): the gather kernel of conv_gather.hip, or one thread per output.
 //
 // All three share the requantisation epilogue of
 // quantizeActivationInt8PerChannelMultiplierAndRShift
 // (lib/Dialect/TPU/Quantization/QuantizationArithmetic.cpp:849-871).
 #include "common.hpp"
 #include "conv_epilogue.hpp"
+#include "conv_gather.hpp"
 
 #include <map>
 #include <mutex>
@@ -52,6 +53,8 @@ struct tpuhip_conv_weights {
   // a FullyConnected whose K is beyond what the conv kernels index (more than 4096 input
   // channels): only the K-splitting FullyConnected kernels, which walk K linearly, run it
   bool fc_only = false;
+  // the direct path's layers where the caller left the choice: their form on the matrix cores (NULL: not covered)
+  GatherPlan *gather = nullptr;
   std::vector<int8_t> host_filter;  // OIHW copy, kept while the layer can still be repacked
   int8_t *w = nullptr;   // packed filter
   int32_t *bias = nullptr;
@@ -4234,8 +4237,14 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
       for (int tap = 0; tap < d.kh * d.kw; ++tap)
         packed[((size_t)(tap / 4) * cw->ocp + c) * 4 + tap % 4] = filter[(size_t)c * d.kh * d.kw + tap];
   } else {
+    if (d.algo == ALGO_AUTO && !dense)
+      if (int rc = gather_prepack(ctx, d, filter, &cw->gather)) {
+        tpuhip_conv2d_weights_destroy(ctx, cw);
+        return rc;
+      }
     cw->ocp = d.oc;
-    packed.assign((size_t)d.oc * d.kh * d.kw * icg, 0);
+    if (!cw->gather) packed.assign((size_t)d.oc * d.kh * d.kw * icg, 0);
+    if (!cw->gather)
     for (int oc = 0; oc < d.oc; ++oc)
       for (int c = 0; c < icg; ++c)
         for (int kh = 0; kh < d.kh; ++kh)
@@ -4271,7 +4280,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   }
   cw->fast = fast ? 1 : 0;
   int rc = TPUHIP_OK;
-  if (algo != ALGO_MFMA) {
+  if (algo != ALGO_MFMA && !cw->gather) {
     rc = tpuhip_malloc(ctx, packed.size(), (void **)&cw->w);
     if (!rc) rc = tpuhip_upload(ctx, cw->w, packed.data(), packed.size());
   }
@@ -4279,7 +4288,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   if (!rc) rc = tpuhip_malloc(ctx, qp.size() * sizeof(QParam), (void **)&cw->qp);
   if (!rc) rc = tpuhip_upload(ctx, cw->bias, b32.data(), b32.size() * sizeof(int32_t));
   if (!rc) rc = tpuhip_upload(ctx, cw->qp, qp.data(), qp.size() * sizeof(QParam));
-  if (!rc && algo != ALGO_DIRECT) {
+  if (!rc && (algo != ALGO_DIRECT || cw->gather)) {
     std::vector<int32_t> planes(3 * nparam);
     for (size_t i = 0; i < nparam; ++i) {
       planes[i] = qp[i].mult;
@@ -4314,6 +4323,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
 int tpuhip_conv2d_weights_destroy(tpuhip_ctx *ctx, tpuhip_conv_weights *w) {
   if (!w) return TPUHIP_OK;
   TPUHIP_REQUIRE(ctx, "tpuhip_conv2d_weights_destroy: NULL context");
+  gather_destroy(ctx, w->gather);
   int rc = tpuhip_free(ctx, w->w);
   int rc2 = tpuhip_free(ctx, w->bias);
   int rc3 = tpuhip_free(ctx, w->qp);
@@ -4447,6 +4457,10 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
                  "overflow the rounding", kTiles[w->tile].name);
   TPUHIP_REQUIRE((w->split_oc != 0) == (post.y2 != nullptr),
                  "conv: weights packed as a pair run through tpuhip_conv2d_pair_i8 (and only they do)");
+  if (w->gather) {
+    TPUHIP_REQUIRE(!post.any() && y, "conv: grouped and transposed convs take no fused work");
+    return gather_run(ctx, w->gather, x, y, w->bias, w->qplanes, w->qplanes + w->nparam, w->qplanes + 2 * w->nparam, w->fast != 0);
+  }
   ConvArgs a;
   fill_args(ctx, w, x, y, &a);
   apply_fusion(&a, y, post);

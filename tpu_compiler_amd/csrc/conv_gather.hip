@@ -1,0 +1,347 @@
+// Convolutions that are no plain implicit GEMM -- groups, zeros inserted between the input's pixels -- as one
+// (core/conv.cpp:11-104; core/deconv.cpp for the transposed form, which reaches the kernels as inserted zeros).
+//
+//   * Inserted zeros.  With S = ins + 1, an output row oh meets real input rows only through the taps kh for which
+//     oh * sh - pt + kh * dh is a multiple of S.  Rows that are congruent modulo P = S / gcd(S, sh) meet the same taps at
+//     the same distance, so a layer is P_h * P_w convs ("phases") over the input as it lies in memory, each with its own
+//     list of (dy, dx) taps, and no multiplication by an inserted zero is left (three quarters of all, doubling a map).
+//   * Groups.  A block of 32 output channels reads the input channels of the groups it covers, one contiguous range; the
+//     filter of that range is packed with zeros where output and input channel belong to different groups.  32 groups of
+//     4 x 4 channels keep an eighth of the matrix pipe's work, which is idle otherwise.
+//
+// A wave owns TM x 32 output channels x TN x 32 pixels of a phase and feeds the MFMAs straight from memory in fragment
+// layout, without LDS for the operands and without barriers: filter fragments are packed as 1 KB runs, an activation
+// fragment is one 16-byte load per lane at the position that the table entry of its (tap, 16 channels) names; a position
+// outside the image reads zeros through the buffer descriptor.  The table of a phase (two entries per 32-byte K slice,
+// one for each half of the wave) sits in LDS.  D slices are in flight per wave.
+//
+// Bound: the trip to memory at the start (few slices per wave: 9 for 3x3 with 32 channels per block) and the vector L1 at
+// 32 bytes per pixel row.  One lane per output element with byte loads, which this replaces, is bound by its serial loads:
+// 4 x 128 x 45 x 53, transposed 4x4 stride 2 -> 90 x 106: 8290 us, here 16; 32 groups 3x3: 41 us, here 7.  (8 x 256 x 60 x 60
+// transposed: 97 us, 0.6 POP/s.)  Six or eight slices in flight are no faster.
+#include "conv_gather.hpp"
+
+#include <algorithm>
+#include <cstring>
+#include <numeric>
+#include <vector>
+
+#include "conv_epilogue.hpp"
+
+namespace tpuhip {
+
+namespace {
+
+struct GatherPhase {
+  int oh0, ow0;        // first output row / column
+  int qh, qw;          // rows and columns of the phase
+  int iy0, ix0;        // input row / column that tap (0, 0) of output (oh0, ow0) stands at
+  int slices;          // 32-byte K slices
+  int tab;             // first table entry
+  uint32_t w;          // byte offset of the phase's packed filter
+};
+
+}  // namespace
+
+struct GatherPlan {
+  tpuhip_conv_desc d;
+  int8_t *w = nullptr;          // packed filters, then the tables, then the phases
+  uint32_t w_bytes = 0;
+  const int2 *tab = nullptr;
+  const GatherPhase *phases = nullptr;
+  int n_phases = 0, max_entries = 0, max_pixels = 0;
+  int ph = 1, pw = 1, step_h = 1, step_w = 1;   // output rows / columns between two of a phase, input ones between them
+  int blocks = 0;               // 32-channel blocks
+  int tm = 1;                   // blocks per wave
+};
+
+namespace {
+
+constexpr int kMaxEntries = 2048;   // table entries of a phase (16 KB of LDS)
+
+struct GatherArgs {
+  const int8_t *x, *w;
+  int8_t *y;
+  const int2 *tab;
+  const GatherPhase *phases;
+  const int32_t *bias, *mult, *shift, *hpot;
+  uint32_t x_bytes, w_bytes;
+  int n, ih, iw, x_cs, oh, ow, y_cs, ocw;
+  int ph, pw, step_h, step_w;
+  int ocg, icg;      // channels per group; grouped layers only: the first channel a block reads is that of its first group
+  int lo, relu_first;
+};
+
+// one 16-byte chunk of requantised channels per lane and pixel
+template <bool FAST>
+__device__ __forceinline__ int32_t requant_one(int32_t v, int32_t mult, int32_t rshift, int32_t hpot) {
+  const int32_t x = srdhm(v, mult);
+  if (FAST) return (x + hpot + (x >> 31)) >> rshift;
+  const int32_t mask = (int32_t)((1u << rshift) - 1u);
+  return rdbp(x, rshift, mask, mask >> 1);
+}
+
+template <int TM, int TN, bool FAST>
+__global__ __launch_bounds__(256) void conv_gather_kernel(GatherArgs a) {
+  extern __shared__ int2 stab[];
+  constexpr int D = 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 31, half = lane >> 5;
+  const GatherPhase p = a.phases[blockIdx.z];
+  for (int i = threadIdx.x; i < 2 * p.slices; i += 256) stab[i] = a.tab[p.tab + i];
+  __syncthreads();
+  const int npix = a.n * p.qh * p.qw;
+  const int pix0 = ((int)blockIdx.x * 4 + wave) * (TN * 32);
+  if (pix0 >= npix) return;
+  const int blk0 = blockIdx.y * TM;
+
+  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
+  const int cbase = a.icg ? (blk0 * 32 / a.ocg * a.icg) & ~15 : 0;
+
+  int iy[TN], ix[TN], off[TN], out[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int q = min(pix0 + j * 32 + col, npix - 1);
+    const int qw = q % p.qw, t = q / p.qw;
+    const int qh = t % p.qh, n = t / p.qh;
+    iy[j] = qh * a.step_h + p.iy0;
+    ix[j] = qw * a.step_w + p.ix0;
+    off[j] = ((n * a.ih + iy[j]) * a.iw + ix[j]) * a.x_cs + cbase;
+    out[j] = (n * a.oh + p.oh0 + qh * a.ph) * a.ow + p.ow0 + qw * a.pw;
+  }
+  uint32_t woff[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+    woff[i] = p.w + (uint32_t)((blk0 + i) * p.slices) * 1024u + (uint32_t)lane * 16u;
+
+  v4i af[D][TM], bf[D][TN];
+  auto load = [&](int slot, int s) {
+    const bool in_k = s < p.slices;
+    const int2 e = stab[min(2 * s + half, max(2 * p.slices - 1, 0))];
+    const int dy = e.y >> 16, dx = (int)(short)(e.y & 0xffff);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) af[slot][i] = buffer_load16(wrsrc, in_k ? woff[i] + (uint32_t)s * 1024u : kOobOffset);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const bool ok = in_k & ((unsigned)(iy[j] + dy) < (unsigned)a.ih) & ((unsigned)(ix[j] + dx) < (unsigned)a.iw);
+      bf[slot][j] = buffer_load16(xrsrc, ok ? (uint32_t)(off[j] + e.x) : kOobOffset);
+    }
+  };
+  v16i acc[TM][TN];
+  const int oc0 = blk0 * 32 + half * 16 * TM;   // a lane's TM * 16 channels are consecutive
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const v4i b = *reinterpret_cast<const v4i *>(a.bias + oc0 + i * 16 + q * 4);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][q * 4 + e] = b[e];
+    }
+  for (int s0 = 0; s0 < p.slices; s0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      // slices past the end are zeros in both operands
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[d][i], bf[d][j], acc[i][j], 0, 0, 0);
+      load(d, s0 + D + d);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int oc = oc0 + i * 16;
+    if (oc >= a.ocw) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      v4i o;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4i m = *reinterpret_cast<const v4i *>(a.mult + oc + q * 4);
+        const v4i r = *reinterpret_cast<const v4i *>(a.shift + oc + q * 4);
+        const v4i h = *reinterpret_cast<const v4i *>(a.hpot + oc + q * 4);
+        int32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          int32_t s = acc[i][j][q * 4 + e];
+          if (a.relu_first) s = max(s, 0);
+          v[e] = requant_one<FAST>(s, m[e], r[e], h[e]);
+        }
+        o[q] = (int)pack_sat4(v[0], v[1], v[2], v[3], a.lo);
+      }
+      if (pix0 + j * 32 + col < npix) *reinterpret_cast<v4i *>(a.y + (int64_t)out[j] * a.y_cs + oc) = o;
+    }
+  }
+}
+
+int floor_div(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
+
+}  // namespace
+
+int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *filter, GatherPlan **out) {
+  *out = nullptr;
+  const int icg = d.ic / d.g, ocg = d.oc / d.g;
+  const int sh = d.ins_h + 1, sw = d.ins_w + 1;
+  const int ph = sh / std::gcd(sh, d.sh), pw = sw / std::gcd(sw, d.sw);
+  // without groups all blocks read the same input channels: two of them per wave halve the activation loads
+  const int tm = d.g == 1 && d.oc > 32 ? 2 : 1;
+  const int blocks = round_up(d.oc, 32 * tm) / 32;
+  // 16-channel groups that a block reads: from the first channel of its first group, down to a multiple of 16
+  int n16 = 0;
+  for (int b = 0; b < blocks; ++b) {
+    if (b * 32 >= d.oc) break;
+    const int first = (b * 32 / ocg * icg) & ~15;
+    const int last = (std::min(b * 32 + 31, d.oc - 1) / ocg + 1) * icg;
+    n16 = std::max(n16, (last - first + 15) / 16);
+  }
+  // where it does not apply: a table entry holds its tap as two 16-bit distances, a phase's table fits its share of LDS,
+  // and every packed filter byte is addressed with 32 bits
+  if (d.x_cs % 16 || ph * pw > 256 || (int64_t)d.kh * d.dh >= 30000 || (int64_t)d.kw * d.dw >= 30000 || d.ih >= 30000 ||
+      d.iw >= 30000 || (int64_t)d.kh * d.kw * n16 + 2 > kMaxEntries ||
+      (int64_t)blocks * ((int64_t)d.kh * d.kw * n16 + 2 * ph * pw) * 512 >= (1ll << 30))
+    return TPUHIP_OK;
+
+  std::vector<GatherPhase> phases;
+  std::vector<int2> tab;
+  std::vector<int8_t> w;
+  int max_entries = 0, max_pixels = 0;
+  struct Tap { int kh, kw, dy, dx; };
+  for (int a = 0; a < std::min(ph, d.oh); ++a)
+    for (int b = 0; b < std::min(pw, d.ow); ++b) {
+      GatherPhase p{};
+      p.oh0 = a;
+      p.ow0 = b;
+      p.qh = (d.oh - a + ph - 1) / ph;
+      p.qw = (d.ow - b + pw - 1) / pw;
+      // position of tap (kh, kw) of the phase's first output, in the input with its zeros: divisible or no tap
+      const int y0 = a * d.sh - d.pt, x0 = b * d.sw - d.pl;
+      p.iy0 = floor_div(y0, sh);
+      p.ix0 = floor_div(x0, sw);
+      std::vector<Tap> taps;
+      for (int kh = 0; kh < d.kh; ++kh)
+        for (int kw = 0; kw < d.kw; ++kw) {
+          const int y = y0 + kh * d.dh, x = x0 + kw * d.dw;
+          if (floor_div(y, sh) * sh != y || floor_div(x, sw) * sw != x) continue;
+          taps.push_back({kh, kw, floor_div(y, sh) - p.iy0, floor_div(x, sw) - p.ix0});
+        }
+      const int entries = (int)taps.size() * n16;
+      p.slices = (entries + 1) / 2;
+      p.tab = (int)tab.size();
+      p.w = (uint32_t)w.size();
+      for (int e = 0; e < 2 * p.slices; ++e) {
+        const Tap t = e < entries ? taps[e / n16] : Tap{0, 0, 0, 0};
+        int2 v;
+        v.x = (int)(((int64_t)t.dy * d.iw + t.dx) * d.x_cs) + (e < entries ? e % n16 : 0) * 16;
+        v.y = (int)(((uint32_t)t.dy << 16) | ((uint32_t)t.dx & 0xffffu));
+        tab.push_back(v);
+      }
+      w.resize(w.size() + (size_t)blocks * p.slices * 1024, 0);
+      for (int blk = 0; blk < blocks; ++blk) {
+        const int c_first = d.g == 1 ? 0 : (blk * 32 / ocg * icg) & ~15;
+        for (int row = 0; row < 32; ++row) {
+          const int oc = blk / tm * tm * 32 + mfma_row_to_oc(blk % tm * 32 + row, tm);
+          if (oc >= d.oc) continue;
+          const int g = oc / ocg;
+          for (int e = 0; e < entries; ++e) {
+            const Tap &t = taps[e / n16];
+            int8_t *to = w.data() + p.w + ((size_t)(blk * p.slices + e / 2) * 64 + row + 32 * (e & 1)) * 16;
+            for (int k = 0; k < 16; ++k) {
+              const int c = c_first + (e % n16) * 16 + k - g * icg;   // channel within the group
+              if (c >= 0 && c < icg) to[k] = filter[(((size_t)oc * icg + c) * d.kh + t.kh) * d.kw + t.kw];
+            }
+          }
+        }
+      }
+      max_entries = std::max(max_entries, 2 * p.slices);
+      max_pixels = std::max(max_pixels, d.n * p.qh * p.qw);
+      phases.push_back(p);
+    }
+  auto *plan = new GatherPlan;
+  plan->d = d;
+  plan->n_phases = (int)phases.size();
+  plan->max_entries = max_entries;
+  plan->max_pixels = max_pixels;
+  plan->ph = ph;
+  plan->pw = pw;
+  plan->step_h = ph * d.sh / sh;
+  plan->step_w = pw * d.sw / sw;
+  plan->blocks = blocks;
+  plan->tm = tm;
+  w.resize(std::max<size_t>(w.size(), 16));
+  plan->w_bytes = (uint32_t)w.size();
+  const size_t tab_at = w.size(), phase_at = tab_at + std::max<size_t>(tab.size(), 1) * sizeof(int2);
+  std::vector<int8_t> image(phase_at + phases.size() * sizeof(GatherPhase), 0);
+  memcpy(image.data(), w.data(), w.size());
+  memcpy(image.data() + tab_at, tab.data(), tab.size() * sizeof(int2));
+  memcpy(image.data() + phase_at, phases.data(), phases.size() * sizeof(GatherPhase));
+  int rc = tpuhip_malloc(ctx, image.size(), (void **)&plan->w);
+  if (!rc) rc = tpuhip_upload(ctx, plan->w, image.data(), image.size());
+  if (rc) {
+    gather_destroy(ctx, plan);
+    return rc;
+  }
+  plan->tab = (const int2 *)(plan->w + tab_at);
+  plan->phases = (const GatherPhase *)(plan->w + phase_at);
+  *out = plan;
+  return TPUHIP_OK;
+}
+
+void gather_destroy(tpuhip_ctx *ctx, GatherPlan *plan) {
+  if (!plan) return;
+  if (plan->w) (void)tpuhip_free(ctx, plan->w);
+  delete plan;
+}
+
+int gather_run(tpuhip_ctx *ctx, const GatherPlan *plan, const void *x, void *y, const int32_t *bias, const int32_t *mult,
+               const int32_t *shift, const int32_t *hpot, bool fast) {
+  const tpuhip_conv_desc &d = plan->d;
+  GatherArgs a{};
+  a.x = (const int8_t *)x;
+  a.y = (int8_t *)y;
+  a.w = plan->w;
+  a.tab = plan->tab;
+  a.phases = plan->phases;
+  a.bias = bias;
+  a.mult = mult;
+  a.shift = shift;
+  a.hpot = hpot;
+  a.x_bytes = (uint32_t)((int64_t)d.n * d.ih * d.iw * d.x_cs);
+  a.w_bytes = plan->w_bytes;
+  a.n = d.n; a.ih = d.ih; a.iw = d.iw; a.x_cs = d.x_cs;
+  a.oh = d.oh; a.ow = d.ow; a.y_cs = d.y_cs; a.ocw = round_up(d.oc, 16);
+  a.ph = plan->ph; a.pw = plan->pw; a.step_h = plan->step_h; a.step_w = plan->step_w;
+  a.ocg = d.oc / d.g;
+  a.icg = d.g > 1 ? d.ic / d.g : 0;
+  a.lo = (d.do_relu && !d.relu_first) ? 0 : -128;
+  a.relu_first = (d.do_relu && d.relu_first) ? 1 : 0;
+  // 64 pixels per wave where that still gives every SIMD two waves, else 32
+  const int groups = plan->blocks / plan->tm;
+  const int64_t waves = (int64_t)((plan->max_pixels + 63) / 64) * groups * plan->n_phases;
+  const bool wide = waves >= (int64_t)ctx->num_cu * 8;
+  const int per_wg = wide ? 256 : 128;
+  const dim3 grid((unsigned)((plan->max_pixels + per_wg - 1) / per_wg), (unsigned)groups, (unsigned)plan->n_phases), block(256);
+  const unsigned lds = (unsigned)std::max(plan->max_entries, 1) * sizeof(int2);
+  auto go = [&](auto kernel) {
+    if (ctx->prof_start)
+      hipExtLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
+    else
+      hipLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, a);
+  };
+  if (plan->tm == 2) {
+    if (wide) fast ? go(conv_gather_kernel<2, 2, true>) : go(conv_gather_kernel<2, 2, false>);
+    else fast ? go(conv_gather_kernel<2, 1, true>) : go(conv_gather_kernel<2, 1, false>);
+  } else {
+    if (wide) fast ? go(conv_gather_kernel<1, 2, true>) : go(conv_gather_kernel<1, 2, false>);
+    else fast ? go(conv_gather_kernel<1, 1, true>) : go(conv_gather_kernel<1, 1, false>);
+  }
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
+}
+
+}  // namespace tpuhip
