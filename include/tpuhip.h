@@ -50,9 +50,11 @@ int tpuhip_ctx_create_on_stream(int device, void *hip_stream, tpuhip_ctx **out);
 int tpuhip_ctx_destroy(tpuhip_ctx *ctx);
 void *tpuhip_ctx_stream(tpuhip_ctx *ctx);
 /* When enabled (the default; TPUHIP_AUTOTUNE=0 in the environment disables it) a
- * dense conv times its tile variants on first use and keeps the fastest.  Every
- * variant produces the same bytes.  The first use of a layer is then not
- * capturable into a HIP graph. */
+ * dense conv times its tile variants on first use and keeps the fastest, unless a layer of
+ * the same shape has been timed before in this process, whose choice it takes.  Every
+ * variant produces the same bytes.  Inside a HIP graph capture nothing is timed: capture
+ * after the first use of a layer (tpuhip_module_interpret_files, which runs a model once,
+ * times nothing either). */
 int tpuhip_ctx_set_autotune(tpuhip_ctx *ctx, int enable);
 const char *tpuhip_last_error(void);
 const char *tpuhip_version(void);

@@ -628,6 +628,7 @@ public:
   // the reference's updateWeightMap reads every tpu.load_weight from the npz
   // (MlirModuleInterpreter.cpp:352-369); here the caller hands the arrays over
   void updateWeightMap(const std::string &name, const float *data, size_t count);
+  void updateWeightMap(const std::string &name, std::vector<float> &&data);
   std::vector<std::string> &outputDetails() { return output_details; }
   void dump(std::string &name);
   std::vector<std::string> getAllTensorName();

@@ -49,11 +49,25 @@ public:
   int keep();
   const std::string &path() const { return filename; }
 
+  // a stored float32 array of exactly count elements, in place in the file's image (any alignment); nullptr otherwise
+  const void *floats(const std::string &name, size_t count) const;
+
 private:
+  // an array of the file: its values stay where they lie in the file's image until somebody asks for them as an NpyArray
+  // (`bytes` is then filled; added arrays have them from the start)
+  struct Member {
+    NpyArray array;
+    const uint8_t *data = nullptr;
+    size_t size = 0;
+    const uint8_t *values() const;
+  };
   void load();
+  static void own(Member &m);
   std::string filename;
   bool readOnly;
-  std::map<std::string, NpyArray> map;
+  mutable std::map<std::string, Member> map;
+  std::shared_ptr<const uint8_t> image;                        // the file's bytes
+  std::vector<std::shared_ptr<std::vector<uint8_t>>> inflated; // members that were compressed
   int changes = 0;
 };
 

@@ -29,8 +29,12 @@ struct tpuhip_ctx {
   // for the dense form of a tensor that takes more than one piece, events behind the pieces; made on first use
   void *stage = nullptr, *landing = nullptr;
   size_t stage_bytes = 0, landing_bytes = 0;
+  size_t stage_used = 0;     // bytes of the pinned buffer that stage_upload has handed out since it was last free
   bool stage_busy = false;   // kernels that read or write the pinned buffer may still be in flight
   std::vector<hipEvent_t> stage_events;
+  // a module is being loaded: packed weights need not be on the device when a prepack call returns, the loader waits once
+  bool loading = false;
+  bool single_pass = false;   // what is issued now runs once: no layer's tile variants are timed for it
 };
 
 // conv.hip: looks up this device's copy of the library's static scratch array (the one the
@@ -41,8 +45,22 @@ extern "C" void tpuhip_static_scratch_forget(const tpuhip_ctx *ctx);
 
 namespace tpuhip {
 
+// sets a flag for as long as it lives
+struct FlagScope {
+  explicit FlagScope(bool &f) : flag(f), before(f) { flag = true; }
+  ~FlagScope() { flag = before; }
+  FlagScope(const FlagScope &) = delete;
+  bool &flag;
+  bool before;
+};
+
 // host/host_io.cpp: frees a context's staging buffers
 void host_io_release(tpuhip_ctx *ctx);
+// host/host_io.cpp: tpuhip_upload without the wait -- src may be reused on return, the bytes are there for what is issued to
+// the context's stream afterwards
+int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes);
+// waits for what a prepack call has issued, unless a module is being loaded: packed weights may be used from any context
+int prepack_done(tpuhip_ctx *ctx);
 
 int set_error(int status, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
@@ -55,8 +56,10 @@ struct tpuhip_conv_weights {
   bool fc_only = false;
   // the direct path's layers where the caller left the choice: their form on the matrix cores (NULL: not covered)
   GatherPlan *gather = nullptr;
-  std::vector<int8_t> host_filter;  // OIHW copy, kept while the layer can still be repacked
+  int8_t *raw = nullptr;     // the filter as OIHW on the device, kept while the layer can still be repacked
   int8_t *w = nullptr;   // packed filter
+  size_t w_room = 0;     // bytes behind w
+  int8_t *params = nullptr;   // one allocation behind bias, qp, qplanes and qc64
   int32_t *bias = nullptr;
   QParam *qp = nullptr;
   int32_t *qplanes = nullptr;   // mult | rshift | hpot planes of nparam entries each
@@ -3705,7 +3708,7 @@ int persist_wgs_per_cu(const tpuhip_conv_weights *w) {
   return c;
 }
 
-// Default tile when the variants are not timed on first use: the persistent tiles,
+// Default tile until the variants have been timed: the persistent tiles,
 // narrow in output channels for thin layers, wide in pixels when there are enough of
 // them to give every CU several tiles.
 int pick_tile(const tpuhip_conv_desc &d, int k16, int num_cu) {
@@ -3744,69 +3747,100 @@ int check_desc(const tpuhip_conv_desc &d) {
   return TPUHIP_OK;
 }
 
+// Packs an OIHW filter for a tile variant: a thread makes one 16-byte K group of one row in the order its kernel reads
+// (2.4 MB in 10 us; the host loop this replaces took 4 ms, once per timed variant).
+struct PackArgs {
+  const int8_t *raw;
+  v4i *out;
+  int oc, ic, taps, c16, kp, bm, bk, tm, reg;
+  int smallc;
+  int64_t total;   // 16-byte groups
+};
+__global__ __launch_bounds__(256) void pack_filter_kernel(PackArgs a) {
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (q >= a.total) return;
+  const int kg = a.kp >> 4;          // 16-byte groups per row
+  int row, kc;
+  if (a.reg == 6) {
+    // [output-channel tile][K step][row][BK bytes]
+    const int per_step = a.bm * (a.bk >> 4), per_tile = a.bm * kg;
+    const int tile = (int)(q / per_tile), r1 = (int)(q - (int64_t)tile * per_tile);
+    const int step = r1 / per_step, r2 = r1 - step * per_step, b16 = a.bk >> 4;
+    row = tile * a.bm + r2 / b16;
+    kc = step * b16 + r2 % b16;
+  } else if (a.reg == 5) {
+    // the LDS image of every output-channel tile: [64-byte K chunk][row][4 x 16 bytes], the 16-byte position XORed
+    // with (row >> 2) & 3
+    const int per_tile = a.bm * kg;
+    const int tile = (int)(q / per_tile), r1 = (int)(q - (int64_t)tile * per_tile);
+    const int k64 = r1 / (a.bm * 4), r2 = r1 - k64 * a.bm * 4, r = r2 >> 2;
+    row = tile * a.bm + r;
+    kc = k64 * 4 + ((r2 & 3) ^ ((r >> 2) & 3));
+  } else if (a.reg == 0 || a.reg == 3 || a.reg == 4) {
+    row = (int)(q / kg);
+    kc = (int)(q - (int64_t)row * kg);
+  } else {
+    // fragment order: [row / 32][K step][kk][lane = (row & 31) + 32 * half]
+    const int lane = (int)(q & 63);
+    const int64_t f = q >> 6;
+    const int per_blk = kg / 2;      // fragments per 32 rows
+    const int blk = (int)(f / per_blk), s = (int)(f - (int64_t)blk * per_blk);
+    row = blk * 32 + (lane & 31);
+    kc = (s >> 1) * 4 + (s & 1) * 2 + (lane >> 5);
+  }
+  const int tile0 = row / a.bm * a.bm;
+  const int oc = tile0 + mfma_row_to_oc(row - tile0, a.tm);
+  uint32_t v[4] = {0, 0, 0, 0};
+  if (oc < a.oc) {
+    const int8_t *src = a.raw + (int64_t)oc * a.ic * a.taps;
+    const int tap0 = kc / a.c16, c0 = (kc - tap0 * a.c16) * 16;
+#pragma unroll
+    for (int b = 0; b < 16; ++b) {
+      const int tap = a.smallc ? kc * 4 + (b >> 2) : tap0, c = a.smallc ? b & 3 : c0 + b;
+      if (tap < a.taps && c < a.ic) v[b >> 2] |= (uint32_t)(uint8_t)src[(int64_t)c * a.taps + tap] << (8 * (b & 3));
+    }
+  }
+  a.out[q] = v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+}
+
 // (re)builds the device filter of an MFMA conv for tile variant `tile`
 int pack_mfma_weights(tpuhip_ctx *ctx, tpuhip_conv_weights *cw, int tile) {
   const tpuhip_conv_desc &d = cw->d;
   const TileCfg &t = kTiles[tile];
   const int tm = t.bm / t.wm / 32;
-  const int icp = round_up(d.ic, 16);
   const int ocp = round_up(d.oc, t.bm);
   cw->smallc = d.ic <= 4 && (t.reg == 0 || t.reg == 3);
-  cw->c16 = icp / 16;
+  cw->c16 = round_up(d.ic, 16) / 16;
   cw->k16 = cw->smallc ? (d.kh * d.kw * 4 + 15) / 16 : d.kh * d.kw * cw->c16;
   cw->kp = round_up(cw->k16 * 16, tile_bk(t));
   if (t.reg == 5 && cw->kp != t.bk) return set_error(TPUHIP_ERR_INVALID, "conv: tile %s holds %d input channels", t.name, t.bk);
-  std::vector<int8_t> packed((size_t)ocp * cw->kp, 0);
-  const int8_t *filter = cw->host_filter.data();
-  std::vector<int8_t> rowbuf((size_t)cw->kp);
-  const int nsteps = cw->kp / 64;
-  for (int row = 0; row < ocp; ++row) {
-    const int tile0 = row / t.bm * t.bm;
-    const int oc = tile0 + mfma_row_to_oc(row - tile0, tm);
-    if (oc >= d.oc) continue;
-    std::fill(rowbuf.begin(), rowbuf.end(), 0);
-    const int8_t *src = filter + (size_t)oc * d.ic * d.kh * d.kw;
-    const int kstride = cw->smallc ? 4 : icp;   // channels per tap in the K order
-    for (int c = 0; c < d.ic; ++c)
-      for (int k = 0; k < d.kh * d.kw; ++k)
-        rowbuf[(size_t)k * kstride + c] = src[(size_t)c * d.kh * d.kw + k];
-    if (t.reg == 0 || t.reg == 3 || t.reg == 4) {
-      memcpy(packed.data() + (size_t)row * cw->kp, rowbuf.data(), rowbuf.size());
-    } else if (t.reg == 6) {
-      // [output-channel tile][K step][row][BK bytes]: every step's tile is contiguous
-      const int r = row - tile0;
-      int8_t *img = packed.data() + (size_t)(tile0 / t.bm) * t.bm * cw->kp;
-      for (int st = 0; st < cw->kp / t.bk; ++st)
-        memcpy(img + ((size_t)st * t.bm + r) * t.bk, rowbuf.data() + (size_t)st * t.bk, t.bk);
-    } else if (t.reg == 5) {
-      // the LDS image of every output-channel tile: [64-byte K chunk][row][4 x 16 bytes], the
-      // 16-byte position XORed with (row >> 2) & 3
-      const int r = row - tile0;
-      int8_t *img = packed.data() + (size_t)(tile0 / t.bm) * t.bm * cw->kp;
-      for (int kc = 0; kc < cw->kp / 64; ++kc)
-        for (int c4 = 0; c4 < 4; ++c4)
-          memcpy(img + ((size_t)(kc * t.bm + r) * 4 + (c4 ^ ((r >> 2) & 3))) * 16,
-                 rowbuf.data() + (size_t)kc * 64 + c4 * 16, 16);
-    } else {
-      // fragment order: [row / 32][K step][kk][lane = (row & 31) + 32 * half][16 bytes]
-      const int blk = row / 32, r = row % 32;
-      for (int step = 0; step < nsteps; ++step)
-        for (int kk = 0; kk < 2; ++kk)
-          for (int half = 0; half < 2; ++half)
-            memcpy(packed.data() + ((size_t)(blk * nsteps + step) * 2 + kk) * 1024 +
-                       (size_t)(r + 32 * half) * 16,
-                   rowbuf.data() + (size_t)step * 64 + (kk * 2 + half) * 16, 16);
-    }
-  }
-  if (cw->w) {
+  const size_t bytes = (size_t)ocp * cw->kp;
+  if (bytes > cw->w_room) {
     if (int rc = tpuhip_free(ctx, cw->w)) return rc;
     cw->w = nullptr;
+    cw->w_room = 0;
+    if (int rc = tpuhip_malloc(ctx, bytes, (void **)&cw->w)) return rc;
+    cw->w_room = bytes;
   }
-  if (int rc = tpuhip_malloc(ctx, packed.size(), (void **)&cw->w)) return rc;
-  if (int rc = tpuhip_upload(ctx, cw->w, packed.data(), packed.size())) return rc;
+  PackArgs a{};
+  a.raw = cw->raw;
+  a.out = (v4i *)cw->w;
+  a.oc = d.oc; a.ic = d.ic; a.taps = d.kh * d.kw;
+  a.c16 = cw->c16; a.kp = cw->kp; a.bm = t.bm; a.bk = t.bk; a.tm = tm; a.reg = t.reg;
+  a.smallc = cw->smallc ? 1 : 0;
+  a.total = (int64_t)bytes / 16;
+  hipLaunchKernelGGL(pack_filter_kernel, dim3((unsigned)ceil_div64(a.total, 256)), dim3(256), 0, ctx->stream, a);
+  TPUHIP_CHECK_HIP(hipGetLastError());
   cw->tile = tile;
   cw->ocp = ocp;
   return TPUHIP_OK;
+}
+
+// the layer keeps its tile: the unpacked filter goes
+void settle_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *cw) {
+  cw->tuned = true;
+  (void)tpuhip_free(ctx, cw->raw);
+  cw->raw = nullptr;
 }
 
 // the fused table lives in the LDS of the LDS kernels
@@ -4066,45 +4100,90 @@ void apply_fusion(ConvArgs *a, const void *y, const PostOps &p) {
   a->y2 = (int8_t *)p.y2;
 }
 
+// Tiles that timing has chosen, by everything the choice can depend on: a layer of the same shape -- a second module, the
+// same model loaded again -- takes its tile from here.  Shared by all contexts, bounded (beyond it, it starts anew).
+using TileKey = std::array<int, 32>;
+std::mutex g_tiles_mu;
+std::map<TileKey, int> g_tiles;
+constexpr size_t kTilesKept = 8192;
+
+TileKey tile_key(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *y, const PostOps &p) {
+  const tpuhip_conv_desc &d = w->d;
+  const tpuhip_fused_add *f = p.has_add() ? p.f : nullptr;
+  return TileKey{ctx->num_cu, d.n, d.ic, d.ih, d.iw, d.oc, d.oh, d.ow, d.kh, d.kw, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw,
+                 d.x_cs, d.y_cs, d.do_relu, d.relu_first, w->fast, w->split_oc, w->y2_cs, w->relu2, y != nullptr,
+                 p.lut != nullptr, p.lut_out != nullptr, f != nullptr,
+                 f && std::abs(f->m_src) <= 127 && std::abs(f->m_conv) <= 127 && f->rshift <= 8, f && f->do_relu,
+                 d.pb, d.pr};
+}
+
+bool tile_usable(const tpuhip_conv_weights *w, int t, const PostOps &post) {
+  if (!tile_is_candidate(w->d, t)) return false;
+  if (post.lut && !tile_has_lds_epilogue(t)) return false;
+  if (w->split_oc && kTiles[t].reg == 4) return false;   // the patch kernel writes one result
+  if (kTiles[t].reg == 5 && (!w->fast || w->split_oc % kTiles[t].bm)) return false;
+  return !((kTiles[t].reg == 6 || kTiles[t].reg == 7) && (!w->fast || w->split_oc));
+}
+
+// Keeps the stream busy for 25 to 50 us, so that the launches behind it are queued before the first of them starts:
+// most layers of one image run shorter than the host needs to launch them, and would otherwise all measure the host.
+// One wave, a fixed number of sleeps.
+__global__ __launch_bounds__(64) void delay_kernel(int rounds) {
+  for (int i = 0; i < rounds; ++i) __builtin_amdgcn_s_sleep(100);   // 6400 clocks
+}
+
 // The fused add (if any) is part of what is timed: it shifts the balance between
 // the tile shapes.  Every launch recomputes the same bytes, so repeating it is safe
 // as long as the sum is not written over its own input.
+// Every candidate runs five times; those within a fifth of the fastest then run twice fifteen times, and the smaller of
+// the two decides.
 int autotune_mfma(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *y,
                   const PostOps &post) {
   hipEvent_t e0, e1;
   TPUHIP_CHECK_HIP(hipEventCreate(&e0));
   TPUHIP_CHECK_HIP(hipEventCreate(&e1));
-  float best_ms = 1e30f;
-  int best = -1;
+  float ms_of[kMaxTiles];
   int rc = TPUHIP_OK;
-  for (int t = 0; t < kNumTiles && !rc; ++t) {
-    if (!tile_is_candidate(w->d, t)) continue;
-    if (post.lut && !tile_has_lds_epilogue(t)) continue;
-    if (w->split_oc && kTiles[t].reg == 4) continue;   // the patch kernel writes one result
-    if (kTiles[t].reg == 5 && (!w->fast || w->split_oc % kTiles[t].bm)) continue;
-    if ((kTiles[t].reg == 6 || kTiles[t].reg == 7) && (!w->fast || w->split_oc)) continue;
+  // mean time of `runs` launches of tile t; a negative value: it cannot be launched
+  auto time_tile = [&](int t, int runs) -> float {
     rc = pack_mfma_weights(ctx, w, t);
-    if (rc) break;
+    if (rc) return -1;
     ConvArgs a;
     fill_args(ctx, w, x, y, &a);
     apply_fusion(&a, y, post);
-    for (int i = 0; i < 2; ++i) launch_conv_mfma(ctx, w, a);
+    hipLaunchKernelGGL(delay_kernel, dim3(1), dim3(64), 0, ctx->stream, 4 + runs);
+    launch_conv_mfma(ctx, w, a);
     hipError_t er = hipEventRecord(e0, ctx->stream);
-    for (int i = 0; i < 5; ++i) launch_conv_mfma(ctx, w, a);
+    for (int i = 0; i < runs; ++i) launch_conv_mfma(ctx, w, a);
     if (er == hipSuccess) er = hipEventRecord(e1, ctx->stream);
     hipError_t es = hipEventSynchronize(e1);
     const hipError_t el = hipGetLastError();
     if (es == hipSuccess) es = er;
-    if (es != hipSuccess || el != hipSuccess) {
-      // a variant that cannot be launched is skipped; the layer fails only if none can
-      set_error(TPUHIP_ERR_HIP, "conv autotune: tile %s failed: %s", kTiles[t].name,
-                hipGetErrorString(es != hipSuccess ? es : el));
-      if (getenv("TPUHIP_DEBUG")) fprintf(stderr, "%s\n", tpuhip_last_error());
-      continue;
-    }
     float ms = 0;
-    if (hipEventElapsedTime(&ms, e0, e1) != hipSuccess) continue;
-    if (ms < best_ms) {
+    if (es == hipSuccess && el == hipSuccess) {
+      es = hipEventElapsedTime(&ms, e0, e1);
+      if (es == hipSuccess) return ms / runs;
+    }
+    // a variant that cannot be launched is skipped; the layer fails only if none can
+    set_error(TPUHIP_ERR_HIP, "conv autotune: tile %s failed: %s", kTiles[t].name,
+              hipGetErrorString(es != hipSuccess ? es : el));
+    if (getenv("TPUHIP_DEBUG")) fprintf(stderr, "%s\n", tpuhip_last_error());
+    return -1;
+  };
+  float least = 1e30f;
+  for (int t = 0; t < kNumTiles && !rc; ++t) {
+    ms_of[t] = tile_usable(w, t, post) ? time_tile(t, 5) : -1;
+    if (ms_of[t] >= 0) least = std::min(least, ms_of[t]);
+  }
+  float best_ms = 1e30f;
+  int best = -1;
+  for (int t = 0; t < kNumTiles && !rc; ++t) {
+    if (ms_of[t] < 0 || ms_of[t] > 1.2f * least) continue;
+    const float a = time_tile(t, 15);
+    if (rc) break;
+    const float b = time_tile(t, 15);
+    const float ms = b >= 0 && (a < 0 || b < a) ? b : a;
+    if (ms >= 0 && ms < best_ms) {
       best_ms = ms;
       best = t;
     }
@@ -4114,10 +4193,47 @@ int autotune_mfma(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *
   if (rc) return rc;
   if (best < 0) return TPUHIP_ERR_HIP;   // the last launch error is still the message
   if (best != w->tile) rc = pack_mfma_weights(ctx, w, best);
-  w->tuned = true;
-  w->host_filter.clear();
-  w->host_filter.shrink_to_fit();
+  if (!rc) settle_tile(ctx, w);
   return rc;
+}
+
+// The tile of a layer that may still choose: one that timing has found before for the same shape, else the fastest, by
+// timing.  The rule's tile stays, for this use, inside a capture, which cannot wait, and where the context says that the
+// model runs once: timing 35 layers takes 100 ms, and a single pass of them is 0.3 ms on either choice.
+int choose_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *y, const PostOps &post) {
+  const TileKey key = tile_key(ctx, w, y, post);
+  int known = -1;
+  {
+    std::lock_guard<std::mutex> l(g_tiles_mu);
+    auto it = g_tiles.find(key);
+    if (it != g_tiles.end()) known = it->second;
+  }
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  (void)hipStreamIsCapturing(ctx->stream, &capturing);
+  if (capturing != hipStreamCaptureStatusNone) return TPUHIP_OK;
+  if (known >= 0) {
+    if (known != w->tile)
+      if (int rc = pack_mfma_weights(ctx, w, known)) return rc;
+    settle_tile(ctx, w);
+    return TPUHIP_OK;
+  }
+  if (ctx->single_pass) return TPUHIP_OK;
+  // the fused work is timed with it unless the sum would overwrite its own operand
+  PostOps tp = post;
+  if (tp.has_add() && tp.add_out == tp.add_src) tp.f = nullptr;
+  void *ty = y;
+  if (!ty && !tp.has_add() && !(tp.lut && tp.lut_out)) {
+    // tuning writes the plain conv result somewhere: borrow a buffer
+    const size_t bytes = (size_t)w->d.n * w->d.oh * w->d.ow * w->d.y_cs;
+    if (int rc = tpuhip_malloc(ctx, bytes, &ty)) return rc;
+  }
+  const int rc = autotune_mfma(ctx, w, x, ty, tp);
+  if (ty != y) tpuhip_free(ctx, ty);
+  if (rc) return rc;
+  std::lock_guard<std::mutex> l(g_tiles_mu);
+  if (g_tiles.size() >= kTilesKept) g_tiles.clear();
+  g_tiles[key] = w->tile;
+  return TPUHIP_OK;
 }
 
 }  // namespace
@@ -4183,17 +4299,16 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   if (algo == ALGO_MFMA) {
     cw->c16 = round_up(d.ic, 16) / 16;
     cw->k16 = d.kh * d.kw * cw->c16;   // refined per tile in pack_mfma_weights
-    cw->host_filter.assign(filter, filter + (size_t)d.oc * per_oc);
     const int tile = forced_tile >= 0 ? forced_tile : pick_tile(d, cw->k16, ctx->num_cu);
-    if (int rc = pack_mfma_weights(ctx, cw, tile)) {
+    int rc = tpuhip_malloc(ctx, (size_t)d.oc * per_oc, (void **)&cw->raw);
+    if (!rc) rc = stage_upload(ctx, cw->raw, filter, (size_t)d.oc * per_oc);
+    if (!rc) rc = pack_mfma_weights(ctx, cw, tile);
+    if (rc) {
       tpuhip_conv2d_weights_destroy(ctx, cw);
       return rc;
     }
-    cw->tuned = forced_tile >= 0 || !ctx->autotune;
-    if (cw->tuned) {
-      cw->host_filter.clear();
-      cw->host_filter.shrink_to_fit();
-    }
+    cw->tuned = false;
+    if (forced_tile >= 0 || !ctx->autotune) settle_tile(ctx, cw);
   } else if (algo == ALGO_DEPTHWISE) {
     // diagonal MFMA A fragments: [32-channel block][tap][lane][16 bytes]; lane l holds row
     // l & 31 (channel mfma_row_to_oc(row) of the block), K bytes 16*(l >> 5) .. +15
@@ -4282,40 +4397,38 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   int rc = TPUHIP_OK;
   if (algo != ALGO_MFMA && !cw->gather) {
     rc = tpuhip_malloc(ctx, packed.size(), (void **)&cw->w);
-    if (!rc) rc = tpuhip_upload(ctx, cw->w, packed.data(), packed.size());
+    if (!rc) rc = stage_upload(ctx, cw->w, packed.data(), packed.size());
   }
-  if (!rc) rc = tpuhip_malloc(ctx, b32.size() * sizeof(int32_t), (void **)&cw->bias);
-  if (!rc) rc = tpuhip_malloc(ctx, qp.size() * sizeof(QParam), (void **)&cw->qp);
-  if (!rc) rc = tpuhip_upload(ctx, cw->bias, b32.data(), b32.size() * sizeof(int32_t));
-  if (!rc) rc = tpuhip_upload(ctx, cw->qp, qp.data(), qp.size() * sizeof(QParam));
-  if (!rc && (algo != ALGO_DIRECT || cw->gather)) {
-    std::vector<int32_t> planes(3 * nparam);
-    for (size_t i = 0; i < nparam; ++i) {
-      planes[i] = qp[i].mult;
-      planes[nparam + i] = qp[i].rshift;
-      planes[2 * nparam + i] = qp[i].hpot;
-    }
-    cw->nparam = (int)nparam;
-    rc = tpuhip_malloc(ctx, planes.size() * sizeof(int32_t), (void **)&cw->qplanes);
-    if (!rc) rc = tpuhip_upload(ctx, cw->qplanes, planes.data(), planes.size() * sizeof(int32_t));
-    // (acc + bias) * mult + 2^30 == acc * mult + c: the addend of the requantisation's 64-bit
-    // multiply-add, as a plane of low and a plane of high words
-    std::vector<int32_t> c64(4 * nparam);
-    for (size_t i = 0; i < nparam; ++i) {
-      const int64_t c = (int64_t)b32[i] * (int64_t)qp[i].mult + (1ll << 30);
-      const int64_t cr = c + ((int64_t)qp[i].hpot << 31);
-      c64[2 * i] = (int32_t)(uint32_t)(c & 0xffffffffll);
-      c64[2 * i + 1] = (int32_t)(c >> 32);
-      c64[2 * nparam + 2 * i] = (int32_t)(uint32_t)(cr & 0xffffffffll);
-      c64[2 * nparam + 2 * i + 1] = (int32_t)(cr >> 32);
-    }
-    if (!rc) rc = tpuhip_malloc(ctx, c64.size() * sizeof(int32_t), (void **)&cw->qc64);
-    if (!rc) rc = tpuhip_upload(ctx, cw->qc64, c64.data(), c64.size() * sizeof(int32_t));
+  // one allocation and one upload: biases, records, the planes of the records' fields, and per channel the addend of the
+  // requantisation's 64-bit multiply-add, (acc + bias) * mult + 2^30 == acc * mult + c, as (low, high) words
+  cw->nparam = (int)nparam;
+  const size_t at_qp = nparam * 4, at_planes = at_qp + nparam * sizeof(QParam), at_c64 = at_planes + 3 * nparam * 4;
+  std::vector<int8_t> image(at_c64 + 4 * nparam * 4);
+  memcpy(image.data(), b32.data(), nparam * 4);
+  memcpy(image.data() + at_qp, qp.data(), nparam * sizeof(QParam));
+  int32_t *planes = (int32_t *)(image.data() + at_planes), *c64 = (int32_t *)(image.data() + at_c64);
+  for (size_t i = 0; i < nparam; ++i) {
+    planes[i] = qp[i].mult;
+    planes[nparam + i] = qp[i].rshift;
+    planes[2 * nparam + i] = qp[i].hpot;
+    const int64_t c = (int64_t)b32[i] * (int64_t)qp[i].mult + (1ll << 30);
+    const int64_t cr = c + ((int64_t)qp[i].hpot << 31);
+    c64[2 * i] = (int32_t)(uint32_t)(c & 0xffffffffll);
+    c64[2 * i + 1] = (int32_t)(c >> 32);
+    c64[2 * nparam + 2 * i] = (int32_t)(uint32_t)(cr & 0xffffffffll);
+    c64[2 * nparam + 2 * i + 1] = (int32_t)(cr >> 32);
   }
+  if (!rc) rc = tpuhip_malloc(ctx, image.size(), (void **)&cw->params);
+  if (!rc) rc = stage_upload(ctx, cw->params, image.data(), image.size());
+  if (!rc) rc = prepack_done(ctx);
   if (rc) {
     tpuhip_conv2d_weights_destroy(ctx, cw);
     return rc;
   }
+  cw->bias = (int32_t *)cw->params;
+  cw->qp = (QParam *)(cw->params + at_qp);
+  cw->qplanes = (int32_t *)(cw->params + at_planes);
+  cw->qc64 = (int32_t *)(cw->params + at_c64);
   *out = cw;
   return TPUHIP_OK;
 }
@@ -4325,12 +4438,10 @@ int tpuhip_conv2d_weights_destroy(tpuhip_ctx *ctx, tpuhip_conv_weights *w) {
   TPUHIP_REQUIRE(ctx, "tpuhip_conv2d_weights_destroy: NULL context");
   gather_destroy(ctx, w->gather);
   int rc = tpuhip_free(ctx, w->w);
-  int rc2 = tpuhip_free(ctx, w->bias);
-  int rc3 = tpuhip_free(ctx, w->qp);
-  int rc4 = tpuhip_free(ctx, w->qplanes);
-  int rc5 = tpuhip_free(ctx, w->qc64);
+  int rc2 = tpuhip_free(ctx, w->raw);
+  int rc3 = tpuhip_free(ctx, w->params);
   delete w;
-  return rc ? rc : rc2 ? rc2 : rc3 ? rc3 : rc4 ? rc4 : rc5;
+  return rc ? rc : rc2 ? rc2 : rc3;
 }
 
 const char *tpuhip_conv2d_tile_name(int tile) {
@@ -4418,21 +4529,8 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
     TPUHIP_REQUIRE(!post.any() && y, "conv: a FullyConnected of more than 4096 input channels takes no fused work");
     return run_fc_one(ctx, w, x, y);
   }
-  if (w->algo == ALGO_MFMA && !w->tuned) {
-    // first use: pick the tile by measurement (not capturable into a HIP graph).  The
-    // fused work is timed with it unless the sum would overwrite its own operand.
-    PostOps tp = post;
-    if (tp.has_add() && tp.add_out == tp.add_src) tp.f = nullptr;
-    void *ty = y;
-    if (!ty && !tp.has_add() && !(tp.lut && tp.lut_out)) {
-      // tuning writes the plain conv result somewhere: borrow a buffer
-      const size_t bytes = (size_t)w->d.n * w->d.oh * w->d.ow * w->d.y_cs;
-      if (int rc = tpuhip_malloc(ctx, bytes, &ty)) return rc;
-    }
-    int rc = autotune_mfma(ctx, const_cast<tpuhip_conv_weights *>(w), x, ty, tp);
-    if (ty != y) tpuhip_free(ctx, ty);
-    if (rc) return rc;
-  }
+  if (w->algo == ALGO_MFMA && !w->tuned)
+    if (int rc = choose_tile(ctx, const_cast<tpuhip_conv_weights *>(w), x, y, post)) return rc;
   TPUHIP_REQUIRE(!post.lut || w->algo == ALGO_DEPTHWISE || w->algo == ALGO_DEPTHWISE_DOT ||
                      w->algo == ALGO_STEM ||
                      (w->algo == ALGO_MFMA && tile_has_lds_epilogue(w->tile)),

@@ -281,7 +281,7 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
   memcpy(image.data() + tab_at, tab.data(), tab.size() * sizeof(int2));
   memcpy(image.data() + phase_at, phases.data(), phases.size() * sizeof(GatherPhase));
   int rc = tpuhip_malloc(ctx, image.size(), (void **)&plan->w);
-  if (!rc) rc = tpuhip_upload(ctx, plan->w, image.data(), image.size());
+  if (!rc) rc = stage_upload(ctx, plan->w, image.data(), image.size());
   if (rc) {
     gather_destroy(ctx, plan);
     return rc;

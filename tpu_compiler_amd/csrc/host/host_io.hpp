@@ -9,6 +9,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 
 #include "common.hpp"
 
@@ -19,6 +20,9 @@ namespace tpuhip {
 bool floats_to_bytes(const float *src, int8_t *dst, size_t n, bool is_unsigned);
 // n int8 (is_unsigned: uint8) -> floats
 void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned);
+
+// piece(0) .. piece(n - 1), on this thread and a few others; returns when all are done.  Pieces throw nothing.
+void parallel_pieces(size_t n, const std::function<void(size_t)> &piece);
 
 // What the host side holds: float-stored integers (converted and checked), int8 bytes, or floats that stay floats.
 enum class HostKind { kFloatStored, kBytes, kFloats };

@@ -3,6 +3,8 @@
 // lib/Dialect/TPU/Interpreter/MlirModuleInterpreter.cpp:73-457.
 #include "tpuhip/interpreter.hpp"
 
+#include "host_io.hpp"
+
 #include <algorithm>
 
 #include <cstdio>
@@ -48,7 +50,15 @@ void ModuleInterpreter::updateWeightMap(const std::string &name, const float *da
   weightMapping[name] = w;
 }
 
+void ModuleInterpreter::updateWeightMap(const std::string &name, std::vector<float> &&data) {
+  auto w = std::make_shared<WeightData>();
+  w->data = std::move(data);
+  weightMapping[name] = w;
+}
+
 void ModuleInterpreter::loadModule(ModuleDesc &module, std::string target_op) {
+  // packed weights arrive in stream order, in front of whatever this module runs: no prepack call waits for them
+  FlagScope loading(ctx_->loading);
   updateKernelList(module, target_op);
   fuseKernels();
   chainConvs();

@@ -43,6 +43,14 @@ int8_t weight_to_i8(float v, const std::string &op, const char *role) {
   return (int8_t)v;
 }
 
+// a float-stored int8 weight array as bytes
+std::vector<int8_t> weights_to_i8(const std::vector<float> &v, const std::string &op, const char *role) {
+  std::vector<int8_t> out(v.size());
+  if (floats_to_bytes(v.data(), out.data(), v.size(), false))
+    for (float f : v) weight_to_i8(f, op, role);   // names the value
+  return out;
+}
+
 void view4(const SyncedDataShape &s, int *n, int *c, int *h, int *w) {
   if (s.empty() || s.size() > 6) fail("tensor rank " + std::to_string(s.size()) + " not supported");
   int64_t d[4] = {1, 1, 1, 1};
@@ -341,8 +349,7 @@ Conv2DOpKernel::Conv2DOpKernel(OpDesc &op, value_map_t &valueMapping, weight_map
   if (filter->size() != fsz) fail("Conv2D '" + name + "': filter size mismatch");
   if (quant_rshift->size() < (size_t)d.oc || quant_multiplier->size() < (size_t)d.oc)
     fail("Conv2D '" + name + "': rshift / multiplier need one entry per output channel");
-  std::vector<int8_t> w8(fsz);
-  for (size_t i = 0; i < fsz; ++i) w8[i] = weight_to_i8(filter->at(i), name, "filter");
+  std::vector<int8_t> w8 = weights_to_i8(filter->data, name, "filter");
   if (transposed) {
     // out(oh) = sum x(ih) * w(kh) over ih*sh + kh*dh - pt == oh (MKLDeconv,
     // NativeCpuImplementation.h:194-280) == a stride-1 conv of the input with sh-1 zeros
@@ -671,8 +678,7 @@ FullyConnectedOpKernel::FullyConnectedOpKernel(OpDesc &op, value_map_t &valueMap
   if (output_data->size() != (size_t)batch * m * n) fail("FullyConnected '" + name + "': result size mismatch");
   if (rshift_data->size() < (size_t)batch || multiplier_data->size() < (size_t)batch)
     fail("FullyConnected '" + name + "': one rshift and one multiplier per batch needed");
-  std::vector<int8_t> w8(filter->size());
-  for (size_t i = 0; i < w8.size(); ++i) w8[i] = weight_to_i8(filter->at(i), name, "filter");
+  std::vector<int8_t> w8 = weights_to_i8(filter->data, name, "filter");
   std::vector<int32_t> b32;
   if (bias) {
     if (bias->size() < (size_t)batch * n) fail("FullyConnected '" + name + "': bias size mismatch");

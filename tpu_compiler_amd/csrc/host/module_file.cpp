@@ -1,6 +1,9 @@
 // Loading a module from the files the reference's tools exchange: a TPU-dialect .mlir
 // (text) whose tpu.weight_file names an .npz of float32 arrays, and the flow of the
 // tpuc-interpreter tool around it.
+#include "host_io.hpp"
+
+#include <cstring>
 #include <fstream>
 #include <sstream>
 
@@ -58,29 +61,26 @@ void ModuleInterpreter::loadModuleFile(const std::string &mlir_path, std::string
     std::string wpath = mm.weight_file;
     if (!exists(wpath) && wpath[0] != '/' && exists(dir_of(mlir_path) + wpath)) wpath = dir_of(mlir_path) + wpath;
     TensorFile wfile(wpath, true);
-    std::vector<float> data;
     for (auto &w : mm.weights) {
       size_t count = 1;
       for (auto v : w.shape) {
         if (v < 0) throw std::runtime_error("weight '" + w.name + "': dynamic shape");
         count *= (size_t)v;
       }
-      data.resize(count);
-      if (!wfile.readTensor(w.name, data.data(), count)) {
-        auto *a = wfile.find(w.name);
-        if (!a) throw std::runtime_error("failed to find tensor " + w.name + " to read in " + wpath);
+      std::vector<float> data;
+      if (const void *p = wfile.floats(w.name, count)) {
+        data.resize(count);
+        if (count) std::memcpy(data.data(), p, count * sizeof(float));
+      } else {
+        if (!wfile.find(w.name)) throw std::runtime_error("failed to find tensor " + w.name + " to read in " + wpath);
         // beyond the reference's float-stored files: arrays kept with their integer storage type
         // (int8 filters, int32 biases, ...) are widened to float
-        std::vector<float> wide;
         std::vector<int64_t> wshape;
-        if (wfile.readTensorAsFloat(w.name, wide, wshape) && wide.size() == count) {
-          updateWeightMap(w.name, wide.data(), count);
-          continue;
-        }
-        throw std::runtime_error("size does not match for tensor " + w.name + " in " + wpath + " (float32 x " +
-                                 std::to_string(count) + " expected)");
+        if (!wfile.readTensorAsFloat(w.name, data, wshape) || data.size() != count)
+          throw std::runtime_error("size does not match for tensor " + w.name + " in " + wpath + " (float32 x " +
+                                   std::to_string(count) + " expected)");
       }
-      updateWeightMap(w.name, data.data(), count);
+      updateWeightMap(w.name, std::move(data));
     }
   }
   loadModule(mm.module, target_op);
@@ -116,7 +116,10 @@ void interpretFiles(ModuleInterpreter &interp, const std::string &mlir_path, con
       interp.setTensor(details[j].first, tensors[i], 0);
     }
   }
-  interp.invoke(0);
+  {
+    FlagScope once(interp.context()->single_pass);
+    interp.invoke(0);
+  }
   if (!tensor_out.empty() && tensor_out != "-") {
     auto out = openOutputTensorFile(tensor_out);
     for (auto &name : interp.output_details) {

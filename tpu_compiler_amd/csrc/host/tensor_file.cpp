@@ -1,9 +1,18 @@
 // .npz reading and writing for TensorFile; see tpuhip/tensor_file.hpp.
 #include "tpuhip/tensor_file.hpp"
 
+#include "host_io.hpp"
+
+#include <fcntl.h>
+#include <sys/stat.h>
+#include <unistd.h>
 #include <zlib.h>
 
+#include <algorithm>
+#include <atomic>
+#include <cerrno>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <stdexcept>
 
@@ -23,8 +32,8 @@ void wr64(std::vector<uint8_t> &v, uint64_t x) { for (int i = 0; i < 8; ++i) v.p
 constexpr uint32_t kLocalSig = 0x04034b50, kCentralSig = 0x02014b50, kEndSig = 0x06054b50;
 constexpr uint32_t kEnd64Sig = 0x06064b50, kEnd64LocSig = 0x07064b50;
 
-// the header dictionary of a .npy member -> dtype, order and shape
-NpyArray parse_npy(const uint8_t *p, size_t n, const std::string &member) {
+// the header dictionary of a .npy member -> dtype, order and shape; *values, *size: where its values lie
+NpyArray parse_npy(const uint8_t *p, size_t n, const std::string &member, const uint8_t **values, size_t *size) {
   if (n < 10 || std::memcmp(p, "\x93NUMPY", 6) != 0) fail("member '" + member + "' is not a .npy array");
   const int major = p[6];
   size_t hlen, hoff;
@@ -78,7 +87,8 @@ NpyArray parse_npy(const uint8_t *p, size_t n, const std::string &member) {
   }
   const size_t want = a.count() * (size_t)a.word_size;
   if (hoff + hlen + want > n) fail("member '" + member + "': data shorter than its shape says");
-  a.bytes.assign(p + hoff + hlen, p + hoff + hlen + want);
+  *values = p + hoff + hlen;
+  *size = want;
   return a;
 }
 
@@ -133,19 +143,33 @@ TensorFile::TensorFile(const std::string &filename_, bool readOnly_, bool newCre
   if (readOnly && map.empty()) fail(filename + " not exist, failed to read for read");
 }
 
+// The whole file is read into one block (by several threads where it is large) and its values stay there: weights go
+// from it straight to where they are used.
 void TensorFile::load() {
-  FILE *f = std::fopen(filename.c_str(), "rb");
-  if (!f) fail(filename + " doesn't exist, please check");
-  std::vector<uint8_t> buf;
-  std::fseek(f, 0, SEEK_END);
-  const long sz = std::ftell(f);
-  std::fseek(f, 0, SEEK_SET);
-  if (sz < 0) { std::fclose(f); fail("cannot size " + filename); }
-  buf.resize((size_t)sz);
-  const size_t got = sz ? std::fread(buf.data(), 1, (size_t)sz, f) : 0;
-  std::fclose(f);
-  if (got != (size_t)sz) fail("short read of " + filename);
-  if (buf.size() < 22) fail(filename + " is not a zip archive");
+  const int fd = ::open(filename.c_str(), O_RDONLY | O_CLOEXEC);
+  if (fd < 0) fail(filename + " doesn't exist, please check");
+  struct stat st;
+  if (::fstat(fd, &st) != 0 || st.st_size < 0) { ::close(fd); fail("cannot size " + filename); }
+  const size_t sz = (size_t)st.st_size;
+  if (sz < 22) { ::close(fd); fail(filename + " is not a zip archive"); }
+  uint8_t *block = (uint8_t *)std::malloc(sz);
+  if (!block) { ::close(fd); fail("no memory for " + filename); }
+  image = std::shared_ptr<const uint8_t>(block, [](const uint8_t *p) { std::free((void *)p); });
+  constexpr size_t kPart = 1 << 20;
+  std::atomic<bool> short_read{false};
+  parallel_pieces((sz + kPart - 1) / kPart, [&](size_t i) {
+    size_t at = i * kPart, end = std::min(sz, at + kPart);
+    while (at < end) {
+      const ssize_t got = ::pread(fd, block + at, end - at, (off_t)at);
+      if (got < 0 && errno == EINTR) continue;
+      if (got <= 0) { short_read.store(true); return; }
+      at += (size_t)got;
+    }
+  });
+  ::close(fd);
+  if (short_read.load()) fail("short read of " + filename);
+  struct { const uint8_t *p; size_t n; const uint8_t &operator[](size_t i) const { return p[i]; } size_t size() const { return n; } }
+      buf{image.get(), sz};
 
   // end of central directory: the last record, possibly followed by a comment
   size_t eocd = std::string::npos;
@@ -192,29 +216,53 @@ void TensorFile::load() {
     std::string name = member;
     if (name.size() > 4 && name.compare(name.size() - 4, 4, ".npy") == 0) name.resize(name.size() - 4);
     if (method == 0) {
-      map[name] = parse_npy(&buf[data], (size_t)csize, member);
+      Member m;
+      m.array = parse_npy(&buf[data], (size_t)csize, member, &m.data, &m.size);
+      map[name] = std::move(m);
     } else if (method == 8) {
       if (csize > 0xffffffffu || usize > 0xffffffffu) fail("compressed member " + member + " is too large");
-      std::vector<uint8_t> raw((size_t)usize);
+      inflated.push_back(std::make_shared<std::vector<uint8_t>>((size_t)usize));
+      std::vector<uint8_t> &raw = *inflated.back();
       z_stream zs{};
       if (inflateInit2(&zs, -MAX_WBITS) != Z_OK) fail("zlib init failed");
-      zs.next_in = &buf[data];
+      zs.next_in = const_cast<Bytef *>(&buf[data]);
       zs.avail_in = (uInt)csize;
       zs.next_out = raw.data();
       zs.avail_out = (uInt)usize;
       const int rc = inflate(&zs, Z_FINISH);
       inflateEnd(&zs);
       if (rc != Z_STREAM_END) fail(filename + ": cannot inflate " + member);
-      map[name] = parse_npy(raw.data(), raw.size(), member);
+      Member m;
+      m.array = parse_npy(raw.data(), raw.size(), member, &m.data, &m.size);
+      map[name] = std::move(m);
     } else {
       fail(filename + ": member " + member + " uses compression method " + std::to_string(method));
     }
   }
 }
 
+void TensorFile::own(Member &m) {
+  if (m.data && m.array.bytes.size() != m.size) m.array.bytes.assign(m.data, m.data + m.size);
+}
+
+const uint8_t *TensorFile::Member::values() const {
+  static const uint8_t none = 0;   // an array without elements has a place all the same
+  return data ? data : array.bytes.empty() ? &none : array.bytes.data();
+}
+
 const NpyArray *TensorFile::find(const std::string &name) const {
   auto it = map.find(name);
-  return it == map.end() ? nullptr : &it->second;
+  if (it == map.end()) return nullptr;
+  own(it->second);
+  return &it->second.array;
+}
+
+const void *TensorFile::floats(const std::string &name, size_t count) const {
+  auto it = map.find(name);
+  if (it == map.end()) return nullptr;
+  const NpyArray &a = it->second.array;
+  const size_t have = it->second.data ? it->second.size : a.num_bytes();
+  return a.kind == 'f' && a.word_size == 4 && have == count * sizeof(float) ? it->second.values() : nullptr;
 }
 
 std::vector<std::string> TensorFile::names() const {
@@ -227,7 +275,7 @@ bool TensorFile::addTensor(const std::string &name, const NpyArray &array) {
   if (readOnly) fail("addTensor on a read-only file");
   if (map.count(name)) return false;
   if (array.bytes.size() != array.count() * (size_t)array.word_size) fail("addTensor: byte count does not match the shape");
-  map[name] = array;
+  map[name].array = array;
   ++changes;
   return true;
 }
@@ -244,11 +292,9 @@ bool TensorFile::addTensor(const std::string &name, const float *data, const std
 }
 
 bool TensorFile::readTensor(const std::string &name, float *data, size_t count) const {
-  auto *a = find(name);
-  if (!a) return false;
-  if (a->kind != 'f' || a->word_size != 4) return false;
-  if (a->num_bytes() != count * sizeof(float)) return false;
-  if (count) std::memcpy(data, a->bytes.data(), a->num_bytes());
+  const void *p = floats(name, count);
+  if (!p) return false;
+  if (count) std::memcpy(data, p, count * sizeof(float));
   return true;
 }
 
@@ -291,10 +337,10 @@ bool TensorFile::deleteTensor(const std::string &name) {
 void TensorFile::readAllTensors(std::vector<std::string> &names_, std::vector<std::vector<float>> &tensors,
                                 std::vector<std::vector<int64_t>> &shapes) const {
   for (auto &kv : map) {
-    const NpyArray &a = kv.second;
+    const NpyArray &a = kv.second.array;
     if (a.kind != 'f' || a.word_size != 4) fail("readAllTensors: '" + kv.first + "' is not float32 (support float only for now)");
     std::vector<float> t(a.count());
-    if (!t.empty()) std::memcpy(t.data(), a.bytes.data(), a.num_bytes());
+    if (!t.empty()) std::memcpy(t.data(), kv.second.values(), t.size() * sizeof(float));
     tensors.push_back(std::move(t));
     shapes.push_back(a.shape);
     names_.push_back(kv.first);
@@ -304,6 +350,12 @@ void TensorFile::readAllTensors(std::vector<std::string> &names_, std::vector<st
 int TensorFile::keep() {
   if (readOnly) fail("keep on a read-only file");
   if (changes == 0) return 0;
+  for (auto &kv : map) {
+    own(kv.second);
+    kv.second.data = nullptr;
+  }
+  image.reset();
+  inflated.clear();
   FILE *f = std::fopen(filename.c_str(), "wb");
   if (!f) fail("cannot create " + filename);
   std::vector<uint8_t> central;
@@ -314,14 +366,15 @@ int TensorFile::keep() {
   };
   for (auto &kv : map) {
     const std::string member = kv.first + ".npy";
-    const std::vector<uint8_t> head = npy_header(kv.second);
-    const uint64_t size = head.size() + kv.second.bytes.size();
+    const NpyArray &array = kv.second.array;
+    const std::vector<uint8_t> head = npy_header(array);
+    const uint64_t size = head.size() + array.bytes.size();
     uLong crc = crc32(0L, Z_NULL, 0);
     crc = crc32(crc, head.data(), (uInt)head.size());
     {
       // crc32 takes 32-bit lengths
-      const uint8_t *p = kv.second.bytes.data();
-      size_t left = kv.second.bytes.size();
+      const uint8_t *p = array.bytes.data();
+      size_t left = array.bytes.size();
       while (left) {
         const size_t n = left > (1u << 30) ? (1u << 30) : left;
         crc = crc32(crc, p, (uInt)n);
@@ -346,7 +399,7 @@ int TensorFile::keep() {
     put(member.data(), member.size());
     put(extra.data(), extra.size());
     put(head.data(), head.size());
-    put(kv.second.bytes.data(), kv.second.bytes.size());
+    put(array.bytes.data(), array.bytes.size());
 
     std::vector<uint8_t> cx;
     if (big) { wr16(cx, 0x0001); wr16(cx, 24); wr64(cx, size); wr64(cx, size); wr64(cx, lho); }
