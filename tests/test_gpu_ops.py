@@ -1545,3 +1545,45 @@ def test_conv_grouped_and_transposed(ctx, case, smallest_shift):
     want = oracle_conv(x, w, bias, rsh, mult, g, stride, pads, dil, ins, relu)
     got, _ = run_conv(ctx, x, w, bias, rsh, mult, g=g, stride=stride, pads=pads, dil=dil, ins=ins, do_relu=relu)
     assert np.array_equal(got, want), "%d mismatches" % (got != want).sum()
+
+
+KSPLIT_TILES = [t for t in range(NUM_TILES) if "_ksplit_" in capi_tile_name(t)]
+
+
+# n, ic, ih, iw, oc, k, stride, relu: fewer K slices than waves, a ragged last block of pixels and of channels, one pixel,
+# more filter than input (channel-block order), several slices per wave
+@pytest.mark.parametrize("case", [(1, 16, 5, 7, 40, 1, 1, True), (2, 48, 9, 9, 33, 3, 2, False), (1, 256, 1, 1, 70, 1, 1, True),
+                                  (1, 512, 7, 7, 96, 3, 1, False), (3, 320, 11, 13, 255, 3, 1, True)])
+@pytest.mark.parametrize("tile", KSPLIT_TILES)
+@pytest.mark.parametrize("post", ["table", "add", "table_add_only"])
+def test_conv_ksplit_epilogues(ctx, case, tile, post):
+    n, ic, ih, iw, oc, k, stride, relu = case
+    rng = np.random.default_rng(ic + oc * 3 + k)
+    x = rnd_i8(rng, (n, ic, ih, iw))
+    w = rnd_w(rng, (oc, ic, k, k), sigma=14)
+    bias, rsh, mult = rnd_params(rng, oc, 5, 11)
+    p = k // 2
+    y_ref = oracle_conv(x, w, bias, rsh, mult, 1, (stride, stride), (p,) * 4, (1, 1), (0, 0), relu)
+    d = conv_desc(x.shape, w.shape, stride=(stride, stride), pads=(p,) * 4, do_relu=relu, algo=16 + tile)
+    xt, other = ctx.from_nchw(x), rnd_i8(rng, y_ref.shape)
+    ot, yt, tt, zt = ctx.from_nchw(other), ctx.tensor(y_ref.shape), ctx.tensor(y_ref.shape), ctx.tensor(y_ref.shape)
+    for t in (yt, tt, zt):
+        ctx._ck(ctx.lib.tpuhip_memset(ctx.h, t.ptr, 0x55, t.nbytes))
+    wh = ctx.conv_prepack(d, w, f2i32(bias), f2i32(mult), f2i32(rsh))
+    table = rnd_i8(rng, 256)
+    table[0] = 77                                  # pad channels must stay 0 all the same
+    t_ref = O.lut_i8(y_ref, table)
+    add = (ot, zt, 37, 51, 5, True)
+    if post == "table":
+        ctx.conv_post(wh, xt, yt, table, tt)
+    elif post == "add":
+        ctx.conv_post(wh, xt, yt, add=add)
+    else:
+        ctx.conv_post(wh, xt, None, table, None, add)
+    checks = {"table": [(yt, y_ref), (tt, t_ref)], "add": [(yt, y_ref), (zt, O.eltwise_add_i8([other, y_ref], [37, 51], [5], True))],
+              "table_add_only": [(zt, O.eltwise_add_i8([other, t_ref], [37, 51], [5], True))]}[post]
+    for t, ref in checks:
+        assert np.array_equal(ctx.to_nchw(t), ref) and not ctx.raw(t)[..., oc:].any()
+    ctx.conv_weights_destroy(wh)
+    for t in (xt, ot, yt, tt, zt):
+        t.free()

@@ -3155,6 +3155,157 @@ conv_mfma_splitk_kernel(ConvArgs a) {
 
 
 // ---------------------------------------------------------------------------
+// K split over all waves of a large workgroup, for layers with so few outputs that the chip is idle but for the length of
+// one wave's chain (one image from 28x28 down: 56 tiles of 32 x 32 at 14x14x256, K 2304).  A workgroup of W waves owns 32
+// output channels x TN x 32 pixels; wave w multiplies the 32-byte K slices w, w + W, ... -- nine or fewer, four in flight,
+// operands straight from memory in fragment layout (the packing of mfma_reg_32x32) -- and parks its partial sums in LDS.
+// Behind the one barrier, wave f < 4 * TN finishes channel quarter f & 3 of pixel block f >> 2: W reads, requantisation, one
+// dword per pixel, with the table and the add in place; the parameters and the add's operand were requested before K.
+// Bound: launch + arguments + one trip to memory + one LDS round trip, about 4 us.  Tiles of a layer with more filter
+// than input bytes run channel block by channel block, so that an XCD reads its own part of the filter only.
+// ---------------------------------------------------------------------------
+template <int W, int TN, bool FAST, bool UNI>
+__global__ __launch_bounds__(W * 64) void conv_mfma_ksplit_kernel(ConvArgs a) {
+  extern __shared__ v4i kpart[];   // [wave][pixel block][quarter][lane], then the table's 256 bytes
+  constexpr int D = 4;
+  gather_conv_args(a);
+  gather_conv_args_more(a);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wt = (int)(blockIdx.x & 7) * a.tiles_per_xcd + (int)(blockIdx.x >> 3);
+  if (wt >= a.n_tiles) return;                 // uniform over the workgroup
+  int pix_tile, oc_tile;
+  if (a.pstep_n) {                             // pixel tiles of a channel block side by side; pstep_n of them
+    oc_tile = a.pstep_n == 1 ? wt : (int)__umulhi((uint32_t)wt, a.magic_pw);
+    pix_tile = wt - oc_tile * a.pstep_n;
+  } else {
+    pix_tile = pixel_tile_of(a, wt);
+    oc_tile = wt - pix_tile * a.n_oc_tiles;
+  }
+  const int oc0 = oc_tile * 32, pix0 = pix_tile * (TN * 32);
+  const OutRoute out = route_out(a, __builtin_amdgcn_readfirstlane(oc0));
+  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
+  const int frow = lane & 31, fk = lane >> 5;
+  const int slices = a.kp / 32;
+
+  int poff[TN], ih0[TN], iw0[TN];
+  const int ow_first = pix0 % a.ow;
+  const int t_first = pix0 / a.ow;
+  const int oh_first = t_first % a.oh;
+  const int n_first = t_first / a.oh;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int delta = j * 32 + frow;
+    const bool pv = pix0 + delta < a.npix;
+    const uint32_t t1 = (uint32_t)(ow_first + delta);
+    const uint32_t q1 = a.ow == 1 ? t1 : __umulhi(t1, a.magic_ow);
+    const int ow = (int)(t1 - q1 * (uint32_t)a.ow);
+    const uint32_t t2 = (uint32_t)oh_first + q1;
+    const uint32_t q2 = a.oh == 1 ? t2 : __umulhi(t2, a.magic_oh);
+    const int oh = (int)(t2 - q2 * (uint32_t)a.oh);
+    const int n = n_first + (int)q2;
+    ih0[j] = pv ? oh * a.sh - a.pt : -(1 << 28);
+    iw0[j] = ow * a.sw - a.pl;
+    poff[j] = ((n * a.ih + (oh * a.sh - a.pt)) * a.iw + iw0[j]) * a.x_cs + (UNI ? fk * 16 : 0);
+  }
+  const uint32_t woff = (uint32_t)(oc_tile * slices) * 1024u + (uint32_t)lane * 16u;
+
+  v4i af[D], bf[D][TN];
+  auto load = [&](int slot, int i) {
+    const int s = wave + i * W;
+    const bool in_k = s < slices;
+    af[slot] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(wrsrc, in_k ? woff : kOobOffset, s * 1024, 0);
+    const uint32_t kg = (uint32_t)(2 * s + (UNI ? 0 : fk));
+    const uint32_t tap = (kg * a.magic_c16) >> 20;
+    const int cgrp = (int)(kg - tap * (uint32_t)a.c16);
+    const int tkh = (int)((tap * a.magic_kw) >> 20);
+    const int tkw = (int)tap - tkh * a.kw;
+    const int dh_off = in_k && (int)kg < a.k16 ? tkh * a.dh : (1 << 28);
+    const int dw_off = tkw * a.dw;
+    const int tap_off = (tkh * a.dh * a.iw + dw_off) * a.x_cs + cgrp * 16;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int ih = ih0[j] + dh_off, iw = iw0[j] + dw_off;
+      const bool ok = ((unsigned)ih < (unsigned)a.ih) & ((unsigned)iw < (unsigned)a.iw);
+      bf[slot][j] = buffer_load16(xrsrc, ok ? (uint32_t)(poff[j] + tap_off) : kOobOffset);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+
+  // what the finishing waves need besides the sums
+  const bool finish = wave < 4 * TN;
+  const int q = wave & 3, oc = oc0 + fk * 16 + q * 4;
+  const int pix = pix0 + (wave >> 2) * 32 + frow;
+  const bool live = finish && oc < a.ocw && pix < a.npix;
+  const int64_t off = (int64_t)pix * out.y_cs + (oc - out.shift);
+  v4i bias = {0, 0, 0, 0}, mult = bias, shift = bias, hpot = bias;
+  uint32_t src = 0;
+  if (finish) {
+    bias = *reinterpret_cast<const v4i *>(a.bias + oc);
+    mult = *reinterpret_cast<const v4i *>(a.qmult + oc);
+    shift = *reinterpret_cast<const v4i *>(a.qshift + oc);
+    hpot = *reinterpret_cast<const v4i *>(a.qhpot + oc);
+    if (a.add_dst && live) src = *reinterpret_cast<const uint32_t *>(a.add_src + off);
+  }
+  uint8_t *lut = reinterpret_cast<uint8_t *>(kpart + W * TN * 256);
+  uint32_t lutv = 0;
+  if (a.has_lut && tid < 64) lutv = a.lut.w[tid];
+
+  v16i acc[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[j][e] = 0;
+  const int mine = (slices - wave + W - 1) / W;
+  auto multiply = [&](int slot) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[slot], bf[slot][j], acc[j], 0, 0, 0);
+  };
+#pragma nounroll
+  for (int i0 = D; i0 < mine; i0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      multiply(d);
+      load(d, i0 + d);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) multiply(d);   // slices past the end are zeros
+  if (a.has_lut && tid < 64) reinterpret_cast<uint32_t *>(lut)[tid] = lutv;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      kpart[((wave * TN + j) * 4 + k) * 64 + lane] = v4i{acc[j][k * 4], acc[j][k * 4 + 1], acc[j][k * 4 + 2], acc[j][k * 4 + 3]};
+  __syncthreads();
+  if (!finish) return;
+  v4i t = bias;
+#pragma unroll
+  for (int w = 0; w < W; ++w) t += kpart[((w * TN + (wave >> 2)) * 4 + q) * 64 + lane];
+  if (a.relu_first) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = max(t[e], 0);
+  }
+  uint32_t o = pack_sat4(requant_core<FAST>(t[0], mult[0], shift[0], hpot[0]), requant_core<FAST>(t[1], mult[1], shift[1], hpot[1]),
+                         requant_core<FAST>(t[2], mult[2], shift[2], hpot[2]), requant_core<FAST>(t[3], mult[3], shift[3], hpot[3]), out.lo);
+  if (!live) return;
+  if (a.store_y) *reinterpret_cast<uint32_t *>(out.y + off) = o;
+  if (a.has_lut) {
+    const uint32_t r = (uint32_t)lut[o & 255u] | ((uint32_t)lut[(o >> 8) & 255u] << 8) | ((uint32_t)lut[(o >> 16) & 255u] << 16) |
+                       ((uint32_t)lut[o >> 24] << 24);
+    const int valid = a.oc - oc;   // channels of this dword that exist
+    o = r & (valid >= 4 ? 0xffffffffu : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u);
+    if (a.lut_dst) *reinterpret_cast<uint32_t *>(a.lut_dst + off) = o;
+  }
+  if (a.add_dst) {
+    const v4i z = fused_add_chunk(v4i{(int)o, 0, 0, 0}, v4i{(int)src, 0, 0, 0}, a.add_m_src, a.add_m_conv, a.add_rshift, a.add_relu, a.add_pk);
+    *reinterpret_cast<uint32_t *>(a.add_dst + off) = (uint32_t)z[0];
+  }
+}
+
+// ---------------------------------------------------------------------------
 // FullyConnected with few rows (the classifier of a network: 32 x 2048 -> 1000): one 32x32
 // block of outputs per 32 output channels, and a K far too long for one wave per block to be
 // anything but a chain of dependent loads.  So K is split over workgroups of ONE wave: wave
@@ -3338,7 +3489,7 @@ struct TileCfg {
   int reg;   // 0: LDS kernel, one tile per workgroup; 1: the LDS-free kernel, bm x bn is the
              // tile of one wave; 2: its split-K form; 3: LDS kernel, persistent workgroups;
              // 4: patch kernel (bn = pixel slots of a tile of whole rows); 5: pointwise kernel;
-             // 6: patch kernel, second form; 7: patch kernel, third form
+             // 6: patch kernel, second form; 7: patch kernel, third form; 8: K split over all waves
   int bk;    // K bytes per step (pointwise kernel: the padded K it holds)
 };
 
@@ -3423,6 +3574,13 @@ struct TileCfg {
   U3(57, "mfma_patch3_64x256_w8", 4, 2, 2)    \
   U3(58, "mfma_patch3_64x192_w8", 3, 2, 2)
 
+// K split over all waves of a workgroup, one barrier: KS(index, name, waves, 32-pixel blocks)
+#define TPUHIP_KSPLIT_TILES(KS)           \
+  KS(60, "mfma_ksplit_32x32_w16", 16, 1)  \
+  KS(61, "mfma_ksplit_32x32_w8", 8, 1)    \
+  KS(62, "mfma_ksplit_32x64_w8", 8, 2)    \
+  KS(63, "mfma_ksplit_32x32_w4", 4, 1)
+
 struct TileTable {
   TileCfg t[64];
   int n = 0;
@@ -3457,6 +3615,11 @@ struct TileTable {
   n = n > i ? n : i + 1;
     TPUHIP_PATCH3_TILES(U3)
 #undef U3
+#define KS(i, name, W, TN) \
+  t[i] = TileCfg{32, TN * 32, 1, 1, name, 8, 64}; \
+  n = n > i ? n : i + 1;
+    TPUHIP_KSPLIT_TILES(KS)
+#undef KS
   }
 };
 const TileTable kTileTable;
@@ -3636,6 +3799,24 @@ void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
   } break;
     TPUHIP_PATCH3_TILES(U3)
 #undef U3
+  }
+}
+
+template <bool FAST, bool UNI>
+void launch_ksplit(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
+  switch (tile) {
+#define KS(i, name, W, TN)                                                                              \
+  case i: {                                                                                             \
+    auto kernel = conv_mfma_ksplit_kernel<W, TN, FAST, UNI>;                                            \
+    const unsigned lds = W * TN * 4096 + 256;                                                           \
+    if (!pw_prepare(kernel, lds)) break;                                                                \
+    if (ctx->prof_start)                                                                                \
+      hipExtLaunchKernelGGL(kernel, grid, dim3(W * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
+    else                                                                                                \
+      hipLaunchKernelGGL(kernel, grid, dim3(W * 64), lds, ctx->stream, a);                              \
+  } break;
+    TPUHIP_KSPLIT_TILES(KS)
+#undef KS
   }
 }
 
@@ -3845,7 +4026,8 @@ void settle_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *cw) {
 
 // the fused table lives in the LDS of the LDS kernels
 bool tile_has_lds_epilogue(int t) {
-  return kTiles[t].reg == 0 || kTiles[t].reg == 3 || kTiles[t].reg == 5 || kTiles[t].reg == 6 || kTiles[t].reg == 7;
+  return kTiles[t].reg == 0 || kTiles[t].reg == 3 || kTiles[t].reg == 5 || kTiles[t].reg == 6 || kTiles[t].reg == 7 ||
+         kTiles[t].reg == 8;
 }
 
 // the pointwise kernels: 1x1 window, no padding, no dilation (any stride), the input channels
@@ -3877,7 +4059,10 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t) {
   if (c.reg == 5 && !pw_shape_ok(d, c)) return false;
   if (c.reg == 6 && patch2_rows(d, c) == 0) return false;
   if (c.reg == 7) return patch3_plan(d, c).th > 0;
-  if (d.ic <= 4 && (c.reg == 1 || c.reg == 2)) return false;   // prefer the 4-channel K packing of the LDS kernels
+  // worth timing only where the tiles are few: with more of them than the chip holds workgroups the layer has parallel
+  // work enough without splitting K sixteen ways
+  if (c.reg == 8 && ceil_div64((int64_t)d.n * d.oh * d.ow, 32) * ceil_div64(d.oc, 32) > 2048) return false;
+  if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8)) return false;   // prefer the 4-channel K packing of the LDS kernels
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle
 }
 
@@ -3930,6 +4115,13 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
     const int n_wgs = t.reg == 1 ? (a.n_tiles + 3) / 4 : a.n_tiles;
     a.tiles_per_xcd = (n_wgs + 7) / 8;
     a.wgs_per_xcd = a.tiles_per_xcd;
+    if (t.reg == 8) {
+      const int n_pix_tiles = a.n_tiles / a.n_oc_tiles;
+      if (a.w_bytes > a.x_bytes && (int64_t)(a.n_tiles + 8 * a.tiles_per_xcd) * n_pix_tiles < (1ll << 32)) {
+        a.pstep_n = n_pix_tiles;
+        a.magic_pw = (uint32_t)(((1ull << 32) + n_pix_tiles - 1) / (uint64_t)n_pix_tiles);
+      }
+    }
     if (t.reg == 4 || t.reg == 6) {
       const int th = t.reg == 4 ? patch_rows(d, t) : patch2_rows(d, t);
       const int tiles_per_img = (d.oh + th - 1) / th;
@@ -4005,6 +4197,11 @@ void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvA
     return;
   }
   const bool uni = (w->c16 % (tile_bk(kTiles[w->tile]) / 16)) == 0;
+  if (kTiles[w->tile].reg == 8) {
+    if (w->fast) uni ? launch_ksplit<true, true>(ctx, w->tile, grid, a) : launch_ksplit<true, false>(ctx, w->tile, grid, a);
+    else uni ? launch_ksplit<false, true>(ctx, w->tile, grid, a) : launch_ksplit<false, false>(ctx, w->tile, grid, a);
+    return;
+  }
   if (w->smallc) {
     if (w->fast)
       launch_mfma<true, kModeSmallC>(ctx, w->tile, grid, a);
