@@ -1587,3 +1587,27 @@ def test_conv_ksplit_epilogues(ctx, case, tile, post):
     ctx.conv_weights_destroy(wh)
     for t in (xt, ot, yt, tt, zt):
         t.free()
+
+
+@pytest.mark.parametrize("axis,extents,y_cs", [
+    (1, (17, 3, 44), None),                  # dwords and groups across two and three inputs
+    (1, (1, 1, 1, 1, 1, 1), 48),             # as many inputs as a launch takes, a stride beyond the channels
+    (1, (5, 2, 9, 16, 1, 30, 7), None),      # one more: a launch per input
+    (2, (3, 1, 5), None), (3, (2, 7), None), (0, (1, 2), None),
+])
+@pytest.mark.parametrize("tables", [False, True])
+def test_concat_of_any_channels_and_tables(ctx, axis, extents, y_cs, tables):
+    rng = np.random.default_rng(axis * 10 + len(extents))
+    xs = [rnd_i8(rng, tuple(e if d == axis else v for d, v in enumerate((2, 37, 4, 3)))) for e in extents]
+    # the first input keeps its bytes, the others are rescaled; relu acts on all of them
+    rsh, mult = [0] + [3] * (len(xs) - 1), [1] + [5] * (len(xs) - 1)
+    want = O.concat_i8(xs, axis, rsh, mult, True) if tables else O.concat_i8(xs, axis)
+    ts = [ctx.from_nchw(a) for a in xs]
+    yt = ctx.tensor(want.shape, y_cs)
+    ctx._ck(ctx.lib.tpuhip_memset(ctx.h, yt.ptr, 0x55, yt.nbytes))
+    if tables:
+        ctx.concat(ts, axis, yt, rsh, mult, True)
+    else:
+        ctx.concat(ts, axis, yt)
+    assert np.array_equal(ctx.to_nchw(yt), want)
+    assert not ctx.raw(yt)[..., want.shape[1]:].any()

@@ -91,6 +91,25 @@ inline void launch(tpuhip_ctx *ctx, F kernel, dim3 grid, dim3 block, Args... arg
 inline int round_up(int v, int m) { return (v + m - 1) / m * m; }
 inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Division of 31-bit numbers by a divisor the host knows, as a multiply and a shift (two instructions; the compiler's own
+// division by an unknown number is some thirty, its 64-bit one a hundred and more): q = (umulhi(x, mul) + x) >> shift with
+// 2^(shift-1) < d <= 2^shift and mul = floor(2^32 * (2^shift - d) / d) + 1, exact for x < 2^31.
+struct FastDiv {
+  uint32_t d = 1, mul = 0, shift = 0;
+  FastDiv() = default;
+  explicit FastDiv(int64_t divisor) : d((uint32_t)divisor) {
+    while ((1ull << shift) < d) ++shift;
+    mul = (uint32_t)(((1ull << 32) * ((1ull << shift) - d)) / d + 1);
+  }
+  __device__ __forceinline__ uint32_t div(uint32_t x) const { return (__umulhi(x, mul) + x) >> shift; }
+  // x -> quotient, remainder in x
+  __device__ __forceinline__ uint32_t split(uint32_t &x) const {
+    const uint32_t q = div(x);
+    x -= q * d;
+    return q;
+  }
+};
+
 // 256-entry int8 table passed to kernels by value (lives in the kernel-argument
 // segment, so no device allocation or copy is needed and launches stay capturable).
 struct Table256 {

@@ -109,94 +109,159 @@ struct LutArgs {
   int c, x_cs, y_cs;  // channels, strides
   int coff;           // channel offset into y (concat)
   int use_table;
+  FastDiv by_groups;  // 16-byte groups per pixel
 };
 
-__device__ __forceinline__ void table_to_lds(const Table256 &t, uint8_t *lds) {
-  // every thread writes the same words; constant indexing keeps the table in SGPRs
-  uint32_t *l32 = reinterpret_cast<uint32_t *>(lds);
-  if (threadIdx.x < 64) {
-#pragma unroll
-    for (int i = 0; i < 64; ++i)
-      if ((int)threadIdx.x == i) l32[i] = t.w[i];
-  }
+// the 64 words of a table, one per thread, out of the kernel arguments (requested first, parked behind the data's request)
+__device__ __forceinline__ uint32_t table_word(const Table256 &t) { return threadIdx.x < 64 ? t.w[threadIdx.x] : 0; }
+__device__ __forceinline__ void park_table(uint32_t word, uint32_t *lds) {
+  if (threadIdx.x < 64) lds[threadIdx.x] = word;
   __syncthreads();
 }
+// four bytes through a table in LDS; bytes from `valid` on are zero
+__device__ __forceinline__ uint32_t look_up4(uint32_t w, const uint8_t *tab, int valid) {
+  const uint32_t o = (uint32_t)tab[w & 255u] | ((uint32_t)tab[(w >> 8) & 255u] << 8) | ((uint32_t)tab[(w >> 16) & 255u] << 16) |
+                     ((uint32_t)tab[w >> 24] << 24);
+  return o & (valid >= 4 ? 0xffffffffu : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u);
+}
 
-// vector form: c16 groups of 16 channels per pixel, strides multiple of 16, coff multiple of 16
+// vector form: groups of 16 channels, strides multiple of 16, coff multiple of 16.  One group per thread: 4 x 120 x 75 x 75 in
+// 3.1 us (8.2 with four groups after one another in a quarter of the threads and a table spread by 64 selects).
 __global__ __launch_bounds__(kThreads) void lut_vec_kernel(LutArgs a, Table256 t) {
-  __shared__ uint8_t tab[256];
-  table_to_lds(t, tab);
-  const int c16 = (a.c + 15) >> 4;
-  const int64_t total = a.pixels * c16;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t pix = i / c16;
-    const int cg = (int)(i - pix * c16);
-    v4i v = *reinterpret_cast<const v4i *>(a.x + pix * a.x_cs + cg * 16);
-    if (a.use_table) {
+  __shared__ uint32_t tab[64];
+  const uint32_t word = a.use_table ? table_word(t) : 0;
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const bool live = i < a.pixels * a.by_groups.d;
+  uint32_t r = (uint32_t)i;
+  const int64_t pix = a.by_groups.split(r);
+  const int cg = (int)r;
+  v4i v = {0, 0, 0, 0};
+  if (live) v = *reinterpret_cast<const v4i *>(a.x + pix * a.x_cs + cg * 16);
+  if (a.use_table) {
+    park_table(word, tab);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t w = (uint32_t)v[q], o = 0;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int ch = cg * 16 + q * 4 + b;
-          const uint32_t e = ch < a.c ? tab[(w >> (8 * b)) & 0xffu] : 0u;
-          o |= e << (8 * b);
-        }
-        v[q] = (int)o;
-      }
-    }
-    *reinterpret_cast<v4i *>(a.y + pix * a.y_cs + a.coff + cg * 16) = v;
+    for (int q = 0; q < 4; ++q) v[q] = (int)look_up4((uint32_t)v[q], reinterpret_cast<const uint8_t *>(tab), a.c - cg * 16 - q * 4);
   }
+  if (live) *reinterpret_cast<v4i *>(a.y + pix * a.y_cs + a.coff + cg * 16) = v;
 }
 
 // byte form for channel offsets / counts that are not multiples of 16
 __global__ __launch_bounds__(kThreads) void lut_byte_kernel(LutArgs a, Table256 t) {
-  __shared__ uint8_t tab[256];
-  table_to_lds(t, tab);
+  __shared__ uint32_t tab[64];
+  park_table(a.use_table ? table_word(t) : 0, tab);
   const int64_t total = a.pixels * a.c;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t pix = i / a.c;
     const int ch = (int)(i - pix * a.c);
     uint8_t v = (uint8_t)a.x[pix * a.x_cs + ch];
-    if (a.use_table) v = tab[v];
+    if (a.use_table) v = reinterpret_cast<const uint8_t *>(tab)[v];
     a.y[pix * a.y_cs + a.coff + ch] = (int8_t)v;
   }
 }
 
-// concat of up to four inputs that changes no byte, along any axis: in channels-last memory every
-// axis is "for each outer index, the inputs' chunks one after the other" (outer = pixel for the
-// channel axis, image row for w, image for h, nothing for n), chunks whole 16-byte groups.
-// One launch, a lane moves one 16-byte group.
-struct ConcatArgs {
-  const int8_t *x[4];
+// Concat of up to kConcatMax inputs as one launch, each input with a table of its own or none.
+constexpr int kConcatMax = 6;
+
+// along the channels: a thread makes 16 channels of an output pixel.  A dword that lies inside one input is one load at any
+// alignment; one that straddles two is put together from bytes.  (Inputs off the 16-channel grid went byte by byte, a
+// launch each and one for the pad channels: 4 x (120 + 120) x 75 x 75 in 22 us, now 5.4, with tables 6.3.)
+struct ConcatChannelArgs {
+  const int8_t *x[kConcatMax];
   int8_t *y;
-  int64_t outer;       // outer indices
-  int64_t stride[4];   // bytes from one outer index to the next in each input
-  int64_t y_stride;    // ... in the output
-  int64_t start[5];    // first 16-byte group of each input's chunk within an output chunk; start[n] = groups per chunk
-  int64_t groups;      // groups written per outer index (>= start[n]; the rest are zero)
-  int n;
+  int start[kConcatMax + 1];   // first output channel of each input; start[n] = output channels
+  int cs[kConcatMax];
+  int n, y_cs, tables;         // tables: bit k set where input k has one
+  FastDiv by_groups;           // groups written per pixel
+  int64_t total;
+};
+struct Tables {
+  Table256 t[kConcatMax];
 };
 
-__global__ __launch_bounds__(kThreads) void concat_chunks_kernel(ConcatArgs a) {
-  const int64_t g16 = a.groups;   // groups written per outer index: those of the inputs, then zero pad groups
-  const int64_t total = a.outer * g16;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t o = i / g16;
-    const int64_t g = i - o * g16;
-    // which input the group comes from: selects, so that no array is indexed by a lane's value
-    const int8_t *src = a.x[0];
-    int64_t stride = a.stride[0], first = 0;
-    if (a.n > 1 && g >= a.start[1]) { src = a.x[1]; stride = a.stride[1]; first = a.start[1]; }
-    if (a.n > 2 && g >= a.start[2]) { src = a.x[2]; stride = a.stride[2]; first = a.start[2]; }
-    if (a.n > 3 && g >= a.start[3]) { src = a.x[3]; stride = a.stride[3]; first = a.start[3]; }
-    v4i v = {0, 0, 0, 0};
-    if (g < a.start[a.n]) v = *reinterpret_cast<const v4i *>(src + o * stride + (g - first) * 16);
-    *reinterpret_cast<v4i *>(a.y + o * a.y_stride + g * 16) = v;
+__global__ __launch_bounds__(kThreads) void concat_channels_kernel(ConcatChannelArgs a, Tables t) {
+  __shared__ uint32_t tab[kConcatMax * 64];
+  if (a.tables) {
+    for (int k = threadIdx.x; k < a.n * 64; k += kThreads) tab[k] = t.t[k >> 6].w[k & 63];
+    __syncthreads();
   }
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= a.total) return;
+  uint32_t r = (uint32_t)i;
+  const int64_t pix = a.by_groups.split(r);
+  const int c0 = (int)r * 16;
+  v4i out;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = c0 + q * 4;
+    int k = 0;
+#pragma unroll
+    for (int j = 1; j < kConcatMax; ++j)
+      if (j < a.n && c >= a.start[j]) k = j;
+    const int8_t *src = a.x[0];
+    int first = 0, last = a.start[1], cs = a.cs[0];
+#pragma unroll
+    for (int j = 1; j < kConcatMax; ++j)
+      if (k == j) { src = a.x[j]; first = a.start[j]; last = a.start[j + 1]; cs = a.cs[j]; }
+    uint32_t w = 0;
+    if (c + 4 <= last) {
+      __builtin_memcpy(&w, src + pix * cs + (c - first), 4);
+      if (a.tables >> k & 1) w = look_up4(w, reinterpret_cast<const uint8_t *>(tab + k * 64), 4);
+    } else {
+      for (int b = 0; b < 4; ++b) {
+        const int cb = c + b;
+        if (cb >= a.start[a.n]) break;   // pad channels are zero
+        int kb = 0;
+        while (kb + 1 < a.n && cb >= a.start[kb + 1]) ++kb;
+        uint32_t v = (uint8_t)a.x[kb][pix * a.cs[kb] + (cb - a.start[kb])];
+        if (a.tables >> kb & 1) v = reinterpret_cast<const uint8_t *>(tab + kb * 64)[v];
+        w |= v << (8 * b);
+      }
+    }
+    out[q] = (int)w;
+  }
+  *reinterpret_cast<v4i *>(a.y + pix * a.y_cs + c0) = out;
+}
+
+// along n, h or w: in channels-last memory these are "for each outer index, the inputs' chunks one after the other" (outer =
+// image row for w, image for h, nothing for n), chunks of whole pixels.  A thread moves one 16-byte group.
+struct ConcatArgs {
+  const int8_t *x[kConcatMax];
+  int8_t *y;
+  int64_t outer;                 // outer indices
+  int64_t stride[kConcatMax];    // bytes from one outer index to the next in each input
+  int64_t y_stride;              // ... in the output
+  int64_t start[kConcatMax + 1]; // first 16-byte group of each input's chunk within an output chunk; start[n] = groups per chunk
+  int n, c, tables;
+  FastDiv by_groups, by_c16;     // groups per outer index, per pixel
+};
+
+__global__ __launch_bounds__(kThreads) void concat_chunks_kernel(ConcatArgs a, Tables t) {
+  __shared__ uint32_t tab[kConcatMax * 64];
+  if (a.tables) {
+    for (int k = threadIdx.x; k < a.n * 64; k += kThreads) tab[k] = t.t[k >> 6].w[k & 63];
+    __syncthreads();
+  }
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= a.outer * a.start[a.n]) return;
+  uint32_t g = (uint32_t)i;
+  const int64_t o = a.by_groups.split(g);
+  // which input the group comes from: selects, so that no array is indexed by a lane's value
+  const int8_t *src = a.x[0];
+  int64_t stride = a.stride[0], first = 0;
+  int k = 0;
+#pragma unroll
+  for (int j = 1; j < kConcatMax; ++j)
+    if (a.n > j && g >= a.start[j]) { src = a.x[j]; stride = a.stride[j]; first = a.start[j]; k = j; }
+  v4i v = *reinterpret_cast<const v4i *>(src + o * stride + (g - first) * 16);
+  if (a.tables >> k & 1) {
+    uint32_t cg = g;   // chunks are whole pixels, so the group's place in its pixel follows from g alone
+    a.by_c16.split(cg);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      v[q] = (int)look_up4((uint32_t)v[q], reinterpret_cast<const uint8_t *>(tab + k * 64), a.c - (int)cg * 16 - q * 4);
+  }
+  *reinterpret_cast<v4i *>(a.y + o * a.y_stride + (int64_t)g * 16) = v;
 }
 
 // zero the channels [c0, c1) of every pixel
@@ -228,26 +293,27 @@ __global__ __launch_bounds__(kThreads) void relu_kernel(const v4i *x, v4i *y, in
 }
 
 // ---------------------------------------------------------------------------
-// nearest upsample (core/upsample.cpp:20-41), channels-last: one 16-byte group
-// of an output pixel per lane.
+// nearest upsample (core/upsample.cpp:20-41), channels-last: a thread reads one 16-byte group of an input pixel and
+// writes it to the sh x sw output pixels it becomes.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void upsample_kernel(const int8_t *x, int8_t *y, int n,
-                                                            int ih, int iw, int sh, int sw,
-                                                            int c16, int x_cs, int y_cs) {
-  const int oh = ih * sh, ow = iw * sw;
-  const int64_t total = (int64_t)n * oh * ow * c16;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int cg = (int)(i % c16);
-    int64_t p = i / c16;
-    const int wo = (int)(p % ow);
-    p /= ow;
-    const int ho = (int)(p % oh);
-    const int b = (int)(p / oh);
-    const int64_t src = ((int64_t)(b * ih + ho / sh) * iw + wo / sw) * x_cs + cg * 16;
-    const int64_t dst = ((int64_t)(b * oh + ho) * ow + wo) * y_cs + cg * 16;
-    *reinterpret_cast<v4i *>(y + dst) = *reinterpret_cast<const v4i *>(x + src);
-  }
+struct UpsampleArgs {
+  const int8_t *x;
+  int8_t *y;
+  FastDiv by_groups, by_iw;   // 16-byte groups per pixel, input columns
+  int sh, sw, ow, x_cs, y_cs;
+  int64_t total;
+};
+__global__ __launch_bounds__(kThreads) void upsample_kernel(UpsampleArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= a.total) return;
+  uint32_t cg = (uint32_t)i;
+  uint32_t pix = a.by_groups.split(cg);
+  const v4i v = *reinterpret_cast<const v4i *>(a.x + (int64_t)pix * a.x_cs + cg * 16);
+  uint32_t w = pix;
+  const uint32_t row = a.by_iw.split(w);   // image * input rows + input row: output rows follow each other the same way
+  int8_t *to = a.y + ((int64_t)row * a.sh * a.ow + (int64_t)w * a.sw) * a.y_cs + cg * 16;
+  for (int r = 0; r < a.sh; ++r, to += (int64_t)a.ow * a.y_cs)
+    for (int s = 0; s < a.sw; ++s) *reinterpret_cast<v4i *>(to + (int64_t)s * a.y_cs) = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -530,8 +596,12 @@ int launch_lut(tpuhip_ctx *ctx, const void *x, void *y, const int8_t *table, int
   const bool vec = (x_cs % 16 == 0) && (y_cs % 16 == 0) && (coff % 16 == 0) &&
                    (c % 16 == 0 || (coff + round_up(c, 16) <= y_cs));
   if (vec) {
-    const int64_t total = pixels * ((c + 15) / 16);
-    launch(ctx, lut_vec_kernel, dim3(grid_for(total, kThreads * 4)), dim3(kThreads), a, t);
+    a.by_groups = FastDiv((c + 15) / 16);
+    const int64_t most = ((1ll << 31) - 1) / a.by_groups.d;   // as many pixels as the 31-bit index reaches
+    for (int64_t p0 = 0; p0 < pixels; p0 += most, a.x += most * x_cs, a.y += most * y_cs) {
+      a.pixels = std::min(most, pixels - p0);
+      launch(ctx, lut_vec_kernel, dim3((unsigned)ceil_div64(a.pixels * a.by_groups.d, kThreads)), dim3(kThreads), a, t);
+    }
   } else {
     launch(ctx, lut_byte_kernel, dim3(grid_for(pixels * c, kThreads * 8)), dim3(kThreads), a, t);
   }
@@ -771,9 +841,21 @@ int tpuhip_upsample_nearest_i8(tpuhip_ctx *ctx, const void *x, void *y, int n, i
   TPUHIP_REQUIRE(x_cs % 16 == 0 && y_cs % 16 == 0 && x_cs >= c && y_cs >= c,
                  "upsample: bad channel strides %d / %d for %d channels", x_cs, y_cs, c);
   const int c16 = (c + 15) / 16;
-  const int64_t total = (int64_t)n * ih * scale_h * iw * scale_w * c16;
-  launch(ctx, upsample_kernel, dim3(grid_for(total, kThreads * 2)), dim3(kThreads), (const int8_t *)x, (int8_t *)y, n, ih, iw, scale_h, scale_w, c16,
-                     x_cs, y_cs);
+  UpsampleArgs a{};
+  a.x = (const int8_t *)x;
+  a.y = (int8_t *)y;
+  a.by_groups = FastDiv(c16);
+  a.by_iw = FastDiv(iw);
+  a.sh = scale_h; a.sw = scale_w; a.ow = iw * scale_w;
+  a.x_cs = x_cs; a.y_cs = y_cs;
+  const int64_t rows = (int64_t)n * ih, row_groups = (int64_t)iw * c16;
+  const int64_t most = std::max<int64_t>(((1ll << 31) - 1) / row_groups, 1);   // as many rows as the 31-bit index reaches
+  for (int64_t r0 = 0; r0 < rows; r0 += most) {
+    a.total = std::min(most, rows - r0) * row_groups;
+    launch(ctx, upsample_kernel, dim3((unsigned)ceil_div64(a.total, kThreads)), dim3(kThreads), a);
+    a.x += most * iw * x_cs;
+    a.y += most * scale_h * a.ow * y_cs;
+  }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }
@@ -802,45 +884,9 @@ int tpuhip_concat_i8(tpuhip_ctx *ctx, const void *const *xs, int nin, const int 
   const int N = out_dims[0], Cc = out_dims[1], H = out_dims[2], W = out_dims[3];
   TPUHIP_REQUIRE(y_cs >= Cc && y_cs % 16 == 0, "concat: bad output channel stride %d", y_cs);
 
-  // A concat that changes no byte (no rescaling that is not the identity; a ReLU would change negative
-  // bytes) of two to four inputs is one launch for all of them: along the channels when every input
-  // has whole 16-channel groups; along n, h or w when all tensors have the channel stride of their channel count (a chunk
-  // is then a run of whole pixels, pad channels included, which are zero in every input).
-  bool plain = nin >= 2 && nin <= 4 && !do_relu;
-  for (int i = 0; i < nin && plain; ++i) {
-    plain = axis == 1 ? in_dims[4 * i + 1] % 16 == 0 : (in_cs[i] == y_cs && y_cs == round_up(Cc, 16));
-    if (need_quant && !(multiplier[i] == 1 && rshift[i] == 0)) plain = false;
-  }
-  if (plain) {
-    ConcatArgs a{};
-    a.y = (int8_t *)y;
-    a.n = nin;
-    // bytes of one step along the axis, and of everything inside one outer index of the output
-    const int64_t unit = axis == 1 ? 1 : axis == 3 ? y_cs : axis == 2 ? (int64_t)W * y_cs : (int64_t)H * W * y_cs;
-    a.outer = axis == 1 ? (int64_t)N * H * W : axis == 3 ? (int64_t)N * H : axis == 2 ? N : 1;
-    a.y_stride = axis == 1 ? y_cs : unit * out_dims[axis];
-    for (int i = 0; i < nin; ++i) {
-      a.x[i] = (const int8_t *)xs[i];
-      a.stride[i] = axis == 1 ? in_cs[i] : unit * in_dims[4 * i + axis];
-      a.start[i + 1] = a.start[i] + unit * in_dims[4 * i + axis] / 16;
-    }
-    // the chunks of an outer index fill the output's: Cc channels of a pixel, or all of its rows / pixels
-    TPUHIP_REQUIRE(a.start[nin] * 16 == unit * out_dims[axis] && a.start[nin] * 16 <= a.y_stride,
-                   "concat: chunks of %lld groups do not fill axis %d", (long long)a.start[nin], axis);
-    TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
-    // along the channels the output's stride may be wider than its channels: the pad groups are written as zero
-    a.groups = axis == 1 ? y_cs / 16 : a.start[nin];
-    launch(ctx, concat_chunks_kernel, dim3(grid_for(a.outer * a.groups, kThreads * 4)), dim3(kThreads), a);
-    TPUHIP_CHECK_HIP(hipGetLastError());
-    return TPUHIP_OK;
-  }
-
   // Each input goes through a 256-entry table: requant (unless m == 1, r == 0) then ReLU
-  // -- both pure functions of the int8 input (core/concat.cpp:66-88).
-  int offset = 0;  // running offset along the concat axis
-  for (int i = 0; i < nin; ++i) {
-    const int *dm = in_dims + 4 * i;
-    int8_t table[256];
+  // -- both pure functions of the int8 input (core/concat.cpp:66-88); the identity is no table.
+  auto table_of = [&](int i, int8_t *table) {
     bool identity = true;
     for (int v = -128; v <= 127; ++v) {
       int8_t o = (int8_t)v;
@@ -850,6 +896,67 @@ int tpuhip_concat_i8(tpuhip_ctx *ctx, const void *const *xs, int nin, const int 
       if (o != (int8_t)v) identity = false;
       table[(uint8_t)(int8_t)v] = o;
     }
+    return !identity;
+  };
+  // One launch for all inputs where the kernels' index arithmetic reaches: along the channels always; along n, h or w when
+  // all tensors have the channel stride of their channel count (a chunk is then a run of whole pixels, pad channels included,
+  // which are zero in every input).
+  bool one = nin <= kConcatMax && (int64_t)N * H * W * (y_cs / 16) < (1ll << 31);
+  for (int i = 0; i < nin && one && axis != 1; ++i) one = in_cs[i] == y_cs && y_cs == round_up(Cc, 16);
+  if (one) {
+    TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
+    Tables t{};
+    int tables = 0;
+    for (int i = 0; i < nin; ++i) {
+      int8_t table[256];
+      if (!(need_quant || do_relu) || !table_of(i, table)) continue;
+      t.t[i] = pack_table(table);
+      tables |= 1 << i;
+    }
+    if (axis == 1) {
+      ConcatChannelArgs a{};
+      a.y = (int8_t *)y;
+      a.n = nin;
+      a.y_cs = y_cs;
+      a.tables = tables;
+      for (int i = 0; i < nin; ++i) {
+        a.x[i] = (const int8_t *)xs[i];
+        a.cs[i] = in_cs[i];
+        a.start[i + 1] = a.start[i] + in_dims[4 * i + 1];
+      }
+      for (int i = nin; i < kConcatMax; ++i) a.start[i + 1] = a.start[nin];
+      // the output's stride may be wider than its channels: the pad groups are written as zero
+      a.by_groups = FastDiv(y_cs / 16);
+      a.total = (int64_t)N * H * W * (y_cs / 16);
+      launch(ctx, concat_channels_kernel, dim3((unsigned)ceil_div64(a.total, kThreads)), dim3(kThreads), a, t);
+    } else {
+      ConcatArgs a{};
+      a.y = (int8_t *)y;
+      a.n = nin;
+      a.c = Cc;
+      a.tables = tables;
+      // bytes of one step along the axis, and of everything inside one outer index of the output
+      const int64_t unit = axis == 3 ? y_cs : axis == 2 ? (int64_t)W * y_cs : (int64_t)H * W * y_cs;
+      a.outer = axis == 3 ? (int64_t)N * H : axis == 2 ? N : 1;
+      a.y_stride = unit * out_dims[axis];
+      for (int i = 0; i < nin; ++i) {
+        a.x[i] = (const int8_t *)xs[i];
+        a.stride[i] = unit * in_dims[4 * i + axis];
+        a.start[i + 1] = a.start[i] + unit * in_dims[4 * i + axis] / 16;
+      }
+      a.by_groups = FastDiv(a.start[nin]);
+      a.by_c16 = FastDiv(y_cs / 16);
+      launch(ctx, concat_chunks_kernel, dim3((unsigned)ceil_div64(a.outer * a.start[nin], kThreads)), dim3(kThreads), a, t);
+    }
+    TPUHIP_CHECK_HIP(hipGetLastError());
+    return TPUHIP_OK;
+  }
+
+  int offset = 0;  // running offset along the concat axis
+  for (int i = 0; i < nin; ++i) {
+    const int *dm = in_dims + 4 * i;
+    int8_t table[256];
+    const bool identity = !table_of(i, table);
     const int8_t *tab = identity ? nullptr : table;
     const int8_t *src = (const int8_t *)xs[i];
     int8_t *dst = (int8_t *)y;
