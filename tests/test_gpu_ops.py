@@ -1611,3 +1611,24 @@ def test_concat_of_any_channels_and_tables(ctx, axis, extents, y_cs, tables):
         ctx.concat(ts, axis, yt)
     assert np.array_equal(ctx.to_nchw(yt), want)
     assert not ctx.raw(yt)[..., want.shape[1]:].any()
+
+
+@pytest.mark.parametrize("shape,k,s,pads", [
+    ((1, 12, 9, 8), (9, 8), (1, 1), (0, 0, 0, 0)),          # one group, just beyond the shuffle kernel
+    ((2, 40, 13, 11), (13, 11), (1, 1), (0, 0, 0, 0)),      # three groups of four
+    ((1, 100, 60, 71), (60, 71), (1, 1), (0, 0, 0, 0)),     # seven groups of eight, slices with a remainder
+    ((1, 300, 33, 30), (33, 30), (1, 1), (0, 0, 0, 0)),     # nineteen groups of sixteen: two blocks
+    ((1, 20, 150, 131), (150, 131), (1, 1), (0, 0, 0, 0)),  # 32 slices
+    ((1, 24, 30, 30), (20, 20), (10, 10), (5, 5, 5, 5)),    # several outputs, padding
+])
+def test_pool_avg_large_windows(ctx, shape, k, s, pads):
+    rng = np.random.default_rng(sum(shape))
+    x = rnd_i8(rng, shape)
+    mult, rs = 200, int(np.log2(k[0] * k[1])) + 2           # sums of some sqrt(taps) * 74: most of the int8 range
+    want = O.pool_avg_i8(x, O.make_pool_desc(shape, k, s, pads), rs, mult)
+    d = pool_desc(shape, k, s, pads)
+    xt, yt = ctx.from_nchw(x), ctx.tensor((d.n, d.c, d.oh, d.ow))
+    ctx._ck(ctx.lib.tpuhip_memset(ctx.h, yt.ptr, 0x55, yt.nbytes))
+    ctx.pool_avg(d, xt, yt, mult, rs)
+    assert np.array_equal(ctx.to_nchw(yt), want)
+    assert not ctx.raw(yt)[..., shape[1]:].any()

@@ -18,6 +18,18 @@ int set_error(int status, const char *fmt, ...) {
   return status;
 }
 
+int grow_workspace(tpuhip_ctx *ctx, size_t bytes) {
+  if (ctx->workspace_bytes >= bytes) return TPUHIP_OK;
+  TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
+  TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  if (ctx->workspace) TPUHIP_CHECK_HIP(hipFree(ctx->workspace));
+  ctx->workspace = nullptr;
+  ctx->workspace_bytes = 0;
+  TPUHIP_CHECK_HIP(hipMalloc(&ctx->workspace, bytes));
+  ctx->workspace_bytes = bytes;
+  return TPUHIP_OK;
+}
+
 }  // namespace tpuhip
 
 using namespace tpuhip;

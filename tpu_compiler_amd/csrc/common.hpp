@@ -62,6 +62,9 @@ int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes);
 // waits for what a prepack call has issued, unless a module is being loaded: packed weights may be used from any context
 int prepack_done(tpuhip_ctx *ctx);
 
+// api.hip: makes ctx->workspace at least this large; waits for the stream when it has to be replaced
+int grow_workspace(tpuhip_ctx *ctx, size_t bytes);
+
 int set_error(int status, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 
 #define TPUHIP_CHECK_HIP(expr)                                                          \

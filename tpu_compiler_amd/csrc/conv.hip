@@ -5062,15 +5062,7 @@ int tpuhip_fc_i8(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, v
   FcPlan p;
   if (!fc_splitk_plan(ctx, w, &p)) return run_conv(ctx, w, x, y, PostOps{});   // many rows: the conv path
   if (w->kp / 64 >= kFcOneWaves) return run_fc_one(ctx, w, x, y);              // long K: one launch
-  if (ctx->workspace_bytes < p.bytes) {
-    TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
-    TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    if (ctx->workspace) TPUHIP_CHECK_HIP(hipFree(ctx->workspace));
-    ctx->workspace = nullptr;
-    ctx->workspace_bytes = 0;
-    TPUHIP_CHECK_HIP(hipMalloc(&ctx->workspace, p.bytes));
-    ctx->workspace_bytes = p.bytes;
-  }
+  if (int rc = grow_workspace(ctx, p.bytes)) return rc;
   return run_fc_splitk(ctx, w, x, y, ctx->workspace, p);
 }
 

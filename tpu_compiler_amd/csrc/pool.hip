@@ -17,6 +17,8 @@ struct PoolArgs {
   int n, c16, ih, iw, oh, ow, kh, kw, sh, sw, pt, pl, x_cs, y_cs;
   float mult;       // (float)multiplier
   float inv_pot;    // 2^-rshift
+  FastDiv by_c16, by_ow, by_oh, by_kw;
+  int64_t total;    // 16-channel groups of all output pixels, below 2^31 (each_part)
 };
 
 __device__ __forceinline__ int32_t sb(int32_t word, int i) {
@@ -33,23 +35,18 @@ __device__ __forceinline__ unsigned xcd_block() {
 // PoolingOpKernel INT8 max (core/pooling.cpp:155-157): MKL-DNN pooling_max skips
 // padded positions.
 __global__ __launch_bounds__(256) void pool_max_kernel(PoolArgs a) {
-  const int64_t total = (int64_t)a.n * a.oh * a.ow * a.c16;
-  for (int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x; i < total;
+  for (int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x; i < a.total;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int cg = (int)(i % a.c16);
-    int64_t p = i / a.c16;
-    const int ow = (int)(p % a.ow);
-    p /= a.ow;
-    const int oh = (int)(p % a.oh);
-    const int b = (int)(p / a.oh);
+    uint32_t cg = (uint32_t)i, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
+    const int b = (int)a.by_oh.split(oh);
     int32_t best[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) best[k] = -128;
     for (int kh = 0; kh < a.kh; ++kh) {
-      const int ih = oh * a.sh - a.pt + kh;
+      const int ih = (int)oh * a.sh - a.pt + kh;
       if (ih < 0 || ih >= a.ih) continue;
       for (int kw = 0; kw < a.kw; ++kw) {
-        const int iw = ow * a.sw - a.pl + kw;
+        const int iw = (int)ow * a.sw - a.pl + kw;
         if (iw < 0 || iw >= a.iw) continue;
         const v4i v = *reinterpret_cast<const v4i *>(
             a.x + ((int64_t)(b * a.ih + ih) * a.iw + iw) * a.x_cs + cg * 16);
@@ -76,23 +73,18 @@ __global__ __launch_bounds__(256) void pool_max_kernel(PoolArgs a) {
 // applyMultiplierAndRShiftAndSaturateInt8 without qdm: float product, float
 // quotient by a power of two, floor(f + 0.5), clamp.
 __global__ __launch_bounds__(256) void pool_avg_kernel(PoolArgs a) {
-  const int64_t total = (int64_t)a.n * a.oh * a.ow * a.c16;
-  for (int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x; i < total;
+  for (int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x; i < a.total;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const int cg = (int)(i % a.c16);
-    int64_t p = i / a.c16;
-    const int ow = (int)(p % a.ow);
-    p /= a.ow;
-    const int oh = (int)(p % a.oh);
-    const int b = (int)(p / a.oh);
+    uint32_t cg = (uint32_t)i, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
+    const int b = (int)a.by_oh.split(oh);
     int32_t sum[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) sum[k] = 0;
     for (int kh = 0; kh < a.kh; ++kh) {
-      const int ih = oh * a.sh - a.pt + kh;
+      const int ih = (int)oh * a.sh - a.pt + kh;
       if (ih < 0 || ih >= a.ih) continue;
       for (int kw = 0; kw < a.kw; ++kw) {
-        const int iw = ow * a.sw - a.pl + kw;
+        const int iw = (int)ow * a.sw - a.pl + kw;
         if (iw < 0 || iw >= a.iw) continue;
         const v4i v = *reinterpret_cast<const v4i *>(
             a.x + ((int64_t)(b * a.ih + ih) * a.iw + iw) * a.x_cs + cg * 16);
@@ -118,23 +110,17 @@ __global__ __launch_bounds__(256) void pool_avg_kernel(PoolArgs a) {
   }
 }
 
-// Global / large-window average pooling: LANES lanes share one (pixel, 16-channel
+// Average pooling over windows of 16 to 64 positions: LANES lanes share one (pixel, 16-channel
 // group) output, each sums every LANES-th window position, and the partial sums
 // meet through wave shuffles.  Keeps enough loads in flight when there are few
 // outputs (a 7x7 global pool has 49 taps per output and only n*c/16 outputs).
 template <int LANES>
 __global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
-  const int64_t total = (int64_t)a.n * a.oh * a.ow * a.c16;
   const int64_t gid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
   const int sub = threadIdx.x % LANES;
-  const bool live = gid < total;
-  const int64_t i = live ? gid : 0;
-  const int cg = (int)(i % a.c16);
-  int64_t p = i / a.c16;
-  const int ow = (int)(p % a.ow);
-  p /= a.ow;
-  const int oh = (int)(p % a.oh);
-  const int b = (int)(p / a.oh);
+  const bool live = gid < a.total;
+  uint32_t cg = live ? (uint32_t)gid : 0, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
+  const int b = (int)a.by_oh.split(oh);
   int32_t sum[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) sum[k] = 0;
@@ -142,14 +128,14 @@ __global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
   // up to MAXT window positions of this lane are requested before any is added, so their
   // latencies overlap instead of lining up one behind the other
   constexpr int MAXT = 8;
-  const uint32_t magic_kw = (1u << 20) / (uint32_t)a.kw + 1;   // t / kw == (t * magic) >> 20 for t < 4095
   for (int t0 = sub; t0 < taps; t0 += LANES * MAXT) {
     v4i v[MAXT];
 #pragma unroll
     for (int u = 0; u < MAXT; ++u) {
       const int t = t0 + u * LANES;
-      const int kh = (int)(((uint32_t)t * magic_kw) >> 20), kw = t - kh * a.kw;
-      const int ih = oh * a.sh - a.pt + kh, iw = ow * a.sw - a.pl + kw;
+      uint32_t kw = (uint32_t)t;
+      const int kh = (int)a.by_kw.split(kw);
+      const int ih = (int)oh * a.sh - a.pt + kh, iw = (int)ow * a.sw - a.pl + (int)kw;
       const bool ok = (t < taps) & ((unsigned)ih < (unsigned)a.ih) & ((unsigned)iw < (unsigned)a.iw);
       v[u] = v4i{0, 0, 0, 0};
       if (ok)
@@ -183,6 +169,117 @@ __global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
   }
 }
 
+// Global average of a large map, few outputs with thousands of window positions each: a workgroup takes G 16-channel groups
+// of an output pixel (lanes along the channels, so that a wave reads whole lines) and one slice of the window, 256 / G lanes
+// deep, four positions in flight per lane; the lanes' sums meet in LDS.  With more than one slice the sums go to `parts`
+// [output][slice][channel] and pool_avg_finish_kernel adds them.  A 75 x 75 window over 4 x 120 channels: 113 us with the
+// kernel above (its eight lanes walk 700 positions each, one workgroup), 7 us with 32 slices.
+template <int G>
+__global__ __launch_bounds__(256) void pool_avg_window_kernel(PoolArgs a, int32_t *parts, int slices, int per_slice,
+                                                              FastDiv by_slices, FastDiv by_blocks) {
+  constexpr int P = 256 / G;
+  __shared__ __attribute__((aligned(16))) int32_t lds[256 * 16];
+  uint32_t slice = blockIdx.x, gb = by_slices.split(slice), pix = by_blocks.split(gb);
+  uint32_t ow = pix, oh = a.by_ow.split(ow);
+  const int b = (int)a.by_oh.split(oh);
+  const int cl = threadIdx.x % G, row = threadIdx.x / G, cg = (int)gb * G + cl;
+  int32_t sum[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) sum[k] = 0;
+  const int end = min(((int)slice + 1) * per_slice, a.kh * a.kw);
+  if (cg < a.c16) {
+    for (int t0 = (int)slice * per_slice + row; t0 < end; t0 += 4 * P) {
+      v4i v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = t0 + u * P;
+        uint32_t kw = (uint32_t)t;
+        const int kh = (int)a.by_kw.split(kw);
+        const int ih = (int)oh * a.sh - a.pt + kh, iw = (int)ow * a.sw - a.pl + (int)kw;
+        v[u] = v4i{0, 0, 0, 0};
+        if ((t < end) & ((unsigned)ih < (unsigned)a.ih) & ((unsigned)iw < (unsigned)a.iw))
+          v[u] = *reinterpret_cast<const v4i *>(a.x + ((int64_t)(b * a.ih + ih) * a.iw + iw) * a.x_cs + cg * 16);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) sum[q * 4 + k] += sb(v[u][q], k);
+    }
+  }
+  // P rows of G * 16 sums: each of the 16 / G parts adds 16 rows, then the first adds the parts
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *reinterpret_cast<v4i *>(lds + (row * G + cl) * 16 + q * 4) = v4i{sum[q * 4], sum[q * 4 + 1], sum[q * 4 + 2], sum[q * 4 + 3]};
+  __syncthreads();
+  const int ch = threadIdx.x % (G * 16), part = threadIdx.x / (G * 16);
+  int32_t s = 0;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s += lds[(part * 16 + r) * G * 16 + ch];
+  if constexpr (G < 16) {
+    __syncthreads();
+    lds[threadIdx.x] = s;
+    __syncthreads();
+    if (part) return;
+#pragma unroll
+    for (int r = 1; r < 16 / G; ++r) s += lds[r * G * 16 + ch];
+  }
+  const int c = (int)gb * G * 16 + ch;
+  if (c >= a.c16 * 16) return;
+  if (parts)
+    parts[((int64_t)pix * slices + slice) * (a.c16 * 16) + c] = s;
+  else
+    a.y[(int64_t)pix * a.y_cs + c] = (int8_t)saturate_int8_f(__fmul_rn(__fmul_rn((float)s, a.mult), a.inv_pot));
+}
+
+// adds the slices of pool_avg_window_kernel: 64 channels of an output pixel per workgroup, four threads per channel
+__global__ __launch_bounds__(256) void pool_avg_finish_kernel(PoolArgs a, const int32_t *parts, int slices) {
+  __shared__ int32_t lds[256];
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63), part = threadIdx.x >> 6, all = a.c16 * 16;
+  int32_t s = 0;
+  if (c < all) {
+#pragma unroll 8
+    for (int k = part; k < slices; k += 4) s += parts[((int64_t)blockIdx.y * slices + k) * all + c];
+  }
+  lds[threadIdx.x] = s;
+  __syncthreads();
+  if (part || c >= all) return;
+  s += lds[c % 64 + 64] + lds[c % 64 + 128] + lds[c % 64 + 192];
+  a.y[(int64_t)blockIdx.y * a.y_cs + c] = (int8_t)saturate_int8_f(__fmul_rn(__fmul_rn((float)s, a.mult), a.inv_pot));
+}
+
+// more than 64 window positions for few outputs
+int run_window(tpuhip_ctx *ctx, const PoolArgs &a) {
+  const int G = a.c16 >= 16 ? 16 : a.c16 > 4 ? 8 : a.c16 > 2 ? 4 : a.c16;
+  const int gblocks = (a.c16 + G - 1) / G, taps = a.kh * a.kw;
+  const int64_t pixels = (int64_t)a.n * a.oh * a.ow, blocks = pixels * gblocks;
+  // two workgroups per CU, while every lane keeps four positions; no slices where the grid of the second launch or the
+  // workspace (which is not grown while the stream is being captured) does not reach
+  int64_t slices = std::min<int64_t>(std::min<int64_t>(2 * ctx->num_cu / blocks, taps / (4 * 256 / G)), 32);
+  if (slices < 2 || pixels > 65535) slices = 1;
+  if (slices > 1) {
+    const size_t bytes = (size_t)(pixels * slices * a.c16 * 16) * sizeof(int32_t);
+    if (ctx->workspace_bytes < bytes) {
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+      if (capture != hipStreamCaptureStatusNone) slices = 1;
+      else if (int rc = grow_workspace(ctx, bytes)) return rc;
+    }
+  }
+  int32_t *parts = slices > 1 ? (int32_t *)ctx->workspace : nullptr;
+  const int per_slice = (int)((taps + slices - 1) / slices);
+  auto *kernel = G == 16 ? pool_avg_window_kernel<16> : G == 8 ? pool_avg_window_kernel<8> : G == 4 ? pool_avg_window_kernel<4>
+                 : G == 2 ? pool_avg_window_kernel<2> : pool_avg_window_kernel<1>;
+  launch(ctx, kernel, dim3((unsigned)(blocks * slices)), dim3(256), a, parts, (int)slices, per_slice, FastDiv(slices),
+         FastDiv(gblocks));
+  if (parts)
+    launch(ctx, pool_avg_finish_kernel, dim3((unsigned)((a.c16 + 3) / 4), (unsigned)pixels), dim3(256), a, (const int32_t *)parts,
+           (int)slices);
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
+}
+
 int fill_args(const tpuhip_pool_desc *d, const void *x, void *y, PoolArgs *a) {
   TPUHIP_REQUIRE(d && x && y, "pool: NULL argument");
   TPUHIP_REQUIRE(d->n > 0 && d->c > 0 && d->ih > 0 && d->iw > 0 && d->oh > 0 && d->ow > 0 &&
@@ -202,13 +299,30 @@ int fill_args(const tpuhip_pool_desc *d, const void *x, void *y, PoolArgs *a) {
   a->kh = d->kh; a->kw = d->kw; a->sh = d->sh; a->sw = d->sw;
   a->pt = d->pt; a->pl = d->pl; a->x_cs = d->x_cs; a->y_cs = d->y_cs;
   a->mult = 0.f; a->inv_pot = 1.f;
+  a->by_c16 = FastDiv(a->c16); a->by_ow = FastDiv(a->ow); a->by_oh = FastDiv(a->oh); a->by_kw = FastDiv(a->kw);
+  const int64_t image = (int64_t)a->oh * a->ow * a->c16;
+  TPUHIP_REQUIRE(image < (1ll << 31), "pool: an image of 2^31 output groups or more");
+  return TPUHIP_OK;
+}
+
+// calls fn(args) for runs of images whose output groups a 31-bit index reaches
+template <class F>
+int each_part(PoolArgs a, F fn) {
+  const int64_t image = (int64_t)a.oh * a.ow * a.c16;
+  const int most = (int)std::min<int64_t>(((1ll << 31) - 1) / image, a.n);
+  for (int left = a.n; left > 0; left -= most) {
+    a.n = std::min(left, most);
+    a.total = image * a.n;
+    if (int rc = fn(a)) return rc;
+    a.x += (int64_t)most * a.ih * a.iw * a.x_cs;
+    a.y += (int64_t)most * a.oh * a.ow * a.y_cs;
+  }
   return TPUHIP_OK;
 }
 
 unsigned blocks_for(const PoolArgs &a) {
-  const int64_t total = (int64_t)a.n * a.oh * a.ow * a.c16;
   // a multiple of 8 (see xcd_block)
-  return 8u * (unsigned)std::max<int64_t>(1, std::min<int64_t>((total + 2047) / 2048, 1 << 13));
+  return 8u * (unsigned)std::max<int64_t>(1, std::min<int64_t>((a.total + 2047) / 2048, 1 << 13));
 }
 
 }  // namespace
@@ -219,9 +333,11 @@ int tpuhip_pool_max_i8(tpuhip_ctx *ctx, const tpuhip_pool_desc *d, const void *x
   TPUHIP_REQUIRE(ctx, "pool_max: NULL context");
   PoolArgs a;
   if (int rc = fill_args(d, x, y, &a)) return rc;
-  launch(ctx, pool_max_kernel, dim3(blocks_for(a)), dim3(256), a);
-  TPUHIP_CHECK_HIP(hipGetLastError());
-  return TPUHIP_OK;
+  return each_part(a, [&](const PoolArgs &part) -> int {
+    launch(ctx, pool_max_kernel, dim3(blocks_for(part)), dim3(256), part);
+    TPUHIP_CHECK_HIP(hipGetLastError());
+    return TPUHIP_OK;
+  });
 }
 
 int tpuhip_pool_avg_i8(tpuhip_ctx *ctx, const tpuhip_pool_desc *d, const void *x, void *y,
@@ -233,15 +349,17 @@ int tpuhip_pool_avg_i8(tpuhip_ctx *ctx, const tpuhip_pool_desc *d, const void *x
   TPUHIP_REQUIRE((int64_t)d->kh * d->kw * 128 < (1 << 24), "pool_avg: window too large");
   a.mult = (float)multiplier;
   a.inv_pot = 1.0f / (float)(1 << rshift);
-  const int64_t outputs = (int64_t)a.n * a.oh * a.ow * a.c16;
-  if (d->kh * d->kw >= 16 && outputs < (1 << 16)) {
-    const unsigned blocks = (unsigned)((outputs * 8 + 255) / 256);
-    launch(ctx, pool_avg_split_kernel<8>, dim3(blocks), dim3(256), a);
-  } else {
-    launch(ctx, pool_avg_kernel, dim3(blocks_for(a)), dim3(256), a);
-  }
-  TPUHIP_CHECK_HIP(hipGetLastError());
-  return TPUHIP_OK;
+  return each_part(a, [&](const PoolArgs &part) -> int {
+    // few outputs with many positions each: several lanes share one (65536 outputs fill the chip without)
+    const int taps = part.kh * part.kw;
+    if (taps > 64 && part.total < (1 << 16)) return run_window(ctx, part);
+    if (taps >= 16 && part.total < (1 << 16))
+      launch(ctx, pool_avg_split_kernel<8>, dim3((unsigned)((part.total * 8 + 255) / 256)), dim3(256), part);
+    else
+      launch(ctx, pool_avg_kernel, dim3(blocks_for(part)), dim3(256), part);
+    TPUHIP_CHECK_HIP(hipGetLastError());
+    return TPUHIP_OK;
+  });
 }
 
 }  // extern "C"
