@@ -1632,3 +1632,33 @@ def test_pool_avg_large_windows(ctx, shape, k, s, pads):
     ctx.pool_avg(d, xt, yt, mult, rs)
     assert np.array_equal(ctx.to_nchw(yt), want)
     assert not ctx.raw(yt)[..., shape[1]:].any()
+
+
+@pytest.mark.parametrize("kind,shape,params,out_shape", [
+    ("pad_const", (2, 40, 3, 4), [0, 5, 1, 0, 1, 30, 0, 2], None),      # runs that begin and end inside a group
+    ("pad_const", (1, 32, 3, 4), [0, -3, 1, -1, 0, -1, 2, 0], None),
+    ("pad_edge", (1, 33, 3, 4), [0, 0, 1, 2, 0, 0, 3, 1], None),
+    ("crop", (2, 50, 4, 5), [0, 3, 1, 1, 1, 1, 2, 1], (2, 44, 2, 4)),   # unaligned loads
+    ("crop", (2, 50, 4, 5), [0, 1, 1, 1, 1, 2, 1, 1], (2, 20, 3, 4)),   # every second channel
+    ("reorg", (1, 3, 6, 4), [2], None),                                  # four runs in a group
+    ("reorg", (2, 20, 6, 9), [3], None),
+    ("tile", (2, 21, 2, 3), [1, 4], None), ("tile", (2, 32, 2, 3), [1, 2], None), ("tile", (2, 20, 2, 3), [0, 3], None),
+    ("tile", (2, 20, 2, 3), [2, 2], None),
+    ("reverse", (2, 37, 2, 3), [1], None), ("reverse", (2, 48, 2, 3), [0], None), ("reverse", (2, 48, 2, 3), [3], None),
+    ("shuffle_channel", (2, 50, 3, 4), [5], None), ("shuffle_channel", (1, 34, 3, 4), [17], None),
+    ("shuffle_channel", (1, 20, 3, 4), [1], None),
+    ("depth_to_space", (2, 4, 3, 4), [2, 0], None), ("depth_to_space", (2, 76, 3, 4), [2, 0], None),
+    ("depth_to_space", (1, 256, 2, 3), [2, 0], None), ("depth_to_space", (2, 80, 3, 4), [2, 1], None),
+    ("depth_to_space", (1, 162, 2, 3), [3, 0], None),
+    ("permute", (2, 3, 270, 250), [1, 0, 2, 3], None),                   # more planes than a grid holds
+])
+def test_data_movement_group_edges(ctx, kind, shape, params, out_shape):
+    rng = np.random.default_rng(len(kind) + shape[1])
+    x = rnd_i8(rng, shape)
+    want = O.move_i8(kind, x, params, out_shape)
+    # a channel stride beyond the channels on either side
+    xt, yt = ctx.from_nchw(x, cs=(shape[1] + 15) // 16 * 16 + 16), ctx.tensor(want.shape, cs=(want.shape[1] + 15) // 16 * 16 + 16)
+    ctx._ck(ctx.lib.tpuhip_memset(ctx.h, yt.ptr, 0x55, yt.nbytes))
+    ctx.move(O.MOVE_KINDS.index(kind), xt, yt, params)
+    assert np.array_equal(ctx.to_nchw(yt), want)
+    assert not ctx.raw(yt)[..., want.shape[1]:].any()

@@ -1,10 +1,9 @@
 // Pure data movement on int8 channels-last tensors: Pad, Crop, Permute, Reorg, Tile,
 // Reverse, ShuffleChannel, DepthToSpace, SwapChannel, Dilate, ReflectionPad (core/pad.cpp, crop.cpp, permute.cpp,
 // reorg.cpp, tile.cpp, reverse.cpp, shuffle_channel.cpp, depthtospace.cpp, swap_channel.cpp,
-// dilate.cpp, reflectionpad.cpp).  Each is an index map from
-// the logical (n, c, h, w) of an output element to that of its source; one kernel
-// evaluates the map per element and moves the byte.  A lane produces four consecutive
-// output channels of a pixel (one dword store); pad channels are written as zero.
+// dilate.cpp, reflectionpad.cpp).  Each is an index map from the logical (n, c, h, w) of an
+// output element to that of its source, known at compile time to the kernel that evaluates it;
+// a lane produces 16 consecutive output channels of a pixel, pad channels written as zero.
 #include "common.hpp"
 
 #include <cstring>
@@ -16,140 +15,216 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr int kThreads = 256;
 
+// the index maps; the three that move single channels are at the end
+enum Form {
+  kPadConst, kPadEdge, kCrop, kReorg, kTile, kTileChannel, kReverse, kDilate, kReflectionPad, kDepthDcr,
+  kReverseChannel, kShuffle, kSwap, kStrided
+};
+
 struct MoveArgs {
   const int8_t *x;
   int8_t *y;
-  int kind;
   int in, ic, ih, iw, ics;
   int on, oc, oh, ow, ocs;
   int p[12];
   int fill;        // the byte of an element without a source (0 except for Dilate)
-  int64_t total;   // output pixels * (ocs / 4)
+  FastDiv by_groups, by_ow, by_oh;
+  FastDiv by_a, by_b, by_c;   // what the map divides by
+  uint32_t pix0;   // first output pixel of this launch
+  int64_t total;   // output pixels * (ocs / 16) of this launch, below 2^31
 };
 
-// source of output element o = (n, c, h, w); false: the element has none and takes a.fill
-__device__ __forceinline__ bool source_of(const MoveArgs &a, const int (&o)[4], int (&s)[4]) {
-  switch (a.kind) {
-    case TPUHIP_MOVE_PAD_CONST: {
-      // p[0..3] where the first kept input element lands, p[4..7] its index, p[8..11] end of
-      // the kept input range
-      bool inside = true;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        s[d] = o[d] - a.p[d] + a.p[4 + d];
-        inside = inside && s[d] >= a.p[4 + d] && s[d] < a.p[8 + d];
-      }
-      return inside;
-    }
-    case TPUHIP_MOVE_PAD_EDGE:
-      s[0] = o[0];
-      s[1] = o[1];
-      s[2] = min(max(o[2] - a.p[2], 0), a.ih - 1);
-      s[3] = min(max(o[3] - a.p[3], 0), a.iw - 1);
-      return true;
-    case TPUHIP_MOVE_CROP:
-#pragma unroll
-      for (int d = 0; d < 4; ++d) s[d] = o[d] * a.p[4 + d] + a.p[d];
-      return true;
-    case TPUHIP_MOVE_PERMUTE:
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        // output dimension d is input dimension p[d]
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (a.p[d] == k) s[k] = o[d];
-      }
-      return true;
-    case TPUHIP_MOVE_REORG: {
-      const int st = a.p[0], off = o[1] / a.ic;
-      s[0] = o[0];
-      s[1] = o[1] - off * a.ic;
-      s[2] = o[2] * st + off / st;
-      s[3] = o[3] * st + off % st;
-      return true;
-    }
-    case TPUHIP_MOVE_TILE: {
-      const int dims[4] = {a.in, a.ic, a.ih, a.iw};
-#pragma unroll
-      for (int d = 0; d < 4; ++d) s[d] = a.p[0] == d ? o[d] % dims[d] : o[d];
-      return true;
-    }
-    case TPUHIP_MOVE_REVERSE: {
-      const int dims[4] = {a.in, a.ic, a.ih, a.iw};
-#pragma unroll
-      for (int d = 0; d < 4; ++d) s[d] = a.p[0] == d ? dims[d] - 1 - o[d] : o[d];
-      return true;
-    }
-    case TPUHIP_MOVE_SHUFFLE_CHANNEL: {
-      const int group = a.p[0], col = a.ic / group;
-      s[0] = o[0];
-      s[1] = (o[1] % group) * col + o[1] / group;
-      s[2] = o[2];
-      s[3] = o[3];
-      return true;
-    }
-    case TPUHIP_MOVE_SWAP_CHANNEL:
-      s[0] = o[0];
-      s[1] = o[1];
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (o[1] == k) s[1] = a.p[k];
-      s[2] = o[2];
-      s[3] = o[3];
-      return true;
-    case TPUHIP_MOVE_DILATE: {
-      // p[0] = ins_w + 1, p[1] = ins_h + 1: input elements sit on that grid
-      const int qh = o[2] / a.p[1], qw = o[3] / a.p[0];
-      s[0] = o[0];
-      s[1] = o[1];
-      s[2] = qh;
-      s[3] = qw;
-      return qh * a.p[1] == o[2] && qw * a.p[0] == o[3];
-    }
-    case TPUHIP_MOVE_REFLECTION_PAD: {
-      // p[0] = columns added on the left; mirrored about the first / last column
-      const int j = o[3] - a.p[0];
-      s[0] = o[0];
-      s[1] = o[1];
-      s[2] = o[2];
-      s[3] = j < 0 ? -j : j >= a.iw ? 2 * (a.iw - 1) - j : j;
-      return true;
-    }
-    default: {   // TPUHIP_MOVE_DEPTH_TO_SPACE: p[0] = upscale factor, p[1] = DCR mode
-      const int r = a.p[0];
-      const int dh = o[2] % r, dw = o[3] % r;
-      s[0] = o[0];
-      s[1] = a.p[1] ? (dh * r + dw) * a.oc + o[1] : o[1] * r * r + dh * r + dw;
-      s[2] = o[2] / r;
-      s[3] = o[3] / r;
-      return true;
-    }
+// where output channel c of pixel (n, h, w) comes from, and how many channels from it on, c included, lie one after the other
+// in the source as well (p null: without a source, that many take a.fill).  A source row that ends with the output's ends in
+// zero pad bytes up to a multiple of 16: `left` is then 16.
+struct Run {
+  const int8_t *p;
+  int left;
+};
+
+template <Form F>
+__device__ __forceinline__ Run run_at(const MoveArgs &a, int n, int h, int w, int c) {
+  auto at = [&](int sn, int sc, int sh, int sw) { return a.x + ((int64_t)(sn * a.ih + sh) * a.iw + sw) * a.ics + sc; };
+  if constexpr (F == kPadConst) {
+    // p[0..3] where the first kept input element lands, p[4..7] its index, p[8..11] end of the kept input range
+    const int sn = n - a.p[0] + a.p[4], sc = c - a.p[1] + a.p[5], sh = h - a.p[2] + a.p[6], sw = w - a.p[3] + a.p[7];
+    if (sn < a.p[4] || sn >= a.p[8] || sh < a.p[6] || sh >= a.p[10] || sw < a.p[7] || sw >= a.p[11] || sc >= a.p[9])
+      return {nullptr, a.oc - c};
+    if (sc < a.p[5]) return {nullptr, a.p[5] - sc};
+    return {at(sn, sc, sh, sw), a.ic == a.oc && sc == c ? 16 : a.p[9] - sc};
+  } else if constexpr (F == kPadEdge) {
+    return {at(n, c, min(max(h - a.p[2], 0), a.ih - 1), min(max(w - a.p[3], 0), a.iw - 1)), 16};
+  } else if constexpr (F == kCrop) {   // p[0..3] offsets, p[4..7] steps, the channels' step 1
+    return {at(n * a.p[4] + a.p[0], c + a.p[1], h * a.p[6] + a.p[2], w * a.p[7] + a.p[3]), a.ic == a.oc ? 16 : a.oc - c};
+  } else if constexpr (F == kReorg) {   // by_a: input channels, by_b: the stride p[0]
+    uint32_t sc = (uint32_t)c, dw = a.by_a.split(sc);
+    const int dh = (int)a.by_b.split(dw);
+    return {at(n, (int)sc, h * a.p[0] + dh, w * a.p[0] + (int)dw), a.ic - (int)sc};
+  } else if constexpr (F == kTile) {   // p[0]: the axis; by_a, by_b, by_c: input n, h, w
+    uint32_t sn = (uint32_t)n, sh = (uint32_t)h, sw = (uint32_t)w;
+    a.by_a.split(sn), a.by_b.split(sh), a.by_c.split(sw);
+    return {at((int)sn, c, (int)sh, (int)sw), 16};
+  } else if constexpr (F == kTileChannel) {   // by_a: input channels
+    uint32_t sc = (uint32_t)c;
+    a.by_a.split(sc);
+    return {at(n, (int)sc, h, w), a.ic - (int)sc};
+  } else if constexpr (F == kReverse) {   // p[0]: the axis
+    return {at(a.p[0] == 0 ? a.in - 1 - n : n, c, a.p[0] == 2 ? a.ih - 1 - h : h, a.p[0] == 3 ? a.iw - 1 - w : w), 16};
+  } else if constexpr (F == kDilate) {   // by_a = ins_w + 1, by_b = ins_h + 1: input elements sit on that grid
+    uint32_t rw = (uint32_t)w, rh = (uint32_t)h;
+    const int sw = (int)a.by_a.split(rw), sh = (int)a.by_b.split(rh);
+    if (rw | rh) return {nullptr, a.oc - c};
+    return {at(n, c, sh, sw), 16};
+  } else if constexpr (F == kReflectionPad) {   // p[0]: columns added on the left; mirrored about the first / last column
+    const int j = w - a.p[0];
+    return {at(n, c, h, j < 0 ? -j : j >= a.iw ? 2 * (a.iw - 1) - j : j), 16};
+  } else {   // kDepthDcr, by_a = the upscale factor p[0]
+    uint32_t dw = (uint32_t)w, dh = (uint32_t)h;
+    const int sw = (int)a.by_a.split(dw), sh = (int)a.by_a.split(dh);
+    return {at(n, ((int)dh * a.p[0] + (int)dw) * a.oc + c, sh, sw), a.oc - c};
   }
 }
 
-__global__ __launch_bounds__(kThreads) void move_kernel(MoveArgs a) {
-  const int c4 = a.ocs >> 2;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int cq = (int)(i % c4);
-    const int pix = (int)(i / c4);
-    const int w = pix % a.ow;
-    const int h = (pix / a.ow) % a.oh;
-    const int n = pix / (a.ow * a.oh);
-    uint32_t word = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int c = cq * 4 + b;
-      if (c >= a.oc) continue;
-      const int o[4] = {n, c, h, w};
-      int s[4] = {0, 0, 0, 0};
-      const int8_t v = source_of(a, o, s)
-                           ? a.x[((int64_t)(s[0] * a.ih + s[2]) * a.iw + s[3]) * a.ics + s[1]]
-                           : (int8_t)a.fill;
-      word |= (uint32_t)(uint8_t)v << (8 * b);
-    }
-    *reinterpret_cast<uint32_t *>(a.y + (int64_t)pix * a.ocs + cq * 4) = word;
+// 16 channels of runs: one load at any alignment where they lie in one run, else a dword or a byte at a time
+template <Form F>
+__device__ __forceinline__ v4i group_of_runs(const MoveArgs &a, int n, int h, int w, int c0) {
+  const uint32_t fill = (uint32_t)(uint8_t)a.fill * 0x01010101u;
+  v4i out = {(int)fill, (int)fill, (int)fill, (int)fill};
+  const Run r = run_at<F>(a, n, h, w, c0);
+  if (r.left >= 16) {
+    if (r.p) __builtin_memcpy(&out, r.p, 16);
+    return out;
   }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = c0 + q * 4;
+    uint32_t word = 0;
+    const Run d = c < a.oc ? run_at<F>(a, n, h, w, c) : Run{nullptr, 0};
+    if (d.left >= 4) {
+      word = fill;
+      if (d.p) __builtin_memcpy(&word, d.p, 4);
+    } else {
+      for (int b = 0; b < 4 && c + b < a.oc; ++b) {
+        const Run e = run_at<F>(a, n, h, w, c + b);
+        word |= (e.p ? (uint32_t)(uint8_t)*e.p : fill & 255u) << (8 * b);
+      }
+    }
+    out[q] = (int)word;
+  }
+  return out;
+}
+
+// 16 channels that do not follow each other in the source: byte loads, all in flight, out of lines the wave shares
+template <Form F>
+__device__ __forceinline__ v4i group_of_bytes(const MoveArgs &a, int n, int h, int w, int c0) {
+  v4i out = {0, 0, 0, 0};
+  const int live = min(a.oc - c0, 16);
+  if constexpr (F == kReverseChannel) {
+    const int8_t *end = a.x + ((int64_t)(n * a.ih + h) * a.iw + w) * a.ics + (a.ic - c0);   // behind channel c0's source
+    if (live == 16) {
+      uint32_t t[4];
+      __builtin_memcpy(t, end - 16, 16);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) out[q] = (int)__builtin_bswap32(t[3 - q]);
+      return out;
+    }
+    for (int b = 0; b < live; ++b) out[b >> 2] |= (int)((uint32_t)(uint8_t)end[-1 - b] << (8 * (b & 3)));
+    return out;
+  }
+  const int8_t *row;
+  int64_t at, step = 1;       // kStrided: bytes from one channel's source to the next one's
+  uint32_t g = 0, col = 0;    // kShuffle: group (by_a) and column (p[1] of them) of the channel
+  if constexpr (F == kStrided) {
+    if (a.p[8]) {             // depth to space, CRD; by_a = the factor p[0]
+      uint32_t dw = (uint32_t)w, dh = (uint32_t)h;
+      const int sw = (int)a.by_a.split(dw), sh = (int)a.by_a.split(dh);
+      row = a.x + ((int64_t)(n * a.ih + sh) * a.iw + sw) * a.ics;
+      step = (int64_t)a.p[0] * a.p[0];
+      at = c0 * step + dh * a.p[0] + dw;
+    } else {                  // crop with a step over the channels
+      row = a.x + ((int64_t)((n * a.p[4] + a.p[0]) * a.ih + h * a.p[6] + a.p[2]) * a.iw + w * a.p[7] + a.p[3]) * a.ics;
+      step = a.p[5];
+      at = c0 * step + a.p[1];
+    }
+  } else {
+    row = a.x + ((int64_t)(n * a.ih + h) * a.iw + w) * a.ics;
+    if constexpr (F == kShuffle) {
+      g = (uint32_t)c0;
+      col = a.by_a.split(g);
+    }
+  }
+  uint32_t bytes[16];
+#pragma unroll
+  for (int b = 0; b < 16; ++b) {
+    if constexpr (F == kSwap) {
+      at = 0;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (b == k) at = a.p[k];
+    } else if constexpr (F == kShuffle) {
+      at = (int64_t)g * a.p[1] + col;
+      if (++g == a.by_a.d) g = 0, ++col;
+    }
+    bytes[b] = b < live ? (uint8_t)row[at] : 0;
+    if constexpr (F == kStrided) at += step;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    out[q] = (int)(bytes[q * 4] | bytes[q * 4 + 1] << 8 | bytes[q * 4 + 2] << 16 | bytes[q * 4 + 3] << 24);
+  return out;
+}
+
+// Bound by memory at size and by the launch below: on 4 x 96 x 78 x 66 the maps that a general kernel made byte by byte,
+// with the map chosen at run time, took 7 to 13 us each.
+template <Form F>
+__global__ __launch_bounds__(kThreads) void move_kernel(MoveArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= a.total) return;
+  uint32_t cg = (uint32_t)i;
+  const uint32_t pix = a.pix0 + a.by_groups.split(cg);
+  uint32_t w = pix, h = a.by_ow.split(w);
+  const int n = (int)a.by_oh.split(h), c0 = (int)cg * 16;
+  v4i out = {0, 0, 0, 0};
+  if (c0 < a.oc) {
+    if constexpr (F >= kReverseChannel) out = group_of_bytes<F>(a, n, (int)h, (int)w, c0);
+    else out = group_of_runs<F>(a, n, (int)h, (int)w, c0);
+  }
+  *reinterpret_cast<v4i *>(a.y + (int64_t)pix * a.ocs + c0) = out;
+}
+
+// depth to space by two, CRD: the four bytes of an input dword go to the same channel of four output pixels.  A lane reads 64
+// bytes of an input pixel and writes a group of each of the four.
+__global__ __launch_bounds__(kThreads) void depth_by_two_kernel(MoveArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= a.total) return;
+  uint32_t cg = (uint32_t)i;
+  const uint32_t pix = a.pix0 + a.by_groups.split(cg);   // input pixel
+  uint32_t w = pix;
+  const uint32_t row = a.by_ow.split(w);                 // by_ow: input columns here
+  const int c0 = (int)cg * 16;
+  uint32_t out[4][4] = {};
+  if (c0 < a.oc) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      // channels past the last are the zero pad bytes of the input's row, or lie beyond its stride
+      v4i v = {0, 0, 0, 0};
+      if (c0 * 4 + q * 16 < a.ics) v = *reinterpret_cast<const v4i *>(a.x + (int64_t)pix * a.ics + c0 * 4 + q * 16);
+      // 4 x 4 bytes transposed
+      const uint32_t lo0 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x05010400u),
+                     hi0 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x07030602u),
+                     lo1 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x05010400u),
+                     hi1 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x07030602u);
+      out[0][q] = __builtin_amdgcn_perm(lo1, lo0, 0x05040100u);
+      out[1][q] = __builtin_amdgcn_perm(lo1, lo0, 0x07060302u);
+      out[2][q] = __builtin_amdgcn_perm(hi1, hi0, 0x05040100u);
+      out[3][q] = __builtin_amdgcn_perm(hi1, hi0, 0x07060302u);
+    }
+  }
+  int8_t *to = a.y + ((int64_t)row * 2 * a.ow + 2 * w) * a.ocs + c0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    *reinterpret_cast<v4i *>(to + ((int64_t)(k >> 1) * a.ow + (k & 1)) * a.ocs) =
+        v4i{(int)out[k][0], (int)out[k][1], (int)out[k][2], (int)out[k][3]};
 }
 
 // QuantOp at the graph edges (core/quant.cpp).  The float side is NCHW like the reference's
@@ -373,10 +448,11 @@ __global__ __launch_bounds__(kThreads) void permute_rows_kernel(PermArgs q, int6
 // the channels change places with dimension j: 64 x 64 byte tiles through LDS, dword loads along
 // the input's channels, dword stores along the output's (pad channels of the output written as
 // zero: tile rows past the end of dimension j are zero)
-__global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermArgs q) {
+__global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermArgs q, int64_t plane0) {
   __shared__ __attribute__((aligned(4))) int8_t tile[64][68];
   const int c0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-  const int ia = (int)(blockIdx.z / q.dim[q.b]), ib = (int)(blockIdx.z % q.dim[q.b]);
+  const uint32_t plane = (uint32_t)(plane0 + blockIdx.z);   // below 2^31, as all pixels are
+  const int ia = (int)(plane / (uint32_t)q.dim[q.b]), ib = (int)(plane % (uint32_t)q.dim[q.b]);
   const int8_t *src = q.x + ia * q.S[q.a] + ib * q.S[q.b];
   int8_t *dst = q.y + ia * q.T[q.a] + ib * q.T[q.b];
   const int tq = threadIdx.x & 15, tr = threadIdx.x >> 4;   // 16 dwords per row, 16 rows per pass
@@ -446,9 +522,10 @@ int run_permute(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const void *x, void 
     q.a = rest[0];
     q.b = rest[1];
     const int64_t batch = (int64_t)q.dim[q.a] * q.dim[q.b];
-    TPUHIP_REQUIRE(batch <= 65535, "permute: more than 65535 planes (%lld)", (long long)batch);
-    const dim3 grid((unsigned)((d->y_cs + 63) / 64), (unsigned)((d->ic + 63) / 64), (unsigned)batch);
-    launch(ctx, permute_tile_kernel, grid, dim3(kThreads), q);
+    for (int64_t p0 = 0; p0 < batch; p0 += 65535) {   // as many planes as a grid holds
+      const dim3 grid((unsigned)((d->y_cs + 63) / 64), (unsigned)((d->ic + 63) / 64), (unsigned)std::min<int64_t>(batch - p0, 65535));
+      launch(ctx, permute_tile_kernel, grid, dim3(kThreads), q, p0);
+    }
   }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
@@ -471,6 +548,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
   const int is[4] = {d->in, d->ic, d->ih, d->iw}, os[4] = {d->on, d->oc, d->oh, d->ow};
   const int *p = d->p;
   MoveArgs a{};
+  Form form = kPadConst;
   // every kind: check that the map stays inside the input for every output element
   switch (d->kind) {
     case TPUHIP_MOVE_PAD_CONST:
@@ -492,6 +570,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
                        k, os[k], is[k] + p[k] + p[4 + k]);
         a.p[k] = p[k];
       }
+      form = kPadEdge;
       break;
     case TPUHIP_MOVE_CROP:
       // p[0..3] offsets, p[4..7] steps
@@ -501,6 +580,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
         a.p[k] = p[k];
         a.p[4 + k] = p[4 + k];
       }
+      form = p[5] == 1 ? kCrop : kStrided;
       break;
     case TPUHIP_MOVE_PERMUTE: {
       int seen = 0;
@@ -509,13 +589,9 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
         seen |= 1 << p[k];
         TPUHIP_REQUIRE(os[k] == is[p[k]], "permute: output dimension %d is %d, expected %d", k, os[k],
                        is[p[k]]);
-        a.p[k] = p[k];
       }
       TPUHIP_REQUIRE(seen == 15, "permute: order is not a permutation");
-      // tiled kernels; the per-byte map below serves the other kinds (and permutes with more
-      // planes than a launch grid holds)
-      if (p[1] == 1 || (int64_t)is[0] * is[2] * is[3] / is[p[1]] <= 65535) return run_permute(ctx, d, x, y);
-      break;
+      return run_permute(ctx, d, x, y);
     }
     case TPUHIP_MOVE_REORG:
       TPUHIP_REQUIRE(p[0] >= 1 && is[2] % p[0] == 0 && is[3] % p[0] == 0, "reorg: bad stride %d", p[0]);
@@ -523,24 +599,33 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
                          os[3] == is[3] / p[0],
                      "reorg: output shape does not match");
       a.p[0] = p[0];
+      a.by_a = FastDiv(is[1]);
+      a.by_b = FastDiv(p[0]);
+      form = kReorg;
       break;
     case TPUHIP_MOVE_TILE:
       TPUHIP_REQUIRE(p[0] >= 0 && p[0] < 4 && p[1] >= 1, "tile: bad axis %d / tiles %d", p[0], p[1]);
       for (int k = 0; k < 4; ++k)
         TPUHIP_REQUIRE(os[k] == (k == p[0] ? is[k] * p[1] : is[k]), "tile: output dimension %d is %d", k,
                        os[k]);
-      a.p[0] = p[0];
+      a.by_a = FastDiv(is[p[0] == 1 ? 1 : 0]);
+      a.by_b = FastDiv(is[2]);
+      a.by_c = FastDiv(is[3]);
+      form = p[0] == 1 ? kTileChannel : kTile;
       break;
     case TPUHIP_MOVE_REVERSE:
       TPUHIP_REQUIRE(p[0] >= 0 && p[0] < 4, "reverse: bad axis %d", p[0]);
       for (int k = 0; k < 4; ++k) TPUHIP_REQUIRE(os[k] == is[k], "reverse: shapes differ");
       a.p[0] = p[0];
+      form = p[0] == 1 ? kReverseChannel : kReverse;
       break;
     case TPUHIP_MOVE_SHUFFLE_CHANNEL:
       TPUHIP_REQUIRE(p[0] >= 1 && is[1] % p[0] == 0, "shuffle_channel: wrong group size, c=%d, group=%d",
                      is[1], p[0]);
       for (int k = 0; k < 4; ++k) TPUHIP_REQUIRE(os[k] == is[k], "shuffle_channel: shapes differ");
-      a.p[0] = p[0];
+      a.p[1] = is[1] / p[0];
+      a.by_a = FastDiv(p[0]);
+      form = kShuffle;
       break;
     case TPUHIP_MOVE_SWAP_CHANNEL:
       TPUHIP_REQUIRE(is[1] <= 8, "swap_channel: at most 8 channels (%d)", is[1]);
@@ -549,6 +634,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
         TPUHIP_REQUIRE(p[k] >= 0 && p[k] < is[1], "swap_channel: channel_order[%d] = %d", k, p[k]);
         a.p[k] = p[k];
       }
+      form = kSwap;
       break;
     case TPUHIP_MOVE_DILATE:
       // p[0] = ins_w, p[1] = ins_h, p[2] = fill_constant
@@ -558,9 +644,10 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
                          (int64_t)os[2] == (int64_t)(is[2] - 1) * (p[1] + 1) + 1 &&
                          (int64_t)os[3] == (int64_t)(is[3] - 1) * (p[0] + 1) + 1,
                      "dilate: output shape does not match");
-      a.p[0] = p[0] + 1;
-      a.p[1] = p[1] + 1;
+      a.by_a = FastDiv((int64_t)p[0] + 1);
+      a.by_b = FastDiv((int64_t)p[1] + 1);
       a.fill = p[2];
+      form = kDilate;
       break;
     case TPUHIP_MOVE_REFLECTION_PAD:
       // p[0] / p[1] columns added on the left / right; a mirror image needs a column to mirror
@@ -569,6 +656,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
       TPUHIP_REQUIRE(os[0] == is[0] && os[1] == is[1] && os[2] == is[2] && os[3] == is[3] + p[0] + p[1],
                      "reflection_pad: output shape does not match");
       a.p[0] = p[0];
+      form = kReflectionPad;
       break;
     default:
       TPUHIP_REQUIRE(p[0] >= 1 && is[1] % (p[0] * p[0]) == 0, "depth_to_space: bad upscale factor %d", p[0]);
@@ -576,18 +664,47 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
                          os[3] == is[3] * p[0],
                      "depth_to_space: output shape does not match");
       a.p[0] = p[0];
-      a.p[1] = p[1] ? 1 : 0;
+      a.p[8] = 1;
+      a.by_a = FastDiv(p[0]);
+      form = p[1] ? kDepthDcr : kStrided;
       break;
   }
   TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
   a.x = (const int8_t *)x; a.y = (int8_t *)y;
-  a.kind = d->kind;
   a.in = d->in; a.ic = d->ic; a.ih = d->ih; a.iw = d->iw; a.ics = d->x_cs;
   a.on = d->on; a.oc = d->oc; a.oh = d->oh; a.ow = d->ow; a.ocs = d->y_cs;
-  a.total = (int64_t)d->on * d->oh * d->ow * (d->y_cs / 4);
-  const unsigned blocks = (unsigned)std::max<int64_t>(
-      1, std::min<int64_t>(ceil_div64(a.total, kThreads), (int64_t)ctx->num_cu * 32));
-  launch(ctx, move_kernel, dim3(blocks), dim3(kThreads), a);
+  a.by_groups = FastDiv(d->y_cs / 16);
+  a.by_ow = FastDiv(d->ow);
+  a.by_oh = FastDiv(d->oh);
+  void (*kernel)(MoveArgs) = nullptr;
+  switch (form) {
+    case kPadConst: kernel = move_kernel<kPadConst>; break;
+    case kPadEdge: kernel = move_kernel<kPadEdge>; break;
+    case kCrop: kernel = move_kernel<kCrop>; break;
+    case kReorg: kernel = move_kernel<kReorg>; break;
+    case kTile: kernel = move_kernel<kTile>; break;
+    case kTileChannel: kernel = move_kernel<kTileChannel>; break;
+    case kReverse: kernel = move_kernel<kReverse>; break;
+    case kDilate: kernel = move_kernel<kDilate>; break;
+    case kReflectionPad: kernel = move_kernel<kReflectionPad>; break;
+    case kDepthDcr: kernel = move_kernel<kDepthDcr>; break;
+    case kReverseChannel: kernel = move_kernel<kReverseChannel>; break;
+    case kShuffle: kernel = move_kernel<kShuffle>; break;
+    case kSwap: kernel = move_kernel<kSwap>; break;
+    case kStrided: kernel = move_kernel<kStrided>; break;
+  }
+  int64_t pixels = (int64_t)d->on * d->oh * d->ow;
+  if (d->kind == TPUHIP_MOVE_DEPTH_TO_SPACE && form == kStrided && d->p[0] == 2) {   // the factor in use, a dword per channel
+    kernel = depth_by_two_kernel;
+    pixels = (int64_t)d->in * d->ih * d->iw;
+    a.by_ow = FastDiv(d->iw);
+  }
+  const int64_t most = ((1ll << 31) - 1) / a.by_groups.d;   // as many pixels as the 31-bit index reaches
+  for (int64_t p0 = 0; p0 < pixels; p0 += most) {
+    a.pix0 = (uint32_t)p0;
+    a.total = std::min(most, pixels - p0) * a.by_groups.d;
+    launch(ctx, kernel, dim3((unsigned)ceil_div64(a.total, kThreads)), dim3(kThreads), a);
+  }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }
