@@ -1,6 +1,7 @@
 """ctypes binding of the tpuhip C ABI (include/tpuhip.h) plus small numpy
 conveniences.  Every call goes to the HIP library; nothing here computes."""
 import ctypes as C
+import struct
 
 import numpy as np
 
@@ -343,6 +344,33 @@ class DeviceTensor:
             self.ptr = None
 
 
+# The ops of a Context: a launch takes the library 2.5 us, and ctypes took 1 to 3 us more to build a descriptor, an array of
+# pointers or numpy's view of an address.  These functions take packed bytes instead, through function objects of their own
+# whose pointer arguments all accept them.
+_OPS = ("conv2d_i8", "fc_i8", "fc_batched_i8", "eltwise_add_i8", "move_i8", "binary_i8", "lut_i8", "leaky_relu_i8", "relu_i8",
+        "upsample_nearest_i8", "concat_i8")
+_SCALARS = (C.c_int, C.c_size_t, C.c_uint32)
+_pack_move, _pack_binary = struct.Struct("19i").pack, struct.Struct("21i").pack
+_ZEROS = (0,) * 8
+
+
+def _pack_ints(pack, values):
+    """the bytes of a descriptor of ints; numbers that no int holds wrap as ctypes wraps them"""
+    try:
+        return pack(*values)
+    except struct.error:
+        return b"".join(bytes(C.c_int(v)) for v in values)
+
+
+class _Ops:
+    def __init__(self, lib):
+        for name in _OPS:
+            fn = lib["tpuhip_" + name]     # not the attribute: a new function object
+            fn.restype = C.c_int
+            fn.argtypes = [t if t in _SCALARS else C.c_void_p for t in PROTOTYPES["tpuhip_" + name][1]]
+            setattr(self, name, fn)
+
+
 class Context:
     """One tpuhip context (one HIP stream) with numpy conveniences."""
 
@@ -351,6 +379,7 @@ class Context:
         h = C.c_void_p()
         check(self.lib, self.lib.tpuhip_ctx_create(device, C.byref(h)))
         self.h = h
+        self._ops = _Ops(self.lib)
 
     def close(self):
         if self.h:
@@ -570,8 +599,9 @@ class Context:
         return w.value
 
     def fc(self, w, x, y, noalloc=False):
-        f = self.lib.tpuhip_fc_i8_noalloc if noalloc else self.lib.tpuhip_fc_i8
-        self._ck(f(self.h, w, x.ptr, y.ptr))
+        f = self.lib.tpuhip_fc_i8_noalloc if noalloc else self._ops.fc_i8
+        if rc := f(self.h, w, x.ptr, y.ptr):
+            self._ck(rc)
 
     def fc_batched_prepack(self, desc, filt, bias, mult, rshift):
         filt = np.ascontiguousarray(filt, dtype=np.int8)
@@ -585,7 +615,8 @@ class Context:
         return w.value
 
     def fc_batched(self, w, x, y):
-        self._ck(self.lib.tpuhip_fc_batched_i8(self.h, w, x.ptr, y.ptr))
+        if rc := self._ops.fc_batched_i8(self.h, w, x.ptr, y.ptr):
+            self._ck(rc)
 
     def fc_batched_destroy(self, w):
         self._ck(self.lib.tpuhip_fc_batched_destroy(self.h, w))
@@ -594,8 +625,8 @@ class Context:
         self._ck(self.lib.tpuhip_conv2d_weights_destroy(self.h, w))
 
     def conv(self, w, x, y):
-        self._ck(self.lib.tpuhip_conv2d_i8(self.h, w, x.ptr if hasattr(x, "ptr") else x,
-                                           y.ptr if hasattr(y, "ptr") else y))
+        if rc := self._ops.conv2d_i8(self.h, w, x.ptr if hasattr(x, "ptr") else x, y.ptr if hasattr(y, "ptr") else y):
+            self._ck(rc)
 
     def conv_add(self, w, x, y, add_src, add_out, m_src, m_conv, rshift, do_relu):
         f = FusedAdd(1, int(m_src), int(m_conv), int(rshift), int(do_relu))
@@ -632,15 +663,18 @@ class Context:
         return self.lib.tpuhip_conv2d_algo_name(w).decode()
 
     def eltwise_add(self, xs, mult, rshift, do_relu, y):
-        ptrs = (C.c_void_p * len(xs))(*[t.ptr for t in xs])
-        m = np.ascontiguousarray(mult, dtype=np.int8)
-        self._ck(self.lib.tpuhip_eltwise_add_i8(self.h, ptrs, len(xs), m.ctypes.data, int(rshift),
-                                                int(do_relu), y.ptr, y.nbytes))
+        ptrs = struct.pack("%dP" % len(xs), *[t.ptr for t in xs])
+        m = np.ascontiguousarray(mult, dtype=np.int8).tobytes()
+        if rc := self._ops.eltwise_add_i8(self.h, ptrs, len(xs), m, int(rshift), int(do_relu), y.ptr, y.nbytes):
+            self._ck(rc)
 
     def move(self, kind, x, y, params):
-        p = (C.c_int * 8)(*(list(params) + [0] * (8 - len(params))))
-        d = MoveDesc(kind, *x.shape, *y.shape, x.cs, y.cs, p)
-        self._ck(self.lib.tpuhip_move_i8(self.h, C.byref(d), x.ptr, y.ptr))
+        p = tuple(params)
+        if len(p) > 8:
+            raise IndexError("move: at most 8 parameters (%d)" % len(p))
+        d = _pack_ints(_pack_move, (kind, *x.shape, *y.shape, x.cs, y.cs, *p, *_ZEROS[len(p):]))
+        if rc := self._ops.move_i8(self.h, d, x.ptr, y.ptr):
+            self._ck(rc)
 
     def prelu(self, x, y, slope, rshift_pos, multiplier_pos, rshift_neg):
         c = x.shape[1]
@@ -657,28 +691,28 @@ class Context:
 
     def binary(self, op, x0, x1, y, m0=1, m1=1, multiplier=0, rshift=0, do_relu=False):
         """x0, x1, y: device tensors made by tensor()/from_nchw() (logical NCHW shapes)"""
-        s0, s1, so = x0.shape, x1.shape, y.shape
-        d = BinaryDesc(op, so[0], so[1], so[2], so[3], s0[0], s0[1], s0[2], s0[3],
-                       s1[0], s1[1], s1[2], s1[3], int(m0), int(m1), int(multiplier), int(rshift),
-                       int(do_relu), x0.cs, x1.cs, y.cs)
-        self._ck(self.lib.tpuhip_binary_i8(self.h, C.byref(d), x0.ptr, x1.ptr, y.ptr))
+        d = _pack_ints(_pack_binary, (op, *y.shape, *x0.shape, *x1.shape, int(m0), int(m1), int(multiplier), int(rshift),
+                                      int(do_relu), x0.cs, x1.cs, y.cs))
+        if rc := self._ops.binary_i8(self.h, d, x0.ptr, x1.ptr, y.ptr):
+            self._ck(rc)
 
     def pool_max(self, d, x, y):
-        self._ck(self.lib.tpuhip_pool_max_i8(self.h, C.byref(d), x.ptr, y.ptr))
+        if rc := self.lib.tpuhip_pool_max_i8(self.h, C.byref(d), x.ptr, y.ptr):
+            self._ck(rc)
 
     def pool_avg(self, d, x, y, mult, rshift):
-        self._ck(self.lib.tpuhip_pool_avg_i8(self.h, C.byref(d), x.ptr, y.ptr, int(mult),
-                                             int(rshift)))
+        if rc := self.lib.tpuhip_pool_avg_i8(self.h, C.byref(d), x.ptr, y.ptr, int(mult), int(rshift)):
+            self._ck(rc)
 
     def lut(self, x, y, table):
         t = np.ascontiguousarray(table, dtype=np.int8)
         assert t.size == 256
-        self._ck(self.lib.tpuhip_lut_i8(self.h, x.ptr, y.ptr, t.ctypes.data, x.pixels,
-                                        x.shape[1], x.cs))
+        if rc := self._ops.lut_i8(self.h, x.ptr, y.ptr, t.tobytes(), x.pixels, x.shape[1], x.cs):
+            self._ck(rc)
 
     def leaky_relu(self, x, y, rp, mp, rn, mn):
-        self._ck(self.lib.tpuhip_leaky_relu_i8(self.h, x.ptr, y.ptr, x.pixels, x.shape[1], x.cs,
-                                               int(rp), int(mp), int(rn), int(mn)))
+        if rc := self._ops.leaky_relu_i8(self.h, x.ptr, y.ptr, x.pixels, x.shape[1], x.cs, int(rp), int(mp), int(rn), int(mn)):
+            self._ck(rc)
 
     def leaky_relu_table(self, rp, mp, rn, mn):
         t = np.empty(256, np.int8)
@@ -693,20 +727,20 @@ class Context:
         return t
 
     def relu(self, x, y):
-        self._ck(self.lib.tpuhip_relu_i8(self.h, x.ptr, y.ptr, x.nbytes))
+        if rc := self._ops.relu_i8(self.h, x.ptr, y.ptr, x.nbytes):
+            self._ck(rc)
 
     def upsample(self, x, y, sh, sw):
         n, c, h, w = x.shape
-        self._ck(self.lib.tpuhip_upsample_nearest_i8(self.h, x.ptr, y.ptr, n, c, h, w, sh, sw,
-                                                     x.cs, y.cs))
+        if rc := self._ops.upsample_nearest_i8(self.h, x.ptr, y.ptr, n, c, h, w, sh, sw, x.cs, y.cs):
+            self._ck(rc)
 
     def concat(self, xs, axis, y, rshift=None, mult=None, do_relu=False):
-        ptrs = (C.c_void_p * len(xs))(*[t.ptr for t in xs])
-        dims = np.ascontiguousarray(np.array([t.shape for t in xs], dtype=np.int32))
-        cs = np.ascontiguousarray(np.array([t.cs for t in xs], dtype=np.int32))
-        r = None if rshift is None else np.ascontiguousarray(rshift, dtype=np.uint32)
-        m = None if mult is None else np.ascontiguousarray(mult, dtype=np.uint32)
-        self._ck(self.lib.tpuhip_concat_i8(
-            self.h, ptrs, len(xs), dims.ctypes.data, cs.ctypes.data, axis,
-            None if r is None else r.ctypes.data, None if m is None else m.ctypes.data,
-            int(do_relu), y.ptr, y.cs))
+        n = len(xs)
+        ptrs = struct.pack("%dP" % n, *[t.ptr for t in xs])
+        dims = struct.pack("%di" % (4 * n), *[v for t in xs for v in t.shape])
+        cs = struct.pack("%di" % n, *[t.cs for t in xs])
+        r = None if rshift is None else np.ascontiguousarray(rshift, dtype=np.uint32).tobytes()
+        m = None if mult is None else np.ascontiguousarray(mult, dtype=np.uint32).tobytes()
+        if rc := self._ops.concat_i8(self.h, ptrs, n, dims, cs, axis, r, m, int(do_relu), y.ptr, y.cs):
+            self._ck(rc)
