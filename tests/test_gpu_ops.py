@@ -1662,3 +1662,15 @@ def test_data_movement_group_edges(ctx, kind, shape, params, out_shape):
     ctx.move(O.MOVE_KINDS.index(kind), xt, yt, params)
     assert np.array_equal(ctx.to_nchw(yt), want)
     assert not ctx.raw(yt)[..., want.shape[1]:].any()
+
+
+@pytest.mark.parametrize("bh,bl,m,k,n,lt,ot,relu", [
+    (1, 3, 33, 520, 31, 0, 0, False),    # two passes through LDS, rows and columns by a tile's edge
+    (2, 3, 31, 33, 300, 1, 1, True),     # two blocks of columns; a multiplier per product that the result's order mixes
+    (1, 2, 64, 1030, 65, 0, 0, True),
+    (2, 5, 40, 72, 257, 1, 0, False),    # rows contiguous in, strided out
+    (2, 5, 40, 72, 129, 0, 1, False),    # and the other way round
+    (3, 17, 5, 8, 8, 0, 0, False),       # channels in the middle: byte by byte on both sides
+])
+def test_fully_connected_batched_tile_edges(ctx, bh, bl, m, k, n, lt, ot, relu):
+    test_fully_connected_batched_and_transposed(ctx, bh, bl, m, k, n, lt, ot, relu)
