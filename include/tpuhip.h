@@ -556,6 +556,9 @@ int tpuhip_module_set_tensor_i8(tpuhip_module *m, const char *name, const int8_t
                                 int bidx);
 int tpuhip_module_get_tensor(tpuhip_module *m, const char *name, float *dst, size_t count,
                              int bidx);
+/* n tensors in one go: their transfers and host passes overlap */
+int tpuhip_module_get_tensors(tpuhip_module *m, int n, const char *const *names, float *const *dsts,
+                              const size_t *counts, int bidx);
 /* same tensor as int8 NCHW, without the float detour */
 int tpuhip_module_get_tensor_i8(tpuhip_module *m, const char *name, int8_t *dst, size_t count,
                                 int bidx);

@@ -54,6 +54,8 @@ struct WeightData {
   float at(size_t i) const { return data.at(i); }
 };
 
+struct HostRead;
+
 // An activation tensor: `batch` slots of one int8 channels-last image set in HBM -- or, at
 // the graph edges only (an fp32 input before its QuantOp, the result of a dequantising
 // QuantOp), of float NCHW data like the reference's tensors.
@@ -81,6 +83,9 @@ public:
   void read(float *dst, size_t num, int32_t bidx) const;
   // slot bidx as int8 NCHW host data (no float detour)
   void read_i8(int8_t *dst, size_t num, int32_t bidx) const;
+  // slots bidx of several tensors of one context at once, float-stored (see read); their transfers overlap
+  static void read_all(const std::vector<const TensorData *> &tensors, const std::vector<float *> &dsts,
+                       const std::vector<size_t> &nums, int32_t bidx);
   // lays the tensor out again with another channel stride (4 for a tensor of at most 4 channels whose
   // only readers take one dword per pixel, else a multiple of 16); the contents are lost
   void set_channel_stride(int new_cs);
@@ -95,6 +100,7 @@ public:
   tpuhip_ctx *ctx() const { return ctx_; }
 
 private:
+  HostRead host_read(void *dst, size_t num, int32_t bidx, bool bytes) const;
   tpuhip_ctx *ctx_;
   size_t size_;
   void *slot(int32_t bidx) const { return (char *)base_ + slot_bytes() * (size_t)bidx; }
@@ -623,6 +629,9 @@ public:
   std::shared_ptr<std::vector<float>> getTensor(std::string &name, int32_t bidx);
   void getTensor(const std::string &name, float *dst, size_t num, int32_t bidx);
   void getTensorI8(const std::string &name, int8_t *dst, size_t num, int32_t bidx);
+  // several tensors in one go: their transfers and host passes overlap
+  void getTensors(const std::vector<std::string> &names, const std::vector<float *> &dsts,
+                  const std::vector<size_t> &nums, int32_t bidx);
   std::vector<int64_t> getTensorShape(std::string &name);
   std::string getDataType(std::string &name);
   // the reference's updateWeightMap reads every tpu.load_weight from the npz

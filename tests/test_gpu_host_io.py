@@ -93,3 +93,28 @@ def test_round_trip_of_fp32_edges(shape):
     m.invoke()
     assert np.array_equal(m.get_tensor("x"), x) and np.array_equal(m.get_tensor("y"), x)
     m.close()
+
+
+# together in one round of the staging buffer; several rounds; a tensor larger than the buffer among small ones
+@pytest.mark.parametrize("shapes", [[(1, 3, 20, 31), (2, 1000, 1, 1)], [(4, 70, 61, 67), (1, 255, 13, 13), (3, 129, 130, 131)],
+                                    [(2, 17, 9, 9), (5, 64, 331, 333), (1, 5, 300, 1)]])
+def test_all_tensors_at_once(shapes):
+    g = graphs.Graph("io", 1)
+    for i, s in enumerate(shapes):
+        g.add(graphs.Op("tpu.input", "x%d" % i, [], s))
+    for i, s in enumerate(shapes):
+        g.add(graphs.Op("tpu.relu", "y%d" % i, ["x%d" % i], s))
+    g.outputs = ["y%d" % i for i in range(len(shapes))]
+    m = module()
+    m.load(g)
+    held = []
+    for k in range(3):      # results that are still held keep their values
+        xs = [np.random.default_rng(k + i).integers(-128, 128, s).astype(np.int8) for i, s in enumerate(shapes)]
+        got = m.run(np.concatenate([x.reshape(-1) for x in xs]))
+        held.append((xs, got, m.get_all_tensor()))
+    for xs, got, every in held:
+        assert sorted(every) == sorted(m.tensor_names())
+        for i, x in enumerate(xs):
+            assert np.array_equal(got["y%d" % i], np.maximum(x, 0)) and np.array_equal(every["y%d" % i], np.maximum(x, 0))
+            assert np.array_equal(every["x%d" % i], x)
+    m.close()

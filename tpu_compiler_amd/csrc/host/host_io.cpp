@@ -77,8 +77,16 @@ __attribute__((target("avx2"))) bool to_bytes_avx2(const float *src, int8_t *dst
   return _mm256_movemask_ps(bad) != 0 || tail;
 }
 
-__attribute__((target("avx512f"))) void to_floats_avx512(const int8_t *src, float *dst, size_t n, bool is_unsigned) {
+__attribute__((target("avx512f"))) void to_floats_avx512(const int8_t *src, float *dst, size_t n, bool is_unsigned, bool past_caches) {
   size_t i = 0;
+  if (past_caches) {
+    for (; i < n && ((uintptr_t)(dst + i) & 63); ++i) dst[i] = is_unsigned ? (float)(uint8_t)src[i] : (float)src[i];
+    for (; i + 16 <= n; i += 16) {
+      const __m128i b = _mm_loadu_si128((const __m128i *)(src + i));
+      _mm512_stream_ps(dst + i, _mm512_cvtepi32_ps(is_unsigned ? _mm512_cvtepu8_epi32(b) : _mm512_cvtepi8_epi32(b)));
+    }
+    _mm_sfence();
+  }
   for (; i + 16 <= n; i += 16) {
     const __m128i b = _mm_loadu_si128((const __m128i *)(src + i));
     _mm512_storeu_ps(dst + i, _mm512_cvtepi32_ps(is_unsigned ? _mm512_cvtepu8_epi32(b) : _mm512_cvtepi8_epi32(b)));
@@ -114,9 +122,9 @@ bool floats_to_bytes(const float *src, int8_t *dst, size_t n, bool is_unsigned) 
   return to_bytes_plain(src, dst, n, lo, hi);
 }
 
-void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned) {
+void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned, bool past_caches) {
 #ifdef TPUHIP_X86
-  if (simd_level() == 2) return to_floats_avx512(src, dst, n, is_unsigned);
+  if (simd_level() == 2) return to_floats_avx512(src, dst, n, is_unsigned, past_caches);
   if (simd_level() == 1) return to_floats_avx2(src, dst, n, is_unsigned);
 #endif
   for (size_t i = 0; i < n; ++i) dst[i] = is_unsigned ? (float)(uint8_t)src[i] : (float)src[i];
@@ -374,83 +382,152 @@ int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const vo
   return tpuhip_nchw_to_nhwc_i8(ctx, land, dst, t.n, t.c, t.h, t.w, t.cs);
 }
 
-int device_to_host(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst) {
-  const size_t count = (size_t)t.n * t.c * t.h * t.w;
-  const size_t per = stage_size(kind), total = count * per;
+// What a round of device_to_host() does: `Fetch`es fill the staging buffer, `Part`s are passed on to the callers' memory.
+namespace {
+
+constexpr size_t kSpan = 8 * kPiece;            // bytes of the staging buffer behind one event
+constexpr size_t kPastCaches = 16 << 20;        // host bytes of a call from which its floats go past the caches: half of the
+                                                // last level; they would evict each other, and the stores read nothing
+struct Part {
+  const HostRead *r;
+  size_t first, count;      // elements
+  size_t at;                // byte of the staging buffer
+  size_t span;              // there when this many spans have arrived
+};
+
+void pass_part(const Part &p, const int8_t *stage, bool past_caches) {
+  const HostRead &r = *p.r;
+  char *to = (char *)r.dst + p.first * host_size(r.kind);
+  if (r.kind == HostKind::kFloatStored)
+    bytes_to_floats(stage + p.at, (float *)to, p.count, r.t.is_unsigned, past_caches);
+  else
+    memcpy(to, stage + p.at, p.count * stage_size(r.kind));
+}
+
+size_t elements(const HostRead &r) { return (size_t)r.t.n * r.t.c * r.t.h * r.t.w; }
+
+}  // namespace
+
+// Tensors of up to two pieces are laid out straight into the staging buffer; the dense form of larger ones is made on the
+// device and comes over in spans.  An event stands behind each span, and behind small tensors that make one up together;
+// the host pass of a span runs on several threads while the next ones are laid out and on the bus, and for small tensors
+// while the launches of those behind them are still being issued.
+int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
+  size_t total = 0, host_total = 0, largest = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const size_t count = elements(reads[i]), bytes = count * stage_size(reads[i].kind);
+    total += (bytes + 63) / 64 * 64;
+    host_total += count * host_size(reads[i].kind);
+    if (bytes > 2 * kPiece && reads[i].kind != HostKind::kFloats) largest = std::max(largest, bytes);
+  }
   if (int rc = stage_ready(ctx, total)) return rc;
+  if (largest)
+    if (int rc = landing_ready(ctx, largest)) return rc;
   int8_t *stage = (int8_t *)ctx->stage;
-  auto pass = [&](size_t first, size_t elements, const int8_t *from) {
-    char *to = (char *)dst + first * host_size(kind);
-    if (kind == HostKind::kFloatStored)
-      bytes_to_floats(from, (float *)to, elements, t.is_unsigned);
-    else
-      memcpy(to, from, elements * per);
+  const size_t room = ctx->stage_bytes;
+  const bool past_caches = host_total >= kPastCaches;
+  auto lay_out = [&](const HostRead &r, void *to) {
+    return tpuhip_nhwc_to_nchw_i8(ctx, r.src, to, r.t.n, r.t.c, r.t.h, r.t.w, r.t.cs);
   };
-  // the host bytes are what the caller's memory costs (fresh pages above all), so they decide on the threads
-  const bool alone = count * host_size(kind) <= kAlone;
-  if (total <= ctx->stage_bytes && (alone || total <= 2 * kPiece)) {
-    const int rc = kind == HostKind::kFloats ? stage_copy(ctx, src, stage, total)
-                                             : tpuhip_nhwc_to_nchw_i8(ctx, src, stage, t.n, t.c, t.h, t.w, t.cs);
+  if (n == 1 && host_total <= kAlone) {   // done before a worker has woken
+    const int rc = reads->kind == HostKind::kFloats ? stage_copy(ctx, reads->src, stage, total) : lay_out(*reads, stage);
     if (rc) return rc;
     TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    if (alone) {
-      pass(0, count, stage);
-      return TPUHIP_OK;
-    }
-    auto job = std::make_shared<HostJob>();
-    const size_t grain = kPiece / host_size(kind);
-    job->pieces = (count + grain - 1) / grain;
-    job->piece = [&](size_t i) { pass(i * grain, std::min(grain, count - i * grain), stage + i * grain * per); };
-    const bool shared = HostWorkers::get().enter(job);
-    finish_job(*job);
-    if (shared) HostWorkers::get().leave();
+    pass_part(Part{reads, 0, elements(*reads), 0, 0}, stage, false);
     return TPUHIP_OK;
   }
-  // The dense form is made on the device and comes over in spans of eight pieces, an event behind each; the host pass
-  // of a span runs while the next ones are on the bus.
-  const void *dense = src;
-  if (kind != HostKind::kFloats) {
-    if (int rc = landing_ready(ctx, total)) return rc;
-    if (int rc = tpuhip_nhwc_to_nchw_i8(ctx, src, ctx->landing, t.n, t.c, t.h, t.w, t.cs)) return rc;
-    dense = ctx->landing;
-  }
-  constexpr size_t kSpan = 8 * kPiece;
-  for (size_t part = 0; part < total; part += ctx->stage_bytes) {
-    const size_t bytes = std::min(total - part, ctx->stage_bytes);
-    const size_t spans = (bytes + kSpan - 1) / kSpan;
+
+  struct Fetch {
+    const HostRead *r;
+    size_t from, bytes, at;   // bytes [from, from + bytes) of the dense form -> byte `at` of the buffer
+    bool whole, closes;       // laid out in one launch; an event behind it
+  };
+  std::vector<Fetch> fetches;
+  std::vector<Part> parts;
+  for (size_t i = 0, done = 0; i < n;) {
+    // a round: what fits the buffer
+    fetches.clear();
+    parts.clear();
+    size_t at = 0, spans = 0, open = 0;   // open: bytes fetched behind the last event
+    while (i < n) {
+      const HostRead &r = reads[i];
+      const size_t per = stage_size(r.kind), bytes = elements(r) * per;
+      if (at && bytes > room - at && bytes <= room) break;   // in parts only where a round of its own does not help
+      const bool whole = bytes <= 2 * kPiece;
+      while (done < bytes && at < room) {
+        const size_t len = std::min({bytes - done, room - at, kSpan});
+        fetches.push_back({&r, done, len, at, whole, false});
+        open += len;
+        for (size_t p = 0; p < len; p += kPiece) {
+          const size_t l = std::min(kPiece, len - p);
+          parts.push_back({&r, (done + p) / per, l / per, at + p, spans});
+        }
+        if (open >= kSpan / 2) {
+          fetches.back().closes = true;
+          ++spans;
+          open = 0;
+        }
+        done += len;
+        at += (len + 63) / 64 * 64;
+      }
+      if (done < bytes) break;
+      ++i;
+      done = 0;
+    }
+    if (open) {
+      fetches.back().closes = true;
+      ++spans;
+    }
     while (ctx->stage_events.size() < spans) {
       hipEvent_t e;
       TPUHIP_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       ctx->stage_events.push_back(e);
     }
-    for (size_t s = 0; s < spans; ++s) {
-      const size_t at = s * kSpan;
-      if (int rc = stage_copy(ctx, (const char *)dense + part + at, stage + at, std::min(kSpan, bytes - at))) return rc;
-      TPUHIP_CHECK_HIP(hipEventRecord(ctx->stage_events[s], ctx->stream));
-    }
     auto job = std::make_shared<HostJob>();
-    job->pieces = (bytes + kPiece - 1) / kPiece;
+    job->pieces = parts.size();
     std::atomic<size_t> arrived{0};     // spans that are in the buffer
     std::atomic<bool> lost{false};      // the device failed: nothing more arrives
-    job->piece = [&, part, bytes](size_t i) {
-      const size_t at = i * kPiece, len = std::min(kPiece, bytes - at);
-      while (arrived.load(std::memory_order_acquire) <= at / kSpan) {
+    job->piece = [&](size_t k) {
+      const Part &p = parts[k];
+      while (arrived.load(std::memory_order_acquire) <= p.span) {
         if (lost.load(std::memory_order_relaxed)) return;
         std::this_thread::yield();
       }
-      pass((part + at) / per, len / per, stage + at);
+      pass_part(p, stage, past_caches);
     };
     HostWorkers &workers = HostWorkers::get();
-    const bool shared = workers.enter(job);
-    hipError_t e = hipSuccess;
-    for (size_t s = 0; s < spans && e == hipSuccess; ++s) {
-      e = hipEventSynchronize(ctx->stage_events[s]);
-      if (e == hipSuccess) arrived.store(s + 1, std::memory_order_release);
+    const bool shared = parts.size() > 1 && workers.enter(job);
+    int rc = TPUHIP_OK;
+    size_t recorded = 0, there = 0;
+    ctx->stage_busy = true;
+    auto hip = [&](hipError_t e, const char *what) {
+      if (!rc && e != hipSuccess) rc = set_error(TPUHIP_ERR_HIP, "%s failed: %s", what, hipGetErrorString(e));
+    };
+    for (const Fetch &f : fetches) {
+      if (f.whole) {
+        rc = f.r->kind == HostKind::kFloats ? stage_copy(ctx, f.r->src, stage + f.at, f.bytes) : lay_out(*f.r, stage + f.at);
+      } else {
+        const void *dense = f.r->src;
+        if (f.r->kind != HostKind::kFloats) {
+          dense = ctx->landing;
+          if (f.from == 0) rc = lay_out(*f.r, ctx->landing);
+        }
+        if (!rc) rc = stage_copy(ctx, (const char *)dense + f.from, stage + f.at, f.bytes);
+      }
+      if (!rc && f.closes) hip(hipEventRecord(ctx->stage_events[recorded++], ctx->stream), "hipEventRecord");
+      if (rc) break;
+      while (there < recorded && hipEventQuery(ctx->stage_events[there]) == hipSuccess)
+        arrived.store(++there, std::memory_order_release);
     }
-    if (e != hipSuccess) lost.store(true);
+    while (!rc && there < spans) {
+      hip(hipEventSynchronize(ctx->stage_events[there]), "hipEventSynchronize");
+      if (!rc) arrived.store(++there, std::memory_order_release);
+    }
+    if (rc) lost.store(true);
     finish_job(*job);
     if (shared) workers.leave();
-    TPUHIP_CHECK_HIP(e);
+    if (rc) return rc;
+    ctx->stage_busy = false;
   }
   return TPUHIP_OK;
 }

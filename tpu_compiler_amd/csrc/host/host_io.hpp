@@ -18,8 +18,8 @@ namespace tpuhip {
 // n floats -> int8; the return value tells whether one of them is no integer in [-128, 127] (is_unsigned: [0, 255],
 // stored as the byte)
 bool floats_to_bytes(const float *src, int8_t *dst, size_t n, bool is_unsigned);
-// n int8 (is_unsigned: uint8) -> floats
-void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned);
+// n int8 (is_unsigned: uint8) -> floats; past_caches: with stores that leave the caches alone
+void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned, bool past_caches = false);
 
 // piece(0) .. piece(n - 1), on this thread and a few others; returns when all are done.  Pieces throw nothing.
 void parallel_pieces(size_t n, const std::function<void(size_t)> &piece);
@@ -35,6 +35,13 @@ struct HostTensor {
 // host -> device, issued to the context's stream; the caller's buffer may be reused on return.  *bad: an element of a
 // float-stored tensor is no integer of the byte range (nothing has been written to dst then).
 int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst, bool *bad);
-// device -> host; waits for the work in front of it
-int device_to_host(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst);
+// device -> host, several tensors in one go; waits for the work in front of it
+struct HostRead {
+  HostTensor t;
+  HostKind kind;
+  const void *src;
+  void *dst;
+};
+int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n);
+
 }  // namespace tpuhip

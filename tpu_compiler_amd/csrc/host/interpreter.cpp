@@ -488,6 +488,17 @@ void ModuleInterpreter::getTensorI8(const std::string &name, int8_t *dst, size_t
   it->second->read_i8(dst, num, bidx);
 }
 
+void ModuleInterpreter::getTensors(const std::vector<std::string> &names, const std::vector<float *> &dsts,
+                                   const std::vector<size_t> &nums, int32_t bidx) {
+  std::vector<const TensorData *> tensors;
+  for (auto &name : names) {
+    auto it = activationMapping.find(name);
+    if (it == activationMapping.end()) fail(" Not Find Op name: " + name + " tensor");
+    tensors.push_back(it->second.get());
+  }
+  TensorData::read_all(tensors, dsts, nums, bidx);
+}
+
 std::vector<int64_t> ModuleInterpreter::getTensorShape(std::string &name) {
   auto it = valueMapping.shapes.find(name);
   if (it == valueMapping.shapes.end()) fail(" Not Find Op name: " + name + " tensor");

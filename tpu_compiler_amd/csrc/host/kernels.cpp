@@ -156,15 +156,28 @@ void TensorData::assign_i8(const int8_t *first, size_t num, int32_t bidx) {
      "TensorData::assign_i8");
 }
 
-void TensorData::read(float *dst, size_t num, int32_t bidx) const {
+HostRead TensorData::host_read(void *dst, size_t num, int32_t bidx, bool bytes) const {
+  const std::string what = bytes ? "TensorData::read_i8" : "TensorData::tensor";
   if (!materialized)
-    fail("TensorData::tensor: this tensor is fused into its consumer and never written "
+    fail(what + ": this tensor is fused into its consumer and never written "
          "(load the module with keep_all_tensors to read it)");
-  if (num != size_) fail("TensorData::tensor: size mismatch");
-  if (bidx < 0 || bidx >= batch) fail("TensorData::tensor: slot out of range");
-  ck(device_to_host(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, f32 ? HostKind::kFloats : HostKind::kFloatStored,
-                    slot(bidx), dst),
-     "TensorData::tensor");
+  if (bytes && f32) fail(what + ": this tensor holds fp32 data");
+  if (num != size_) fail(what + ": size mismatch");
+  if (bidx < 0 || bidx >= batch) fail(what + ": slot out of range");
+  return HostRead{HostTensor{n, c, h, w, cs, is_unsigned},
+                  bytes ? HostKind::kBytes : f32 ? HostKind::kFloats : HostKind::kFloatStored, slot(bidx), dst};
+}
+
+void TensorData::read(float *dst, size_t num, int32_t bidx) const {
+  const HostRead r = host_read(dst, num, bidx, false);
+  ck(device_to_host(ctx_, &r, 1), "TensorData::tensor");
+}
+
+void TensorData::read_all(const std::vector<const TensorData *> &tensors, const std::vector<float *> &dsts,
+                          const std::vector<size_t> &nums, int32_t bidx) {
+  std::vector<HostRead> reads;
+  for (size_t i = 0; i < tensors.size(); ++i) reads.push_back(tensors[i]->host_read(dsts[i], nums[i], bidx, false));
+  if (!reads.empty()) ck(device_to_host(tensors[0]->ctx_, reads.data(), reads.size()), "TensorData::tensor");
 }
 
 std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
@@ -174,13 +187,8 @@ std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
 }
 
 void TensorData::read_i8(int8_t *dst, size_t num, int32_t bidx) const {
-  if (!materialized)
-    fail("TensorData::read_i8: this tensor is fused into its consumer and never written "
-         "(load the module with keep_all_tensors to read it)");
-  if (f32) fail("TensorData::read_i8: this tensor holds fp32 data");
-  if (num != size_) fail("TensorData::read_i8: size mismatch");
-  if (bidx < 0 || bidx >= batch) fail("TensorData::read_i8: slot out of range");
-  ck(device_to_host(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, HostKind::kBytes, slot(bidx), dst), "TensorData::read_i8");
+  const HostRead r = host_read(dst, num, bidx, true);
+  ck(device_to_host(ctx_, &r, 1), "TensorData::read_i8");
 }
 
 // ---------------------------------------------------------------------------

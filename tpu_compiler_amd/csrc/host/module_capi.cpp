@@ -147,6 +147,17 @@ int tpuhip_module_get_tensor_i8(tpuhip_module *m, const char *name, int8_t *dst,
   })
 }
 
+int tpuhip_module_get_tensors(tpuhip_module *m, int n, const char *const *names, float *const *dsts, const size_t *counts,
+                              int bidx) {
+  GUARD(m, {
+    if (n < 0 || (n && (!names || !dsts || !counts))) throw std::runtime_error("get_tensors: NULL argument");
+    for (int i = 0; i < n; ++i)
+      if (!names[i] || !dsts[i]) throw std::runtime_error("get_tensors: NULL argument");
+    m->interp->getTensors(std::vector<std::string>(names, names + n), std::vector<float *>(dsts, dsts + n),
+                          std::vector<size_t>(counts, counts + n), bidx);
+  })
+}
+
 int tpuhip_module_invoke(tpuhip_module *m, int bidx) { GUARD(m, m->interp->invoke(bidx)) }
 
 int tpuhip_module_invoke_to(tpuhip_module *m, const char *name, int bidx) {
