@@ -55,6 +55,7 @@ struct WeightData {
 };
 
 struct HostRead;
+struct AheadRead;
 
 // An activation tensor: `batch` slots of one int8 channels-last image set in HBM -- or, at
 // the graph edges only (an fp32 input before its QuantOp, the result of a dequantising
@@ -69,7 +70,7 @@ public:
   TensorData &operator=(const TensorData &) = delete;
 
   size_t size() const { return size_; }          // logical elements of one slot
-  void *data() const { return ptr_; }            // device address of the current slot
+  void *data() const;                            // device address of the current slot
   void set_batch_idx(int32_t bidx);
   int32_t batch_idx() const { return cur_; }
   // float-stored NCHW host data -> slot bidx (values must be integers in [-128,127])
@@ -86,6 +87,14 @@ public:
   // slots bidx of several tensors of one context at once, float-stored (see read); their transfers overlap
   static void read_all(const std::vector<const TensorData *> &tensors, const std::vector<float *> &dsts,
                        const std::vector<size_t> &nums, int32_t bidx);
+  // A module's result on its way to the host while the kernels behind it run, for a read that is expected: the current
+  // slot's bytes are taken as they are now.  Dropped when the tensor may be written again, never done for a tensor whose
+  // address has been handed to others.
+  void read_ahead();
+  void drop_ahead() const { ahead_slot_ = -1; }
+  bool exposed() const { return exposed_; }
+  // whether the tensor was read since the last call of this
+  bool take_was_read() const;
   // lays the tensor out again with another channel stride (4 for a tensor of at most 4 channels whose
   // only readers take one dword per pixel, else a multiple of 16); the contents are lost
   void set_channel_stride(int new_cs);
@@ -101,6 +110,10 @@ public:
 
 private:
   HostRead host_read(void *dst, size_t num, int32_t bidx, bool bytes) const;
+  bool finish_ahead(const HostRead &r, int32_t bidx) const;
+  std::unique_ptr<AheadRead> ahead_;
+  mutable int32_t ahead_slot_ = -1;      // the slot ahead_ holds
+  mutable bool exposed_ = false, was_read_ = false;
   tpuhip_ctx *ctx_;
   size_t size_;
   void *slot(int32_t bidx) const { return (char *)base_ + slot_bytes() * (size_t)bidx; }
@@ -139,6 +152,7 @@ public:
 
   std::string get_name() { return name; }
   const std::vector<Operand> &operands() const { return opdTensors; }
+  const SyncedData &result_tensor() const { return resTensor; }
   SyncedDataShape get_shape() { return shape; }
   std::string get_data_type();
   void set_name(std::string n) { name = std::move(n); }
@@ -677,6 +691,15 @@ private:
   void pairConvs();
   void packInputs();
   void spreadDirtiness();
+  void planAhead();
+  void dropAhead();
+  bool capturing() const;
+  struct Ahead {
+    CPUOpKernel *behind;   // the kernel at whose position the tensor is complete
+    TensorData *tensor;
+    bool wanted;           // the last invoke's result was read
+  };
+  std::vector<Ahead> ahead_;
   // kernels that run as one launch (a conv with the table op / add folded into it, the two
   // convs of a pair): rebuilt by every loadModule
   std::vector<std::vector<CPUOpKernel *>> launch_groups_;

@@ -118,3 +118,34 @@ def test_all_tensors_at_once(shapes):
             assert np.array_equal(got["y%d" % i], np.maximum(x, 0)) and np.array_equal(every["y%d" % i], np.maximum(x, 0))
             assert np.array_equal(every["x%d" % i], x)
     m.close()
+
+
+# results complete before the last kernel: large enough to be read ahead, and not
+@pytest.mark.parametrize("shape", [(1, 70, 50, 41), (3, 64, 40, 40), (1, 5, 20, 20)])
+def test_an_early_output_is_what_the_last_invoke_made_of_it(shape):
+    g = graphs.Graph("early", 1)
+    g.add(graphs.Op("tpu.input", "x", [], shape))
+    g.add(graphs.Op("tpu.relu", "first", ["x"], shape))
+    g.add(graphs.Op("tpu.upsample", "second", ["x"], shape[:2] + (2 * shape[2], 2 * shape[3]), dict(scale_h=2, scale_w=2)))
+    g.outputs = ["first", "second"]
+    m = module()
+    m.load(g)
+    rng = np.random.default_rng(9)
+    xs = [rng.integers(-128, 128, shape).astype(np.int8) for _ in range(5)]
+    for x in xs:
+        m.set_tensor_i8("x", x)
+        m.invoke()
+        for _ in range(2):
+            assert np.array_equal(m.get_tensor_i8("first"), np.maximum(x, 0))
+        assert np.array_equal(m.get_tensor("second"), x.repeat(2, 2).repeat(2, 3))
+    m.set_tensor_i8("x", xs[0])                     # no invoke: the old result
+    assert np.array_equal(m.get_tensor_i8("first"), np.maximum(xs[-1], 0))
+    m.invoke_to("first")
+    assert np.array_equal(m.get_tensor("first"), np.maximum(xs[0], 0))
+    m.set_tensor_i8("first", xs[1])                 # written by hand
+    assert np.array_equal(m.get_tensor_i8("first"), xs[1])
+    m.invoke()
+    m.invoke()                                      # two in a row, the first one's result is never read
+    got = m.run(xs[2])
+    assert np.array_equal(got["first"], np.maximum(xs[2], 0)) and np.array_equal(got["second"], xs[2].repeat(2, 2).repeat(2, 3))
+    m.close()

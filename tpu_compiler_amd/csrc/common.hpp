@@ -34,6 +34,8 @@ struct tpuhip_ctx {
   std::vector<hipEvent_t> stage_events;
   // a module is being loaded: packed weights need not be on the device when a prepack call returns, the loader waits once
   bool loading = false;
+  bool in_interpreter = false;   // a module loads or invokes its kernels: device addresses asked for now go to those
+  hipStream_t copy_stream = nullptr;   // results laid out early leave on it while `stream` works on; made on first use
   bool single_pass = false;   // what is issued now runs once: no layer's tile variants are timed for it
 };
 

@@ -532,6 +532,55 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
   return TPUHIP_OK;
 }
 
+AheadRead::~AheadRead() {
+  if (dense) (void)hipFree(dense);
+  if (pinned) (void)hipHostFree(pinned);
+}
+
+// behind the launch whose writes it announces
+__global__ void arrived_kernel(uint32_t *flag, uint32_t value) {
+  __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src) {
+  const size_t bytes = ((size_t)t.n * t.c * t.h * t.w + 63) / 64 * 64;
+  if (!ctx->copy_stream) TPUHIP_CHECK_HIP(hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking));
+  if (!a.pinned) {
+    TPUHIP_CHECK_HIP(hipMalloc(&a.dense, bytes + 256));
+    TPUHIP_CHECK_HIP(hipHostMalloc(&a.pinned, bytes + 64, hipHostMallocDefault));
+    a.flag = (uint32_t *)((char *)a.pinned + bytes);
+    *a.flag = 0;
+  }
+  if (int rc = tpuhip_nhwc_to_nchw_i8(ctx, src, a.dense, t.n, t.c, t.h, t.w, t.cs)) return rc;
+  launch(ctx, arrived_kernel, dim3(1), dim3(1), a.flag, ++a.serial);
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
+}
+
+// The host sees from the flag that the dense form is there and starts a copy engine on it: that needs no wait of one
+// stream for another (which costs the host 12 us a piece, 60 in front of a copy), and unlike a kernel the engine takes no
+// compute unit from the launches that are still running.
+int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r) {
+  for (int spin = 0; __atomic_load_n(a.flag, __ATOMIC_ACQUIRE) != a.serial; ++spin) {
+    if (spin % 256 == 255) {   // a stream that is done, or has failed, without the flag: nothing more will come
+      const hipError_t e = hipStreamQuery(ctx->stream);
+      if (e != hipErrorNotReady && __atomic_load_n(a.flag, __ATOMIC_ACQUIRE) != a.serial) {
+        TPUHIP_CHECK_HIP(e);
+        return set_error(TPUHIP_ERR_HIP, "a result laid out early did not arrive");
+      }
+    }
+    std::this_thread::yield();
+  }
+  const size_t count = elements(r), grain = kPiece / host_size(r.kind);
+  TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
+  TPUHIP_CHECK_HIP(hipMemcpyAsync(a.pinned, a.dense, count, hipMemcpyDeviceToHost, ctx->copy_stream));
+  TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->copy_stream));
+  parallel_pieces((count + grain - 1) / grain, [&](size_t i) {
+    pass_part(Part{&r, i * grain, std::min(grain, count - i * grain), i * grain, 0}, (const int8_t *)a.pinned, false);
+  });
+  return TPUHIP_OK;
+}
+
 int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes) {
   constexpr size_t kRoom = 4 << 20;   // many small uploads pass without a wait between them
   for (size_t at = 0; at < bytes;) {
@@ -563,6 +612,8 @@ void host_io_release(tpuhip_ctx *ctx) {
   if (ctx->stage) (void)hipHostFree(ctx->stage);
   if (ctx->landing) (void)hipFree(ctx->landing);
   for (hipEvent_t e : ctx->stage_events) (void)hipEventDestroy(e);
+  if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
+  ctx->copy_stream = nullptr;
   ctx->stage = ctx->landing = nullptr;
   ctx->stage_bytes = ctx->landing_bytes = 0;
   ctx->stage_events.clear();

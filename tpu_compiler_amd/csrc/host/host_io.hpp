@@ -44,4 +44,15 @@ struct HostRead {
 };
 int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n);
 
+// A result that is complete while its stream still has work in front of it: read_ahead() lays it out for the host there
+// and then, finish_ahead() fetches it beside the rest of that work.
+struct AheadRead {
+  void *dense = nullptr, *pinned = nullptr;
+  uint32_t *flag = nullptr, serial = 0;   // the flag, in pinned memory, shows the serial of what lies in `dense`
+  ~AheadRead();
+};
+int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src);
+// the host pass from a's bytes instead of r.src
+int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r);
+
 }  // namespace tpuhip

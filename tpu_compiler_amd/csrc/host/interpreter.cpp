@@ -58,13 +58,41 @@ void ModuleInterpreter::updateWeightMap(const std::string &name, std::vector<flo
 
 void ModuleInterpreter::loadModule(ModuleDesc &module, std::string target_op) {
   // packed weights arrive in stream order, in front of whatever this module runs: no prepack call waits for them
-  FlagScope loading(ctx_->loading);
+  FlagScope loading(ctx_->loading), inside(ctx_->in_interpreter);
+  ahead_.clear();
   updateKernelList(module, target_op);
   fuseKernels();
   chainConvs();
   pairConvs();
   packInputs();
   spreadDirtiness();
+  planAhead();
+}
+
+// Outputs that are complete while kernels remain to be run can be on their way to the host beside those.  From 128 KB
+// (reading less takes hardly longer than the two launches that prepare for it) to 64 MB of pinned memory a module.
+void ModuleInterpreter::planAhead() {
+  size_t room = 64 << 20;
+  for (auto &name : output_details) {
+    auto it = activationMapping.find(name);
+    if (it == activationMapping.end()) continue;
+    TensorData *t = it->second.get();
+    if (t->f32 || t->size() < (128 << 10) || t->size() > room) continue;
+    CPUOpKernel *behind = nullptr;
+    for (auto &k : kernel_list_)
+      if (k->result_tensor().get() == t) behind = k.get();
+    if (!behind || behind == kernel_list_.back().get() || dynamic_cast<InputOpKernel *>(behind)) continue;
+    if (std::any_of(ahead_.begin(), ahead_.end(), [&](const Ahead &a) { return a.tensor == t; })) continue;
+    ahead_.push_back({behind, t, false});
+    room -= t->size();
+  }
+}
+
+void ModuleInterpreter::dropAhead() {
+  for (auto &a : ahead_) {
+    a.tensor->drop_ahead();
+    a.wanted = a.tensor->take_was_read();
+  }
 }
 
 // The dirty flag of the reference (MlirModuleInterpreter.cpp:85-116, 383-405) belongs to one
@@ -429,17 +457,29 @@ void ModuleInterpreter::updateKernelList(ModuleDesc &module, std::string &target
   }
 }
 
+// a graph that a caller records would announce the same serial at every replay
+bool ModuleInterpreter::capturing() const {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx_->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
 // MlirModuleInterpreter.cpp:371-381
 void ModuleInterpreter::invokeTo(std::string name, int32_t bidx) {
+  FlagScope inside(ctx_->in_interpreter);
+  dropAhead();
   for (auto &kv : valueMapping) kv.second->set_batch_idx(bidx);
   for (auto &krnl : kernel_list_) {
     krnl->invoke();
+    for (auto &a : ahead_)
+      if (a.wanted && a.behind == krnl.get() && !capturing()) a.tensor->read_ahead();
     if (!name.empty() && name == krnl->name) break;
   }
 }
 
 // MlirModuleInterpreter.cpp:383-405
 void ModuleInterpreter::fastInvokeAllBatch(std::string name, int32_t batch) {
+  FlagScope inside(ctx_->in_interpreter);
+  dropAhead();
   bool last_batch = false;
   for (int i = 0; i < batch; i++) {
     if (i == batch - 1) last_batch = true;
@@ -530,6 +570,8 @@ std::vector<std::pair<std::string, float>> ModuleInterpreter::timeKernels(int32_
   // dispatch fills with the begin and end of its execution on the module's stream:
   // the duration of the kernel itself, in place, with the caches as a real step
   // leaves them.  An op that launches no kernel reports 0.
+  FlagScope inside(ctx_->in_interpreter);
+  dropAhead();
   if (iters < 1) iters = 1;
   for (auto &kv : valueMapping) kv.second->set_batch_idx(bidx);
   const size_t nk = kernel_list_.size();

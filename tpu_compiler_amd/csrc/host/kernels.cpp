@@ -110,12 +110,39 @@ TensorData::TensorData(tpuhip_ctx *ctx, int32_t batch_, const SyncedDataShape &s
   ptr_ = base_;
 }
 
+void *TensorData::data() const {
+  drop_ahead();
+  if (!ctx_->in_interpreter) exposed_ = true;
+  return ptr_;
+}
+
+bool TensorData::take_was_read() const {
+  const bool was = was_read_;
+  was_read_ = false;
+  return was;
+}
+
+void TensorData::read_ahead() {
+  if (exposed_ || !materialized || f32) return;
+  if (!ahead_) ahead_ = std::make_unique<AheadRead>();
+  ck(tpuhip::read_ahead(ctx_, *ahead_, HostTensor{n, c, h, w, cs, is_unsigned}, ptr_), "TensorData::read_ahead");
+  ahead_slot_ = cur_;
+}
+
+bool TensorData::finish_ahead(const HostRead &r, int32_t bidx) const {
+  was_read_ = true;
+  if (ahead_slot_ < 0 || ahead_slot_ != bidx || exposed_) return false;
+  ck(tpuhip::finish_ahead(ctx_, *ahead_, r), "TensorData::tensor");
+  return true;
+}
+
 TensorData::~TensorData() {
   if (base_) tpuhip_free(ctx_, base_);
 }
 
 void TensorData::set_channel_stride(int new_cs) {
   if (f32 || new_cs == cs) return;
+  drop_ahead();
   if (new_cs < c || (new_cs % 16 != 0 && new_cs != 4)) fail("TensorData::set_channel_stride: bad stride");
   if (base_) ck(tpuhip_free(ctx_, base_), "TensorData::set_channel_stride");
   base_ = nullptr;
@@ -133,6 +160,7 @@ void TensorData::set_batch_idx(int32_t bidx) {
 
 void TensorData::assign(const float *first, size_t num, int32_t bidx) {
   if (num != size_) fail("TensorData::assign: size mismatch");
+  drop_ahead();
   if (bidx < 0 || bidx >= batch) fail("TensorData::assign: slot out of range");
   bool bad = false;
   ck(host_to_device(ctx_, HostTensor{n, c, h, w, cs, is_unsigned}, f32 ? HostKind::kFloats : HostKind::kFloatStored, first,
@@ -149,6 +177,7 @@ void TensorData::assign(const float *first, size_t num, int32_t bidx) {
 
 void TensorData::assign_i8(const int8_t *first, size_t num, int32_t bidx) {
   if (num != size_) fail("TensorData::assign_i8: size mismatch");
+  drop_ahead();
   if (bidx < 0 || bidx >= batch) fail("TensorData::assign_i8: slot out of range");
   if (f32) fail("TensorData::assign_i8: this tensor holds fp32 data");
   bool bad = false;
@@ -170,6 +199,7 @@ HostRead TensorData::host_read(void *dst, size_t num, int32_t bidx, bool bytes) 
 
 void TensorData::read(float *dst, size_t num, int32_t bidx) const {
   const HostRead r = host_read(dst, num, bidx, false);
+  if (finish_ahead(r, bidx)) return;
   ck(device_to_host(ctx_, &r, 1), "TensorData::tensor");
 }
 
@@ -177,6 +207,12 @@ void TensorData::read_all(const std::vector<const TensorData *> &tensors, const 
                           const std::vector<size_t> &nums, int32_t bidx) {
   std::vector<HostRead> reads;
   for (size_t i = 0; i < tensors.size(); ++i) reads.push_back(tensors[i]->host_read(dsts[i], nums[i], bidx, false));
+  // what is there already first: the device may still be working on the others
+  for (size_t i = 0, k = 0; i < tensors.size(); ++i)
+    if (tensors[i]->finish_ahead(reads[k], bidx))
+      reads.erase(reads.begin() + (ptrdiff_t)k);
+    else
+      ++k;
   if (!reads.empty()) ck(device_to_host(tensors[0]->ctx_, reads.data(), reads.size()), "TensorData::tensor");
 }
 
@@ -188,6 +224,7 @@ std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
 
 void TensorData::read_i8(int8_t *dst, size_t num, int32_t bidx) const {
   const HostRead r = host_read(dst, num, bidx, true);
+  if (finish_ahead(r, bidx)) return;
   ck(device_to_host(ctx_, &r, 1), "TensorData::read_i8");
 }
 
