@@ -239,9 +239,8 @@ constexpr size_t kPiece = 256 << 10;        // bytes of the staging buffer per p
 constexpr size_t kAlone = 192 << 10;        // up to here one thread is done before a worker has woken
 // Floats on their way to the device: below this many bytes of them one thread converts nearly as fast as the bus takes the
 // result (19 MB: 300 us alone, 184 on eight threads; 38 MB, beyond the last-level cache: 1220 and 324), and the caller's
-// buffer stays in the caches of the core that will write it again.  Bytes keep up with the bus alone up to here (4.8 MB: 160
-// us either way) and fall behind where the caller's tensors no longer stay in the caches (9.6 MB: 380 us, 269 on several).
-constexpr size_t kSharedFloats = 12 << 20, kSharedBytes = 6 << 20;
+// buffer stays in the caches of the core that will write it again.  Bytes are copied faster than the bus at any size.
+constexpr size_t kSharedFloats = 12 << 20;
 constexpr size_t kStageMax = 32 << 20;      // the staging buffer grows to this; larger tensors go through it in parts
 
 // the pinned buffer, free to be written: transfers out of it that are still in flight have ended
@@ -353,7 +352,7 @@ int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const vo
       there[i].store(1, std::memory_order_release);
     };
     HostWorkers &workers = HostWorkers::get();
-    const bool shared = (kind == HostKind::kBytes ? total >= kSharedBytes : count * sizeof(float) >= kSharedFloats) && workers.enter(job);
+    const bool shared = kind != HostKind::kBytes && count * sizeof(float) >= kSharedFloats && workers.enter(job);
     int rc = TPUHIP_OK;
     size_t sent = 0;   // pieces handed to the device
     ctx->stage_busy = true;
