@@ -20,6 +20,7 @@
 #include <list>
 #include <map>
 #include <memory>
+#include <cstring>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -48,8 +49,58 @@ struct OpDesc {
 
 // A weight tensor as tpu.load_weight yields it: float-stored values
 // (MlirModuleInterpreter.cpp:353-369).
+// The values of a weight: its own, or those of a file kept in memory for it, where they lie there (at any alignment).
+// Reads as a vector does; at() and raw() take the values from where they are, whatever hands out floats by address makes
+// them its own first.
+class WeightValues {
+public:
+  WeightValues() = default;
+  WeightValues(std::vector<float> v) : own_(std::move(v)) {}
+  WeightValues(const void *values, size_t count, std::shared_ptr<const void> keep)
+      : view_((const unsigned char *)values), count_(count), keep_(std::move(keep)) {}
+  size_t size() const { return keep_ ? count_ : own_.size(); }
+  bool empty() const { return size() == 0; }
+  const void *raw() const { return keep_ ? (const void *)view_ : own_.data(); }
+  float at(size_t i) const {
+    if (i >= size()) throw std::out_of_range("WeightValues::at");
+    if (!keep_) return own_[i];
+    float v;
+    std::memcpy(&v, view_ + i * sizeof(float), sizeof v);
+    return v;
+  }
+  const float *data() const { return own().data(); }
+  float *data() { return own().data(); }
+  const float *begin() const { return data(); }
+  const float *end() const { return data() + size(); }
+  float operator[](size_t i) const { return own()[i]; }
+  float &operator[](size_t i) { return own()[i]; }
+  operator std::vector<float>() const { return own(); }
+  template <typename It>
+  void assign(It first, It last) {
+    own_.assign(first, last);
+    keep_.reset();
+  }
+  void resize(size_t n) { own().resize(n); }
+  void push_back(float v) { own().push_back(v); }
+
+private:
+  std::vector<float> &own() const {
+    if (keep_) {
+      own_.resize(count_);
+      if (count_) std::memcpy(own_.data(), view_, count_ * sizeof(float));
+      keep_.reset();
+    }
+    return own_;
+  }
+  mutable std::vector<float> own_;
+  const unsigned char *view_ = nullptr;
+  size_t count_ = 0;
+  mutable std::shared_ptr<const void> keep_;
+};
+
 struct WeightData {
-  std::vector<float> data;
+  WeightValues data;
+  std::vector<int8_t> bytes;   // the values as int8 where a load has converted them already, for the kernel that takes them
   size_t size() const { return data.size(); }
   float at(size_t i) const { return data.at(i); }
 };
@@ -651,7 +702,7 @@ public:
   // the reference's updateWeightMap reads every tpu.load_weight from the npz
   // (MlirModuleInterpreter.cpp:352-369); here the caller hands the arrays over
   void updateWeightMap(const std::string &name, const float *data, size_t count);
-  void updateWeightMap(const std::string &name, std::vector<float> &&data);
+  void updateWeightMap(const std::string &name, WeightValues data);
   std::vector<std::string> &outputDetails() { return output_details; }
   void dump(std::string &name);
   std::vector<std::string> getAllTensorName();
@@ -692,6 +743,7 @@ private:
   void packInputs();
   void spreadDirtiness();
   void planAhead();
+  void convertFilters(const ModuleDesc &module);
   void dropAhead();
   bool capturing() const;
   struct Ahead {

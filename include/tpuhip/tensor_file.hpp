@@ -51,6 +51,8 @@ public:
 
   // a stored float32 array of exactly count elements, in place in the file's image (any alignment); nullptr otherwise
   const void *floats(const std::string &name, size_t count) const;
+  // holds what floats() of a read-only file points to, also beyond the file object
+  std::shared_ptr<const void> kept() const;
 
 private:
   // an array of the file: its values stay where they lie in the file's image until somebody asks for them as an NpyArray

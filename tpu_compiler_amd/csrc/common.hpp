@@ -8,10 +8,29 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <map>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "tpuhip.h"
+
+namespace tpuhip {
+// one filter to be packed for a tile variant (conv.hip)
+struct FilterPack {
+  const int8_t *raw;
+  void *out;
+  int oc, ic, taps, c16, kp, bm, bk, tm, reg;
+  int smallc;
+  int64_t total;   // 16-byte groups
+};
+// one piece of the pinned buffer on its way to the device, in dwords
+struct StagedCopy {
+  const uint32_t *src;
+  uint32_t *dst;
+  size_t dwords;
+};
+}  // namespace tpuhip
 
 struct tpuhip_ctx {
   int device = 0;
@@ -32,8 +51,20 @@ struct tpuhip_ctx {
   size_t stage_used = 0;     // bytes of the pinned buffer that stage_upload has handed out since it was last free
   bool stage_busy = false;   // kernels that read or write the pinned buffer may still be in flight
   std::vector<hipEvent_t> stage_events;
-  // a module is being loaded: packed weights need not be on the device when a prepack call returns, the loader waits once
+  // Memory of a module's tensors and packed weights, most of them small and made by the hundred: parts of slabs
+  // (api.hip), while `loading`
+  struct Slab {
+    char *base;
+    size_t size;
+    std::map<size_t, size_t> unused;   // offset -> bytes
+  };
+  std::vector<Slab> slabs;
+  std::unordered_map<void *, std::pair<char *, size_t>> slab_parts;   // allocation -> its slab's base, its bytes
+  // a module is being loaded: packed weights need not be on the device when a prepack call returns, and what is to be
+  // uploaded and packed for them gathers here until flush_uploads() (host_io.cpp) issues all of it in two launches
   bool loading = false;
+  std::vector<tpuhip::StagedCopy> staged;
+  std::vector<tpuhip::FilterPack> packs;
   bool in_interpreter = false;   // a module loads or invokes its kernels: device addresses asked for now go to those
   hipStream_t copy_stream = nullptr;   // results laid out early leave on it while `stream` works on; made on first use
   bool single_pass = false;   // what is issued now runs once: no layer's tile variants are timed for it
@@ -61,6 +92,10 @@ void host_io_release(tpuhip_ctx *ctx);
 // host/host_io.cpp: tpuhip_upload without the wait -- src may be reused on return, the bytes are there for what is issued to
 // the context's stream afterwards
 int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes);
+// issues what has gathered in ctx->staged and ctx->packs
+int flush_uploads(tpuhip_ctx *ctx);
+// conv.hip: packs n filters; the list is in memory the device reads
+int pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t largest);
 // waits for what a prepack call has issued, unless a module is being loaded: packed weights may be used from any context
 int prepack_done(tpuhip_ctx *ctx);
 

@@ -3930,16 +3930,20 @@ int check_desc(const tpuhip_conv_desc &d) {
 
 // Packs an OIHW filter for a tile variant: a thread makes one 16-byte K group of one row in the order its kernel reads
 // (2.4 MB in 10 us; the host loop this replaces took 4 ms, once per timed variant).
-struct PackArgs {
-  const int8_t *raw;
-  v4i *out;
-  int oc, ic, taps, c16, kp, bm, bk, tm, reg;
-  int smallc;
-  int64_t total;   // 16-byte groups
-};
-__global__ __launch_bounds__(256) void pack_filter_kernel(PackArgs a) {
-  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (q >= a.total) return;
+constexpr int kPackDepthwise = -1;   // the diagonal fragments of the depthwise kernels, not a tile's form
+__device__ __forceinline__ void pack_filter_group(const FilterPack &a, int64_t q) {
+  if (a.reg == kPackDepthwise) {   // 64 fragments a tap, nearly all zeros: 0.5 MB for the 1728 bytes of 192 channels
+    const int lane = (int)(q & 63), f = (int)(q >> 6), cb = f / a.taps, tap = f - cb * a.taps;
+    const int in_block = mfma_row_to_oc(lane & 31, 1), ch = cb * 32 + in_block, j = in_block - 16 * (lane >> 5);
+    uint32_t v[4] = {0, 0, 0, 0};
+    if (ch < a.oc && j >= 0 && j < 16) {
+      const uint32_t byte = (uint32_t)(uint8_t)a.raw[(int64_t)ch * a.taps + tap] << (8 * (j & 3));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = k == j >> 2 ? byte : 0;
+    }
+    ((v4i *)a.out)[q] = v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+    return;
+  }
   const int kg = a.kp >> 4;          // 16-byte groups per row
   int row, kc;
   if (a.reg == 6) {
@@ -3981,7 +3985,29 @@ __global__ __launch_bounds__(256) void pack_filter_kernel(PackArgs a) {
       if (tap < a.taps && c < a.ic) v[b >> 2] |= (uint32_t)(uint8_t)src[(int64_t)c * a.taps + tap] << (8 * (b & 3));
     }
   }
-  a.out[q] = v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+  ((v4i *)a.out)[q] = v4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
+}
+
+__global__ __launch_bounds__(256) void pack_filter_kernel(FilterPack a) {
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (q < a.total) pack_filter_group(a, q);
+}
+
+// the filters of a loading module, a row of workgroups each
+__global__ __launch_bounds__(256) void pack_filters_kernel(const FilterPack *list) {
+  const FilterPack a = list[blockIdx.y];
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < a.total; q += (int64_t)gridDim.x * 256) pack_filter_group(a, q);
+}
+
+// now, or with the others of the module that is being loaded
+int pack_filter(tpuhip_ctx *ctx, const FilterPack &a) {
+  if (ctx->loading) {
+    ctx->packs.push_back(a);
+    return TPUHIP_OK;
+  }
+  hipLaunchKernelGGL(pack_filter_kernel, dim3((unsigned)ceil_div64(a.total, 256)), dim3(256), 0, ctx->stream, a);
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
 }
 
 // (re)builds the device filter of an MFMA conv for tile variant `tile`
@@ -4003,15 +4029,14 @@ int pack_mfma_weights(tpuhip_ctx *ctx, tpuhip_conv_weights *cw, int tile) {
     if (int rc = tpuhip_malloc(ctx, bytes, (void **)&cw->w)) return rc;
     cw->w_room = bytes;
   }
-  PackArgs a{};
+  FilterPack a{};
   a.raw = cw->raw;
-  a.out = (v4i *)cw->w;
+  a.out = cw->w;
   a.oc = d.oc; a.ic = d.ic; a.taps = d.kh * d.kw;
   a.c16 = cw->c16; a.kp = cw->kp; a.bm = t.bm; a.bk = t.bk; a.tm = tm; a.reg = t.reg;
   a.smallc = cw->smallc ? 1 : 0;
   a.total = (int64_t)bytes / 16;
-  hipLaunchKernelGGL(pack_filter_kernel, dim3((unsigned)ceil_div64(a.total, 256)), dim3(256), 0, ctx->stream, a);
-  TPUHIP_CHECK_HIP(hipGetLastError());
+  if (int rc = pack_filter(ctx, a)) return rc;
   cw->tile = tile;
   cw->ocp = ocp;
   return TPUHIP_OK;
@@ -4435,6 +4460,13 @@ int choose_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *y,
 
 }  // namespace
 
+int tpuhip::pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t largest) {
+  const dim3 grid((unsigned)std::min<int64_t>(ceil_div64(largest, 256), 32), (unsigned)n);
+  hipLaunchKernelGGL(pack_filters_kernel, grid, dim3(256), 0, ctx->stream, list);
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
+}
+
 extern "C" {
 
 int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const int8_t *filter,
@@ -4511,16 +4543,19 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
     // l & 31 (channel mfma_row_to_oc(row) of the block), K bytes 16*(l >> 5) .. +15
     cw->ocp = round_up(d.oc, 16);
     const int taps = d.kh * d.kw, n_cb = (cw->ocp + 31) / 32;
-    packed.assign((size_t)n_cb * taps * 1024, 0);
-    for (int cb = 0; cb < n_cb; ++cb)
-      for (int t = 0; t < taps; ++t)
-        for (int lane = 0; lane < 64; ++lane) {
-          const int ch_in_block = mfma_row_to_oc(lane & 31, 1);
-          const int ch = cb * 32 + ch_in_block;
-          const int j = ch_in_block - 16 * (lane >> 5);
-          if (ch < d.oc && j >= 0 && j < 16)
-            packed[((size_t)(cb * taps + t) * 64 + lane) * 16 + j] = filter[(size_t)ch * taps + t];
-        }
+    int rc = tpuhip_malloc(ctx, (size_t)d.oc * taps, (void **)&cw->raw);
+    if (!rc) rc = stage_upload(ctx, cw->raw, filter, (size_t)d.oc * taps);
+    if (!rc) rc = tpuhip_malloc(ctx, (size_t)n_cb * taps * 1024, (void **)&cw->w);
+    FilterPack a{};
+    a.raw = cw->raw;
+    a.out = cw->w;
+    a.oc = d.oc; a.taps = taps; a.reg = kPackDepthwise;
+    a.total = (int64_t)n_cb * taps * 64;
+    if (!rc) rc = pack_filter(ctx, a);
+    if (rc) {
+      tpuhip_conv2d_weights_destroy(ctx, cw);
+      return rc;
+    }
   } else if (algo == ALGO_STEM) {
     // A fragments [32-channel block][filter row][lane][16 bytes]: lane l holds MFMA row l & 31
     // (channel mfma_row_to_oc(row) of the block) and K bytes 16*(l >> 5) .. +15 of the
@@ -4579,9 +4614,13 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
       q.rshift = rshift[i];
       q.mask = (int32_t)((1ll << rshift[i]) - 1);
       q.hpot = rshift[i] > 0 ? (int32_t)(1ll << (rshift[i] - 1)) : 0;
-      int64_t sumw = 0;
-      for (size_t k = 0; k < per_oc; ++k) sumw += std::abs((int)filter[(size_t)i * per_oc + k]);
-      const int64_t bound = 128 * sumw + std::llabs((long long)b32[i]) + 1 + q.hpot;
+      const int64_t rest = std::llabs((long long)b32[i]) + 1 + q.hpot;
+      int64_t sumw = 128 * (int64_t)per_oc;   // no filter's sum is larger; it is taken only where that is not small enough
+      if (128 * sumw + rest >= (1ll << 31)) {
+        sumw = 0;
+        for (size_t k = 0; k < per_oc; ++k) sumw += std::abs((int)filter[(size_t)i * per_oc + k]);
+      }
+      const int64_t bound = 128 * sumw + rest;
       if (rshift[i] < 1 || bound >= (1ll << 31)) fast = false;
     } else {
       q.rshift = 1;   // pad channels: multiplier 0 gives 0 on either path
@@ -4592,7 +4631,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   }
   cw->fast = fast ? 1 : 0;
   int rc = TPUHIP_OK;
-  if (algo != ALGO_MFMA && !cw->gather) {
+  if (!packed.empty()) {
     rc = tpuhip_malloc(ctx, packed.size(), (void **)&cw->w);
     if (!rc) rc = stage_upload(ctx, cw->w, packed.data(), packed.size());
   }

@@ -27,11 +27,12 @@ namespace tpuhip {
 // ---------------------------------------------------------------------------
 namespace {
 
-bool to_bytes_plain(const float *src, int8_t *dst, size_t n, float lo, float hi) {
+bool to_bytes_plain(const char *src, int8_t *dst, size_t n, float lo, float hi) {
   unsigned bad = 0;
   const float magic = 12582912.0f;   // 1.5 * 2^23: adding and subtracting it rounds below 2^22
   for (size_t i = 0; i < n; ++i) {
-    const float v = src[i];
+    float v;
+    memcpy(&v, src + i * sizeof(float), sizeof v);
     bad |= (unsigned)!(v >= lo && v <= hi) | (unsigned)((v + magic) - magic != v);
     const float in_range = v >= lo && v <= hi ? v : 0.0f;
     dst[i] = (int8_t)(int32_t)in_range;
@@ -40,22 +41,22 @@ bool to_bytes_plain(const float *src, int8_t *dst, size_t n, float lo, float hi)
 }
 
 #ifdef TPUHIP_X86
-__attribute__((target("avx512f,avx512bw"))) bool to_bytes_avx512(const float *src, int8_t *dst, size_t n, float lo, float hi) {
+__attribute__((target("avx512f,avx512bw"))) bool to_bytes_avx512(const char *src, int8_t *dst, size_t n, float lo, float hi) {
   const __m512 vlo = _mm512_set1_ps(lo), vhi = _mm512_set1_ps(hi);
   __mmask16 bad = 0;
   size_t i = 0;
   for (; i + 16 <= n; i += 16) {
-    const __m512 v = _mm512_loadu_ps(src + i);
+    const __m512 v = _mm512_loadu_ps(src + i * sizeof(float));
     const __m512i q = _mm512_cvtps_epi32(v);   // rounds to nearest even
     bad |= _mm512_cmp_ps_mask(v, vlo, _CMP_NGE_UQ) | _mm512_cmp_ps_mask(v, vhi, _CMP_NLE_UQ) |
            _mm512_cmp_ps_mask(v, _mm512_cvtepi32_ps(q), _CMP_NEQ_UQ);
     _mm_storeu_si128((__m128i *)(dst + i), _mm512_cvtepi32_epi8(q));   // keeps the low byte
   }
-  const bool tail = to_bytes_plain(src + i, dst + i, n - i, lo, hi);
+  const bool tail = to_bytes_plain(src + i * sizeof(float), dst + i, n - i, lo, hi);
   return bad != 0 || tail;
 }
 
-__attribute__((target("avx2"))) bool to_bytes_avx2(const float *src, int8_t *dst, size_t n, float lo, float hi) {
+__attribute__((target("avx2"))) bool to_bytes_avx2(const char *src, int8_t *dst, size_t n, float lo, float hi) {
   const __m256 vlo = _mm256_set1_ps(lo), vhi = _mm256_set1_ps(hi);
   const __m256i low = _mm256_set1_epi32(0xff);
   const __m256i order = _mm256_setr_epi32(0, 4, 1, 5, 2, 6, 3, 7);
@@ -64,7 +65,7 @@ __attribute__((target("avx2"))) bool to_bytes_avx2(const float *src, int8_t *dst
   for (; i + 32 <= n; i += 32) {
     __m256i q[4];
     for (int k = 0; k < 4; ++k) {
-      const __m256 v = _mm256_loadu_ps(src + i + 8 * k);
+      const __m256 v = _mm256_loadu_ps((const float *)(src + (i + 8 * k) * sizeof(float)));
       q[k] = _mm256_cvtps_epi32(v);
       bad = _mm256_or_ps(bad, _mm256_or_ps(_mm256_or_ps(_mm256_cmp_ps(v, vlo, _CMP_NGE_UQ), _mm256_cmp_ps(v, vhi, _CMP_NLE_UQ)),
                                            _mm256_cmp_ps(v, _mm256_cvtepi32_ps(q[k]), _CMP_NEQ_UQ)));
@@ -73,7 +74,7 @@ __attribute__((target("avx2"))) bool to_bytes_avx2(const float *src, int8_t *dst
     const __m256i a = _mm256_packus_epi32(q[0], q[1]), b = _mm256_packus_epi32(q[2], q[3]);
     _mm256_storeu_si256((__m256i *)(dst + i), _mm256_permutevar8x32_epi32(_mm256_packus_epi16(a, b), order));
   }
-  const bool tail = to_bytes_plain(src + i, dst + i, n - i, lo, hi);
+  const bool tail = to_bytes_plain(src + i * sizeof(float), dst + i, n - i, lo, hi);
   return _mm256_movemask_ps(bad) != 0 || tail;
 }
 
@@ -113,7 +114,8 @@ int simd_level() {
 
 }  // namespace
 
-bool floats_to_bytes(const float *src, int8_t *dst, size_t n, bool is_unsigned) {
+bool floats_to_bytes(const void *values, int8_t *dst, size_t n, bool is_unsigned) {
+  const char *src = (const char *)values;
   const float lo = is_unsigned ? 0.0f : -128.0f, hi = is_unsigned ? 255.0f : 127.0f;
 #ifdef TPUHIP_X86
   if (simd_level() == 2) return to_bytes_avx512(src, dst, n, lo, hi);
@@ -246,6 +248,7 @@ constexpr size_t kStageMax = 32 << 20;      // the staging buffer grows to this;
 // the pinned buffer, free to be written: transfers out of it that are still in flight have ended
 int stage_ready(tpuhip_ctx *ctx, size_t bytes) {
   TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
+  if (int rc = flush_uploads(ctx)) return rc;   // left by a load that failed
   if (ctx->stage_busy) {
     TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     ctx->stage_busy = false;
@@ -319,7 +322,7 @@ int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const vo
   if (int rc = stage_ready(ctx, total)) return rc;
   auto pass = [&](size_t first, size_t elements, int8_t *to) {
     const char *from = (const char *)src + first * host_size(kind);
-    if (kind == HostKind::kFloatStored) return floats_to_bytes((const float *)from, to, elements, t.is_unsigned);
+    if (kind == HostKind::kFloatStored) return floats_to_bytes(from, to, elements, t.is_unsigned);
     memcpy(to, from, elements * per);
     return false;
   };
@@ -581,18 +584,63 @@ int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r) {
   return TPUHIP_OK;
 }
 
+// the copies of a loading module, a row of workgroups each; the list lies in the pinned buffer too
+__global__ __launch_bounds__(256) void staged_copies_kernel(const StagedCopy *list) {
+  const StagedCopy c = list[blockIdx.y];
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < c.dwords; i += stride) c.dst[i] = c.src[i];
+}
+
+// A network of 52 convs took three launches for each, 440 us of a 5 ms tool run; all of them together take two.
+int flush_uploads(tpuhip_ctx *ctx) {
+  if (ctx->staged.empty() && ctx->packs.empty()) return TPUHIP_OK;
+  auto place = [&](const void *list, size_t bytes) -> void * {   // stage_upload() leaves the room for it
+    void *at = (int8_t *)ctx->stage + ctx->stage_used;
+    memcpy(at, list, bytes);
+    ctx->stage_used += (bytes + 15) / 16 * 16;
+    return at;
+  };
+  ctx->stage_busy = true;
+  if (!ctx->staged.empty()) {
+    size_t largest = 0;
+    for (auto &c : ctx->staged) largest = std::max(largest, c.dwords);
+    const dim3 grid((unsigned)std::min<size_t>((largest + 1023) / 1024, 16), (unsigned)ctx->staged.size());
+    const void *list = place(ctx->staged.data(), ctx->staged.size() * sizeof(StagedCopy));
+    hipLaunchKernelGGL(staged_copies_kernel, grid, dim3(256), 0, ctx->stream, (const StagedCopy *)list);
+    ctx->staged.clear();
+    TPUHIP_CHECK_HIP(hipGetLastError());
+  }
+  if (!ctx->packs.empty()) {
+    int64_t largest = 0;
+    for (auto &f : ctx->packs) largest = std::max(largest, f.total);
+    const void *list = place(ctx->packs.data(), ctx->packs.size() * sizeof(FilterPack));
+    const size_t n = ctx->packs.size();
+    ctx->packs.clear();
+    if (int rc = pack_filters(ctx, (const FilterPack *)list, n, largest)) return rc;
+  }
+  return TPUHIP_OK;
+}
+
 int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes) {
-  constexpr size_t kRoom = 4 << 20;   // many small uploads pass without a wait between them
+  // many small uploads pass without a wait between them, those of a usual module without any
+  const size_t kRoom = ctx->loading ? 8 << 20 : 4 << 20;
+  constexpr size_t kLists = 64 << 10, kMost = 256;   // room for flush_uploads(), and the launches it gathers at most
   for (size_t at = 0; at < bytes;) {
-    if (!ctx->stage || ctx->stage_used + 16 > ctx->stage_bytes || (at == 0 && bytes <= kRoom && ctx->stage_used + bytes > ctx->stage_bytes))
-      if (int rc = stage_ready(ctx, kRoom)) return rc;
-    const size_t len = std::min(bytes - at, ctx->stage_bytes - ctx->stage_used);
+    if (ctx->staged.size() >= kMost || ctx->packs.size() >= kMost)
+      if (int rc = flush_uploads(ctx)) return rc;
+    if (!ctx->stage || ctx->stage_used + kLists + 16 > ctx->stage_bytes ||
+        (at == 0 && bytes + kLists <= kRoom && ctx->stage_used + bytes + kLists > ctx->stage_bytes)) {
+      if (int rc = stage_ready(ctx, kRoom)) return rc;   // issues what has gathered first
+    }
+    const size_t len = std::min(bytes - at, ctx->stage_bytes - kLists - ctx->stage_used);
     int8_t *to = (int8_t *)ctx->stage + ctx->stage_used;
     memcpy(to, (const char *)src + at, len);
     ctx->stage_busy = true;
     if (len % 4) {   // a ragged end: whole dwords are copied, and dst need not have the room for the last one
       hipError_t e = hipMemcpyAsync((char *)dst + at, to, len, hipMemcpyHostToDevice, ctx->stream);
       TPUHIP_CHECK_HIP(e);
+    } else if (ctx->loading) {
+      ctx->staged.push_back({(const uint32_t *)to, (uint32_t *)((char *)dst + at), len / 4});
     } else if (int rc = stage_copy(ctx, to, (char *)dst + at, len)) {
       return rc;
     }

@@ -8,6 +8,7 @@
 #include "host_io.hpp"
 
 #include <algorithm>
+#include <charconv>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -44,10 +45,12 @@ int8_t weight_to_i8(float v, const std::string &op, const char *role) {
 }
 
 // a float-stored int8 weight array as bytes
-std::vector<int8_t> weights_to_i8(const std::vector<float> &v, const std::string &op, const char *role) {
-  std::vector<int8_t> out(v.size());
-  if (floats_to_bytes(v.data(), out.data(), v.size(), false))
-    for (float f : v) weight_to_i8(f, op, role);   // names the value
+std::vector<int8_t> weights_to_i8(WeightData &w, const std::string &op, const char *role) {
+  if (!w.bytes.empty()) return std::move(w.bytes);
+  const size_t n = w.size();
+  std::vector<int8_t> out(n);
+  if (floats_to_bytes(w.data.raw(), out.data(), n, false))
+    for (size_t i = 0; i < n; ++i) weight_to_i8(w.at(i), op, role);   // names the value
   return out;
 }
 
@@ -87,14 +90,17 @@ double OpDesc::attr(const std::string &key) const {
 }
 
 std::string OpDesc::signature() const {
-  std::ostringstream os;
-  os << type << "|" << quant << "|" << param_type << "|";
-  for (auto d : shape) os << d << "x";
-  os << "|";
-  for (auto &o : operands) os << o << ",";
-  os << "|";
-  for (auto &kv : attrs) os << kv.first << "=" << kv.second << ";";
-  return os.str();
+  std::string out;
+  out.reserve(512);
+  char digits[40];
+  auto number = [&](auto v) { out.append(digits, std::to_chars(digits, digits + sizeof digits, v).ptr); };
+  out += type; out += '|'; out += quant; out += '|'; out += param_type; out += '|';
+  for (auto d : shape) { number(d); out += 'x'; }
+  out += '|';
+  for (auto &o : operands) { out += o; out += ','; }
+  out += '|';
+  for (auto &kv : attrs) { out += kv.first; out += '='; number(kv.second); out += ';'; }
+  return out;
 }
 
 // ---------------------------------------------------------------------------
@@ -394,7 +400,7 @@ Conv2DOpKernel::Conv2DOpKernel(OpDesc &op, value_map_t &valueMapping, weight_map
   if (filter->size() != fsz) fail("Conv2D '" + name + "': filter size mismatch");
   if (quant_rshift->size() < (size_t)d.oc || quant_multiplier->size() < (size_t)d.oc)
     fail("Conv2D '" + name + "': rshift / multiplier need one entry per output channel");
-  std::vector<int8_t> w8 = weights_to_i8(filter->data, name, "filter");
+  std::vector<int8_t> w8 = weights_to_i8(*filter, name, "filter");
   if (transposed) {
     // out(oh) = sum x(ih) * w(kh) over ih*sh + kh*dh - pt == oh (MKLDeconv,
     // NativeCpuImplementation.h:194-280) == a stride-1 conv of the input with sh-1 zeros
@@ -723,7 +729,7 @@ FullyConnectedOpKernel::FullyConnectedOpKernel(OpDesc &op, value_map_t &valueMap
   if (output_data->size() != (size_t)batch * m * n) fail("FullyConnected '" + name + "': result size mismatch");
   if (rshift_data->size() < (size_t)batch || multiplier_data->size() < (size_t)batch)
     fail("FullyConnected '" + name + "': one rshift and one multiplier per batch needed");
-  std::vector<int8_t> w8 = weights_to_i8(filter->data, name, "filter");
+  std::vector<int8_t> w8 = weights_to_i8(*filter, name, "filter");
   std::vector<int32_t> b32;
   if (bias) {
     if (bias->size() < (size_t)batch * n) fail("FullyConnected '" + name + "': bias size mismatch");

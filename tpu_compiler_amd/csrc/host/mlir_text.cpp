@@ -59,9 +59,10 @@ private:
     if (s[i] == '\n') ++line;
     ++i;
   }
+  static bool space(char c) { return c == ' ' || (c >= '\t' && c <= '\r'); }
   void ws() {
     for (;;) {
-      while (!eof() && std::isspace((unsigned char)s[i])) bump();
+      while (!eof() && space(s[i])) bump();
       if (peek() == '/' && peek(1) == '/') {
         while (!eof() && s[i] != '\n') ++i;
         continue;
@@ -78,7 +79,9 @@ private:
   void expect(char c) {
     if (!eat(c)) fail(std::string("expected '") + c + "', found '" + (eof() ? std::string("end of file") : std::string(1, peek())) + "'");
   }
-  static bool ident_char(char c) { return std::isalnum((unsigned char)c) || c == '_' || c == '.' || c == '$'; }
+  static bool ident_char(char c) {
+    return (c >= 'a' && c <= 'z') || (c >= 'A' && c <= 'Z') || (c >= '0' && c <= '9') || c == '_' || c == '.' || c == '$';
+  }
   // consumes `w` if it is the next token (not a prefix of a longer identifier)
   bool word(const char *w) {
     ws();
@@ -114,6 +117,13 @@ private:
     bump();
     std::string out;
     while (!eof() && s[i] != '"') {
+      size_t e = i;   // most strings are one stretch
+      while (e < s.size() && s[e] != '"' && s[e] != '\\' && s[e] != '\n') ++e;
+      if (e > i) {
+        out.append(s, i, e - i);
+        i = e;
+        continue;
+      }
       char c = s[i];
       if (c == '\\' && i + 1 < s.size()) {
         char d = s[i + 1];
@@ -192,6 +202,7 @@ private:
     t.text = s.substr(b, i - b);
     if (head == "tensor" || head == "memref") {
       t.shaped = true;
+      t.shape.reserve(4);
       // dims up to the element type; a memref layout after a top-level ',' is ignored
       size_t p = 0;
       for (;;) {
@@ -226,6 +237,7 @@ private:
     std::vector<MlirType> out;
     expect('(');
     if (eat(')')) return out;
+    out.reserve(8);
     do out.push_back(type()); while (eat(','));
     expect(')');
     return out;
@@ -235,12 +247,12 @@ private:
     MlirAttr d;
     d.kind = MlirAttr::Dict;
     if (eat('}')) return d;
+    d.fields.reserve(8);
     do {
       ws();
       std::string key = peek() == '"' ? quoted() : ident();
-      MlirAttr v;
-      if (eat('=')) v = value();
-      d.fields.emplace_back(std::move(key), std::move(v));
+      d.fields.emplace_back(std::move(key), MlirAttr());
+      if (eat('=')) d.fields.back().second = value();
     } while (eat(','));
     expect('}');
     return d;

@@ -5,6 +5,7 @@
 
 #include <cstring>
 #include <fstream>
+#include <future>
 #include <sstream>
 
 #include "tpuhip/interpreter.hpp"
@@ -41,6 +42,25 @@ bool name_match(const std::string &a, const std::string &b) {
   return a.substr(0, b.size()) == b;
 }
 
+// as written (relative to the working directory, like the reference), else beside the .mlir
+std::string weight_path(const std::string &mlir_path, const std::string &written) {
+  if (!written.empty() && !exists(written) && written[0] != '/' && exists(dir_of(mlir_path) + written))
+    return dir_of(mlir_path) + written;
+  return written;
+}
+
+// what a look at the text says the filename of tpu.weight_file is, "" if it does not say so plainly
+std::string likely_weight_file(const std::string &text) {
+  size_t k = text.find("\"tpu.weight_file\"");
+  if (k == std::string::npos) return "";
+  const size_t end = text.find('\n', k), name = text.find("filename = \"", k);
+  if (name == std::string::npos || name > end) return "";
+  const size_t b = name + 12, e = text.find('"', b);
+  if (e == std::string::npos || e > end) return "";
+  const std::string file = text.substr(b, e - b);
+  return file.find('\\') == std::string::npos ? file : "";
+}
+
 }  // namespace
 
 MlirModule readMlirFile(const std::string &mlir_path) {
@@ -51,16 +71,23 @@ MlirModule readMlirFile(const std::string &mlir_path) {
 // pymlir.cpp py_module::load): every tpu.load_weight is read from the weight file as float32
 // of exactly the element count of its result type.
 void ModuleInterpreter::loadModuleFile(const std::string &mlir_path, std::string target_op) {
-  MlirModule mm = readMlirFile(mlir_path);
+  const std::string text = read_text(mlir_path);
+  // the weights are read while the text is parsed (14 MB: 0.3 ms; 67 KB of text: 0.6 ms)
+  const std::string guess = likely_weight_file(text);
+  std::future<std::unique_ptr<TensorFile>> reading;
+  if (!guess.empty())
+    reading = std::async(std::launch::async, [&] { return std::make_unique<TensorFile>(weight_path(mlir_path, guess), true); });
+  MlirModule mm = moduleFromMlir(parseMlirText(text));
   weight_file_path_ = mm.weight_file;
   op_info_.clear();
   for (auto &o : mm.module.ops) op_info_.push_back({o.name, o.type, o.quant});
   if (!mm.weights.empty()) {
     if (mm.weight_file.empty()) throw std::runtime_error(mlir_path + ": tpu.load_weight without a tpu.weight_file");
-    // as written (relative to the working directory, like the reference), else beside the .mlir
-    std::string wpath = mm.weight_file;
-    if (!exists(wpath) && wpath[0] != '/' && exists(dir_of(mlir_path) + wpath)) wpath = dir_of(mlir_path) + wpath;
-    TensorFile wfile(wpath, true);
+    const std::string wpath = weight_path(mlir_path, mm.weight_file);
+    const std::unique_ptr<TensorFile> opened =
+        reading.valid() && guess == mm.weight_file ? reading.get() : std::make_unique<TensorFile>(wpath, true);
+    TensorFile &wfile = *opened;
+    const std::shared_ptr<const void> kept = wfile.kept();
     for (auto &w : mm.weights) {
       size_t count = 1;
       for (auto v : w.shape) {
@@ -68,9 +95,9 @@ void ModuleInterpreter::loadModuleFile(const std::string &mlir_path, std::string
         count *= (size_t)v;
       }
       std::vector<float> data;
-      if (const void *p = wfile.floats(w.name, count)) {
-        data.resize(count);
-        if (count) std::memcpy(data.data(), p, count * sizeof(float));
+      if (const void *p = wfile.floats(w.name, count)) {   // they stay where the file was read to
+        updateWeightMap(w.name, WeightValues(p, count, kept));
+        continue;
       } else {
         if (!wfile.find(w.name)) throw std::runtime_error("failed to find tensor " + w.name + " to read in " + wpath);
         // beyond the reference's float-stored files: arrays kept with their integer storage type

@@ -4,6 +4,7 @@
 #include "host_io.hpp"
 
 #include <fcntl.h>
+#include <sys/mman.h>
 #include <sys/stat.h>
 #include <unistd.h>
 #include <zlib.h>
@@ -152,7 +153,11 @@ void TensorFile::load() {
   if (::fstat(fd, &st) != 0 || st.st_size < 0) { ::close(fd); fail("cannot size " + filename); }
   const size_t sz = (size_t)st.st_size;
   if (sz < 22) { ::close(fd); fail(filename + " is not a zip archive"); }
-  uint8_t *block = (uint8_t *)std::malloc(sz);
+  // large files in large pages: 14 MB in small ones are 3500 faults, which the readers take from one another
+  constexpr size_t kLargePage = 2 << 20;
+  uint8_t *block = (uint8_t *)(sz >= 2 * kLargePage ? std::aligned_alloc(kLargePage, (sz + kLargePage - 1) / kLargePage * kLargePage)
+                                                     : std::malloc(sz));
+  if (block && sz >= 2 * kLargePage) (void)::madvise(block, sz, MADV_HUGEPAGE);
   if (!block) { ::close(fd); fail("no memory for " + filename); }
   image = std::shared_ptr<const uint8_t>(block, [](const uint8_t *p) { std::free((void *)p); });
   constexpr size_t kPart = 1 << 20;
@@ -264,6 +269,8 @@ const void *TensorFile::floats(const std::string &name, size_t count) const {
   const size_t have = it->second.data ? it->second.size : a.num_bytes();
   return a.kind == 'f' && a.word_size == 4 && have == count * sizeof(float) ? it->second.values() : nullptr;
 }
+
+std::shared_ptr<const void> TensorFile::kept() const { return std::make_shared<std::pair<decltype(image), decltype(inflated)>>(image, inflated); }
 
 std::vector<std::string> TensorFile::names() const {
   std::vector<std::string> out;

@@ -56,8 +56,9 @@ _WEIGHT_OPERANDS = {
 class _ResultMemory:
     """Memory of results.  A result of many pages in fresh memory costs more in page faults than in data (75 MB of
     floats: 6.3 ms against 2.6 in pages that are mapped), so an array handed out stays known here and its memory is
-    handed out again once the caller has dropped it -- the array, its views, whatever holds one of them.  At most LIMIT
-    bytes are kept; they go with the module or its next load()."""
+    handed out again once the caller has dropped it -- the array, its views, whatever holds one of them.  The first array
+    of a shape is the caller's alone: what is read once leaves nothing behind.  At most LIMIT bytes are kept; they go with
+    the module or its next load()."""
     SMALL = 64 << 10     # below this the allocator gives mapped memory anyway
     LIMIT = 256 << 20
 
@@ -71,7 +72,11 @@ class _ResultMemory:
     def take(self, shape, dtype):
         """(array, its address)"""
         with self._lock:
-            kept = self._kept.setdefault((shape, dtype), [])
+            kept = self._kept.get((shape, dtype))
+            if kept is None:
+                self._kept[shape, dtype] = []
+                out = np.empty(shape, dtype)
+                return out, out.ctypes.data
             for owner, address in kept:
                 if sys.getrefcount(owner) == 3:      # the list's tuple, this loop, the call: no array of a caller
                     return owner.view(), address
