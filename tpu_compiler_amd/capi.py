@@ -349,7 +349,7 @@ class DeviceTensor:
 # pointers or numpy's view of an address.  These functions take packed bytes instead, through function objects of their own
 # whose pointer arguments all accept them.
 _OPS = ("conv2d_i8", "fc_i8", "fc_batched_i8", "eltwise_add_i8", "move_i8", "binary_i8", "lut_i8", "leaky_relu_i8", "relu_i8",
-        "upsample_nearest_i8", "concat_i8")
+        "upsample_nearest_i8", "concat_i8", "pool_max_i8", "pool_avg_i8")
 _SCALARS = (C.c_int, C.c_size_t, C.c_uint32)
 _pack_move, _pack_binary = struct.Struct("19i").pack, struct.Struct("21i").pack
 _ZEROS = (0,) * 8
@@ -361,6 +361,14 @@ def _pack_ints(pack, values):
         return pack(*values)
     except struct.error:
         return b"".join(bytes(C.c_int(v)) for v in values)
+
+
+def _packed(code, values, dtype):
+    """the bytes of a sequence of numbers: what numpy makes of them, by a shorter way where they are ints that fit"""
+    try:
+        return struct.pack("%d%s" % (len(values), code), *values)
+    except (struct.error, TypeError):
+        return np.ascontiguousarray(values, dtype=dtype).tobytes()
 
 
 class _Ops:
@@ -665,7 +673,7 @@ class Context:
 
     def eltwise_add(self, xs, mult, rshift, do_relu, y):
         ptrs = struct.pack("%dP" % len(xs), *[t.ptr for t in xs])
-        m = np.ascontiguousarray(mult, dtype=np.int8).tobytes()
+        m = _packed("b", mult, np.int8)
         if rc := self._ops.eltwise_add_i8(self.h, ptrs, len(xs), m, int(rshift), int(do_relu), y.ptr, y.nbytes):
             self._ck(rc)
 
@@ -698,11 +706,11 @@ class Context:
             self._ck(rc)
 
     def pool_max(self, d, x, y):
-        if rc := self.lib.tpuhip_pool_max_i8(self.h, C.byref(d), x.ptr, y.ptr):
+        if rc := self._ops.pool_max_i8(self.h, C.byref(d), x.ptr, y.ptr):
             self._ck(rc)
 
     def pool_avg(self, d, x, y, mult, rshift):
-        if rc := self.lib.tpuhip_pool_avg_i8(self.h, C.byref(d), x.ptr, y.ptr, int(mult), int(rshift)):
+        if rc := self._ops.pool_avg_i8(self.h, C.byref(d), x.ptr, y.ptr, int(mult), int(rshift)):
             self._ck(rc)
 
     def lut(self, x, y, table):
@@ -741,7 +749,7 @@ class Context:
         ptrs = struct.pack("%dP" % n, *[t.ptr for t in xs])
         dims = struct.pack("%di" % (4 * n), *[v for t in xs for v in t.shape])
         cs = struct.pack("%di" % n, *[t.cs for t in xs])
-        r = None if rshift is None else np.ascontiguousarray(rshift, dtype=np.uint32).tobytes()
-        m = None if mult is None else np.ascontiguousarray(mult, dtype=np.uint32).tobytes()
+        r = None if rshift is None else _packed("I", rshift, np.uint32)
+        m = None if mult is None else _packed("I", mult, np.uint32)
         if rc := self._ops.concat_i8(self.h, ptrs, n, dims, cs, axis, r, m, int(do_relu), y.ptr, y.cs):
             self._ck(rc)

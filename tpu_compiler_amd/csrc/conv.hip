@@ -3387,17 +3387,16 @@ __global__ __launch_bounds__(256) void fc_reduce_kernel(ConvArgs a, const v4i *p
     epilogue_rows<1, FAST>(sum, a, oc, a.qmult + oc, a.qshift + oc, a.qhpot + oc, pb * 32 + frow, 32, nullptr, out);
 }
 
-// The same product in ONE launch, for K of at least kFcOneWaves x 64: a workgroup of sixteen waves
-// per 32x32 block of outputs, wave w multiplying K steps [w * spw, (w + 1) * spw) with the
-// loads of two steps in flight at a time.  The sixteen partial sums meet in LDS (64 KiB,
-// [wave][quarter][lane] of four dwords): every thread adds one quarter of four waves in place,
-// wave 0 adds the four groups and the bias and runs the epilogue.  No scratch in device
-// memory and no second launch, which on a classifier of 32 rows is most of the time.
-constexpr int kFcOneWaves = 16;
-
-template <bool FAST>
-__global__ __launch_bounds__(64 * kFcOneWaves) void fc_one_kernel(ConvArgs a, int steps_per_wave) {
-  __shared__ v4i part[kFcOneWaves * 4 * 64];
+// The same product in ONE launch: a workgroup of W waves per 32x32 block of outputs, wave w multiplying
+// K steps [w * spw, (w + 1) * spw) with the loads of two steps in flight at a time.  The W partial sums
+// meet in LDS ([wave][quarter][lane] of four dwords): every thread adds one quarter of four waves in
+// place, wave 0 adds the groups and the bias and runs the epilogue.  No scratch in device memory and no
+// second launch, which on a classifier of 32 rows is most of the time.  Four, eight or sixteen waves: the
+// fewest that request all of their K at once (K of 512 or 1024), sixteen beyond.  (K below 1024 took the
+// two launches: 22 x 232 x 23 in 8.0 us, 4.2 in one.)
+template <bool FAST, int W>
+__global__ __launch_bounds__(64 * W) void fc_one_kernel(ConvArgs a, int steps_per_wave) {
+  __shared__ v4i part[W * 4 * 64];
   gather_conv_args(a);
   gather_conv_args_more(a);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -3457,7 +3456,7 @@ __global__ __launch_bounds__(64 * kFcOneWaves) void fc_one_kernel(ConvArgs a, in
   for (int q = 0; q < 4; ++q) {
     v4i t = *reinterpret_cast<const v4i *>(a.bias + oc + q * 4);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) t += part[((g * 4) * 4 + q) * 64 + lane];
+    for (int g = 0; g < W / 4; ++g) t += part[((g * 4) * 4 + q) * 64 + lane];
     sum[0][q * 4 + 0] = t[0]; sum[0][q * 4 + 1] = t[1]; sum[0][q * 4 + 2] = t[2]; sum[0][q * 4 + 3] = t[3];
   }
   const OutRoute out{a.y, a.y_cs, a.lo, 0};
@@ -5066,9 +5065,12 @@ static int run_fc_one(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void 
   const int nsteps = w->kp / 64;
   const int64_t tiles = (int64_t)((w->d.n + 31) / 32) * a.n_oc_tiles;
   TPUHIP_REQUIRE(tiles < (1ll << 31), "fc: too many blocks of 32 x 32 outputs");
-  const int steps_per_wave = (nsteps + kFcOneWaves - 1) / kFcOneWaves;
-  auto kernel = w->fast ? fc_one_kernel<true> : fc_one_kernel<false>;
-  const dim3 grid((unsigned)tiles), block(64 * kFcOneWaves);
+  const int waves = nsteps <= 8 ? 4 : nsteps <= 16 ? 8 : 16;
+  const int steps_per_wave = (nsteps + waves - 1) / waves;
+  auto kernel = waves == 4   ? (w->fast ? fc_one_kernel<true, 4> : fc_one_kernel<false, 4>)
+                : waves == 8 ? (w->fast ? fc_one_kernel<true, 8> : fc_one_kernel<false, 8>)
+                             : (w->fast ? fc_one_kernel<true, 16> : fc_one_kernel<false, 16>);
+  const dim3 grid((unsigned)tiles), block(64 * waves);
   if (ctx->prof_start || ctx->prof_stop)
     hipExtLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a, steps_per_wave);
   else
@@ -5100,9 +5102,7 @@ int tpuhip_fc_i8(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, v
   TPUHIP_REQUIRE(ctx && w && x && y, "tpuhip_fc_i8: NULL argument");
   FcPlan p;
   if (!fc_splitk_plan(ctx, w, &p)) return run_conv(ctx, w, x, y, PostOps{});   // many rows: the conv path
-  if (w->kp / 64 >= kFcOneWaves) return run_fc_one(ctx, w, x, y);              // long K: one launch
-  if (int rc = grow_workspace(ctx, p.bytes)) return rc;
-  return run_fc_splitk(ctx, w, x, y, ctx->workspace, p);
+  return run_fc_one(ctx, w, x, y);
 }
 
 int tpuhip_fc_i8_noalloc(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y) {

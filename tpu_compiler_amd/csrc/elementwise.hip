@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 using namespace tpuhip;
 
@@ -30,21 +31,21 @@ __device__ __forceinline__ int32_t sb(int32_t word, int i) {
 // sum / 2^r in float; both are exact for |sum| < 2^24 (at most 8 inputs of
 // 128 * 128), so the integer form floor((sum + 2^(r-1)) / 2^r) is identical.
 // ---------------------------------------------------------------------------
+template <int NIN>
 struct EltArgs {
-  const int8_t *x[8];
+  const int8_t *x[NIN];
   int8_t *y;
-  int32_t m[8];
-  int nin;
+  int32_t m[NIN];
   int rshift;
   int relu;
   int64_t n16;   // number of 16-byte groups
 };
 
+// one group a thread (two of them one after the other: 4.4 us on 4 x 120 x 75 x 75, now 3.4)
 template <int NIN>
-__global__ __launch_bounds__(kThreads) void eltwise_add_kernel(EltArgs a) {
+__global__ __launch_bounds__(kThreads) void eltwise_add_kernel(EltArgs<NIN> a) {
   const int32_t rnd = a.rshift > 0 ? (1 << (a.rshift - 1)) : 0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n16;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < a.n16; i += (int64_t)gridDim.x * kThreads) {
     v4i in[NIN];
 #pragma unroll
     for (int k = 0; k < NIN; ++k) in[k] = reinterpret_cast<const v4i *>(a.x[k])[i];
@@ -125,6 +126,37 @@ __device__ __forceinline__ uint32_t look_up4(uint32_t w, const uint8_t *tab, int
   return o & (valid >= 4 ? 0xffffffffu : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u);
 }
 
+// A table that follows from numbers, made by the kernel: thread v & 255 computes the entry of input v.  (Its 256 bytes as an
+// argument cost a launch 0.5 us and the host's loop 0.2 us or more.)  The float overload of
+// applyMultiplierAndRShiftAndSaturateInt8: product, quotient by a power of two, floor(f + 0.5), clamp.
+__device__ __forceinline__ int32_t rescaled(int32_t v, float m, float inv_pot) {
+  return saturate_int8_f(__fmul_rn(__fmul_rn((float)v, m), inv_pot));
+}
+struct LeakyRule {
+  float m_pos, inv_pos, m_neg, inv_neg;   // m_pos 0: positive inputs stay
+};
+__device__ __forceinline__ void park_leaky(const LeakyRule &r, uint32_t *lds) {
+  const int32_t v = (int32_t)(int8_t)threadIdx.x;
+  const int32_t o = v <= 0 ? rescaled(v, r.m_neg, r.inv_neg) : r.m_pos != 0.f ? rescaled(v, r.m_pos, r.inv_pos) : v;
+  reinterpret_cast<int8_t *>(lds)[threadIdx.x] = (int8_t)o;
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(kThreads) void leaky_vec_kernel(LutArgs a, LeakyRule rule) {
+  __shared__ uint32_t tab[64];
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const bool live = i < a.pixels * a.by_groups.d;
+  uint32_t r = (uint32_t)i;
+  const int64_t pix = a.by_groups.split(r);
+  const int cg = (int)r;
+  v4i v = {0, 0, 0, 0};
+  if (live) v = *reinterpret_cast<const v4i *>(a.x + pix * a.x_cs + cg * 16);
+  park_leaky(rule, tab);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = (int)look_up4((uint32_t)v[q], reinterpret_cast<const uint8_t *>(tab), a.c - cg * 16 - q * 4);
+  if (live) *reinterpret_cast<v4i *>(a.y + pix * a.y_cs + cg * 16) = v;
+}
+
 // vector form: groups of 16 channels, strides multiple of 16, coff multiple of 16.  One group per thread: 4 x 120 x 75 x 75 in
 // 3.1 us (8.2 with four groups after one another in a quarter of the threads and a table spread by 64 selects).
 __global__ __launch_bounds__(kThreads) void lut_vec_kernel(LutArgs a, Table256 t) {
@@ -166,55 +198,70 @@ constexpr int kConcatMax = 6;
 // along the channels: a thread makes 16 channels of an output pixel.  A dword that lies inside one input is one load at any
 // alignment; one that straddles two is put together from bytes.  (Inputs off the 16-channel grid went byte by byte, a
 // launch each and one for the pad channels: 4 x (120 + 120) x 75 x 75 in 22 us, now 5.4, with tables 6.3.)
+template <int N>
 struct ConcatChannelArgs {
-  const int8_t *x[kConcatMax];
+  const int8_t *x[N];
   int8_t *y;
-  int start[kConcatMax + 1];   // first output channel of each input; start[n] = output channels
-  int cs[kConcatMax];
-  int n, y_cs, tables;         // tables: bit k set where input k has one
+  int start[N + 1];            // first output channel of each input; start[N] = output channels
+  int cs[N];
+  int y_cs;
   FastDiv by_groups;           // groups written per pixel
-  int64_t total;
+  uint32_t total;
 };
-struct Tables {
-  Table256 t[kConcatMax];
+// requantisation and ReLU of each input: tables made by the kernel
+template <int N>
+struct ConcatRules {
+  float m[N], inv_pot[N];      // m 0 with inv_pot 0: values stay
+  int relu;
 };
-
-__global__ __launch_bounds__(kThreads) void concat_channels_kernel(ConcatChannelArgs a, Tables t) {
-  __shared__ uint32_t tab[kConcatMax * 64];
-  if (a.tables) {
-    for (int k = threadIdx.x; k < a.n * 64; k += kThreads) tab[k] = t.t[k >> 6].w[k & 63];
-    __syncthreads();
+template <int N>
+__device__ __forceinline__ void park_rules(const ConcatRules<N> &r, uint32_t *tab) {
+  const int32_t v = (int32_t)(int8_t)threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    int32_t o = r.inv_pot[k] != 0.f ? rescaled(v, r.m[k], r.inv_pot[k]) : v;
+    if (r.relu) o = max(o, 0);
+    reinterpret_cast<int8_t *>(tab + k * 64)[threadIdx.x] = (int8_t)o;
   }
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  __syncthreads();
+}
+struct NoRules {};
+
+// Two inputs have kernels of their own: their arguments stay below the 112 bytes up to which a launch is 0.5 us cheaper.
+template <int N, class Rules>
+__global__ __launch_bounds__(kThreads) void concat_channels_kernel(ConcatChannelArgs<N> a, Rules rules) {
+  constexpr bool kTables = !std::is_same<Rules, NoRules>::value;
+  __shared__ uint32_t tab[kTables ? N * 64 : 1];
+  if constexpr (kTables) park_rules<N>(rules, tab);
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= a.total) return;
-  uint32_t r = (uint32_t)i;
+  uint32_t r = i;
   const int64_t pix = a.by_groups.split(r);
   const int c0 = (int)r * 16;
   v4i out;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int c = c0 + q * 4;
-    int k = 0;
-#pragma unroll
-    for (int j = 1; j < kConcatMax; ++j)
-      if (j < a.n && c >= a.start[j]) k = j;
     const int8_t *src = a.x[0];
-    int first = 0, last = a.start[1], cs = a.cs[0];
+    int k = 0, first = 0, last = a.start[1], cs = a.cs[0];
 #pragma unroll
-    for (int j = 1; j < kConcatMax; ++j)
-      if (k == j) { src = a.x[j]; first = a.start[j]; last = a.start[j + 1]; cs = a.cs[j]; }
+    for (int j = 1; j < N; ++j)
+      if (c >= a.start[j]) { k = j; src = a.x[j]; first = a.start[j]; last = a.start[j + 1]; cs = a.cs[j]; }
     uint32_t w = 0;
     if (c + 4 <= last) {
       __builtin_memcpy(&w, src + pix * cs + (c - first), 4);
-      if (a.tables >> k & 1) w = look_up4(w, reinterpret_cast<const uint8_t *>(tab + k * 64), 4);
+      if constexpr (kTables) w = look_up4(w, reinterpret_cast<const uint8_t *>(tab + k * 64), 4);
     } else {
       for (int b = 0; b < 4; ++b) {
         const int cb = c + b;
-        if (cb >= a.start[a.n]) break;   // pad channels are zero
-        int kb = 0;
-        while (kb + 1 < a.n && cb >= a.start[kb + 1]) ++kb;
-        uint32_t v = (uint8_t)a.x[kb][pix * a.cs[kb] + (cb - a.start[kb])];
-        if (a.tables >> kb & 1) v = reinterpret_cast<const uint8_t *>(tab + kb * 64)[v];
+        if (cb >= a.start[N]) break;   // pad channels are zero
+        const int8_t *from = a.x[0];
+        int kb = 0, at = 0, bcs = a.cs[0];
+#pragma unroll
+        for (int j = 1; j < N; ++j)
+          if (cb >= a.start[j]) { kb = j; from = a.x[j]; at = a.start[j]; bcs = a.cs[j]; }
+        uint32_t v = (uint8_t)from[pix * bcs + (cb - at)];
+        if constexpr (kTables) v = reinterpret_cast<const uint8_t *>(tab + kb * 64)[v];
         w |= v << (8 * b);
       }
     }
@@ -232,16 +279,15 @@ struct ConcatArgs {
   int64_t stride[kConcatMax];    // bytes from one outer index to the next in each input
   int64_t y_stride;              // ... in the output
   int64_t start[kConcatMax + 1]; // first 16-byte group of each input's chunk within an output chunk; start[n] = groups per chunk
-  int n, c, tables;
+  int n, c;
   FastDiv by_groups, by_c16;     // groups per outer index, per pixel
 };
 
-__global__ __launch_bounds__(kThreads) void concat_chunks_kernel(ConcatArgs a, Tables t) {
-  __shared__ uint32_t tab[kConcatMax * 64];
-  if (a.tables) {
-    for (int k = threadIdx.x; k < a.n * 64; k += kThreads) tab[k] = t.t[k >> 6].w[k & 63];
-    __syncthreads();
-  }
+template <class Rules>
+__global__ __launch_bounds__(kThreads) void concat_chunks_kernel(ConcatArgs a, Rules rules) {
+  constexpr bool kTables = !std::is_same<Rules, NoRules>::value;
+  __shared__ uint32_t tab[kTables ? kConcatMax * 64 : 1];
+  if constexpr (kTables) park_rules<kConcatMax>(rules, tab);
   const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (i >= a.outer * a.start[a.n]) return;
   uint32_t g = (uint32_t)i;
@@ -254,7 +300,7 @@ __global__ __launch_bounds__(kThreads) void concat_chunks_kernel(ConcatArgs a, T
   for (int j = 1; j < kConcatMax; ++j)
     if (a.n > j && g >= a.start[j]) { src = a.x[j]; stride = a.stride[j]; first = a.start[j]; k = j; }
   v4i v = *reinterpret_cast<const v4i *>(src + o * stride + (g - first) * 16);
-  if (a.tables >> k & 1) {
+  if constexpr (kTables) {
     uint32_t cg = g;   // chunks are whole pixels, so the group's place in its pixel follows from g alone
     a.by_c16.split(cg);
 #pragma unroll
@@ -685,27 +731,29 @@ int tpuhip_eltwise_add_i8(tpuhip_ctx *ctx, const void *const *xs, int nin,
   TPUHIP_REQUIRE(rshift >= 0 && rshift <= 30, "eltwise_add: rshift %d outside [0,30]", rshift);
   TPUHIP_REQUIRE(bytes % 16 == 0, "eltwise_add: byte count %zu not a multiple of 16", bytes);
   if (bytes == 0) return TPUHIP_OK;
-  EltArgs a{};
-  for (int i = 0; i < nin; ++i) {
-    TPUHIP_REQUIRE(xs[i], "eltwise_add: input %d is NULL", i);
-    a.x[i] = (const int8_t *)xs[i];
-    a.m[i] = multiplier[i];
-  }
-  a.y = (int8_t *)y;
-  a.nin = nin;
-  a.rshift = rshift;
-  a.relu = do_relu ? 1 : 0;
-  a.n16 = (int64_t)(bytes / 16);
-  const dim3 grid(grid_for(a.n16, kThreads * 2)), block(kThreads);
+  for (int i = 0; i < nin; ++i) TPUHIP_REQUIRE(xs[i], "eltwise_add: input %d is NULL", i);
+  auto run = [&](auto count) {
+    constexpr int NIN = decltype(count)::value;
+    EltArgs<NIN> a{};
+    for (int i = 0; i < NIN; ++i) {
+      a.x[i] = (const int8_t *)xs[i];
+      a.m[i] = multiplier[i];
+    }
+    a.y = (int8_t *)y;
+    a.rshift = rshift;
+    a.relu = do_relu ? 1 : 0;
+    a.n16 = (int64_t)(bytes / 16);
+    launch(ctx, eltwise_add_kernel<NIN>, dim3(grid_for(a.n16, kThreads, 1 << 20)), dim3(kThreads), a);
+  };
   switch (nin) {
-    case 1: launch(ctx, eltwise_add_kernel<1>, grid, block, a); break;
-    case 2: launch(ctx, eltwise_add_kernel<2>, grid, block, a); break;
-    case 3: launch(ctx, eltwise_add_kernel<3>, grid, block, a); break;
-    case 4: launch(ctx, eltwise_add_kernel<4>, grid, block, a); break;
-    case 5: launch(ctx, eltwise_add_kernel<5>, grid, block, a); break;
-    case 6: launch(ctx, eltwise_add_kernel<6>, grid, block, a); break;
-    case 7: launch(ctx, eltwise_add_kernel<7>, grid, block, a); break;
-    default: launch(ctx, eltwise_add_kernel<8>, grid, block, a); break;
+    case 1: run(std::integral_constant<int, 1>()); break;
+    case 2: run(std::integral_constant<int, 2>()); break;
+    case 3: run(std::integral_constant<int, 3>()); break;
+    case 4: run(std::integral_constant<int, 4>()); break;
+    case 5: run(std::integral_constant<int, 5>()); break;
+    case 6: run(std::integral_constant<int, 6>()); break;
+    case 7: run(std::integral_constant<int, 7>()); break;
+    default: run(std::integral_constant<int, 8>()); break;
   }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
@@ -817,11 +865,27 @@ int tpuhip_clip_table(float minv, float maxv, uint32_t rshift, uint32_t multipli
 int tpuhip_leaky_relu_i8(tpuhip_ctx *ctx, const void *x, void *y, size_t pixels, int c, int cs,
                          uint32_t rshift_pos, uint32_t multiplier_pos, uint32_t rshift_neg,
                          uint32_t multiplier_neg) {
-  int8_t table[256];
-  if (int rc = tpuhip_leaky_relu_table(rshift_pos, multiplier_pos, rshift_neg, multiplier_neg,
-                                       table))
-    return rc;
-  return tpuhip_lut_i8(ctx, x, y, table, pixels, c, cs);
+  TPUHIP_REQUIRE(rshift_pos <= 30 && rshift_neg <= 30, "leaky_relu: rshift outside [0,30]");
+  TPUHIP_REQUIRE(ctx && x && y, "leaky_relu: NULL argument");
+  TPUHIP_REQUIRE(c > 0 && cs >= c && cs % 16 == 0, "leaky_relu: bad channels %d / stride %d", c, cs);
+  if (pixels == 0) return TPUHIP_OK;
+  const int groups = (c + 15) / 16;
+  if ((int64_t)pixels * groups >= (1ll << 31)) {
+    int8_t table[256];
+    if (int rc = tpuhip_leaky_relu_table(rshift_pos, multiplier_pos, rshift_neg, multiplier_neg, table)) return rc;
+    return tpuhip_lut_i8(ctx, x, y, table, pixels, c, cs);
+  }
+  LutArgs a{};
+  a.x = (const int8_t *)x;
+  a.y = (int8_t *)y;
+  a.pixels = (int64_t)pixels;
+  a.c = c;
+  a.x_cs = a.y_cs = cs;
+  a.by_groups = FastDiv(groups);
+  launch(ctx, leaky_vec_kernel, dim3((unsigned)ceil_div64((int64_t)pixels * groups, kThreads)), dim3(kThreads), a,
+         LeakyRule{(float)multiplier_pos, 1.0f / (float)(1 << rshift_pos), (float)multiplier_neg, 1.0f / (float)(1 << rshift_neg)});
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
 }
 
 int tpuhip_relu_i8(tpuhip_ctx *ctx, const void *x, void *y, size_t bytes) {
@@ -906,36 +970,46 @@ int tpuhip_concat_i8(tpuhip_ctx *ctx, const void *const *xs, int nin, const int 
   for (int i = 0; i < nin && one && axis != 1; ++i) one = in_cs[i] == y_cs && y_cs == round_up(Cc, 16);
   if (one) {
     TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
-    Tables t{};
-    int tables = 0;
-    for (int i = 0; i < nin; ++i) {
-      int8_t table[256];
-      if (!(need_quant || do_relu) || !table_of(i, table)) continue;
-      t.t[i] = pack_table(table);
-      tables |= 1 << i;
-    }
-    if (axis == 1) {
-      ConcatChannelArgs a{};
-      a.y = (int8_t *)y;
-      a.n = nin;
-      a.y_cs = y_cs;
-      a.tables = tables;
-      for (int i = 0; i < nin; ++i) {
-        a.x[i] = (const int8_t *)xs[i];
-        a.cs[i] = in_cs[i];
-        a.start[i + 1] = a.start[i] + in_dims[4 * i + 1];
+    const bool rules = need_quant || do_relu;
+    auto fill_rules = [&](auto &r, int n) {
+      for (int i = 0; i < n; ++i) {
+        const bool stays = i >= nin || !need_quant || (multiplier[i] == 1 && rshift[i] == 0);
+        r.m[i] = stays ? 0.f : (float)multiplier[i];
+        r.inv_pot[i] = stays ? 0.f : 1.0f / (float)(1 << rshift[i]);
       }
-      for (int i = nin; i < kConcatMax; ++i) a.start[i + 1] = a.start[nin];
-      // the output's stride may be wider than its channels: the pad groups are written as zero
-      a.by_groups = FastDiv(y_cs / 16);
-      a.total = (int64_t)N * H * W * (y_cs / 16);
-      launch(ctx, concat_channels_kernel, dim3((unsigned)ceil_div64(a.total, kThreads)), dim3(kThreads), a, t);
+      r.relu = do_relu ? 1 : 0;
+    };
+    if (axis == 1) {
+      auto run = [&](auto count) {
+        constexpr int M = decltype(count)::value;
+        ConcatChannelArgs<M> a{};
+        a.y = (int8_t *)y;
+        a.y_cs = y_cs;
+        for (int i = 0; i < M; ++i) {   // inputs that are not there start where the channels end
+          a.x[i] = (const int8_t *)xs[std::min(i, nin - 1)];
+          a.cs[i] = in_cs[std::min(i, nin - 1)];
+          a.start[i + 1] = a.start[i] + (i < nin ? in_dims[4 * i + 1] : 0);
+        }
+        // the output's stride may be wider than its channels: the pad groups are written as zero
+        a.by_groups = FastDiv(y_cs / 16);
+        a.total = (uint32_t)((int64_t)N * H * W * (y_cs / 16));
+        const dim3 grid((unsigned)ceil_div64(a.total, kThreads));
+        if (!rules) {
+          launch(ctx, concat_channels_kernel<M, NoRules>, grid, dim3(kThreads), a, NoRules());
+          return;
+        }
+        ConcatRules<M> r{};
+        fill_rules(r, M);
+        launch(ctx, concat_channels_kernel<M, ConcatRules<M>>, grid, dim3(kThreads), a, r);
+      };
+      static_assert(sizeof(ConcatChannelArgs<2>) + sizeof(ConcatRules<2>) <= 112, "see the kernel");
+      if (nin <= 2) run(std::integral_constant<int, 2>());
+      else run(std::integral_constant<int, kConcatMax>());
     } else {
       ConcatArgs a{};
       a.y = (int8_t *)y;
       a.n = nin;
       a.c = Cc;
-      a.tables = tables;
       // bytes of one step along the axis, and of everything inside one outer index of the output
       const int64_t unit = axis == 3 ? y_cs : axis == 2 ? (int64_t)W * y_cs : (int64_t)H * W * y_cs;
       a.outer = axis == 3 ? (int64_t)N * H : axis == 2 ? N : 1;
@@ -947,7 +1021,14 @@ int tpuhip_concat_i8(tpuhip_ctx *ctx, const void *const *xs, int nin, const int 
       }
       a.by_groups = FastDiv(a.start[nin]);
       a.by_c16 = FastDiv(y_cs / 16);
-      launch(ctx, concat_chunks_kernel, dim3((unsigned)ceil_div64(a.outer * a.start[nin], kThreads)), dim3(kThreads), a, t);
+      const dim3 grid((unsigned)ceil_div64(a.outer * a.start[nin], kThreads));
+      if (rules) {
+        ConcatRules<kConcatMax> r{};
+        fill_rules(r, kConcatMax);
+        launch(ctx, concat_chunks_kernel<ConcatRules<kConcatMax>>, grid, dim3(kThreads), a, r);
+      } else {
+        launch(ctx, concat_chunks_kernel<NoRules>, grid, dim3(kThreads), a, NoRules());
+      }
     }
     TPUHIP_CHECK_HIP(hipGetLastError());
     return TPUHIP_OK;

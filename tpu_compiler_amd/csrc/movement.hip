@@ -17,11 +17,13 @@ constexpr int kThreads = 256;
 
 // the index maps; the three that move single channels are at the end
 enum Form {
-  kPadConst, kPadEdge, kCrop, kReorg, kTile, kTileChannel, kReverse, kDilate, kReflectionPad, kDepthDcr,
+  kPadConst, kPadCut, kPadEdge, kCrop, kReorg, kTile, kTileChannel, kReverse, kDilate, kReflectionPad, kDepthDcr,
   kReverseChannel, kShuffle, kSwap, kStrided
 };
 
-struct MoveArgs {
+// What a kernel reads of it is in the MoveArgs of its form: up to 112 bytes of arguments a launch costs the host 3.1 us
+// back to back, with more 3.65 us, and these kernels take less than that (ten of them on 4 x 96 x 78 x 66: 43 -> 38 us).
+struct MovePlan {
   const int8_t *x;
   int8_t *y;
   int in, ic, ih, iw, ics;
@@ -30,9 +32,95 @@ struct MoveArgs {
   int fill;        // the byte of an element without a source (0 except for Dilate)
   FastDiv by_groups, by_ow, by_oh;
   FastDiv by_a, by_b, by_c;   // what the map divides by
-  uint32_t pix0;   // first output pixel of this launch
-  int64_t total;   // output pixels * (ocs / 16) of this launch, below 2^31
 };
+
+struct MoveBase {
+  const int8_t *x;
+  int8_t *y;
+  int ih, iw, ics, oc;
+  FastDiv by_groups, by_ow, by_oh;
+  uint32_t pix0;   // first output pixel of this launch
+  uint32_t total;  // output pixels * 16-channel groups of this launch, below 2^31
+  __host__ __device__ int ocs() const { return (int)by_groups.d * 16; }
+};
+template <int N, bool A = false, bool B = false>
+struct MoveTail {
+  int ic;
+  int p[N];
+  FastDiv by_a, by_b;
+  void take(const MovePlan &m) {
+    ic = m.ic;
+    for (int k = 0; k < N; ++k) p[k] = m.p[k];
+    by_a = m.by_a, by_b = m.by_b;
+  }
+};
+template <int N>
+struct MoveTail<N, true, false> {
+  int ic;
+  int p[N];
+  FastDiv by_a;
+  void take(const MovePlan &m) {
+    ic = m.ic;
+    for (int k = 0; k < N; ++k) p[k] = m.p[k];
+    by_a = m.by_a;
+  }
+};
+template <int N>
+struct MoveTail<N, false, false> {
+  int ic;
+  int p[N];
+  void take(const MovePlan &m) {
+    ic = m.ic;
+    for (int k = 0; k < N; ++k) p[k] = m.p[k];
+  }
+};
+struct MoveTailTile {
+  FastDiv by_a, by_b, by_c;
+  void take(const MovePlan &m) { by_a = m.by_a, by_b = m.by_b, by_c = m.by_c; }
+};
+struct MoveTailDilate {
+  int fill;
+  FastDiv by_a, by_b;
+  void take(const MovePlan &m) { fill = m.fill, by_a = m.by_a, by_b = m.by_b; }
+};
+struct MoveTailCrop {   // p[0..7] less the channels' step
+  int p[8];
+  void take(const MovePlan &m) {
+    for (int k = 0; k < 8; ++k) p[k] = m.p[k];
+    p[5] = m.ic;
+  }
+};
+struct MoveTailReverse {
+  int in, axis;
+  void take(const MovePlan &m) { in = m.in, axis = m.p[0]; }
+};
+struct MoveTailDepth {
+  int ow;
+  void take(const MovePlan &m) { ow = m.ow; }
+};
+
+template <Form F> struct TailOf { using type = MoveTail<1>; };                     // kReflectionPad, kReverseChannel
+template <> struct TailOf<kPadConst> { using type = MoveTail<5>; };                // p[4]: input images
+template <> struct TailOf<kPadCut> { using type = MoveTail<12>; };
+template <> struct TailOf<kPadEdge> { using type = MoveTail<4>; };
+template <> struct TailOf<kCrop> { using type = MoveTailCrop; };
+template <> struct TailOf<kReorg> { using type = MoveTail<1, true, true>; };
+template <> struct TailOf<kTile> { using type = MoveTailTile; };
+template <> struct TailOf<kTileChannel> { using type = MoveTail<1, true>; };
+template <> struct TailOf<kReverse> { using type = MoveTailReverse; };
+template <> struct TailOf<kDilate> { using type = MoveTailDilate; };
+template <> struct TailOf<kDepthDcr> { using type = MoveTail<1, true>; };
+template <> struct TailOf<kShuffle> { using type = MoveTail<2, true>; };
+template <> struct TailOf<kSwap> { using type = MoveTail<8>; };
+template <> struct TailOf<kStrided> { using type = MoveTail<9, true>; };
+
+template <class Tail>
+struct MoveWith : MoveBase, Tail {};
+template <Form F>
+using MoveArgs = MoveWith<typename TailOf<F>::type>;
+static_assert(sizeof(MoveArgs<kTile>) <= 112 && sizeof(MoveArgs<kCrop>) <= 112 && sizeof(MoveArgs<kReorg>) <= 112 &&
+                  sizeof(MoveArgs<kPadConst>) <= 112 && sizeof(MoveArgs<kSwap>) <= 112 && sizeof(MoveArgs<kDilate>) <= 112,
+              "see MovePlan");
 
 // where output channel c of pixel (n, h, w) comes from, and how many channels from it on, c included, lie one after the other
 // in the source as well (p null: without a source, that many take a.fill).  A source row that ends with the output's ends in
@@ -43,9 +131,14 @@ struct Run {
 };
 
 template <Form F>
-__device__ __forceinline__ Run run_at(const MoveArgs &a, int n, int h, int w, int c) {
+__device__ __forceinline__ Run run_at(const MoveArgs<F> &a, int n, int h, int w, int c) {
   auto at = [&](int sn, int sc, int sh, int sw) { return a.x + ((int64_t)(sn * a.ih + sh) * a.iw + sw) * a.ics + sc; };
-  if constexpr (F == kPadConst) {
+  if constexpr (F == kPadConst) {   // nothing is cut: p[0..3] where the input's first element lands, p[4] its images
+    const int sn = n - a.p[0], sc = c - a.p[1], sh = h - a.p[2], sw = w - a.p[3];
+    if (sn < 0 || sn >= a.p[4] || sh < 0 || sh >= a.ih || sw < 0 || sw >= a.iw || sc >= a.ic) return {nullptr, a.oc - c};
+    if (sc < 0) return {nullptr, -sc};
+    return {at(sn, sc, sh, sw), a.ic == a.oc && sc == c ? 16 : a.ic - sc};
+  } else if constexpr (F == kPadCut) {
     // p[0..3] where the first kept input element lands, p[4..7] its index, p[8..11] end of the kept input range
     const int sn = n - a.p[0] + a.p[4], sc = c - a.p[1] + a.p[5], sh = h - a.p[2] + a.p[6], sw = w - a.p[3] + a.p[7];
     if (sn < a.p[4] || sn >= a.p[8] || sh < a.p[6] || sh >= a.p[10] || sw < a.p[7] || sw >= a.p[11] || sc >= a.p[9])
@@ -54,8 +147,8 @@ __device__ __forceinline__ Run run_at(const MoveArgs &a, int n, int h, int w, in
     return {at(sn, sc, sh, sw), a.ic == a.oc && sc == c ? 16 : a.p[9] - sc};
   } else if constexpr (F == kPadEdge) {
     return {at(n, c, min(max(h - a.p[2], 0), a.ih - 1), min(max(w - a.p[3], 0), a.iw - 1)), 16};
-  } else if constexpr (F == kCrop) {   // p[0..3] offsets, p[4..7] steps, the channels' step 1
-    return {at(n * a.p[4] + a.p[0], c + a.p[1], h * a.p[6] + a.p[2], w * a.p[7] + a.p[3]), a.ic == a.oc ? 16 : a.oc - c};
+  } else if constexpr (F == kCrop) {   // p[0..3] offsets, p[4..7] steps, but for the channels' (1), whose place has the input's channels
+    return {at(n * a.p[4] + a.p[0], c + a.p[1], h * a.p[6] + a.p[2], w * a.p[7] + a.p[3]), a.p[5] == a.oc ? 16 : a.oc - c};
   } else if constexpr (F == kReorg) {   // by_a: input channels, by_b: the stride p[0]
     uint32_t sc = (uint32_t)c, dw = a.by_a.split(sc);
     const int dh = (int)a.by_b.split(dw);
@@ -68,8 +161,8 @@ __device__ __forceinline__ Run run_at(const MoveArgs &a, int n, int h, int w, in
     uint32_t sc = (uint32_t)c;
     a.by_a.split(sc);
     return {at(n, (int)sc, h, w), a.ic - (int)sc};
-  } else if constexpr (F == kReverse) {   // p[0]: the axis
-    return {at(a.p[0] == 0 ? a.in - 1 - n : n, c, a.p[0] == 2 ? a.ih - 1 - h : h, a.p[0] == 3 ? a.iw - 1 - w : w), 16};
+  } else if constexpr (F == kReverse) {
+    return {at(a.axis == 0 ? a.in - 1 - n : n, c, a.axis == 2 ? a.ih - 1 - h : h, a.axis == 3 ? a.iw - 1 - w : w), 16};
   } else if constexpr (F == kDilate) {   // by_a = ins_w + 1, by_b = ins_h + 1: input elements sit on that grid
     uint32_t rw = (uint32_t)w, rh = (uint32_t)h;
     const int sw = (int)a.by_a.split(rw), sh = (int)a.by_b.split(rh);
@@ -87,8 +180,9 @@ __device__ __forceinline__ Run run_at(const MoveArgs &a, int n, int h, int w, in
 
 // 16 channels of runs: one load at any alignment where they lie in one run, else a dword or a byte at a time
 template <Form F>
-__device__ __forceinline__ v4i group_of_runs(const MoveArgs &a, int n, int h, int w, int c0) {
-  const uint32_t fill = (uint32_t)(uint8_t)a.fill * 0x01010101u;
+__device__ __forceinline__ v4i group_of_runs(const MoveArgs<F> &a, int n, int h, int w, int c0) {
+  uint32_t fill = 0;
+  if constexpr (F == kDilate) fill = (uint32_t)(uint8_t)a.fill * 0x01010101u;
   v4i out = {(int)fill, (int)fill, (int)fill, (int)fill};
   const Run r = run_at<F>(a, n, h, w, c0);
   if (r.left >= 16) {
@@ -116,7 +210,7 @@ __device__ __forceinline__ v4i group_of_runs(const MoveArgs &a, int n, int h, in
 
 // 16 channels that do not follow each other in the source: byte loads, all in flight, out of lines the wave shares
 template <Form F>
-__device__ __forceinline__ v4i group_of_bytes(const MoveArgs &a, int n, int h, int w, int c0) {
+__device__ __forceinline__ v4i group_of_bytes(const MoveArgs<F> &a, int n, int h, int w, int c0) {
   v4i out = {0, 0, 0, 0};
   const int live = min(a.oc - c0, 16);
   if constexpr (F == kReverseChannel) {
@@ -177,10 +271,10 @@ __device__ __forceinline__ v4i group_of_bytes(const MoveArgs &a, int n, int h, i
 // Bound by memory at size and by the launch below: on 4 x 96 x 78 x 66 the maps that a general kernel made byte by byte,
 // with the map chosen at run time, took 7 to 13 us each.
 template <Form F>
-__global__ __launch_bounds__(kThreads) void move_kernel(MoveArgs a) {
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+__global__ __launch_bounds__(kThreads) void move_kernel(MoveArgs<F> a) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= a.total) return;
-  uint32_t cg = (uint32_t)i;
+  uint32_t cg = i;
   const uint32_t pix = a.pix0 + a.by_groups.split(cg);
   uint32_t w = pix, h = a.by_ow.split(w);
   const int n = (int)a.by_oh.split(h), c0 = (int)cg * 16;
@@ -189,15 +283,15 @@ __global__ __launch_bounds__(kThreads) void move_kernel(MoveArgs a) {
     if constexpr (F >= kReverseChannel) out = group_of_bytes<F>(a, n, (int)h, (int)w, c0);
     else out = group_of_runs<F>(a, n, (int)h, (int)w, c0);
   }
-  *reinterpret_cast<v4i *>(a.y + (int64_t)pix * a.ocs + c0) = out;
+  *reinterpret_cast<v4i *>(a.y + (int64_t)pix * a.ocs() + c0) = out;
 }
 
 // depth to space by two, CRD: the four bytes of an input dword go to the same channel of four output pixels.  A lane reads 64
 // bytes of an input pixel and writes a group of each of the four.
-__global__ __launch_bounds__(kThreads) void depth_by_two_kernel(MoveArgs a) {
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+__global__ __launch_bounds__(kThreads) void depth_by_two_kernel(MoveWith<MoveTailDepth> a) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= a.total) return;
-  uint32_t cg = (uint32_t)i;
+  uint32_t cg = i;
   const uint32_t pix = a.pix0 + a.by_groups.split(cg);   // input pixel
   uint32_t w = pix;
   const uint32_t row = a.by_ow.split(w);                 // by_ow: input columns here
@@ -220,10 +314,10 @@ __global__ __launch_bounds__(kThreads) void depth_by_two_kernel(MoveArgs a) {
       out[3][q] = __builtin_amdgcn_perm(hi1, hi0, 0x07060302u);
     }
   }
-  int8_t *to = a.y + ((int64_t)row * 2 * a.ow + 2 * w) * a.ocs + c0;
+  int8_t *to = a.y + ((int64_t)row * 2 * a.ow + 2 * w) * a.ocs() + c0;
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    *reinterpret_cast<v4i *>(to + ((int64_t)(k >> 1) * a.ow + (k & 1)) * a.ocs) =
+    *reinterpret_cast<v4i *>(to + ((int64_t)(k >> 1) * a.ow + (k & 1)) * a.ocs()) =
         v4i{(int)out[k][0], (int)out[k][1], (int)out[k][2], (int)out[k][3]};
 }
 
@@ -417,44 +511,50 @@ namespace {
 // Permute without the per-byte index map.  S[k]: byte stride of input dimension k in the input,
 // T[k]: byte stride, in the output, of the output dimension that input dimension k becomes.
 // ---------------------------------------------------------------------------
-struct PermArgs {
+struct PermRowsArgs {
   const int8_t *x;
   int8_t *y;
-  int dim[4];        // input dimensions (n, c, h, w)
-  int64_t S[4], T[4];
-  int ocs;           // channel stride of the output
-  int ics;           // channel stride of the input
-  int j, a, b;       // j: the input dimension that becomes the output's channels; a, b: the other two besides c
+  int64_t S[3], T[3];   // of n, h and w
+  FastDiv by_groups, by_w, by_h;
+  int ics;              // channel stride of the input
+  uint32_t total;       // input pixels * 16-byte groups of an output row, below 2^31
 };
 
 // channels stay channels (j == 1): a pixel's channel row moves as 16-byte chunks.  The two channel
 // strides may differ (a padded stride on either side): groups of the output row beyond the input's
 // stride are written as zero, never read from the next pixel.
-__global__ __launch_bounds__(kThreads) void permute_rows_kernel(PermArgs q, int64_t total) {
-  const int c16 = q.ocs >> 4;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    const int cg = (int)(i % c16);
-    int64_t pix = i / c16;                       // input pixel (n, h, w) in input order
-    const int w = (int)(pix % q.dim[3]);
-    pix /= q.dim[3];
-    const int h = (int)(pix % q.dim[2]);
-    const int n = (int)(pix / q.dim[2]);
-    v4i v = {0, 0, 0, 0};
-    if (cg * 16 < q.ics) v = *reinterpret_cast<const v4i *>(q.x + n * q.S[0] + h * q.S[2] + w * q.S[3] + cg * 16);
-    *reinterpret_cast<v4i *>(q.y + n * q.T[0] + h * q.T[2] + w * q.T[3] + cg * 16) = v;
-  }
+__global__ __launch_bounds__(kThreads) void permute_rows_kernel(PermRowsArgs q) {
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= q.total) return;
+  uint32_t cg = i, w = q.by_groups.split(cg), h = q.by_w.split(w);   // an input pixel, in input order
+  const int64_t n = q.by_h.split(h);
+  v4i v = {0, 0, 0, 0};
+  if ((int)cg * 16 < q.ics) v = *reinterpret_cast<const v4i *>(q.x + n * q.S[0] + h * q.S[1] + w * q.S[2] + cg * 16);
+  *reinterpret_cast<v4i *>(q.y + n * q.T[0] + h * q.T[1] + w * q.T[2] + cg * 16) = v;
 }
+
+// j: the input dimension that becomes the output's channels; a, b: the other two besides c
+struct PermTileArgs {
+  const int8_t *x;
+  int8_t *y;
+  int64_t Sj, Sa, Sb, Tc, Ta, Tb;
+  FastDiv by_b;
+  int dim_j, dim_c;
+  int ocs;           // channel stride of the output
+  uint32_t plane0;   // first of this launch's (a, b) pairs
+};
+static_assert(sizeof(PermRowsArgs) <= 112 && sizeof(PermTileArgs) <= 112, "see MovePlan");
 
 // the channels change places with dimension j: 64 x 64 byte tiles through LDS, dword loads along
 // the input's channels, dword stores along the output's (pad channels of the output written as
 // zero: tile rows past the end of dimension j are zero)
-__global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermArgs q, int64_t plane0) {
+__global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermTileArgs q) {
   __shared__ __attribute__((aligned(4))) int8_t tile[64][68];
   const int c0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-  const uint32_t plane = (uint32_t)(plane0 + blockIdx.z);   // below 2^31, as all pixels are
-  const int ia = (int)(plane / (uint32_t)q.dim[q.b]), ib = (int)(plane % (uint32_t)q.dim[q.b]);
-  const int8_t *src = q.x + ia * q.S[q.a] + ib * q.S[q.b];
-  int8_t *dst = q.y + ia * q.T[q.a] + ib * q.T[q.b];
+  uint32_t ib = q.plane0 + blockIdx.z;   // below 2^31, as all pixels are
+  const int64_t ia = q.by_b.split(ib);
+  const int8_t *src = q.x + ia * q.Sa + ib * q.Sb;
+  int8_t *dst = q.y + ia * q.Ta + ib * q.Tb;
   const int tq = threadIdx.x & 15, tr = threadIdx.x >> 4;   // 16 dwords per row, 16 rows per pass
 #pragma unroll
   for (int r = tr; r < 64; r += 16) {
@@ -462,17 +562,17 @@ __global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermArgs q, int6
     uint32_t v = 0;
     // the input's pad channels are zero and its channel stride is a multiple of 16, so a dword
     // that starts inside the row may be read whole
-    if (jj < q.dim[q.j] && cc < q.dim[1]) v = *reinterpret_cast<const uint32_t *>(src + jj * q.S[q.j] + cc);
+    if (jj < q.dim_j && cc < q.dim_c) v = *reinterpret_cast<const uint32_t *>(src + jj * q.Sj + cc);
     *reinterpret_cast<uint32_t *>(&tile[r][tq * 4]) = v;
   }
   __syncthreads();
 #pragma unroll
   for (int r = tr; r < 64; r += 16) {
     const int cc = c0 + r, jj = j0 + tq * 4;
-    if (cc < q.dim[1] && jj < q.ocs) {
+    if (cc < q.dim_c && jj < q.ocs) {
       const uint32_t v = (uint32_t)(uint8_t)tile[tq * 4][r] | ((uint32_t)(uint8_t)tile[tq * 4 + 1][r] << 8) |
                          ((uint32_t)(uint8_t)tile[tq * 4 + 2][r] << 16) | ((uint32_t)(uint8_t)tile[tq * 4 + 3][r] << 24);
-      *reinterpret_cast<uint32_t *>(dst + cc * q.T[1] + jj) = v;
+      *reinterpret_cast<uint32_t *>(dst + cc * q.Tc + jj) = v;
     }
   }
 }
@@ -498,33 +598,39 @@ __global__ __launch_bounds__(kThreads) void permute_flat_kernel(FlatPermArgs q) 
   }
 }
 
+// S[k]: byte stride of input dimension k in the input, T[k]: byte stride, in the output, of the output dimension that input
+// dimension k becomes
 int run_permute(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const void *x, void *y) {
-  PermArgs q{};
-  q.x = (const int8_t *)x;
-  q.y = (int8_t *)y;
-  q.dim[0] = d->in; q.dim[1] = d->ic; q.dim[2] = d->ih; q.dim[3] = d->iw;
-  q.S[0] = (int64_t)d->ih * d->iw * d->x_cs; q.S[1] = 1; q.S[2] = (int64_t)d->iw * d->x_cs; q.S[3] = d->x_cs;
+  const int dim[4] = {d->in, d->ic, d->ih, d->iw};
+  const int64_t S[4] = {(int64_t)d->ih * d->iw * d->x_cs, 1, (int64_t)d->iw * d->x_cs, d->x_cs};
   const int64_t tout[4] = {(int64_t)d->oh * d->ow * d->y_cs, 1, (int64_t)d->ow * d->y_cs, d->y_cs};
-  for (int k = 0; k < 4; ++k) q.T[d->p[k]] = tout[k];   // output dimension k is input dimension p[k]
-  q.ocs = d->y_cs;
-  q.ics = d->x_cs;
-  q.j = d->p[1];
+  int64_t T[4];
+  for (int k = 0; k < 4; ++k) T[d->p[k]] = tout[k];   // output dimension k is input dimension p[k]
+  const int j = d->p[1];
   TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
-  if (q.j == 1) {
-    const int64_t total = (int64_t)d->in * d->ih * d->iw * (d->y_cs / 16);
-    const unsigned blocks = (unsigned)std::max<int64_t>(
-        1, std::min<int64_t>(ceil_div64(total, kThreads), (int64_t)ctx->num_cu * 32));
-    launch(ctx, permute_rows_kernel, dim3(blocks), dim3(kThreads), q, total);
+  if (j == 1) {
+    PermRowsArgs q{(const int8_t *)x, (int8_t *)y, {S[0], S[2], S[3]}, {T[0], T[2], T[3]}, FastDiv(d->y_cs / 16), FastDiv(d->iw),
+                   FastDiv(d->ih), d->x_cs, 0};
+    const int64_t image = (int64_t)d->ih * d->iw * (d->y_cs / 16);
+    TPUHIP_REQUIRE(image < (1ll << 31), "permute: an image of 2^31 16-byte groups or more");
+    const int most = (int)std::min<int64_t>(((1ll << 31) - 1) / image, d->in);   // images a 31-bit index reaches
+    for (int left = d->in; left > 0; left -= most) {
+      q.total = (uint32_t)(image * std::min(left, most));
+      launch(ctx, permute_rows_kernel, dim3((unsigned)ceil_div64(q.total, kThreads)), dim3(kThreads), q);
+      q.x += most * S[0];
+      q.y += most * T[0];
+    }
   } else {
     int rest[2], nr = 0;
     for (int k = 0; k < 4; ++k)
-      if (k != 1 && k != q.j) rest[nr++] = k;
-    q.a = rest[0];
-    q.b = rest[1];
-    const int64_t batch = (int64_t)q.dim[q.a] * q.dim[q.b];
+      if (k != 1 && k != j) rest[nr++] = k;
+    const int a = rest[0], b = rest[1];
+    PermTileArgs q{(const int8_t *)x, (int8_t *)y, S[j], S[a], S[b], T[1], T[a], T[b], FastDiv(dim[b]), dim[j], dim[1], d->y_cs, 0};
+    const int64_t batch = (int64_t)dim[a] * dim[b];
     for (int64_t p0 = 0; p0 < batch; p0 += 65535) {   // as many planes as a grid holds
       const dim3 grid((unsigned)((d->y_cs + 63) / 64), (unsigned)((d->ic + 63) / 64), (unsigned)std::min<int64_t>(batch - p0, 65535));
-      launch(ctx, permute_tile_kernel, grid, dim3(kThreads), q, p0);
+      q.plane0 = (uint32_t)p0;
+      launch(ctx, permute_tile_kernel, grid, dim3(kThreads), q);
     }
   }
   TPUHIP_CHECK_HIP(hipGetLastError());
@@ -547,7 +653,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
                  "move: tensor too large");
   const int is[4] = {d->in, d->ic, d->ih, d->iw}, os[4] = {d->on, d->oc, d->oh, d->ow};
   const int *p = d->p;
-  MoveArgs a{};
+  MovePlan a{};
   Form form = kPadConst;
   // every kind: check that the map stays inside the input for every output element
   switch (d->kind) {
@@ -560,7 +666,9 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
         a.p[4 + k] = p[k] < 0 ? -p[k] : 0;
         a.p[8 + k] = p[4 + k] < 0 ? is[k] + p[4 + k] : is[k];
         TPUHIP_REQUIRE(a.p[4 + k] <= a.p[8 + k], "pad: dimension %d is cut away entirely", k);
+        if (p[k] < 0 || p[4 + k] < 0) form = kPadCut;
       }
+      if (form == kPadConst) a.p[4] = is[0];
       break;
     case TPUHIP_MOVE_PAD_EDGE:
       TPUHIP_REQUIRE(p[0] == 0 && p[1] == 0 && p[4] == 0 && p[5] == 0, "pad: edge mode pads h and w only");
@@ -676,34 +784,41 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
   a.by_groups = FastDiv(d->y_cs / 16);
   a.by_ow = FastDiv(d->ow);
   a.by_oh = FastDiv(d->oh);
-  void (*kernel)(MoveArgs) = nullptr;
-  switch (form) {
-    case kPadConst: kernel = move_kernel<kPadConst>; break;
-    case kPadEdge: kernel = move_kernel<kPadEdge>; break;
-    case kCrop: kernel = move_kernel<kCrop>; break;
-    case kReorg: kernel = move_kernel<kReorg>; break;
-    case kTile: kernel = move_kernel<kTile>; break;
-    case kTileChannel: kernel = move_kernel<kTileChannel>; break;
-    case kReverse: kernel = move_kernel<kReverse>; break;
-    case kDilate: kernel = move_kernel<kDilate>; break;
-    case kReflectionPad: kernel = move_kernel<kReflectionPad>; break;
-    case kDepthDcr: kernel = move_kernel<kDepthDcr>; break;
-    case kReverseChannel: kernel = move_kernel<kReverseChannel>; break;
-    case kShuffle: kernel = move_kernel<kShuffle>; break;
-    case kSwap: kernel = move_kernel<kSwap>; break;
-    case kStrided: kernel = move_kernel<kStrided>; break;
-  }
-  int64_t pixels = (int64_t)d->on * d->oh * d->ow;
+  auto run = [&](auto args, auto *kernel, int64_t pixels) {
+    args.x = a.x; args.y = a.y; args.ih = a.ih; args.iw = a.iw; args.ics = a.ics; args.oc = a.oc;
+    args.by_groups = a.by_groups; args.by_ow = a.by_ow; args.by_oh = a.by_oh;
+    args.take(a);
+    const int64_t most = ((1ll << 31) - 1) / a.by_groups.d;   // as many pixels as the 31-bit index reaches
+    for (int64_t p0 = 0; p0 < pixels; p0 += most) {
+      args.pix0 = (uint32_t)p0;
+      args.total = (uint32_t)(std::min(most, pixels - p0) * a.by_groups.d);
+      launch(ctx, kernel, dim3((unsigned)ceil_div64(args.total, kThreads)), dim3(kThreads), args);
+    }
+  };
+  const int64_t pixels = (int64_t)d->on * d->oh * d->ow;
   if (d->kind == TPUHIP_MOVE_DEPTH_TO_SPACE && form == kStrided && d->p[0] == 2) {   // the factor in use, a dword per channel
-    kernel = depth_by_two_kernel;
-    pixels = (int64_t)d->in * d->ih * d->iw;
     a.by_ow = FastDiv(d->iw);
-  }
-  const int64_t most = ((1ll << 31) - 1) / a.by_groups.d;   // as many pixels as the 31-bit index reaches
-  for (int64_t p0 = 0; p0 < pixels; p0 += most) {
-    a.pix0 = (uint32_t)p0;
-    a.total = std::min(most, pixels - p0) * a.by_groups.d;
-    launch(ctx, kernel, dim3((unsigned)ceil_div64(a.total, kThreads)), dim3(kThreads), a);
+    run(MoveWith<MoveTailDepth>(), depth_by_two_kernel, (int64_t)d->in * d->ih * d->iw);
+  } else {
+    switch (form) {
+#define TPUHIP_MOVE_FORM(F) case F: run(MoveArgs<F>(), move_kernel<F>, pixels); break
+      TPUHIP_MOVE_FORM(kPadConst);
+      TPUHIP_MOVE_FORM(kPadCut);
+      TPUHIP_MOVE_FORM(kPadEdge);
+      TPUHIP_MOVE_FORM(kCrop);
+      TPUHIP_MOVE_FORM(kReorg);
+      TPUHIP_MOVE_FORM(kTile);
+      TPUHIP_MOVE_FORM(kTileChannel);
+      TPUHIP_MOVE_FORM(kReverse);
+      TPUHIP_MOVE_FORM(kDilate);
+      TPUHIP_MOVE_FORM(kReflectionPad);
+      TPUHIP_MOVE_FORM(kDepthDcr);
+      TPUHIP_MOVE_FORM(kReverseChannel);
+      TPUHIP_MOVE_FORM(kShuffle);
+      TPUHIP_MOVE_FORM(kSwap);
+      TPUHIP_MOVE_FORM(kStrided);
+#undef TPUHIP_MOVE_FORM
+    }
   }
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;

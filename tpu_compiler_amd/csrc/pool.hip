@@ -11,15 +11,19 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 namespace {
 
-struct PoolArgs {
+struct PoolArgs {   // up to 112 bytes: a launch with more of arguments costs the host 0.5 us more
   const int8_t *x;
   int8_t *y;
-  int n, c16, ih, iw, oh, ow, kh, kw, sh, sw, pt, pl, x_cs, y_cs;
+  int ih, iw, kh, kw, sh, sw, pt, pl, x_cs, y_cs;
   float mult;       // (float)multiplier
   float inv_pot;    // 2^-rshift
-  FastDiv by_c16, by_ow, by_oh, by_kw;
-  int64_t total;    // 16-channel groups of all output pixels, below 2^31 (each_part)
+  FastDiv by_c16, by_ow, by_oh;
+  uint32_t total;   // 16-channel groups of all output pixels, below 2^31 (each_part)
+  __host__ __device__ int c16() const { return (int)by_c16.d; }
+  __host__ __device__ int oh() const { return (int)by_oh.d; }
+  __host__ __device__ int ow() const { return (int)by_ow.d; }
 };
+static_assert(sizeof(PoolArgs) <= 112, "see above");
 
 __device__ __forceinline__ int32_t sb(int32_t word, int i) {
   return (int32_t)(int8_t)(word >> (8 * i));
@@ -32,39 +36,65 @@ __device__ __forceinline__ unsigned xcd_block() {
   return (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
 }
 
-// PoolingOpKernel INT8 max (core/pooling.cpp:155-157): MKL-DNN pooling_max skips
-// padded positions.
-__global__ __launch_bounds__(256) void pool_max_kernel(PoolArgs a) {
-  for (int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x; i < a.total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    uint32_t cg = (uint32_t)i, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
-    const int b = (int)a.by_oh.split(oh);
-    int32_t best[16];
+// The window positions of a thread's output group.  K > 0: a K x K window, whose loads are all requested before one is
+// used; one after the other behind their bounds checks, the nine of a 3 x 3 window took 5.7 us on 4 x 120 x 75 x 75, 3.9
+// now.  For a max, a position outside the image is the nearest one inside, which belongs to the window as well; for a sum
+// it is zero.
+template <int K, bool MAX, class F>
+__device__ __forceinline__ void each_tap(const PoolArgs &a, int b, int oh, int ow, int cg, F fn) {
+  const int8_t *base = a.x + (int64_t)b * a.ih * a.iw * a.x_cs + cg * 16;
+  if constexpr (K > 0) {
+    v4i v[K * K];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) best[k] = -128;
+    for (int kh = 0; kh < K; ++kh)
+#pragma unroll
+      for (int kw = 0; kw < K; ++kw) {
+        const int ih = oh * a.sh - a.pt + kh, iw = ow * a.sw - a.pl + kw;
+        const int h = min(max(ih, 0), a.ih - 1), w = min(max(iw, 0), a.iw - 1);
+        v4i t = *reinterpret_cast<const v4i *>(base + ((int64_t)h * a.iw + w) * a.x_cs);
+        if (!MAX && (h != ih || w != iw)) t = v4i{0, 0, 0, 0};
+        v[kh * K + kw] = t;
+      }
+#pragma unroll
+    for (int t = 0; t < K * K; ++t) fn(v[t]);
+  } else {
     for (int kh = 0; kh < a.kh; ++kh) {
-      const int ih = (int)oh * a.sh - a.pt + kh;
+      const int ih = oh * a.sh - a.pt + kh;
       if (ih < 0 || ih >= a.ih) continue;
       for (int kw = 0; kw < a.kw; ++kw) {
-        const int iw = (int)ow * a.sw - a.pl + kw;
+        const int iw = ow * a.sw - a.pl + kw;
         if (iw < 0 || iw >= a.iw) continue;
-        const v4i v = *reinterpret_cast<const v4i *>(
-            a.x + ((int64_t)(b * a.ih + ih) * a.iw + iw) * a.x_cs + cg * 16);
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) best[q * 4 + k] = max(best[q * 4 + k], sb(v[q], k));
+        fn(*reinterpret_cast<const v4i *>(base + ((int64_t)ih * a.iw + iw) * a.x_cs));
       }
     }
+  }
+}
+
+// PoolingOpKernel INT8 max (core/pooling.cpp:155-157): MKL-DNN pooling_max skips
+// padded positions.  Bytes compare as the upper halves of 16-bit words.
+template <int K>
+__global__ __launch_bounds__(256) void pool_max_kernel(PoolArgs a) {
+  typedef short v2s __attribute__((ext_vector_type(2)));
+  for (uint32_t i = xcd_block() * 256 + threadIdx.x; i < a.total; i += gridDim.x * 256) {
+    uint32_t cg = i, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
+    const int b = (int)a.by_oh.split(oh);
+    v2s best[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) best[k] = v2s{-32768, -32768};
+    each_tap<K, true>(a, b, (int)oh, (int)ow, (int)cg, [&](v4i v) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t word = (uint32_t)v[q];
+        best[q * 2] = __builtin_elementwise_max(best[q * 2], __builtin_bit_cast(v2s, word << 8));
+        best[q * 2 + 1] = __builtin_elementwise_max(best[q * 2 + 1], __builtin_bit_cast(v2s, word));
+      }
+    });
     v4i out;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint32_t w = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) w |= ((uint32_t)best[q * 4 + k] & 0xffu) << (8 * k);
-      out[q] = (int)w;
-    }
-    *reinterpret_cast<v4i *>(a.y + ((int64_t)(b * a.oh + oh) * a.ow + ow) * a.y_cs + cg * 16) = out;
+    for (int q = 0; q < 4; ++q)
+      out[q] = (int)((__builtin_bit_cast(uint32_t, best[q * 2]) >> 8 & 0x00ff00ffu) |
+                     (__builtin_bit_cast(uint32_t, best[q * 2 + 1]) & 0xff00ff00u));
+    *reinterpret_cast<v4i *>(a.y + ((int64_t)(b * a.oh() + oh) * a.ow() + ow) * a.y_cs + cg * 16) = out;
   }
 }
 
@@ -72,28 +102,20 @@ __global__ __launch_bounds__(256) void pool_max_kernel(PoolArgs a) {
 // sum with zero padding, then the float overload of
 // applyMultiplierAndRShiftAndSaturateInt8 without qdm: float product, float
 // quotient by a power of two, floor(f + 0.5), clamp.
+template <int K>
 __global__ __launch_bounds__(256) void pool_avg_kernel(PoolArgs a) {
-  for (int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x; i < a.total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    uint32_t cg = (uint32_t)i, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
+  for (uint32_t i = xcd_block() * 256 + threadIdx.x; i < a.total; i += gridDim.x * 256) {
+    uint32_t cg = i, ow = a.by_c16.split(cg), oh = a.by_ow.split(ow);
     const int b = (int)a.by_oh.split(oh);
     int32_t sum[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) sum[k] = 0;
-    for (int kh = 0; kh < a.kh; ++kh) {
-      const int ih = (int)oh * a.sh - a.pt + kh;
-      if (ih < 0 || ih >= a.ih) continue;
-      for (int kw = 0; kw < a.kw; ++kw) {
-        const int iw = (int)ow * a.sw - a.pl + kw;
-        if (iw < 0 || iw >= a.iw) continue;
-        const v4i v = *reinterpret_cast<const v4i *>(
-            a.x + ((int64_t)(b * a.ih + ih) * a.iw + iw) * a.x_cs + cg * 16);
+    each_tap<K, false>(a, b, (int)oh, (int)ow, (int)cg, [&](v4i v) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-          for (int k = 0; k < 4; ++k) sum[q * 4 + k] += sb(v[q], k);
-      }
-    }
+        for (int k = 0; k < 4; ++k) sum[q * 4 + k] += sb(v[q], k);
+    });
     v4i out;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -106,7 +128,7 @@ __global__ __launch_bounds__(256) void pool_avg_kernel(PoolArgs a) {
       }
       out[q] = (int)w;
     }
-    *reinterpret_cast<v4i *>(a.y + ((int64_t)(b * a.oh + oh) * a.ow + ow) * a.y_cs + cg * 16) = out;
+    *reinterpret_cast<v4i *>(a.y + ((int64_t)(b * a.oh() + oh) * a.ow() + ow) * a.y_cs + cg * 16) = out;
   }
 }
 
@@ -115,7 +137,7 @@ __global__ __launch_bounds__(256) void pool_avg_kernel(PoolArgs a) {
 // meet through wave shuffles.  Keeps enough loads in flight when there are few
 // outputs (a 7x7 global pool has 49 taps per output and only n*c/16 outputs).
 template <int LANES>
-__global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
+__global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a, FastDiv by_kw) {
   const int64_t gid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LANES;
   const int sub = threadIdx.x % LANES;
   const bool live = gid < a.total;
@@ -134,7 +156,7 @@ __global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
     for (int u = 0; u < MAXT; ++u) {
       const int t = t0 + u * LANES;
       uint32_t kw = (uint32_t)t;
-      const int kh = (int)a.by_kw.split(kw);
+      const int kh = (int)by_kw.split(kw);
       const int ih = (int)oh * a.sh - a.pt + kh, iw = (int)ow * a.sw - a.pl + (int)kw;
       const bool ok = (t < taps) & ((unsigned)ih < (unsigned)a.ih) & ((unsigned)iw < (unsigned)a.iw);
       v[u] = v4i{0, 0, 0, 0};
@@ -165,7 +187,7 @@ __global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
       }
       out[q] = (int)w;
     }
-    *reinterpret_cast<v4i *>(a.y + ((int64_t)(b * a.oh + oh) * a.ow + ow) * a.y_cs + cg * 16) = out;
+    *reinterpret_cast<v4i *>(a.y + ((int64_t)(b * a.oh() + oh) * a.ow() + ow) * a.y_cs + cg * 16) = out;
   }
 }
 
@@ -175,7 +197,7 @@ __global__ __launch_bounds__(256) void pool_avg_split_kernel(PoolArgs a) {
 // [output][slice][channel] and pool_avg_finish_kernel adds them.  A 75 x 75 window over 4 x 120 channels: 113 us with the
 // kernel above (its eight lanes walk 700 positions each, one workgroup), 7 us with 32 slices.
 template <int G>
-__global__ __launch_bounds__(256) void pool_avg_window_kernel(PoolArgs a, int32_t *parts, int slices, int per_slice,
+__global__ __launch_bounds__(256) void pool_avg_window_kernel(PoolArgs a, FastDiv by_kw, int32_t *parts, int slices, int per_slice,
                                                               FastDiv by_slices, FastDiv by_blocks) {
   constexpr int P = 256 / G;
   __shared__ __attribute__((aligned(16))) int32_t lds[256 * 16];
@@ -187,14 +209,14 @@ __global__ __launch_bounds__(256) void pool_avg_window_kernel(PoolArgs a, int32_
 #pragma unroll
   for (int k = 0; k < 16; ++k) sum[k] = 0;
   const int end = min(((int)slice + 1) * per_slice, a.kh * a.kw);
-  if (cg < a.c16) {
+  if (cg < a.c16()) {
     for (int t0 = (int)slice * per_slice + row; t0 < end; t0 += 4 * P) {
       v4i v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int t = t0 + u * P;
         uint32_t kw = (uint32_t)t;
-        const int kh = (int)a.by_kw.split(kw);
+        const int kh = (int)by_kw.split(kw);
         const int ih = (int)oh * a.sh - a.pt + kh, iw = (int)ow * a.sw - a.pl + (int)kw;
         v[u] = v4i{0, 0, 0, 0};
         if ((t < end) & ((unsigned)ih < (unsigned)a.ih) & ((unsigned)iw < (unsigned)a.iw))
@@ -226,21 +248,27 @@ __global__ __launch_bounds__(256) void pool_avg_window_kernel(PoolArgs a, int32_
     for (int r = 1; r < 16 / G; ++r) s += lds[r * G * 16 + ch];
   }
   const int c = (int)gb * G * 16 + ch;
-  if (c >= a.c16 * 16) return;
+  if (c >= a.c16() * 16) return;
   if (parts)
-    parts[((int64_t)pix * slices + slice) * (a.c16 * 16) + c] = s;
+    parts[((int64_t)pix * slices + slice) * (a.c16() * 16) + c] = s;
   else
     a.y[(int64_t)pix * a.y_cs + c] = (int8_t)saturate_int8_f(__fmul_rn(__fmul_rn((float)s, a.mult), a.inv_pot));
 }
 
 // adds the slices of pool_avg_window_kernel: 64 channels of an output pixel per workgroup, four threads per channel
-__global__ __launch_bounds__(256) void pool_avg_finish_kernel(PoolArgs a, const int32_t *parts, int slices) {
+struct FinishArgs {
+  const int32_t *parts;
+  int8_t *y;
+  int slices, channels, y_cs;
+  float mult, inv_pot;
+};
+__global__ __launch_bounds__(256) void pool_avg_finish_kernel(FinishArgs a) {
   __shared__ int32_t lds[256];
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63), part = threadIdx.x >> 6, all = a.c16 * 16;
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63), part = threadIdx.x >> 6, all = a.channels;
   int32_t s = 0;
   if (c < all) {
 #pragma unroll 8
-    for (int k = part; k < slices; k += 4) s += parts[((int64_t)blockIdx.y * slices + k) * all + c];
+    for (int k = part; k < a.slices; k += 4) s += a.parts[((int64_t)blockIdx.y * a.slices + k) * all + c];
   }
   lds[threadIdx.x] = s;
   __syncthreads();
@@ -251,15 +279,16 @@ __global__ __launch_bounds__(256) void pool_avg_finish_kernel(PoolArgs a, const 
 
 // more than 64 window positions for few outputs
 int run_window(tpuhip_ctx *ctx, const PoolArgs &a) {
-  const int G = a.c16 >= 16 ? 16 : a.c16 > 4 ? 8 : a.c16 > 2 ? 4 : a.c16;
-  const int gblocks = (a.c16 + G - 1) / G, taps = a.kh * a.kw;
-  const int64_t pixels = (int64_t)a.n * a.oh * a.ow, blocks = pixels * gblocks;
+  const int c16 = a.c16();
+  const int G = c16 >= 16 ? 16 : c16 > 4 ? 8 : c16 > 2 ? 4 : c16;
+  const int gblocks = (c16 + G - 1) / G, taps = a.kh * a.kw;
+  const int64_t pixels = a.total / c16, blocks = pixels * gblocks;
   // two workgroups per CU, while every lane keeps four positions; no slices where the grid of the second launch or the
   // workspace (which is not grown while the stream is being captured) does not reach
   int64_t slices = std::min<int64_t>(std::min<int64_t>(2 * ctx->num_cu / blocks, taps / (4 * 256 / G)), 32);
   if (slices < 2 || pixels > 65535) slices = 1;
   if (slices > 1) {
-    const size_t bytes = (size_t)(pixels * slices * a.c16 * 16) * sizeof(int32_t);
+    const size_t bytes = (size_t)(pixels * slices * c16 * 16) * sizeof(int32_t);
     if (ctx->workspace_bytes < bytes) {
       hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
       TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
@@ -271,11 +300,11 @@ int run_window(tpuhip_ctx *ctx, const PoolArgs &a) {
   const int per_slice = (int)((taps + slices - 1) / slices);
   auto *kernel = G == 16 ? pool_avg_window_kernel<16> : G == 8 ? pool_avg_window_kernel<8> : G == 4 ? pool_avg_window_kernel<4>
                  : G == 2 ? pool_avg_window_kernel<2> : pool_avg_window_kernel<1>;
-  launch(ctx, kernel, dim3((unsigned)(blocks * slices)), dim3(256), a, parts, (int)slices, per_slice, FastDiv(slices),
-         FastDiv(gblocks));
+  launch(ctx, kernel, dim3((unsigned)(blocks * slices)), dim3(256), a, FastDiv(a.kw), parts, (int)slices, per_slice,
+         FastDiv(slices), FastDiv(gblocks));
   if (parts)
-    launch(ctx, pool_avg_finish_kernel, dim3((unsigned)((a.c16 + 3) / 4), (unsigned)pixels), dim3(256), a, (const int32_t *)parts,
-           (int)slices);
+    launch(ctx, pool_avg_finish_kernel, dim3((unsigned)((c16 + 3) / 4), (unsigned)pixels), dim3(256),
+           FinishArgs{parts, a.y, (int)slices, c16 * 16, a.y_cs, a.mult, a.inv_pot});
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }
@@ -294,35 +323,36 @@ int fill_args(const tpuhip_pool_desc *d, const void *x, void *y, PoolArgs *a) {
                  "pool: an output window lies entirely in the padding");
   a->x = (const int8_t *)x;
   a->y = (int8_t *)y;
-  a->n = d->n; a->c16 = (d->c + 15) / 16;
-  a->ih = d->ih; a->iw = d->iw; a->oh = d->oh; a->ow = d->ow;
+  a->ih = d->ih; a->iw = d->iw;
   a->kh = d->kh; a->kw = d->kw; a->sh = d->sh; a->sw = d->sw;
   a->pt = d->pt; a->pl = d->pl; a->x_cs = d->x_cs; a->y_cs = d->y_cs;
   a->mult = 0.f; a->inv_pot = 1.f;
-  a->by_c16 = FastDiv(a->c16); a->by_ow = FastDiv(a->ow); a->by_oh = FastDiv(a->oh); a->by_kw = FastDiv(a->kw);
-  const int64_t image = (int64_t)a->oh * a->ow * a->c16;
+  a->by_c16 = FastDiv((d->c + 15) / 16); a->by_ow = FastDiv(d->ow); a->by_oh = FastDiv(d->oh);
+  const int64_t image = (int64_t)d->oh * d->ow * a->c16();
   TPUHIP_REQUIRE(image < (1ll << 31), "pool: an image of 2^31 output groups or more");
   return TPUHIP_OK;
 }
 
 // calls fn(args) for runs of images whose output groups a 31-bit index reaches
 template <class F>
-int each_part(PoolArgs a, F fn) {
-  const int64_t image = (int64_t)a.oh * a.ow * a.c16;
-  const int most = (int)std::min<int64_t>(((1ll << 31) - 1) / image, a.n);
-  for (int left = a.n; left > 0; left -= most) {
-    a.n = std::min(left, most);
-    a.total = image * a.n;
+int each_part(PoolArgs a, int n, F fn) {
+  const int64_t image = (int64_t)a.oh() * a.ow() * a.c16();
+  const int most = (int)std::min<int64_t>(((1ll << 31) - 1) / image, n);
+  for (int left = n; left > 0; left -= most) {
+    a.total = (uint32_t)(image * std::min(left, most));
     if (int rc = fn(a)) return rc;
     a.x += (int64_t)most * a.ih * a.iw * a.x_cs;
-    a.y += (int64_t)most * a.oh * a.ow * a.y_cs;
+    a.y += (int64_t)most * a.oh() * a.ow() * a.y_cs;
   }
   return TPUHIP_OK;
 }
 
+// the side of a square window, 0 otherwise
+int square(const PoolArgs &a) { return a.kh == a.kw ? a.kh : 0; }
+
 unsigned blocks_for(const PoolArgs &a) {
   // a multiple of 8 (see xcd_block)
-  return 8u * (unsigned)std::max<int64_t>(1, std::min<int64_t>((a.total + 2047) / 2048, 1 << 13));
+  return 8u * (unsigned)std::max<int64_t>(1, std::min<int64_t>(((int64_t)a.total + 2047) / 2048, 1 << 13));
 }
 
 }  // namespace
@@ -333,8 +363,9 @@ int tpuhip_pool_max_i8(tpuhip_ctx *ctx, const tpuhip_pool_desc *d, const void *x
   TPUHIP_REQUIRE(ctx, "pool_max: NULL context");
   PoolArgs a;
   if (int rc = fill_args(d, x, y, &a)) return rc;
-  return each_part(a, [&](const PoolArgs &part) -> int {
-    launch(ctx, pool_max_kernel, dim3(blocks_for(part)), dim3(256), part);
+  auto *kernel = square(a) == 3 ? pool_max_kernel<3> : square(a) == 2 ? pool_max_kernel<2> : pool_max_kernel<0>;
+  return each_part(a, d->n, [&](const PoolArgs &part) -> int {
+    launch(ctx, kernel, dim3(blocks_for(part)), dim3(256), part);
     TPUHIP_CHECK_HIP(hipGetLastError());
     return TPUHIP_OK;
   });
@@ -349,14 +380,15 @@ int tpuhip_pool_avg_i8(tpuhip_ctx *ctx, const tpuhip_pool_desc *d, const void *x
   TPUHIP_REQUIRE((int64_t)d->kh * d->kw * 128 < (1 << 24), "pool_avg: window too large");
   a.mult = (float)multiplier;
   a.inv_pot = 1.0f / (float)(1 << rshift);
-  return each_part(a, [&](const PoolArgs &part) -> int {
+  auto *kernel = square(a) == 3 ? pool_avg_kernel<3> : square(a) == 2 ? pool_avg_kernel<2> : pool_avg_kernel<0>;
+  return each_part(a, d->n, [&](const PoolArgs &part) -> int {
     // few outputs with many positions each: several lanes share one (65536 outputs fill the chip without)
     const int taps = part.kh * part.kw;
     if (taps > 64 && part.total < (1 << 16)) return run_window(ctx, part);
     if (taps >= 16 && part.total < (1 << 16))
-      launch(ctx, pool_avg_split_kernel<8>, dim3((unsigned)((part.total * 8 + 255) / 256)), dim3(256), part);
+      launch(ctx, pool_avg_split_kernel<8>, dim3((unsigned)(((int64_t)part.total * 8 + 255) / 256)), dim3(256), part, FastDiv(part.kw));
     else
-      launch(ctx, pool_avg_kernel, dim3(blocks_for(part)), dim3(256), part);
+      launch(ctx, kernel, dim3(blocks_for(part)), dim3(256), part);
     TPUHIP_CHECK_HIP(hipGetLastError());
     return TPUHIP_OK;
   });
