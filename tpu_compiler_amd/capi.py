@@ -634,7 +634,11 @@ class Context:
         self._ck(self.lib.tpuhip_conv2d_weights_destroy(self.h, w))
 
     def conv(self, w, x, y):
-        if rc := self._ops.conv2d_i8(self.h, w, x.ptr if hasattr(x, "ptr") else x, y.ptr if hasattr(y, "ptr") else y):
+        try:
+            x, y = x.ptr, y.ptr
+        except AttributeError:      # addresses
+            x, y = getattr(x, "ptr", x), getattr(y, "ptr", y)
+        if rc := self._ops.conv2d_i8(self.h, w, x, y):
             self._ck(rc)
 
     def conv_add(self, w, x, y, add_src, add_out, m_src, m_conv, rshift, do_relu):

@@ -4792,7 +4792,7 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
                  "conv: weights packed as a pair run through tpuhip_conv2d_pair_i8 (and only they do)");
   if (w->gather) {
     TPUHIP_REQUIRE(!post.any() && y, "conv: grouped and transposed convs take no fused work");
-    return gather_run(ctx, w->gather, x, y, w->bias, w->qplanes, w->qplanes + w->nparam, w->qplanes + 2 * w->nparam, w->fast != 0);
+    return gather_run(ctx, w->gather, x, y, w->bias, w->qplanes, w->nparam, w->fast != 0);
   }
   ConvArgs a;
   fill_args(ctx, w, x, y, &a);

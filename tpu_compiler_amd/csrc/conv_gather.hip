@@ -37,7 +37,6 @@ struct GatherPhase {
   int qh, qw;          // rows and columns of the phase
   int iy0, ix0;        // input row / column that tap (0, 0) of output (oh0, ow0) stands at
   int slices;          // 32-byte K slices
-  int tab;             // first table entry
   uint32_t w;          // byte offset of the phase's packed filter
 };
 
@@ -45,10 +44,9 @@ struct GatherPhase {
 
 struct GatherPlan {
   tpuhip_conv_desc d;
-  int8_t *w = nullptr;          // packed filters, then the tables, then the phases
+  int8_t *w = nullptr;          // packed filters, then a table of max_entries per phase, then the phases
   uint32_t w_bytes = 0;
-  const int2 *tab = nullptr;
-  const GatherPhase *phases = nullptr;
+  uint32_t tab_at = 0, phase_at = 0;
   int n_phases = 0, max_entries = 0, max_pixels = 0;
   int ph = 1, pw = 1, step_h = 1, step_w = 1;   // output rows / columns between two of a phase, input ones between them
   int blocks = 0;               // 32-channel blocks
@@ -59,18 +57,19 @@ namespace {
 
 constexpr int kMaxEntries = 2048;   // table entries of a phase (16 KB of LDS)
 
-struct GatherArgs {
+struct GatherArgs {   // up to 112 bytes: a launch with more of arguments costs the host 0.5 us more
   const int8_t *x, *w;
   int8_t *y;
-  const int2 *tab;
-  const GatherPhase *phases;
-  const int32_t *bias, *mult, *shift, *hpot;
-  uint32_t x_bytes, w_bytes;
+  const int32_t *bias, *planes;   // planes: multiplier, rshift and 2^(rshift-1), nparam entries each
+  int nparam;
+  uint32_t tab_at, phase_at, x_bytes, w_bytes;
   int n, ih, iw, x_cs, oh, ow, y_cs, ocw;
-  int ph, pw, step_h, step_w;
+  uint16_t ph, pw, step_h, step_w;
   int ocg, icg;      // channels per group; grouped layers only: the first channel a block reads is that of its first group
-  int lo, relu_first;
+  uint16_t entries;  // table entries per phase
+  uint8_t relu, relu_first;
 };
+static_assert(sizeof(GatherArgs) <= 112, "see above");
 
 // one 16-byte chunk of requantised channels per lane and pixel
 template <bool FAST>
@@ -83,17 +82,25 @@ __device__ __forceinline__ int32_t requant_one(int32_t v, int32_t mult, int32_t 
 
 template <int TM, int TN, bool FAST>
 __global__ __launch_bounds__(256) void conv_gather_kernel(GatherArgs a) {
-  extern __shared__ int2 stab[];
+  extern __shared__ __attribute__((aligned(16))) int8_t gather_lds[];
+  int32_t *sparam = reinterpret_cast<int32_t *>(gather_lds);              // [multiplier, rshift, 2^(rshift-1)][TM * 32]
+  int2 *stab = reinterpret_cast<int2 *>(gather_lds + 3 * TM * 32 * 4);
   constexpr int D = 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 31, half = lane >> 5;
-  const GatherPhase p = a.phases[blockIdx.z];
-  for (int i = threadIdx.x; i < 2 * p.slices; i += 256) stab[i] = a.tab[p.tab + i];
+  const int blk0 = blockIdx.y * TM;
+  // the phase, its table and the channels' parameters in one trip to memory
+  const int2 *tab = reinterpret_cast<const int2 *>(a.w + a.tab_at) + blockIdx.z * a.entries;
+  const GatherPhase p = reinterpret_cast<const GatherPhase *>(a.w + a.phase_at)[blockIdx.z];
+  int32_t param = 0;
+  if (threadIdx.x < 3 * TM * 32)
+    param = a.planes[(int)(threadIdx.x / (TM * 32)) * a.nparam + blk0 * 32 + (int)(threadIdx.x % (TM * 32))];
+  for (int i = threadIdx.x; i < a.entries; i += 256) stab[i] = tab[i];
+  if (threadIdx.x < 3 * TM * 32) sparam[threadIdx.x] = param;
   __syncthreads();
   const int npix = a.n * p.qh * p.qw;
   const int pix0 = ((int)blockIdx.x * 4 + wave) * (TN * 32);
   if (pix0 >= npix) return;
-  const int blk0 = blockIdx.y * TM;
 
   const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
@@ -163,9 +170,10 @@ __global__ __launch_bounds__(256) void conv_gather_kernel(GatherArgs a) {
       v4i o;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const v4i m = *reinterpret_cast<const v4i *>(a.mult + oc + q * 4);
-        const v4i r = *reinterpret_cast<const v4i *>(a.shift + oc + q * 4);
-        const v4i h = *reinterpret_cast<const v4i *>(a.hpot + oc + q * 4);
+        const int32_t *at = sparam + (oc - blk0 * 32) + q * 4;
+        const v4i m = *reinterpret_cast<const v4i *>(at);
+        const v4i r = *reinterpret_cast<const v4i *>(at + TM * 32);
+        const v4i h = *reinterpret_cast<const v4i *>(at + 2 * TM * 32);
         int32_t v[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -173,7 +181,7 @@ __global__ __launch_bounds__(256) void conv_gather_kernel(GatherArgs a) {
           if (a.relu_first) s = max(s, 0);
           v[e] = requant_one<FAST>(s, m[e], r[e], h[e]);
         }
-        o[q] = (int)pack_sat4(v[0], v[1], v[2], v[3], a.lo);
+        o[q] = (int)pack_sat4(v[0], v[1], v[2], v[3], a.relu ? 0 : -128);
       }
       if (pix0 + j * 32 + col < npix) *reinterpret_cast<v4i *>(a.y + (int64_t)out[j] * a.y_cs + oc) = o;
     }
@@ -203,12 +211,12 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
   // where it does not apply: a table entry holds its tap as two 16-bit distances, a phase's table fits its share of LDS,
   // and every packed filter byte is addressed with 32 bits
   if (d.x_cs % 16 || ph * pw > 256 || (int64_t)d.kh * d.dh >= 30000 || (int64_t)d.kw * d.dw >= 30000 || d.ih >= 30000 ||
-      d.iw >= 30000 || (int64_t)d.kh * d.kw * n16 + 2 > kMaxEntries ||
+      d.iw >= 30000 || d.sh >= 256 || d.sw >= 256 || (int64_t)d.kh * d.kw * n16 + 2 > kMaxEntries ||
       (int64_t)blocks * ((int64_t)d.kh * d.kw * n16 + 2 * ph * pw) * 512 >= (1ll << 30))
     return TPUHIP_OK;
 
   std::vector<GatherPhase> phases;
-  std::vector<int2> tab;
+  std::vector<std::vector<int2>> tabs;
   std::vector<int8_t> w;
   int max_entries = 0, max_pixels = 0;
   struct Tap { int kh, kw, dy, dx; };
@@ -232,8 +240,8 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
         }
       const int entries = (int)taps.size() * n16;
       p.slices = (entries + 1) / 2;
-      p.tab = (int)tab.size();
       p.w = (uint32_t)w.size();
+      std::vector<int2> tab;
       for (int e = 0; e < 2 * p.slices; ++e) {
         const Tap t = e < entries ? taps[e / n16] : Tap{0, 0, 0, 0};
         int2 v;
@@ -241,6 +249,7 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
         v.y = (int)(((uint32_t)t.dy << 16) | ((uint32_t)t.dx & 0xffffu));
         tab.push_back(v);
       }
+      tabs.push_back(std::move(tab));
       w.resize(w.size() + (size_t)blocks * p.slices * 1024, 0);
       for (int blk = 0; blk < blocks; ++blk) {
         const int c_first = d.g == 1 ? 0 : (blk * 32 / ocg * icg) & ~15;
@@ -275,19 +284,21 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
   plan->tm = tm;
   w.resize(std::max<size_t>(w.size(), 16));
   plan->w_bytes = (uint32_t)w.size();
-  const size_t tab_at = w.size(), phase_at = tab_at + std::max<size_t>(tab.size(), 1) * sizeof(int2);
+  const size_t tab_bytes = (size_t)max_entries * sizeof(int2);
+  const size_t tab_at = w.size(), phase_at = tab_at + std::max<size_t>(tabs.size() * tab_bytes, 16);
   std::vector<int8_t> image(phase_at + phases.size() * sizeof(GatherPhase), 0);
   memcpy(image.data(), w.data(), w.size());
-  memcpy(image.data() + tab_at, tab.data(), tab.size() * sizeof(int2));
+  for (size_t i = 0; i < tabs.size(); ++i)
+    if (!tabs[i].empty()) memcpy(image.data() + tab_at + i * tab_bytes, tabs[i].data(), tabs[i].size() * sizeof(int2));
   memcpy(image.data() + phase_at, phases.data(), phases.size() * sizeof(GatherPhase));
+  plan->tab_at = (uint32_t)tab_at;
+  plan->phase_at = (uint32_t)phase_at;
   int rc = tpuhip_malloc(ctx, image.size(), (void **)&plan->w);
   if (!rc) rc = stage_upload(ctx, plan->w, image.data(), image.size());
   if (rc) {
     gather_destroy(ctx, plan);
     return rc;
   }
-  plan->tab = (const int2 *)(plan->w + tab_at);
-  plan->phases = (const GatherPhase *)(plan->w + phase_at);
   *out = plan;
   return TPUHIP_OK;
 }
@@ -298,27 +309,28 @@ void gather_destroy(tpuhip_ctx *ctx, GatherPlan *plan) {
   delete plan;
 }
 
-int gather_run(tpuhip_ctx *ctx, const GatherPlan *plan, const void *x, void *y, const int32_t *bias, const int32_t *mult,
-               const int32_t *shift, const int32_t *hpot, bool fast) {
+int gather_run(tpuhip_ctx *ctx, const GatherPlan *plan, const void *x, void *y, const int32_t *bias, const int32_t *planes,
+               int nparam, bool fast) {
   const tpuhip_conv_desc &d = plan->d;
   GatherArgs a{};
   a.x = (const int8_t *)x;
   a.y = (int8_t *)y;
   a.w = plan->w;
-  a.tab = plan->tab;
-  a.phases = plan->phases;
+  a.tab_at = plan->tab_at;
+  a.phase_at = plan->phase_at;
+  a.entries = (uint16_t)plan->max_entries;
   a.bias = bias;
-  a.mult = mult;
-  a.shift = shift;
-  a.hpot = hpot;
+  a.planes = planes;
+  a.nparam = nparam;
   a.x_bytes = (uint32_t)((int64_t)d.n * d.ih * d.iw * d.x_cs);
   a.w_bytes = plan->w_bytes;
   a.n = d.n; a.ih = d.ih; a.iw = d.iw; a.x_cs = d.x_cs;
   a.oh = d.oh; a.ow = d.ow; a.y_cs = d.y_cs; a.ocw = round_up(d.oc, 16);
-  a.ph = plan->ph; a.pw = plan->pw; a.step_h = plan->step_h; a.step_w = plan->step_w;
+  a.ph = (uint16_t)plan->ph; a.pw = (uint16_t)plan->pw;
+  a.step_h = (uint16_t)plan->step_h; a.step_w = (uint16_t)plan->step_w;
   a.ocg = d.oc / d.g;
   a.icg = d.g > 1 ? d.ic / d.g : 0;
-  a.lo = (d.do_relu && !d.relu_first) ? 0 : -128;
+  a.relu = d.do_relu && !d.relu_first;
   a.relu_first = (d.do_relu && d.relu_first) ? 1 : 0;
   // 64 pixels per wave where that still gives every SIMD two waves, else 32
   const int groups = plan->blocks / plan->tm;
@@ -326,7 +338,7 @@ int gather_run(tpuhip_ctx *ctx, const GatherPlan *plan, const void *x, void *y, 
   const bool wide = waves >= (int64_t)ctx->num_cu * 8;
   const int per_wg = wide ? 256 : 128;
   const dim3 grid((unsigned)((plan->max_pixels + per_wg - 1) / per_wg), (unsigned)groups, (unsigned)plan->n_phases), block(256);
-  const unsigned lds = (unsigned)std::max(plan->max_entries, 1) * sizeof(int2);
+  const unsigned lds = (unsigned)(3 * plan->tm * 32 * 4 + std::max(plan->max_entries, 1) * sizeof(int2));
   auto go = [&](auto kernel) {
     if (ctx->prof_start)
       hipExtLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);

@@ -12,9 +12,9 @@ struct GatherPlan;
 // *out stays NULL where it does not.  filter: OIHW int8 on the host (G x OC/G x IC/G x KH x KW).
 int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *filter, GatherPlan **out);
 void gather_destroy(tpuhip_ctx *ctx, GatherPlan *plan);
-// bias and the planes of multiplier, rshift and 2^(rshift-1), indexed by output channel and padded beyond a multiple of
-// 64 channels; fast: the layer's requantisation cannot overflow
-int gather_run(tpuhip_ctx *ctx, const GatherPlan *plan, const void *x, void *y, const int32_t *bias, const int32_t *mult,
-               const int32_t *shift, const int32_t *hpot, bool fast);
+// bias, and the planes of multiplier, rshift and 2^(rshift-1) of nparam entries each, indexed by output channel and padded
+// beyond a multiple of 64 channels; fast: the layer's requantisation cannot overflow
+int gather_run(tpuhip_ctx *ctx, const GatherPlan *plan, const void *x, void *y, const int32_t *bias, const int32_t *planes,
+               int nparam, bool fast);
 
 }  // namespace tpuhip
