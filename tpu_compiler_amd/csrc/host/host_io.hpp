@@ -16,8 +16,8 @@
 namespace tpuhip {
 
 // n floats (at any alignment) -> int8; the return value tells whether one of them is no integer in [-128, 127] (is_unsigned: [0, 255],
-// stored as the byte)
-bool floats_to_bytes(const void *src, int8_t *dst, size_t n, bool is_unsigned);
+// stored as the byte).  past_caches: with stores that leave the caches alone
+bool floats_to_bytes(const void *src, int8_t *dst, size_t n, bool is_unsigned, bool past_caches = false);
 // n int8 (is_unsigned: uint8) -> floats; past_caches: with stores that leave the caches alone
 void bytes_to_floats(const int8_t *src, float *dst, size_t n, bool is_unsigned, bool past_caches = false);
 
