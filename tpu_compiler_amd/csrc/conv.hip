@@ -3165,11 +3165,9 @@ conv_mfma_splitk_kernel(ConvArgs a) {
 // than input bytes run channel block by channel block, so that an XCD reads its own part of the filter only.
 // ---------------------------------------------------------------------------
 template <int W, int TN, bool FAST, bool UNI>
-__global__ __launch_bounds__(W * 64) void conv_mfma_ksplit_kernel(ConvArgs a) {
+__device__ __forceinline__ void ksplit_body(const ConvArgs &a) {
   extern __shared__ v4i kpart[];   // [wave][pixel block][quarter][lane], then the table's 256 bytes
   constexpr int D = 4;
-  gather_conv_args(a);
-  gather_conv_args_more(a);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wt = (int)(blockIdx.x & 7) * a.tiles_per_xcd + (int)(blockIdx.x >> 3);
@@ -3303,6 +3301,57 @@ __global__ __launch_bounds__(W * 64) void conv_mfma_ksplit_kernel(ConvArgs a) {
     const v4i z = fused_add_chunk(v4i{(int)o, 0, 0, 0}, v4i{(int)src, 0, 0, 0}, a.add_m_src, a.add_m_conv, a.add_rshift, a.add_relu, a.add_pk);
     *reinterpret_cast<uint32_t *>(a.add_dst + off) = (uint32_t)z[0];
   }
+}
+
+template <int W, int TN, bool FAST, bool UNI>
+__global__ __launch_bounds__(W * 64) void conv_mfma_ksplit_kernel(ConvArgs a) {
+  gather_conv_args(a);
+  gather_conv_args_more(a);
+  ksplit_body<W, TN, FAST, UNI>(a);
+}
+
+// The arguments of a conv with nothing fused behind it whose numbers fit these types: two cache lines instead of ten for the
+// kernel to wait for, and below the 112 bytes up to which a launch costs the host 0.5 us less.  64 -> 64 channels 3x3 on
+// 1 x 56 x 56, called from Python: 4.45 us, now 3.93.
+struct LeanArgs {
+  const int8_t *x, *w;
+  int8_t *y;
+  const int32_t *bias;
+  int nparam;                  // the planes of the requantisation lie behind nparam biases and records
+  uint32_t x_bytes;
+  int npix, n_tiles, tiles_per_xcd, pstep_n;
+  uint32_t magic_tile, magic_ow, magic_oh, magic_c16, magic_kw;
+  uint16_t ih, iw, oh, ow, x_cs, y_cs, oc, c16, k16, n_oc_tiles;
+  uint8_t kw, sh, sw, pt, pl, dh, dw;
+  uint8_t relu;                // 1: behind the requantisation, 2: in front of it
+};
+static_assert(sizeof(LeanArgs) <= 112, "see above");
+
+__device__ __forceinline__ void unpack_args(const LeanArgs &l, ConvArgs *a) {
+  a->x = l.x; a->w = l.w; a->y = l.y; a->bias = l.bias;
+  a->qmult = reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(l.bias) + (int64_t)l.nparam * (4 + sizeof(QParam)));
+  a->qshift = a->qmult + l.nparam;
+  a->qhpot = a->qshift + l.nparam;
+  a->x_bytes = l.x_bytes;
+  a->npix = l.npix; a->n_tiles = l.n_tiles; a->tiles_per_xcd = l.tiles_per_xcd; a->pstep_n = l.pstep_n;
+  a->magic_pw = a->magic_oc_tiles = l.magic_tile;
+  a->magic_ow = l.magic_ow; a->magic_oh = l.magic_oh; a->magic_c16 = l.magic_c16; a->magic_kw = l.magic_kw;
+  a->ih = l.ih; a->iw = l.iw; a->oh = l.oh; a->ow = l.ow; a->x_cs = l.x_cs; a->y_cs = l.y_cs;
+  a->oc = l.oc; a->ocw = (l.oc + 15) & ~15; a->c16 = l.c16; a->k16 = l.k16; a->n_oc_tiles = l.n_oc_tiles;
+  a->kp = (l.k16 + 3 & ~3) * 16;
+  a->w_bytes = (uint32_t)(l.n_oc_tiles * 32) * (uint32_t)a->kp;
+  a->kw = l.kw; a->sh = l.sh; a->sw = l.sw; a->pt = l.pt; a->pl = l.pl; a->dh = l.dh; a->dw = l.dw;
+  a->lo = l.relu == 1 ? 0 : -128;
+  a->relu_first = l.relu >> 1;
+  a->store_y = 1;
+  a->has_lut = 0; a->lut_dst = nullptr; a->add_src = nullptr; a->add_dst = nullptr; a->split_oc = 0; a->y2 = nullptr;
+}
+
+template <int W, int TN, bool FAST, bool UNI>
+__global__ __launch_bounds__(W * 64) void conv_mfma_ksplit_lean_kernel(LeanArgs l) {
+  ConvArgs a;
+  unpack_args(l, &a);
+  ksplit_body<W, TN, FAST, UNI>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -3801,13 +3850,44 @@ void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
   }
 }
 
+// the short form of a K-split launch's arguments; false: something is fused, or a number does not fit
+bool lean_args(const ConvArgs &a, LeanArgs *out) {
+  if (a.has_lut || a.add_dst || a.split_oc || !a.store_y || !a.y) return false;
+  auto u16 = [](int v) { return v >= 0 && v < 65536; };
+  auto u8 = [](int v) { return v >= 0 && v < 256; };
+  if (!u16(a.ih) || !u16(a.iw) || !u16(a.oh) || !u16(a.ow) || !u16(a.x_cs) || !u16(a.y_cs) || !u16(a.oc) || !u16(a.c16) ||
+      !u16(a.k16) || !u16(a.n_oc_tiles) || !u8(a.kw) || !u8(a.sh) || !u8(a.sw) || !u8(a.pt) || !u8(a.pl) || !u8(a.dh) || !u8(a.dw))
+    return false;
+  const int64_t nparam = a.qshift - a.qmult;
+  const int kp = (a.k16 + 3 & ~3) * 16;
+  if ((const char *)a.qmult - (const char *)a.bias != nparam * (int64_t)(4 + sizeof(QParam)) || a.qhpot - a.qshift != nparam ||
+      a.kp != kp || a.w_bytes != (uint32_t)(a.n_oc_tiles * 32) * (uint32_t)kp || a.ocw != (a.oc + 15 & ~15))
+    return false;
+  *out = LeanArgs{a.x, a.w, a.y, a.bias, (int)nparam, a.x_bytes, a.npix, a.n_tiles, a.tiles_per_xcd, a.pstep_n,
+                  a.pstep_n ? a.magic_pw : a.magic_oc_tiles, a.magic_ow, a.magic_oh, a.magic_c16, a.magic_kw,
+                  (uint16_t)a.ih, (uint16_t)a.iw, (uint16_t)a.oh, (uint16_t)a.ow, (uint16_t)a.x_cs, (uint16_t)a.y_cs, (uint16_t)a.oc,
+                  (uint16_t)a.c16, (uint16_t)a.k16, (uint16_t)a.n_oc_tiles, (uint8_t)a.kw, (uint8_t)a.sh, (uint8_t)a.sw,
+                  (uint8_t)a.pt, (uint8_t)a.pl, (uint8_t)a.dh, (uint8_t)a.dw, (uint8_t)(a.relu_first ? 2 : a.lo == 0 ? 1 : 0)};
+  return true;
+}
+
 template <bool FAST, bool UNI>
 void launch_ksplit(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
   switch (tile) {
 #define KS(i, name, W, TN)                                                                              \
   case i: {                                                                                             \
-    auto kernel = conv_mfma_ksplit_kernel<W, TN, FAST, UNI>;                                            \
     const unsigned lds = W * TN * 4096 + 256;                                                           \
+    LeanArgs l;                                                                                         \
+    if (lean_args(a, &l)) {                                                                             \
+      auto lean = conv_mfma_ksplit_lean_kernel<W, TN, FAST, UNI>;                                       \
+      if (!pw_prepare(lean, lds)) break;                                                                \
+      if (ctx->prof_start)                                                                              \
+        hipExtLaunchKernelGGL(lean, grid, dim3(W * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, l); \
+      else                                                                                              \
+        hipLaunchKernelGGL(lean, grid, dim3(W * 64), lds, ctx->stream, l);                              \
+      break;                                                                                            \
+    }                                                                                                   \
+    auto kernel = conv_mfma_ksplit_kernel<W, TN, FAST, UNI>;                                            \
     if (!pw_prepare(kernel, lds)) break;                                                                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(W * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
