@@ -1674,3 +1674,56 @@ def test_data_movement_group_edges(ctx, kind, shape, params, out_shape):
 ])
 def test_fully_connected_batched_tile_edges(ctx, bh, bl, m, k, n, lt, ot, relu):
     test_fully_connected_batched_and_transposed(ctx, bh, bl, m, k, n, lt, ot, relu)
+
+
+# the number of waves that share K changes at K = 512 and 1024; fewer K steps than waves; rows and channels around a block of 32
+@pytest.mark.parametrize("m,k,n,relu", [(1, 1, 1, False), (1, 16, 33, True), (31, 64, 32, False), (32, 65, 31, True), (33, 512, 64, False),
+                                        (2, 513, 10, True), (65, 1024, 33, False), (3, 1025, 1000, True)])
+def test_fully_connected_in_one_launch(ctx, m, k, n, relu):
+    test_fully_connected(ctx, m, k, n, relu)
+
+
+# n, ic, ih, iw, oc, kernel, stride, pads, dilation: a stride, a padding or a dilation that the short form of the arguments
+# holds (255) and one that it does not (256)
+@pytest.mark.parametrize("case", [(1, 32, 300, 2, 40, (2, 1), (255, 1), (0, 215, 0, 0), (1, 1)),
+                                  (1, 32, 300, 2, 40, (2, 1), (256, 1), (0, 215, 0, 0), (1, 1)),
+                                  (1, 48, 2, 300, 33, (1, 2), (1, 1), (0, 0, 0, 0), (1, 255)),
+                                  (1, 48, 2, 300, 33, (1, 2), (1, 1), (0, 0, 0, 0), (1, 256)),
+                                  (2, 16, 3, 4, 32, (1, 300), (1, 1), (0, 0, 255, 60), (1, 1)),
+                                  (2, 16, 3, 4, 32, (1, 200), (1, 1), (0, 0, 199, 60), (1, 1)),
+                                  (3, 80, 5, 7, 70, (3, 3), (2, 1), (1, 1, 0, 2), (1, 2))])
+@pytest.mark.parametrize("tile", KSPLIT_TILES)
+@pytest.mark.parametrize("relu", [False, True])
+def test_conv_ksplit_argument_ranges(ctx, case, tile, relu):
+    n, ic, ih, iw, oc, k, stride, pads, dil = case
+    rng = np.random.default_rng(ic + oc + ih)
+    x = rnd_i8(rng, (n, ic, ih, iw))
+    w = rnd_w(rng, (oc, ic) + k, sigma=14)
+    bias, rsh, mult = rnd_params(rng, oc, 5, 11)
+    want = oracle_conv(x, w, bias, rsh, mult, 1, stride, pads, dil, (0, 0), relu)
+    d = conv_desc(x.shape, w.shape, stride=stride, pads=pads, dil=dil, do_relu=relu, algo=16 + tile)
+    xt, yt = ctx.from_nchw(x), ctx.tensor(want.shape)
+    wh = ctx.conv_prepack(d, w, f2i32(bias), f2i32(mult), f2i32(rsh))
+    ctx._ck(ctx.lib.tpuhip_memset(ctx.h, yt.ptr, 0x55, yt.nbytes))
+    ctx.conv(wh, xt, yt)
+    assert np.array_equal(ctx.to_nchw(yt), want) and not ctx.raw(yt)[..., oc:].any()
+    ctx.conv_weights_destroy(wh)
+
+
+@pytest.mark.parametrize("shape,k,s,pads", [
+    ((1, 1, 1, 1), 2, (1, 1), (1, 1, 1, 1)), ((1, 16, 1, 1), 3, (1, 1), (2, 2, 2, 2)),     # every window mostly padding
+    ((2, 17, 5, 7), 2, (1, 2), (1, 0, 0, 1)), ((3, 40, 7, 5), 3, (2, 1), (2, 0, 1, 2)),
+    ((1, 33, 9, 9), 2, (3, 3), (0, 0, 0, 0)), ((2, 64, 6, 8), 3, (3, 2), (0, 2, 2, 0)),
+])
+def test_pool_square_windows(ctx, shape, k, s, pads):
+    rng = np.random.default_rng(sum(shape) + k)
+    x = rnd_i8(rng, shape)
+    x.reshape(-1)[:2] = (-128, 127)[:x.size]
+    od, d = O.make_pool_desc(shape, (k, k), s, pads), pool_desc(shape, (k, k), s, pads)
+    xt, yt = ctx.from_nchw(x), ctx.tensor((d.n, d.c, d.oh, d.ow))
+    for run, want in [(lambda: ctx.pool_max(d, xt, yt), O.pool_max_i8(x, od)),
+                      (lambda: ctx.pool_avg(d, xt, yt, 57, 8), O.pool_avg_i8(x, od, 8, 57))]:
+        ctx._ck(ctx.lib.tpuhip_memset(ctx.h, yt.ptr, 0x55, yt.nbytes))
+        run()
+        assert np.array_equal(ctx.to_nchw(yt), want)
+        assert not ctx.raw(yt)[..., shape[1]:].any()
