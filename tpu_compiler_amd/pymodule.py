@@ -9,8 +9,8 @@ reference's; `get_tensor_i8` is the cheaper int8 view of the same data.
 """
 import ctypes as C
 import os
-import sys
 import threading
+import weakref
 
 import numpy as np
 
@@ -53,12 +53,22 @@ _WEIGHT_OPERANDS = {
 }
 
 
+class _Lease:
+    """What every array over a piece of result memory rests on: numpy keeps it alive for an array and for all that is
+    made of that array without a copy (views, views of views, memoryviews), so it is gone when the last of them is."""
+    __slots__ = ("__array_interface__", "__weakref__")
+
+    def __init__(self, interface):
+        self.__array_interface__ = interface
+
+
 class _ResultMemory:
     """Memory of results.  A result of many pages in fresh memory costs more in page faults than in data (75 MB of
     floats: 6.3 ms against 2.6 in pages that are mapped), so an array handed out stays known here and its memory is
     handed out again once the caller has dropped it -- the array, its views, whatever holds one of them.  The first array
     of a shape is the caller's alone: what is read once leaves nothing behind.  At most LIMIT bytes are kept; they go with
-    the module or its next load()."""
+    the module or its next load(), those of arrays that are still held with the last of these.  Such arrays do not
+    own their memory (resize() in place wants a copy)."""
     SMALL = 64 << 10     # below this the allocator gives mapped memory anyway
     LIMIT = 256 << 20
 
@@ -69,6 +79,16 @@ class _ResultMemory:
     def clear(self):
         self._kept, self._bytes = {}, 0
 
+    class _Piece:
+        def __init__(self, owner):
+            self.interface = dict(owner.__array_interface__, owner=owner)      # what lends it keeps it
+            self.address, self.lease = owner.ctypes.data, None
+
+        def lend(self):
+            lease = _Lease(self.interface)
+            self.lease = weakref.ref(lease)
+            return np.asarray(lease), self.address
+
     def take(self, shape, dtype):
         """(array, its address)"""
         with self._lock:
@@ -77,16 +97,15 @@ class _ResultMemory:
                 self._kept[shape, dtype] = []
                 out = np.empty(shape, dtype)
                 return out, out.ctypes.data
-            for owner, address in kept:
-                if sys.getrefcount(owner) == 3:      # the list's tuple, this loop, the call: no array of a caller
-                    return owner.view(), address
+            for piece in kept:
+                if piece.lease() is None:
+                    return piece.lend()
             owner = np.empty(shape, dtype)
-            address = owner.ctypes.data
             if owner.nbytes < self.SMALL or self._bytes + owner.nbytes > self.LIMIT:
-                return owner, address
+                return owner, owner.ctypes.data
             self._bytes += owner.nbytes
-            kept.append((owner, address))
-            return owner.view(), address
+            kept.append(self._Piece(owner))
+            return kept[-1].lend()
 
 
 class module:
