@@ -745,7 +745,8 @@ private:
   void planAhead();
   void convertFilters(const ModuleDesc &module);
   void dropAhead();
-  bool capturing() const;
+  void noteCapture();
+  bool captured_ = false;   // an invoke of this module has been recorded into a graph
   struct Ahead {
     CPUOpKernel *behind;   // the kernel at whose position the tensor is complete
     TensorData *tensor;

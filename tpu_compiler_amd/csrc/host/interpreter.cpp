@@ -480,21 +480,23 @@ void ModuleInterpreter::updateKernelList(ModuleDesc &module, std::string &target
   }
 }
 
-// a graph that a caller records would announce the same serial at every replay
-bool ModuleInterpreter::capturing() const {
+// A graph that a caller records writes the results without this module's knowing, at every replay: from the first
+// recorded invoke on nothing is read ahead, of a plain invoke between replays neither.
+void ModuleInterpreter::noteCapture() {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(ctx_->stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx_->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) captured_ = true;
 }
 
 // MlirModuleInterpreter.cpp:371-381
 void ModuleInterpreter::invokeTo(std::string name, int32_t bidx) {
   FlagScope inside(ctx_->in_interpreter);
+  noteCapture();
   dropAhead();
   for (auto &kv : valueMapping) kv.second->set_batch_idx(bidx);
   for (auto &krnl : kernel_list_) {
     krnl->invoke();
     for (auto &a : ahead_)
-      if (a.wanted && a.behind == krnl.get() && !capturing()) a.tensor->read_ahead();
+      if (a.wanted && a.behind == krnl.get() && !captured_) a.tensor->read_ahead();
     if (!name.empty() && name == krnl->name) break;
   }
 }
@@ -502,6 +504,7 @@ void ModuleInterpreter::invokeTo(std::string name, int32_t bidx) {
 // MlirModuleInterpreter.cpp:383-405
 void ModuleInterpreter::fastInvokeAllBatch(std::string name, int32_t batch) {
   FlagScope inside(ctx_->in_interpreter);
+  noteCapture();
   dropAhead();
   bool last_batch = false;
   for (int i = 0; i < batch; i++) {
