@@ -53,15 +53,6 @@ _WEIGHT_OPERANDS = {
 }
 
 
-class _Lease:
-    """What every array over a piece of result memory rests on: numpy keeps it alive for an array and for all that is
-    made of that array without a copy (views, views of views, memoryviews), so it is gone when the last of them is."""
-    __slots__ = ("__array_interface__", "__weakref__")
-
-    def __init__(self, interface):
-        self.__array_interface__ = interface
-
-
 class _ResultMemory:
     """Memory of results.  A result of many pages in fresh memory costs more in page faults than in data (75 MB of
     floats: 6.3 ms against 2.6 in pages that are mapped), so an array handed out stays known here and its memory is
@@ -80,14 +71,18 @@ class _ResultMemory:
         self._kept, self._bytes = {}, 0
 
     class _Piece:
+        """Memory for arrays of one shape, one at a time.  It is no array itself: numpy lets a view rest on what its base
+        rests on only where that is an array, so views (and views of views, memoryviews) of an array lent here keep
+        that array alive, and it is gone when the last of them is."""
+
         def __init__(self, owner):
-            self.interface = dict(owner.__array_interface__, owner=owner)      # what lends it keeps it
-            self.address, self.lease = owner.ctypes.data, None
+            self.raw = (C.c_char * owner.nbytes).from_buffer(owner)
+            self.shape, self.dtype, self.address = owner.shape, owner.dtype, owner.ctypes.data
 
         def lend(self):
-            lease = _Lease(self.interface)
-            self.lease = weakref.ref(lease)
-            return np.asarray(lease), self.address
+            out = np.ndarray(self.shape, self.dtype, self.raw)
+            self.lent = weakref.ref(out)
+            return out, self.address
 
     def take(self, shape, dtype):
         """(array, its address)"""
@@ -98,7 +93,7 @@ class _ResultMemory:
                 out = np.empty(shape, dtype)
                 return out, out.ctypes.data
             for piece in kept:
-                if piece.lease() is None:
+                if piece.lent() is None:
                     return piece.lend()
             owner = np.empty(shape, dtype)
             if owner.nbytes < self.SMALL or self._bytes + owner.nbytes > self.LIMIT:
