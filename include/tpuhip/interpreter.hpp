@@ -129,7 +129,7 @@ public:
   // int8 NCHW host data -> slot bidx, for callers that hold bytes already: a quarter of the
   // float form's transfer and no host pass over the elements
   void assign_i8(const int8_t *first, size_t num, int32_t bidx);
-  // slot bidx as float-stored NCHW host data
+  // slot bidx as float-stored NCHW host data; this and every other read waits for all the context has issued
   std::shared_ptr<std::vector<float>> tensor(int32_t bidx) const;
   // the same into the caller's buffer
   void read(float *dst, size_t num, int32_t bidx) const;
@@ -142,7 +142,7 @@ public:
   // slot's bytes are taken as they are now.  Dropped when the tensor may be written again, never done for a tensor whose
   // address has been handed to others.
   void read_ahead();
-  void drop_ahead() const { ahead_slot_ = -1; }
+  void drop_ahead() const;
   bool exposed() const { return exposed_; }
   // whether the tensor was read since the last call of this
   bool take_was_read() const;

@@ -3,6 +3,7 @@ get_tensor in one piece, in several, and through more than the staging buffer ho
 import numpy as np
 import pytest
 
+from gpu_capture import Graph
 from tpu_compiler_amd import capi, graphs, module
 
 pytestmark = pytest.mark.gpu
@@ -148,4 +149,36 @@ def test_an_early_output_is_what_the_last_invoke_made_of_it(shape):
     m.invoke()                                      # two in a row, the first one's result is never read
     got = m.run(xs[2])
     assert np.array_equal(got["first"], np.maximum(xs[2], 0)) and np.array_equal(got["second"], xs[2].repeat(2, 2).repeat(2, 3))
+    m.close()
+
+
+@pytest.mark.parametrize("read", ["get_tensor", "get_tensor_i8", "get_tensors", "run"])
+def test_reading_an_early_output_waits_for_the_whole_invoke(read):
+    shape, big, behind = (1, 70, 50, 41), (1, 64, 1024, 1024), 40      # 40 passes over 2 x 67 MB: about a millisecond
+    g = graphs.Graph("early", 1)
+    g.add(graphs.Op("tpu.input", "x", [], shape))
+    g.add(graphs.Op("tpu.input", "z", [], big))
+    g.add(graphs.Op("tpu.relu", "first", ["x"], shape))
+    g.add(graphs.Op("tpu.relu", "other", ["x"], shape))
+    last = "z"
+    for i in range(behind):
+        g.add(graphs.Op("tpu.relu", "z%d" % i, [last], big))
+        last = "z%d" % i
+    g.outputs = ["first", "other"]
+    m = module()
+    m.load(g)
+    graph = Graph(m.context_handle())
+    rng = np.random.default_rng(29)
+    z = rng.integers(-128, 128, big).astype(np.int8)
+    m.set_tensor_i8("z", z)
+    for _ in range(3):
+        x = rng.integers(-128, 128, shape).astype(np.int8)
+        m.set_tensor_i8("x", x)
+        m.invoke()
+        got = m._get_tensors(["first"])["first"] if read == "get_tensors" else \
+            m._get_tensors(["first", "other"])["first"] if read == "run" else getattr(m, read)("first")
+        assert graph.idle()
+        assert np.array_equal(got, np.maximum(x, 0))
+        assert np.array_equal(m.get_tensor_i8("other"), np.maximum(x, 0)) and graph.idle()
+    assert np.array_equal(m.get_tensor_i8(last), np.maximum(z, 0))
     m.close()

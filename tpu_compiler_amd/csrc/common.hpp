@@ -24,6 +24,7 @@ struct FilterPack {
   int smallc;
   int64_t total;   // 16-byte groups
 };
+struct AheadRead;   // host/host_io.hpp
 // one piece of the pinned buffer on its way to the device, in dwords
 struct StagedCopy {
   const uint32_t *src;
@@ -67,6 +68,7 @@ struct tpuhip_ctx {
   std::vector<tpuhip::FilterPack> packs;
   bool in_interpreter = false;   // a module loads or invokes its kernels: device addresses asked for now go to those
   hipStream_t copy_stream = nullptr;   // results laid out early leave on it while `stream` works on; made on first use
+  std::vector<tpuhip::AheadRead *> ahead;   // those that may still be asked for
   bool single_pass = false;   // what is issued now runs once: no layer's tile variants are timed for it
 };
 

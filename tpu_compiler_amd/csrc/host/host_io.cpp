@@ -593,6 +593,7 @@ __global__ void arrived_kernel(uint32_t *flag, uint32_t value) {
 int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src) {
   const size_t bytes = ((size_t)t.n * t.c * t.h * t.w + 63) / 64 * 64;
   if (!ctx->copy_stream) TPUHIP_CHECK_HIP(hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking));
+  drop_ahead(ctx, a);
   if (!a.pinned) {
     TPUHIP_CHECK_HIP(hipMalloc(&a.dense, bytes + 256));
     TPUHIP_CHECK_HIP(hipHostMalloc(&a.pinned, bytes + 64, hipHostMallocDefault));
@@ -602,13 +603,21 @@ int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *s
   if (int rc = tpuhip_nhwc_to_nchw_i8(ctx, src, a.dense, t.n, t.c, t.h, t.w, t.cs)) return rc;
   launch(ctx, arrived_kernel, dim3(1), dim3(1), a.flag, ++a.serial);
   TPUHIP_CHECK_HIP(hipGetLastError());
+  a.bytes = (size_t)t.n * t.c * t.h * t.w;
+  a.fetched = false;
+  ctx->ahead.push_back(&a);
   return TPUHIP_OK;
+}
+
+void drop_ahead(tpuhip_ctx *ctx, AheadRead &a) {
+  ctx->ahead.erase(std::remove(ctx->ahead.begin(), ctx->ahead.end(), &a), ctx->ahead.end());
 }
 
 // The host sees from the flag that the dense form is there and starts a copy engine on it: that needs no wait of one
 // stream for another (which costs the host 12 us a piece, 60 in front of a copy), and unlike a kernel the engine takes no
 // compute unit from the launches that are still running.
-int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r) {
+static int fetch_ahead(tpuhip_ctx *ctx, AheadRead &a) {
+  if (a.fetched) return TPUHIP_OK;
   for (int spin = 0; __atomic_load_n(a.flag, __ATOMIC_ACQUIRE) != a.serial; ++spin) {
     if (spin % 256 == 255) {   // a stream that is done, or has failed, without the flag: nothing more will come
       const hipError_t e = hipStreamQuery(ctx->stream);
@@ -619,13 +628,27 @@ int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r) {
     }
     std::this_thread::yield();
   }
-  const size_t count = elements(r), grain = kPiece / host_size(r.kind);
   TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
-  TPUHIP_CHECK_HIP(hipMemcpyAsync(a.pinned, a.dense, count, hipMemcpyDeviceToHost, ctx->copy_stream));
+  TPUHIP_CHECK_HIP(hipMemcpyAsync(a.pinned, a.dense, a.bytes, hipMemcpyDeviceToHost, ctx->copy_stream));
+  a.fetched = true;
+  return TPUHIP_OK;
+}
+
+int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r) {
+  if (int rc = fetch_ahead(ctx, a)) return rc;
   TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->copy_stream));
+  const size_t count = elements(r), grain = kPiece / host_size(r.kind);
   parallel_pieces((count + grain - 1) / grain, [&](size_t i) {
     pass_part(Part{&r, i * grain, std::min(grain, count - i * grain), i * grain, 0}, (const int8_t *)a.pinned, false);
   });
+  return TPUHIP_OK;
+}
+
+int settle_ahead(tpuhip_ctx *ctx) {
+  for (AheadRead *a : ctx->ahead)
+    if (int rc = fetch_ahead(ctx, *a)) return rc;
+  TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  if (ctx->copy_stream) TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->copy_stream));
   return TPUHIP_OK;
 }
 

@@ -45,14 +45,20 @@ struct HostRead {
 int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n);
 
 // A result that is complete while its stream still has work in front of it: read_ahead() lays it out for the host there
-// and then, finish_ahead() fetches it beside the rest of that work.
+// and then, finish_ahead() fetches it beside the rest of that work, settle_ahead() waits for that rest.
 struct AheadRead {
   void *dense = nullptr, *pinned = nullptr;
   uint32_t *flag = nullptr, serial = 0;   // the flag, in pinned memory, shows the serial of what lies in `dense`
+  size_t bytes = 0;
+  bool fetched = false;                   // `pinned` holds it, or a copy to there is in flight (not beyond settle_ahead())
   ~AheadRead();
 };
 int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src);
 // the host pass from a's bytes instead of r.src
 int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r);
+// waits for everything the context has issued; what else has been laid out early is fetched meanwhile
+int settle_ahead(tpuhip_ctx *ctx);
+// nobody will ask for it any more
+void drop_ahead(tpuhip_ctx *ctx, AheadRead &a);
 
 }  // namespace tpuhip

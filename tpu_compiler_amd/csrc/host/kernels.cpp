@@ -122,6 +122,12 @@ void *TensorData::data() const {
   return ptr_;
 }
 
+void TensorData::drop_ahead() const {
+  if (ahead_slot_ < 0) return;
+  ahead_slot_ = -1;
+  tpuhip::drop_ahead(ctx_, *ahead_);
+}
+
 bool TensorData::take_was_read() const {
   const bool was = was_read_;
   was_read_ = false;
@@ -143,6 +149,7 @@ bool TensorData::finish_ahead(const HostRead &r, int32_t bidx) const {
 }
 
 TensorData::~TensorData() {
+  drop_ahead();
   if (base_) tpuhip_free(ctx_, base_);
 }
 
@@ -205,8 +212,7 @@ HostRead TensorData::host_read(void *dst, size_t num, int32_t bidx, bool bytes) 
 
 void TensorData::read(float *dst, size_t num, int32_t bidx) const {
   const HostRead r = host_read(dst, num, bidx, false);
-  if (finish_ahead(r, bidx)) return;
-  ck(device_to_host(ctx_, &r, 1), "TensorData::tensor");
+  ck(finish_ahead(r, bidx) ? settle_ahead(ctx_) : device_to_host(ctx_, &r, 1), "TensorData::tensor");
 }
 
 void TensorData::read_all(const std::vector<const TensorData *> &tensors, const std::vector<float *> &dsts,
@@ -219,7 +225,9 @@ void TensorData::read_all(const std::vector<const TensorData *> &tensors, const 
       reads.erase(reads.begin() + (ptrdiff_t)k);
     else
       ++k;
-  if (!reads.empty()) ck(device_to_host(tensors[0]->ctx_, reads.data(), reads.size()), "TensorData::tensor");
+  if (tensors.empty()) return;
+  tpuhip_ctx *ctx = tensors[0]->ctx_;
+  ck(reads.empty() ? settle_ahead(ctx) : device_to_host(ctx, reads.data(), reads.size()), "TensorData::tensor");
 }
 
 std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
@@ -230,8 +238,7 @@ std::shared_ptr<std::vector<float>> TensorData::tensor(int32_t bidx) const {
 
 void TensorData::read_i8(int8_t *dst, size_t num, int32_t bidx) const {
   const HostRead r = host_read(dst, num, bidx, true);
-  if (finish_ahead(r, bidx)) return;
-  ck(device_to_host(ctx_, &r, 1), "TensorData::read_i8");
+  ck(finish_ahead(r, bidx) ? settle_ahead(ctx_) : device_to_host(ctx_, &r, 1), "TensorData::read_i8");
 }
 
 // ---------------------------------------------------------------------------
