@@ -52,9 +52,10 @@ void *tpuhip_ctx_stream(tpuhip_ctx *ctx);
 /* When enabled (the default; TPUHIP_AUTOTUNE=0 in the environment disables it) a
  * dense conv times its tile variants on first use and keeps the fastest, unless a layer of
  * the same shape has been timed before in this process, whose choice it takes.  Every
- * variant produces the same bytes.  Inside a HIP graph capture nothing is timed: capture
- * after the first use of a layer (tpuhip_module_interpret_files, which runs a model once,
- * times nothing either). */
+ * variant produces the same bytes.  Nothing is timed inside a HIP graph capture: a layer
+ * whose first use that would be is refused there with TPUHIP_ERR_INVALID.
+ * tpuhip_module_interpret_files, which runs a model once, times nothing either: a layer that
+ * ran so is timed at its next use, or keeps the tile it ran with if that use is captured. */
 int tpuhip_ctx_set_autotune(tpuhip_ctx *ctx, int enable);
 const char *tpuhip_last_error(void);
 const char *tpuhip_version(void);

@@ -3,8 +3,9 @@ between, and what cannot be recorded is refused."""
 import numpy as np
 import pytest
 
+import oracle_graph
 from gpu_capture import Graph
-from tpu_compiler_amd import capi, graphs, module
+from tpu_compiler_amd import capi, graphs, mlir_text, module
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +53,61 @@ def test_results_of_replays_are_read_not_those_of_earlier_invokes(all_batch):
         check(x)
     graph.close()
     m.close()
+
+
+def _run_files(m, g, folder):
+    path = folder / "model.mlir"
+    mlir_text.write_mlir(g, path)
+    np.savez(folder / "in.npz", **{g.input_op().name: g.input_op().data.astype(np.float32)})
+    m.interpret_files(path, folder / "in.npz", folder / "out.npz")
+
+
+def _check_replays(m, g, graph, plain):
+    rng = np.random.default_rng(3)
+    name, shape = g.input_op().name, g.input_op().shape
+    for k in range(4):
+        x = rng.integers(-128, 128, shape).astype(np.int8)
+        want = oracle_graph.run(g, input_data=x)
+        m.set_tensor_i8(name, x)
+        if k % 2:
+            plain()
+        else:
+            graph.replay()
+        for op in g.ops:
+            assert np.array_equal(m.get_tensor_i8(op.name), want[op.name].reshape(op.shape)), (k, op.name)
+
+
+# sides that nothing else here uses: no layer finds its tile remembered
+@pytest.mark.parametrize("make", [lambda: graphs.cfg3_resnet50(batch=1, hw=72), lambda: graphs.cfg4_mobilenet_v2(batch=1, hw=72),
+                                  lambda: graphs.cfg5_yolo_v3(batch=1, hw=96)])
+def test_a_network_that_ran_once_from_files_can_be_recorded(make, tmp_path):
+    g, m = make(), module()
+    _run_files(m, g, tmp_path)
+    graph = Graph(m.context_handle())
+    with graph.recording():
+        m.invoke()
+    tiles = m.kernels()
+    _check_replays(m, g, graph, m.invoke)
+    assert m.kernels() == tiles          # the graph reads the filters as they were packed then
+    graph.close()
+    m.close()
+
+
+def test_a_layer_whose_first_use_is_recorded_is_refused():
+    g = graphs.cfg3_resnet50(batch=1, hw=88)
+    for remembered in (False, True):     # the second module's shapes have been timed by the first
+        m = module()
+        m.load(g)
+        graph = Graph(m.context_handle())
+        with graph.recording():
+            with pytest.raises(capi.TpuHipError, match="captured"):
+                m.invoke()
+        graph.close()
+        m.set_tensor_i8(g.input_op().name, g.input_op().data.astype(np.int8))
+        m.invoke()
+        m.sync()
+        with graph.recording():
+            m.invoke()
+        _check_replays(m, g, graph, m.invoke)
+        graph.close()
+        m.close()

@@ -48,6 +48,7 @@ struct tpuhip_conv_weights {
   int fast = 0;          // the overflow-free requant form is provably exact for this layer
   bool smallc = false;   // ic <= 4: K packs 4 taps x 4 channels per 16-byte group (LDS kernels only)
   bool tuned = true;     // false: the tile is chosen by timing the candidates on first use
+  bool ran_untimed = false;   // it has run with the tile it was packed for, in a pass that no timing was worth
   // a pair of convs over one input packed as one: first channel, channel stride and ReLU of
   // the second result (split_oc == 0: an ordinary conv)
   int split_oc = 0, y2_cs = 0, relu2 = 0;
@@ -4499,9 +4500,18 @@ int autotune_mfma(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *
 }
 
 // The tile of a layer that may still choose: one that timing has found before for the same shape, else the fastest, by
-// timing.  The rule's tile stays, for this use, inside a capture, which cannot wait, and where the context says that the
-// model runs once: timing 35 layers takes 100 ms, and a single pass of them is 0.3 ms on either choice.
+// timing.  The rule's tile stays, for this use, where the context says that the model runs once: timing 35 layers takes
+// 100 ms, and a single pass of them is 0.3 ms on either choice.  A graph that is being recorded will read the filter as it
+// lies now at every replay: a layer that has run so keeps its tile for good, one that never ran is refused.
 int choose_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *y, const PostOps &post) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
+  if (capturing != hipStreamCaptureStatusNone) {
+    TPUHIP_REQUIRE(w->ran_untimed, "conv: a layer's tile cannot be chosen while its stream is captured: run it once before (or "
+                                   "switch autotune off)");
+    w->tuned = true;   // the unpacked filter goes with the layer: freeing it would wait for the stream
+    return TPUHIP_OK;
+  }
   const TileKey key = tile_key(ctx, w, y, post);
   int known = -1;
   {
@@ -4509,16 +4519,16 @@ int choose_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *y,
     auto it = g_tiles.find(key);
     if (it != g_tiles.end()) known = it->second;
   }
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  (void)hipStreamIsCapturing(ctx->stream, &capturing);
-  if (capturing != hipStreamCaptureStatusNone) return TPUHIP_OK;
   if (known >= 0) {
     if (known != w->tile)
       if (int rc = pack_mfma_weights(ctx, w, known)) return rc;
     settle_tile(ctx, w);
     return TPUHIP_OK;
   }
-  if (ctx->single_pass) return TPUHIP_OK;
+  if (ctx->single_pass) {
+    w->ran_untimed = true;
+    return TPUHIP_OK;
+  }
   // the fused work is timed with it unless the sum would overwrite its own operand
   PostOps tp = post;
   if (tp.has_add() && tp.add_out == tp.add_src) tp.f = nullptr;
