@@ -5,6 +5,7 @@ import pytest
 
 import oracle_graph
 from gpu_capture import Graph
+from gpu_helpers import conv_desc, run_conv
 from tpu_compiler_amd import capi, graphs, mlir_text, module
 
 pytestmark = pytest.mark.gpu
@@ -111,3 +112,56 @@ def test_a_layer_whose_first_use_is_recorded_is_refused():
         _check_replays(m, g, graph, m.invoke)
         graph.close()
         m.close()
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 20, 31), (4, 70, 61, 67)])     # one piece of the staging buffer, several
+def test_host_tensors_are_refused_while_the_stream_is_captured(shape):
+    m = _two_outputs(shape)
+    rng = np.random.default_rng(11)
+    xs = [rng.integers(-128, 128, shape).astype(np.int8) for _ in range(4)]
+    for x in xs[:2]:
+        m.set_tensor_i8("x", x)
+        m.invoke()
+        assert np.array_equal(m.get_tensor_i8("first"), np.maximum(x, 0))
+    m.invoke()                           # "first" of xs[1], laid out early where it is large enough
+    graph = Graph(m.context_handle())
+    with graph.recording():
+        for call in (lambda: m.get_tensor_i8("first"), lambda: m.get_tensor("second"), lambda: m._get_tensors(["first", "second"]),
+                     lambda: m.set_tensor_i8("x", xs[3]), lambda: m.set_tensor("x", xs[3])):
+            with pytest.raises(capi.TpuHipError, match="being captured"):
+                call()
+        m.invoke()
+    assert graph.nodes() == 2            # the two kernels of the invoke: nothing of the refused calls
+    for x in xs[1:3] * 2:
+        m.set_tensor_i8("x", x)
+        graph.replay()
+        assert np.array_equal(m.get_tensor_i8("first"), np.maximum(x, 0))
+        assert np.array_equal(m.get_tensor("second"), x.repeat(2, 2).repeat(2, 3))
+    graph.close()
+    m.close()
+
+
+# dense, stem, depthwise, grouped, transposed
+@pytest.mark.parametrize("ic,oc,k,kw", [(32, 32, 1, {}), (3, 16, 3, {}), (32, 32, 3, dict(g=32)), (32, 32, 3, dict(g=4)),
+                                        (16, 16, 3, dict(ins=(1, 1)))])
+def test_packing_weights_is_refused_while_the_stream_is_captured(ic, oc, k, kw):
+    ctx = capi.Context(0)
+    rng = np.random.default_rng(31)
+    x = rng.integers(-128, 128, (1, ic, 12, 12)).astype(np.int8)
+    w = rng.integers(-64, 65, (oc, ic // kw.get("g", 1), k, k)).astype(np.int8)
+    bias, rshift, mult = rng.integers(-500, 500, oc).astype(np.float32), np.full(oc, 9, np.float32), np.full(oc, 1 << 30, np.float32)
+    want, _ = run_conv(ctx, x, w, bias, rshift, mult, **kw)
+    a, y = ctx.from_nchw(x), ctx.tensor(want.shape)
+    graph = Graph(ctx.h)
+    with graph.recording():
+        with pytest.raises(capi.TpuHipError, match="being captured"):
+            ctx.conv_prepack(conv_desc(x.shape, w.shape, **kw), w, bias.astype(np.int32), mult.astype(np.int32), rshift.astype(np.int32))
+        ctx._ck(ctx.lib.tpuhip_memset(ctx.h, y.ptr, 3, y.nbytes))
+    assert graph.nodes() == 1
+    graph.replay()
+    again, _ = run_conv(ctx, x, w, bias, rshift, mult, **kw)
+    assert np.array_equal(again, want) and (ctx.raw(y) == 3).all()
+    graph.close()
+    a.free()
+    y.free()
+    ctx.close()

@@ -91,6 +91,8 @@ struct FlagScope {
 
 // host/host_io.cpp: frees a context's staging buffers
 void host_io_release(tpuhip_ctx *ctx);
+// host/host_io.cpp: refuses what moves host memory while the context's stream is being captured
+int not_captured(tpuhip_ctx *ctx, const char *what);
 // host/host_io.cpp: tpuhip_upload without the wait -- src may be reused on return, the bytes are there for what is issued to
 // the context's stream afterwards
 int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes);

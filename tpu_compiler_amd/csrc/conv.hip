@@ -4565,6 +4565,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
                  "tpuhip_conv2d_prepack: NULL argument");
   const tpuhip_conv_desc &d = *desc;
   if (int rc = check_desc(d)) return rc;
+  if (int rc = not_captured(ctx, "conv: packing weights")) return rc;
   for (int i = 0; i < d.oc; ++i)
     TPUHIP_REQUIRE(rshift[i] >= 0 && rshift[i] <= 31, "conv: rshift[%d] = %d outside [0,31]", i,
                    rshift[i]);

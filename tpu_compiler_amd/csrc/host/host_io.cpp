@@ -345,6 +345,14 @@ size_t stage_size(HostKind k) { return k == HostKind::kFloats ? sizeof(float) : 
 
 }  // namespace
 
+// A recorded copy would take, at every replay, whatever lies in the pinned buffer then, and a wait cannot be recorded.
+int not_captured(tpuhip_ctx *ctx, const char *what) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
+  TPUHIP_REQUIRE(capturing == hipStreamCaptureStatusNone, "%s: the context's stream is being captured", what);
+  return TPUHIP_OK;
+}
+
 void parallel_pieces(size_t n, const std::function<void(size_t)> &piece) {
   if (n < 2) {
     if (n) piece(0);
@@ -360,6 +368,7 @@ void parallel_pieces(size_t n, const std::function<void(size_t)> &piece) {
 
 int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const void *src, void *dst, bool *bad) {
   *bad = false;
+  if (int rc = not_captured(ctx, "a tensor from the host")) return rc;
   const size_t count = (size_t)t.n * t.c * t.h * t.w;
   const size_t per = stage_size(kind), total = count * per;
   if (int rc = stage_ready(ctx, total)) return rc;
@@ -461,6 +470,7 @@ size_t elements(const HostRead &r) { return (size_t)r.t.n * r.t.c * r.t.h * r.t.
 // the host pass of a span runs on several threads while the next ones are laid out and on the bus, and for small tensors
 // while the launches of those behind them are still being issued.
 int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
+  if (int rc = not_captured(ctx, "a tensor to the host")) return rc;
   size_t total = 0, host_total = 0, largest = 0;
   for (size_t i = 0; i < n; ++i) {
     const size_t count = elements(reads[i]), bytes = count * stage_size(reads[i].kind);
@@ -635,6 +645,7 @@ static int fetch_ahead(tpuhip_ctx *ctx, AheadRead &a) {
 }
 
 int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r) {
+  if (int rc = not_captured(ctx, "a tensor to the host")) return rc;
   if (int rc = fetch_ahead(ctx, a)) return rc;
   TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->copy_stream));
   const size_t count = elements(r), grain = kPiece / host_size(r.kind);
@@ -662,6 +673,7 @@ __global__ __launch_bounds__(256) void staged_copies_kernel(const StagedCopy *li
 // A network of 52 convs took three launches for each, 440 us of a 5 ms tool run; all of them together take two.
 int flush_uploads(tpuhip_ctx *ctx) {
   if (ctx->staged.empty() && ctx->packs.empty()) return TPUHIP_OK;
+  if (int rc = not_captured(ctx, "packed weights")) return rc;
   auto place = [&](const void *list, size_t bytes) -> void * {   // stage_upload() leaves the room for it
     void *at = (int8_t *)ctx->stage + ctx->stage_used;
     memcpy(at, list, bytes);
