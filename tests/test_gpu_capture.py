@@ -4,8 +4,9 @@ import numpy as np
 import pytest
 
 import oracle_graph
+import oracle_lib as O
 from gpu_capture import Graph
-from gpu_helpers import conv_desc, run_conv
+from gpu_helpers import conv_desc, pool_desc, run_conv
 from tpu_compiler_amd import capi, graphs, mlir_text, module
 
 pytestmark = pytest.mark.gpu
@@ -164,4 +165,47 @@ def test_packing_weights_is_refused_while_the_stream_is_captured(ic, oc, k, kw):
     graph.close()
     a.free()
     y.free()
+    ctx.close()
+
+
+@pytest.mark.parametrize("shape", [(1, 120, 40, 40), (2, 17, 75, 75), (1, 16, 33, 47)])
+def test_a_recorded_average_over_a_large_window_needs_no_memory_of_its_context(shape):
+    other = (2 * shape[0], 2 * shape[1], 100, 90)      # a plain pool that takes a larger workspace
+    ctx = capi.Context(0)
+    rng = np.random.default_rng(sum(shape))
+
+    def pool(s):
+        d = pool_desc(s, s[2:], (1, 1), (0, 0, 0, 0), (1, 1))
+        x, y = ctx.tensor(s), ctx.tensor(s[:2] + (1, 1))
+        mult = min(255, int(4428 / (s[2] * s[3]) ** 0.5))
+        return d, x, y, lambda: ctx.pool_avg(d, x, y, mult, 13)
+
+    def check(s, x, y, call):
+        data = rng.integers(-128, 128, s).astype(np.int8)
+        filled = ctx.from_nchw(data, x.cs)
+        ctx._ck(ctx.lib.tpuhip_memset(ctx.h, y.ptr, 0x55, y.nbytes))
+        ctx._ck(ctx.lib.tpuhip_download(ctx.h, host.ctypes.data, filled.ptr, filled.nbytes))
+        ctx._ck(ctx.lib.tpuhip_upload(ctx.h, x.ptr, host.ctypes.data, filled.nbytes))
+        filled.free()
+        call()
+        want = O.pool_avg_i8(data, O.make_pool_desc(s, s[2:], (1, 1), (0, 0, 0, 0)), 13,
+                             min(255, int(4428 / (s[2] * s[3]) ** 0.5)))
+        assert np.array_equal(ctx.to_nchw(y), want)
+        assert not ctx.raw(y)[..., s[1]:].any()
+
+    _, x, y, plain = pool(shape)
+    _, x2, y2, larger = pool(other)
+    host = np.empty(max(x.nbytes, x2.nbytes), np.int8)
+    check(shape, x, y, plain)              # the workspace is there
+    graph = Graph(ctx.h)
+    with graph.recording():
+        plain()
+    assert graph.nodes() == 1              # no second launch that adds up partial sums in the workspace
+    for k in range(3):
+        check(shape, x, y, graph.replay)
+        check(other, x2, y2, larger)       # outgrows it
+        check(shape, x, y, plain)
+    graph.close()
+    for t in (x, y, x2, y2):
+        t.free()
     ctx.close()

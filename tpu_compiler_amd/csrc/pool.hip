@@ -283,18 +283,15 @@ int run_window(tpuhip_ctx *ctx, const PoolArgs &a) {
   const int G = c16 >= 16 ? 16 : c16 > 4 ? 8 : c16 > 2 ? 4 : c16;
   const int gblocks = (c16 + G - 1) / G, taps = a.kh * a.kw;
   const int64_t pixels = a.total / c16, blocks = pixels * gblocks;
-  // two workgroups per CU, while every lane keeps four positions; no slices where the grid of the second launch or the
-  // workspace (which is not grown while the stream is being captured) does not reach
+  // two workgroups per CU, while every lane keeps four positions; no slices where the grid of the second launch does not
+  // reach, nor in a recorded launch: a graph may outlive this context's workspace, or replay beside another one
   int64_t slices = std::min<int64_t>(std::min<int64_t>(2 * ctx->num_cu / blocks, taps / (4 * 256 / G)), 32);
   if (slices < 2 || pixels > 65535) slices = 1;
   if (slices > 1) {
-    const size_t bytes = (size_t)(pixels * slices * c16 * 16) * sizeof(int32_t);
-    if (ctx->workspace_bytes < bytes) {
-      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-      TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-      if (capture != hipStreamCaptureStatusNone) slices = 1;
-      else if (int rc = grow_workspace(ctx, bytes)) return rc;
-    }
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
+    if (capture != hipStreamCaptureStatusNone) slices = 1;
+    else if (int rc = grow_workspace(ctx, (size_t)(pixels * slices * c16 * 16) * sizeof(int32_t))) return rc;
   }
   int32_t *parts = slices > 1 ? (int32_t *)ctx->workspace : nullptr;
   const int per_slice = (int)((taps + slices - 1) / slices);
