@@ -1,5 +1,7 @@
 """Tensors between host memory and the device: the layout kernels at the edges of their tiles, and set_tensor /
 get_tensor in one piece, in several, and through more than the staging buffer holds."""
+import time
+
 import numpy as np
 import pytest
 
@@ -181,4 +183,30 @@ def test_reading_an_early_output_waits_for_the_whole_invoke(read):
         assert np.array_equal(got, np.maximum(x, 0))
         assert np.array_equal(m.get_tensor_i8("other"), np.maximum(x, 0)) and graph.idle()
     assert np.array_equal(m.get_tensor_i8(last), np.maximum(z, 0))
+    m.close()
+
+
+def test_a_read_behind_long_work_keeps_one_thread_waiting():
+    shape, behind, invokes = (1, 64, 1024, 1024), 40, 30      # 1200 passes over 2 x 67 MB: some 30 ms
+    g = graphs.Graph("long", 1)
+    g.add(graphs.Op("tpu.input", "y0", [], shape))
+    for i in range(behind):
+        g.add(graphs.Op("tpu.relu", "y%d" % (i + 1), ["y%d" % i], shape))
+    g.outputs = ["y%d" % behind]
+    m = module()
+    m.load(g)
+    x = np.random.default_rng(41).integers(-128, 128, shape).astype(np.int8)
+    m.set_tensor_i8("y0", x)
+    for _ in range(3):                  # nothing is in the staging buffer any more, the result's memory is there
+        m.invoke()
+        got = m.get_tensor_i8(g.outputs[0])
+    for _ in range(invokes):
+        m.invoke()
+    wall, cpu = time.perf_counter(), time.process_time()
+    got = m.get_tensor_i8(g.outputs[0])
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert np.array_equal(got, np.maximum(x, 0))
+    print("read: %.1f ms, CPU time %.1f ms" % (wall * 1e3, cpu * 1e3))
+    # eight threads for the pieces of the result, a few milliseconds, one for the rest: eight for all of it would be 8
+    assert cpu < 3 * wall
     m.close()

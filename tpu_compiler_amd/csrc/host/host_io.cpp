@@ -1,10 +1,12 @@
 #include "host_io.hpp"
 
-#include <sched.h>
+#include "host_cpus.hpp"
+
 #include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <condition_variable>
 #include <cstring>
@@ -236,11 +238,8 @@ class HostWorkers {
 
   void start() {
     pid_ = getpid();
-    cpu_set_t set;
-    int cpus = 1;
-    if (sched_getaffinity(0, sizeof(set), &set) == 0) cpus = CPU_COUNT(&set);
     // seven beside the caller reach the memory bandwidth of a socket's share; never more than the CPUs there are
-    const int count = std::max(0, std::min(7, cpus - 1));
+    const int count = std::max(0, std::min(7, usable_cpus() - 1));
     for (int i = 0; i < count; ++i) threads_.emplace_back([this] { work(); });
   }
 
@@ -468,7 +467,9 @@ size_t elements(const HostRead &r) { return (size_t)r.t.n * r.t.c * r.t.h * r.t.
 // Tensors of up to two pieces are laid out straight into the staging buffer; the dense form of larger ones is made on the
 // device and comes over in spans.  An event stands behind each span, and behind small tensors that make one up together;
 // the host pass of a span runs on several threads while the next ones are laid out and on the bus, and for small tensors
-// while the launches of those behind them are still being issued.
+// while the launches of those behind them are still being issued.  Those threads wait for spans by looking again and again:
+// they are called once the work in front of the first one has ended, which this thread waits for alone (a read 25 ms behind
+// its launch kept all eight busy for as long, 200 ms of CPU time).
 int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
   if (int rc = not_captured(ctx, "a tensor to the host")) return rc;
   size_t total = 0, host_total = 0, largest = 0;
@@ -536,7 +537,7 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
       fetches.back().closes = true;
       ++spans;
     }
-    while (ctx->stage_events.size() < spans) {
+    while (ctx->stage_events.size() < spans + 1) {   // the last one stands behind the work in front
       hipEvent_t e;
       TPUHIP_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       ctx->stage_events.push_back(e);
@@ -554,14 +555,22 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
       pass_part(p, stage, past_caches);
     };
     HostWorkers &workers = HostWorkers::get();
-    const bool shared = parts.size() > 1 && workers.enter(job);
+    bool called = false, shared = false;
+    auto call_workers = [&] {
+      called = true;
+      shared = parts.size() > 1 && workers.enter(job);
+    };
     int rc = TPUHIP_OK;
     size_t recorded = 0, there = 0;
-    ctx->stage_busy = true;
     auto hip = [&](hipError_t e, const char *what) {
       if (!rc && e != hipSuccess) rc = set_error(TPUHIP_ERR_HIP, "%s failed: %s", what, hipGetErrorString(e));
     };
+    const hipEvent_t front = ctx->stage_events[spans];
+    if (hipStreamQuery(ctx->stream) == hipSuccess) call_workers();
+    else hip(hipEventRecord(front, ctx->stream), "hipEventRecord");
+    ctx->stage_busy = true;
     for (const Fetch &f : fetches) {
+      if (rc) break;
       if (f.whole) {
         rc = f.r->kind == HostKind::kFloats ? stage_copy(ctx, f.r->src, stage + f.at, f.bytes) : lay_out(*f.r, stage + f.at);
       } else {
@@ -574,8 +583,13 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
       }
       if (!rc && f.closes) hip(hipEventRecord(ctx->stage_events[recorded++], ctx->stream), "hipEventRecord");
       if (rc) break;
+      if (!called && hipEventQuery(front) == hipSuccess) call_workers();
       while (there < recorded && hipEventQuery(ctx->stage_events[there]) == hipSuccess)
         arrived.store(++there, std::memory_order_release);
+    }
+    if (!rc && !called) {
+      hip(hipEventSynchronize(front), "hipEventSynchronize");
+      call_workers();
     }
     while (!rc && there < spans) {
       hip(hipEventSynchronize(ctx->stage_events[there]), "hipEventSynchronize");
@@ -626,6 +640,8 @@ void drop_ahead(tpuhip_ctx *ctx, AheadRead &a) {
 // The host sees from the flag that the dense form is there and starts a copy engine on it: that needs no wait of one
 // stream for another (which costs the host 12 us a piece, 60 in front of a copy), and unlike a kernel the engine takes no
 // compute unit from the launches that are still running.
+// A wait of some milliseconds gives its CPU back in between.
+constexpr int kLooks = 4096;
 static int fetch_ahead(tpuhip_ctx *ctx, AheadRead &a) {
   if (a.fetched) return TPUHIP_OK;
   for (int spin = 0; __atomic_load_n(a.flag, __ATOMIC_ACQUIRE) != a.serial; ++spin) {
@@ -636,7 +652,8 @@ static int fetch_ahead(tpuhip_ctx *ctx, AheadRead &a) {
         return set_error(TPUHIP_ERR_HIP, "a result laid out early did not arrive");
       }
     }
-    std::this_thread::yield();
+    if (spin < kLooks) std::this_thread::yield();
+    else std::this_thread::sleep_for(std::chrono::microseconds(20));
   }
   TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
   TPUHIP_CHECK_HIP(hipMemcpyAsync(a.pinned, a.dense, a.bytes, hipMemcpyDeviceToHost, ctx->copy_stream));
