@@ -146,6 +146,8 @@ public:
   bool exposed() const { return exposed_; }
   // whether the tensor was read since the last call of this
   bool take_was_read() const;
+  // zeros in every slot, pad bytes included: memory comes as it is
+  void clear();
   // lays the tensor out again with another channel stride (4 for a tensor of at most 4 channels whose
   // only readers take one dword per pixel, else a multiple of 16); the contents are lost
   void set_channel_stride(int new_cs);

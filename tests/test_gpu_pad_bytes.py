@@ -1,0 +1,73 @@
+"""Device tensors hold zeros between their channels and their channel stride, whatever lay in their memory before a module
+was loaded: tests/cpp/pad_bytes_example.cpp, built by __graft_entry__.build(), counts them."""
+import os
+import re
+import subprocess
+
+import numpy as np
+import pytest
+
+from tpu_compiler_amd import graphs, mlir_text
+
+pytestmark = pytest.mark.gpu
+HERE = os.path.dirname(os.path.abspath(__file__))
+BIN, GOLDEN = os.path.join(HERE, "cpp", "pad_bytes_example.bin"), os.path.join(HERE, "golden")
+
+
+def _count(g, tmp_path):
+    path = tmp_path / "model.mlir"
+    mlir_text.write_mlir(g, path)
+    shape = g.input_op().shape
+    return _count_file(path, tmp_path, input=np.random.default_rng(1).integers(-128, 128, shape).astype(np.float32))
+
+
+def _count_file(path, tmp_path, **inputs):
+    assert os.path.exists(BIN), "build it with __graft_entry__.build()"
+    np.savez(tmp_path / "in.npz", **inputs)
+    res = subprocess.run([BIN, str(path), str(tmp_path / "in.npz")], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=100)
+    assert res.returncode == 0, res.stderr
+    return {line.split()[0]: [int(v) for v in line.split()[1:]] for line in res.stdout.splitlines()}
+
+
+@pytest.mark.parametrize("x_shape,w_shape,y_shape,lt,ot", [
+    ((4, 3, 28), (4, 5, 28), (4, 3, 5), 0, 0), ((4, 3, 28), (5, 28), (4, 3, 5), 0, 0),
+    ((2, 8, 3, 48), (6, 20, 48), (2, 3, 8, 20), 1, 0), ((2, 3, 8, 48), (6, 20, 48), (2, 8, 3, 20), 0, 1),
+    ((2, 8, 3, 48), (2, 3, 20, 48), (2, 8, 3, 20), 1, 1)])
+def test_pads_behind_matrix_products(x_shape, w_shape, y_shape, lt, ot, tmp_path):
+    rng = np.random.default_rng(4)
+    g = graphs.Graph("pads", 1)
+    g.add(graphs.Op("tpu.input", "input", [], x_shape))
+    g.add(graphs.Op("tpu.relu", "r", ["input"], x_shape))       # its place in the reused memory goes to what follows
+    batch = int(np.prod(w_shape[:-2]))
+    g.add(graphs.Op("tpu.fully_connected", "y", ["r"], y_shape, dict(do_relu=0, input_transpose=lt, output_transpose=ot),
+                    dict(filter=rng.integers(-50, 51, w_shape).astype(np.float32),
+                         bias=rng.integers(-2000, 2000, (batch, w_shape[-2])).astype(np.float32),
+                         rshift=np.full(batch, 9, np.float32), multiplier=np.full(batch, 1 << 30, np.float32)),
+                    "RSHIFT_AND_M_I32"))
+    last = "y"
+    if len(y_shape) == 4:                                       # movement kernels take the pads along
+        n, c, h, w = y_shape
+        g.add(graphs.Op("tpu.pad", "p", ["y"], (n, c, h + 2, w + 2), {"const_val": 0, "pads0": 0, "pads1": 0, "pads2": 1, "pads3": 1, "pads4": 0, "pads5": 0, "pads6": 1, "pads7": 1}))
+        last = "p"
+    g.outputs = [last]
+    counts = _count(g, tmp_path)
+    assert set(counts) == {"input", "r", "y"} | {last} and counts["y"][1] > 0
+    assert all(nonzero == 0 for nonzero, _ in counts.values()), counts
+
+
+@pytest.mark.parametrize("make", [lambda: graphs.cfg3_resnet50(batch=1, hw=64), lambda: graphs.cfg4_mobilenet_v2(batch=2, hw=64),
+                                  lambda: graphs.cfg5_yolo_v3(batch=1, hw=96)])
+def test_pads_of_networks(make, tmp_path):
+    g = make()
+    counts = _count(g, tmp_path)
+    assert len(counts) >= len(g.ops) and all(nonzero == 0 for nonzero, _ in counts.values()), counts
+
+
+@pytest.mark.parametrize("name", ["mini_net", "movers", "se_block", "uint8_front", "fp32_edges"])
+def test_pads_of_other_ops(name, tmp_path):
+    path = os.path.join(GOLDEN, name + ".mlir")
+    with open(path) as f:
+        names = re.findall(r'"tpu.input".*?name = "([^"]+)"', f.read())
+    with np.load(os.path.join(GOLDEN, name + "_io.npz")) as z:
+        counts = _count_file(path, tmp_path, **{n: z[n].astype(np.float32) for n in names})
+    assert names and counts and all(nonzero == 0 for nonzero, _ in counts.values()), counts

@@ -161,8 +161,13 @@ void TensorData::set_channel_stride(int new_cs) {
   base_ = nullptr;
   cs = new_cs;
   ck(tpuhip_malloc(ctx_, slot_bytes() * (size_t)batch, &base_), "TensorData::set_channel_stride");
-  ck(tpuhip_memset(ctx_, base_, 0, slot_bytes() * (size_t)batch), "TensorData::set_channel_stride");
+  clear();
   ptr_ = (char *)base_ + slot_bytes() * (size_t)cur_;
+}
+
+void TensorData::clear() {
+  drop_ahead();
+  ck(tpuhip_memset(ctx_, base_, 0, slot_bytes() * (size_t)batch), "TensorData::clear");
 }
 
 void TensorData::set_batch_idx(int32_t bidx) {
@@ -764,6 +769,7 @@ FullyConnectedOpKernel::FullyConnectedOpKernel(OpDesc &op, value_map_t &valueMap
     ck(tpuhip_fc_batched_prepack(ctx, &d, w8.data(), bias ? b32.data() : nullptr, mu.data(), rs.data(),
                                  &packed_batched),
        who.c_str());
+    output_data->clear();   // the kernels write the logical elements alone
   }
 }
 
