@@ -1,6 +1,6 @@
 // Loads a module into device memory that other tensors of the same context had filled, runs it and counts, per tensor, the
-// bytes between its channels and its channel stride that are not zero: `pad_bytes_example model.mlir input.npz` prints
-// "<tensor> <nonzero pad bytes> <pad bytes>" per line.
+// bytes between its channels and its channel stride that are not zero: `pad_bytes_example model.mlir input.npz all.npz`
+// prints "<tensor> <nonzero pad bytes> <pad bytes>" per line and writes every tensor to the last file.
 #include <cstdio>
 #include <fstream>
 #include <iterator>
@@ -13,7 +13,7 @@
 using namespace tpuhip;
 
 int main(int argc, char **argv) {
-  if (argc != 3) return 2;
+  if (argc != 4) return 2;
   try {
     ModuleInterpreter interp;
     auto check = [](int status) {
@@ -50,7 +50,10 @@ int main(int argc, char **argv) {
     for (size_t i = 0; i < names.size(); ++i) interp.setTensor(names[i], values[i], 0);
     interp.invoke(0);
     interp.sync();
+    auto out = openOutputTensorFile(argv[3]);
     for (auto &kv : interp.valueMapping) {
+      std::string name = kv.first;
+      out->addTensor(name, interp.getTensor(name, 0)->data(), interp.getTensorShape(name));
       const TensorData &t = *kv.second;
       if (t.f32 || !t.materialized) continue;
       std::vector<int8_t> bytes(t.slot_bytes());
@@ -60,6 +63,7 @@ int main(int argc, char **argv) {
         for (int c = t.c; c < t.cs; ++c, ++pads) nonzero += bytes[p + (size_t)c] != 0;
       printf("%s %zu %zu\n", kv.first.c_str(), nonzero, pads);
     }
+    out->keep();
   } catch (const std::exception &e) {
     fprintf(stderr, "%s\n", e.what());
     return 1;

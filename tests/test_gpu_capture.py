@@ -95,6 +95,20 @@ def test_a_network_that_ran_once_from_files_can_be_recorded(make, tmp_path):
     m.close()
 
 
+def test_a_network_that_ran_once_from_files_chooses_its_tiles_at_the_next_use(tmp_path):
+    g, m = graphs.cfg3_resnet50(batch=1, hw=104), module()
+    _run_files(m, g, tmp_path)
+    untimed = m.kernels()
+    graph = Graph(m.context_handle())
+    m.invoke()                           # times the variants and packs the filters again
+    assert m.kernels() != untimed
+    with graph.recording():
+        m.invoke()
+    _check_replays(m, g, graph, m.invoke)
+    graph.close()
+    m.close()
+
+
 def test_a_layer_whose_first_use_is_recorded_is_refused():
     g = graphs.cfg3_resnet50(batch=1, hw=88)
     for remembered in (False, True):     # the second module's shapes have been timed by the first

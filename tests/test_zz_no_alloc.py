@@ -1,8 +1,7 @@
 """The allocation-free FullyConnected entry point (tpuhip_fc_i8_noalloc) through the C ABI: its
-output must equal that of tpuhip_fc_i8 -- one launch with the partial sums in LDS for the
-first, long-K layer; for the second the same split-K kernels with a scratch buffer the library
-allocates -- byte for byte, on two calls in a row, the second on a smaller input (the static
-scratch keeps the first call's partial sums)."""
+output must equal that of tpuhip_fc_i8 -- one launch with the partial sums in LDS, of sixteen
+waves for the first, long-K layer, of four for the second -- byte for byte, on two calls in a
+row, the second on a smaller input (the static scratch keeps the first call's partial sums)."""
 import numpy as np
 import pytest
 
@@ -35,8 +34,8 @@ def test_fc_noalloc_equals_fc_on_two_calls_in_a_row():
         ctx.fc(wh, xt, y_ws)
         ctx.fc(wh, xt, y_static, noalloc=True)
         a, b = ctx.to_nchw(y_ws).reshape(m, n), ctx.to_nchw(y_static).reshape(m, n)
-        assert np.array_equal(a, want), "the workspace path differs from the oracle"
-        assert np.array_equal(b, a), "the static-scratch path differs from the workspace path"
+        assert np.array_equal(a, want), "the one-launch path differs from the oracle"
+        assert np.array_equal(b, a), "the static-scratch path differs from the one-launch path"
         assert np.array_equal(ctx.raw(y_static), ctx.raw(y_ws))             # pad channels too
         # once more on the same buffers
         ctx._ck(ctx.lib.tpuhip_memset(ctx.h, y_static.ptr, 0x55, y_static.nbytes))
