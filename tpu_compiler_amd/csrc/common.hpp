@@ -42,7 +42,8 @@ struct tpuhip_ctx {
   // when set, every kernel launch carries these events: they bracket the dispatch
   // itself (begin / end of execution), not the gaps around it
   hipEvent_t prof_start = nullptr, prof_stop = nullptr;
-  // device memory kernels use beyond their operands (split-K partial sums): allocated on first need, grown when a larger layer comes, freed with the context
+  // device memory kernels use beyond their operands (partial sums of average pools over large windows): allocated on first
+  // need, replaced when a larger one comes, freed with the context; never used by a launch that is being recorded
   void *workspace = nullptr;
   size_t workspace_bytes = 0;
   // host tensors on their way to and from the device (host/host_io.cpp): a pinned buffer of at most 32 MiB, device memory

@@ -57,7 +57,8 @@ struct tpuhip_conv_weights {
   bool fc_only = false;
   // the direct path's layers where the caller left the choice: their form on the matrix cores (NULL: not covered)
   GatherPlan *gather = nullptr;
-  int8_t *raw = nullptr;     // the filter as OIHW on the device, kept while the layer can still be repacked
+  int8_t *raw = nullptr;     // the filter as OIHW on the device: until the tile is settled; of a depthwise layer, and of one
+                             // whose tile a recorded graph fixed, as long as the layer
   int8_t *w = nullptr;   // packed filter
   size_t w_room = 0;     // bytes behind w
   int8_t *params = nullptr;   // one allocation behind bias, qp, qplanes and qc64
@@ -3312,8 +3313,10 @@ __global__ __launch_bounds__(W * 64) void conv_mfma_ksplit_kernel(ConvArgs a) {
 }
 
 // The arguments of a conv with nothing fused behind it whose numbers fit these types: two cache lines instead of ten for the
-// kernel to wait for, and below the 112 bytes up to which a launch costs the host 0.5 us less.  64 -> 64 channels 3x3 on
-// 1 x 56 x 56, called from Python: 4.45 us, now 3.93.
+// kernel to wait for, and below the 112 bytes up to which a launch costs the host less.  64 -> 64 channels 3x3 on
+// 1 x 56 x 56, called from Python, medians of eight processes of each: 4.20 us, now 3.84.  Processes fall into two groups by
+// where the runtime keeps the arguments: 3.55 to 3.43 in the one, 4.3 to 3.87 in the other; 512 -> 512 on 7 x 7, bound by the
+// kernel, 7.05 to 6.92.
 struct LeanArgs {
   const int8_t *x, *w;
   int8_t *y;
@@ -4165,7 +4168,9 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t) {
   if (c.reg == 6 && patch2_rows(d, c) == 0) return false;
   if (c.reg == 7) return patch3_plan(d, c).th > 0;
   // worth timing only where the tiles are few: with more of them than the chip holds workgroups the layer has parallel
-  // work enough without splitting K sixteen ways
+  // work enough without splitting K.  Of 18 layers of one image (1x1 and 3x3, 64 to 512 channels) the K-split forms were the
+  // fastest of all in 10 at 256 tiles (256 -> 256 channels 3x3: 5.3 us against 7.4), in 3 at 512, in none at 1024 (14.3
+  // against 8.2) and 2048 (27.0 against 13.2): the line is four times where they were last seen to win
   if (c.reg == 8 && ceil_div64((int64_t)d.n * d.oh * d.ow, 32) * ceil_div64(d.oc, 32) > 2048) return false;
   if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8)) return false;   // prefer the 4-channel K packing of the LDS kernels
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle

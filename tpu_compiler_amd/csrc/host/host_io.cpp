@@ -277,13 +277,16 @@ void finish_job(HostJob &job) {
 
 constexpr size_t kPiece = 256 << 10;        // bytes of the staging buffer per piece of a host pass
 constexpr size_t kAlone = 192 << 10;        // up to here one thread is done before a worker has woken
-// Floats on their way to the device: below this many bytes of them one thread converts nearly as fast as the bus takes the
-// result (19 MB: 300 us alone, 184 on eight threads; 38 MB, beyond the last-level cache: 1220 and 324), and the caller's
-// buffer stays in the caches of the core that will write it again.  Bytes are copied faster than the bus at any size.
+// Floats on their way to the device: from this many bytes of them on the conversion is worth eight threads.  set_tensor of a
+// buffer written just before, alone / on eight: 4 MB 136 / 69 us, 8 MB 268 / 95, 12 MB 407 / 119, 16 MB 531 / 145, 32 MB 1073 /
+// 255; with the caller's next write of the buffer, whose lines the other cores then hold, 4 MB 238 / 181, 8 MB 436 / 301, 12 MB
+// 638 / 409.  So eight are faster from 2 MB on (142 / 124); the line lies higher because below it they take two to three times
+// the CPU time for it.  Bytes are copied by one thread at any size.
 constexpr size_t kSharedFloats = 12 << 20;
-// The lines of the staging buffer are written past the caches where that is not slower: 8 images of 3 x 608 x 608 bytes 347 us
-// with cached stores (the lines are fetched to be overwritten, and the bus takes them out of the caches again), 257 to 297 so;
-// below these bytes the copy returns earlier with cached ones and the transfer ends no later.
+// From these bytes on the lines of the staging buffer are written past the caches: cached stores fetch the lines to overwrite
+// them, and the bus takes them out of the caches again.  Until the transfer has ended, cached / past the caches, source in the
+// caches: 1 MB 60 / 60 us, 2 MB 100 / 87, 4 MB 194 / 166, 6 MB 267 / 222, 8 MB 349 / 292, 12 MB 515 / 418, 24 MB 1270 / 800.  The
+// gain begins at 2 MB; with the caller's next write of the source it is 2 MB 130 / 133, 4 MB 272 / 246, 6 MB 366 / 337.
 constexpr size_t kCachedBytes = 6 << 20;
 constexpr size_t kStageMax = 32 << 20;      // the staging buffer grows to this; larger tensors go through it in parts
 
