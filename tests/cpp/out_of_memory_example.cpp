@@ -1,0 +1,100 @@
+// Calls that would rather have more memory do without it: this program defines the allocation functions that the library
+// calls, refuses what the running case says (with the runtime's own error), and compares the results with those of plenty.
+// `out_of_memory_example <case>` exits with 0 when they agree.
+#include <dlfcn.h>
+
+#include <cstdio>
+#include <cstring>
+#include <functional>
+#include <vector>
+
+#include "tpuhip/interpreter.hpp"
+
+using namespace tpuhip;
+
+namespace {
+std::function<bool(size_t)> refuse;   // whether an allocation of that many bytes fails
+int refused = 0;
+constexpr size_t kNever = (size_t)1 << 60;
+
+template <class F>
+F next(const char *name) {
+  return reinterpret_cast<F>(dlsym(RTLD_NEXT, name));
+}
+}  // namespace
+
+extern "C" int hipMalloc(void **p, size_t bytes) {
+  static const auto real = next<int (*)(void **, size_t)>("hipMalloc");
+  if (refuse && refuse(bytes)) ++refused, bytes = kNever;
+  return real(p, bytes);
+}
+extern "C" int hipHostMalloc(void **p, size_t bytes, unsigned flags) {
+  static const auto real = next<int (*)(void **, size_t, unsigned)>("hipHostMalloc");
+  if (refuse && refuse(bytes)) ++refused, bytes = kNever;
+  return real(p, bytes, flags);
+}
+
+namespace {
+
+void check(int status) {
+  if (status != TPUHIP_OK) throw std::runtime_error(tpuhip_last_error());
+}
+void expect(bool ok, const char *what) {
+  if (!ok) throw std::runtime_error(what);
+}
+
+OpDesc op(const char *type, const std::string &name, SyncedDataShape shape, std::vector<std::string> operands) {
+  OpDesc d;
+  d.type = type;
+  d.name = name;
+  d.shape = std::move(shape);
+  d.operands = std::move(operands);
+  return d;
+}
+
+std::vector<int8_t> values(size_t n, unsigned seed) {
+  std::vector<int8_t> v(n);
+  for (auto &x : v) x = (int8_t)((seed = seed * 1664525u + 1013904223u) >> 24);
+  return v;
+}
+
+// an output that is complete before the last kernel, read after every invoke
+void early_output() {
+  const SyncedDataShape shape = {1, 70, 50, 41};
+  const size_t n = 70 * 50 * 41;
+  ModuleDesc m;
+  m.ops = {op("tpu.input", "x", shape, {}), op("tpu.relu", "first", shape, {"x"}), op("tpu.relu", "second", shape, {"x"})};
+  m.returns = {"first", "second"};
+  ModuleInterpreter interp;
+  interp.loadModule(m);
+  for (unsigned k = 0; k < 5; ++k) {
+    const auto x = values(n, k);
+    interp.setTensorI8("x", x.data(), n, 0);
+    refuse = [](size_t bytes) { return bytes > (128 << 10); };   // only what is laid out early is as large by now
+    if (k == 0) refuse = nullptr;
+    interp.invoke(0);
+    for (const char *name : {"first", "second"}) {
+      std::vector<int8_t> y(n);
+      interp.getTensorI8(name, y.data(), n, 0);
+      for (size_t i = 0; i < n; ++i) expect(y[i] == (x[i] < 0 ? 0 : x[i]), name);
+    }
+  }
+  refuse = nullptr;
+  expect(refused > 0, "nothing was refused");
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  if (argc != 2) return 2;
+  try {
+    const std::string which = argv[1];
+    if (which == "early_output") early_output();
+    else return 2;
+  } catch (const std::exception &e) {
+    refuse = nullptr;
+    fprintf(stderr, "%s\n", e.what());
+    return 1;
+  }
+  return 0;
+}

@@ -617,13 +617,20 @@ __global__ void arrived_kernel(uint32_t *flag, uint32_t value) {
   __hip_atomic_store(flag, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src) {
+int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src, bool *done) {
+  *done = false;
   const size_t bytes = ((size_t)t.n * t.c * t.h * t.w + 63) / 64 * 64;
-  if (!ctx->copy_stream) TPUHIP_CHECK_HIP(hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking));
   drop_ahead(ctx, a);
   if (!a.pinned) {
-    TPUHIP_CHECK_HIP(hipMalloc(&a.dense, bytes + 256));
-    TPUHIP_CHECK_HIP(hipHostMalloc(&a.pinned, bytes + 64, hipHostMallocDefault));
+    if (a.refused) return TPUHIP_OK;
+    if ((!ctx->copy_stream && hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking) != hipSuccess) ||
+        hipMalloc(&a.dense, bytes + 256) != hipSuccess || hipHostMalloc(&a.pinned, bytes + 64, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();   // a read does without
+      if (a.dense) (void)hipFree(a.dense);
+      a.dense = nullptr;
+      a.refused = true;
+      return TPUHIP_OK;
+    }
     a.flag = (uint32_t *)((char *)a.pinned + bytes);
     *a.flag = 0;
   }
@@ -633,6 +640,7 @@ int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *s
   a.bytes = (size_t)t.n * t.c * t.h * t.w;
   a.fetched = false;
   ctx->ahead.push_back(&a);
+  *done = true;
   return TPUHIP_OK;
 }
 

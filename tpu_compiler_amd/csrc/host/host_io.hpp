@@ -50,10 +50,11 @@ struct AheadRead {
   void *dense = nullptr, *pinned = nullptr;
   uint32_t *flag = nullptr, serial = 0;   // the flag, in pinned memory, shows the serial of what lies in `dense`
   size_t bytes = 0;
+  bool refused = false;                   // there is no memory for it
   bool fetched = false;                   // `pinned` holds it, or a copy to there is in flight (not beyond settle_ahead())
   ~AheadRead();
 };
-int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src);
+int read_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostTensor &t, const void *src, bool *done);   // !*done: there is no memory for it
 // the host pass from a's bytes instead of r.src
 int finish_ahead(tpuhip_ctx *ctx, AheadRead &a, const HostRead &r);
 // waits for everything the context has issued; what else has been laid out early is fetched meanwhile

@@ -137,8 +137,9 @@ bool TensorData::take_was_read() const {
 void TensorData::read_ahead() {
   if (exposed_ || !materialized || f32) return;
   if (!ahead_) ahead_ = std::make_unique<AheadRead>();
-  ck(tpuhip::read_ahead(ctx_, *ahead_, HostTensor{n, c, h, w, cs, is_unsigned}, ptr_), "TensorData::read_ahead");
-  ahead_slot_ = cur_;
+  bool done = false;
+  ck(tpuhip::read_ahead(ctx_, *ahead_, HostTensor{n, c, h, w, cs, is_unsigned}, ptr_, &done), "TensorData::read_ahead");
+  if (done) ahead_slot_ = cur_;
 }
 
 bool TensorData::finish_ahead(const HostRead &r, int32_t bidx) const {
