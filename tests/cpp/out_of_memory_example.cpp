@@ -3,6 +3,7 @@
 // `out_of_memory_example <case>` exits with 0 when they agree.
 #include <dlfcn.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <functional>
@@ -83,6 +84,40 @@ void early_output() {
   expect(refused > 0, "nothing was refused");
 }
 
+// a global average over a large map, whose partial sums would go to a workspace
+void pool_workspace() {
+  tpuhip_ctx *ctx = nullptr;
+  check(tpuhip_ctx_create(0, &ctx));
+  const int n = 2, c = 120, h = 60, w = 50, cs = 128;
+  const auto x = values((size_t)n * c * h * w, 3);
+  void *dense = nullptr, *in = nullptr, *out = nullptr;
+  check(tpuhip_malloc(ctx, x.size(), &dense));
+  check(tpuhip_malloc(ctx, (size_t)n * h * w * cs, &in));
+  check(tpuhip_malloc(ctx, (size_t)n * cs, &out));
+  check(tpuhip_upload(ctx, dense, x.data(), x.size()));
+  check(tpuhip_nchw_to_nhwc_i8(ctx, dense, in, n, c, h, w, cs));
+  const tpuhip_pool_desc d = {n, c, h, w, 1, 1, h, w, 1, 1, 0, 0, 0, 0, cs, cs};
+  std::vector<int8_t> got[2];
+  for (int with = 0; with < 2; ++with) {
+    refuse = [with](size_t) { return with == 0; };
+    check(tpuhip_memset(ctx, out, 0x55, (size_t)n * cs));
+    check(tpuhip_pool_avg_i8(ctx, &d, in, out, 81, 13));
+    got[with].resize((size_t)n * cs);
+    check(tpuhip_download(ctx, got[with].data(), out, got[with].size()));
+  }
+  refuse = nullptr;
+  for (void *p : {dense, in, out}) check(tpuhip_free(ctx, p));
+  check(tpuhip_ctx_destroy(ctx));
+  expect(refused > 0, "nothing was refused");
+  expect(got[0] == got[1], "the averages differ");
+  for (int k = 0; k < c; ++k) {
+    int32_t s = 0;
+    for (int i = 0; i < h * w; ++i) s += x[(size_t)k * h * w + i];
+    const float q = std::fmin(std::fmax((float)s * 81.0f / 8192.0f, -128.0f), 127.0f);   // sat8
+    expect(std::fabs((float)got[0][k] - q) <= 0.5f, "an average is wrong");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -90,6 +125,7 @@ int main(int argc, char **argv) {
   try {
     const std::string which = argv[1];
     if (which == "early_output") early_output();
+    else if (which == "pool_workspace") pool_workspace();
     else return 2;
   } catch (const std::exception &e) {
     refuse = nullptr;

@@ -26,7 +26,13 @@ int grow_workspace(tpuhip_ctx *ctx, size_t bytes) {
   if (ctx->workspace) TPUHIP_CHECK_HIP(hipFree(ctx->workspace));
   ctx->workspace = nullptr;
   ctx->workspace_bytes = 0;
-  TPUHIP_CHECK_HIP(hipMalloc(&ctx->workspace, bytes));
+  const hipError_t e = hipMalloc(&ctx->workspace, bytes);
+  if (e == hipErrorOutOfMemory) {
+    ctx->workspace = nullptr;
+    (void)hipGetLastError();
+    return set_error(TPUHIP_ERR_NOMEM, "no device memory for a workspace of %zu bytes", bytes);
+  }
+  TPUHIP_CHECK_HIP(e);
   ctx->workspace_bytes = bytes;
   return TPUHIP_OK;
 }

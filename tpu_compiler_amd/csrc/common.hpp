@@ -104,7 +104,8 @@ int pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t larg
 // waits for what a prepack call has issued, unless a module is being loaded: packed weights may be used from any context
 int prepack_done(tpuhip_ctx *ctx);
 
-// api.hip: makes ctx->workspace at least this large; waits for the stream when it has to be replaced
+// api.hip: makes ctx->workspace at least this large; waits for the stream when it has to be replaced.  TPUHIP_ERR_NOMEM: there
+// is none, and the call may do without
 int grow_workspace(tpuhip_ctx *ctx, size_t bytes);
 
 int set_error(int status, const char *fmt, ...) __attribute__((format(printf, 2, 3)));

@@ -284,14 +284,18 @@ int run_window(tpuhip_ctx *ctx, const PoolArgs &a) {
   const int gblocks = (c16 + G - 1) / G, taps = a.kh * a.kw;
   const int64_t pixels = a.total / c16, blocks = pixels * gblocks;
   // two workgroups per CU, while every lane keeps four positions; no slices where the grid of the second launch does not
-  // reach, nor in a recorded launch: a graph may outlive this context's workspace, or replay beside another one
+  // reach or there is no memory, nor in a recorded launch: a graph may outlive this context's workspace, or replay beside
+  // another one
   int64_t slices = std::min<int64_t>(std::min<int64_t>(2 * ctx->num_cu / blocks, taps / (4 * 256 / G)), 32);
   if (slices < 2 || pixels > 65535) slices = 1;
   if (slices > 1) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     TPUHIP_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &capture));
-    if (capture != hipStreamCaptureStatusNone) slices = 1;
-    else if (int rc = grow_workspace(ctx, (size_t)(pixels * slices * c16 * 16) * sizeof(int32_t))) return rc;
+    const int rc = capture != hipStreamCaptureStatusNone
+                       ? TPUHIP_ERR_NOMEM
+                       : grow_workspace(ctx, (size_t)(pixels * slices * c16 * 16) * sizeof(int32_t));
+    if (rc == TPUHIP_ERR_NOMEM) slices = 1;
+    else if (rc) return rc;
   }
   int32_t *parts = slices > 1 ? (int32_t *)ctx->workspace : nullptr;
   const int per_slice = (int)((taps + slices - 1) / slices);
