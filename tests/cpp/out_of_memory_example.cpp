@@ -118,6 +118,28 @@ void pool_workspace() {
   }
 }
 
+// a module loads where there is no room for the slabs that its tensors and weights would share
+void slab() {
+  const SyncedDataShape shape = {1, 16, 20, 20};
+  const size_t n = 16 * 20 * 20;
+  ModuleDesc m;
+  m.ops = {op("tpu.input", "x", shape, {}), op("tpu.relu", "y", shape, {"x"}), op("tpu.relu", "z", shape, {"y"})};
+  m.returns = {"z"};
+  refuse = [](size_t bytes) { return bytes >= ((size_t)16 << 20); };
+  for (int again = 0; again < 2; ++again) {   // and gives its memory back
+    ModuleInterpreter interp;
+    interp.loadModule(m);
+    const auto x = values(n, 5);
+    interp.setTensorI8("x", x.data(), n, 0);
+    interp.invoke(0);
+    std::vector<int8_t> y(n);
+    interp.getTensorI8("z", y.data(), n, 0);
+    for (size_t i = 0; i < n; ++i) expect(y[i] == (x[i] < 0 ? 0 : x[i]), "z");
+  }
+  refuse = nullptr;
+  expect(refused > 0, "nothing was refused");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -126,6 +148,7 @@ int main(int argc, char **argv) {
     const std::string which = argv[1];
     if (which == "early_output") early_output();
     else if (which == "pool_workspace") pool_workspace();
+    else if (which == "slab") slab();
     else return 2;
   } catch (const std::exception &e) {
     refuse = nullptr;

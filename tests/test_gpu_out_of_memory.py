@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "out_of_memory_example.bin")
 
 
-@pytest.mark.parametrize("case", ["early_output", "pool_workspace"])
+@pytest.mark.parametrize("case", ["early_output", "pool_workspace", "slab"])
 def test_results_without_the_memory_a_call_would_like(case):
     assert os.path.exists(BIN), "build it with __graft_entry__.build()"
     res = subprocess.run([BIN, case], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=100)

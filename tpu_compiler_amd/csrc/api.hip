@@ -57,7 +57,10 @@ static int slab_malloc(tpuhip_ctx *ctx, size_t bytes, void **dptr) {
       }
     void *base = nullptr;
     const hipError_t e = hipMalloc(&base, kSlab);
-    if (e == hipErrorOutOfMemory) return TPUHIP_ERR_NOMEM;
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      return TPUHIP_ERR_NOMEM;
+    }
     TPUHIP_CHECK_HIP(e);
     tpuhip_ctx::Slab s{(char *)base, kSlab, {}};
     s.unused[0] = kSlab;
@@ -177,8 +180,7 @@ int tpuhip_malloc(tpuhip_ctx *ctx, size_t bytes, void **dptr) {
   // past the logical end of a tensor.
   if (ctx->loading && bytes <= kSlabPart) {
     const int rc = slab_malloc(ctx, bytes + 256, dptr);
-    if (rc == TPUHIP_ERR_NOMEM) return set_error(rc, "tpuhip_malloc: out of device memory (%zu bytes)", bytes);
-    return rc;
+    if (rc != TPUHIP_ERR_NOMEM) return rc;   // where there is no room for a slab there may be for this
   }
   hipError_t e = hipMalloc(dptr, bytes + 256);
   if (e == hipErrorOutOfMemory)
