@@ -1,7 +1,10 @@
-// Calls that would rather have more memory do without it: this program defines the allocation functions that the library
-// calls, refuses what the running case says (with the runtime's own error), and compares the results with those of plenty.
-// `out_of_memory_example <case>` exits with 0 when they agree.
+// Calls that would rather have more memory, or threads, do without them: this program defines the functions that the library
+// gets them by, refuses what the running case says (memory with the runtime's own error), and checks the results.
+// `doing_without_example <case> [model.mlir]` exits with 0 when they are right.
 #include <dlfcn.h>
+#include <pthread.h>
+
+#include <cerrno>
 
 #include <cmath>
 #include <cstdio>
@@ -15,6 +18,7 @@ using namespace tpuhip;
 
 namespace {
 std::function<bool(size_t)> refuse;   // whether an allocation of that many bytes fails
+bool no_threads = false;
 int refused = 0;
 constexpr size_t kNever = (size_t)1 << 60;
 
@@ -33,6 +37,15 @@ extern "C" int hipHostMalloc(void **p, size_t bytes, unsigned flags) {
   static const auto real = next<int (*)(void **, size_t, unsigned)>("hipHostMalloc");
   if (refuse && refuse(bytes)) ++refused, bytes = kNever;
   return real(p, bytes, flags);
+}
+
+extern "C" int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *arg) {
+  static const auto real = next<int (*)(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *)>("pthread_create");
+  if (no_threads) {
+    ++refused;
+    return EAGAIN;
+  }
+  return real(t, a, f, arg);
 }
 
 namespace {
@@ -140,18 +153,61 @@ void slab() {
   expect(refused > 0, "nothing was refused");
 }
 
+// the host passes of large tensors and the reading of weights beside the text
+void threads(const char *model) {
+  const SyncedDataShape shape = {4, 64, 128, 128};
+  const size_t n = (size_t)4 * 64 * 128 * 128;
+  ModuleDesc m;
+  m.ops = {op("tpu.input", "x", shape, {}), op("tpu.relu", "y", shape, {"x"})};
+  m.returns = {"y"};
+  ModuleInterpreter interp;
+  interp.loadModule(m);
+  std::string in = "x";
+  const auto x = values(n, 7);
+  interp.setTensorI8(in, x.data(), n, 0);   // on one thread: what the runtime starts for transfers, it has started then
+  interp.invoke(0);
+  interp.sync();
+  for (bool without : {true, false}) {
+    no_threads = without;
+    std::vector<float> f(n), got(n);
+    for (size_t i = 0; i < n; ++i) f[i] = (float)(without ? x[i] : x[n - 1 - i]);
+    interp.setTensor(in, f, 0);
+    interp.invoke(0);
+    interp.getTensor("y", got.data(), n, 0);
+    for (size_t i = 0; i < n; ++i) expect(got[i] == (f[i] < 0 ? 0 : f[i]), "y");
+  }
+  ModuleInterpreter first, second;
+  std::vector<float> results[2];
+  for (int k = 0; k < 2; ++k) {
+    ModuleInterpreter &file = k ? second : first;
+    no_threads = k == 0;
+    file.loadModuleFile(model);
+    const size_t count = file.input_details[0].second;
+    const auto v = values(count, 9);
+    file.setTensorI8(file.input_details[0].first, v.data(), count, 0);
+    file.invoke(0);
+    no_threads = false;
+    std::string out = file.output_details[0];
+    results[k] = *file.getTensor(out, 0);
+  }
+  expect(results[0] == results[1], "the results differ");
+  expect(refused > 1, "nothing was refused");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-  if (argc != 2) return 2;
+  if (argc < 2) return 2;
   try {
     const std::string which = argv[1];
     if (which == "early_output") early_output();
     else if (which == "pool_workspace") pool_workspace();
     else if (which == "slab") slab();
+    else if (which == "threads" && argc == 3) threads(argv[2]);
     else return 2;
   } catch (const std::exception &e) {
     refuse = nullptr;
+    no_threads = false;
     fprintf(stderr, "%s\n", e.what());
     return 1;
   }

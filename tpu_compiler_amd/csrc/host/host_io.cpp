@@ -13,6 +13,7 @@
 #include <functional>
 #include <memory>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -240,7 +241,10 @@ class HostWorkers {
     pid_ = getpid();
     // seven beside the caller reach the memory bandwidth of a socket's share; never more than the CPUs there are
     const int count = std::max(0, std::min(7, usable_cpus() - 1));
-    for (int i = 0; i < count; ++i) threads_.emplace_back([this] { work(); });
+    try {
+      for (int i = 0; i < count; ++i) threads_.emplace_back([this] { work(); });
+    } catch (const std::system_error &) {   // those there are, or none: the caller does what they do not
+    }
   }
 
   void work() {

@@ -7,6 +7,7 @@
 #include <fstream>
 #include <future>
 #include <sstream>
+#include <system_error>
 
 #include "tpuhip/interpreter.hpp"
 #include "tpuhip/mlir_text.hpp"
@@ -75,8 +76,11 @@ void ModuleInterpreter::loadModuleFile(const std::string &mlir_path, std::string
   // the weights are read while the text is parsed (14 MB: 0.3 ms; 67 KB of text: 0.6 ms)
   const std::string guess = likely_weight_file(text);
   std::future<std::unique_ptr<TensorFile>> reading;
-  if (!guess.empty())
-    reading = std::async(std::launch::async, [&] { return std::make_unique<TensorFile>(weight_path(mlir_path, guess), true); });
+  try {
+    if (!guess.empty())
+      reading = std::async(std::launch::async, [&] { return std::make_unique<TensorFile>(weight_path(mlir_path, guess), true); });
+  } catch (const std::system_error &) {   // no thread to be had: behind the text then
+  }
   MlirModule mm = moduleFromMlir(parseMlirText(text));
   weight_file_path_ = mm.weight_file;
   op_info_.clear();
