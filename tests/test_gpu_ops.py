@@ -1727,3 +1727,15 @@ def test_pool_square_windows(ctx, shape, k, s, pads):
         run()
         assert np.array_equal(ctx.to_nchw(yt), want)
         assert not ctx.raw(yt)[..., shape[1]:].any()
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_a_freed_input_is_refused_by_the_library(ctx, which):
+    x = np.ones((1, 16, 4, 4), np.int8)
+    xs, y, joined = [ctx.from_nchw(x), ctx.from_nchw(x)], ctx.tensor(x.shape), ctx.tensor((1, 32, 4, 4))
+    xs[which].free()
+    for call in (lambda: ctx.eltwise_add(xs, [1, 1], 0, False, y), lambda: ctx.concat(xs, 1, joined)):
+        with pytest.raises(capi.TpuHipError, match="input %d is NULL" % which):
+            call()
+    for t in (xs[1 - which], y, joined):
+        t.free()

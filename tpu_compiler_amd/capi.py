@@ -676,7 +676,7 @@ class Context:
         return self.lib.tpuhip_conv2d_algo_name(w).decode()
 
     def eltwise_add(self, xs, mult, rshift, do_relu, y):
-        ptrs = struct.pack("%dP" % len(xs), *[t.ptr for t in xs])
+        ptrs = struct.pack("%dP" % len(xs), *[t.ptr or 0 for t in xs])
         m = _packed("b", mult, np.int8)
         if rc := self._ops.eltwise_add_i8(self.h, ptrs, len(xs), m, int(rshift), int(do_relu), y.ptr, y.nbytes):
             self._ck(rc)
@@ -750,7 +750,7 @@ class Context:
 
     def concat(self, xs, axis, y, rshift=None, mult=None, do_relu=False):
         n = len(xs)
-        ptrs = struct.pack("%dP" % n, *[t.ptr for t in xs])
+        ptrs = struct.pack("%dP" % n, *[t.ptr or 0 for t in xs])
         dims = struct.pack("%di" % (4 * n), *[v for t in xs for v in t.shape])
         cs = struct.pack("%di" % n, *[t.cs for t in xs])
         r = None if rshift is None else _packed("I", rshift, np.uint32)
