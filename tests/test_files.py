@@ -294,3 +294,29 @@ def test_damaged_files_raise_errors_and_never_crash(tmp_path):
         except capi.TpuHipError:
             refused += 1
     assert refused > 150
+
+
+@pytest.mark.parametrize("shape,word,fits", [
+    ("(4,)", 4, True), ("(5,)", 4, False), ("(0,)", 4, True), ("(0, 9223372036854775807)", 4, True), ("()", 4, True),
+    ("(4611686018427387896,)", 4, False), ("(2305843009213693948, 2)", 4, False), ("(2147483648, 2147483648, 4)", 4, False),
+    ("(9223372036854775807, 9223372036854775807)", 8, False), ("(2, 2)", 4, True), ("(2, 2)", 8, False)])
+def test_shapes_are_held_against_the_bytes_that_are_there(tmp_path, shape, word, fits):
+    """... also those whose product wraps to what is there, or to less"""
+    import ctypes as C
+    import zipfile
+    header = ("{'descr': '<f%d', 'fortran_order': False, 'shape': %s, }" % (word, shape)).encode()
+    header += b" " * (-(10 + len(header) + 1) % 64) + b"\n"
+    path = tmp_path / "shaped.npz"
+    with zipfile.ZipFile(path, "w") as z:
+        z.writestr("a.npy", b"\x93NUMPY\x01\x00" + len(header).to_bytes(2, "little") + header + np.arange(4, dtype=np.float32).tobytes())
+    if not fits:
+        with pytest.raises(capi.TpuHipError, match="data shorter"):
+            capi.TensorFile(path)
+        return
+    f = capi.TensorFile(path)
+    count = int(np.prod(f.info("a")[0])) if "9223" not in shape else 0
+    out = np.zeros(8, np.float32)
+    assert f.lib.tpuhip_npz_read_f32(f.h, b"a", out.ctypes.data, C.c_size_t(count)) == 0
+    assert np.array_equal(out[:count], np.arange(count)) and not out[count:].any()
+    assert f.lib.tpuhip_npz_read_f32(f.h, b"a", out.ctypes.data, C.c_size_t(count + (1 << 62))) != 0
+    f.close()

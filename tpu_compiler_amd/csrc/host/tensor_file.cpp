@@ -86,8 +86,14 @@ NpyArray parse_npy(const uint8_t *p, size_t n, const std::string &member, const 
       while (q < t.size() && t[q] == 'L') ++q;
     }
   }
-  const size_t want = a.count() * (size_t)a.word_size;
-  if (hoff + hlen + want > n) fail("member '" + member + "': data shorter than its shape says");
+  // shapes come from the file: each factor against what is left, so that a product near 2^64 cannot wrap
+  const size_t left = n - hoff - hlen;
+  size_t want = std::count(a.shape.begin(), a.shape.end(), 0) ? 0 : (size_t)a.word_size;
+  for (size_t i = 0; want && i < a.shape.size(); ++i) {
+    if (want > left / (size_t)a.shape[i]) fail("member '" + member + "': data shorter than its shape says");
+    want *= (size_t)a.shape[i];
+  }
+  if (want > left) fail("member '" + member + "': data shorter than its shape says");
   *values = p + hoff + hlen;
   *size = want;
   return a;
@@ -267,7 +273,7 @@ const void *TensorFile::floats(const std::string &name, size_t count) const {
   if (it == map.end()) return nullptr;
   const NpyArray &a = it->second.array;
   const size_t have = it->second.data ? it->second.size : a.num_bytes();
-  return a.kind == 'f' && a.word_size == 4 && have == count * sizeof(float) ? it->second.values() : nullptr;
+  return a.kind == 'f' && a.word_size == 4 && have / sizeof(float) == count ? it->second.values() : nullptr;
 }
 
 std::shared_ptr<const void> TensorFile::kept() const { return std::make_shared<std::pair<decltype(image), decltype(inflated)>>(image, inflated); }
