@@ -122,6 +122,9 @@ struct ConvArgs {
   // lut_dst (may be null) receives table[y]; the add then takes table[y]
   int has_lut;
   int8_t *lut_dst;
+  // a table that is max(y, (y * slope_m + 2^(slope_r - 1)) >> slope_r) (a leaky ReLU's) is computed instead: slope_m > 0,
+  // has_lut 0, the rest as with a table
+  int slope_m, slope_r;
   Table256 lut;
 #ifdef TPUHIP_TRACE
   unsigned long long *trace;   // development builds: 32 shader-clock stamps per workgroup
@@ -263,7 +266,10 @@ __device__ __forceinline__ void requant_rows(const v16i (&acc)[TN], int relu_fir
 __device__ __forceinline__ void finish_chunk(v4i o, const v4i &sv, int64_t off, int oc, const ConvArgs &a,
                                              int8_t *ydst, const uint8_t *lut) {
   if (a.store_y) *reinterpret_cast<v4i *>(ydst + off) = o;
-  if (lut) {
+  if (a.slope_m) {
+    o = leaky_chunk(o, a.slope_m, a.slope_r);
+    if (a.lut_dst) *reinterpret_cast<v4i *>(a.lut_dst + off) = o;
+  } else if (lut) {
     // table lookup per byte (index = the two's-complement byte); the 256-byte table
     // covers each LDS bank once, so any 64 indices are conflict-free.  Pad channels
     // stay zero whatever table[0] is.
@@ -3292,7 +3298,10 @@ __device__ __forceinline__ void ksplit_body(const ConvArgs &a) {
                          requant_core<FAST>(t[2], mult[2], shift[2], hpot[2]), requant_core<FAST>(t[3], mult[3], shift[3], hpot[3]), out.lo);
   if (!live) return;
   if (a.store_y) *reinterpret_cast<uint32_t *>(out.y + off) = o;
-  if (a.has_lut) {
+  if (a.slope_m) {
+    o = leaky_word(o, a.slope_m, a.slope_r);
+    if (a.lut_dst) *reinterpret_cast<uint32_t *>(a.lut_dst + off) = o;
+  } else if (a.has_lut) {
     const uint32_t r = (uint32_t)lut[o & 255u] | ((uint32_t)lut[(o >> 8) & 255u] << 8) | ((uint32_t)lut[(o >> 16) & 255u] << 16) |
                        ((uint32_t)lut[o >> 24] << 24);
     const int valid = a.oc - oc;   // channels of this dword that exist
@@ -3348,7 +3357,7 @@ __device__ __forceinline__ void unpack_args(const LeanArgs &l, ConvArgs *a) {
   a->lo = l.relu == 1 ? 0 : -128;
   a->relu_first = l.relu >> 1;
   a->store_y = 1;
-  a->has_lut = 0; a->lut_dst = nullptr; a->add_src = nullptr; a->add_dst = nullptr; a->split_oc = 0; a->y2 = nullptr;
+  a->has_lut = 0; a->slope_m = 0; a->lut_dst = nullptr; a->add_src = nullptr; a->add_dst = nullptr; a->split_oc = 0; a->y2 = nullptr;
 }
 
 template <int W, int TN, bool FAST, bool UNI>
@@ -3856,7 +3865,7 @@ void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
 
 // the short form of a K-split launch's arguments; false: something is fused, or a number does not fit
 bool lean_args(const ConvArgs &a, LeanArgs *out) {
-  if (a.has_lut || a.add_dst || a.split_oc || !a.store_y || !a.y) return false;
+  if (a.has_lut || a.slope_m || a.add_dst || a.split_oc || !a.store_y || !a.y) return false;
   auto u16 = [](int v) { return v >= 0 && v < 65536; };
   auto u8 = [](int v) { return v >= 0 && v < 256; };
   if (!u16(a.ih) || !u16(a.iw) || !u16(a.oh) || !u16(a.ow) || !u16(a.x_cs) || !u16(a.y_cs) || !u16(a.oc) || !u16(a.c16) ||
@@ -4388,11 +4397,42 @@ bool stem_pool_plan(const tpuhip_conv_weights *w, const tpuhip_pool_desc &p, int
   return true;
 }
 
-void apply_fusion(ConvArgs *a, const void *y, const PostOps &p) {
+// Whether a table is y -> max(y, (y * m + 2^(r - 1)) >> r) for some 0 < m <= 2^r whose products stay within 16 bits, and the
+// smallest such r.  The negative entries say how steep the line may be: (-k m + 2^(r-1)) >> r == t holds exactly where
+// m / 2^r is in ((-t - 1/2) / k, (1/2 - t) / k]; what comes out is held against the whole table.  0.1 us a call.
+bool slope_of_table(const int8_t *t, int *slope_m, int *slope_r) {
+  for (int y = 0; y < 128; ++y)
+    if (t[y] != y) return false;
+  double above = 0, upto = 1;
+  for (int k = 1; k <= 128; ++k) {
+    const double v = t[256 - k], inv = 1.0 / k;
+    above = std::max(above, (-v - 0.5) * inv);
+    upto = std::min(upto, (0.5 - v) * inv);
+  }
+  for (int r = 1; r <= 14 && above < upto + 1e-9; ++r) {
+    const int half = 1 << (r - 1);
+    for (int m = std::max(1, (int)(above * (1 << r)) - 1); m <= (int)(upto * (1 << r)) + 1 && m <= 1 << r && 128 * m + half < 32768; ++m) {
+      bool all = true;
+      for (int k = 1; k <= 128; ++k) all &= t[256 - k] == std::max(-k, (half - k * m) >> r);
+      if (all) {
+        *slope_m = m;
+        *slope_r = r;
+        return true;
+      }
+    }
+  }
+  return false;
+}
+
+// slope: the kernels of the launch can compute a leaky ReLU's table (all but the dot-product depthwise one).  A lookup takes
+// 16 instructions and four LDS reads per four outputs, the line 10 and none.
+void apply_fusion(ConvArgs *a, const void *y, const PostOps &p, bool slope = true) {
   if (p.lut) {
-    a->has_lut = 1;
     a->lut_dst = (int8_t *)p.lut_out;
-    memcpy(a->lut.w, p.lut, 256);
+    if (!slope || !slope_of_table(p.lut, &a->slope_m, &a->slope_r)) {
+      a->has_lut = 1;
+      memcpy(a->lut.w, p.lut, 256);
+    }
   }
   if (p.has_add()) {
     a->add_src = (const int8_t *)p.add_src;
@@ -4892,7 +4932,7 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
   }
   ConvArgs a;
   fill_args(ctx, w, x, y, &a);
-  apply_fusion(&a, y, post);
+  apply_fusion(&a, y, post, w->algo != ALGO_DEPTHWISE_DOT);
   if (w->algo == ALGO_MFMA) {
     launch_conv_mfma(ctx, w, a);
   } else if (w->algo == ALGO_DEPTHWISE) {
