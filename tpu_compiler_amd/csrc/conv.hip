@@ -66,6 +66,8 @@ struct tpuhip_conv_weights {
   QParam *qp = nullptr;
   int32_t *qplanes = nullptr;   // mult | rshift | hpot planes of nparam entries each
   int32_t *qc64 = nullptr;      // (low, high) pairs of bias * mult + 2^30, then the same + 2^(rshift-1) * 2^31
+  int32_t *qnarrow = nullptr;   // the two lists of pairs, multiplier, scale and unit planes of requant_rows_narrow; NULL: a channel
+                                // does not allow it
   int nparam = 0;
   int ocp = 0;           // padded output channels (rows of w / entries of bias, qp)
   int kp = 0;            // padded K in bytes (row stride of w) for the MFMA path
@@ -83,6 +85,7 @@ struct ConvArgs {
   // requantisation's 64-bit multiply-add; qc64r = qc64 + 2^(rshift-1) * 2^31, which also carries
   // the rounding term of the right shift (layers with a fused ReLU)
   const int32_t *qc64, *qc64r;
+  int narrow;      // qc64, qc64r, qmult, qshift, qhpot are the planes of requant_rows_narrow
   int8_t *y;
   int n, ih, iw, x_cs;
   int oh, ow, y_cs;
@@ -349,6 +352,22 @@ __device__ __forceinline__ void stage_rows(const v16i (&acc)[TM][TN], int relu_f
   }
 }
 
+template <int TM, int TN, int BM>
+__device__ __forceinline__ void stage_rows_narrow(const v16i (&acc)[TM][TN], bool relu, int8_t *stage, int row0, int col0,
+                                                  const int32_t *pc64, const int32_t *pmult, const int32_t *pscale,
+                                                  const int32_t *punit) {
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    uint32_t outw[TN][4];
+    if (relu) requant_rows_narrow<TN, true>(acc[i], pc64 + i * 32, pmult + i * 16, pscale + i * 16, punit + i * 16, outw);
+    else requant_rows_narrow<TN, false>(acc[i], pc64 + i * 32, pmult + i * 16, pscale + i * 16, punit + i * 16, outw);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      *reinterpret_cast<v4i *>(stage + (row0 + j * 32) * stage_row_bytes<BM>() + col0 + i * 16) =
+          v4i{(int)outw[j][0], (int)outw[j][1], (int)outw[j][2], (int)outw[j][3]};
+  }
+}
+
 // chunks of 16 bytes of a BM x BN tile handled per thread
 template <int BM, int BN, int NT>
 constexpr int flush_chunks() { return (BN * (BM / 16) + NT - 1) / NT; }
@@ -573,7 +592,9 @@ __global__ __launch_bounds__(256) void conv_depthwise_kernel(ConvArgs a) {
 // parameters of the channel tile sit in LDS, and the first K tiles of the next
 // pixel tile are fetched before the epilogue of the current one, so the global
 // latency at the head of a tile hides behind the VALU work at the tail of the last.
-template <int BM, int BN, int WM, int WN, int BK, int DEPTH, int OCC, bool PERSIST, bool FAST,
+// NARROW: the layer has the planes of requant_rows_narrow (a kernel of its own: with both forms in one the 64x64 tiles lost a
+// wave per SIMD to registers and 1 us a launch)
+template <int BM, int BN, int WM, int WN, int BK, int DEPTH, int OCC, bool PERSIST, bool FAST, bool NARROW,
           int MODE>
 __global__ __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1))) void
 conv_mfma_kernel(ConvArgs a) {
@@ -600,8 +621,9 @@ conv_mfma_kernel(ConvArgs a) {
   static_assert(DEPTH % 2 == 0 && DEPTH >= 2 && DEPTH <= 12, "register ring depth");
 
   __shared__ v4i lds[2][(BM + BN) * CH];
-  // bias | multiplier | rshift | 2^(rshift-1) of the workgroup's BM channels
-  __shared__ __attribute__((aligned(16))) int32_t qlds[PERSIST ? 4 * BM : 4];
+  // bias | multiplier | rshift | 2^(rshift-1) of the workgroup's BM channels, or the narrow form's (low, high) pairs |
+  // multiplier | scale | unit
+  __shared__ __attribute__((aligned(16))) int32_t qlds[PERSIST ? (NARROW ? 5 : 4) * BM : 4];
   __shared__ uint32_t lutw[64];   // fused table (published by the first barrier of the K loop)
 
   const int tid = threadIdx.x;
@@ -630,9 +652,11 @@ conv_mfma_kernel(ConvArgs a) {
   if (a.has_lut && tid < 64) lutv = a.lut.w[tid];
   const uint8_t *lut = a.has_lut ? reinterpret_cast<const uint8_t *>(lutw) : nullptr;
   static_assert(!PERSIST || BM <= NT, "one parameter row per thread");
-  int32_t qv[4] = {0, 0, 0, 0};
+  const int32_t *const c64 = NARROW ? out.lo == 0 ? a.qc64r : a.qc64 : nullptr;
+  int32_t qv[5] = {0, 0, 0, 0, 0};
   if (PERSIST && tid < BM) {
-    qv[0] = a.bias[oc0 + tid];
+    qv[0] = NARROW ? c64[2 * (oc0 + tid)] : a.bias[oc0 + tid];
+    if (NARROW) qv[4] = c64[2 * (oc0 + tid) + 1];
     qv[1] = a.qmult[oc0 + tid];
     qv[2] = a.qshift[oc0 + tid];
     qv[3] = a.qhpot[oc0 + tid];
@@ -834,10 +858,12 @@ conv_mfma_kernel(ConvArgs a) {
   if (a.has_lut && tid < 64) lutw[tid] = lutv;   // (published by the first barrier of the K loop at the latest)
   if (PERSIST) {
     if (tid < BM) {
-      qlds[tid] = qv[0];
-      qlds[BM + tid] = qv[1];
-      qlds[2 * BM + tid] = qv[2];
-      qlds[3 * BM + tid] = qv[3];
+      constexpr int planes = NARROW ? 2 * BM : BM;
+      qlds[NARROW ? 2 * tid : tid] = qv[0];
+      if (NARROW) qlds[2 * tid + 1] = qv[4];
+      qlds[planes + tid] = qv[1];
+      qlds[planes + BM + tid] = qv[2];
+      qlds[planes + 2 * BM + tid] = qv[3];
     }
     __syncthreads();   // publishes qlds
   }
@@ -845,7 +871,16 @@ conv_mfma_kernel(ConvArgs a) {
   // After the last barrier of a tile no wave reads LDS data it still needs, so the
   // first store of the next tile may overtake slower waves of the workgroup.
   for (;;) {
-    // accumulators start from the bias (the int32 add of the epilogue commutes with the sum)
+    // accumulators start from the bias (the int32 add of the epilogue commutes with the sum); the narrow form has it in
+    // its addend
+    if (NARROW) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = 0;
+    } else
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const v4i *bp = PERSIST ? reinterpret_cast<const v4i *>(qlds + lch0 + i * 16)
@@ -919,7 +954,14 @@ conv_mfma_kernel(ConvArgs a) {
     static_assert(BN * stage_row_bytes<BM>() <= (int)sizeof(lds), "the staged tile must fit the K tiles");
     v4i sv[flush_chunks<BM, BN, NT>()];
     flush_prefetch<BM, BN, NT>(a, tid, pix_done, a.npix, oc0, out, sv);
-    if (PERSIST)
+    if constexpr (NARROW) {
+      if (PERSIST)
+        stage_rows_narrow<TM, TN, BM>(acc, out.lo == 0, stage, wn * TN * 32 + frow, lch0, qlds + 2 * lch0, qlds + 2 * BM + lch0,
+                                      qlds + 3 * BM + lch0, qlds + 4 * BM + lch0);
+      else
+        stage_rows_narrow<TM, TN, BM>(acc, out.lo == 0, stage, wn * TN * 32 + frow, lch0, c64 + 2 * ocw0, a.qmult + ocw0,
+                                      a.qshift + ocw0, a.qhpot + ocw0);
+    } else if (PERSIST)
       stage_rows<TM, TN, BM, FAST>(acc, a.relu_first, out.lo, stage, wn * TN * 32 + frow, lch0,
                                    qlds + BM + lch0, qlds + 2 * BM + lch0, qlds + 3 * BM + lch0);
     else
@@ -1223,7 +1265,7 @@ conv_patch_kernel(ConvArgs a) {
 // some 130 clocks, a 32x32x32 MFMA 32 to 34
 constexpr int frag_prefetch(int mfmas_per_slice) { return mfmas_per_slice >= 8 ? 1 : mfmas_per_slice >= 4 ? 2 : 3; }
 
-template <int BM, int BN, int WM, int WN, int KP, int SD, int OCC>
+template <int BM, int BN, int WM, int WN, int KP, int SD, int OCC, bool NARROW>
 __global__ __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void
 conv_pw_kernel(ConvArgs a) {
   gather_conv_args(a);
@@ -1341,7 +1383,7 @@ conv_pw_kernel(ConvArgs a) {
       qlds[2 * tid] = c_lo;
       qlds[2 * tid + 1] = c_hi;
       qlds[2 * BM + tid] = qm;
-      qlds[3 * BM + tid] = qs - (out.lo == 0 ? 1 : 0);
+      qlds[3 * BM + tid] = qs - (out.lo == 0 && !NARROW ? 1 : 0);
       qlds[4 * BM + tid] = qh;
     }
 #pragma unroll
@@ -1422,12 +1464,8 @@ conv_pw_kernel(ConvArgs a) {
     for (int i = 0; i < TM; ++i) {
       uint32_t outw[TN][4];
       const int lc = lch0 + i * 16;
-      if (out.lo == 0)
-        requant_rows_c64<TN, true>(acc[i], 0, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc,
-                                   qlds + 4 * BM + lc, outw);
-      else
-        requant_rows_c64<TN, false>(acc[i], out.lo, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc,
-                                    qlds + 4 * BM + lc, outw);
+      requant_rows_planes<TN, NARROW>(acc[i], out.lo == 0, out.lo, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc,
+                              qlds + 4 * BM + lc, outw);
 #pragma unroll
       for (int j = 0; j < TN; ++j)
         *reinterpret_cast<v4i *>(stage + ((wn * TN + j) * 32 + frow) * SROW + lc) =
@@ -1470,7 +1508,7 @@ conv_pw_kernel(ConvArgs a) {
 // 2 * (C + 16) + kPatch2RowPad is a multiple of 128 for every C that is a multiple of 64
 constexpr int kPatch2RowPad = 96;
 
-template <int BM, int BN, int WM, int WN, int BK, int OCC>
+template <int BM, int BN, int WM, int WN, int BK, int OCC, bool NARROW>
 __global__ __launch_bounds__(WM *WN * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void
 conv_patch2_kernel(ConvArgs a) {
 #ifdef TPUHIP_TRACE
@@ -1620,7 +1658,7 @@ conv_patch2_kernel(ConvArgs a) {
     qlds[2 * tid] = qv[0];
     qlds[2 * tid + 1] = qv[1];
     qlds[2 * BM + tid] = qv[2];
-    qlds[3 * BM + tid] = qv[3] - (relu ? 1 : 0);
+    qlds[3 * BM + tid] = qv[3] - (relu && !NARROW ? 1 : 0);
     qlds[4 * BM + tid] = qv[4];
   }
   if (a.has_lut && tid < 64) lutw[tid] = lutv;
@@ -1725,11 +1763,8 @@ conv_patch2_kernel(ConvArgs a) {
   for (int i = 0; i < TM; ++i) {
     uint32_t outw[TN][4];
     const int lc = lch0 + i * 16;
-    if (relu)
-      requant_rows_c64<TN, true>(acc[i], 0, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc, qlds + 4 * BM + lc, outw);
-    else
-      requant_rows_c64<TN, false>(acc[i], a.lo, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc, qlds + 4 * BM + lc,
-                                  outw);
+    requant_rows_planes<TN, NARROW>(acc[i], relu, a.lo, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc,
+                            qlds + 4 * BM + lc, outw);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       *reinterpret_cast<v4i *>(stage + ((wn * TN + j) * 32 + frow) * stage_row_bytes<BM>() + lc) =
@@ -1778,7 +1813,7 @@ conv_patch2_kernel(ConvArgs a) {
 //   a.magic_kw = ceil(2^32 / H), a.magic_oh = ceil(2^32 / (H * W)), a.pstep_ow = LDS bytes
 // LDS (dynamic): parameters | table | patch, then the partial sums, then the staged tile.
 // ---------------------------------------------------------------------------
-template <int NB2, int PW, int OB>
+template <int NB2, int PW, int OB, bool NARROW>
 __global__ __launch_bounds__(256 * PW) void conv_patch3_kernel(ConvArgs a) {
 #ifdef TPUHIP_TRACE
   unsigned long long ts[32] = {};
@@ -1928,7 +1963,7 @@ __global__ __launch_bounds__(256 * PW) void conv_patch3_kernel(ConvArgs a) {
     qlds[2 * tid] = qv[0];
     qlds[2 * tid + 1] = qv[1];
     qlds[2 * BM + tid] = qv[2];
-    qlds[3 * BM + tid] = qv[3] - (relu ? 1 : 0);
+    qlds[3 * BM + tid] = qv[3] - (relu && !NARROW ? 1 : 0);
     qlds[4 * BM + tid] = qv[4];
   }
   if (a.has_lut && tid < 64) lutw[tid] = lutv;
@@ -2069,10 +2104,8 @@ __global__ __launch_bounds__(256 * PW) void conv_patch3_kernel(ConvArgs a) {
       if ((j & 3) == kg && j < nb) {
         const v16i one[1] = {acc[ob][j]};
         uint32_t outw[1][4];
-        if (relu)
-          requant_rows_c64<1, true>(one, 0, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc, qlds + 4 * BM + lc, outw);
-        else
-          requant_rows_c64<1, false>(one, a.lo, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc, qlds + 4 * BM + lc, outw);
+        requant_rows_planes<1, NARROW>(one, relu, a.lo, qlds + 2 * lc, qlds + 2 * BM + lc, qlds + 3 * BM + lc,
+                               qlds + 4 * BM + lc, outw);
         *reinterpret_cast<v4i *>(stage + ((pg * NB2 + j) * 32 + frow) * stage_row_bytes<BM>() + lc) =
             v4i{(int)outw[0][0], (int)outw[0][1], (int)outw[0][2], (int)outw[0][3]};
       }
@@ -2246,7 +2279,7 @@ struct DwRowsArgs {
   uint32_t magic_x, magic_r, magic_w;   // ceil(2^32 / d) of xblocks, rblocks, width: x / d == umulhi(x, magic), x, d < 2^16
 };
 
-template <bool SHIFT>
+template <bool SHIFT, bool NARROW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SHIFT ? 4 : 3, SHIFT ? 4 : 3))) void
 conv_depthwise_rows_kernel(ConvArgs a, DwRowsArgs r) {
   __shared__ uint32_t lutw[64];
@@ -2288,7 +2321,7 @@ conv_depthwise_rows_kernel(ConvArgs a, DwRowsArgs r) {
   {
     int32_t *q = qlds[wave];
     q[lane] = qv0;
-    q[64 + lane] = fk == 0 ? qv1 : qv2 - (relu ? 1 : 0);
+    q[64 + lane] = fk == 0 ? qv1 : qv2 - (relu && !NARROW ? 1 : 0);
     if (fk == 0) q[128 + lane] = qv3;
   }
   if (a.has_lut && threadIdx.x < 64) lutw[threadIdx.x] = lutv;
@@ -2400,8 +2433,7 @@ conv_depthwise_rows_kernel(ConvArgs a, DwRowsArgs r) {
     const bool more = b < b_end;
     if (more) request(bt);          // into the registers the MFMAs have just consumed
     uint32_t outw[1][4];
-    if (relu) requant_rows_c64<1, true>(acc, 0, pc64, pmult, pshift, phpot, outw);
-    else requant_rows_c64<1, false>(acc, a.lo, pc64, pmult, pshift, phpot, outw);
+    requant_rows_planes<1, NARROW>(acc, relu, a.lo, pc64, pmult, pshift, phpot, outw);
     if (st_ok) {
       const v4i o = {(int)outw[0][0], (int)outw[0][1], (int)outw[0][2], (int)outw[0][3]};
       finish_chunk(o, o, (int64_t)pix * out.y_cs + oc, oc, a, out.y, lut);
@@ -2645,7 +2677,7 @@ __global__ __launch_bounds__(512) void conv_stem_pool_kernel(ConvArgs a, StemPoo
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       pm[4 * q + e] = m4[e];
-      pr[4 * q + e] = r4[e] - 1;
+      pr[4 * q + e] = a.narrow ? r4[e] : r4[e] - 1;   // a right shift; at even e the narrow form's pair of scales
     }
   }
   v4i areg[7];
@@ -2716,17 +2748,22 @@ __global__ __launch_bounds__(512) void conv_stem_pool_kernel(ConvArgs a, StemPoo
         }
       }
       uint32_t outw[4];
+      auto requant = [&](auto narrow) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        int32_t y[4];
+        for (int q = 0; q < 4; ++q) {
+          int32_t y[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          // the ReLU form of requant_rows_c64: floor((acc * m + c) / 2^(31 + rshift)), clamped below
-          const int64_t prod = (int64_t)acc[4 * q + e] * (int64_t)pm[4 * q + e] + pc[4 * q + e];
-          y[e] = (int32_t)(prod >> 32) >> pr[4 * q + e];
+          for (int e = 0; e < 4; ++e) {
+            // the ReLU forms of requant_rows_narrow and requant_rows_c64: floor((acc * m + c) / 2^(31 + rshift)), clamped below
+            const int64_t prod = (int64_t)acc[4 * q + e] * (int64_t)pm[4 * q + e] + pc[4 * q + e];
+            y[e] = (int32_t)(prod >> 32);
+            if (!decltype(narrow)::value) y[e] >>= pr[4 * q + e];
+          }
+          outw[q] = decltype(narrow)::value ? pack_narrow_relu(y, pr[4 * q], pr[4 * q + 2]) : pack_sat4(y[0], y[1], y[2], y[3], 0);
         }
-        outw[q] = pack_sat4(y[0], y[1], y[2], y[3], 0);
-      }
+      };
+      if (a.narrow) requant(std::true_type());
+      else requant(std::false_type());
       if (pl < cpix) {
         uint2 *dst = reinterpret_cast<uint2 *>(ctile + p * kStemPoolCRow + lc);
         dst[0] = uint2{outw[0], outw[1]};
@@ -3738,7 +3775,7 @@ void launch_pw(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
   switch (tile) {
 #define W(i, name, BM, BN, WM, WN, KP, SD, O)                                                           \
   case i: {                                                                                             \
-    auto kernel = conv_pw_kernel<BM, BN, WM, WN, KP, SD, O>;                                            \
+    auto kernel = a.narrow ? conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, true> : conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, false>; \
     constexpr unsigned lds = pw_lds_bytes(BM, BN, KP, SD);                                              \
     if (!pw_prepare(kernel, lds)) break;                                                                \
     if (ctx->prof_start)                                                                                \
@@ -3752,14 +3789,15 @@ void launch_pw(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
 }
 
 // workgroups of pointwise tile variant `tile` that fit on one CU at once
+template <bool NARROW>
 int pw_occupancy(int tile) {
   int n = 0;
   hipError_t e = hipErrorInvalidValue;
   switch (tile) {
 #define W(i, name, BM, BN, WM, WN, KP, SD, O)                                                           \
   case i:                                                                                               \
-    if (pw_prepare(conv_pw_kernel<BM, BN, WM, WN, KP, SD, O>, pw_lds_bytes(BM, BN, KP, SD)))             \
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, conv_pw_kernel<BM, BN, WM, WN, KP, SD, O>, WM * WN * 64, \
+    if (pw_prepare(conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, NARROW>, pw_lds_bytes(BM, BN, KP, SD)))     \
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, NARROW>, WM * WN * 64, \
                                                        pw_lds_bytes(BM, BN, KP, SD));                   \
     break;
     TPUHIP_PW_TILES(W)
@@ -3797,7 +3835,7 @@ void launch_patch2(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
   switch (tile) {
 #define V(i, name, BM, BN, WM, WN, BK, O)                                                               \
   case i: {                                                                                             \
-    auto kernel = conv_patch2_kernel<BM, BN, WM, WN, BK, O>;                                            \
+    auto kernel = a.narrow ? conv_patch2_kernel<BM, BN, WM, WN, BK, O, true> : conv_patch2_kernel<BM, BN, WM, WN, BK, O, false>; \
     if (!pw_prepare(kernel, (unsigned)kLdsBytes)) break;                                                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(WM * WN * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
@@ -3851,7 +3889,7 @@ void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
   switch (tile) {
 #define U3(i, name, NB2, PW, OB)                                                                        \
   case i: {                                                                                             \
-    auto kernel = conv_patch3_kernel<NB2, PW, OB>;                                                      \
+    auto kernel = a.narrow ? conv_patch3_kernel<NB2, PW, OB, true> : conv_patch3_kernel<NB2, PW, OB, false>; \
     if (!pw_prepare(kernel, (unsigned)kLdsBytes)) break;                                                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(256 * PW), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
@@ -3912,13 +3950,18 @@ void launch_ksplit(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
   }
 }
 
-template <bool FAST, int MODE>
+// what a layer's constants allow: the general requantisation, the overflow-free one, and that with its last steps on packed int16
+constexpr int kGeneral = 0, kFast = 1, kNarrow = 2;
+int requant_form(const tpuhip_conv_weights *w) { return w->qnarrow ? kNarrow : w->fast ? kFast : kGeneral; }
+
+template <int FORM, int MODE>
 void launch_mfma(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
+  constexpr bool FAST = FORM != kGeneral;
   constexpr bool UNI = MODE == kModeUniform;
   switch (tile) {
 #define X(i, name, P, BM, BN, WM, WN, BK, D, O)                                             \
   case i:                                                                                   \
-    launch(ctx, (conv_mfma_kernel<BM, BN, WM, WN, BK, D, O, P, FAST, MODE>), grid,          \
+    launch(ctx, (conv_mfma_kernel<BM, BN, WM, WN, BK, D, O, P, FAST, FORM == kNarrow, MODE>), grid, \
            dim3(WM * WN * 64), a);                                                          \
     break;
     TPUHIP_LDS_TILES(X)
@@ -3935,7 +3978,7 @@ void launch_mfma(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
 }
 
 // workgroups of LDS tile variant `tile` that fit on one CU at once
-template <bool FAST, int MODE>
+template <int FORM, int MODE>
 int persist_occupancy(int tile) {
   int n = 0;
   hipError_t e = hipErrorInvalidValue;
@@ -3943,7 +3986,7 @@ int persist_occupancy(int tile) {
 #define X(i, name, P, BM, BN, WM, WN, BK, D, O)                                              \
   case i:                                                                                    \
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(                                        \
-        &n, conv_mfma_kernel<BM, BN, WM, WN, BK, D, O, P, FAST, MODE>, WM * WN * 64, 0);     \
+        &n, conv_mfma_kernel<BM, BN, WM, WN, BK, D, O, P, FORM != kGeneral, FORM == kNarrow, MODE>, WM * WN * 64, 0); \
     break;
     TPUHIP_LDS_TILES(X)
 #undef X
@@ -3961,21 +4004,24 @@ int conv_mode(const tpuhip_conv_weights *w) {
 int persist_wgs_per_cu(const tpuhip_conv_weights *w) {
   // 0 = not asked yet.  Contexts on several host threads may ask at once: every writer
   // stores the same value, so relaxed atomics are all that is needed.
-  static std::atomic<int> cache[kMaxTiles][2][3];
+  static std::atomic<int> cache[kMaxTiles][3][3];
   const int mode = kTiles[w->tile].reg == 5 ? 0 : conv_mode(w);
-  std::atomic<int> &slot = cache[w->tile][w->fast ? 1 : 0][mode];
+  const int form = requant_form(w);
+  std::atomic<int> &slot = cache[w->tile][form][mode];
   int c = slot.load(std::memory_order_relaxed);
   if (c == 0) {
+    auto ask = [&](auto f) {
+      constexpr int F = decltype(f)::value;
+      return mode == kModeSmallC     ? persist_occupancy<F, kModeSmallC>(w->tile)
+             : mode == kModeUniform ? persist_occupancy<F, kModeUniform>(w->tile)
+                                    : persist_occupancy<F, kModeGeneral>(w->tile);
+    };
     if (kTiles[w->tile].reg == 5)
-      c = pw_occupancy(w->tile);
-    else if (w->fast)
-      c = mode == kModeSmallC ? persist_occupancy<true, kModeSmallC>(w->tile)
-          : mode == kModeUniform ? persist_occupancy<true, kModeUniform>(w->tile)
-                                 : persist_occupancy<true, kModeGeneral>(w->tile);
+      c = form == kNarrow ? pw_occupancy<true>(w->tile) : pw_occupancy<false>(w->tile);
     else
-      c = mode == kModeSmallC ? persist_occupancy<false, kModeSmallC>(w->tile)
-          : mode == kModeUniform ? persist_occupancy<false, kModeUniform>(w->tile)
-                                 : persist_occupancy<false, kModeGeneral>(w->tile);
+      c = form == kNarrow ? ask(std::integral_constant<int, kNarrow>())
+          : form == kFast ? ask(std::integral_constant<int, kFast>())
+                          : ask(std::integral_constant<int, kGeneral>());
     slot.store(c, std::memory_order_relaxed);
   }
   return c;
@@ -4185,6 +4231,17 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t) {
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle
 }
 
+// the planes of requant_rows_narrow, for the kernels that know the form, where the layer has them
+void take_narrow(const tpuhip_conv_weights *w, ConvArgs *a) {
+  if (!w->qnarrow) return;
+  a->narrow = 1;
+  a->qc64 = w->qnarrow;
+  a->qc64r = w->qnarrow + 2 * w->nparam;
+  a->qmult = w->qnarrow + 4 * w->nparam;
+  a->qshift = a->qmult + w->nparam;
+  a->qhpot = a->qshift + w->nparam;
+}
+
 void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y,
                ConvArgs *out) {
   const tpuhip_conv_desc &d = w->d;
@@ -4198,6 +4255,8 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
   a.qhpot = w->qplanes + 2 * w->nparam;
   a.qc64 = w->qc64;
   a.qc64r = w->qc64 + 2 * w->nparam;
+  const int reg = w->algo == ALGO_MFMA ? kTiles[w->tile].reg : -1;
+  if (reg == 0 || reg == 3 || reg == 5 || reg == 6 || reg == 7) take_narrow(w, &a);
   a.y = (int8_t *)y;
   a.n = d.n; a.ih = d.ih; a.iw = d.iw; a.x_cs = d.x_cs;
   a.oh = d.oh; a.ow = d.ow; a.y_cs = d.y_cs;
@@ -4321,19 +4380,16 @@ void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvA
     else uni ? launch_ksplit<false, true>(ctx, w->tile, grid, a) : launch_ksplit<false, false>(ctx, w->tile, grid, a);
     return;
   }
-  if (w->smallc) {
-    if (w->fast)
-      launch_mfma<true, kModeSmallC>(ctx, w->tile, grid, a);
-    else
-      launch_mfma<false, kModeSmallC>(ctx, w->tile, grid, a);
-  } else if (w->fast && uni) {
-    launch_mfma<true, kModeUniform>(ctx, w->tile, grid, a);
-  } else if (w->fast) {
-    launch_mfma<true, kModeGeneral>(ctx, w->tile, grid, a);
-  } else if (uni) {
-    launch_mfma<false, kModeUniform>(ctx, w->tile, grid, a);
-  } else {
-    launch_mfma<false, kModeGeneral>(ctx, w->tile, grid, a);
+  auto go = [&](auto form) {
+    constexpr int F = decltype(form)::value;
+    if (w->smallc) launch_mfma<F, kModeSmallC>(ctx, w->tile, grid, a);
+    else if (uni) launch_mfma<F, kModeUniform>(ctx, w->tile, grid, a);
+    else launch_mfma<F, kModeGeneral>(ctx, w->tile, grid, a);
+  };
+  switch (requant_form(w)) {
+    case kNarrow: go(std::integral_constant<int, kNarrow>()); break;
+    case kFast: go(std::integral_constant<int, kFast>()); break;
+    default: go(std::integral_constant<int, kGeneral>());
   }
 }
 
@@ -4773,8 +4829,9 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   // one allocation and one upload: biases, records, the planes of the records' fields, and per channel the addend of the
   // requantisation's 64-bit multiply-add, (acc + bias) * mult + 2^30 == acc * mult + c, as (low, high) words
   cw->nparam = (int)nparam;
-  const size_t at_qp = nparam * 4, at_planes = at_qp + nparam * sizeof(QParam), at_c64 = at_planes + 3 * nparam * 4;
-  std::vector<int8_t> image(at_c64 + 4 * nparam * 4);
+  const size_t at_qp = nparam * 4, at_planes = at_qp + nparam * sizeof(QParam), at_c64 = at_planes + 3 * nparam * 4,
+               at_narrow = at_c64 + 4 * nparam * 4;
+  std::vector<int8_t> image(at_narrow + 7 * nparam * 4);
   memcpy(image.data(), b32.data(), nparam * 4);
   memcpy(image.data() + at_qp, qp.data(), nparam * sizeof(QParam));
   int32_t *planes = (int32_t *)(image.data() + at_planes), *c64 = (int32_t *)(image.data() + at_c64);
@@ -4789,6 +4846,22 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
     c64[2 * nparam + 2 * i] = (int32_t)(uint32_t)(cr & 0xffffffffll);
     c64[2 * nparam + 2 * i + 1] = (int32_t)(cr >> 32);
   }
+  // the same for requant_rows_narrow; pad channels stay zero
+  bool narrow = fast && !d.relu_first;
+  int32_t *nc = (int32_t *)(image.data() + at_narrow), *nplanes = nc + 4 * nparam;
+  for (int i = 0; i < d.oc && narrow; ++i) {
+    const int64_t c = (int64_t)b32[i] * (int64_t)qp[i].mult + (1ll << 30);
+    int32_t scale = 0;
+    for (int relu = 0; relu < 2 && narrow; ++relu) {
+      int64_t cn = 0;
+      narrow = narrow_requant(c + (relu ? (int64_t)qp[i].hpot << 31 : 0), qp[i].mult, qp[i].rshift, &cn, &nplanes[i], &scale,
+                              &nplanes[2 * nparam + i]);
+      nc[2 * (relu * nparam + i)] = (int32_t)(uint32_t)(cn & 0xffffffffll);
+      nc[2 * (relu * nparam + i) + 1] = (int32_t)(cn >> 32);
+    }
+    nplanes[nparam + (i & ~1)] |= scale << (16 * (i & 1));
+  }
+  if (!narrow) image.resize(at_narrow);
   if (!rc) rc = tpuhip_malloc(ctx, image.size(), (void **)&cw->params);
   if (!rc) rc = stage_upload(ctx, cw->params, image.data(), image.size());
   if (!rc) rc = prepack_done(ctx);
@@ -4800,6 +4873,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   cw->qp = (QParam *)(cw->params + at_qp);
   cw->qplanes = (int32_t *)(cw->params + at_planes);
   cw->qc64 = (int32_t *)(cw->params + at_c64);
+  if (narrow) cw->qnarrow = (int32_t *)(cw->params + at_narrow);
   *out = cw;
   return TPUHIP_OK;
 }
@@ -4946,9 +5020,11 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
       const unsigned wgs = 8 * (unsigned)std::max<int64_t>(
           (n_cb + 3) / 4, std::min<int64_t>(ceil_div64(waves_r, 32), std::max(1, ctx->num_cu * (dr.halo ? 4 : 3) / 8)));
       const bool shift = dr.halo == 1;
+      take_narrow(w, &a);
       dw_rows_walk(&dr, wgs, n_cb);
       a.magic_c16 = n_cb > 1 ? (uint32_t)(((1ull << 32) + n_cb - 1) / (uint64_t)n_cb) : 0u;   // wave index / n_cb
-      auto kernel = shift ? conv_depthwise_rows_kernel<true> : conv_depthwise_rows_kernel<false>;
+      auto kernel = a.narrow ? (shift ? conv_depthwise_rows_kernel<true, true> : conv_depthwise_rows_kernel<false, true>)
+                             : (shift ? conv_depthwise_rows_kernel<true, false> : conv_depthwise_rows_kernel<false, false>);
       if (ctx->prof_start)
         hipExtLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a, dr);
       else
@@ -4975,6 +5051,7 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
     TPUHIP_REQUIRE(!post.lut && !post.has_add() && post.pool_out && stem_pool_plan(w, *post.pool, ctx->num_cu, &sp, &lds),
                    "conv: this stem cannot take the max pool into its launch (tpuhip_conv2d_can_fuse_pool)");
     sp.py = (int8_t *)post.pool_out;
+    take_narrow(w, &a);
     a.magic_ow = (uint32_t)(((1ull << 32) + a.ow - 1) / (uint64_t)a.ow);
     TPUHIP_REQUIRE(pw_prepare(conv_stem_pool_kernel, 160u * 1024), "conv: raising the stem + pool kernel's LDS limit failed");
     const int per_cu = std::max(1, std::min(4, (int)(160u * 1024 / lds)));

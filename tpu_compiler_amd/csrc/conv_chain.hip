@@ -44,6 +44,7 @@ struct ChainArgs {
   int n_tiles, n_full;     // tiles in all; the first n_full hold BN pixels, the rest 32
   uint32_t x_bytes;
   int lo1, lo2;            // 0: the conv clamps at 0 (ReLU) and its planes hold the short form
+  int narrow1, narrow2;    // the planes are those of requant_rows_narrow
   int add_m_src, add_m_conv, add_rshift, add_relu, add_pk;
 #ifdef TPUHIP_TRACE
   unsigned long long *trace;   // development builds: 32 shader-clock stamps per wave
@@ -232,10 +233,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
           uint32_t outw[1][4];
           const int cb = wave * (32 * TM1) + fk * (16 * TM1) + i * 16;   // the lane's 16 channels of block i
           const v16i (&blk)[1] = reinterpret_cast<const v16i (&)[1]>(acc[i][j]);
-          if (a.lo1 == 0)
-            requant_rows_c64<1, true>(blk, 0, q1 + 2 * cb, q1 + 2 * OC1 + cb, q1 + 3 * OC1 + cb, q1 + 4 * OC1 + cb, outw);
-          else
-            requant_rows_c64<1, false>(blk, -128, q1 + 2 * cb, q1 + 2 * OC1 + cb, q1 + 3 * OC1 + cb, q1 + 4 * OC1 + cb, outw);
+          auto requant = [&](auto narrow) {
+            requant_rows_planes<1, decltype(narrow)::value>(blk, a.lo1 == 0, -128, q1 + 2 * cb, q1 + 2 * OC1 + cb,
+                                                            q1 + 3 * OC1 + cb, q1 + 4 * OC1 + cb, outw);
+          };
+          if (a.narrow1) requant(std::true_type());
+          else requant(std::false_type());
           *reinterpret_cast<v4i *>(stage + (j * 32 + frow) * SROW + cb) =
               v4i{(int)outw[0][0], (int)outw[0][1], (int)outw[0][2], (int)outw[0][3]};
         }
@@ -285,10 +288,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
                                                         *reinterpret_cast<const v4i *>(brow + ks * 32), acc2[0], 0, 0, 0);
       uint32_t outw[1][4];
       const int cb = ob * 32 + fk * 16;
-      if (a.lo2 == 0)
-        requant_rows_c64<1, true>(acc2, 0, q2 + 2 * cb, q2 + 2 * OC2 + cb, q2 + 3 * OC2 + cb, q2 + 4 * OC2 + cb, outw);
-      else
-        requant_rows_c64<1, false>(acc2, -128, q2 + 2 * cb, q2 + 2 * OC2 + cb, q2 + 3 * OC2 + cb, q2 + 4 * OC2 + cb, outw);
+      auto requant = [&](auto narrow) {
+        requant_rows_planes<1, decltype(narrow)::value>(acc2, a.lo2 == 0, -128, q2 + 2 * cb, q2 + 2 * OC2 + cb, q2 + 3 * OC2 + cb,
+                                                        q2 + 4 * OC2 + cb, outw);
+      };
+      if (a.narrow2) requant(std::true_type());
+      else requant(std::false_type());
       const v4u o2 = {outw[0][0], outw[0][1], outw[0][2], outw[0][3]};
       __builtin_amdgcn_raw_buffer_store_b128(o2, ybrsrc, (uint32_t)((pix0 + pb * 32 + frow) * OC2 + cb), 0, 0);
     }
@@ -399,6 +404,8 @@ int tpuhip_conv2d_chain_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *da, con
   ch->variant = v;
   ch->kp1 = c.kp1;
   ch->name = c.name;
+  ch->narrow1 = narrow_planes(da->oc, da->oc, mult_a, rshift_a, &p1);
+  ch->narrow2 = narrow_planes(db->oc, db->oc, mult_b, rshift_b, &p2);
   const std::vector<int8_t> f1 = mfma_a_fragments(filter_a, c.oc1, c.oc1 / 32, da->ic, c.kp1, c.oc1 / 8 / 32);
   const std::vector<int8_t> f2 = mfma_a_fragments(filter_b, c.oc2, c.oc2 / 32, db->ic, c.oc1, 1);
   int rc = upload_vec(ctx, f1, &ch->w1);
@@ -514,6 +521,8 @@ int tpuhip_conv2d_chain_i8(tpuhip_ctx *ctx, const tpuhip_conv_chain *ch, const v
   a.x_cs = da.x_cs;
   a.x_bytes = (uint32_t)((int64_t)a.npix * da.x_cs);
   a.lo1 = da.do_relu ? 0 : -128;
+  a.narrow1 = ch->narrow1;
+  a.narrow2 = ch->narrow2;
   a.lo2 = ch->db.do_relu ? 0 : -128;
 #ifdef TPUHIP_TRACE
   a.trace = getenv("TPUHIP_TRACE_PTR") ? (unsigned long long *)strtoull(getenv("TPUHIP_TRACE_PTR"), nullptr, 16) : nullptr;

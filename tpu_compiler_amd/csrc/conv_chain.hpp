@@ -21,6 +21,7 @@ struct tpuhip_conv_chain {
   int8_t *w1 = nullptr, *w2 = nullptr, *w3 = nullptr;
   uint32_t *w2d = nullptr;       // kind 3: the depthwise filter as one dword per lane and tap
   int32_t *q1 = nullptr, *q2 = nullptr, *q3 = nullptr;
+  int narrow1 = 0, narrow2 = 0;   // kind 1: q1, q2 hold the planes of requant_rows_narrow
   std::string name;
 };
 
@@ -55,6 +56,22 @@ inline bool requant_planes(int oc, int ocp, size_t per_oc, bool relu, const int8
     (*out)[3 * ocp + i] = rshift[i] - (relu ? 1 : 0);
     (*out)[4 * ocp + i] = (int32_t)hpot;
   }
+  return true;
+}
+
+// The planes of requant_planes() rewritten for requant_rows_narrow where every channel allows it; false: left as they are.
+inline bool narrow_planes(int oc, int ocp, const int32_t *mult, const int32_t *rshift, std::vector<int32_t> *planes) {
+  std::vector<int32_t> n((size_t)5 * ocp, 0);
+  for (int i = 0; i < ocp; ++i) {
+    const int64_t c = (int64_t)(((uint64_t)(uint32_t)(*planes)[2 * i + 1] << 32) | (uint32_t)(*planes)[2 * i]);
+    int64_t cn = 0;
+    int32_t scale = 0;
+    if (i < oc && !narrow_requant(c, mult[i], rshift[i], &cn, &n[2 * ocp + i], &scale, &n[4 * ocp + i])) return false;
+    n[2 * i] = (int32_t)(uint32_t)(cn & 0xffffffffll);
+    n[2 * i + 1] = (int32_t)(cn >> 32);
+    n[3 * ocp + (i & ~1)] |= scale << (16 * (i & 1));
+  }
+  planes->swap(n);
   return true;
 }
 
