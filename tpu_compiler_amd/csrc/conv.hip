@@ -264,6 +264,21 @@ __device__ __forceinline__ void requant_rows(const v16i (&acc)[TN], int relu_fir
   }
 }
 
+// table lookup per byte (index = the two's-complement byte); the 256-byte table covers each LDS bank once, so any 64 indices are
+// conflict-free.  Pad channels (from channel `channels` on) stay zero whatever table[0] is.
+__device__ __forceinline__ v4i lookup_chunk(v4i o, const uint8_t *lut, int channels) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t wd = (uint32_t)o[q];
+    const uint32_t r = (uint32_t)lut[wd & 255u] | ((uint32_t)lut[(wd >> 8) & 255u] << 8) |
+                       ((uint32_t)lut[(wd >> 16) & 255u] << 16) | ((uint32_t)lut[wd >> 24] << 24);
+    const int valid = channels - q * 4;   // channels of this dword that exist
+    const uint32_t mask = valid >= 4 ? 0xffffffffu : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u;
+    o[q] = (int)(r & mask);
+  }
+  return o;
+}
+
 // What happens to 16 requantised channels (first channel oc of the launch, byte offset off in
 // the tensor written): the store, the fused table, the fused add with its operand sv.
 __device__ __forceinline__ void finish_chunk(v4i o, const v4i &sv, int64_t off, int oc, const ConvArgs &a,
@@ -273,18 +288,7 @@ __device__ __forceinline__ void finish_chunk(v4i o, const v4i &sv, int64_t off, 
     o = leaky_chunk(o, a.slope_m, a.slope_r);
     if (a.lut_dst) *reinterpret_cast<v4i *>(a.lut_dst + off) = o;
   } else if (lut) {
-    // table lookup per byte (index = the two's-complement byte); the 256-byte table
-    // covers each LDS bank once, so any 64 indices are conflict-free.  Pad channels
-    // stay zero whatever table[0] is.
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t wd = (uint32_t)o[q];
-      const uint32_t r = (uint32_t)lut[wd & 255u] | ((uint32_t)lut[(wd >> 8) & 255u] << 8) |
-                         ((uint32_t)lut[(wd >> 16) & 255u] << 16) | ((uint32_t)lut[wd >> 24] << 24);
-      const int valid = a.oc - (oc + q * 4);   // channels of this dword that exist
-      const uint32_t mask = valid >= 4 ? 0xffffffffu : valid <= 0 ? 0u : (1u << (8 * valid)) - 1u;
-      o[q] = (int)(r & mask);
-    }
+    o = lookup_chunk(o, lut, a.oc - oc);
     if (a.lut_dst) *reinterpret_cast<v4i *>(a.lut_dst + off) = o;
   }
   if (a.add_dst)
@@ -2123,6 +2127,295 @@ __global__ __launch_bounds__(256 * PW) void conv_patch3_kernel(ConvArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// 3x3 / pad 1 convolutions of stride 1 or 2, fourth form of the row-patch kernel ("rows"), for layers of many pixels.  What the
+// second form spends its K loop on there is LDS and issue: it reads two fragments per MFMA or nearly so, writes every filter
+// tile into LDS besides, and meets a barrier and an LDS round trip per 128 or 256 bytes of K.  Here
+//   * WOC x WPX waves split the tile's channels and pixels; a wave owns OB blocks of 32 channels and NB blocks of 32 pixels:
+//     per 32-byte slice of K it takes OB filter fragments and NB pixel fragments for OB * NB MFMAs;
+//   * the filter never enters LDS: a fragment is 1 KB contiguous in the packed filter ([channel block][slice][lane][16 bytes], as
+//     in the third form), requested straight into registers U slices ahead, and the WPX waves that want the same one find it in
+//     the vector L1;
+//   * nothing synchronises between the patch's arrival and the staged epilogue, and what is not an MFMA stands between MFMAs
+//     (see slice(): in front of them it cost as long as they do; 128 -> 256 channels on 8 x 76 x 76: 18.8 -> 17.1 us).  G slices
+//     lie in one tap, so that addresses change once per group.
+// The patch is (rows - 1) * stride + 3 input rows, fetched as one byte stream (see conv_patch3_kernel).  With stride 2 a row's
+// even and odd positions lie apart (the first 'half' positions of an LDS row are the even ones), so that the lanes of a
+// fragment read consecutive positions whatever the tap.
+// Two kinds of tiles.  Large ones, one workgroup per CU (128 x 384: 5 rows of 76, 256 workgroups): of 31 000 clocks 6 000 are the
+// patch's way into LDS, 16 300 the K loop (its MFMAs: 14 900), 8 500 requantisation, leaky ReLU and stores.  Small ones of four
+// waves, three workgroups per CU, whose phases overlap: 64 -> 128 on 8 x 152 x 152 (with leaky ReLU and add) 24.2 us at three
+// waves per SIMD, 29.5 at two.
+// Against the fastest of the other forms, with leaky ReLU and add, 8 images: 32 -> 64 on 304 x 304 45.0 -> 38.2 us, 64 -> 128 on
+// 152 x 152 32.0 -> 24.2, 128 -> 256 on 76 x 76 25.4 -> 18.6, 256 -> 512 on 38 x 38 20.6 -> 16.5; stride 2, 128 -> 256 from
+// 152 x 152 24.6 -> 22.5; 64 -> 64 on 64 x 56 x 56 17.8 -> 13.3.  No faster: few pixels (one image below 200 x 200), and
+// stride 2 from maps whose three rows fill the LDS (608 x 32 channels).
+//   a.pstep_pix = rows of a tile, a.pstep_n = tiles per image (a.magic_oh its ceil(2^32 / d)), a.pstep_oh = log2(C),
+//   a.magic_c16 = ceil(2^32 / 16-byte chunks of an input row), a.magic_pw = bytes of a patch row, a.tile_imgs = half (stride 2),
+//   a.pstep_ow = LDS bytes.  C: a power of two from 32 * G to 1024.
+// LDS (dynamic): parameters | table | patch, then the staged tile.
+// ---------------------------------------------------------------------------
+template <int WOC, int WPX, int OB, int NB, int G, int U, int OCC>
+__global__ __launch_bounds__(WOC *WPX * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void conv_rows_kernel(ConvArgs a) {
+#ifdef TPUHIP_TRACE
+  unsigned long long ts[32] = {};
+#endif
+  TPUHIP_TS(0);
+  gather_conv_args(a);
+  gather_conv_args_more(a);
+  constexpr int NWAVES = WOC * WPX, NT = NWAVES * 64, BM = WOC * OB * 32, BN = WPX * NB * 32;
+  static_assert(U % 2 == 0 && U % G == 0 && U <= 9, "slices in flight: whole groups, no more than the shortest K holds");
+  constexpr int NPL = NWAVES == 8 ? 10 : 12;       // 1 KB pieces of the input span per wave and pass
+  static_assert(BM <= NT, "one parameter row per thread");
+  extern __shared__ __attribute__((aligned(16))) v4i rows_smem[];
+  int32_t *const qlds = reinterpret_cast<int32_t *>(rows_smem);               // 5 * BM dwords
+  uint32_t *const lutw = reinterpret_cast<uint32_t *>(qlds + 5 * BM);         // 64 dwords
+  int8_t *const patch = reinterpret_cast<int8_t *>(lutw + 64);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wo = wave / WPX, wp = wave % WPX;
+  const int logical = (int)(blockIdx.x & 7) * a.tiles_per_xcd + (int)(blockIdx.x >> 3);
+  if (logical >= a.n_tiles) return;
+  const int pt = pixel_tile_of(a, logical);
+  const int ocb = logical - pt * a.n_oc_tiles;
+  const int oc0 = ocb * BM;
+  const int img = a.pstep_n == 1 ? pt : (int)__umulhi((uint32_t)pt, a.magic_oh);
+  const int r0 = (pt - img * a.pstep_n) * a.pstep_pix;
+  const int rows = min(a.pstep_pix, a.oh - r0);
+  const int pix_base = (img * a.oh + r0) * a.ow;
+  const int npx = rows * a.ow;
+  const int pix_limit = pix_base + npx;
+  const int s = a.sh;
+  const int lgc = a.pstep_oh, C = 1 << lgc;
+  const int prow = C + 16, rowb = (int)a.magic_pw;  // bytes of a patch position and of a patch row
+  const bool relu = a.lo == 0;
+
+  const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
+  // requested first and parked last: loads return in order, and nothing waits for these alone
+  int32_t qv[5] = {0, 0, 0, 0, 0};
+  if (tid < BM) {
+    const int32_t *c64 = relu ? a.qc64r : a.qc64;
+    qv[0] = c64[2 * (oc0 + tid)];
+    qv[1] = c64[2 * (oc0 + tid) + 1];
+    qv[2] = a.qmult[oc0 + tid];
+    qv[3] = a.qshift[oc0 + tid];
+    qv[4] = a.qhpot[oc0 + tid];
+  }
+  uint32_t lutv = 0;
+  if (a.has_lut && tid < 64) lutv = a.lut.w[tid];
+
+  // ---- the filter: slice i of channel block b is the 1 KB fragment b * nsl + i.  (Requests past the last group of slices
+  // repeat it: never used.)
+  const int nsl = a.kp >> 5, trips = 9 << (lgc - 5);
+  uint32_t wlane[OB];
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob) {
+    wlane[ob] = (uint32_t)lane * 16u + (uint32_t)(ob * nsl) * 1024u;
+    asm volatile("" : "+v"(wlane[ob]));
+  }
+  int wslice = (ocb * WOC + wo) * OB * nsl * 1024;   // byte of the first slice of the group being requested
+  const int wlast = wslice + (trips - G) * 1024;
+  v4i af[U][OB];
+  auto load_A = [&](v4i &dst, int ob, int t) {        // slice t (< 4) of the group
+    dst = (v4i)__builtin_amdgcn_raw_buffer_load_b128(wrsrc, wlane[ob] + (uint32_t)t * 1024u, wslice, 0);
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int ob = 0; ob < OB; ++ob) load_A(af[u][ob], ob, u % G);
+    if (u % G == G - 1) wslice = min(wslice + G * 1024, wlast);
+  }
+
+  // ---- the patch
+  TPUHIP_TS(1);
+  {
+    const int cshift = lgc - 4, chunks_in = a.iw << cshift;
+    const int first = r0 * s - 1;                           // input row of patch row 0
+    const int row_f = max(first, 0), row_l = min((r0 + rows - 1) * s + 1, a.ih - 1);
+    const int span_chunks = (row_l - row_f + 1) * chunks_in, span_bytes = span_chunks << 4;
+    const int8_t *span = a.x + ((size_t)((img * a.ih + row_f) * a.iw) << lgc);
+    const int pieces = (span_bytes + 1023) >> 10;
+    uint32_t lane16 = (uint32_t)lane * 16u;
+    asm volatile("" : "+v"(lane16));
+    const int total_chunks = ((a.pstep_pix - 1) * s + 3) * rowb >> 4;
+    int piece0 = wave;
+    do {   // every wave makes the first pass: the barrier inside is the workgroup's
+      v4i preg[NPL];
+#pragma unroll
+      for (int u = 0; u < NPL; ++u) {
+        const int off = (piece0 + u * NWAVES) << 10;
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc((void *)(span + min(off, span_bytes)), 0, max(span_bytes - off, 0), 0x00020000);
+        preg[u] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rs, lane16, 0, 0);
+      }
+      if (piece0 == wave) {
+        for (int q = tid; q < total_chunks; q += NT) *reinterpret_cast<v4i *>(patch + q * 16) = v4i{0, 0, 0, 0};
+        __syncthreads();
+        TPUHIP_TS(2);
+      }
+#pragma unroll
+      for (int u = 0; u < NPL; ++u) {
+        const int c = ((piece0 + u * NWAVES) << 6) + lane;                 // chunk of the span
+        const int g = (int)__umulhi((uint32_t)c, a.magic_c16);            // its row in the span
+        const int p = c - g * chunks_in, at = (p >> cshift) + 1;          // position: the border is position 0
+        const int pos = s == 1 ? at : (at & 1) * a.tile_imgs + (at >> 1);
+        if (c < span_chunks && (s == 1 || at <= 2 * a.ow))
+          *reinterpret_cast<v4i *>(patch + (g + row_f - first) * rowb + pos * prow + (p & ((1 << cshift) - 1)) * 16) = preg[u];
+      }
+      piece0 += NWAVES * NPL;
+    } while (piece0 < pieces);
+  }
+  if (tid < BM) {
+    qlds[2 * tid] = qv[0];
+    qlds[2 * tid + 1] = qv[1];
+    qlds[2 * BM + tid] = qv[2];
+    qlds[3 * BM + tid] = qv[3];
+    qlds[4 * BM + tid] = qv[4];
+  }
+  if (a.has_lut && tid < 64) lutw[tid] = lutv;
+  const uint8_t *lut = a.has_lut ? reinterpret_cast<const uint8_t *>(lutw) : nullptr;
+
+  const int frow = lane & 31, fk = lane >> 5;
+  int bbase[NB];   // lane bases of the pixel fragments: slot -> its patch position
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int p = (wp * NB + j) * 32 + frow;
+    const int pr = a.ow == 1 ? p : (int)__umulhi((uint32_t)p, a.magic_ow);
+    bbase[j] = (p < npx ? pr * s * rowb + (p - pr * a.ow) * prow : 0) + fk * 16;   // idle slots read position 0
+  }
+  TPUHIP_TS(3);
+  __syncthreads();
+  TPUHIP_TS(4);
+
+  v16i acc[OB][NB];
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[ob][j][e] = 0;
+
+  // patch offsets of the taps of a filter row: 0, step1, step1 + step2
+  const int step1 = s == 1 ? prow : a.tile_imgs * prow, step2 = s == 1 ? prow : prow - a.tile_imgs * prow;
+  // a group of G slices lies in one tap: its patch offset, for one group after the other (past the last tap: the last one again)
+  int c0 = 0, tap = 0, tw = 0, tapoff = 0;
+  auto next_group = [&]() {
+    const int off = tapoff + c0;
+    c0 += 32 * G;
+    if (c0 == C) {
+      c0 = 0;
+      if (tap < 8) {
+        ++tap;
+        if (tw == 0) { tw = 1; tapoff += step1; }
+        else if (tw == 1) { tw = 2; tapoff += step2; }
+        else { tw = 0; tapoff += rowb - step1 - step2; }
+      }
+    }
+    return off;
+  };
+  // An MFMA occupies its pipe for 32 clocks in which the wave may issue what is independent of it: the reads of the next
+  // slice's pixel fragments, the request of a filter fragment and the arithmetic of the next group each stand behind an MFMA.
+  v4i bf[2][NB];
+  int addr[NB];
+  {
+    const int off = next_group();
+#pragma unroll
+    for (int j = 0; j < NB; ++j) addr[j] = bbase[j] + off;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) bf[0][j] = *reinterpret_cast<const v4i *>(patch + addr[j]);
+  }
+  auto slice = [&](auto uc, bool request) {
+    constexpr int u = decltype(uc)::value, t = u % G;
+    int off = 0;
+    if (t == G - 1) off = next_group();
+#pragma unroll
+    for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        acc[ob][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[u][ob], bf[u & 1][j], acc[ob][j], 0, 0, 0);
+        if (ob == 0) {
+          if (t == G - 1) addr[j] = bbase[j] + off;
+          bf[(u + 1) & 1][j] = *reinterpret_cast<const v4i *>(patch + addr[j] + (t == G - 1 ? 0 : (t + 1) * 32));
+        }
+        if (request && j == NB - 1) load_A(af[u][ob], ob, t);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    if (request && t == G - 1) wslice = min(wslice + G * 1024, wlast);
+  };
+  int i0 = 0;
+  for (; i0 + U <= trips; i0 += U) static_for<U>([&](auto uc) { slice(uc, true); });
+  static_for<U - 1>([&](auto uc) {
+    if (i0 + decltype(uc)::value < trips) slice(uc, false);
+  });
+
+  TPUHIP_TS(5);
+  // ---- requantisation into the staged tile (the patch's space), then out in memory order through buffer descriptors: 32-bit
+  // offsets, pixels past the tile's last are dropped by the range check, lanes past the last channel group stay out of range
+  constexpr int CPR = BM / 16, NU = BN * CPR / NT;
+  static_assert(NT % CPR == 0 && NU * NT == BN * CPR, "whole passes of the workgroup");
+  const int row0 = tid / CPR, cc = tid % CPR;
+  const int64_t base = (int64_t)pix_base * a.y_cs + oc0;
+  const uint32_t bytes = (uint32_t)(npx * a.y_cs - oc0), vo = oc0 + cc * 16 < a.ocw ? (uint32_t)(row0 * a.y_cs + cc * 16) : kOobOffset;
+  const uint32_t vstep = (uint32_t)(NT / CPR * a.y_cs);
+  const __amdgpu_buffer_rsrc_t srsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(a.add_src + base), 0, a.add_dst ? bytes : 0, 0x00020000);
+  v4i sv[NU];
+  if (a.add_dst) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) sv[u] = buffer_load16(srsrc, vo + u * vstep);
+  }
+  __syncthreads();   // every wave is done with the patch
+  TPUHIP_TS(6);
+  int8_t *const stage = patch;
+#pragma unroll
+  for (int ob = 0; ob < OB; ++ob) {
+    uint32_t outw[NB][4];
+    const int lc = wo * OB * 32 + fk * 16 * OB + ob * 16;
+    const int32_t *const q = qlds + lc;
+    requant_rows_planes<NB, true>(acc[ob], relu, a.lo, q + lc, q + 2 * BM, q + 3 * BM, q + 4 * BM, outw);
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      *reinterpret_cast<v4i *>(stage + ((wp * NB + j) * 32 + frow) * stage_row_bytes<BM>() + lc) =
+          v4i{(int)outw[j][0], (int)outw[j][1], (int)outw[j][2], (int)outw[j][3]};
+  }
+  TPUHIP_TS(7);
+  __syncthreads();
+  TPUHIP_TS(8);
+  const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.y + base), 0, a.store_y ? bytes : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t trsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(a.lut_dst + base), 0, a.lut_dst ? bytes : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t zrsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(a.add_dst + base), 0, a.add_dst ? bytes : 0, 0x00020000);
+  const int8_t *const from = stage + row0 * stage_row_bytes<BM>() + cc * 16;
+  v4i o[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) o[u] = *reinterpret_cast<const v4i *>(from + u * (NT / CPR) * stage_row_bytes<BM>());
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    if (a.store_y) __builtin_amdgcn_raw_buffer_store_b128((v4u)o[u], yrsrc, vo + u * vstep, 0, 0);
+    if (a.slope_m) {
+      o[u] = leaky_chunk(o[u], a.slope_m, a.slope_r);
+    } else if (lut) {
+      o[u] = lookup_chunk(o[u], lut, a.oc - (oc0 + cc * 16));
+    }
+    if (a.lut_dst) __builtin_amdgcn_raw_buffer_store_b128((v4u)o[u], trsrc, vo + u * vstep, 0, 0);
+    if (a.add_dst) {
+      const v4i z = fused_add_chunk(o[u], sv[u], a.add_m_src, a.add_m_conv, a.add_rshift, a.add_relu, a.add_pk);
+      __builtin_amdgcn_raw_buffer_store_b128((v4u)z, zrsrc, vo + u * vstep, 0, 0);
+    }
+  }
+  TPUHIP_TS(9);
+#ifdef TPUHIP_TRACE
+  asm volatile("s_waitcnt vmcnt(0)");
+  TPUHIP_TS(10);
+  if (a.trace && (tid & 63) == 0) {
+    for (int k = 0; k < 32; ++k) a.trace[((size_t)blockIdx.x * 8 + (tid >> 6)) * 32 + k] = ts[k];
+  }
+#endif
+}
+
+// ---------------------------------------------------------------------------
 // depthwise on the matrix cores.  A depthwise tap is a 32x32 DIAGONAL matrix times
 // the 32 channels x 32 pixels activation block: D[c][pix] += W_t[c][c] * X_t[pix][c],
 // one v_mfma_i32_32x32x32_i8 per tap (K = the 32 channels).  31/32 of the multiplies
@@ -3587,8 +3880,9 @@ struct TileCfg {
   int reg;   // 0: LDS kernel, one tile per workgroup; 1: the LDS-free kernel, bm x bn is the
              // tile of one wave; 2: its split-K form; 3: LDS kernel, persistent workgroups;
              // 4: patch kernel (bn = pixel slots of a tile of whole rows); 5: pointwise kernel;
-             // 6: patch kernel, second form; 7: patch kernel, third form; 8: K split over all waves
+             // 6: patch kernel, second form; 7: patch kernel, third form; 8: K split over all waves; 9: patch kernel, fourth form
   int bk;    // K bytes per step (pointwise kernel: the padded K it holds)
+  int cmod;  // fourth form of the patch kernel: the input channels are a multiple of this
 };
 
 // The tile variants, in the order of their public index (conv desc algo = 16 + index).
@@ -3679,8 +3973,28 @@ struct TileCfg {
   KS(62, "mfma_ksplit_32x64_w8", 8, 2)    \
   KS(63, "mfma_ksplit_32x32_w4", 4, 1)
 
+// row-patch kernels, fourth form (3x3 / stride 1 or 2 / pad 1, input channels a power of two from 128, 64 or 32 to 1024):
+// U4(index, name, waves along channels, along pixels, channel blocks and pixel blocks per wave, slices per group, slices in
+// flight, waves per SIMD).  Indices 64 to 71 are not used: the variants below them, without a gap from 0, are those that take
+// any dense conv or are one of the families before this one.  Each is the fastest of all at several of 190 shapes (stages of
+// a detector of 320 to 608 pixels, 1 to 8 images, and of a residual classifier, 8 to 64 images); variants that came within 2 %
+// of another everywhere were left out.
+#define TPUHIP_ROWS_TILES(U4)                         \
+  U4(72, "mfma_rows_256x256", 4, 2, 2, 4, 4, 4, 2)    \
+  U4(73, "mfma_rows_256x160", 8, 1, 1, 5, 4, 8, 2)    \
+  U4(74, "mfma_rows_128x384", 4, 2, 1, 6, 4, 8, 2)    \
+  U4(75, "mfma_rows_128x192", 4, 2, 1, 3, 4, 4, 4)    \
+  U4(76, "mfma_rows_128x160", 4, 1, 1, 5, 4, 4, 3)    \
+  U4(77, "mfma_rows_128x128", 4, 1, 1, 4, 4, 8, 3)    \
+  U4(78, "mfma_rows_64x192", 2, 2, 1, 3, 4, 8, 4)     \
+  U4(79, "mfma_rows_128x160_c64", 4, 1, 1, 5, 2, 4, 3)\
+  U4(80, "mfma_rows_128x128_c64", 4, 1, 1, 4, 2, 4, 4)\
+  U4(81, "mfma_rows_64x320_c32", 2, 2, 1, 5, 1, 4, 3) \
+  U4(82, "mfma_rows_64x256_c32", 2, 2, 1, 4, 1, 4, 4) 
+
+constexpr int kMaxTiles = 96;
 struct TileTable {
-  TileCfg t[64];
+  TileCfg t[kMaxTiles] = {};   // name NULL: no such variant
   int n = 0;
   TileTable() {
 #define X(i, name, P, BM, BN, WM, WN, BK, D, O) \
@@ -3718,12 +4032,16 @@ struct TileTable {
   n = n > i ? n : i + 1;
     TPUHIP_KSPLIT_TILES(KS)
 #undef KS
+#define U4(i, name, WOC, WPX, OB, NB, G, U, O) \
+  t[i] = TileCfg{WOC * OB * 32, WPX * NB * 32, WOC, WPX, name, 9, 64, 32 * G}; \
+  n = n > i ? n : i + 1;
+    TPUHIP_ROWS_TILES(U4)
+#undef U4
   }
 };
 const TileTable kTileTable;
 const TileCfg *const kTiles = kTileTable.t;
 inline int tile_bk(const TileCfg &t) { return t.bk; }
-constexpr int kMaxTiles = 64;
 #define kNumTiles (kTileTable.n)
 
 template <bool SPLIT, int TM, int TN, int D, int O, bool FAST, bool UNI>
@@ -3883,6 +4201,56 @@ Patch3Plan patch3_plan(const tpuhip_conv_desc &d, const TileCfg &c) {
   }
   pl.lds = (unsigned)lds_bytes(pl.th, pl.imgs);
   return pl;
+}
+
+// ---- row-patch kernels, fourth form
+struct RowsPlan {
+  int th = 0;        // rows of a tile (0: the layer does not fit this kernel)
+  int half = 0;      // stride 2: positions of an LDS row before the odd ones
+  int rowb = 0;      // bytes of an LDS row
+  unsigned lds = 0;
+};
+
+RowsPlan rows_plan(const tpuhip_conv_desc &d, const TileCfg &c) {
+  RowsPlan pl;
+  const int s = d.sh;
+  const bool shape_ok = d.g == 1 && d.kh == 3 && d.kw == 3 && (s == 1 || s == 2) && d.sw == s && d.dh == 1 && d.dw == 1 && d.pt == 1 &&
+                        d.pl == 1 && !d.ins_h && !d.ins_w && !d.relu_first && d.oh == (d.ih + s - 1) / s && d.ow == (d.iw + s - 1) / s &&
+                        d.x_cs == d.ic && d.ic >= 32 && d.ic <= 1024 && (d.ic & (d.ic - 1)) == 0 && d.ic % c.cmod == 0;
+  if (!shape_ok || d.ow > c.bn) return pl;
+  const int prow = d.ic + 16;
+  pl.half = s == 2 ? d.ow + 1 : 0;
+  // positions 0 .. ow + 1, or 0 .. 2 ow as two halves; the pitch makes a wrap from one image row into the next look like
+  // consecutive positions to the banks (stride 1; see kPatch2RowPad)
+  pl.rowb = s == 1 ? (d.ow + 2) * prow + (128 - 2 * prow % 128) % 128 : 2 * pl.half * prow;
+  auto bytes = [&](int th) {
+    return (int64_t)(5 * c.bm * 4 + 256) + std::max<int64_t>((int64_t)((th - 1) * s + 3) * pl.rowb, (int64_t)c.bn * (c.bm + 16));
+  };
+  int th = std::min(c.bn / d.ow, d.oh);
+  // (span chunks are divided by a multiply that is exact below 2^16 of them)
+  while (th >= 1 && (bytes(th) > kLdsBytes || ((th - 1) * s + 3) * (int64_t)d.iw * (d.ic / 16) > 60000)) --th;
+  if (th < 1) return pl;
+  const int tiles = (d.oh + th - 1) / th;      // evened out over the image
+  if ((int64_t)d.n * tiles * tiles >= (1ll << 32)) return pl;
+  pl.th = (d.oh + tiles - 1) / tiles;
+  pl.lds = (unsigned)bytes(pl.th);
+  return pl;
+}
+
+void launch_rows(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsigned lds) {
+  switch (tile) {
+#define U4(i, name, WOC, WPX, OB, NB, G, U, O)                                                                \
+  case i: {                                                                                             \
+    auto kernel = conv_rows_kernel<WOC, WPX, OB, NB, G, U, O>;                                                \
+    if (!pw_prepare(kernel, (unsigned)kLdsBytes)) break;                                                \
+    if (ctx->prof_start)                                                                                \
+      hipExtLaunchKernelGGL(kernel, grid, dim3(WOC * WPX * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
+    else                                                                                                \
+      hipLaunchKernelGGL(kernel, grid, dim3(WOC * WPX * 64), lds, ctx->stream, a);                      \
+  } break;
+    TPUHIP_ROWS_TILES(U4)
+#undef U4
+  }
 }
 
 void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsigned lds) {
@@ -4190,7 +4558,7 @@ void settle_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *cw) {
 // the fused table lives in the LDS of the LDS kernels
 bool tile_has_lds_epilogue(int t) {
   return kTiles[t].reg == 0 || kTiles[t].reg == 3 || kTiles[t].reg == 5 || kTiles[t].reg == 6 || kTiles[t].reg == 7 ||
-         kTiles[t].reg == 8;
+         kTiles[t].reg == 8 || kTiles[t].reg == 9;
 }
 
 // the pointwise kernels: 1x1 window, no padding, no dilation (any stride), the input channels
@@ -4218,6 +4586,8 @@ int patch_rows(const tpuhip_conv_desc &d, const TileCfg &c) {
 
 bool tile_is_candidate(const tpuhip_conv_desc &d, int t) {
   const TileCfg &c = kTiles[t];
+  if (!c.name) return false;
+  if (c.reg == 9 && rows_plan(d, c).th == 0) return false;
   if (c.reg == 4 && patch_rows(d, c) == 0) return false;
   if (c.reg == 5 && !pw_shape_ok(d, c)) return false;
   if (c.reg == 6 && patch2_rows(d, c) == 0) return false;
@@ -4256,7 +4626,7 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
   a.qc64 = w->qc64;
   a.qc64r = w->qc64 + 2 * w->nparam;
   const int reg = w->algo == ALGO_MFMA ? kTiles[w->tile].reg : -1;
-  if (reg == 0 || reg == 3 || reg == 5 || reg == 6 || reg == 7) take_narrow(w, &a);
+  if (reg == 0 || reg == 3 || reg == 5 || reg == 6 || reg == 7 || reg == 9) take_narrow(w, &a);
   a.y = (int8_t *)y;
   a.n = d.n; a.ih = d.ih; a.iw = d.iw; a.x_cs = d.x_cs;
   a.oh = d.oh; a.ow = d.ow; a.y_cs = d.y_cs;
@@ -4322,6 +4692,25 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
         a.pstep_ow = (int)patch2_lds_bytes(t, th, d.ow, d.ic);                   // dynamic LDS of the launch
       }
     }
+    if (t.reg == 9) {
+      const RowsPlan pl = rows_plan(d, t);
+      const int tiles_per_img = (d.oh + pl.th - 1) / pl.th;
+      const int n_pix_tiles = d.n * tiles_per_img;
+      a.n_tiles = n_pix_tiles * a.n_oc_tiles;
+      a.tiles_per_xcd = (n_pix_tiles + 7) / 8 * a.n_oc_tiles;
+      a.wgs_per_xcd = a.tiles_per_xcd;
+      a.pstep_pix = pl.th;
+      a.pstep_n = tiles_per_img;
+      a.magic_oh = (uint32_t)(((1ull << 32) + tiles_per_img - 1) / (uint64_t)tiles_per_img);
+      a.tile_imgs = pl.half;
+      int lgc = 5;
+      while ((1 << lgc) < d.ic) ++lgc;
+      a.pstep_oh = lgc;                                                          // log2(C)
+      const uint32_t rowchunks = (uint32_t)d.iw * (uint32_t)(d.ic / 16);
+      a.magic_c16 = (uint32_t)(((1ull << 32) + rowchunks - 1) / rowchunks);      // q / rowchunks == umulhi(q, magic), q < 2^16
+      a.magic_pw = (uint32_t)pl.rowb;
+      a.pstep_ow = (int)pl.lds;                                                  // dynamic LDS of the launch
+    }
     if (t.reg == 7) {
       const Patch3Plan pl = patch3_plan(d, t);
       const int tiles_per_img = (d.oh + pl.th - 1) / pl.th;
@@ -4372,6 +4761,10 @@ void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvA
   }
   if (kTiles[w->tile].reg == 7) {
     launch_patch3(ctx, w->tile, grid, a, (unsigned)a.pstep_ow);
+    return;
+  }
+  if (kTiles[w->tile].reg == 9) {
+    launch_rows(ctx, w->tile, grid, a, (unsigned)a.pstep_ow);
     return;
   }
   const bool uni = (w->c16 % (tile_bk(kTiles[w->tile]) / 16)) == 0;
@@ -4525,6 +4918,7 @@ bool tile_usable(const tpuhip_conv_weights *w, int t, const PostOps &post) {
   if (post.lut && !tile_has_lds_epilogue(t)) return false;
   if (w->split_oc && kTiles[t].reg == 4) return false;   // the patch kernel writes one result
   if (kTiles[t].reg == 5 && (!w->fast || w->split_oc % kTiles[t].bm)) return false;
+  if (kTiles[t].reg == 9 && (!w->qnarrow || w->split_oc)) return false;
   return !((kTiles[t].reg == 6 || kTiles[t].reg == 7) && (!w->fast || w->split_oc));
 }
 
@@ -4679,7 +5073,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   if (algo >= 16) {   // MFMA with an explicit tile variant (tests, tuning)
     forced_tile = algo - 16;
     algo = ALGO_MFMA;
-    TPUHIP_REQUIRE(forced_tile < kNumTiles, "conv: unknown MFMA tile %d", forced_tile);
+    TPUHIP_REQUIRE(forced_tile < kNumTiles && kTiles[forced_tile].name, "conv: unknown MFMA tile %d", forced_tile);
   }
   // the stem kernel: one dword per pixel, the taps of a filter row side by side
   const bool stem_ok = dense && d.ic <= 4 && d.dh == 1 && d.dw == 1 && d.kw <= 8 && d.kh <= 7 &&
@@ -4993,6 +5387,11 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
                  "conv: tile variant %s needs a single 3x3 / stride 1 / pad 1 conv with 64, 128, 256, 512 or 1024 input "
                  "channels on a map narrow enough for its row patch, right shifts of at least 1 and sums that cannot "
                  "overflow the rounding", kTiles[w->tile].name);
+  TPUHIP_REQUIRE(!(w->algo == ALGO_MFMA && kTiles[w->tile].reg == 9) ||
+                     (!w->split_oc && w->qnarrow && rows_plan(w->d, kTiles[w->tile]).th > 0),
+                 "conv: tile variant %s needs a single 3x3 / pad 1 conv of stride 1 or 2 with 32 to 1024 input channels (a power of "
+                 "two) on a map narrow enough for its row patch, and constants that requantise on packed int16",
+                 kTiles[w->tile].name);
   TPUHIP_REQUIRE(!(w->algo == ALGO_MFMA && kTiles[w->tile].reg == 6) ||
                      (!w->split_oc && w->fast && patch2_rows(w->d, kTiles[w->tile]) > 0),
                  "conv: tile variant %s needs a single 3x3 / stride 1 / pad 1 conv with 64, 128, 256, 512 or 1024 input "
@@ -5365,7 +5764,7 @@ int tpuhip_fc_prepack(tpuhip_ctx *ctx, int m, int k, int n, int x_cs, int y_cs, 
   // (and so is a K beyond the conv kernels' reach, whatever the rows)
   if ((m <= 256 && (n + 31) / 32 * ((m + 31) / 32) <= kFcMaxTiles) || k > 4096) {
     for (int t = 0; t < kNumTiles; ++t)
-      if (std::string(kTiles[t].name) == "mfma_reg_32x32") d.algo = 16 + t;
+      if (kTiles[t].name && std::string(kTiles[t].name) == "mfma_reg_32x32") d.algo = 16 + t;
   }
   std::vector<int32_t> mult((size_t)n, multiplier), rs((size_t)n, rshift);
   return tpuhip_conv2d_prepack(ctx, &d, filter_nk, bias, mult.data(), rs.data(), out);
