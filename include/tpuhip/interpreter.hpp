@@ -327,6 +327,7 @@ private:
   SyncedData pool_dst;
   tpuhip_pool_desc pool_desc{};
   int8_t lut_table[256];
+  int lut_slope_m = 0, lut_slope_r = 0;    // the table as a leaky ReLU's line, 0: it is none
   bool store_lut = true;
   bool plain = false;                      // an ordinary dense conv (not transposed)
   std::vector<int8_t> host_w;

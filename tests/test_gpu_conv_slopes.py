@@ -66,3 +66,34 @@ def test_conv_with_a_line_behind_it(ctx, form, table):
     ctx.conv_weights_destroy(wh)
     for v in (xt, yt, tt):
         v.free()
+
+
+def test_a_module_finds_lines_of_more_bits():
+    """a leaky ReLU of multiplier 102, right shift 10, which no line of 7 bits equals, fused behind a conv of a loaded network"""
+    import oracle_graph
+    from tpu_compiler_amd import graphs, module
+    rng = np.random.default_rng(2)
+    one = lambda v: np.array([v], np.float32)
+    g = graphs.Graph("line", 1)
+    g.add(graphs.Op("tpu.input", "x", [], (1, 64, 40, 41)))
+    w = np.clip(np.rint(rng.normal(0, 32, (72, 64, 3, 3))), -127, 127).astype(np.float32)
+    attrs = dict(kernel_h=3, kernel_w=3, stride_h=1, stride_w=1, dilation_h=1, dilation_w=1, padding_t=1, padding_b=1, padding_l=1,
+                 padding_r=1, group=1, is_dw=0, with_bias=1, do_relu=0, pad_value=0)
+    g.add(graphs.Op("tpu.conv_2d", "conv", ["x"], (1, 72, 40, 41), attrs,
+                    dict(filter=w, bias=rng.integers(-4096, 4097, 72).astype(np.float32), rshift=np.full(72, 9, np.float32),
+                         multiplier=(rng.integers(1 << 23, 1 << 24, 72) * 128.0).astype(np.float32)), "RSHIFT_AND_M_I32"))
+    g.add(graphs.Op("tpu.leaky_relu", "leaky", ["conv"], (1, 72, 40, 41), dict(negative_slope=0.1),
+                    dict(rshift_pos=one(0), multiplier_pos=one(1), rshift_neg=one(10), multiplier_neg=one(102)), "RSHIFT_AND_M_I8"))
+    g.outputs = ["leaky"]
+    x = rng.integers(-128, 128, (1, 64, 40, 41)).astype(np.int8)
+    want = oracle_graph.run(g, input_data=x)
+    for keep in (1, 0):
+        m = module()
+        m.set_option("keep_all_tensors", keep)
+        m.load(g)
+        for _ in range(2):
+            m.set_tensor_i8("x", x)
+            m.invoke()
+            assert np.array_equal(m.get_tensor_i8("leaky"), want["leaky"])
+            assert not keep or np.array_equal(m.get_tensor_i8("conv"), want["conv"])
+        m.close()

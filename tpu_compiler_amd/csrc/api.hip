@@ -193,7 +193,7 @@ int tpuhip_free(tpuhip_ctx *ctx, void *dptr) {
   TPUHIP_REQUIRE(ctx, "tpuhip_free: NULL context");
   if (!dptr) return TPUHIP_OK;
   TPUHIP_CHECK_HIP(hipSetDevice(ctx->device));
-  if (!ctx->staged.empty() || !ctx->packs.empty())   // one of them may be for this memory
+  if (!ctx->staged.empty() || !ctx->packs.empty() || !ctx->params.empty())   // one of them may be for this memory
     if (int rc = flush_uploads(ctx)) return rc;
   TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   if (slab_free(ctx, dptr)) return TPUHIP_OK;

@@ -31,6 +31,14 @@ struct StagedCopy {
   uint32_t *dst;
   size_t dwords;
 };
+
+// A layer's requantisation parameters, made from the three numbers of each channel (conv.hip)
+struct ParamExpand {
+  const int32_t *raw;    // biases, multipliers, right shifts of oc channels
+  int32_t *out;          // nparam biases, then [records], planes, [addends or the narrow form's planes]
+  int oc, nparam;
+  int records, narrow;
+};
 }  // namespace tpuhip
 
 struct tpuhip_ctx {
@@ -63,10 +71,11 @@ struct tpuhip_ctx {
   std::vector<Slab> slabs;
   std::unordered_map<void *, std::pair<char *, size_t>> slab_parts;   // allocation -> its slab's base, its bytes
   // a module is being loaded: packed weights need not be on the device when a prepack call returns, and what is to be
-  // uploaded and packed for them gathers here until flush_uploads() (host_io.cpp) issues all of it in two launches
+  // uploaded, packed and expanded for them gathers here until flush_uploads() (host_io.cpp) issues all of it in three launches
   bool loading = false;
   std::vector<tpuhip::StagedCopy> staged;
   std::vector<tpuhip::FilterPack> packs;
+  std::vector<tpuhip::ParamExpand> params;
   bool in_interpreter = false;   // a module loads or invokes its kernels: device addresses asked for now go to those
   hipStream_t copy_stream = nullptr;   // results laid out early leave on it while `stream` works on; made on first use
   std::vector<tpuhip::AheadRead *> ahead;   // those that may still be asked for
@@ -97,10 +106,22 @@ int not_captured(tpuhip_ctx *ctx, const char *what);
 // host/host_io.cpp: tpuhip_upload without the wait -- src may be reused on return, the bytes are there for what is issued to
 // the context's stream afterwards
 int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes);
-// issues what has gathered in ctx->staged and ctx->packs
+// issues what has gathered in ctx->staged, ctx->packs and ctx->params
 int flush_uploads(tpuhip_ctx *ctx);
+// A 256-entry table that is y -> max(y, (y * m + 2^(r - 1)) >> r) with 0 < m <= 2^r and products within 16 bits: a leaky ReLU's,
+// which the conv kernels compute instead of looking it up.  m == 0: none.
+struct LeakySlope {
+  int m = 0, r = 0;
+};
+// conv.hip: the line of the fewest bits, if the table is one (1.3 us: for whoever loads a model, not for a call)
+bool slope_of_table(const int8_t *table, LeakySlope *out);
+// conv.hip: tpuhip_conv2d_post_i8 by a caller that knows what slope_of_table() says of post->lut (NULL: does not)
+int conv2d_post(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y, const tpuhip_conv_post *post,
+                const LeakySlope *slope);
 // conv.hip: packs n filters; the list is in memory the device reads
 int pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t largest);
+// conv.hip: makes the requantisation parameters of n layers; the list likewise
+int expand_params(tpuhip_ctx *ctx, const ParamExpand *list, size_t n, int largest);
 // waits for what a prepack call has issued, unless a module is being loaded: packed weights may be used from any context
 int prepack_done(tpuhip_ctx *ctx);
 

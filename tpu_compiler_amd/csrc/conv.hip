@@ -61,7 +61,7 @@ struct tpuhip_conv_weights {
                              // whose tile a recorded graph fixed, as long as the layer
   int8_t *w = nullptr;   // packed filter
   size_t w_room = 0;     // bytes behind w
-  int8_t *params = nullptr;   // one allocation behind bias, qp, qplanes and qc64
+  int8_t *params = nullptr;   // one allocation behind bias, qp (the direct kernel's), qplanes and qc64 or qnarrow
   int32_t *bias = nullptr;
   QParam *qp = nullptr;
   int32_t *qplanes = nullptr;   // mult | rshift | hpot planes of nparam entries each
@@ -3628,10 +3628,7 @@ __device__ __forceinline__ void ksplit_body(const ConvArgs &a) {
                          requant_core<FAST>(t[2], mult[2], shift[2], hpot[2]), requant_core<FAST>(t[3], mult[3], shift[3], hpot[3]), out.lo);
   if (!live) return;
   if (a.store_y) *reinterpret_cast<uint32_t *>(out.y + off) = o;
-  if (a.slope_m) {
-    o = leaky_word(o, a.slope_m, a.slope_r);
-    if (a.lut_dst) *reinterpret_cast<uint32_t *>(a.lut_dst + off) = o;
-  } else if (a.has_lut) {
+  if (a.has_lut) {
     const uint32_t r = (uint32_t)lut[o & 255u] | ((uint32_t)lut[(o >> 8) & 255u] << 8) | ((uint32_t)lut[(o >> 16) & 255u] << 16) |
                        ((uint32_t)lut[o >> 24] << 24);
     const int valid = a.oc - oc;   // channels of this dword that exist
@@ -3660,7 +3657,7 @@ struct LeanArgs {
   const int8_t *x, *w;
   int8_t *y;
   const int32_t *bias;
-  int nparam;                  // the planes of the requantisation lie behind nparam biases and records
+  int nparam;                  // the planes of the requantisation lie behind nparam biases
   uint32_t x_bytes;
   int npix, n_tiles, tiles_per_xcd, pstep_n;
   uint32_t magic_tile, magic_ow, magic_oh, magic_c16, magic_kw;
@@ -3672,7 +3669,7 @@ static_assert(sizeof(LeanArgs) <= 112, "see above");
 
 __device__ __forceinline__ void unpack_args(const LeanArgs &l, ConvArgs *a) {
   a->x = l.x; a->w = l.w; a->y = l.y; a->bias = l.bias;
-  a->qmult = reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(l.bias) + (int64_t)l.nparam * (4 + sizeof(QParam)));
+  a->qmult = l.bias + l.nparam;
   a->qshift = a->qmult + l.nparam;
   a->qhpot = a->qshift + l.nparam;
   a->x_bytes = l.x_bytes;
@@ -3687,7 +3684,7 @@ __device__ __forceinline__ void unpack_args(const LeanArgs &l, ConvArgs *a) {
   a->lo = l.relu == 1 ? 0 : -128;
   a->relu_first = l.relu >> 1;
   a->store_y = 1;
-  a->has_lut = 0; a->slope_m = 0; a->lut_dst = nullptr; a->add_src = nullptr; a->add_dst = nullptr; a->split_oc = 0; a->y2 = nullptr;
+  a->has_lut = 0; a->lut_dst = nullptr; a->add_src = nullptr; a->add_dst = nullptr; a->split_oc = 0; a->y2 = nullptr;
 }
 
 template <int W, int TN, bool FAST, bool UNI>
@@ -4271,7 +4268,7 @@ void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
 
 // the short form of a K-split launch's arguments; false: something is fused, or a number does not fit
 bool lean_args(const ConvArgs &a, LeanArgs *out) {
-  if (a.has_lut || a.slope_m || a.add_dst || a.split_oc || !a.store_y || !a.y) return false;
+  if (a.has_lut || a.add_dst || a.split_oc || !a.store_y || !a.y) return false;
   auto u16 = [](int v) { return v >= 0 && v < 65536; };
   auto u8 = [](int v) { return v >= 0 && v < 256; };
   if (!u16(a.ih) || !u16(a.iw) || !u16(a.oh) || !u16(a.ow) || !u16(a.x_cs) || !u16(a.y_cs) || !u16(a.oc) || !u16(a.c16) ||
@@ -4279,7 +4276,7 @@ bool lean_args(const ConvArgs &a, LeanArgs *out) {
     return false;
   const int64_t nparam = a.qshift - a.qmult;
   const int kp = (a.k16 + 3 & ~3) * 16;
-  if ((const char *)a.qmult - (const char *)a.bias != nparam * (int64_t)(4 + sizeof(QParam)) || a.qhpot - a.qshift != nparam ||
+  if (a.qmult - a.bias != nparam || a.qhpot - a.qshift != nparam ||
       a.kp != kp || a.w_bytes != (uint32_t)(a.n_oc_tiles * 32) * (uint32_t)kp || a.ocw != (a.oc + 15 & ~15))
     return false;
   *out = LeanArgs{a.x, a.w, a.y, a.bias, (int)nparam, a.x_bytes, a.npix, a.n_tiles, a.tiles_per_xcd, a.pstep_n,
@@ -4505,6 +4502,55 @@ __global__ __launch_bounds__(256) void pack_filters_kernel(const FilterPack *lis
   for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < a.total; q += (int64_t)gridDim.x * 256) pack_filter_group(a, q);
 }
 
+// ParamExpand, one entry of the arrays per thread: the reference's numbers and what the kernels' forms of the requantisation
+// want of them; channels past oc get zeros (a right shift of 1), which requantise to zero
+__device__ __forceinline__ void expand_param(const ParamExpand &e, int i) {
+  const bool real = i < e.oc;
+  const int32_t b = real ? e.raw[i] : 0, m = real ? e.raw[e.oc + i] : 0, r = real ? e.raw[2 * e.oc + i] : 1;
+  const int n = e.nparam;
+  const int32_t hpot = r > 0 ? (int32_t)(1u << (r - 1)) : 0;
+  int32_t *at = e.out + n;
+  e.out[i] = b;
+  if (e.records) {
+    reinterpret_cast<QParam *>(at)[i] = QParam{m, r, (int32_t)((1ll << r) - 1), hpot};
+    at += 4 * n;
+  }
+  at[i] = m;
+  at[n + i] = r;
+  at[2 * n + i] = hpot;
+  at += 3 * n;
+  const int64_t c = (int64_t)b * (int64_t)m + (1ll << 30);
+  int64_t c2[2] = {real || !e.narrow ? c : 0, real || !e.narrow ? c + ((int64_t)hpot << 31) : 0};
+  if (e.narrow) {
+    int32_t mn = 0, scale = 0, unit = 0;
+    if (real) {
+      (void)narrow_requant(c2[0], m, r, &c2[0], &mn, &scale, &unit);
+      (void)narrow_requant(c2[1], m, r, &c2[1], &mn, &scale, &unit);
+    }
+    at[4 * n + i] = mn;
+    if (i & 1) at[5 * n + i] = 0;
+    reinterpret_cast<int16_t *>(at + 5 * n + (i & ~1))[i & 1] = (int16_t)scale;
+    at[6 * n + i] = unit;
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    at[2 * (k * n + i)] = (int32_t)(uint32_t)(c2[k] & 0xffffffffll);
+    at[2 * (k * n + i) + 1] = (int32_t)(c2[k] >> 32);
+  }
+}
+
+__global__ __launch_bounds__(256) void expand_param_kernel(ParamExpand e) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i < e.nparam) expand_param(e, i);
+}
+
+// those of a loading module, a row of workgroups each
+__global__ __launch_bounds__(256) void expand_params_kernel(const ParamExpand *list) {
+  const ParamExpand e = list[blockIdx.y];
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i < e.nparam) expand_param(e, i);
+}
+
 // now, or with the others of the module that is being loaded
 int pack_filter(tpuhip_ctx *ctx, const FilterPack &a) {
   if (ctx->loading) {
@@ -4624,7 +4670,7 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
   a.qshift = w->qplanes + w->nparam;
   a.qhpot = w->qplanes + 2 * w->nparam;
   a.qc64 = w->qc64;
-  a.qc64r = w->qc64 + 2 * w->nparam;
+  a.qc64r = w->qc64 ? w->qc64 + 2 * w->nparam : nullptr;
   const int reg = w->algo == ALGO_MFMA ? kTiles[w->tile].reg : -1;
   if (reg == 0 || reg == 3 || reg == 5 || reg == 6 || reg == 7 || reg == 9) take_narrow(w, &a);
   a.y = (int8_t *)y;
@@ -4791,6 +4837,7 @@ void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvA
 // what runs behind the requantisation in the epilogue
 struct PostOps {
   const int8_t *lut = nullptr;   // host table, 256 entries
+  const LeakySlope *slope = nullptr;
   void *lut_out = nullptr;
   const tpuhip_fused_add *f = nullptr;
   const void *add_src = nullptr;
@@ -4846,39 +4893,29 @@ bool stem_pool_plan(const tpuhip_conv_weights *w, const tpuhip_pool_desc &p, int
   return true;
 }
 
-// Whether a table is y -> max(y, (y * m + 2^(r - 1)) >> r) for some 0 < m <= 2^r whose products stay within 16 bits, and the
-// smallest such r.  The negative entries say how steep the line may be: (-k m + 2^(r-1)) >> r == t holds exactly where
-// m / 2^r is in ((-t - 1/2) / k, (1/2 - t) / k]; what comes out is held against the whole table.  0.1 us a call.
-bool slope_of_table(const int8_t *t, int *slope_m, int *slope_r) {
-  for (int y = 0; y < 128; ++y)
-    if (t[y] != y) return false;
-  double above = 0, upto = 1;
-  for (int k = 1; k <= 128; ++k) {
-    const double v = t[256 - k], inv = 1.0 / k;
-    above = std::max(above, (-v - 0.5) * inv);
-    upto = std::min(upto, (0.5 - v) * inv);
-  }
-  for (int r = 1; r <= 14 && above < upto + 1e-9; ++r) {
-    const int half = 1 << (r - 1);
-    for (int m = std::max(1, (int)(above * (1 << r)) - 1); m <= (int)(upto * (1 << r)) + 1 && m <= 1 << r && 128 * m + half < 32768; ++m) {
-      bool all = true;
-      for (int k = 1; k <= 128; ++k) all &= t[256 - k] == std::max(-k, (half - k * m) >> r);
-      if (all) {
-        *slope_m = m;
-        *slope_r = r;
-        return true;
-      }
-    }
-  }
-  return false;
+// whether a table is the line of LeakySlope{m, r}
+bool is_line(const int8_t *t, int m, int r) {
+  const int half = 1 << (r - 1);
+  bool all = 128 * m + half < 32768;
+  for (int y = 0; y < 128; ++y) all &= t[y] == y;
+  for (int k = 1; k <= 128; ++k) all &= t[256 - k] == std::max(-k, (half - k * m) >> r);
+  return all;
 }
 
-// slope: the kernels of the launch can compute a leaky ReLU's table (all but the dot-product depthwise one).  A lookup takes
-// 16 instructions and four LDS reads per four outputs, the line 10 and none.
-void apply_fusion(ConvArgs *a, const void *y, const PostOps &p, bool slope = true) {
+// slope: what the caller knows of the table (conv2d_post); else only a line of 7 bits is looked for, whose slope the last entry
+// tells: 60 ns, where looking for any takes 1.3 us.  A lookup takes 16 instructions and four LDS reads per four outputs, the line
+// 10 and none.
+void apply_fusion(ConvArgs *a, const void *y, const PostOps &p, bool can_slope) {
   if (p.lut) {
     a->lut_dst = (int8_t *)p.lut_out;
-    if (!slope || !slope_of_table(p.lut, &a->slope_m, &a->slope_r)) {
+    LeakySlope s;
+    if (can_slope) {
+      if (p.slope) s = *p.slope;
+      else if (p.lut[128] < 0 && is_line(p.lut, -p.lut[128], 7)) s = LeakySlope{-p.lut[128], 7};
+    }
+    a->slope_m = s.m;
+    a->slope_r = s.r;
+    if (!s.m) {
       a->has_lut = 1;
       memcpy(a->lut.w, p.lut, 256);
     }
@@ -4896,6 +4933,12 @@ void apply_fusion(ConvArgs *a, const void *y, const PostOps &p, bool slope = tru
   a->y2 = (int8_t *)p.y2;
 }
 
+// the kernels of the layer that compute a leaky ReLU's line: not the dot-product depthwise one, and not the K-split ones, where a
+// lane has four outputs and a lookup is 0.25 us faster (512 -> 1024 3x3 on 13 x 13: 8.10 us, the line 8.35)
+bool can_slope(const tpuhip_conv_weights *w) {
+  return w->algo != ALGO_DEPTHWISE_DOT && !(w->algo == ALGO_MFMA && kTiles[w->tile].reg == 8);
+}
+
 // Tiles that timing has chosen, by everything the choice can depend on: a layer of the same shape -- a second module, the
 // same model loaded again -- takes its tile from here.  Shared by all contexts, bounded (beyond it, it starts anew).
 using TileKey = std::array<int, 32>;
@@ -4907,7 +4950,7 @@ TileKey tile_key(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void
   const tpuhip_conv_desc &d = w->d;
   const tpuhip_fused_add *f = p.has_add() ? p.f : nullptr;
   return TileKey{ctx->num_cu, d.n, d.ic, d.ih, d.iw, d.oc, d.oh, d.ow, d.kh, d.kw, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw,
-                 d.x_cs, d.y_cs, d.do_relu, d.relu_first, w->fast, w->split_oc, w->y2_cs, w->relu2, y != nullptr,
+                 d.x_cs, d.y_cs, d.do_relu, d.relu_first, requant_form(w), w->split_oc, w->y2_cs, w->relu2, y != nullptr,
                  p.lut != nullptr, p.lut_out != nullptr, f != nullptr,
                  f && std::abs(f->m_src) <= 127 && std::abs(f->m_conv) <= 127 && f->rshift <= 8, f && f->do_relu,
                  d.pb, d.pr};
@@ -4947,7 +4990,7 @@ int autotune_mfma(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *
     if (rc) return -1;
     ConvArgs a;
     fill_args(ctx, w, x, y, &a);
-    apply_fusion(&a, y, post);
+    apply_fusion(&a, y, post, can_slope(w));
     hipLaunchKernelGGL(delay_kernel, dim3(1), dim3(64), 0, ctx->stream, 4 + runs);
     launch_conv_mfma(ctx, w, a);
     hipError_t er = hipEventRecord(e0, ctx->stream);
@@ -5044,9 +5087,33 @@ int choose_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *y,
 
 }  // namespace
 
+// The negative entries say how steep the line may be: (-k m + 2^(r-1)) >> r == t holds exactly where m / 2^r is in
+// ((-t - 1/2) / k, (1/2 - t) / k]; what comes out is held against the whole table.
+bool tpuhip::slope_of_table(const int8_t *t, LeakySlope *out) {
+  double above = 0, upto = 1;
+  for (int k = 1; k <= 128; ++k) {
+    above = std::max(above, (-t[256 - k] - 0.5) / k);
+    upto = std::min(upto, (0.5 - t[256 - k]) / k);
+  }
+  for (int r = 1; r <= 14 && above < upto + 1e-9; ++r)
+    for (int m = std::max(1, (int)(above * (1 << r)) - 1); m <= (int)(upto * (1 << r)) + 1 && m <= 1 << r; ++m)
+      if (is_line(t, m, r)) {
+        *out = LeakySlope{m, r};
+        return true;
+      }
+  return false;
+}
+
 int tpuhip::pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t largest) {
   const dim3 grid((unsigned)std::min<int64_t>(ceil_div64(largest, 256), 32), (unsigned)n);
   hipLaunchKernelGGL(pack_filters_kernel, grid, dim3(256), 0, ctx->stream, list);
+  TPUHIP_CHECK_HIP(hipGetLastError());
+  return TPUHIP_OK;
+}
+
+int tpuhip::expand_params(tpuhip_ctx *ctx, const ParamExpand *list, size_t n, int largest) {
+  const dim3 grid((unsigned)ceil_div64(largest, 256), (unsigned)n);
+  hipLaunchKernelGGL(expand_params_kernel, grid, dim3(256), 0, ctx->stream, list);
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }
@@ -5188,86 +5255,57 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   // for every channel, 1 <= rshift and |acc + bias| + 1 + 2^(rshift-1) cannot reach
   // 2^31: |acc| <= 128 * sum|w|, and |x| <= |v| + 1 after the doubling high multiply.
   const size_t nparam = (size_t)round_up(d.oc, 256) + 16;   // covers every tile's padding
-  std::vector<int32_t> b32(nparam, 0);
-  std::vector<QParam> qp(nparam);
-  bool fast = true;
-  for (int i = 0; i < (int)qp.size(); ++i) {
-    QParam q{};
-    if (i < d.oc) {
-      b32[i] = (d.with_bias && bias) ? bias[i] : 0;
-      q.mult = multiplier[i];
-      q.rshift = rshift[i];
-      q.mask = (int32_t)((1ll << rshift[i]) - 1);
-      q.hpot = rshift[i] > 0 ? (int32_t)(1ll << (rshift[i] - 1)) : 0;
-      const int64_t rest = std::llabs((long long)b32[i]) + 1 + q.hpot;
-      int64_t sumw = 128 * (int64_t)per_oc;   // no filter's sum is larger; it is taken only where that is not small enough
-      if (128 * sumw + rest >= (1ll << 31)) {
-        sumw = 0;
-        for (size_t k = 0; k < per_oc; ++k) sumw += std::abs((int)filter[(size_t)i * per_oc + k]);
-      }
-      const int64_t bound = 128 * sumw + rest;
-      if (rshift[i] < 1 || bound >= (1ll << 31)) fast = false;
-    } else {
-      q.rshift = 1;   // pad channels: multiplier 0 gives 0 on either path
-      q.mask = 1;
-      q.hpot = 1;
+  std::vector<int32_t> raw(3 * (size_t)d.oc);
+  bool fast = true, narrow = !d.relu_first;
+  for (int i = 0; i < d.oc; ++i) {
+    const int32_t b = (d.with_bias && bias) ? bias[i] : 0, m = multiplier[i], r = rshift[i];
+    raw[i] = b;
+    raw[d.oc + i] = m;
+    raw[2 * d.oc + i] = r;
+    narrow &= allows_narrow(m, r);
+    const int64_t rest = std::llabs((long long)b) + 1 + (r > 0 ? 1ll << (r - 1) : 0);
+    int64_t sumw = 128 * (int64_t)per_oc;   // no filter's sum is larger; it is taken only where that is not small enough
+    if (128 * sumw + rest >= (1ll << 31)) {
+      sumw = 0;
+      for (size_t k = 0; k < per_oc; ++k) sumw += std::abs((int)filter[(size_t)i * per_oc + k]);
     }
-    qp[i] = q;
+    if (r < 1 || 128 * sumw + rest >= (1ll << 31)) fast = false;
   }
+  narrow &= fast;
   cw->fast = fast ? 1 : 0;
   int rc = TPUHIP_OK;
   if (!packed.empty()) {
     rc = tpuhip_malloc(ctx, packed.size(), (void **)&cw->w);
     if (!rc) rc = stage_upload(ctx, cw->w, packed.data(), packed.size());
   }
-  // one allocation and one upload: biases, records, the planes of the records' fields, and per channel the addend of the
-  // requantisation's 64-bit multiply-add, (acc + bias) * mult + 2^30 == acc * mult + c, as (low, high) words
+  // one allocation: biases, the direct kernel's records, planes, the addends of the requantisation's 64-bit multiply-add or the
+  // planes of requant_rows_narrow -- made on the device (48 bytes a channel, padded, took the host and the bus longer than all
+  // filters of a light network) from three numbers per channel behind them
   cw->nparam = (int)nparam;
-  const size_t at_qp = nparam * 4, at_planes = at_qp + nparam * sizeof(QParam), at_c64 = at_planes + 3 * nparam * 4,
-               at_narrow = at_c64 + 4 * nparam * 4;
-  std::vector<int8_t> image(at_narrow + 7 * nparam * 4);
-  memcpy(image.data(), b32.data(), nparam * 4);
-  memcpy(image.data() + at_qp, qp.data(), nparam * sizeof(QParam));
-  int32_t *planes = (int32_t *)(image.data() + at_planes), *c64 = (int32_t *)(image.data() + at_c64);
-  for (size_t i = 0; i < nparam; ++i) {
-    planes[i] = qp[i].mult;
-    planes[nparam + i] = qp[i].rshift;
-    planes[2 * nparam + i] = qp[i].hpot;
-    const int64_t c = (int64_t)b32[i] * (int64_t)qp[i].mult + (1ll << 30);
-    const int64_t cr = c + ((int64_t)qp[i].hpot << 31);
-    c64[2 * i] = (int32_t)(uint32_t)(c & 0xffffffffll);
-    c64[2 * i + 1] = (int32_t)(c >> 32);
-    c64[2 * nparam + 2 * i] = (int32_t)(uint32_t)(cr & 0xffffffffll);
-    c64[2 * nparam + 2 * i + 1] = (int32_t)(cr >> 32);
-  }
-  // the same for requant_rows_narrow; pad channels stay zero
-  bool narrow = fast && !d.relu_first;
-  int32_t *nc = (int32_t *)(image.data() + at_narrow), *nplanes = nc + 4 * nparam;
-  for (int i = 0; i < d.oc && narrow; ++i) {
-    const int64_t c = (int64_t)b32[i] * (int64_t)qp[i].mult + (1ll << 30);
-    int32_t scale = 0;
-    for (int relu = 0; relu < 2 && narrow; ++relu) {
-      int64_t cn = 0;
-      narrow = narrow_requant(c + (relu ? (int64_t)qp[i].hpot << 31 : 0), qp[i].mult, qp[i].rshift, &cn, &nplanes[i], &scale,
-                              &nplanes[2 * nparam + i]);
-      nc[2 * (relu * nparam + i)] = (int32_t)(uint32_t)(cn & 0xffffffffll);
-      nc[2 * (relu * nparam + i) + 1] = (int32_t)(cn >> 32);
+  const bool records = cw->algo == ALGO_DIRECT && !cw->gather;
+  const size_t at_planes = nparam * (records ? 5 : 1), at_last = at_planes + 3 * nparam, at_raw = at_last + nparam * (narrow ? 7 : 4);
+  if (!rc) rc = tpuhip_malloc(ctx, (at_raw + raw.size()) * 4, (void **)&cw->params);
+  int32_t *const p = (int32_t *)cw->params;
+  if (!rc) rc = stage_upload(ctx, p + at_raw, raw.data(), raw.size() * 4);
+  if (!rc) {
+    const ParamExpand e{p + at_raw, p, d.oc, (int)nparam, records ? 1 : 0, narrow ? 1 : 0};
+    if (ctx->loading) {
+      ctx->params.push_back(e);
+    } else {
+      hipLaunchKernelGGL(expand_param_kernel, dim3((unsigned)ceil_div64(e.nparam, 256)), dim3(256), 0, ctx->stream, e);
+      const hipError_t launched = hipGetLastError();
+      if (launched != hipSuccess) rc = set_error(TPUHIP_ERR_HIP, "conv: parameters: %s", hipGetErrorString(launched));
     }
-    nplanes[nparam + (i & ~1)] |= scale << (16 * (i & 1));
   }
-  if (!narrow) image.resize(at_narrow);
-  if (!rc) rc = tpuhip_malloc(ctx, image.size(), (void **)&cw->params);
-  if (!rc) rc = stage_upload(ctx, cw->params, image.data(), image.size());
   if (!rc) rc = prepack_done(ctx);
   if (rc) {
     tpuhip_conv2d_weights_destroy(ctx, cw);
     return rc;
   }
-  cw->bias = (int32_t *)cw->params;
-  cw->qp = (QParam *)(cw->params + at_qp);
-  cw->qplanes = (int32_t *)(cw->params + at_planes);
-  cw->qc64 = (int32_t *)(cw->params + at_c64);
-  if (narrow) cw->qnarrow = (int32_t *)(cw->params + at_narrow);
+  cw->bias = p;
+  cw->qp = records ? (QParam *)(p + nparam) : nullptr;
+  cw->qplanes = p + at_planes;
+  (narrow ? cw->qnarrow : cw->qc64) = p + at_last;
   *out = cw;
   return TPUHIP_OK;
 }
@@ -5405,7 +5443,7 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
   }
   ConvArgs a;
   fill_args(ctx, w, x, y, &a);
-  apply_fusion(&a, y, post, w->algo != ALGO_DEPTHWISE_DOT);
+  apply_fusion(&a, y, post, can_slope(w));
   if (w->algo == ALGO_MFMA) {
     launch_conv_mfma(ctx, w, a);
   } else if (w->algo == ALGO_DEPTHWISE) {
@@ -5529,6 +5567,13 @@ int tpuhip_conv2d_add_i8(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const vo
 
 int tpuhip_conv2d_post_i8(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y,
                           const tpuhip_conv_post *post) {
+  return conv2d_post(ctx, w, x, y, post, nullptr);
+}
+
+}  // extern "C"
+
+int tpuhip::conv2d_post(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y, const tpuhip_conv_post *post,
+                        const LeakySlope *slope) {
   TPUHIP_REQUIRE(ctx && w && x && post, "tpuhip_conv2d_post_i8: NULL argument");
   PostOps p;
   if (post->lut) {
@@ -5536,6 +5581,7 @@ int tpuhip_conv2d_post_i8(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const v
                        w->algo == ALGO_STEM,
                    "conv2d_post: only dense convs on the MFMA or stem path and depthwise convs can fuse a table");
     p.lut = post->lut;
+    p.slope = slope;
     p.lut_out = post->lut_out;
   }
   if (post->add.enable) {
@@ -5553,6 +5599,8 @@ int tpuhip_conv2d_post_i8(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const v
   TPUHIP_REQUIRE(y || p.lut_out || p.add_out || p.pool_out, "conv2d_post: nothing would be written");
   return run_conv(ctx, w, x, y, p);
 }
+
+extern "C" {
 
 int tpuhip_conv2d_can_fuse_pool(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const tpuhip_pool_desc *pool) {
   if (!ctx || !w || !pool) return 0;

@@ -166,12 +166,16 @@ __device__ __forceinline__ void requant_rows_narrow(const v16i (&acc)[TN], const
   }
 }
 
+__host__ __device__ inline bool allows_narrow(int32_t mult, int32_t rshift) {
+  const int f = rshift > 9 ? rshift - 9 : 0;
+  return rshift >= 2 && rshift <= 31 && !(mult & (int32_t)((1u << f) - 1u));
+}
 // One channel's constants for requant_rows_narrow; false: they do not allow it (a right shift of 1 or less, or a multiplier
 // without the trailing zeros: one that was stored as a float has at least 7 below 2^31, which covers right shifts to 16).
 // relu: c holds the rounding term of the short form.
-inline bool narrow_requant(int64_t c, int32_t mult, int32_t rshift, int64_t *cn, int32_t *mn, int32_t *scale, int32_t *unit) {
+__host__ __device__ inline bool narrow_requant(int64_t c, int32_t mult, int32_t rshift, int64_t *cn, int32_t *mn, int32_t *scale, int32_t *unit) {
   const int f = rshift > 9 ? rshift - 9 : 0, s = rshift - 1 - f;
-  if (rshift < 2 || rshift > 31 || (mult & (int32_t)((1u << f) - 1u))) return false;
+  if (!allows_narrow(mult, rshift)) return false;
   *cn = c >> f;
   *mn = mult >> f;
   *scale = 1 << (8 - s);

@@ -702,9 +702,9 @@ __global__ __launch_bounds__(256) void staged_copies_kernel(const StagedCopy *li
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < c.dwords; i += stride) c.dst[i] = c.src[i];
 }
 
-// A network of 52 convs took three launches for each, 440 us of a 5 ms tool run; all of them together take two.
+// A network of 52 convs took three launches for each, 440 us of a 5 ms tool run; all of them together take three.
 int flush_uploads(tpuhip_ctx *ctx) {
-  if (ctx->staged.empty() && ctx->packs.empty()) return TPUHIP_OK;
+  if (ctx->staged.empty() && ctx->packs.empty() && ctx->params.empty()) return TPUHIP_OK;
   if (int rc = not_captured(ctx, "packed weights")) return rc;
   auto place = [&](const void *list, size_t bytes) -> void * {   // stage_upload() leaves the room for it
     void *at = (int8_t *)ctx->stage + ctx->stage_used;
@@ -730,6 +730,14 @@ int flush_uploads(tpuhip_ctx *ctx) {
     ctx->packs.clear();
     if (int rc = pack_filters(ctx, (const FilterPack *)list, n, largest)) return rc;
   }
+  if (!ctx->params.empty()) {
+    int largest = 0;
+    for (auto &p : ctx->params) largest = std::max(largest, p.nparam);
+    const void *list = place(ctx->params.data(), ctx->params.size() * sizeof(ParamExpand));
+    const size_t n = ctx->params.size();
+    ctx->params.clear();
+    if (int rc = expand_params(ctx, (const ParamExpand *)list, n, largest)) return rc;
+  }
   return TPUHIP_OK;
 }
 
@@ -738,7 +746,7 @@ int stage_upload(tpuhip_ctx *ctx, void *dst, const void *src, size_t bytes) {
   const size_t kRoom = ctx->loading ? 8 << 20 : 4 << 20;
   constexpr size_t kLists = 64 << 10, kMost = 256;   // room for flush_uploads(), and the launches it gathers at most
   for (size_t at = 0; at < bytes;) {
-    if (ctx->staged.size() >= kMost || ctx->packs.size() >= kMost)
+    if (ctx->staged.size() >= kMost || ctx->packs.size() >= kMost || ctx->params.size() >= kMost)
       if (int rc = flush_uploads(ctx)) return rc;
     if (!ctx->stage || ctx->stage_used + kLists + 16 > ctx->stage_bytes ||
         (at == 0 && bytes + kLists <= kRoom && ctx->stage_used + bytes + kLists > ctx->stage_bytes)) {

@@ -600,9 +600,8 @@ void Conv2DOpKernel::invoke() {
     post.add_src = add_src->data();
     post.add_out = add_dst->data();
   }
-  ck(tpuhip_conv2d_post_i8(ctx, packed, input_data->data(),
-                           store_result ? output_data->data() : nullptr, &post),
-     name.c_str());
+  const LeakySlope slope{lut_slope_m, lut_slope_r};
+  ck(conv2d_post(ctx, packed, input_data->data(), store_result ? output_data->data() : nullptr, &post, &slope), name.c_str());
 }
 
 bool Conv2DOpKernel::can_fuse_add() const {
@@ -645,6 +644,10 @@ void Conv2DOpKernel::fuse_lut(const int8_t *table, SyncedData dst) {
   if (!dst || dst->slot_bytes() != output_data->slot_bytes() || dst->cs != output_data->cs)
     fail("Conv2D '" + name + "': a fused table's result must match the conv result's shape");
   memcpy(lut_table, table, 256);
+  LeakySlope slope;
+  (void)slope_of_table(table, &slope);
+  lut_slope_m = slope.m;
+  lut_slope_r = slope.r;
   lut_dst = dst;
   store_lut = true;
 }
