@@ -1,0 +1,64 @@
+"""Transposed convs of eight 32-byte slices or more per output (zeros between the input's pixels): phases that differ in size
+and in taps or have none, strides and dilations against the zeros, odd numbers of 16-channel groups, ragged tiles and channel
+blocks, patches past 64 KB, and both sides of the rule that takes a layer to the patch kernel."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from gpu_helpers import conv_desc, f2i32
+from tpu_compiler_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0)
+    yield c
+    c.close()
+
+
+# n, ic, ih, iw, oc, (kh, kw), stride, pads (t, b, l, r), dil, ins, relu, relu_first
+CASES = [
+    (2, 128, 13, 11, 70, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),
+    (1, 64, 9, 33, 33, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), False, 1),         # eight slices; relu before
+    (1, 48, 9, 33, 33, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), False, 0),         # six: the other kernel
+    (3, 80, 6, 7, 16, (4, 4), (1, 1), (2, 1, 1, 2), (1, 1), (1, 1), True, 0),           # 5 groups of 16, odd result sizes
+    (1, 136, 5, 6, 100, (3, 3), (1, 1), (1, 2, 1, 2), (1, 1), (1, 1), False, 0),        # taps 1, 2, 2, 4; an odd count of entries
+    (2, 272, 4, 9, 40, (3, 3), (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), True, 0),          # 17 groups of 16
+    (1, 256, 6, 5, 40, (2, 2), (1, 1), (0, 1, 0, 1), (1, 1), (2, 2), True, 0),          # phases without a tap
+    (1, 128, 7, 6, 20, (4, 3), (1, 1), (2, 2, 1, 1), (1, 1), (1, 0), False, 0),         # two phases
+    (1, 64, 7, 8, 64, (5, 4), (3, 3), (3, 2, 2, 2), (1, 1), (1, 1), True, 0),           # stride 3 against the zeros
+    (1, 64, 8, 9, 33, (4, 4), (1, 2), (3, 3, 3, 3), (2, 1), (2, 2), False, 0),          # nine phases, stride and dilation
+    (2, 512, 1, 1, 40, (4, 4), (1, 1), (3, 3, 3, 3), (1, 1), (1, 1), True, 0),          # one pixel to 4 x 4
+    (1, 512, 2, 1, 24, (2, 3), (1, 1), (0, 0, 1, 1), (1, 1), (1, 1), False, 0),         # a single result column
+    (1, 256, 5, 101, 40, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # three rows of patch: 84 KB
+    (1, 256, 3, 250, 36, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # no patch: the other kernel
+    (1, 64, 201, 200, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # 40200 pixels: the other kernel
+    (1, 64, 200, 200, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), False, 0),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])))
+@pytest.mark.parametrize("smallest_shift", [0, 1])
+def test_against_the_oracle(ctx, case, smallest_shift):
+    n, ic, ih, iw, oc, k, stride, pads, dil, ins, relu, relu_first = case
+    rng = np.random.default_rng(ic + ih * 3 + oc + k[0])
+    x = rng.integers(-128, 128, (n, ic, ih, iw)).astype(np.int8)
+    w = np.clip(np.rint(rng.normal(0, 16, (oc, ic, *k))), -127, 127).astype(np.int8)
+    bias, mult = rng.integers(-4096, 4097, oc).astype(np.float32), (rng.integers(1 << 23, 1 << 24, oc) * 128).astype(np.float32)
+    rsh = rng.integers(7, 12, oc).astype(np.float32)
+    rsh[::7] = smallest_shift                       # 0: the form of the requantisation that may overflow
+    if relu_first:   # relu before the requantisation with multipliers above 0 is relu after it
+        relu = True
+    want = O.conv2d_i8(x, w, bias, rsh, mult, O.make_conv_desc(x.shape, w.shape, 1, stride, pads, dil, ins, relu, True, None))
+    d = conv_desc(x.shape, w.shape, stride=stride, pads=pads, dil=dil, ins=ins, do_relu=relu, relu_first=relu_first)
+    xt, yt = ctx.from_nchw(x), ctx.tensor(want.shape)
+    ctx._ck(ctx.lib.tpuhip_memset(ctx.h, yt.ptr, 0x55, yt.nbytes))
+    wh = ctx.conv_prepack(d, w, f2i32(bias), f2i32(mult), f2i32(rsh))
+    ctx.conv(wh, xt, yt)
+    assert np.array_equal(ctx.to_nchw(yt), want) and not ctx.raw(yt)[..., oc:].any()
+    assert len(np.unique(want)) > 8
+    ctx.conv_weights_destroy(wh)
+    xt.free()
+    yt.free()
