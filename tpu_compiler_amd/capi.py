@@ -355,18 +355,31 @@ _pack_move, _pack_binary = struct.Struct("19i").pack, struct.Struct("21i").pack
 _ZEROS = (0,) * 8
 
 
-def _pack_ints(pack, values):
-    """the bytes of a descriptor of ints; numbers that no int holds wrap as ctypes wraps them"""
-    try:
-        return pack(*values)
-    except struct.error:
-        return b"".join(bytes(C.c_int(v)) for v in values)
+def _wrapped(values):
+    """the bytes of ints of which some fit no C int: they wrap as ctypes wraps them"""
+    return b"".join(bytes(C.c_int(v)) for v in values)
 
 
-def _packed(code, values, dtype):
+class _Packers(dict):
+    """count -> what packs that many numbers of one type (a bounded number of counts: concats and sums of many tensors)"""
+
+    def __init__(self, code):
+        self.code = code
+
+    def __missing__(self, n):
+        pack = struct.Struct("%d%s" % (n, self.code)).pack
+        if n <= 64:
+            self[n] = pack
+        return pack
+
+
+_pack_pointers, _pack_int, _pack_int8, _pack_uint32 = (_Packers(c) for c in "PibI")
+
+
+def _packed(packers, values, dtype):
     """the bytes of a sequence of numbers: what numpy makes of them, by a shorter way where they are ints that fit"""
     try:
-        return struct.pack("%d%s" % (len(values), code), *values)
+        return packers[len(values)](*values)
     except (struct.error, TypeError):
         return np.ascontiguousarray(values, dtype=dtype).tobytes()
 
@@ -676,16 +689,19 @@ class Context:
         return self.lib.tpuhip_conv2d_algo_name(w).decode()
 
     def eltwise_add(self, xs, mult, rshift, do_relu, y):
-        ptrs = struct.pack("%dP" % len(xs), *[t.ptr or 0 for t in xs])
-        m = _packed("b", mult, np.int8)
+        ptrs = _pack_pointers[len(xs)](*[t.ptr or 0 for t in xs])
+        m = _packed(_pack_int8, mult, np.int8)
         if rc := self._ops.eltwise_add_i8(self.h, ptrs, len(xs), m, int(rshift), int(do_relu), y.ptr, y.nbytes):
             self._ck(rc)
 
     def move(self, kind, x, y, params):
-        p = tuple(params)
-        if len(p) > 8:
-            raise IndexError("move: at most 8 parameters (%d)" % len(p))
-        d = _pack_ints(_pack_move, (kind, *x.shape, *y.shape, x.cs, y.cs, *p, *_ZEROS[len(p):]))
+        n = len(p := tuple(params))
+        if n > 8:
+            raise IndexError("move: at most 8 parameters (%d)" % n)
+        try:
+            d = _pack_move(kind, *x.shape, *y.shape, x.cs, y.cs, *p, *_ZEROS[n:])
+        except struct.error:
+            d = _wrapped((kind, *x.shape, *y.shape, x.cs, y.cs, *p, *_ZEROS[n:]))
         if rc := self._ops.move_i8(self.h, d, x.ptr, y.ptr):
             self._ck(rc)
 
@@ -704,8 +720,11 @@ class Context:
 
     def binary(self, op, x0, x1, y, m0=1, m1=1, multiplier=0, rshift=0, do_relu=False):
         """x0, x1, y: device tensors made by tensor()/from_nchw() (logical NCHW shapes)"""
-        d = _pack_ints(_pack_binary, (op, *y.shape, *x0.shape, *x1.shape, int(m0), int(m1), int(multiplier), int(rshift),
-                                      int(do_relu), x0.cs, x1.cs, y.cs))
+        try:
+            d = _pack_binary(op, *y.shape, *x0.shape, *x1.shape, m0, m1, multiplier, rshift, do_relu, x0.cs, x1.cs, y.cs)
+        except struct.error:
+            d = _wrapped((op, *y.shape, *x0.shape, *x1.shape, int(m0), int(m1), int(multiplier), int(rshift), int(do_relu),
+                          x0.cs, x1.cs, y.cs))
         if rc := self._ops.binary_i8(self.h, d, x0.ptr, x1.ptr, y.ptr):
             self._ck(rc)
 
@@ -718,13 +737,15 @@ class Context:
             self._ck(rc)
 
     def lut(self, x, y, table):
-        t = np.ascontiguousarray(table, dtype=np.int8)
+        t = np.ascontiguousarray(table, np.int8)
         assert t.size == 256
-        if rc := self._ops.lut_i8(self.h, x.ptr, y.ptr, t.tobytes(), x.pixels, x.shape[1], x.cs):
+        n, c, h, w = x.shape
+        if rc := self._ops.lut_i8(self.h, x.ptr, y.ptr, t.tobytes(), n * h * w, c, x.cs):
             self._ck(rc)
 
     def leaky_relu(self, x, y, rp, mp, rn, mn):
-        if rc := self._ops.leaky_relu_i8(self.h, x.ptr, y.ptr, x.pixels, x.shape[1], x.cs, int(rp), int(mp), int(rn), int(mn)):
+        n, c, h, w = x.shape
+        if rc := self._ops.leaky_relu_i8(self.h, x.ptr, y.ptr, n * h * w, c, x.cs, int(rp), int(mp), int(rn), int(mn)):
             self._ck(rc)
 
     def leaky_relu_table(self, rp, mp, rn, mn):
@@ -750,10 +771,13 @@ class Context:
 
     def concat(self, xs, axis, y, rshift=None, mult=None, do_relu=False):
         n = len(xs)
-        ptrs = struct.pack("%dP" % n, *[t.ptr or 0 for t in xs])
-        dims = struct.pack("%di" % (4 * n), *[v for t in xs for v in t.shape])
-        cs = struct.pack("%di" % n, *[t.cs for t in xs])
-        r = None if rshift is None else _packed("I", rshift, np.uint32)
-        m = None if mult is None else _packed("I", mult, np.uint32)
-        if rc := self._ops.concat_i8(self.h, ptrs, n, dims, cs, axis, r, m, int(do_relu), y.ptr, y.cs):
+        ptrs, dims, cs = [], [], []
+        for t in xs:
+            ptrs.append(t.ptr or 0)
+            dims += t.shape
+            cs.append(t.cs)
+        r = None if rshift is None else _packed(_pack_uint32, rshift, np.uint32)
+        m = None if mult is None else _packed(_pack_uint32, mult, np.uint32)
+        if rc := self._ops.concat_i8(self.h, _pack_pointers[n](*ptrs), n, _pack_int[4 * n](*dims), _pack_int[n](*cs), axis, r, m,
+                                     int(do_relu), y.ptr, y.cs):
             self._ck(rc)
