@@ -2898,6 +2898,148 @@ conv_stem_kernel(ConvArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// The stem of layers whose constants allow the narrow requantisation (requant_rows_narrow).  What the kernel above spends its
+// time on is vector arithmetic: the wide requantisation, and one load, its two divisions and its range check per pixel of a patch
+// of three (seven) input rows for every output row.  Here a workgroup takes `rows` whole output rows of an image: its patch is
+// (rows - 1) * sh + kh input rows, fetched with one 16-byte load per four pixels (kStemPad dwords in front of the image's first
+// column keep those aligned; where the image's rows are no multiple of four pixels or pixels lie 16 bytes apart, four loads of a
+// dword), and its pixels are one run in memory, of which a wave takes 32 * NB at a time, so that maps of any width leave at most
+// the run's last lanes idle and addresses are 32-bit offsets into buffers whose range check drops those.
+// 8 x 608 x 608, 3x3 to 32 channels with a leaky ReLU 61 -> 39 us (ReLU 53 -> 28.5), 64 x 224 x 224 at stride 2 20.4 -> 12.6,
+// 32 x 224 x 224, 7x7 at stride 2 to 64 22 -> 18, one image of 416 x 416 7.9 -> 7.0.  Bound: 23 us of the 39 are the arithmetic
+// (requantisation 23 clocks an output and SIMD, leaky ReLU 11), 17 the LDS reads (a third of them the fragments, the rest the
+// channels' parameters; all of those in registers: 56 more, 44 us), 17 the stores.  The next tile's pixels in flight while one
+// is computed, by resident workgroups: 40 us; four blocks of pixels per wave: 44.
+//   a.pstep_pix = rows of a tile, a.pstep_n = tiles per image (a.magic_oh its ceil(2^32 / d)), a.stem_pw = dwords of a patch row,
+//   a.magic_c16 = ceil(2^32 / 16-byte chunks of it).  ow > 1; sw 1 or 2.  LDS (dynamic): parameters | table | patch.
+// ---------------------------------------------------------------------------
+constexpr int kStemPad = 8;   // dwords of a patch row before the image's first column: the left padding, to a whole chunk
+constexpr int stem_waves(int kh, int tm) { return kh * tm <= 3 ? 4 : kh * tm <= 7 ? 3 : 2; }
+template <int KH, int TM, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stem_waves(KH, TM), stem_waves(KH, TM)))) void
+conv_stem_rows_kernel(ConvArgs a) {
+  gather_conv_args(a);
+  gather_conv_args_more(a);
+  constexpr int QW = 5 * TM * 32;
+  extern __shared__ __attribute__((aligned(16))) v4i stem_smem[];
+  int32_t *const qlds = reinterpret_cast<int32_t *>(stem_smem);       // pairs, multiplier, scale, unit
+  uint32_t *const lutw = reinterpret_cast<uint32_t *>(qlds + QW);     // 64 dwords
+  uint32_t *const patch = lutw + 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int frow = lane & 31, fk = lane >> 5;
+  const int logical = (int)(blockIdx.x & 7) * a.tiles_per_xcd + (int)(blockIdx.x >> 3);
+  if (logical >= a.n_tiles) return;
+  const int img = a.pstep_n == 1 ? logical : (int)__umulhi((uint32_t)logical, a.magic_oh);
+  const int r0 = (logical - img * a.pstep_n) * a.pstep_pix;
+  const int rows = min(a.pstep_pix, a.oh - r0), npx = rows * a.ow;
+  const bool relu = a.lo == 0;
+
+  // parameters, table, filter and patch in one trip to memory
+  int32_t qv[(QW + 255) / 256];
+#pragma unroll
+  for (int k = 0; k < (QW + 255) / 256; ++k) {
+    const int i = tid + k * 256, plane = i / (TM * 32), c = i % (TM * 32);
+    const int32_t *c64 = relu ? a.qc64r : a.qc64;
+    const int32_t *src = plane < 2 ? c64 + i : (plane == 2 ? a.qmult : plane == 3 ? a.qshift : a.qhpot) + c;
+    qv[k] = i < QW ? *src : 0;
+  }
+  uint32_t lutv = 0;
+  if (a.has_lut && tid < 64) lutv = a.lut.w[tid];
+  v4i areg[TM][KH];
+  {
+    const v4i *afrag = reinterpret_cast<const v4i *>(a.w) + lane;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int r = 0; r < KH; ++r) areg[i][r] = afrag[(i * KH + r) * 64];
+  }
+  // ---- the patch, four pixels per lane; what lies outside the image is loaded as zeros
+  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+  const int pw = a.stem_pw, row_chunks = pw >> 2;
+  const int total = ((a.pstep_pix - 1) * a.sh + a.kh) * row_chunks;
+  const int ih0 = r0 * a.sh - a.pt, in_row0 = img * a.ih;
+  const bool whole = a.x_cs == 4 && !(a.iw & 3);
+  constexpr int NP = 4;
+  for (int d0 = tid; d0 < total; d0 += NP * 256) {
+    v4i v[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int d = d0 + u * 256;
+      const int r = (int)__umulhi((uint32_t)d, a.magic_c16), iw = (d - r * row_chunks) * 4 - kStemPad, ih = ih0 + r;
+      const bool row_ok = (d < total) & ((unsigned)ih < (unsigned)a.ih);
+      const uint32_t at = (uint32_t)((in_row0 + ih) * a.iw + iw) * (uint32_t)a.x_cs;
+      if (whole) {
+        v[u] = buffer_load16(xrsrc, row_ok & ((unsigned)iw < (unsigned)a.iw) ? at : kOobOffset);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[u][e] = __builtin_amdgcn_raw_buffer_load_b32(
+              xrsrc, row_ok & ((unsigned)(iw + e) < (unsigned)a.iw) ? at + (uint32_t)(e * a.x_cs) : kOobOffset, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      if (d0 + u * 256 < total) *reinterpret_cast<v4i *>(patch + (d0 + u * 256) * 4) = v[u];
+  }
+#pragma unroll
+  for (int k = 0; k < (QW + 255) / 256; ++k)
+    if (tid + k * 256 < QW) qlds[tid + k * 256] = qv[k];
+  if (a.has_lut && tid < 64) lutw[tid] = lutv;
+  const uint8_t *lut = a.has_lut ? reinterpret_cast<const uint8_t *>(lutw) : nullptr;
+  __syncthreads();
+
+  // ---- the tile's pixels in memory order, 32 * NB at a time per wave
+  const int64_t base = (int64_t)(img * a.oh + r0) * a.ow * a.y_cs;
+  const uint32_t bytes = (uint32_t)(npx * a.y_cs);
+  const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.y + base), 0, a.store_y ? bytes : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t trsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(a.lut_dst + base), 0, a.lut_dst ? bytes : 0, 0x00020000);
+  const int tap0 = kStemPad - a.pl + fk * 4, row_step = a.sh * pw;
+  const uint32_t lane_off = (uint32_t)(frow * a.y_cs + fk * 16);
+  for (int p0 = wave * 32 * NB; p0 < npx; p0 += 128 * NB) {
+    const uint32_t *src[NB];
+    uint32_t off[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int q = p0 + j * 32 + frow, p = min(q, npx - 1);
+      const int row = (int)__umulhi((uint32_t)p, a.magic_ow);
+      const int col = p - __mul24(row, a.ow);
+      src[j] = patch + __mul24(row, row_step) + (col << (a.sw - 1)) + tap0;
+      off[j] = lane_off + (uint32_t)((p0 + j * 32) * a.y_cs);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int oc = i * 32 + fk * 16;
+      v16i acc[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[j][e] = 0;
+#pragma unroll
+      for (int r = 0; r < KH; ++r)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const uint32_t *at = src[j] + min(r, a.kh - 1) * pw;
+          const v4i b = {(int)at[0], (int)at[1], (int)at[2], (int)at[3]};
+          acc[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(areg[i][r], b, acc[j], 0, 0, 0);
+        }
+      uint32_t outw[NB][4];
+      const int32_t *const q = qlds + oc;
+      requant_rows_planes<NB, true>(acc, relu, a.lo, q + oc, q + 2 * TM * 32, q + 3 * TM * 32, q + 4 * TM * 32, outw);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const uint32_t at = oc < a.ocw ? off[j] + i * 32 : kOobOffset;
+        v4i o = {(int)outw[j][0], (int)outw[j][1], (int)outw[j][2], (int)outw[j][3]};
+        if (a.store_y) __builtin_amdgcn_raw_buffer_store_b128((v4u)o, yrsrc, at, 0, 0);
+        if (a.slope_m) o = leaky_chunk(o, a.slope_m, a.slope_r);
+        else if (lut) o = lookup_chunk(o, lut, a.oc - oc);
+        if (a.lut_dst) __builtin_amdgcn_raw_buffer_store_b128((v4u)o, trsrc, at, 0, 0);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // The stem with the max pool behind it (conv 7x7 / stride 2 + ReLU, pool 3x3 / stride 2: the
 // head of the ImageNet networks) as one launch.  A workgroup of 8 waves owns `rows` pooled rows
 // of one image over its whole width:
@@ -5400,6 +5542,46 @@ static void dw_rows_walk(DwRowsArgs *r, unsigned wgs, int n_cb) {
   }
 }
 
+// conv_stem_rows_kernel's tiles and its patch's pitch and LDS; false: the other stem kernel's layer.  The rows of a tile: rounds
+// of resident workgroups, times the passes of their four waves and two more for a tile's start.  (8 x 608 x 608: 5 rows, 2 to 5
+// take 39 to 40.5 us; 64 x 112 x 112: 7 rows 12.6, 2 15.9, 14 13.9; 32 x 112 x 112 of 7x7: 7 rows 18.0, 3 24; one image: 1 row.)
+static bool stem_rows_plan(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, ConvArgs *a, unsigned *lds) {
+  if (!w->qnarrow || w->split_oc || a->add_dst || a->pl > kStemPad || a->ow == 1 || a->ow > 16384) return false;
+  const int tm = a->oc <= 32 ? 1 : 2, per_cu = stem_waves(a->kh <= 3 ? 3 : 7, tm);
+  // up to a round and a half of the other kernel's workgroups of 128 pixels it is done sooner: 1 x 320 x 320 5.4 us against 6.0,
+  // 8 x 101 x 101 results 5.05 against 5.6; 1 x 416 x 416 7.9, here 6.9, 8 x 112 x 112 of 64 channels 8.9, here 7.3
+  if (2 * tm * (int64_t)a->n * a->oh * ((a->ow + 127) / 128) <= 9 * (int64_t)ctx->num_cu) return false;
+  // from kStemPad dwords in front of the image to the last one that the last column's taps (and the zeros behind them) meet
+  const int64_t pw = ((int64_t)(a->ow - 1) * a->sw + kStemPad - a->pl + 8 + 3) / 4 * 4;
+  auto bytes = [&](int rows) { return 5 * tm * 32 * 4 + 256 + ((int64_t)(rows - 1) * a->sh + a->kh) * pw * 4; };
+  int rows = 0;
+  uint32_t best = UINT32_MAX;
+  const uint32_t slots = (uint32_t)(ctx->num_cu * per_cu);
+  for (int r = 1; r <= std::min(a->oh, 8) && bytes(r) <= std::min(64, 160 / per_cu) * 1024; ++r) {   // (at every launch: 0.1 us)
+    const uint32_t tiles = (uint32_t)a->n * (uint32_t)((a->oh + r - 1) / r);
+    const uint32_t cost = (tiles + slots - 1) / slots * (uint32_t)((r * a->ow + 255) / 256 + 2);
+    if (cost < best) {
+      best = cost;
+      rows = r;
+    }
+  }
+  if (!rows) return false;
+  const int tiles = (a->oh + rows - 1) / rows;
+  if ((int64_t)a->n * tiles * tiles >= (1ll << 32) || (int64_t)rows * a->ow * a->y_cs >= (1ll << 31)) return false;
+  auto magic = [](int d) { return (uint32_t)(((1ull << 32) + d - 1) / (uint64_t)d); };
+  take_narrow(w, a);
+  a->stem_pw = (int)pw;
+  a->magic_c16 = magic((int)(pw / 4));
+  a->magic_ow = magic(a->ow);
+  a->pstep_pix = rows;
+  a->pstep_n = tiles;
+  a->magic_oh = magic(tiles);
+  a->n_tiles = a->n * tiles;
+  a->tiles_per_xcd = (a->n_tiles + 7) / 8;
+  *lds = (unsigned)bytes(rows);
+  return true;
+}
+
 static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y,
                     const PostOps &post) {
   if (w->fc_only) {
@@ -5502,6 +5684,22 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
     // segment) tiles
     const int64_t tiles = (int64_t)a.n * a.oh * ((a.ow + 127) / 128);
     const bool k3 = a.kh <= 3, one = a.oc <= 32;
+    unsigned lds = 0;
+    if (stem_rows_plan(ctx, w, &a, &lds)) {
+      auto go = [&](auto kernel) {
+        const dim3 wgs((unsigned)a.tiles_per_xcd * 8);
+        if (ctx->prof_start)
+          hipExtLaunchKernelGGL(kernel, wgs, dim3(256), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
+        else
+          hipLaunchKernelGGL(kernel, wgs, dim3(256), lds, ctx->stream, a);
+      };
+      if (k3 && one) go(conv_stem_rows_kernel<3, 1, 2>);
+      else if (k3) go(conv_stem_rows_kernel<3, 2, 2>);
+      else if (one) go(conv_stem_rows_kernel<7, 1, 2>);
+      else go(conv_stem_rows_kernel<7, 2, 2>);
+      TPUHIP_CHECK_HIP(hipGetLastError());
+      return TPUHIP_OK;
+    }
     const int64_t per_xcd = (tiles + 7) / 8;
     const dim3 grid((unsigned)(8 * std::min<int64_t>(per_xcd, std::max(1, ctx->num_cu * 3 / 8)))), block(256);
 #define STEM(KH, TM)                                                                   \
