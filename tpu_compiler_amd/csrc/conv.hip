@@ -85,7 +85,6 @@ struct ConvArgs {
   // requantisation's 64-bit multiply-add; qc64r = qc64 + 2^(rshift-1) * 2^31, which also carries
   // the rounding term of the right shift (layers with a fused ReLU)
   const int32_t *qc64, *qc64r;
-  int narrow;      // qc64, qc64r, qmult, qshift, qhpot are the planes of requant_rows_narrow
   int8_t *y;
   int n, ih, iw, x_cs;
   int oh, ow, y_cs;
@@ -109,6 +108,7 @@ struct ConvArgs {
   uint32_t magic_pw;      // floor(2^20 / stem_pw) + 1
   int lo;          // lower clamp bound: 0 with ReLU after saturation, else -128
   int relu_first;  // ReLU on the sum before requantisation (FC)
+  int narrow;      // qc64, qc64r, qmult, qshift, qhpot are the planes of requant_rows_narrow
   // optional fused eltwise add on the conv result (same shape and channel stride as y):
   // add_dst = sat8(floor(relu?(add_src * add_m_src + y * add_m_conv) / 2^add_rshift + 0.5))
   const int8_t *add_src;
@@ -120,14 +120,14 @@ struct ConvArgs {
   // from split_oc on (a multiple of 128, 0 = no second conv) belong to the second one and
   // go to y2 with its own channel stride and ReLU
   int split_oc, y2_cs, lo2;
+  int slope_m;            // see has_lut
   int8_t *y2;
   // optional fused 256-entry table on the conv result, applied before the fused add:
   // lut_dst (may be null) receives table[y]; the add then takes table[y]
-  int has_lut;
-  int8_t *lut_dst;
   // a table that is max(y, (y * slope_m + 2^(slope_r - 1)) >> slope_r) (a leaky ReLU's) is computed instead: slope_m > 0,
-  // has_lut 0, the rest as with a table
-  int slope_m, slope_r;
+  // has_lut 0, the rest as with a table.  (Numbers between pointers stand in pairs.)
+  int has_lut, slope_r;
+  int8_t *lut_dst;
   Table256 lut;
 #ifdef TPUHIP_TRACE
   unsigned long long *trace;   // development builds: 32 shader-clock stamps per workgroup
