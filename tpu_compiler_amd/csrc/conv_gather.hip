@@ -371,9 +371,8 @@ uint32_t magic_of(int d) { return d == 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1
 
 int floor_div(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
 
-// The patch kernel's tiles, where the layer is the patch kernel's; rows stays 0 elsewhere.  It needs several phases that one
-// workgroup of at most 16 waves computes (nine without a common row of 64 pixels, zeros of 3 x 3, still fit) and their patch in
-// LDS.  Fewer than eight slices are in flight at once without it, and nothing is shared: 64 -> 64 channels, 2x2 on
+// The patch kernel's tiles, where the layer is the patch kernel's; rows stays 0 elsewhere.  It needs several phases, at most
+// 16 waves of 64 pixels for one row of all of them, and their patch in LDS.  Fewer than eight slices are in flight at once without it, and nothing is shared: 64 -> 64 channels, 2x2 on
 // 2 x 40 x 40 3.8 us, in the patch kernel 4.0; eight, 64 -> 64, 4x4 on 20 x 30, 4.2 -> 3.8.  Of eight to twelve slices it keeps
 // those of many pixels: 6 x 100 x 90 16.3 us against 17.3, 4 x 100 x 90 13.0 -> 12.1.
 // The rows of a tile: fewest groups of 64 pixels on the busiest CU, a tile's start counted as one more.  (4 x 128 x 45 x 53:
