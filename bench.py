@@ -185,10 +185,11 @@ def main():
             args.tiles = recorded
     if args.tiles:
         from tpu_compiler_amd import capi
-        # (some numbers below the last variant's name none)
-        tile_names = [(capi.bind().tpuhip_conv2d_tile_name(i) or b"").decode() for i in range(256)]
+        tile_names = []
+        while capi.bind().tpuhip_conv2d_tile_name(len(tile_names)):
+            tile_names.append(capi.bind().tpuhip_conv2d_tile_name(len(tile_names)).decode())
         for name, algo in json.load(open(args.tiles)).items():
-            if algo and algo in tile_names:
+            if algo in tile_names:
                 g.by_name[name].attrs["algo"] = 16 + tile_names.index(algo)
     m = module(device=0)
     m.set_option("keep_all_tensors", 1 if args.keep_all else 0)

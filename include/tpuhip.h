@@ -267,8 +267,7 @@ const char *tpuhip_conv2d_chain_variant_name(int variant);
 int tpuhip_conv2d_set_input_stride(tpuhip_conv_weights *w, int x_cs);
 /* name of the kernel variant a prepacked conv dispatches to (for profiling) */
 const char *tpuhip_conv2d_algo_name(const tpuhip_conv_weights *w);
-/* name of MFMA tile variant `tile` (selected with algo = 16 + tile); NULL where there is none: past the last one, 83 today,
- * and for 64 to 71 */
+/* name of MFMA tile variant `tile` (selected with algo = 16 + tile), NULL past the last one */
 const char *tpuhip_conv2d_tile_name(int tile);
 /* 1 when tpuhip_conv2d_post_i8 can apply a 256-entry table in this packed conv's epilogue: depthwise
  * and stem kernels always, a dense conv unless its tile variant is fixed (asked for by the caller, or

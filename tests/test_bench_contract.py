@@ -41,6 +41,16 @@ def test_recorded_tiles_name_layers_and_variants_that_exist():
         assert len(tiles) >= {"cfg3": 40, "cfg4": 30, "cfg5": 60}[cfg]      # every MFMA conv of the graph
 
 
+def test_tile_variants_are_numbered_without_a_gap():
+    """the header's promise: tpuhip_conv2d_tile_name is NULL past the last variant and nowhere before it"""
+    from tpu_compiler_amd import capi
+    lib = capi.bind()
+    names = [lib.tpuhip_conv2d_tile_name(t) for t in range(1024)]
+    last = max(t for t, name in enumerate(names) if name)
+    assert all(names[:last + 1]) and len(set(names[:last + 1])) == last + 1
+    assert lib.tpuhip_conv2d_tile_name(-1) is None
+
+
 def test_committed_traffic_figures_name_kernel_variants_the_library_still_has():
     """bench.py takes roofline.traffic from profiles/resnet50_b32_bench_traffic.json by kernel variant name:
     a variant renamed or removed in the library must not leave a stale entry behind"""

@@ -24,7 +24,9 @@ PATCH2_TILES = [t for t in range(NUM_TILES) if "mfma_patch2_" in capi_tile_name(
 PW_TILES = [t for t in range(NUM_TILES) if "_pw_" in capi_tile_name(t)]
 # their third form: the same layers again; the four waves of a pixel group split K
 PATCH3_TILES = [t for t in range(NUM_TILES) if "mfma_patch3_" in capi_tile_name(t)]
-GENERAL_TILES = [t for t in range(NUM_TILES) if t not in PATCH_TILES + PATCH2_TILES + PATCH3_TILES + PW_TILES]
+# their fourth form: 3x3 / pad 1 layers of either stride, only with constants that requantise on packed int16
+ROWS_TILES = [t for t in range(NUM_TILES) if "mfma_rows_" in capi_tile_name(t)]
+GENERAL_TILES = [t for t in range(NUM_TILES) if t not in PATCH_TILES + PATCH2_TILES + PATCH3_TILES + PW_TILES + ROWS_TILES]
 
 
 def tile_bn(tile):
@@ -696,7 +698,7 @@ def test_conv_random_shapes_every_tile_variant(ctx, seed):
         z_ref = O.eltwise_add_i8([other, want], [61, 47], [6], True)
         xt, ot = ctx.from_nchw(x), ctx.from_nchw(other)
         yt, zt = ctx.tensor(want.shape), ctx.tensor(want.shape)
-        for tile in GENERAL_TILES + PATCH_TILES + PATCH2_TILES + PATCH3_TILES + PW_TILES:
+        for tile in GENERAL_TILES + PATCH_TILES + PATCH2_TILES + PATCH3_TILES + PW_TILES + ROWS_TILES:
             d = conv_desc(x.shape, w.shape, stride=stride, pads=pads, dil=dil, do_relu=relu, algo=16 + tile)
             try:
                 wh = ctx.conv_prepack(d, w, f2i32(bias), f2i32(mult), f2i32(rsh))
@@ -722,6 +724,7 @@ def test_conv_random_shapes_every_tile_variant(ctx, seed):
         for t in (xt, ot, yt, zt):
             t.free()
     assert len(ran) >= 15, sorted(ran)
+    assert any("_rows_" in name for name in ran), sorted(ran)
 
 
 @pytest.mark.parametrize("tile", PATCH_TILES)
@@ -737,7 +740,16 @@ def test_conv_patch_tiles_refuse_other_layers(ctx, tile):
         with pytest.raises(capi.TpuHipError, match="3x3 / stride 1 / pad 1"):
             ctx.conv(wh, xt, yt)
         ctx.conv_weights_destroy(wh)
-    # nor do they run a pair
+    _refuse_a_pair(ctx, tile)
+
+
+@pytest.mark.parametrize("tile", ROWS_TILES)
+def test_conv_rows_tiles_refuse_a_pair(ctx, tile):
+    _refuse_a_pair(ctx, tile)
+
+
+def _refuse_a_pair(ctx, tile):
+    z = lambda oc, ic, k: (np.zeros((oc, ic, k, k), np.int8), None, np.full(oc, 1 << 30, np.int32), np.full(oc, 8, np.int32))
     da, db = conv_desc((1, 64, 8, 8), (128, 64, 3, 3), pads=(1, 1, 1, 1), algo=16 + tile), \
         conv_desc((1, 64, 8, 8), (16, 64, 3, 3), pads=(1, 1, 1, 1), algo=16 + tile)
     wp = ctx.conv_prepack_pair(da, db, z(128, 64, 3), z(16, 64, 3))

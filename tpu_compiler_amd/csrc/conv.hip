@@ -4114,26 +4114,25 @@ struct TileCfg {
 
 // row-patch kernels, fourth form (3x3 / stride 1 or 2 / pad 1, input channels a power of two from 128, 64 or 32 to 1024):
 // U4(index, name, waves along channels, along pixels, channel blocks and pixel blocks per wave, slices per group, slices in
-// flight, waves per SIMD).  Indices 64 to 71 are not used: the variants below them, without a gap from 0, are those that take
-// any dense conv or are one of the families before this one.  Each is the fastest of all at several of 190 shapes (stages of
+// flight, waves per SIMD).  Each is the fastest of all at several of 190 shapes (stages of
 // a detector of 320 to 608 pixels, 1 to 8 images, and of a residual classifier, 8 to 64 images); variants that came within 2 %
 // of another everywhere were left out.
 #define TPUHIP_ROWS_TILES(U4)                         \
-  U4(72, "mfma_rows_256x256", 4, 2, 2, 4, 4, 4, 2)    \
-  U4(73, "mfma_rows_256x160", 8, 1, 1, 5, 4, 8, 2)    \
-  U4(74, "mfma_rows_128x384", 4, 2, 1, 6, 4, 8, 2)    \
-  U4(75, "mfma_rows_128x192", 4, 2, 1, 3, 4, 4, 4)    \
-  U4(76, "mfma_rows_128x160", 4, 1, 1, 5, 4, 4, 3)    \
-  U4(77, "mfma_rows_128x128", 4, 1, 1, 4, 4, 8, 3)    \
-  U4(78, "mfma_rows_64x192", 2, 2, 1, 3, 4, 8, 4)     \
-  U4(79, "mfma_rows_128x160_c64", 4, 1, 1, 5, 2, 4, 3)\
-  U4(80, "mfma_rows_128x128_c64", 4, 1, 1, 4, 2, 4, 4)\
-  U4(81, "mfma_rows_64x320_c32", 2, 2, 1, 5, 1, 4, 3) \
-  U4(82, "mfma_rows_64x256_c32", 2, 2, 1, 4, 1, 4, 4) 
+  U4(64, "mfma_rows_256x256", 4, 2, 2, 4, 4, 4, 2)    \
+  U4(65, "mfma_rows_256x160", 8, 1, 1, 5, 4, 8, 2)    \
+  U4(66, "mfma_rows_128x384", 4, 2, 1, 6, 4, 8, 2)    \
+  U4(67, "mfma_rows_128x192", 4, 2, 1, 3, 4, 4, 4)    \
+  U4(68, "mfma_rows_128x160", 4, 1, 1, 5, 4, 4, 3)    \
+  U4(69, "mfma_rows_128x128", 4, 1, 1, 4, 4, 8, 3)    \
+  U4(70, "mfma_rows_64x192", 2, 2, 1, 3, 4, 8, 4)     \
+  U4(71, "mfma_rows_128x160_c64", 4, 1, 1, 5, 2, 4, 3)\
+  U4(72, "mfma_rows_128x128_c64", 4, 1, 1, 4, 2, 4, 4)\
+  U4(73, "mfma_rows_64x320_c32", 2, 2, 1, 5, 1, 4, 3) \
+  U4(74, "mfma_rows_64x256_c32", 2, 2, 1, 4, 1, 4, 4) 
 
 constexpr int kMaxTiles = 96;
 struct TileTable {
-  TileCfg t[kMaxTiles] = {};   // name NULL: no such variant
+  TileCfg t[kMaxTiles] = {};   // numbered from 0 without a gap: a caller finds the last one at the first name that is NULL
   int n = 0;
   TileTable() {
 #define X(i, name, P, BM, BN, WM, WN, BK, D, O) \
@@ -4774,7 +4773,6 @@ int patch_rows(const tpuhip_conv_desc &d, const TileCfg &c) {
 
 bool tile_is_candidate(const tpuhip_conv_desc &d, int t) {
   const TileCfg &c = kTiles[t];
-  if (!c.name) return false;
   if (c.reg == 9 && rows_plan(d, c).th == 0) return false;
   if (c.reg == 4 && patch_rows(d, c) == 0) return false;
   if (c.reg == 5 && !pw_shape_ok(d, c)) return false;
@@ -5282,7 +5280,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   if (algo >= 16) {   // MFMA with an explicit tile variant (tests, tuning)
     forced_tile = algo - 16;
     algo = ALGO_MFMA;
-    TPUHIP_REQUIRE(forced_tile < kNumTiles && kTiles[forced_tile].name, "conv: unknown MFMA tile %d", forced_tile);
+    TPUHIP_REQUIRE(forced_tile < kNumTiles, "conv: unknown MFMA tile %d", forced_tile);
   }
   // the stem kernel: one dword per pixel, the taps of a filter row side by side
   const bool stem_ok = dense && d.ic <= 4 && d.dh == 1 && d.dw == 1 && d.kw <= 8 && d.kh <= 7 &&
@@ -6010,7 +6008,7 @@ int tpuhip_fc_prepack(tpuhip_ctx *ctx, int m, int k, int n, int x_cs, int y_cs, 
   // (and so is a K beyond the conv kernels' reach, whatever the rows)
   if ((m <= 256 && (n + 31) / 32 * ((m + 31) / 32) <= kFcMaxTiles) || k > 4096) {
     for (int t = 0; t < kNumTiles; ++t)
-      if (kTiles[t].name && std::string(kTiles[t].name) == "mfma_reg_32x32") d.algo = 16 + t;
+      if (std::string(kTiles[t].name) == "mfma_reg_32x32") d.algo = 16 + t;
   }
   std::vector<int32_t> mult((size_t)n, multiplier), rs((size_t)n, rshift);
   return tpuhip_conv2d_prepack(ctx, &d, filter_nk, bias, mult.data(), rs.data(), out);
