@@ -269,6 +269,10 @@ int tpuhip_conv2d_set_input_stride(tpuhip_conv_weights *w, int x_cs);
 const char *tpuhip_conv2d_algo_name(const tpuhip_conv_weights *w);
 /* name of MFMA tile variant `tile` (selected with algo = 16 + tile), NULL past the last one */
 const char *tpuhip_conv2d_tile_name(int tile);
+/* 1 when the choice by timing tries variant `tile` on a dense conv of this shape on a device of num_cu compute units (the layer's
+ * constants and what is fused behind it may rule the variant out besides).  Asking for it with algo = 16 + tile is another
+ * matter: that is refused only where the variant cannot run the layer. */
+int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu);
 /* 1 when tpuhip_conv2d_post_i8 can apply a 256-entry table in this packed conv's epilogue: depthwise
  * and stem kernels always, a dense conv unless its tile variant is fixed (asked for by the caller, or
  * already chosen by timing) to one without a table stage.  The interpreter asks before it folds a

@@ -56,3 +56,31 @@ def test_host_side_tables_need_no_gpu():
     t = np.empty(256, np.int8)
     assert lib.tpuhip_leaky_relu_table(31, 1, 0, 1, t.ctypes.data) == capi.C.c_int(1).value
     assert b"rshift" in lib.tpuhip_last_error()
+
+
+def test_row_patch_variants_are_timed_only_on_layers_of_many_workgroups():
+    """which variants the choice by timing tries is a rule on shapes: host code"""
+    from gpu_helpers import conv_desc
+    lib = capi.bind()
+    names = []
+    while lib.tpuhip_conv2d_tile_name(len(names)):
+        names.append(lib.tpuhip_conv2d_tile_name(len(names)).decode())
+
+    def tried(n, ic, oc, h, w, s=1, num_cu=256):
+        d = conv_desc((n, ic, h, w), (oc, ic, 3, 3), stride=(s, s), pads=(1,) * 4)
+        return {m for t, m in enumerate(names) if lib.tpuhip_conv2d_tile_timed(d, t, num_cu)}
+
+    rows = lambda *a, **k: {m for m in tried(*a, **k) if "_rows_" in m}
+    # the 3x3 layers of a residual classifier and of a detector's late stages on one image: other forms only
+    for c, side in ((64, 56), (128, 28), (256, 14), (512, 7)):
+        assert not rows(1, c, c, side, side) and tried(1, c, c, side, side)
+        assert rows(64, c, c, side, side)
+    assert not rows(1, 256, 512, 38, 38) and not rows(1, 128, 256, 76, 76, 2)
+    # one workgroup per image row: 127 of them and 128; 63 on a device of 128 CUs, 64
+    assert "mfma_rows_128x128" not in rows(1, 128, 128, 127, 128) and "mfma_rows_128x128" in rows(1, 128, 128, 128, 128)
+    assert "mfma_rows_128x128" not in rows(1, 128, 128, 63, 128, num_cu=128)
+    assert "mfma_rows_128x128" in rows(1, 128, 128, 64, 128, num_cu=128)
+    assert not lib.tpuhip_conv2d_tile_timed(None, 0, 256)
+    d = conv_desc((1, 64, 8, 8), (64, 64, 3, 3), pads=(1,) * 4)
+    assert lib.tpuhip_conv2d_tile_timed(d, 0, 256) and not lib.tpuhip_conv2d_tile_timed(d, len(names), 256)
+    assert not lib.tpuhip_conv2d_tile_timed(d, -1, 256)

@@ -2147,8 +2147,8 @@ __global__ __launch_bounds__(256 * PW) void conv_patch3_kernel(ConvArgs a) {
 // waves per SIMD, 29.5 at two.
 // Against the fastest of the other forms, with leaky ReLU and add, 8 images: 32 -> 64 on 304 x 304 45.0 -> 38.2 us, 64 -> 128 on
 // 152 x 152 32.0 -> 24.2, 128 -> 256 on 76 x 76 25.4 -> 18.6, 256 -> 512 on 38 x 38 20.6 -> 16.5; stride 2, 128 -> 256 from
-// 152 x 152 24.6 -> 22.5; 64 -> 64 on 64 x 56 x 56 17.8 -> 13.3.  No faster: few pixels (one image below 200 x 200), and
-// stride 2 from maps whose three rows fill the LDS (608 x 32 channels).
+// 152 x 152 24.6 -> 22.5; 64 -> 64 on 64 x 56 x 56 17.8 -> 13.3.  No faster: fewer workgroups than
+// half the CUs (tile_is_candidate() leaves those out), and stride 2 from maps whose three rows fill the LDS (608 x 32 channels).
 //   a.pstep_pix = rows of a tile, a.pstep_n = tiles per image (a.magic_oh its ceil(2^32 / d)), a.pstep_oh = log2(C),
 //   a.magic_c16 = ceil(2^32 / 16-byte chunks of an input row), a.magic_pw = bytes of a patch row, a.tile_imgs = half (stride 2),
 //   a.pstep_ow = LDS bytes.  C: a power of two from 32 * G to 1024.
@@ -4114,9 +4114,9 @@ struct TileCfg {
 
 // row-patch kernels, fourth form (3x3 / stride 1 or 2 / pad 1, input channels a power of two from 128, 64 or 32 to 1024):
 // U4(index, name, waves along channels, along pixels, channel blocks and pixel blocks per wave, slices per group, slices in
-// flight, waves per SIMD).  Each is the fastest of all at several of 190 shapes (stages of
-// a detector of 320 to 608 pixels, 1 to 8 images, and of a residual classifier, 8 to 64 images); variants that came within 2 %
-// of another everywhere were left out.
+// flight, waves per SIMD).  Of 347 layers (profiles/conv_rows_tiles.txt) one of them is the fastest of all in 69: the 128x128 in
+// 25 (by up to 8 %), 64x256_c32 in 12 (18 %), 64x192 in 11 (11 %), 128x128_c64 in 6 (24 %), 64x320_c32 in 5 (21 %), 128x192 in 3
+// (12 %), 256x160 and 128x160_c64 in 2 (11 and 4 %), 256x256 in one (9 %); 128x384 and 128x160 lead once, by 1 % and less.
 #define TPUHIP_ROWS_TILES(U4)                         \
   U4(64, "mfma_rows_256x256", 4, 2, 2, 4, 4, 4, 2)    \
   U4(65, "mfma_rows_256x160", 8, 1, 1, 5, 4, 8, 2)    \
@@ -4771,9 +4771,17 @@ int patch_rows(const tpuhip_conv_desc &d, const TileCfg &c) {
   return (d.oh + tiles - 1) / tiles;
 }
 
-bool tile_is_candidate(const tpuhip_conv_desc &d, int t) {
+bool tile_is_candidate(const tpuhip_conv_desc &d, int t, int num_cu) {
   const TileCfg &c = kTiles[t];
-  if (c.reg == 9 && rows_plan(d, c).th == 0) return false;
+  if (c.reg == 9) {
+    // worth timing only where its workgroups take half the CUs: one holds rows x channels enough for a CU of its own, and with
+    // fewer of them than that the other forms spread the layer wider.  Of 347 layers (profiles/conv_rows_tiles.txt) no variant
+    // with fewer than 128 workgroups on 256 CUs came within 3 % of the fastest other form (64 -> 64 on 56 x 56, one image: 28
+    // workgroups 7.4 us against 3.9; 128 -> 128 on 28 x 28, four: 40, 7.8 against 6.0), up to 159 none beat it, and from 160 on
+    // they win: 128 -> 252 on 6 x 95 x 54 168 workgroups 15.0 us against 16.7
+    const int th = rows_plan(d, c).th;
+    if (th == 0 || 2 * (int64_t)d.n * ((d.oh + th - 1) / th) * ((d.oc + c.bm - 1) / c.bm) < num_cu) return false;
+  }
   if (c.reg == 4 && patch_rows(d, c) == 0) return false;
   if (c.reg == 5 && !pw_shape_ok(d, c)) return false;
   if (c.reg == 6 && patch2_rows(d, c) == 0) return false;
@@ -5096,8 +5104,8 @@ TileKey tile_key(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void
                  d.pb, d.pr};
 }
 
-bool tile_usable(const tpuhip_conv_weights *w, int t, const PostOps &post) {
-  if (!tile_is_candidate(w->d, t)) return false;
+bool tile_usable(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, int t, const PostOps &post) {
+  if (!tile_is_candidate(w->d, t, ctx->num_cu)) return false;
   if (post.lut && !tile_has_lds_epilogue(t)) return false;
   if (w->split_oc && kTiles[t].reg == 4) return false;   // the patch kernel writes one result
   if (kTiles[t].reg == 5 && (!w->fast || w->split_oc % kTiles[t].bm)) return false;
@@ -5152,7 +5160,7 @@ int autotune_mfma(tpuhip_ctx *ctx, tpuhip_conv_weights *w, const void *x, void *
   };
   float least = 1e30f;
   for (int t = 0; t < kNumTiles && !rc; ++t) {
-    ms_of[t] = tile_usable(w, t, post) ? time_tile(t, 5) : -1;
+    ms_of[t] = tile_usable(ctx, w, t, post) ? time_tile(t, 5) : -1;
     if (ms_of[t] >= 0) least = std::min(least, ms_of[t]);
   }
   float best_ms = 1e30f;
@@ -5463,6 +5471,10 @@ int tpuhip_conv2d_weights_destroy(tpuhip_ctx *ctx, tpuhip_conv_weights *w) {
 
 const char *tpuhip_conv2d_tile_name(int tile) {
   return tile >= 0 && tile < kNumTiles ? kTiles[tile].name : nullptr;
+}
+
+int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu) {
+  return desc && tile >= 0 && tile < kNumTiles && !check_desc(*desc) && tile_is_candidate(*desc, tile, num_cu) ? 1 : 0;
 }
 
 int tpuhip_conv2d_can_fuse_table(const tpuhip_conv_weights *w) {
