@@ -34,8 +34,14 @@ CASES = [
     (1, 512, 2, 1, 24, (2, 3), (1, 1), (0, 0, 1, 1), (1, 1), (1, 1), False, 0),         # a single result column
     (1, 256, 5, 101, 40, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # three rows of patch: 84 KB
     (1, 256, 3, 250, 36, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # no patch: the other kernel
-    (1, 64, 201, 200, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # 40200 pixels: the other kernel
+    (1, 64, 201, 200, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),
     (1, 64, 200, 200, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), False, 0),
+    (1, 64, 340, 340, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # many outputs: the other kernel
+    (1, 80, 96, 96, 16, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),         # one channel block: 36864 outputs
+    (1, 80, 96, 95, 16, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), False, 0),        # fewer: the other kernel
+    (2, 256, 33, 32, 70, (2, 2), (1, 1), (0, 1, 0, 1), (1, 1), (2, 2), True, 0),        # nine phases, some without a tap
+    (4, 128, 24, 49, 33, (4, 4), (1, 2), (3, 3, 3, 3), (2, 1), (2, 2), False, 0),       # nine phases, stride and dilation
+    (2, 112, 40, 35, 70, (6, 6), (1, 1), (4, 4, 4, 4), (1, 1), (2, 2), True, 0),        # fewer than 128 channels: the other kernel
 ]
 
 

@@ -372,9 +372,21 @@ uint32_t magic_of(int d) { return d == 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1
 int floor_div(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
 
 // The patch kernel's tiles, where the layer is the patch kernel's; rows stays 0 elsewhere.  It needs several phases, at most
-// 16 waves of 64 pixels for one row of all of them, and their patch in LDS.  Fewer than eight slices are in flight at once without it, and nothing is shared: 64 -> 64 channels, 2x2 on
-// 2 x 40 x 40 3.8 us, in the patch kernel 4.0; eight, 64 -> 64, 4x4 on 20 x 30, 4.2 -> 3.8.  Of eight to twelve slices it keeps
-// those of many pixels: 6 x 100 x 90 16.3 us against 17.3, 4 x 100 x 90 13.0 -> 12.1.
+// 16 waves of 64 pixels for one row of all of them, and their patch in LDS.  Fewer than eight slices are in flight at once
+// without it, and nothing is shared: 64 -> 64 channels, 2x2 on 2 x 40 x 40 3.8 us, in the patch kernel 4.0.
+// From eight slices on, of 2482 layers (profiles/conv_transposed_kernels.txt: 2 to 16 phases, 32 to 512 channels to 24 to 256):
+//   * four phases and fewer: faster in the patch kernel (4x4, 128 -> 128 on 8 x 45 x 53 14.7 us, without 23.2; 2x2, 352 -> 24 on
+//     250 x 250 10.5 and 25.2), but for two kinds.  A layer of a single block of 32 channels and few outputs has less to fetch
+//     without the patch, whose first row waits for the last (4x4, 64 -> 24 on 45 x 53 4.4 us, 5.0 with it; eight images of it 7.1
+//     and 6.3) -- not where positions lie 128 bytes apart or a multiple, which the gathering loads are slower from (128 -> 24
+//     on 45 x 53 5.8 and 5.7, 192 -> 24 5.7 and 6.2).
+//     And where the chip is filled many times over, a patch's way into LDS is paid by every block of channels and no wait is
+//     left to save: fewer than twelve slices of fewer than 128 channels (4x4, 64 -> 128 on 8 x 100 x 90 35.0 us, 39.4 with it);
+//   * more phases: a workgroup has a wave for each, so that its tiles hold a few pixels, which the same many rows of patch are
+//     fetched for.  6x6 to three times the size, 64 -> 64 on 16 x 60 x 60 31.1 us, 39.1 with it.  The patch is faster on many
+//     outputs and from 128 channels (128 -> 64: 54.2 us, 44.7 with it) or 16 slices on.
+// By that line (few: 144 outputs x blocks a CU; many: 1800) the layers take 0.4 % longer than with the faster kernel each, at
+// most 1.34 times; all in the patch kernel 2.0 % and 1.63, none 22 % and 3.6.
 // The rows of a tile: fewest groups of 64 pixels on the busiest CU, a tile's start counted as one more.  (4 x 128 x 45 x 53:
 // three rows 8.0 us, one 8.9, two 9.7, four 9.3; 4 x 256 x 30 x 30: one 12.2, two and four 8.8.)
 void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
@@ -406,10 +418,15 @@ void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
   if (!taps_max || row_min < -30000 || col_min < -30000) return;
   const int n16 = (round_up(d.ic, 16)) / 16, slices = (taps_max * n16 + 1) / 2;
   const int entries = 2 * (round_up(slices, 4) + 4), phases = nh * nw;
-  if (entries * phases > kMaxEntries || slices < 8 || (slices < 12 && (int64_t)d.n * qh * qw > 40000)) return;
+  if (entries * phases > kMaxEntries || slices < 8) return;
+  const int blocks = (d.oc + 31) / 32;
+  const int64_t work = (int64_t)d.n * d.oh * d.ow * blocks;
+  const bool few = work < 144 * (int64_t)ctx->num_cu, many = work > 1800 * (int64_t)ctx->num_cu;
+  if (phases <= 4 ? (few && blocks == 1 && d.x_cs % 128) || (many && slices < 12 && d.x_cs < 128)
+                  : few || (slices < 16 && d.x_cs < 128))
+    return;
   const int prow = d.x_cs + (d.x_cs % 32 ? 0 : 16);   // an odd number of 16 bytes: the lanes of a fragment spread over the banks
   const int64_t cols = (int64_t)(qw - 1) * step_w + col_max - col_min + 1, span = row_max - row_min + 1;
-  const int blocks = (d.oc + 31) / 32;
   int64_t best = INT64_MAX;
   for (int rows = 1; rows <= qh; ++rows) {
     const int64_t lds = 3 * 32 * 4 + (int64_t)phases * entries * 4 + ((rows - 1) * (int64_t)step_h + span) * cols * prow;
