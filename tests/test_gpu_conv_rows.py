@@ -1,5 +1,5 @@
 """The fourth form of the row-patch kernel, every variant: stride 1 and 2, maps that leave slots, rows and channel blocks over,
-maps as wide as the tile, patches of more than one pass, with an add and a table behind them."""
+maps as wide as the tile, patches of more than one pass, with an add, a table, and a leaky ReLU that is computed behind them."""
 import numpy as np
 import pytest
 
@@ -49,7 +49,7 @@ WIDE = {160: [(1, 64, 3, 160, 40, 1, True), (1, 32, 5, 319, 40, 2, False)], 256:
 
 @pytest.mark.parametrize("tile,case", [(t, c) for t in ROWS_TILES for c in CASES + WIDE.get(_bn(t), []) if -(-c[3] // c[5]) <= _bn(t) and c[1] % _channels(t) == 0],
                          ids=lambda v: _name(v) if isinstance(v, int) else "x".join(map(str, v)))
-@pytest.mark.parametrize("post", ["plain", "add", "table_add"])
+@pytest.mark.parametrize("post", ["plain", "add", "table_add", "line", "line_add"])
 def test_against_the_oracle(ctx, tile, case, post):
     n, ic, ih, iw, oc, s, relu = case
     rng = np.random.default_rng(ic + ih * 3 + oc + s)
@@ -71,12 +71,22 @@ def test_against_the_oracle(ctx, tile, case, post):
         elif post == "add":
             ctx.conv_add(wh, xt, yt, ot, zt, 61, -47, 6, True)
             checks.append((zt, O.eltwise_add_i8([other, y_ref], [61, -47], [6], True)))
-        else:
+        elif post == "table_add":
             table = rng.integers(-128, 128, 256).astype(np.int8)
             table[0] = 77                                  # pad channels must stay 0 all the same
             t_ref = O.lut_i8(y_ref, table)
             ctx.conv_post(wh, xt, yt, table, tt, (ot, zt, 37, 51, 5, False))
             checks += [(tt, t_ref), (zt, O.eltwise_add_i8([other, t_ref], [37, 51], [5], False))]
+        else:
+            v = np.arange(256).astype(np.int8).astype(int)
+            table = np.maximum(v, (v * 13 + 64) >> 7).astype(np.int8)      # leaky ReLU of 13 / 128: computed
+            t_ref = O.lut_i8(y_ref, table)
+            if post == "line":
+                ctx.conv_post(wh, xt, None, table, tt)
+                checks = [(tt, t_ref)]
+            else:            # the residual blocks of a detector: only the sum is kept
+                ctx.conv_post(wh, xt, None, table, None, (ot, zt, 37, 51, 5, False))
+                checks = [(zt, O.eltwise_add_i8([other, t_ref], [37, 51], [5], False))]
     except capi.TpuHipError as e:     # a row of the patch beyond the LDS
         assert "tile variant" in str(e) and (s + 2) * iw * (ic + 16) > 140 << 10, str(e)
         checks = []

@@ -30,7 +30,8 @@ TABLES = {"0.1": _line(13, 7), "102/1024": _line(102, 10), "nothing": _line(1, 9
           "one below": _line(13, 7, 200), "last": _line(13, 7, 128), "positive": _line(13, 7, 100), "zero": _line(13, 7, 0)}
 # algorithm or tile name, channels, kernel
 FORMS = [("mfma_p_64x64", 48, 72, 3), ("mfma_pw_64x128_k64", 64, 72, 1), ("mfma_patch2_64x128", 64, 72, 3),
-         ("mfma_patch3_32x128", 64, 40, 3), ("mfma_ksplit_32x32_w8", 48, 41, 3), ("depthwise", 40, 40, 3),
+         ("mfma_patch3_32x128", 64, 40, 3), ("mfma_rows_64x192", 128, 72, 3), ("mfma_rows_128x160_c64", 64, 72, 3),
+         ("mfma_rows_256x256", 128, 290, 3), ("mfma_rows_64x256_c32", 32, 72, 3), ("mfma_ksplit_32x32_w8", 48, 41, 3), ("depthwise", 40, 40, 3),
          ("depthwise_dot", 40, 40, 3), ("depthwise", 24, 24, 5), ("stem", 3, 33, 3)]
 
 
@@ -39,7 +40,7 @@ FORMS = [("mfma_p_64x64", 48, 72, 3), ("mfma_pw_64x128_k64", 64, 72, 1), ("mfma_
 def test_conv_with_a_line_behind_it(ctx, form, table):
     name, ic, oc, k = form
     dw = name.startswith("depthwise")
-    tiles = {ctx.lib.tpuhip_conv2d_tile_name(t).decode(): t for t in range(64) if ctx.lib.tpuhip_conv2d_tile_name(t)}
+    tiles = {ctx.lib.tpuhip_conv2d_tile_name(t).decode(): t for t in range(256) if ctx.lib.tpuhip_conv2d_tile_name(t)}
     algo = {"depthwise": capi.ALGO_DEPTHWISE, "depthwise_dot": capi.ALGO_DEPTHWISE_DOT, "stem": 5}.get(name, 16 + tiles.get(name, 0))
     rng = np.random.default_rng(ic + k)
     x = rng.integers(-128, 128, (2, ic, 13, 11)).astype(np.int8)

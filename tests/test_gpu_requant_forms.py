@@ -18,7 +18,7 @@ def ctx():
 
 
 def _tile(ctx, name):
-    return next(16 + t for t in range(64) if ctx.lib.tpuhip_conv2d_tile_name(t) == name.encode())
+    return next(16 + t for t in range(256) if ctx.lib.tpuhip_conv2d_tile_name(t) == name.encode())
 
 
 # multipliers with the trailing zeros of a float (1.0, the smallest and largest normal ones, a power of two that makes ties),
@@ -30,6 +30,8 @@ SHIFTS = {"fits": [2, 3, 8, 9, 10, 11, 15, 16], "one": [1, 2, 9, 9, 10, 11, 15, 
 FORMS = [("mfma_p_64x64", 64, 3), ("mfma_64x64_k128", 48, 1), ("mfma_64x128_k128", 80, 3), ("mfma_p_32x128", 3, 3),
          ("mfma_pw_64x128_k64", 64, 1), ("mfma_pw_128x64_k256_w8", 256, 1), ("mfma_patch2_64x128", 64, 3),
          ("mfma_patch3_32x128", 64, 3), ("depthwise", 64, 3), ("depthwise", 64, 1)]
+# these run no other form: a layer with a channel that does not fit is refused (test_gpu_conv_rows)
+NARROW_ONLY = [("mfma_rows_128x128_c64", 64, 3), ("mfma_rows_64x192", 128, 3), ("mfma_rows_64x320_c32", 32, 3)]
 
 
 def _layer(ic, oc, k, dw, shifts, seed):
@@ -48,9 +50,9 @@ def _layer(ic, oc, k, dw, shifts, seed):
     return w.astype(np.int8), bias.astype(np.float32), rsh, mult
 
 
-@pytest.mark.parametrize("shifts", sorted(SHIFTS))
+@pytest.mark.parametrize("form,shifts", [(f, s) for f in FORMS for s in sorted(SHIFTS)] + [(f, "fits") for f in NARROW_ONLY],
+                         ids=lambda f: "%s_%d_%d" % f if isinstance(f, tuple) else f)
 @pytest.mark.parametrize("relu", [False, True])
-@pytest.mark.parametrize("form", FORMS, ids=lambda f: "%s_%d_%d" % f)
 def test_rounding_and_saturation(ctx, form, relu, shifts):
     name, ic, k = form
     dw = name == "depthwise"
@@ -120,3 +122,37 @@ def test_stem_and_pool(ctx, shifts):
     best = np.max([padded[:, :, i:i + 13:2, j:j + 13:2] for i in range(3) for j in range(3)], axis=0)
     assert np.array_equal(ctx.to_nchw(pt), best)
     ctx.conv_weights_destroy(wh)
+
+
+@pytest.mark.parametrize("shifts", [("fits", "fits"), ("fits", "one"), ("one", "fits"), ("beyond", "fits")])
+@pytest.mark.parametrize("triple", [(64, 256, 64), (128, 512, 128)])
+@pytest.mark.parametrize("form", ["residual", "kept", "no add"])
+def test_two_convs_in_one_launch(ctx, triple, shifts, form):
+    """a pointwise conv, an add and another pointwise conv: each conv requantises in its own form"""
+    ic, oc1, oc2 = triple
+    n, h, w_ = 2, 9, 11
+    (wa, ba, ra, ma), (wb, bb, rb, mb) = _layer(ic, oc1, 1, False, shifts[0], ic), _layer(oc1, oc2, 1, False, shifts[1], oc1)
+    # of every eight channels the multipliers move on by one with the shifts: all of SHIFTS are in either conv
+    assert {int(v) for v in ra} == set(SHIFTS[shifts[0]]) and {int(v) for v in rb} == set(SHIFTS[shifts[1]])
+    relu_a, relu_b = form == "kept", form != "kept"
+    pw = lambda x, w, b, r, m, relu: O.conv2d_i8(x, w, b, r, m, O.make_conv_desc(x.shape, w.shape, 1, (1, 1), (0,) * 4, (1, 1), (0, 0),
+                                                                                 relu, True, None))
+    rng = np.random.default_rng(oc1 + 1)
+    x = rng.integers(-128, 128, (n, ic, h, w_)).astype(np.int8)
+    other = rng.integers(-128, 128, (n, oc1, h, w_)).astype(np.int8)
+    ya = pw(x, wa, ba, ra, ma, relu_a)
+    mid = ya if form == "no add" else O.eltwise_add_i8([other, ya], [61, 47], [6], True)
+    yb = pw(mid, wb, bb, rb, mb, relu_b)
+    assert {127, 0 if relu_a else -128} <= set(np.unique(ya)) and {127, 0 if relu_b else -128} <= set(np.unique(yb))
+    ch = ctx.conv_chain_prepack(conv_desc(x.shape, wa.shape, do_relu=relu_a), conv_desc(ya.shape, wb.shape, do_relu=relu_b),
+                                (wa, f2i32(ba), f2i32(ma), f2i32(ra)), (wb, f2i32(bb), f2i32(mb), f2i32(rb)))
+    xt, ot, yat, zt, ybt = ctx.from_nchw(x), ctx.from_nchw(other), ctx.tensor(ya.shape), ctx.tensor(ya.shape), ctx.tensor(yb.shape)
+    for t in (yat, zt, ybt):
+        ctx._ck(ctx.lib.tpuhip_memset(ctx.h, t.ptr, 0x55, t.nbytes))
+    ctx.conv_chain(ch, xt, ybt, yat if form == "kept" else None, None if form == "no add" else (ot, zt, 61, 47, 6, True))
+    assert np.array_equal(ctx.to_nchw(ybt), yb)
+    assert form != "kept" or np.array_equal(ctx.to_nchw(yat), ya)
+    assert form == "no add" or np.array_equal(ctx.to_nchw(zt), mid)
+    ctx.conv_chain_destroy(ch)
+    for t in (xt, ot, yat, zt, ybt):
+        t.free()
