@@ -41,6 +41,15 @@ struct __attribute__((aligned(16))) QParam {
   int32_t hpot;   // 2^(rshift-1), 0 for rshift 0
 };
 
+// the tiles of conv_stem_rows_kernel
+struct StemRows {
+  int rows = 0;                 // result rows of a tile; 0: the other stem kernel's layer
+  int tiles = 0;                // tiles of an image
+  int pw = 0;                   // dwords of a patch row
+  unsigned lds = 0;
+  uint32_t magic_chunks = 0, magic_ow = 0, magic_tiles = 0;   // ceil(2^32 / x) of 16-byte chunks of a patch row, columns, tiles
+};
+
 struct tpuhip_conv_weights {
   tpuhip_conv_desc d;
   int algo = ALGO_DIRECT;
@@ -73,6 +82,7 @@ struct tpuhip_conv_weights {
   int kp = 0;            // padded K in bytes (row stride of w) for the MFMA path
   int c16 = 0;           // input 16-channel groups per tap
   int k16 = 0;           // 16-byte K groups in total
+  StemRows stem_rows;    // the stem path: the row form's tiles, where that takes the layer
 };
 
 struct ConvArgs {
@@ -5266,6 +5276,44 @@ int tpuhip::expand_params(tpuhip_ctx *ctx, const ParamExpand *list, size_t n, in
   return TPUHIP_OK;
 }
 
+// conv_stem_rows_kernel's tiles and its patch's pitch and LDS; rows stays 0: the other stem kernel's layer.  The rows of a tile:
+// rounds of resident workgroups, times the passes of their four waves and two more for a tile's start.  (8 x 608 x 608: 5 rows, 2
+// to 5 take 39 to 40.5 us; 64 x 112 x 112: 7 rows 12.6, 2 15.9, 14 13.9; 32 x 112 x 112 of 7x7: 7 rows 18.0, 3 24; one image: 1.)
+static StemRows stem_rows_plan(const tpuhip_ctx *ctx, const tpuhip_conv_desc &d) {
+  StemRows p;
+  if (d.pl > kStemPad || d.ow == 1 || d.ow > 16384) return p;
+  const int tm = d.oc <= 32 ? 1 : 2, per_cu = stem_waves(d.kh <= 3 ? 3 : 7, tm);
+  // up to a round and a half of the other kernel's workgroups of 128 pixels it is done sooner: 1 x 320 x 320 5.4 us against 6.0,
+  // 8 x 101 x 101 results 5.05 against 5.6; 1 x 416 x 416 7.9, here 6.9, 8 x 112 x 112 of 64 channels 8.9, here 7.3
+  if (2 * tm * (int64_t)d.n * d.oh * ((d.ow + 127) / 128) <= 9 * (int64_t)ctx->num_cu) return p;
+  // from kStemPad dwords in front of the image to the last one that the last column's taps (and the zeros behind them) meet
+  const int64_t pw = ((int64_t)(d.ow - 1) * d.sw + kStemPad - d.pl + 8 + 3) / 4 * 4;
+  auto bytes = [&](int rows) { return 5 * tm * 32 * 4 + 256 + ((int64_t)(rows - 1) * d.sh + d.kh) * pw * 4; };
+  int rows = 0;
+  uint32_t best = UINT32_MAX;
+  const uint32_t slots = (uint32_t)(ctx->num_cu * per_cu);
+  for (int r = 1; r <= std::min(d.oh, 8) && bytes(r) <= std::min(64, 160 / per_cu) * 1024; ++r) {
+    const uint32_t tiles = (uint32_t)d.n * (uint32_t)((d.oh + r - 1) / r);
+    const uint32_t cost = (tiles + slots - 1) / slots * (uint32_t)((r * d.ow + 255) / 256 + 2);
+    if (cost < best) {
+      best = cost;
+      rows = r;
+    }
+  }
+  if (!rows) return p;
+  const int tiles = (d.oh + rows - 1) / rows;
+  if ((int64_t)d.n * tiles * tiles >= (1ll << 32) || (int64_t)rows * d.ow * d.y_cs >= (1ll << 31)) return p;
+  auto magic = [](int v) { return (uint32_t)(((1ull << 32) + v - 1) / (uint64_t)v); };
+  p.rows = rows;
+  p.tiles = tiles;
+  p.pw = (int)pw;
+  p.lds = (unsigned)bytes(rows);
+  p.magic_chunks = magic((int)(pw / 4));
+  p.magic_ow = magic(d.ow);
+  p.magic_tiles = magic(tiles);
+  return p;
+}
+
 extern "C" {
 
 int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const int8_t *filter,
@@ -5454,6 +5502,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   cw->qp = records ? (QParam *)(p + nparam) : nullptr;
   cw->qplanes = p + at_planes;
   (narrow ? cw->qnarrow : cw->qc64) = p + at_last;
+  if (algo == ALGO_STEM && narrow) cw->stem_rows = stem_rows_plan(ctx, d);
   *out = cw;
   return TPUHIP_OK;
 }
@@ -5550,46 +5599,6 @@ static void dw_rows_walk(DwRowsArgs *r, unsigned wgs, int n_cb) {
     r->start_rb[x] = (int)((b / r->xblocks) % r->rblocks);
     r->start_n[x] = (int)(b / ((int64_t)r->xblocks * r->rblocks));
   }
-}
-
-// conv_stem_rows_kernel's tiles and its patch's pitch and LDS; false: the other stem kernel's layer.  The rows of a tile: rounds
-// of resident workgroups, times the passes of their four waves and two more for a tile's start.  (8 x 608 x 608: 5 rows, 2 to 5
-// take 39 to 40.5 us; 64 x 112 x 112: 7 rows 12.6, 2 15.9, 14 13.9; 32 x 112 x 112 of 7x7: 7 rows 18.0, 3 24; one image: 1 row.)
-static bool stem_rows_plan(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, ConvArgs *a, unsigned *lds) {
-  if (!w->qnarrow || w->split_oc || a->add_dst || a->pl > kStemPad || a->ow == 1 || a->ow > 16384) return false;
-  const int tm = a->oc <= 32 ? 1 : 2, per_cu = stem_waves(a->kh <= 3 ? 3 : 7, tm);
-  // up to a round and a half of the other kernel's workgroups of 128 pixels it is done sooner: 1 x 320 x 320 5.4 us against 6.0,
-  // 8 x 101 x 101 results 5.05 against 5.6; 1 x 416 x 416 7.9, here 6.9, 8 x 112 x 112 of 64 channels 8.9, here 7.3
-  if (2 * tm * (int64_t)a->n * a->oh * ((a->ow + 127) / 128) <= 9 * (int64_t)ctx->num_cu) return false;
-  // from kStemPad dwords in front of the image to the last one that the last column's taps (and the zeros behind them) meet
-  const int64_t pw = ((int64_t)(a->ow - 1) * a->sw + kStemPad - a->pl + 8 + 3) / 4 * 4;
-  auto bytes = [&](int rows) { return 5 * tm * 32 * 4 + 256 + ((int64_t)(rows - 1) * a->sh + a->kh) * pw * 4; };
-  int rows = 0;
-  uint32_t best = UINT32_MAX;
-  const uint32_t slots = (uint32_t)(ctx->num_cu * per_cu);
-  for (int r = 1; r <= std::min(a->oh, 8) && bytes(r) <= std::min(64, 160 / per_cu) * 1024; ++r) {   // (at every launch: 0.1 us)
-    const uint32_t tiles = (uint32_t)a->n * (uint32_t)((a->oh + r - 1) / r);
-    const uint32_t cost = (tiles + slots - 1) / slots * (uint32_t)((r * a->ow + 255) / 256 + 2);
-    if (cost < best) {
-      best = cost;
-      rows = r;
-    }
-  }
-  if (!rows) return false;
-  const int tiles = (a->oh + rows - 1) / rows;
-  if ((int64_t)a->n * tiles * tiles >= (1ll << 32) || (int64_t)rows * a->ow * a->y_cs >= (1ll << 31)) return false;
-  auto magic = [](int d) { return (uint32_t)(((1ull << 32) + d - 1) / (uint64_t)d); };
-  take_narrow(w, a);
-  a->stem_pw = (int)pw;
-  a->magic_c16 = magic((int)(pw / 4));
-  a->magic_ow = magic(a->ow);
-  a->pstep_pix = rows;
-  a->pstep_n = tiles;
-  a->magic_oh = magic(tiles);
-  a->n_tiles = a->n * tiles;
-  a->tiles_per_xcd = (a->n_tiles + 7) / 8;
-  *lds = (unsigned)bytes(rows);
-  return true;
 }
 
 static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y,
@@ -5694,14 +5703,22 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
     // segment) tiles
     const int64_t tiles = (int64_t)a.n * a.oh * ((a.ow + 127) / 128);
     const bool k3 = a.kh <= 3, one = a.oc <= 32;
-    unsigned lds = 0;
-    if (stem_rows_plan(ctx, w, &a, &lds)) {
+    if (const StemRows &p = w->stem_rows; p.rows) {
+      take_narrow(w, &a);
+      a.stem_pw = p.pw;
+      a.magic_c16 = p.magic_chunks;
+      a.magic_ow = p.magic_ow;
+      a.pstep_pix = p.rows;
+      a.pstep_n = p.tiles;
+      a.magic_oh = p.magic_tiles;
+      a.n_tiles = a.n * p.tiles;
+      a.tiles_per_xcd = (a.n_tiles + 7) / 8;
       auto go = [&](auto kernel) {
         const dim3 wgs((unsigned)a.tiles_per_xcd * 8);
         if (ctx->prof_start)
-          hipExtLaunchKernelGGL(kernel, wgs, dim3(256), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
+          hipExtLaunchKernelGGL(kernel, wgs, dim3(256), p.lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
         else
-          hipLaunchKernelGGL(kernel, wgs, dim3(256), lds, ctx->stream, a);
+          hipLaunchKernelGGL(kernel, wgs, dim3(256), p.lds, ctx->stream, a);
       };
       if (k3 && one) go(conv_stem_rows_kernel<3, 1, 2>);
       else if (k3) go(conv_stem_rows_kernel<3, 2, 2>);
