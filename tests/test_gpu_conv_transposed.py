@@ -32,6 +32,9 @@ CASES = [
     (1, 64, 8, 9, 33, (4, 4), (1, 2), (3, 3, 3, 3), (2, 1), (2, 2), False, 0),          # nine phases, stride and dilation
     (2, 512, 1, 1, 40, (4, 4), (1, 1), (3, 3, 3, 3), (1, 1), (1, 1), True, 0),          # one pixel to 4 x 4
     (1, 512, 2, 1, 24, (2, 3), (1, 1), (0, 0, 1, 1), (1, 1), (1, 1), False, 0),         # a single result column
+    (1, 256, 1, 1, 40, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), (1, 1), False, 0),         # one phase of results: the other kernel
+    (3, 256, 5, 1, 70, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), (0, 1), True, 0),          # likewise, of one column
+    (2, 384, 1, 6, 24, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), (1, 0), False, 1),         # and of one row
     (1, 256, 5, 101, 40, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # three rows of patch: 84 KB
     (1, 256, 3, 250, 36, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),        # no patch: the other kernel
     (1, 64, 201, 200, 8, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), True, 0),

@@ -264,7 +264,7 @@ __global__ __launch_bounds__(1024) void conv_gather_patch_kernel(GatherPatchArgs
   int pat[NP];
 #pragma unroll
   for (int u = 0; u < NP; ++u) fetch(tid + u * nt, pv[u], pat[u]);
-  int32_t param = 0;
+  int32_t param = 0;   // (a workgroup has two waves at least: one per phase)
   if (tid < 96) param = a.planes[(tid >> 5) * a.nparam + blk * 32 + (tid & 31)];
   const int32_t *tab = reinterpret_cast<const int32_t *>(a.w + a.tab_at);
   const GatherPhase *phases = reinterpret_cast<const GatherPhase *>(a.w + a.phase_at);
@@ -393,13 +393,15 @@ void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
   const int sh = d.ins_h + 1, sw = d.ins_w + 1;
   const int ph = sh / std::gcd(sh, d.sh), pw = sw / std::gcd(sw, d.sw);
   const int step_h = ph * d.sh / sh, step_w = pw * d.sw / sw;
-  if (d.g != 1 || ph * pw == 1 || ph * pw > 64 || d.x_cs % 16 || d.x_cs > 4096 || step_h > 255 || step_w > 255) return;
+  // one phase of results -- no zeros that matter, or a result of one row or column across them -- shares its patch with none (and
+  // would leave the kernel a workgroup of one wave, which does not fetch all of its block's parameters)
+  const int nh = std::min(ph, d.oh), nw = std::min(pw, d.ow);
+  if (d.g != 1 || nh * nw == 1 || ph * pw > 64 || d.x_cs % 16 || d.x_cs > 4096 || step_h > 255 || step_w > 255) return;
   for (int v : {d.ih, d.iw, d.oh, d.ow, d.kh * d.dh, d.kw * d.dw, d.pt, d.pl})
     if (v >= 30000) return;
   if (d.y_cs > 65535 || (int64_t)d.ih * d.iw * d.x_cs >= (1ll << 31) - 1 || (int64_t)d.n * d.oh * d.ow >= (1ll << 31)) return;
   // what the taps of all phases reach
   int row_min = INT_MAX, row_max = INT_MIN, col_min = INT_MAX, col_max = INT_MIN, taps_max = 0;
-  const int nh = std::min(ph, d.oh), nw = std::min(pw, d.ow);
   const int qh = (d.oh + ph - 1) / ph, qw = (d.ow + pw - 1) / pw;
   for (int a = 0; a < nh; ++a)
     for (int b = 0; b < nw; ++b) {
