@@ -25,6 +25,7 @@ CASES = [
     (1, 48, 9, 33, 33, (4, 4), (1, 1), (2, 2, 2, 2), (1, 1), (1, 1), False, 0),         # six: the other kernel
     (3, 80, 6, 7, 16, (4, 4), (1, 1), (2, 1, 1, 2), (1, 1), (1, 1), True, 0),           # 5 groups of 16, odd result sizes
     (1, 136, 5, 6, 100, (3, 3), (1, 1), (1, 2, 1, 2), (1, 1), (1, 1), False, 0),        # taps 1, 2, 2, 4; an odd count of entries
+    (1, 144, 20, 40, 40, (3, 3), (1, 1), (1, 2, 1, 2), (1, 1), (1, 1), False, 0),       # likewise, many channels a slice
     (2, 272, 4, 9, 40, (3, 3), (1, 1), (0, 0, 0, 0), (1, 1), (1, 1), True, 0),          # 17 groups of 16
     (1, 256, 6, 5, 40, (2, 2), (1, 1), (0, 1, 0, 1), (1, 1), (2, 2), True, 0),          # phases without a tap
     (1, 128, 7, 6, 20, (4, 3), (1, 1), (2, 2, 1, 1), (1, 1), (1, 0), False, 0),         # two phases

@@ -5526,6 +5526,13 @@ int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu)
   return desc && tile >= 0 && tile < kNumTiles && !check_desc(*desc) && tile_is_candidate(*desc, tile, num_cu) ? 1 : 0;
 }
 
+int tpuhip_conv2d_gather_form(const tpuhip_conv_desc *desc, int num_cu, int *reach) {
+  if (!desc || num_cu <= 0 || check_desc(*desc)) return 0;
+  const bool inserted = desc->ins_h || desc->ins_w;
+  if (desc->algo != ALGO_AUTO || (!inserted && (desc->g == 1 || (desc->g == desc->ic && desc->g == desc->oc)))) return 0;
+  return gather_form(*desc, num_cu, reach);
+}
+
 int tpuhip_conv2d_can_fuse_table(const tpuhip_conv_weights *w) {
   if (!w) return 0;
   if (w->algo == ALGO_DEPTHWISE || w->algo == ALGO_DEPTHWISE_DOT || w->algo == ALGO_STEM) return 1;

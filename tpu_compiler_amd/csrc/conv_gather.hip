@@ -389,7 +389,7 @@ int floor_div(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
 // most 1.34 times; all in the patch kernel 2.0 % and 1.63, none 22 % and 3.6.
 // The rows of a tile: fewest groups of 64 pixels on the busiest CU, a tile's start counted as one more.  (4 x 128 x 45 x 53:
 // three rows 8.0 us, one 8.9, two 9.7, four 9.3; 4 x 256 x 30 x 30: one 12.2, two and four 8.8.)
-void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
+void patch_plan(int num_cu, const tpuhip_conv_desc &d, GatherPlan *g) {
   const int sh = d.ins_h + 1, sw = d.ins_w + 1;
   const int ph = sh / std::gcd(sh, d.sh), pw = sw / std::gcd(sw, d.sw);
   const int step_h = ph * d.sh / sh, step_w = pw * d.sw / sw;
@@ -423,7 +423,7 @@ void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
   if (entries * phases > kMaxEntries || slices < 8) return;
   const int blocks = (d.oc + 31) / 32;
   const int64_t work = (int64_t)d.n * d.oh * d.ow * blocks;
-  const bool few = work < 144 * (int64_t)ctx->num_cu, many = work > 1800 * (int64_t)ctx->num_cu;
+  const bool few = work < 144 * (int64_t)num_cu, many = work > 1800 * (int64_t)num_cu;
   if (phases <= 4 ? (few && blocks == 1 && d.x_cs % 128) || (many && slices < 12 && d.x_cs < 128)
                   : few || (slices < 16 && d.x_cs < 128))
     return;
@@ -436,7 +436,7 @@ void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
     const int64_t wgs = (int64_t)d.n * tiles * blocks;
     if (lds > kPatchLds || groups * phases > 16) break;
     if (wgs >= 65536 || tiles >= 65536 || cols > 30000) continue;
-    const int64_t cost = (wgs + ctx->num_cu - 1) / ctx->num_cu * (groups * phases + 1);
+    const int64_t cost = (wgs + num_cu - 1) / num_cu * (groups * phases + 1);
     if (cost >= best) continue;
     best = cost;
     g->rows = rows;
@@ -446,13 +446,6 @@ void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
     g->lds = (unsigned)lds;
   }
   if (!g->rows) return;
-  if (g->lds > 64 * 1024)
-    for (const void *kernel : {(const void *)conv_gather_patch_kernel<true>, (const void *)conv_gather_patch_kernel<false>})
-      if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPatchLds) != hipSuccess) {
-        (void)hipGetLastError();
-        g->rows = 0;
-        return;
-      }
   g->row_min = row_min;
   g->span = (int)span;
   g->col_min = col_min;
@@ -461,15 +454,22 @@ void patch_plan(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, GatherPlan *g) {
   g->max_entries = entries;
 }
 
-}  // namespace
+// A layer's plan, phases and tables, and its packed filter; filter NULL: all but the bytes of the filter.
+struct GatherLayer {
+  GatherPlan plan;
+  std::vector<GatherPhase> phases;
+  std::vector<std::vector<int2>> tabs;
+  std::vector<int8_t> w;
+};
 
-int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *filter, GatherPlan **out) {
-  *out = nullptr;
+// false: not the gather kernels' layer.  patch: whether it may go to the patch kernel
+bool gather_layer(int num_cu, const tpuhip_conv_desc &d, const int8_t *filter, bool patch, GatherLayer *out) {
   const int icg = d.ic / d.g, ocg = d.oc / d.g;
   const int sh = d.ins_h + 1, sw = d.ins_w + 1;
   const int ph = sh / std::gcd(sh, d.sh), pw = sw / std::gcd(sw, d.sw);
-  GatherPlan geo;
-  patch_plan(ctx, d, &geo);
+  *out = GatherLayer();
+  GatherPlan &geo = out->plan;
+  if (patch) patch_plan(num_cu, d, &geo);
   // without groups all blocks read the same input channels: two of them per wave halve the activation loads
   const int tm = d.g == 1 && d.oc > 32 && !geo.rows ? 2 : 1;
   const int blocks = round_up(d.oc, 32 * tm) / 32;
@@ -486,11 +486,12 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
   if (d.x_cs % 16 || ph * pw > 256 || (int64_t)d.kh * d.dh >= 30000 || (int64_t)d.kw * d.dw >= 30000 || d.ih >= 30000 ||
       d.iw >= 30000 || d.sh >= 256 || d.sw >= 256 || (int64_t)d.kh * d.kw * n16 + 2 > kMaxEntries ||
       (int64_t)blocks * ((int64_t)d.kh * d.kw * n16 + 2 * ph * pw) * 512 >= (1ll << 30))
-    return TPUHIP_OK;
+    return false;
 
-  std::vector<GatherPhase> phases;
-  std::vector<std::vector<int2>> tabs;
-  std::vector<int8_t> w;
+  auto &phases = out->phases;
+  auto &tabs = out->tabs;
+  auto &w = out->w;
+  size_t w_bytes = 0;
   int max_entries = 0, max_pixels = 0;
   struct Tap { int kh, kw, dy, dx; };
   for (int a = 0; a < std::min(ph, d.oh); ++a)
@@ -514,18 +515,21 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
       const int entries = (int)taps.size() * n16;
       p.slices = (entries + 1) / 2;
       p.magic_qw = magic_of(p.qw);
-      p.w = (uint32_t)w.size();
+      p.w = (uint32_t)w_bytes;
       std::vector<int2> tab;
       for (int e = 0; e < 2 * p.slices; ++e) {
-        const Tap t = e < entries ? taps[e / n16] : Tap{0, 0, 0, 0};
+        // the second half of an odd last slice: zeros in the filter, and the last real tap's position, which the patch holds
+        // whatever taps the phase has
+        const Tap t = taps[std::min(e, entries - 1) / n16];
         int2 v;
         v.x = (int)(((int64_t)t.dy * d.iw + t.dx) * d.x_cs) + (e < entries ? e % n16 : 0) * 16;
         v.y = (int)(((uint32_t)t.dy << 16) | ((uint32_t)t.dx & 0xffffu));
         tab.push_back(v);
       }
       tabs.push_back(std::move(tab));
-      w.resize(w.size() + (size_t)blocks * p.slices * 1024, 0);
-      for (int blk = 0; blk < blocks; ++blk) {
+      w_bytes += (size_t)blocks * p.slices * 1024;
+      if (filter) w.resize(w_bytes, 0);
+      for (int blk = 0; blk < blocks && filter; ++blk) {
         const int c_first = d.g == 1 ? 0 : (blk * 32 / ocg * icg) & ~15;
         for (int row = 0; row < 32; ++row) {
           const int oc = blk / tm * tm * 32 + mfma_row_to_oc(blk % tm * 32 + row, tm);
@@ -559,26 +563,41 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
       tabs[i] = std::move(t);
     }
   }
-  auto *plan = new GatherPlan(geo);
-  plan->d = d;
-  plan->n_phases = (int)phases.size();
-  plan->max_entries = max_entries;
-  plan->max_pixels = max_pixels;
-  plan->ph = ph;
-  plan->pw = pw;
-  plan->step_h = ph * d.sh / sh;
-  plan->step_w = pw * d.sw / sw;
-  plan->blocks = blocks;
-  plan->tm = tm;
-  w.resize(std::max<size_t>(w.size(), 16));
-  plan->w_bytes = (uint32_t)w.size();
-  const size_t tab_bytes = (size_t)max_entries * (geo.rows ? sizeof(int) : sizeof(int2));
-  const size_t tab_at = w.size(), phase_at = tab_at + std::max<size_t>(tabs.size() * tab_bytes, 16);
-  std::vector<int8_t> image(phase_at + phases.size() * sizeof(GatherPhase), 0);
-  memcpy(image.data(), w.data(), w.size());
-  for (size_t i = 0; i < tabs.size(); ++i)
-    if (!tabs[i].empty()) memcpy(image.data() + tab_at + i * tab_bytes, tabs[i].data(), tabs[i].size() * sizeof(int2));
-  memcpy(image.data() + phase_at, phases.data(), phases.size() * sizeof(GatherPhase));
+  geo.d = d;
+  geo.n_phases = (int)phases.size();
+  geo.max_entries = max_entries;
+  geo.max_pixels = max_pixels;
+  geo.ph = ph;
+  geo.pw = pw;
+  geo.step_h = ph * d.sh / sh;
+  geo.step_w = pw * d.sw / sw;
+  geo.blocks = blocks;
+  geo.tm = tm;
+  geo.w_bytes = (uint32_t)std::max<size_t>(w_bytes, 16);
+  return true;
+}
+
+}  // namespace
+
+int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *filter, GatherPlan **out) {
+  *out = nullptr;
+  GatherLayer l;
+  if (!gather_layer(ctx->num_cu, d, filter, true, &l)) return TPUHIP_OK;
+  if (l.plan.lds > 64 * 1024)
+    for (const void *kernel : {(const void *)conv_gather_patch_kernel<true>, (const void *)conv_gather_patch_kernel<false>})
+      if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPatchLds) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)gather_layer(ctx->num_cu, d, filter, false, &l);
+        break;
+      }
+  auto *plan = new GatherPlan(l.plan);
+  const size_t tab_bytes = (size_t)plan->max_entries * (plan->rows ? sizeof(int) : sizeof(int2));
+  const size_t tab_at = plan->w_bytes, phase_at = tab_at + std::max<size_t>(l.tabs.size() * tab_bytes, 16);
+  std::vector<int8_t> image(phase_at + l.phases.size() * sizeof(GatherPhase), 0);
+  if (!l.w.empty()) memcpy(image.data(), l.w.data(), l.w.size());
+  for (size_t i = 0; i < l.tabs.size(); ++i)
+    if (!l.tabs[i].empty()) memcpy(image.data() + tab_at + i * tab_bytes, l.tabs[i].data(), l.tabs[i].size() * sizeof(int2));
+  memcpy(image.data() + phase_at, l.phases.data(), l.phases.size() * sizeof(GatherPhase));
   plan->tab_at = (uint32_t)tab_at;
   plan->phase_at = (uint32_t)phase_at;
   int rc = tpuhip_malloc(ctx, image.size(), (void **)&plan->w);
@@ -589,6 +608,29 @@ int gather_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc &d, const int8_t *fil
   }
   *out = plan;
   return TPUHIP_OK;
+}
+
+int gather_form(const tpuhip_conv_desc &d, int num_cu, int *reach) {
+  GatherLayer l;
+  if (!gather_layer(num_cu, d, nullptr, true, &l)) return 0;
+  const GatherPlan &g = l.plan;
+  if (!g.rows) return 1;
+  const int patch = 3 * 32 * 4 + g.n_phases * g.max_entries * 4;
+  int64_t low = 0, high = 0;
+  for (size_t i = 0; i < l.phases.size(); ++i) {
+    const GatherPhase &p = l.phases[i];
+    const int64_t last = ((int64_t)(std::min(g.rows, p.qh) - 1) * g.step_h * g.cols + (int64_t)(p.qw - 1) * g.step_w) * g.prow;
+    for (const int2 &e : l.tabs[i])
+      for (int at : {e.x, e.y}) {
+        low = std::min<int64_t>(low, at);
+        high = std::max<int64_t>(high, last + at);
+      }
+  }
+  if (reach) {
+    const int64_t r[5] = {patch, patch + low, patch + high + 16, (int64_t)g.lds, g.waves * 64};
+    for (int i = 0; i < 5; ++i) reach[i] = (int)std::clamp<int64_t>(r[i], INT_MIN, INT_MAX);
+  }
+  return 2;
 }
 
 void gather_destroy(tpuhip_ctx *ctx, GatherPlan *plan) {
