@@ -273,6 +273,9 @@ const char *tpuhip_conv2d_tile_name(int tile);
  * constants and what is fused behind it may rule the variant out besides).  Asking for it with algo = 16 + tile is another
  * matter: that is refused only where the variant cannot run the layer. */
 int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu);
+/* the number of shapes (with what is fused behind them) whose tile variant timing has chosen in this process and is kept: a layer of
+ * such a shape takes it without timing */
+int tpuhip_conv2d_tiles_known(void);
 /* How a grouped conv or one over inserted zeros (algo 0) of this shape runs on a device of num_cu compute units: 2 from a patch of
  * its input in LDS, 1 with every fragment straight from memory, 0 otherwise.  Of 2, reach (may be NULL) receives five numbers of a
  * workgroup: the LDS byte at which its patch begins, the first byte and the one past the last that its fragment reads reach, its

@@ -98,3 +98,29 @@ def test_a_module_finds_lines_of_more_bits():
             assert np.array_equal(m.get_tensor_i8("leaky"), want["leaky"])
             assert not keep or np.array_equal(m.get_tensor_i8("conv"), want["conv"])
         m.close()
+
+
+def test_a_tile_is_chosen_apart_for_a_line_and_another_table(ctx):
+    """a computed line and a lookup are other epilogues: what timing chose for a shape with one is not taken for the other"""
+    rng = np.random.default_rng(5)
+    x = rng.integers(-128, 128, (1, 64, 19, 23)).astype(np.int8)
+    w = rng.integers(-60, 61, (88, 64, 1, 1)).astype(np.int8)
+    mult, rsh = np.full(88, 1 << 30, np.int32), np.full(88, 8, np.int32)
+    d = conv_desc(x.shape, w.shape, with_bias=False)
+    xt, yt, tt = ctx.from_nchw(x), ctx.tensor((1, 88, 19, 23)), ctx.tensor((1, 88, 19, 23))
+    other = rng.integers(-128, 128, 256).astype(np.int8)
+    y_ref = O.conv2d_i8(x, w, None, rsh.astype(np.float32), mult.astype(np.float32),
+                        O.make_conv_desc(x.shape, w.shape, 1, (1, 1), (0, 0, 0, 0), (1, 1), (0, 0), False, False, None))
+    known = ctx.lib.tpuhip_conv2d_tiles_known()
+    for table, new in ((TABLES["0.1"], 1), (other, 1), (TABLES["half"], 0), (TABLES["one below"], 0), (None, 1)):
+        wh = ctx.conv_prepack(d, w, None, mult, rsh)
+        if table is None:
+            ctx.conv(wh, xt, tt)
+        else:
+            ctx.conv_post(wh, xt, yt, table, tt)
+        assert np.array_equal(ctx.to_nchw(tt), y_ref if table is None else O.lut_i8(y_ref, table))
+        known += new
+        assert ctx.lib.tpuhip_conv2d_tiles_known() == known
+        ctx.conv_weights_destroy(wh)
+    for t in (xt, yt, tt):
+        t.free()

@@ -5060,17 +5060,19 @@ bool is_line(const int8_t *t, int m, int r) {
   return all;
 }
 
-// slope: what the caller knows of the table (conv2d_post); else only a line of 7 bits is looked for, whose slope the last entry
-// tells: 60 ns, where looking for any takes 1.3 us.  A lookup takes 16 instructions and four LDS reads per four outputs, the line
-// 10 and none.
+// The line that a fused table is, m == 0: none.  What the caller knows of the table (conv2d_post); else only a line of 7 bits is
+// looked for, whose slope the last entry tells: 60 ns, where looking for any takes 1.3 us.
+LeakySlope line_of(const PostOps &p) {
+  if (!p.lut) return LeakySlope();
+  if (p.slope) return *p.slope;
+  return p.lut[128] < 0 && is_line(p.lut, -p.lut[128], 7) ? LeakySlope{-p.lut[128], 7} : LeakySlope();
+}
+
+// A lookup takes 16 instructions and four LDS reads per four outputs, the line 10 and none.
 void apply_fusion(ConvArgs *a, const void *y, const PostOps &p, bool can_slope) {
   if (p.lut) {
     a->lut_dst = (int8_t *)p.lut_out;
-    LeakySlope s;
-    if (can_slope) {
-      if (p.slope) s = *p.slope;
-      else if (p.lut[128] < 0 && is_line(p.lut, -p.lut[128], 7)) s = LeakySlope{-p.lut[128], 7};
-    }
+    const LeakySlope s = can_slope ? line_of(p) : LeakySlope();
     a->slope_m = s.m;
     a->slope_r = s.r;
     if (!s.m) {
@@ -5109,7 +5111,7 @@ TileKey tile_key(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void
   const tpuhip_fused_add *f = p.has_add() ? p.f : nullptr;
   return TileKey{ctx->num_cu, d.n, d.ic, d.ih, d.iw, d.oc, d.oh, d.ow, d.kh, d.kw, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw,
                  d.x_cs, d.y_cs, d.do_relu, d.relu_first, requant_form(w), w->split_oc, w->y2_cs, w->relu2, y != nullptr,
-                 p.lut != nullptr, p.lut_out != nullptr, f != nullptr,
+                 !p.lut ? 0 : line_of(p).m ? 2 : 1, p.lut_out != nullptr, f != nullptr,
                  f && std::abs(f->m_src) <= 127 && std::abs(f->m_conv) <= 127 && f->rshift <= 8, f && f->do_relu,
                  d.pb, d.pr};
 }
@@ -5524,6 +5526,11 @@ const char *tpuhip_conv2d_tile_name(int tile) {
 
 int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu) {
   return desc && tile >= 0 && tile < kNumTiles && !check_desc(*desc) && tile_is_candidate(*desc, tile, num_cu) ? 1 : 0;
+}
+
+int tpuhip_conv2d_tiles_known(void) {
+  std::lock_guard<std::mutex> l(g_tiles_mu);
+  return (int)g_tiles.size();
 }
 
 int tpuhip_conv2d_gather_form(const tpuhip_conv_desc *desc, int num_cu, int *reach) {
