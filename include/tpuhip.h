@@ -273,6 +273,8 @@ const char *tpuhip_conv2d_tile_name(int tile);
  * constants and what is fused behind it may rule the variant out besides).  Asking for it with algo = 16 + tile is another
  * matter: that is refused only where the variant cannot run the layer. */
 int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu);
+/* a conv on the stem path: the result rows of a tile where the kernel of whole rows takes the layer, 0 where the other one does */
+int tpuhip_conv2d_stem_rows(const tpuhip_conv_weights *w);
 /* the number of shapes (with what is fused behind them) whose tile variant timing has chosen in this process and is kept: a layer of
  * such a shape takes it without timing */
 int tpuhip_conv2d_tiles_known(void);

@@ -20,7 +20,7 @@ def ctx():
 
 # n, ic, ih, iw, oc, (kh, kw), (sh, sw), pads (t, b, l, r), x_cs, relu
 CASES = [
-    (2, 3, 24, 32, 32, (3, 3), (1, 1), (1, 1, 1, 1), 4, True),        # few tiles: the other kernel
+    (2, 3, 24, 32, 32, (3, 3), (1, 1), (1, 1, 1, 1), 4, True),
     (40, 3, 30, 32, 32, (3, 3), (1, 1), (1, 1, 1, 1), 4, True), (70, 3, 34, 32, 32, (3, 3), (2, 2), (1, 1, 1, 1), 4, False),
     (70, 3, 19, 45, 24, (3, 3), (1, 1), (1, 1, 1, 1), 4, False), (140, 3, 19, 45, 24, (3, 3), (2, 2), (0, 1, 0, 1), 16, True),
     (70, 4, 17, 30, 64, (7, 7), (2, 2), (3, 3, 3, 3), 4, True), (70, 4, 31, 36, 33, (7, 8), (3, 2), (3, 3, 8, 7), 4, False),
@@ -28,14 +28,18 @@ CASES = [
     (1200, 3, 3, 32, 16, (3, 3), (1, 1), (0, 0, 1, 1), 4, True), (40, 3, 40, 3, 16, (3, 3), (1, 1), (1, 1, 0, 0), 4, True),
     (150, 3, 8, 2, 16, (3, 2), (1, 1), (1, 1, 1, 0), 4, False), (70, 3, 64, 64, 32, (3, 3), (2, 2), (1, 1, 1, 1), 4, True),
     (40, 3, 60, 61, 64, (7, 7), (2, 2), (3, 3, 3, 3), 4, False), (9, 3, 130, 257, 20, (3, 3), (1, 1), (1, 1, 1, 1), 4, True),
-    (11, 3, 8, 1700, 64, (7, 7), (1, 1), (3, 3, 3, 3), 4, True),     # the patch of one row passes its share of LDS: the other kernel
+    (11, 3, 8, 1700, 64, (7, 7), (1, 1), (3, 3, 3, 3), 4, True),
 ]
+# few tiles, one column of results, and a patch of one row that passes its share of LDS
+OTHER_KERNEL = [CASES[0], CASES[10], (11, 3, 8, 2400, 64, (7, 7), (1, 1), (3, 3, 3, 3), 4, True)]
+CASES += OTHER_KERNEL[2:]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])))
 @pytest.mark.parametrize("post", ["plain", "leaky", "table", "shift_1"])
 def test_against_the_oracle(ctx, case, post):
     n, ic, ih, iw, oc, k, s, pads, x_cs, relu = case
+    rows = case not in OTHER_KERNEL and post != "shift_1"
     rng = np.random.default_rng(ic + ih * 3 + oc + k[0] * 7)
     x = rng.integers(-128, 128, (n, ic, ih, iw)).astype(np.int8)
     w = np.clip(np.rint(rng.normal(0, 40, (oc, ic, *k))), -127, 127).astype(np.int8)
@@ -49,7 +53,7 @@ def test_against_the_oracle(ctx, case, post):
     for t in (yt, tt):
         ctx._ck(ctx.lib.tpuhip_memset(ctx.h, t.ptr, 0x55, t.nbytes))
     wh = ctx.conv_prepack(d, w, f2i32(bias), f2i32(mult), f2i32(rsh))
-    assert ctx.conv_algo_name(wh) == "stem"
+    assert ctx.conv_algo_name(wh) == "stem" and (ctx.lib.tpuhip_conv2d_stem_rows(wh) > 0) == rows
     if post == "leaky":
         table = ctx.leaky_relu_table(0, 1, 10, 102)
         ctx.conv_post(wh, xt, yt, table, tt)

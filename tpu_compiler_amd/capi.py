@@ -100,6 +100,7 @@ PROTOTYPES = {
     "tpuhip_conv2d_algo_name": (C.c_char_p, [C.c_void_p]),
     "tpuhip_conv2d_tile_name": (C.c_char_p, [C.c_int]),
     "tpuhip_conv2d_tile_timed": (C.c_int, [C.POINTER(ConvDesc), C.c_int, C.c_int]),
+    "tpuhip_conv2d_stem_rows": (C.c_int, [C.c_void_p]),
     "tpuhip_conv2d_tiles_known": (C.c_int, []),
     "tpuhip_conv2d_gather_form": (C.c_int, [C.POINTER(ConvDesc), C.c_int, C.POINTER(C.c_int)]),
     "tpuhip_conv2d_can_fuse_table": (C.c_int, [C.c_void_p]),

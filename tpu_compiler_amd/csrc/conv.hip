@@ -5528,6 +5528,8 @@ int tpuhip_conv2d_tile_timed(const tpuhip_conv_desc *desc, int tile, int num_cu)
   return desc && tile >= 0 && tile < kNumTiles && !check_desc(*desc) && tile_is_candidate(*desc, tile, num_cu) ? 1 : 0;
 }
 
+int tpuhip_conv2d_stem_rows(const tpuhip_conv_weights *w) { return w && w->algo == ALGO_STEM ? w->stem_rows.rows : 0; }
+
 int tpuhip_conv2d_tiles_known(void) {
   std::lock_guard<std::mutex> l(g_tiles_mu);
   return (int)g_tiles.size();
