@@ -1,0 +1,35 @@
+"""Several tensors laid out for the host by one launch: more of them than one list holds, vectors among them, up to what goes
+straight into the staging buffer and beyond it."""
+import numpy as np
+import pytest
+
+from tpu_compiler_amd import graphs, module
+
+pytestmark = pytest.mark.gpu
+
+RAGGED = [(1, 3, 5, 7), (2, 64, 16, 8), (1, 65, 1, 129), (3, 13, 1, 1), (1, 255, 13, 13), (2, 17, 9, 127), (1, 1, 1, 128), (1, 4, 3, 43)]
+
+
+@pytest.mark.parametrize("shapes", [RAGGED[:2], RAGGED[:4], RAGGED[:5], RAGGED * 3 + RAGGED[:1],
+                                    RAGGED * 3 + [(1, 70, 61, 67), (2, 129, 65, 131)]])
+@pytest.mark.parametrize("i8", [False, True])
+def test_every_tensor_of_a_graph(shapes, i8):
+    g = graphs.Graph("list", 1)
+    for i, s in enumerate(shapes):
+        g.add(graphs.Op("tpu.input", "x%d" % i, [], s))
+        g.add(graphs.Op("tpu.relu", "y%d" % i, ["x%d" % i], s))
+    g.outputs = ["y%d" % i for i in range(len(shapes))]
+    m = module()
+    m.load(g)
+    for k in range(2):
+        xs = [np.random.default_rng(k + i).integers(-128, 128, s).astype(np.int8) for i, s in enumerate(shapes)]
+        for i, x in enumerate(xs):
+            m.set_tensor_i8("x%d" % i, x)
+        m.invoke()
+        if i8:
+            every = {n: m.get_tensor_i8(n) for n in m.tensor_names()}
+        else:
+            every = m.get_all_tensor()
+        for i, x in enumerate(xs):
+            assert np.array_equal(every["x%d" % i], x) and np.array_equal(every["y%d" % i], np.maximum(x, 0)), i
+    m.close()

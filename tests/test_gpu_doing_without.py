@@ -22,6 +22,10 @@ def test_results_without_the_memory_a_call_would_like(case):
     _run(case)
 
 
+def test_several_results_without_room_for_their_dense_forms_together():
+    _run("many_results")
+
+
 def test_results_without_threads(tmp_path):
     path = tmp_path / "model.mlir"
     mlir_text.write_mlir(graphs.cfg3_resnet50(batch=1, hw=64), path)

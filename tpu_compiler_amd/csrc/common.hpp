@@ -118,6 +118,14 @@ bool slope_of_table(const int8_t *table, LeakySlope *out);
 // conv.hip: tpuhip_conv2d_post_i8 by a caller that knows what slope_of_table() says of post->lut (NULL: does not)
 int conv2d_post(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y, const tpuhip_conv_post *post,
                 const LeakySlope *slope);
+// elementwise.hip: channels-last int8 tensors to dense NCHW bytes, all in one launch as far as it takes them
+struct DenseItem {
+  const int8_t *src;
+  int8_t *dst;
+  int64_t hw;
+  int n, c, h, w, cs;
+};
+int lay_out_dense(tpuhip_ctx *ctx, const DenseItem *items, size_t n);
 // conv.hip: packs n filters; the list is in memory the device reads
 int pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t largest);
 // conv.hip: makes the requantisation parameters of n layers; the list likewise

@@ -448,7 +448,9 @@ int host_to_device(tpuhip_ctx *ctx, const HostTensor &t, HostKind kind, const vo
 // What a round of device_to_host() does: `Fetch`es fill the staging buffer, `Part`s are passed on to the callers' memory.
 namespace {
 
-constexpr size_t kSpan = 8 * kPiece;            // bytes of the staging buffer behind one event
+constexpr size_t kTurn = 8 * kPiece;            // bytes of the staging buffer behind one event
+constexpr size_t kDirect = 2 * kPiece;          // laid out straight into the staging buffer up to here
+constexpr size_t kSpanLeast = 4 * kPiece, kSpanMost = 8 * kPiece;
 constexpr size_t kPastCaches = 16 << 20;        // host bytes of a call from which its floats go past the caches: half of the
                                                 // last level; they would evict each other, and the stores read nothing
 struct Part {
@@ -471,37 +473,127 @@ size_t elements(const HostRead &r) { return (size_t)r.t.n * r.t.c * r.t.h * r.t.
 
 }  // namespace
 
-// Tensors of up to two pieces are laid out straight into the staging buffer; the dense form of larger ones is made on the
-// device and comes over in spans.  An event stands behind each span, and behind small tensors that make one up together;
-// the host pass of a span runs on several threads while the next ones are laid out and on the bus, and for small tensors
-// while the launches of those behind them are still being issued.  Those threads wait for spans by looking again and again:
-// they are called once the work in front of the first one has ended, which this thread waits for alone (a read 25 ms behind
-// its launch kept all eight busy for as long, 200 ms of CPU time).
-int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
-  if (int rc = not_captured(ctx, "a tensor to the host")) return rc;
-  size_t total = 0, host_total = 0, largest = 0;
+// events of the context, at least so many
+static int events_ready(tpuhip_ctx *ctx, size_t n) {
+  while (ctx->stage_events.size() < n) {
+    hipEvent_t e;
+    TPUHIP_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    ctx->stage_events.push_back(e);
+  }
+  return TPUHIP_OK;
+}
+
+// int8 tensors that fit the staging buffer one by one: their dense forms are made on the device in one launch per filling of the
+// buffer.  Up to kDirect together they are laid out straight into it; otherwise they lie in the landing buffer as they will lie
+// there and come over in spans of half of what is left, within bounds: a launch and an event cost the bus 5 us a span, and the
+// host passes of the last span have no transfer to hide behind.  The host passes run on several threads while the next spans are
+// on the bus.  Those threads wait for spans by looking again and again: they are called once the work in front has ended, which
+// this thread waits for alone (a read 25 ms behind its launch kept all eight busy for as long, 200 ms of CPU time).
+// *done: false where there is no memory for it.
+static int read_dense(tpuhip_ctx *ctx, const std::vector<HostRead> &reads, bool past_caches, bool *done) {
+  *done = false;
+  size_t total = 0;
+  for (const HostRead &r : reads) total += (elements(r) + 63) / 64 * 64;
+  if (int rc = stage_ready(ctx, total)) return rc;
+  const bool direct = total <= kDirect;
+  if (!direct && landing_ready(ctx, std::min(total, ctx->stage_bytes)) != TPUHIP_OK) {
+    (void)hipGetLastError();
+    return TPUHIP_OK;
+  }
+  *done = true;
+  int8_t *stage = (int8_t *)ctx->stage, *to = direct ? stage : (int8_t *)ctx->landing;
+  std::vector<Part> parts;
+  std::vector<DenseItem> dense;
+  std::vector<size_t> ends;   // of the spans
+  for (size_t i = 0; i < reads.size();) {
+    parts.clear();
+    dense.clear();
+    ends.clear();
+    size_t at = 0;
+    for (; i < reads.size(); ++i) {
+      const HostRead &r = reads[i];
+      const size_t bytes = elements(r);
+      if (bytes > ctx->stage_bytes - at) break;
+      dense.push_back({(const int8_t *)r.src, to + at, (int64_t)r.t.h * r.t.w, r.t.n, r.t.c, r.t.h, r.t.w, r.t.cs});
+      for (size_t p = 0; p < bytes; p += kPiece) parts.push_back({&r, p, std::min(kPiece, bytes - p), at + p, 0});
+      at += (bytes + 63) / 64 * 64;
+    }
+    ctx->stage_busy = true;
+    if (direct) {
+      if (int rc = lay_out_dense(ctx, dense.data(), dense.size())) return rc;
+      TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+      ctx->stage_busy = false;
+      parallel_pieces(parts.size(), [&](size_t k) { pass_part(parts[k], stage, past_caches); });
+      return TPUHIP_OK;
+    }
+    for (size_t from = 0; from < at; from = ends.back())
+      ends.push_back(std::min(at, from + std::min(std::max((at - from) / 2 / kPiece * kPiece, kSpanLeast), kSpanMost)));
+    size_t span = 0;
+    for (Part &p : parts) {
+      while (p.at + p.count > ends[span]) ++span;
+      p.span = span;
+    }
+    if (int rc = events_ready(ctx, ends.size() + 1)) return rc;
+    auto job = std::make_shared<HostJob>();
+    job->pieces = parts.size();
+    std::atomic<size_t> arrived{0};     // spans that are in the buffer
+    std::atomic<bool> lost{false};      // the device failed: nothing more arrives
+    job->piece = [&](size_t k) {
+      const Part &p = parts[k];
+      while (arrived.load(std::memory_order_acquire) <= p.span) {
+        if (lost.load(std::memory_order_relaxed)) return;
+        std::this_thread::yield();
+      }
+      pass_part(p, stage, past_caches);
+    };
+    HostWorkers &workers = HostWorkers::get();
+    int rc = TPUHIP_OK;
+    auto hip = [&](hipError_t e, const char *what) {
+      if (!rc && e != hipSuccess) rc = set_error(TPUHIP_ERR_HIP, "%s failed: %s", what, hipGetErrorString(e));
+    };
+    const hipEvent_t front = ctx->stage_events[ends.size()];
+    const bool waits = hipStreamQuery(ctx->stream) != hipSuccess;
+    if (waits) hip(hipEventRecord(front, ctx->stream), "hipEventRecord");
+    if (!rc) rc = lay_out_dense(ctx, dense.data(), dense.size());
+    for (size_t k = 0, from = 0; !rc && k < ends.size(); from = ends[k++]) {
+      rc = stage_copy(ctx, (const int8_t *)ctx->landing + from, stage + from, ends[k] - from);
+      if (!rc) hip(hipEventRecord(ctx->stage_events[k], ctx->stream), "hipEventRecord");
+    }
+    if (waits && !rc) hip(hipEventSynchronize(front), "hipEventSynchronize");
+    const bool shared = !rc && parts.size() > 1 && workers.enter(job);
+    for (size_t k = 0; !rc && k < ends.size(); ++k) {
+      hip(hipEventSynchronize(ctx->stage_events[k]), "hipEventSynchronize");
+      if (!rc) arrived.store(k + 1, std::memory_order_release);
+    }
+    if (rc) lost.store(true);
+    finish_job(*job);
+    if (shared) workers.leave();
+    if (rc) return rc;
+    ctx->stage_busy = false;
+  }
+  return TPUHIP_OK;
+}
+
+// Float tensors, those that are larger than the staging buffer, and others where read_dense() has no memory.  Tensors of up to
+// two pieces are laid out straight into the staging buffer; the dense form of larger ones is made on the device and comes over
+// in spans, with an event behind each, and behind small tensors that make one up together.  The threads of the host pass are
+// called as there.
+static int read_in_turn(tpuhip_ctx *ctx, const std::vector<HostRead> &reads, bool past_caches) {
+  const size_t n = reads.size();
+  size_t total = 0, largest = 0;
   for (size_t i = 0; i < n; ++i) {
-    const size_t count = elements(reads[i]), bytes = count * stage_size(reads[i].kind);
+    const size_t bytes = elements(reads[i]) * stage_size(reads[i].kind);
     total += (bytes + 63) / 64 * 64;
-    host_total += count * host_size(reads[i].kind);
-    if (bytes > 2 * kPiece && reads[i].kind != HostKind::kFloats) largest = std::max(largest, bytes);
+    if (bytes > kDirect && reads[i].kind != HostKind::kFloats) largest = std::max(largest, bytes);
   }
   if (int rc = stage_ready(ctx, total)) return rc;
   if (largest)
     if (int rc = landing_ready(ctx, largest)) return rc;
   int8_t *stage = (int8_t *)ctx->stage;
   const size_t room = ctx->stage_bytes;
-  const bool past_caches = host_total >= kPastCaches;
   auto lay_out = [&](const HostRead &r, void *to) {
     return tpuhip_nhwc_to_nchw_i8(ctx, r.src, to, r.t.n, r.t.c, r.t.h, r.t.w, r.t.cs);
   };
-  if (n == 1 && host_total <= kAlone) {   // done before a worker has woken
-    const int rc = reads->kind == HostKind::kFloats ? stage_copy(ctx, reads->src, stage, total) : lay_out(*reads, stage);
-    if (rc) return rc;
-    TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    pass_part(Part{reads, 0, elements(*reads), 0, 0}, stage, false);
-    return TPUHIP_OK;
-  }
 
   struct Fetch {
     const HostRead *r;
@@ -519,16 +611,16 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
       const HostRead &r = reads[i];
       const size_t per = stage_size(r.kind), bytes = elements(r) * per;
       if (at && bytes > room - at && bytes <= room) break;   // in parts only where a round of its own does not help
-      const bool whole = bytes <= 2 * kPiece;
+      const bool whole = bytes <= kDirect;
       while (done < bytes && at < room) {
-        const size_t len = std::min({bytes - done, room - at, kSpan});
+        const size_t len = std::min({bytes - done, room - at, kTurn});
         fetches.push_back({&r, done, len, at, whole, false});
         open += len;
         for (size_t p = 0; p < len; p += kPiece) {
           const size_t l = std::min(kPiece, len - p);
           parts.push_back({&r, (done + p) / per, l / per, at + p, spans});
         }
-        if (open >= kSpan / 2) {
+        if (open >= kTurn / 2) {
           fetches.back().closes = true;
           ++spans;
           open = 0;
@@ -544,11 +636,7 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
       fetches.back().closes = true;
       ++spans;
     }
-    while (ctx->stage_events.size() < spans + 1) {   // the last one stands behind the work in front
-      hipEvent_t e;
-      TPUHIP_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-      ctx->stage_events.push_back(e);
-    }
+    if (int rc = events_ready(ctx, spans + 1)) return rc;   // the last one stands behind the work in front
     auto job = std::make_shared<HostJob>();
     job->pieces = parts.size();
     std::atomic<size_t> arrived{0};     // spans that are in the buffer
@@ -609,6 +697,34 @@ int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
     ctx->stage_busy = false;
   }
   return TPUHIP_OK;
+}
+
+int device_to_host(tpuhip_ctx *ctx, const HostRead *reads, size_t n) {
+  if (int rc = not_captured(ctx, "a tensor to the host")) return rc;
+  size_t host_total = 0;
+  std::vector<HostRead> dense, others;
+  for (size_t i = 0; i < n; ++i) {
+    host_total += elements(reads[i]) * host_size(reads[i].kind);
+    (reads[i].kind != HostKind::kFloats && elements(reads[i]) <= kStageMax ? dense : others).push_back(reads[i]);
+  }
+  if (n == 1 && host_total <= kAlone) {   // done before a worker has woken
+    const size_t bytes = elements(*reads) * stage_size(reads->kind);
+    if (int rc = stage_ready(ctx, bytes)) return rc;
+    const HostTensor &t = reads->t;
+    const int rc = reads->kind == HostKind::kFloats ? stage_copy(ctx, reads->src, ctx->stage, bytes)
+                                                    : tpuhip_nhwc_to_nchw_i8(ctx, reads->src, ctx->stage, t.n, t.c, t.h, t.w, t.cs);
+    if (rc) return rc;
+    TPUHIP_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    pass_part(Part{reads, 0, elements(*reads), 0, 0}, (const int8_t *)ctx->stage, false);
+    return TPUHIP_OK;
+  }
+  const bool past_caches = host_total >= kPastCaches;
+  if (!dense.empty()) {
+    bool done = false;
+    if (int rc = read_dense(ctx, dense, past_caches, &done)) return rc;
+    if (!done) others.insert(others.end(), dense.begin(), dense.end());
+  }
+  return others.empty() ? TPUHIP_OK : read_in_turn(ctx, others, past_caches);
 }
 
 AheadRead::~AheadRead() {
