@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <iterator>
+#include <mutex>
 
 namespace tpuhip {
 
@@ -17,6 +18,17 @@ int set_error(int status, const char *fmt, ...) {
   va_end(ap);
   g_last_error = buf;
   return status;
+}
+
+bool raise_lds_limit(const void *kernel, unsigned bytes) {
+  static std::mutex mu;
+  static std::map<const void *, unsigned> raised;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = raised.find(kernel);
+  if (it != raised.end() && it->second >= bytes) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+  raised[kernel] = bytes;
+  return true;
 }
 
 int grow_workspace(tpuhip_ctx *ctx, size_t bytes) {

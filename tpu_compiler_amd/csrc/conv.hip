@@ -13,6 +13,7 @@
 #include "common.hpp"
 #include "conv_epilogue.hpp"
 #include "conv_gather.hpp"
+#include "conv_split.hpp"
 
 #include <map>
 #include <mutex>
@@ -83,6 +84,11 @@ struct tpuhip_conv_weights {
   int c16 = 0;           // input 16-channel groups per tap
   int k16 = 0;           // 16-byte K groups in total
   StemRows stem_rows;    // the stem path: the row form's tiles, where that takes the layer
+  // a tile variant of the K-split kernel with blocks of 16 x 16: its launch's arguments but the pointers, and whether they hold
+  // the layer's numbers
+  SplitArgs split;
+  SplitPlan split_plan;
+  bool split_fits = false;
 };
 
 struct ConvArgs {
@@ -4029,9 +4035,11 @@ struct TileCfg {
   int reg;   // 0: LDS kernel, one tile per workgroup; 1: the LDS-free kernel, bm x bn is the
              // tile of one wave; 2: its split-K form; 3: LDS kernel, persistent workgroups;
              // 4: patch kernel (bn = pixel slots of a tile of whole rows); 5: pointwise kernel;
-             // 6: patch kernel, second form; 7: patch kernel, third form; 8: K split over all waves; 9: patch kernel, fourth form
+             // 6: patch kernel, second form; 7: patch kernel, third form; 8: K split over all waves; 9: patch kernel, fourth form;
+             // 10: K split over waves, blocks of 16 x 16
   int bk;    // K bytes per step (pointwise kernel: the padded K it holds)
   int cmod;  // fourth form of the patch kernel: the input channels are a multiple of this
+  SplitVariant split;   // 10
 };
 
 // The tile variants, in the order of their public index (conv desc algo = 16 + index).
@@ -4140,6 +4148,20 @@ struct TileCfg {
   U4(73, "mfma_rows_64x320_c32", 2, 2, 1, 5, 1, 4, 3) \
   U4(74, "mfma_rows_64x256_c32", 2, 2, 1, 4, 1, 4, 4) 
 
+// K split over the waves of a workgroup, blocks of 16 x 16 (conv_split.hip):
+// SP(index, name, waves along K, along the pixels, blocks of 16 pixels and of 16 channels per wave).  Of 52 layers of 1 to 4 images
+// of 5 to 60 pixels a side (1x1 to 5x5, stride 1 and 2, dilation, 64 to 1024 channels) one of them is the fastest of all in 36, by
+// 1 % to 2.7 times (profiles/conv_split_tiles.txt): 16x32 in 13 (by up to 17 % over the next of them), 16x16_w4 in 10 (14 %), 16x16
+// in 5 (18 %), 32x32 in 5 (55 %), 32x64 in 2 (13 %), 16x64 in one (22 %); 32x128 leads at 128 -> 256 on 52 x 52 (2 %).
+#define TPUHIP_SPLIT_TILES(SP)               \
+  SP(75, "mfma_split_16x16_w4", 4, 1, 1, 1)  \
+  SP(76, "mfma_split_16x16", 8, 1, 1, 1)     \
+  SP(77, "mfma_split_16x32", 8, 1, 2, 1)     \
+  SP(78, "mfma_split_16x64", 8, 1, 4, 1)     \
+  SP(79, "mfma_split_32x32", 8, 1, 2, 2)     \
+  SP(80, "mfma_split_32x64", 8, 1, 4, 2)     \
+  SP(81, "mfma_split_32x128", 4, 2, 4, 2)
+
 constexpr int kMaxTiles = 96;
 struct TileTable {
   TileCfg t[kMaxTiles] = {};   // numbered from 0 without a gap: a caller finds the last one at the first name that is NULL
@@ -4185,6 +4207,11 @@ struct TileTable {
   n = n > i ? n : i + 1;
     TPUHIP_ROWS_TILES(U4)
 #undef U4
+#define SP(i, name, KW, PW, NB, OB) \
+  t[i] = TileCfg{16 * OB, PW * NB * 16, KW, PW, name, 10, 64, 0, {KW, PW, NB, OB}}; \
+  n = n > i ? n : i + 1;
+    TPUHIP_SPLIT_TILES(SP)
+#undef SP
   }
 };
 const TileTable kTileTable;
@@ -4201,20 +4228,6 @@ void launch_reg(tpuhip_ctx *ctx, dim3 grid, const ConvArgs &a) {
 }
 
 // the patch kernel's LDS patch is dynamic: (rows + 2) x (W + 2) x C bytes of this layer
-// Raises a kernel's dynamic LDS limit, once per kernel and size (kernels of one signature share
-// their function-pointer type, so the record is keyed by the kernel's address); on failure the
-// runtime's last error stays set for the caller to report.
-bool raise_lds_limit(const void *kernel, unsigned bytes) {
-  static std::mutex mu;
-  static std::map<const void *, unsigned> raised;
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = raised.find(kernel);
-  if (it != raised.end() && it->second >= bytes) return true;
-  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
-  raised[kernel] = bytes;
-  return true;
-}
-
 template <typename F>
 void launch_patch(tpuhip_ctx *ctx, F kernel, dim3 grid, const ConvArgs &a, bool dynamic, unsigned stage_bytes) {
   if (dynamic) (void)raise_lds_limit((const void *)kernel, kPatchBytesDyn);
@@ -4615,6 +4628,13 @@ __device__ __forceinline__ void pack_filter_group(const FilterPack &a, int64_t q
     const int k64 = r1 / (a.bm * 4), r2 = r1 - k64 * a.bm * 4, r = r2 >> 2;
     row = tile * a.bm + r;
     kc = k64 * 4 + ((r2 & 3) ^ ((r >> 2) & 3));
+  } else if (a.reg == 10) {
+    // fragment order of 16 rows: [row / 16][64 bytes of K][lane = (row & 15) + 16 * 16-byte group]
+    const int lane = (int)(q & 63);
+    const int64_t f = q >> 6;
+    const int per_blk = kg / 4, blk = (int)(f / per_blk), s = (int)(f - (int64_t)blk * per_blk);
+    row = blk * 16 + (lane & 15);
+    kc = s * 4 + (lane >> 4);
   } else if (a.reg == 0 || a.reg == 3 || a.reg == 4) {
     row = (int)(q / kg);
     kc = (int)(q - (int64_t)row * kg);
@@ -4628,7 +4648,7 @@ __device__ __forceinline__ void pack_filter_group(const FilterPack &a, int64_t q
     kc = (s >> 1) * 4 + (s & 1) * 2 + (lane >> 5);
   }
   const int tile0 = row / a.bm * a.bm;
-  const int oc = tile0 + mfma_row_to_oc(row - tile0, a.tm);
+  const int oc = a.reg == 10 ? row : tile0 + mfma_row_to_oc(row - tile0, a.tm);
   uint32_t v[4] = {0, 0, 0, 0};
   if (oc < a.oc) {
     const int8_t *src = a.raw + (int64_t)oc * a.ic * a.taps;
@@ -4714,10 +4734,18 @@ int pack_filter(tpuhip_ctx *ctx, const FilterPack &a) {
 }
 
 // (re)builds the device filter of an MFMA conv for tile variant `tile`
+// whenever the tile, the parameters or a stride have changed
+void split_ready(tpuhip_conv_weights *cw) {
+  if (cw->algo != ALGO_MFMA || kTiles[cw->tile].reg != 10 || !cw->nparam) return;
+  const SplitVariant &v = kTiles[cw->tile].split;
+  cw->split_plan = split_plan(cw->d, v, cw->fast);
+  cw->split_fits = split_args(cw->d, v, cw->split_plan, cw->nparam, &cw->split);
+}
+
 int pack_mfma_weights(tpuhip_ctx *ctx, tpuhip_conv_weights *cw, int tile) {
   const tpuhip_conv_desc &d = cw->d;
   const TileCfg &t = kTiles[tile];
-  const int tm = t.bm / t.wm / 32;
+  const int tm = t.reg == 10 ? 1 : t.bm / t.wm / 32;
   const int ocp = round_up(d.oc, t.bm);
   cw->smallc = d.ic <= 4 && (t.reg == 0 || t.reg == 3);
   cw->c16 = round_up(d.ic, 16) / 16;
@@ -4742,6 +4770,7 @@ int pack_mfma_weights(tpuhip_ctx *ctx, tpuhip_conv_weights *cw, int tile) {
   if (int rc = pack_filter(ctx, a)) return rc;
   cw->tile = tile;
   cw->ocp = ocp;
+  split_ready(cw);
   return TPUHIP_OK;
 }
 
@@ -4755,7 +4784,7 @@ void settle_tile(tpuhip_ctx *ctx, tpuhip_conv_weights *cw) {
 // the fused table lives in the LDS of the LDS kernels
 bool tile_has_lds_epilogue(int t) {
   return kTiles[t].reg == 0 || kTiles[t].reg == 3 || kTiles[t].reg == 5 || kTiles[t].reg == 6 || kTiles[t].reg == 7 ||
-         kTiles[t].reg == 8 || kTiles[t].reg == 9;
+         kTiles[t].reg == 8 || kTiles[t].reg == 9 || kTiles[t].reg == 10;
 }
 
 // the pointwise kernels: 1x1 window, no padding, no dilation (any stride), the input channels
@@ -4801,7 +4830,10 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t, int num_cu) {
   // fastest of all in 10 at 256 tiles (256 -> 256 channels 3x3: 5.3 us against 7.4), in 3 at 512, in none at 1024 (14.3
   // against 8.2) and 2048 (27.0 against 13.2): the line is four times where they were last seen to win
   if (c.reg == 8 && ceil_div64((int64_t)d.n * d.oh * d.ow, 32) * ceil_div64(d.oc, 32) > 2048) return false;
-  if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8)) return false;   // prefer the 4-channel K packing of the LDS kernels
+  // likewise: of 74 layers the most tiles with which a variant was the fastest were 512 (512 -> 2048 channels 1x1 on 7 x 7: 2.95 us
+  // against 3.00); with 832 (256 -> 1024 on 14 x 14) 3.5 against 2.9 of the blocks of 32 x 32.  The line is twice the former
+  if (c.reg == 10 && split_tiles(d, c.split, split_plan(d, c.split, true)) > 1024) return false;
+  if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8 || c.reg == 10)) return false;   // prefer the 4-channel K packing of the LDS kernels
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle
 }
 
@@ -4953,6 +4985,22 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
   *out = a;
 }
 
+void launch_split(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvArgs &a) {
+  SplitArgs s = w->split;
+  s.x = a.x;
+  s.w = a.w;
+  s.y = a.y;
+  s.bias = a.bias;
+  const bool uni = w->c16 % 4 == 0;
+  if (!a.has_lut && !a.add_dst && !a.split_oc && a.store_y) {
+    split_launch(ctx, kTiles[w->tile].split, w->split_plan, w->fast, uni, s, nullptr);
+    return;
+  }
+  SplitPost p{s, a.add_src, a.add_dst, a.lut_dst, a.y2, a.add_m_src, a.add_m_conv, a.add_rshift, a.add_relu, a.add_pk, a.store_y,
+              a.split_oc, a.y2_cs, a.lo2, a.has_lut, a.lut};
+  split_launch(ctx, kTiles[w->tile].split, w->split_plan, w->fast, uni, s, &p);
+}
+
 void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvArgs &a) {
   dim3 grid((unsigned)(a.wgs_per_xcd * 8));
   if (kTiles[w->tile].reg == 5) {
@@ -4969,6 +5017,10 @@ void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvA
   }
   if (kTiles[w->tile].reg == 9) {
     launch_rows(ctx, w->tile, grid, a, (unsigned)a.pstep_ow);
+    return;
+  }
+  if (kTiles[w->tile].reg == 10) {
+    launch_split(ctx, w, a);
     return;
   }
   const bool uni = (w->c16 % (tile_bk(kTiles[w->tile]) / 16)) == 0;
@@ -5096,7 +5148,7 @@ void apply_fusion(ConvArgs *a, const void *y, const PostOps &p, bool can_slope) 
 // the kernels of the layer that compute a leaky ReLU's line: not the dot-product depthwise one, and not the K-split ones, where a
 // lane has four outputs and a lookup is 0.25 us faster (512 -> 1024 3x3 on 13 x 13: 8.10 us, the line 8.35)
 bool can_slope(const tpuhip_conv_weights *w) {
-  return w->algo != ALGO_DEPTHWISE_DOT && !(w->algo == ALGO_MFMA && kTiles[w->tile].reg == 8);
+  return w->algo != ALGO_DEPTHWISE_DOT && !(w->algo == ALGO_MFMA && (kTiles[w->tile].reg == 8 || kTiles[w->tile].reg == 10));
 }
 
 // Tiles that timing has chosen, by everything the choice can depend on: a layer of the same shape -- a second module, the
@@ -5122,6 +5174,8 @@ bool tile_usable(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, int t, con
   if (w->split_oc && kTiles[t].reg == 4) return false;   // the patch kernel writes one result
   if (kTiles[t].reg == 5 && (!w->fast || w->split_oc % kTiles[t].bm)) return false;
   if (kTiles[t].reg == 9 && (!w->qnarrow || w->split_oc)) return false;
+  SplitArgs args;
+  if (kTiles[t].reg == 10 && !split_args(w->d, kTiles[t].split, split_plan(w->d, kTiles[t].split, w->fast), w->nparam, &args)) return false;
   return !((kTiles[t].reg == 6 || kTiles[t].reg == 7) && (!w->fast || w->split_oc));
 }
 
@@ -5505,6 +5559,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   cw->qplanes = p + at_planes;
   (narrow ? cw->qnarrow : cw->qc64) = p + at_last;
   if (algo == ALGO_STEM && narrow) cw->stem_rows = stem_rows_plan(ctx, d);
+  split_ready(cw);
   *out = cw;
   return TPUHIP_OK;
 }
@@ -5556,6 +5611,7 @@ int tpuhip_conv2d_set_input_stride(tpuhip_conv_weights *w, int x_cs) {
   TPUHIP_REQUIRE((int64_t)w->d.n * (w->d.ih + w->d.pt + w->d.pb + 2) * (w->d.iw + w->d.pl + w->d.pr + 2) * x_cs < (1ll << 31),
                  "conv: tensor too large");
   w->d.x_cs = x_cs;
+  split_ready(w);
   return TPUHIP_OK;
 }
 
@@ -5652,6 +5708,9 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
                  "conv: tile variant %s needs a single 3x3 / stride 1 / pad 1 conv with 64, 128, 256, 512 or 1024 input "
                  "channels on a map narrow enough for its row patch, right shifts of at least 1 and sums that cannot "
                  "overflow the rounding", kTiles[w->tile].name);
+  TPUHIP_REQUIRE(!(w->algo == ALGO_MFMA && kTiles[w->tile].reg == 10) || w->split_fits,
+                 "conv: tile variant %s takes sides, strides, paddings and channels below 65536 and fewer outputs",
+                 kTiles[w->tile].name);
   TPUHIP_REQUIRE((w->split_oc != 0) == (post.y2 != nullptr),
                  "conv: weights packed as a pair run through tpuhip_conv2d_pair_i8 (and only they do)");
   if (w->gather) {
@@ -5895,6 +5954,7 @@ int tpuhip_conv2d_prepack_pair(tpuhip_ctx *ctx, const tpuhip_conv_desc *da, cons
   if (int rc = tpuhip_conv2d_prepack(ctx, &m, filter.data(), bias.data(), mult.data(), rshift.data(), &cw))
     return rc;
   cw->d.y_cs = a.y_cs;
+  split_ready(cw);
   cw->split_oc = a.oc;
   cw->y2_cs = b.y_cs;
   cw->relu2 = b.do_relu ? 1 : 0;
