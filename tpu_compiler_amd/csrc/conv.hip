@@ -3934,83 +3934,6 @@ __global__ __launch_bounds__(256) void fc_reduce_kernel(ConvArgs a, const v4i *p
     epilogue_rows<1, FAST>(sum, a, oc, a.qmult + oc, a.qshift + oc, a.qhpot + oc, pb * 32 + frow, 32, nullptr, out);
 }
 
-// The same product in ONE launch: a workgroup of W waves per 32x32 block of outputs, wave w multiplying
-// K steps [w * spw, (w + 1) * spw) with the loads of two steps in flight at a time.  The W partial sums
-// meet in LDS ([wave][quarter][lane] of four dwords): every thread adds one quarter of four waves in
-// place, wave 0 adds the groups and the bias and runs the epilogue.  No scratch in device memory and no
-// second launch, which on a classifier of 32 rows is most of the time.  Four, eight or sixteen waves: the
-// fewest that request all of their K at once (K of 512 or 1024), sixteen beyond.  (K below 1024 took the
-// two launches: 22 x 232 x 23 in 8.0 us, 4.2 in one.)
-template <bool FAST, int W>
-__global__ __launch_bounds__(64 * W) void fc_one_kernel(ConvArgs a, int steps_per_wave) {
-  __shared__ v4i part[W * 4 * 64];
-  gather_conv_args(a);
-  gather_conv_args_more(a);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tile = (int)blockIdx.x;
-  const int ob = tile % a.n_oc_tiles, pb = tile / a.n_oc_tiles;
-  const int nsteps = a.kp / 64;
-  const int s0 = min(nsteps, wave * steps_per_wave), s1 = min(nsteps, s0 + steps_per_wave);
-  const __amdgpu_buffer_rsrc_t xrsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t wrsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
-  const int frow = lane & 31, fk = lane >> 5;
-  const int row = pb * 32 + frow;
-  const uint32_t xoff = row < a.npix ? (uint32_t)(row * a.x_cs + fk * 16) : kOobOffset;
-  const uint32_t woff = (uint32_t)(ob * nsteps) * 2048u + (uint32_t)lane * 16u;
-  v16i acc;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = 0;
-  int s = s0;
-  for (; s + 2 <= s1; s += 2) {
-    v4i af[4], bf[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      af[u] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(wrsrc, woff, s * 2048 + u * 1024, 0);
-      bf[u] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(xrsrc, xoff, s * 64 + u * 32, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[u], bf[u], acc, 0, 0, 0);
-  }
-  if (s < s1) {
-    v4i af[2], bf[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      af[u] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(wrsrc, woff, s * 2048 + u * 1024, 0);
-      bf[u] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(xrsrc, xoff, s * 64 + u * 32, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[u], bf[u], acc, 0, 0, 0);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    part[(wave * 4 + q) * 64 + lane] = v4i{acc[q * 4 + 0], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
-  __syncthreads();
-  {
-    // thread (group g of four waves, quarter q, lane): the sum lands where only it has read
-    const int g = wave >> 2, q = wave & 3;
-    v4i t = part[((g * 4 + 0) * 4 + q) * 64 + lane];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) t += part[((g * 4 + w) * 4 + q) * 64 + lane];
-    part[((g * 4) * 4 + q) * 64 + lane] = t;
-  }
-  __syncthreads();
-  if (wave != 0) return;
-  const int oc = ob * 32 + fk * 16;                 // this lane's 16 channels
-  v16i sum[1];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    v4i t = *reinterpret_cast<const v4i *>(a.bias + oc + q * 4);
-#pragma unroll
-    for (int g = 0; g < W / 4; ++g) t += part[((g * 4) * 4 + q) * 64 + lane];
-    sum[0][q * 4 + 0] = t[0]; sum[0][q * 4 + 1] = t[1]; sum[0][q * 4 + 2] = t[2]; sum[0][q * 4 + 3] = t[3];
-  }
-  const OutRoute out{a.y, a.y_cs, a.lo, 0};
-  if (oc < a.ocw)
-    epilogue_rows<1, FAST>(sum, a, oc, a.qmult + oc, a.qshift + oc, a.qhpot + oc, pb * 32 + frow, 32, nullptr, out);
-}
-
 // The scratch of the allocation-free entry point: one array per device the library is loaded
 // on.  Nothing in it has to start at zero: every partial sum the second launch reads was
 // written by the first.
@@ -6022,20 +5945,9 @@ static int run_fc_splitk(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const vo
 static int run_fc_one(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x, void *y) {
   ConvArgs a;
   fill_args(ctx, w, x, y, &a);
-  a.n_oc_tiles = w->ocp / 32;
-  const int nsteps = w->kp / 64;
-  const int64_t tiles = (int64_t)((w->d.n + 31) / 32) * a.n_oc_tiles;
-  TPUHIP_REQUIRE(tiles < (1ll << 31), "fc: too many blocks of 32 x 32 outputs");
-  const int waves = nsteps <= 8 ? 4 : nsteps <= 16 ? 8 : 16;
-  const int steps_per_wave = (nsteps + waves - 1) / waves;
-  auto kernel = waves == 4   ? (w->fast ? fc_one_kernel<true, 4> : fc_one_kernel<false, 4>)
-                : waves == 8 ? (w->fast ? fc_one_kernel<true, 8> : fc_one_kernel<false, 8>)
-                             : (w->fast ? fc_one_kernel<true, 16> : fc_one_kernel<false, 16>);
-  const dim3 grid((unsigned)tiles), block(64 * waves);
-  if (ctx->prof_start || ctx->prof_stop)
-    hipExtLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a, steps_per_wave);
-  else
-    hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, a, steps_per_wave);
+  TPUHIP_REQUIRE(a.qmult == a.bias + w->nparam, "fc: parameters out of place");
+  const FcArgs f{a.x, a.w, a.y, a.bias, w->nparam, a.x_bytes, a.w_bytes, a.npix, a.oc, a.x_cs, a.y_cs, w->kp / 64, a.relu_first, a.lo};
+  fc_split(ctx, f, w->fast);
   TPUHIP_CHECK_HIP(hipGetLastError());
   return TPUHIP_OK;
 }

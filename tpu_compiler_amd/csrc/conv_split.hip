@@ -298,6 +298,99 @@ __global__ __launch_bounds__(KW * PW * 64) void conv_split_post_kernel(SplitPost
   split_body<KW, PW, NB, OB, FAST, UNI, PATCH, NS, true>(p.a, &p);
 }
 
+// FullyConnected of few rows (a classifier) the same way, from the filter in fragments of 32 channels that fc_prepack() makes: 16
+// rows of a fragment are 256 contiguous bytes of it, channels 0-7 and 16-23 of the block of 32, or the others.  A workgroup of
+// eight waves per 16 * OB channels x 16 * NB rows; K split over the waves, four slices of 64 bytes in flight each.
+// Bound: launch, one trip to memory, one meeting in LDS; from 64 rows on the operands' way into a CU (98 KB each at 100 x 2048 x
+// 1000).  Replayed from a graph, against sixteen waves per block of 32 x 32, two barriers and one wave that finished 16 channels a
+// lane: 1 x 2048 x 1000 3.63 -> 2.35 us, 32 rows 4.92 -> 3.18, 100 rows 5.11 -> 4.25, 16 x 8192 x 4096 10.2 -> 6.9, 256 x 1024 x
+// 4096 8.14 -> 8.25.
+template <int NB, int OB, bool FAST>
+__global__ __launch_bounds__(512) void fc_split_kernel(FcArgs a) {
+  constexpr int KW = 8, B = NB * OB, D = kDepth;
+  static_assert(B <= KW, "a wave finishes one block");
+  __shared__ v4i sums[KW * B * 64];
+  asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.x_bytes), "s"(a.w_bytes), "s"(a.rows), "s"(a.oc), "s"(a.x_cs), "s"(a.slices),
+               "s"(a.nparam));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int oc_tile = blockIdx.x, row0 = blockIdx.y * (NB * 16);
+  const int first = OB == 2 ? oc_tile * 32 : (oc_tile >> 1) * 32 + (oc_tile & 1) * 8;   // its first channel
+  if (first >= ((a.oc + 15) & ~15)) return;    // uniform over the workgroup
+  const int px = lane & 15, chunk = lane >> 4;
+  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, 0, a.w_bytes, 0x00020000);
+  const uint32_t wbase = (uint32_t)(first >> 5) * (uint32_t)a.slices * 2048u + (OB == 2 ? 0u : (uint32_t)(oc_tile & 1) * 256u);
+  const uint32_t woff = (uint32_t)(chunk >> 1) * 1024u + (uint32_t)(px + 32 * (chunk & 1)) * 16u;
+  uint32_t xoff[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int row = row0 + j * 16 + px;
+    xoff[j] = row < a.rows ? (uint32_t)row * (uint32_t)a.x_cs + chunk * 16 : kOobOffset;
+  }
+  v4i af[D][OB], bf[D][NB];
+  auto load = [&](int slot, int s) {
+    const bool in_k = s < a.slices;
+#pragma unroll
+    for (int o = 0; o < OB; ++o)
+      af[slot][o] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(wrsrc, in_k ? woff : kOobOffset, wbase + s * 2048 + o * 256, 0);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) bf[slot][j] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(xrsrc, in_k ? xoff[j] : kOobOffset, s * 64, 0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (wave + d * KW < a.slices) load(d, wave + d * KW);   // (256 x 1024 x 4096, two slices a wave: 9.0 us with loads of nothing)
+
+  // block b: channels of half b / NB, rows of block b % NB
+  const int oc = first + (wave / NB) * 8 + (chunk & 1) * 16 + (chunk >> 1) * 4, row = row0 + (wave % NB) * 16 + px;
+  v4i bias = {0, 0, 0, 0}, mult = bias, shift = bias, hpot = bias;
+  if (wave < B) {
+    bias = *reinterpret_cast<const v4i *>(a.bias + oc);
+    mult = *reinterpret_cast<const v4i *>(a.bias + a.nparam + oc);
+    shift = *reinterpret_cast<const v4i *>(a.bias + 2 * a.nparam + oc);
+    hpot = *reinterpret_cast<const v4i *>(a.bias + 3 * a.nparam + oc);
+  }
+  v4i acc[OB][NB];
+#pragma unroll
+  for (int o = 0; o < OB; ++o)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[o][j] = v4i{0, 0, 0, 0};
+  auto multiply = [&](int slot) {
+#pragma unroll
+    for (int o = 0; o < OB; ++o)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[o][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[slot][o], bf[slot][j], acc[o][j], 0, 0, 0);
+  };
+  const int mine = (a.slices - wave + KW - 1) / KW;
+  int last = 0;                                // first slice of the wave's last round
+#pragma nounroll
+  for (; last + D < mine; last += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      multiply(d);
+      load(d, wave + (last + D + d) * KW);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < mine - last) multiply(d);
+#pragma unroll
+  for (int o = 0; o < OB; ++o)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) sums[(wave * B + o * NB + j) * 64 + lane] = acc[o][j];
+  __syncthreads();
+  if (wave >= B) return;
+  v4i t = bias;
+#pragma unroll
+  for (int k = 0; k < KW; ++k) t += sums[(k * B + wave) * 64 + lane];
+  if (a.relu_first) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = max(t[e], 0);
+  }
+  const uint32_t o = pack_sat4(requant_one<FAST>(t[0], mult[0], shift[0], hpot[0]), requant_one<FAST>(t[1], mult[1], shift[1], hpot[1]),
+                               requant_one<FAST>(t[2], mult[2], shift[2], hpot[2]), requant_one<FAST>(t[3], mult[3], shift[3], hpot[3]), a.lo);
+  if (row < a.rows && oc < ((a.oc + 15) & ~15)) *reinterpret_cast<uint32_t *>(a.y + (int64_t)row * a.y_cs + oc) = o;
+}
+
 uint32_t magic_of(int64_t d) { return (uint32_t)(0xffffffffull / (uint64_t)d); }
 
 template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, int NS>
@@ -411,4 +504,37 @@ void tpuhip::split_launch(tpuhip_ctx *ctx, const SplitVariant &v, const SplitPla
   if (v.kw == KW && v.pw == PW && v.nb == NB && v.ob == OB) return launch_variant<KW, PW, NB, OB>(ctx, pl, fast, uni, a, post);
   TPUHIP_SPLIT_VARIANTS(TPUHIP_FORM)
 #undef TPUHIP_FORM
+}
+
+// The blocks of a workgroup: those with which the busiest CU fetches the least, a workgroup fetching as many rows of operands as
+// it has channels and rows.  Of nine shapes timed with all four it names the fastest in seven (100 x 2048 x 1000: 4.33, 4.21, 4.36,
+// 6.29 us in the order below; 32 rows: 3.15, 4.05, 4.26, 4.93), 4 % from it in the others.
+void tpuhip::fc_split(tpuhip_ctx *ctx, const FcArgs &a, bool fast) {
+  const int kinds[][2] = {{1, 1}, {2, 1}, {2, 2}, {4, 2}};
+  int best = 0;
+  int64_t least = INT64_MAX;
+  for (int k = 0; k < 4; ++k) {
+    const int nb = kinds[k][0], ob = kinds[k][1];
+    const int64_t tiles = ceil_div64(a.oc, 16 * ob) * ceil_div64(a.rows, 16 * nb);
+    const int64_t cost = ceil_div64(tiles, ctx->num_cu) * (std::min(a.rows, 16 * nb) + 16 * ob);
+    if (cost < least) {
+      least = cost;
+      best = k;
+    }
+  }
+  const int nb = kinds[best][0], ob = kinds[best][1];
+  // channel tiles in whole rounds of the XCDs: those of one tile of channels meet its filter in one L2
+  const dim3 grid((unsigned)ceil_div64(ob == 2 ? ceil_div64(a.oc, 32) : 2 * ceil_div64(a.oc, 32), 8) * 8, (unsigned)ceil_div64(a.rows, 16 * nb));
+  auto go = [&](auto kernel) {
+    if (ctx->prof_start || ctx->prof_stop)
+      hipExtLaunchKernelGGL(kernel, grid, dim3(512), 0, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
+    else
+      hipLaunchKernelGGL(kernel, grid, dim3(512), 0, ctx->stream, a);
+  };
+  switch (best) {
+    case 0: return fast ? go(fc_split_kernel<1, 1, true>) : go(fc_split_kernel<1, 1, false>);
+    case 1: return fast ? go(fc_split_kernel<2, 1, true>) : go(fc_split_kernel<2, 1, false>);
+    case 2: return fast ? go(fc_split_kernel<2, 2, true>) : go(fc_split_kernel<2, 2, false>);
+    default: return fast ? go(fc_split_kernel<4, 2, true>) : go(fc_split_kernel<4, 2, false>);
+  }
 }

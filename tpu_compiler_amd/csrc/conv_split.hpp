@@ -55,4 +55,16 @@ bool split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const SplitPla
 void split_launch(tpuhip_ctx *ctx, const SplitVariant &v, const SplitPlan &pl, bool fast, bool uni, const SplitArgs &a,
                   const SplitPost *post);
 
+// FullyConnected from the filter as fragments of 32 channels x 32 bytes of K (the packing of mfma_reg_32x32)
+struct FcArgs {
+  const int8_t *x, *w;
+  int8_t *y;
+  const int32_t *bias;     // the planes as in SplitArgs
+  int nparam;
+  uint32_t x_bytes, w_bytes;
+  int rows, oc, x_cs, y_cs, slices;   // slices of 64 bytes of K
+  int relu_first, lo;
+};
+void fc_split(tpuhip_ctx *ctx, const FcArgs &a, bool fast);
+
 }  // namespace tpuhip
