@@ -4,7 +4,7 @@
 // permutes the result back; here the kernels find the operands through the tensors' 4-d views, and
 // so need no permuted copies (any batch, either transpose, results of rank 3 or 4).  The plain
 // [m,k] x [n,k] case runs on the conv path (tpuhip_fc_prepack).
-#include "common.hpp"
+#include "conv_epilogue.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -17,6 +17,7 @@ struct tpuhip_fc_batched_weights {
   int8_t *filter = nullptr;   // [batch][n][k], or its fragments (packed_filter)
   bool matrix = false;        // runs on fc_batched_mfma_kernel
   bool uniform = false;       // one (rshift, multiplier) for the whole batch
+  bool fast = false;          // no sum can overflow the requantisation's rounding
   int32_t *params = nullptr;  // bias [batch][n] (zeros without one), then multiplier[batch], rshift[batch]
   int64_t total = 0;          // result elements
 };
@@ -95,13 +96,14 @@ __global__ __launch_bounds__(256) void fc_batched_kernel(FcbArgs a) {
 // with four consecutive m per lane and register, is stored 16 bytes at a time (YM).  Any other view (m between, as in a
 // [batch_high, batch_low, m, k] tensor) is read and written byte by byte at the places that its index gives.
 //
-// Bound: the trip to memory for the rows and the filter, one after the other behind a barrier, then the launch: 32 products
-// of 160 x 64 by 64 x 160 took one lane per element 111 us, here 5.9.
+// Four steps of the filter, the bias and the pair (multiplier, shift) are requested before the rows are waited for; a block of 16
+// outputs a lane is requantised with that pair in scalars where one serves all of it.
+// Bound: launch and one trip to memory.  Replayed from a graph, before (a trip each for the rows, the second step and the
+// parameters; one WG of five blocks; pairs looked up per output) and now: 32 products of 160 x 64 x 160 5.33 -> 3.75 us, 12 of 384 x
+// 64 x 384 6.41 -> 4.21, 96 of 128 x 128 x 128 5.43 -> 4.31, 96 of 384 x 128 x 384 25.8 -> 16.0.
 // ---------------------------------------------------------------------------
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-
 constexpr int kChunkSteps = 16;                  // K steps of 32 per pass through LDS
+constexpr int kAhead = 4;                        // filter fragments in flight, before the rows are waited for
 constexpr int kRowBytes = kChunkSteps * 32 + 16;  // 16 bytes apart from the next bank cycle: 16-byte reads by row do not collide
 
 struct View {
@@ -120,26 +122,40 @@ struct FcbMfmaArgs {
   const int32_t *bias, *mult, *rshift;
   int8_t *y;
   View xv, yv;
-  int m, k, n, low, steps, tiles, relu, uniform, in_t, out_t;
+  int m, k, n, low, steps, tiles, per_wg, relu, uniform, in_t, out_t;   // per_wg: blocks of columns of a workgroup
   FastDiv by_mtiles, by_nblocks, by_low, by_mn;
 };
 
-template <bool XM, bool YM>
+// SIMPLE: one multiplier and shift for all that a workgroup writes, and sums that cannot overflow the rounding
+template <bool XM, bool YM, bool SIMPLE>
 __global__ __launch_bounds__(256) void fc_batched_mfma_kernel(FcbMfmaArgs a) {
   __shared__ __attribute__((aligned(16))) int8_t rows[32 * kRowBytes];
   __shared__ uint32_t base[32], stride[32];
+  asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.mult), "s"(a.rshift), "s"(a.y), "s"(a.xv.cs), "s"(a.yv.cs), "s"(a.m), "s"(a.k),
+               "s"(a.n), "s"(a.low), "s"(a.steps), "s"(a.tiles), "s"(a.per_wg), "s"(a.by_mtiles.mul), "s"(a.by_nblocks.mul),
+               "s"(a.by_low.mul));   // named here they arrive together
   uint32_t nb = blockIdx.x, mt = a.by_nblocks.split(nb), b = a.by_mtiles.split(mt);
   uint32_t lb = b;
   const uint32_t hb = a.by_low.split(lb);
   const int m0 = (int)mt * 32, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
-  const int t0 = (int)nb * 8 + wave, t1 = t0 + 4;   // this wave's blocks of columns
-  const bool have0 = t0 < a.tiles, have1 = t1 < a.tiles;
+  const int t0 = (int)nb * a.per_wg + wave, t1 = t0 + 4;   // this wave's blocks of columns
+  const bool have0 = wave < a.per_wg && t0 < a.tiles, have1 = wave + 4 < a.per_wg && t1 < a.tiles;
   const int8_t *w0 = a.w + (((int64_t)b * a.tiles + (have0 ? t0 : 0)) * a.steps * 64 + lane) * 16;
   const int8_t *w1 = a.w + (((int64_t)b * a.tiles + (have1 ? t1 : 0)) * a.steps * 64 + lane) * 16;
   v16i acc0 = {}, acc1 = {};
-  v4i f0 = {}, f1 = {};
-  if (have0) f0 = *reinterpret_cast<const v4i *>(w0);
-  if (have1) f1 = *reinterpret_cast<const v4i *>(w1);
+  v4i f0[kAhead] = {}, f1[kAhead] = {};
+#pragma unroll
+  for (int d = 0; d < kAhead; ++d) {
+    if (have0 && d < a.steps) f0[d] = *reinterpret_cast<const v4i *>(w0 + d * 1024);
+    if (have1 && d < a.steps) f1[d] = *reinterpret_cast<const v4i *>(w1 + d * 1024);
+  }
+  int32_t bias_of[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int nn = (t ? t1 : t0) * 32 + col;
+    bias_of[t] = (t ? have1 : have0) && nn < a.n ? a.bias[(int64_t)b * a.n + nn] : 0;
+  }
+  const int32_t mult_b = a.mult[b], shift_b = a.rshift[b];
   if (!XM && threadIdx.x < 32) {
     // logical index of the row's first element, byte offset and the bytes from one element to the next
     const uint32_t mm = (uint32_t)min(m0 + (int)threadIdx.x, a.m - 1);
@@ -180,15 +196,19 @@ __global__ __launch_bounds__(256) void fc_batched_mfma_kernel(FcbMfmaArgs a) {
     }
     __syncthreads();
     const int8_t *mine = rows + col * kRowBytes + half * 16;
-    for (int s = 0; s < steps; ++s) {
-      const v4i fa = *reinterpret_cast<const v4i *>(mine + s * 32);
-      const v4i g0 = f0, g1 = f1;
-      if (s0 + s + 1 < a.steps) {   // the next step's fragments while this one is multiplied
-        if (have0) f0 = *reinterpret_cast<const v4i *>(w0 + (int64_t)(s0 + s + 1) * 1024);
-        if (have1) f1 = *reinterpret_cast<const v4i *>(w1 + (int64_t)(s0 + s + 1) * 1024);
+    for (int s = 0; s < steps; s += kAhead) {
+#pragma unroll
+      for (int d = 0; d < kAhead; ++d) {
+        if (s + d >= steps) break;
+        const v4i fa = *reinterpret_cast<const v4i *>(mine + (s + d) * 32);
+        acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, f0[d], acc0, 0, 0, 0);
+        if (have1) acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, f1[d], acc1, 0, 0, 0);
+        const int next = s0 + s + d + kAhead;   // (kChunkSteps is a multiple of kAhead: a step's slot is the same in every pass)
+        if (next < a.steps) {
+          if (have0) f0[d] = *reinterpret_cast<const v4i *>(w0 + (int64_t)next * 1024);
+          if (have1) f1[d] = *reinterpret_cast<const v4i *>(w1 + (int64_t)next * 1024);
+        }
       }
-      acc0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, g0, acc0, 0, 0, 0);
-      if (have1) acc1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, g1, acc1, 0, 0, 0);
     }
   }
   // a lane holds, of column col, rows 8 * (i / 4) + 4 * half + i % 4
@@ -197,9 +217,34 @@ __global__ __launch_bounds__(256) void fc_batched_mfma_kernel(FcbMfmaArgs a) {
     const v16i &acc = t ? acc1 : acc0;
     const int nn = (t ? t1 : t0) * 32 + col;
     if (!(t ? have1 : have0)) continue;
-    const int32_t bias = nn < a.n ? a.bias[(int64_t)b * a.n + nn] : 0;
-    int32_t mult = a.mult[b], e = a.rshift[b];
+    const int32_t bias = bias_of[t];
+    int32_t mult = mult_b, e = shift_b;
     uint32_t word[4];
+    if constexpr (SIMPLE) {
+      const int32_t hpot = 1 << (e - 1);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        int32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          int32_t s = acc[q * 4 + i] + bias;
+          if (a.relu) s = max(s, 0);
+          const int32_t x = srdhm(s, mult);
+          v[i] = (x + hpot + (x >> 31)) >> e;
+        }
+        const uint32_t w = pack_sat4(v[0], v[1], v[2], v[3], -128);
+        const int mm = m0 + 8 * q + 4 * half, live = a.m - mm;
+        word[q] = live >= 4 ? w : live > 0 ? w & ((1u << (8 * live)) - 1u) : 0;
+        if (!YM && nn < a.n) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (i < live) {
+              const uint32_t f = a.out_t ? ((hb * a.m + (uint32_t)(mm + i)) * a.low + lb) * a.n + nn : (b * a.m + (uint32_t)(mm + i)) * a.n + nn;
+              a.y[a.yv.at(f)] = (int8_t)(w >> (8 * i));
+            }
+        }
+      }
+    } else
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       int32_t s = acc[i] + bias;
@@ -290,10 +335,16 @@ int tpuhip_fc_batched_prepack(tpuhip_ctx *ctx, const tpuhip_fc_batched_desc *des
   // on the matrix cores unless padding the filter to 32 x 32 would blow it up beyond reason, or the grid (2^24 workgroups) or
   // the kernel's 31-bit byte offsets do not reach
   const int64_t padded = batch * round_up(d.n, 32) * round_up(d.k, 32);
-  const int64_t groups = batch * ((d.m + 31) / 32) * ((d.n + 255) / 256);
+  const int64_t groups = batch * ((d.m + 31) / 32) * ((d.n + 255) / 256);   // as many as of one block a wave stay below 4 a CU
   const int64_t x_bytes = batch * d.m * d.k / d.x_c * d.x_cs, y_bytes = batch * d.m * d.n / d.y_c * d.y_cs;
   w->matrix = padded <= std::max<int64_t>(32 << 20, 4 * batch * d.n * d.k) && groups < (1 << 24) && x_bytes < (1ll << 31) &&
               y_bytes < (1ll << 31);
+  // RoundingDivideByPOT without its sign-dependent mask: shifts of 1 and more, and sums that with the rounding term fit 32 bits
+  int64_t largest = 0;
+  for (int64_t i = 0; bias && i < batch * d.n; ++i) largest = std::max<int64_t>(largest, std::abs((int64_t)bias[i]));
+  w->fast = true;
+  for (int64_t i = 0; i < batch; ++i)
+    w->fast &= rshift[i] >= 1 && (int64_t)d.k * 128 * 128 + largest + 1 + (1ll << (rshift[i] - 1)) < (1ll << 31);
   w->uniform = std::count(multiplier, multiplier + batch, multiplier[0]) == batch && std::count(rshift, rshift + batch, rshift[0]) == batch;
   std::vector<int8_t> packed;
   if (w->matrix) {
@@ -346,7 +397,12 @@ int tpuhip_fc_batched_i8(tpuhip_ctx *ctx, const tpuhip_fc_batched_weights *w, co
     a.tiles = (d.n + 31) / 32;
     a.relu = d.do_relu; a.uniform = w->uniform;
     a.in_t = d.input_transpose; a.out_t = d.output_transpose;
-    const int mtiles = (d.m + 31) / 32, nblocks = (d.n + 255) / 256;
+    // a wave takes two blocks of columns only where there are workgroups enough without that: 32 products of 160 x 64 x 160 are 160
+    // of them so, one wave in four with two blocks, and 320 of three and two blocks without
+    const int mtiles = (d.m + 31) / 32;
+    const bool wide = batch * mtiles * ((a.tiles + 3) / 4) > 4 * (int64_t)ctx->num_cu;
+    const int nblocks = wide ? (a.tiles + 7) / 8 : (a.tiles + 3) / 4;
+    a.per_wg = (a.tiles + nblocks - 1) / nblocks;
     a.by_mtiles = FastDiv(mtiles); a.by_nblocks = FastDiv(nblocks); a.by_low = FastDiv(d.batch_low);
     a.by_mn = FastDiv((int64_t)d.m * d.n);
     // m contiguous: the view's channels are the rows and the rest is one product's (or one batch_high's) columns
@@ -354,8 +410,11 @@ int tpuhip_fc_batched_i8(tpuhip_ctx *ctx, const tpuhip_fc_batched_weights *w, co
                     (uintptr_t)x % 4 == 0;
     const bool ym = d.y_c == d.m && (int64_t)d.y_h * d.y_w == (d.output_transpose ? (int64_t)d.batch_low * d.n : d.n) && d.y_cs % 16 == 0 &&
                     (uintptr_t)y % 16 == 0;
-    auto *kernel = xm ? ym ? fc_batched_mfma_kernel<true, true> : fc_batched_mfma_kernel<true, false>
-                      : ym ? fc_batched_mfma_kernel<false, true> : fc_batched_mfma_kernel<false, false>;
+    const bool simple = w->fast && (w->uniform || !d.output_transpose);
+    auto *kernel = xm   ? ym ? simple ? fc_batched_mfma_kernel<true, true, true> : fc_batched_mfma_kernel<true, true, false>
+                             : simple ? fc_batched_mfma_kernel<true, false, true> : fc_batched_mfma_kernel<true, false, false>
+                   : ym ? simple ? fc_batched_mfma_kernel<false, true, true> : fc_batched_mfma_kernel<false, true, false>
+                        : simple ? fc_batched_mfma_kernel<false, false, true> : fc_batched_mfma_kernel<false, false, false>;
     launch(ctx, kernel, dim3((unsigned)(batch * mtiles * nblocks)), dim3(256), a);
     TPUHIP_CHECK_HIP(hipGetLastError());
     return TPUHIP_OK;
