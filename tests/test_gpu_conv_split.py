@@ -42,6 +42,11 @@ CASES = [
     (1, 1024, 14, 14, 70, (1, 1), (1, 1), (0, 0, 0, 0), (1, 1), False),     # straight from memory
     (2, 256, 9, 7, 130, (1, 1), (2, 2), (0, 0, 0, 0), (1, 1), True),
     (1, 96, 11, 5, 24, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), True),         # slices that straddle taps
+    (2, 100, 9, 13, 40, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), False),       # 63 groups of 16 bytes: one past the end of K
+    (1, 37, 20, 21, 50, (5, 5), (2, 2), (2, 2, 2, 2), (1, 1), True),        # 75 groups
+    (1, 250, 8, 30, 48, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), True), (2, 16, 12, 7, 20, (2, 4), (1, 1), (1, 0, 2, 1), (2, 1), False),
+    (1, 290, 9, 11, 33, (3, 3), (1, 1), (1, 1, 1, 1), (1, 1), False), (2, 64, 9, 9, 20, (7, 7), (1, 1), (3, 3, 3, 3), (1, 1), True),
+    (1, 130, 30, 9, 24, (7, 1), (1, 1), (3, 3, 0, 0), (1, 1), True),
     (3, 16, 5, 6, 33, (1, 1), (1, 1), (0, 0, 0, 0), (1, 1), False), (1, 3, 8, 9, 40, (3, 3), (2, 2), (1, 1, 1, 1), (1, 1), True),
 ]
 
@@ -89,7 +94,7 @@ def test_against_the_oracle(ctx, tile, case, post):
 
 
 @pytest.mark.parametrize("tile", SPLIT_TILES, ids=_name)
-@pytest.mark.parametrize("case", [CASES[0], CASES[12], CASES[14]], ids=lambda c: "x".join(map(str, c[:5])))
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[12], CASES[14]], ids=lambda c: "x".join(map(str, c[:5])))
 @pytest.mark.parametrize("relu_first", [0, 1])
 def test_shifts_of_zero_and_a_relu_in_front(ctx, tile, case, relu_first):
     """the requantisation that may overflow, without the patch; a ReLU on the sum"""

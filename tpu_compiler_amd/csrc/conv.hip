@@ -4072,10 +4072,11 @@ struct TileCfg {
   U4(74, "mfma_rows_64x256_c32", 2, 2, 1, 4, 1, 4, 4) 
 
 // K split over the waves of a workgroup, blocks of 16 x 16 (conv_split.hip):
-// SP(index, name, waves along K, along the pixels, blocks of 16 pixels and of 16 channels per wave).  Of 52 layers of 1 to 4 images
-// of 5 to 60 pixels a side (1x1 to 5x5, stride 1 and 2, dilation, 64 to 1024 channels) one of them is the fastest of all in 36, by
-// 1 % to 2.7 times (profiles/conv_split_tiles.txt): 16x32 in 13 (by up to 17 % over the next of them), 16x16_w4 in 10 (14 %), 16x16
-// in 5 (18 %), 32x32 in 5 (55 %), 32x64 in 2 (13 %), 16x64 in one (22 %); 32x128 leads at 128 -> 256 on 52 x 52 (2 %).
+// SP(index, name, waves along K, along the pixels, blocks of 16 pixels and of 16 channels per wave).  Of 114 layers (the networks of
+// one image, and layers drawn of 1 to 8 images of 5 to 107 pixels a side, 16 to 1024 channels, 1x1 to 5x5, stride 1 and 2, dilation)
+// one of them is the fastest of all in 91, by 1 % to 2.8 times (profiles/conv_split_tiles.txt): 16x16_w4 in 32 (by up to 12 % over
+// the next of them), 32x32 in 16 (52 %), 16x32 in 15 (16 %), 32x64 in 13 (32 %), 16x16 in 12 (17 %), 32x128 in 2 (5 %), 16x64 in one
+// (25 %).
 #define TPUHIP_SPLIT_TILES(SP)               \
   SP(75, "mfma_split_16x16_w4", 4, 1, 1, 1)  \
   SP(76, "mfma_split_16x16", 8, 1, 1, 1)     \
@@ -4753,9 +4754,9 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t, int num_cu) {
   // fastest of all in 10 at 256 tiles (256 -> 256 channels 3x3: 5.3 us against 7.4), in 3 at 512, in none at 1024 (14.3
   // against 8.2) and 2048 (27.0 against 13.2): the line is four times where they were last seen to win
   if (c.reg == 8 && ceil_div64((int64_t)d.n * d.oh * d.ow, 32) * ceil_div64(d.oc, 32) > 2048) return false;
-  // likewise: of 74 layers the most tiles with which a variant was the fastest were 512 (512 -> 2048 channels 1x1 on 7 x 7: 2.95 us
-  // against 3.00); with 832 (256 -> 1024 on 14 x 14) 3.5 against 2.9 of the blocks of 32 x 32.  The line is twice the former
-  if (c.reg == 10 && split_tiles(d, c.split, split_plan(d, c.split, true)) > 1024) return false;
+  // likewise: of 114 layers the most tiles with which a variant was the fastest were 752 (64 -> 255 channels 1x1 on 44 x 17: 2.66 us
+  // against 2.88 of the blocks of 32 x 32).  The line lies at nearly three times that
+  if (c.reg == 10 && split_tiles(d, c.split, split_plan(d, c.split, true)) > 2048) return false;
   if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8 || c.reg == 10)) return false;   // prefer the 4-channel K packing of the LDS kernels
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle
 }

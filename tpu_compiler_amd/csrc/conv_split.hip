@@ -14,9 +14,10 @@
 // wave, four channels of a pixel per lane.
 //
 // Replayed from a graph (a launch of nothing is 1.7 us there), against the best of the other forms: 3x3 of 512 channels on 7 x 7
-// 6.7 -> 4.0 us, 256 on 14 x 14 4.84 -> 3.34, 256 -> 512 on 26 x 26 6.87 -> 5.4, 512 -> 1024 on 13 x 13 7.1 -> 5.2, at stride 2
-// from 26 x 26 7.2 -> 5.9; 1x1 2048 -> 512 on 7 x 7 4.5 -> 3.1, 1024 -> 256 on 14 x 14 3.5 -> 2.6; 5x5 at stride 2, 128 channels on
-// 4 x 45 x 53, 9.0 -> 6.9.  What is left of the large ones is the same link: 112 KB per CU at 26 x 26 are 1.9 us.
+// 6.7 -> 4.0 us, 256 on 14 x 14 4.84 -> 3.37, 64 on 56 x 56 3.21 -> 2.84, 256 -> 512 on 26 x 26 6.87 -> 5.5, 512 -> 1024 on 13 x 13
+// 7.1 -> 5.2, at stride 2 from 26 x 26 7.2 -> 6.0; 1x1 2048 -> 512 on 7 x 7 4.5 -> 3.2, 1024 -> 256 on 14 x 14 3.5 -> 2.65; 5x5 at
+// stride 2, 128 channels on 4 x 45 x 53, 9.0 -> 6.9.  What is left of the large ones is the same link: 112 KB per CU at 26 x 26 are
+// 1.9 us.
 #include "conv_split.hpp"
 
 #include "conv_epilogue.hpp"
@@ -46,7 +47,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   // named here, the arguments leave the scalar cache together instead of one by one where they are first needed
   asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.x_bytes), "s"(a.n_tiles), "s"(a.n_pix), "s"(a.shape), "s"(a.magic_tile),
                "s"(a.magic_img), "s"(a.magic_row), "s"(a.magic_c16), "s"(a.magic_kw), "s"(a.magic_pw), "s"((int)a.per_img), "s"((int)a.ih),
-               "s"((int)a.x_cs), "s"((int)a.sh), "s"((int)a.dh), "s"((int)a.slices_relu), "s"((int)a.nparam16));
+               "s"((int)a.x_cs), "s"((int)a.sh), "s"((int)a.dh), "s"((int)a.slices_pad_relu), "s"((int)a.nparam16));
   extern __shared__ v4i lds[];   // the patch, [group][wave of K][block][lane] sums, the table's 256 bytes
   constexpr int T = KW * PW * 64, B = NB * OB, FIN = (B + KW - 1) / KW;   // FIN: blocks that a wave finishes
   const int tid = threadIdx.x, lane = tid & 63;
@@ -66,7 +67,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
     oc_tile = wt - major * n_oc;
   }
   const int oc0 = (int)oc_tile * (16 * OB);
-  const int slices = a.slices_relu >> 2;
+  const int slices = a.slices_pad_relu >> 4, groups = 4 * slices - (a.slices_pad_relu >> 2 & 3);   // groups of 16 bytes of K
   const int px = lane & 15, chunk = lane >> 4;
   const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t wrsrc =
@@ -79,7 +80,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   bool out_ok[FIN];
   uint32_t out_base = 0, img = 0;
   int oh0 = 0, ow0 = 0, rows = 0, cols = 0;
-  const int pitch = a.c16 * 16 + 16;           // of a position in LDS
+  const int pitch = (a.c16 | 1) * 16;          // of a position in LDS: an odd number of 16 bytes, for 16 positions on all banks
   const int th = a.shape & 255, tw = a.shape >> 8 & 255, ph = a.shape >> 16;
   const int pw = (tw - 1) * a.sw + (a.kw - 1) * a.dw + 1;
   if (PATCH) {
@@ -98,7 +99,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
     if (PATCH) {
       const uint32_t r = row_of(slot), c = slot - r * tw;
       const bool ok = (int)r < rows && (int)c < cols;
-      at[j] = ok ? (r * a.sh * pw + c * a.sw) * pitch + chunk * 16 : chunk * 16;
+      at[j] = (ok ? (r * a.sh * pw + c * a.sw) * pitch : 0) + (UNI ? chunk * 16 : 0);
     } else {
       const uint32_t pix = pix_tile * (PW * NB * 16) + slot;
       const uint32_t q = div_by(pix, a.magic_row), c = pix - q * a.ow, n = div_by(q, a.magic_img), r = q - n * a.oh;
@@ -156,6 +157,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   if (PATCH) fetch_patch(0);
 #pragma unroll
   for (int d = 0; d < D; ++d) {
+    if (!PATCH && wk + d * KW >= slices) break;
     load_filter(d, wk + d * KW);
     if (!PATCH) load_input(d, wk + d * KW);
   }
@@ -164,7 +166,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   const bool second = POST && post->split_oc > 0 && oc0 >= post->split_oc;
   int8_t *const y = second ? post->y2 : a.y;
   const int y_cs = second ? post->y2_cs : a.y_cs, oc_shift = second ? post->split_oc : 0;
-  const int lo = second ? post->lo2 : (a.slices_relu & 3) == 1 ? 0 : -128;
+  const int lo = second ? post->lo2 : (a.slices_pad_relu & 3) == 1 ? 0 : -128;
   v4i bias[FIN], mult[FIN], shift[FIN], hpot[FIN];
   uint32_t src[FIN];
   int64_t off[FIN];
@@ -194,7 +196,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
       if (POST && ok && post->add_dst) src[f] = *reinterpret_cast<const uint32_t *>(post->add_src + off[f]);
     }
   }
-  v4i *const sums = lds + (PATCH ? ph * pw * (a.c16 + 1) : 0);
+  v4i *const sums = lds + (PATCH ? ph * pw * (a.c16 | 1) : 0);
   uint8_t *const lut = reinterpret_cast<uint8_t *>(sums + KW * PW * B * 64);
   uint32_t lutv = 0;
   if (POST && post->has_lut && tid < 64) lutv = post->lut.w[tid];
@@ -219,7 +221,8 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   auto multiply = [&](int slot, int s) {
     v4i b[NB];
     if (PATCH) {
-      const uint32_t kg = 4u * (uint32_t)min(s, slices - 1);   // past the end the filter is zeros
+      // past the end the filter is zeros
+      const uint32_t kg = UNI ? 4u * (uint32_t)min(s, slices - 1) : (uint32_t)min(4 * s + chunk, groups - 1);
       const uint32_t tap = div_by(kg, a.magic_c16), cgrp = kg - tap * a.c16, tkh = div_by(tap, a.magic_kw), tkw = tap - tkh * a.kw;
       const char *from = reinterpret_cast<const char *>(lds) + (tkh * a.dh * pw + tkw * a.dw) * pitch + cgrp * 16;
 #pragma unroll
@@ -244,7 +247,10 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
     }
   }
 #pragma unroll
-  for (int d = 0; d < D; ++d) multiply(d, wk + (i0 + d) * KW);   // slices past the end are zeros
+  for (int d = 0; d < D; ++d) {
+    if (!PATCH && i0 + d >= mine) break;
+    multiply(d, wk + (i0 + d) * KW);   // patch form: slices past the end are zeros
+  }
 
   // ---- the sums meet
   if (POST && post->has_lut && tid < 64) reinterpret_cast<uint32_t *>(lut)[tid] = lutv;
@@ -260,7 +266,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
     v4i t = bias[f];
 #pragma unroll
     for (int k = 0; k < KW; ++k) t += sums[((wg * KW + k) * B + b) * 64 + lane];
-    if (a.slices_relu & 2) {
+    if (a.slices_pad_relu & 2) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) t[e] = max(t[e], 0);
     }
@@ -413,8 +419,9 @@ void launch_form(tpuhip_ctx *ctx, unsigned lds, const SplitArgs &a, const SplitP
 template <int KW, int PW, int NB, int OB>
 void launch_variant(tpuhip_ctx *ctx, const SplitPlan &pl, bool fast, bool uni, const SplitArgs &a, const SplitPost *post) {
   if (pl.th) {
-    const int mine = ((a.slices_relu >> 2) + KW - 1) / KW;
-    if (mine <= 2) launch_form<KW, PW, NB, OB, true, true, true, 2>(ctx, pl.lds, a, post);
+    const int mine = ((a.slices_pad_relu >> 4) + KW - 1) / KW;
+    if (!uni) mine <= 3 ? launch_form<KW, PW, NB, OB, true, false, true, 3>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, true, false, true, 6>(ctx, pl.lds, a, post);
+    else if (mine <= 2) launch_form<KW, PW, NB, OB, true, true, true, 2>(ctx, pl.lds, a, post);
     else if (mine <= 3) launch_form<KW, PW, NB, OB, true, true, true, 3>(ctx, pl.lds, a, post);
     else if (mine <= 5) launch_form<KW, PW, NB, OB, true, true, true, 5>(ctx, pl.lds, a, post);
     else launch_form<KW, PW, NB, OB, true, true, true, 9>(ctx, pl.lds, a, post);
@@ -426,17 +433,23 @@ void launch_variant(tpuhip_ctx *ctx, const SplitPlan &pl, bool fast, bool uni, c
 
 }  // namespace
 
-// The patch form: a window that overlaps itself, channels in whole slices, a patch that fits; as many whole rows as the slots
-// hold, or the part of a row that they hold, evened out over the image.
+// The patch form: a window of more than one tap, a patch that fits; as many whole rows as the slots hold, or the part of a row
+// that they hold, evened out over the image.  It saves what the taps of a block's pixels share and costs a trip through LDS and a
+// barrier, so the line lies by the K that is fetched and the pixels of a wave.  Straight from memory / as a patch, from a graph:
+//   16 pixels and 32: 64 -> 512 on 2 x 6 x 40 at stride 2 (9 slices) 2.43 / 3.05 us, 192 -> 96 on 35 x 19 (27) 2.97 / 3.86, 256 ->
+//     256 on 14 x 14 (36) 3.5 / 3.37, 512 -> 512 on 7 x 7 (72) 4.54 / 4.03, 512 -> 1024 on 13 x 13 (72) 7.89 / 5.23;
+//   64 and 128: 64 -> 64 on 56 x 56 (9) 3.07 / 3.7, 128 -> 256 on 52 x 52 (18) 6.5 / 5.87, 256 -> 512 on 26 x 26 (36) 7.56 / 5.54.
 SplitPlan tpuhip::split_plan(const tpuhip_conv_desc &d, const SplitVariant &v, bool fast) {
   SplitPlan pl;
   const int slots = v.pw * v.nb * 16;
   const unsigned rest = (unsigned)(v.kw * v.pw * v.nb * v.ob) * 1024u + 256u;
   pl.lds = rest;
-  if (!fast || d.ic % 64 || d.kh * d.kw == 1) return pl;
+  const int slices = (d.kh * d.kw * ((d.ic + 15) / 16) + 3) / 4;
+  if (!fast || d.kh * d.kw == 1 || slices <= (v.nb <= 2 ? 32 : 16)) return pl;
+  const int pitch = ((d.ic + 15) / 16 | 1) * 16;
   auto width = [&](int tw) { return (int64_t)(tw - 1) * d.sw + (int64_t)(d.kw - 1) * d.dw + 1; };
   auto height = [&](int th) { return (int64_t)(th - 1) * d.sh + (int64_t)(d.kh - 1) * d.dh + 1; };
-  auto bytes = [&](int th, int tw) { return height(th) * width(tw) * (d.ic + 16) + rest; };
+  auto bytes = [&](int th, int tw) { return height(th) * width(tw) * pitch + rest; };
   int th = std::max(1, std::min(d.oh, slots / std::min(d.ow, slots))), tw = std::min(d.ow, slots);
   while (th > 1 && bytes(th, tw) > kLdsBytes) --th;
   while (tw > 1 && bytes(th, tw) > kLdsBytes) --tw;
@@ -461,7 +474,7 @@ bool tpuhip::split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const 
   const int c16 = (d.ic + 15) / 16, slices = (d.kh * d.kw * c16 + 3) / 4;
   const int64_t n_oc = ceil_div64(d.oc, 16 * v.ob), tiles = split_tiles(d, v, pl), n_pix = tiles / n_oc;
   const int64_t npix = (int64_t)d.n * d.oh * d.ow, in_bytes = (int64_t)d.n * d.ih * d.iw * d.x_cs;
-  for (int64_t u16 : {d.ih, d.iw, d.oh, d.ow, d.x_cs, d.y_cs, d.oc, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw, d.kw, 4 * slices + 2, nparam / 16})
+  for (int64_t u16 : {d.ih, d.iw, d.oh, d.ow, d.x_cs, d.y_cs, d.oc, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw, d.kw, 16 * slices + 15, nparam / 16})
     if (u16 < 0 || u16 > 65535) return false;
   // the divisions by multiplying are exact where number * divisor stays below 2^32
   if (nparam % 16 || in_bytes >= 1ll << 31 || n_oc * v.ob * slices * 1024 >= 1ll << 31) return false;
@@ -493,7 +506,7 @@ bool tpuhip::split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const 
   a.sh = (uint16_t)d.sh; a.sw = (uint16_t)d.sw; a.pt = (uint16_t)d.pt; a.pl = (uint16_t)d.pl;
   a.dh = (uint16_t)d.dh; a.dw = (uint16_t)d.dw; a.kw = (uint16_t)d.kw;
   a.nparam16 = (uint16_t)(nparam / 16);
-  a.slices_relu = (uint16_t)(slices * 4 + (!d.do_relu ? 0 : d.relu_first ? 2 : 1));
+  a.slices_pad_relu = (uint16_t)(slices * 16 + (4 * slices - d.kh * d.kw * c16) * 4 + (!d.do_relu ? 0 : d.relu_first ? 2 : 1));
   *out = a;
   return true;
 }

@@ -23,7 +23,8 @@ struct SplitArgs {
   uint16_t ih, iw, oh, ow, x_cs, y_cs, oc, c16;
   uint16_t sh, sw, pt, pl, dh, dw, kw;
   uint16_t nparam16;           // entries of a plane, by 16
-  uint16_t slices_relu;        // slices of 64 bytes of K, times 4; 1: ReLU behind the requantisation, 2: in front of it
+  uint16_t slices_pad_relu;    // slices of 64 bytes of K << 4 | groups of 16 bytes past its end << 2 | 1: ReLU behind the
+                               // requantisation, 2: in front of it
 };
 static_assert(sizeof(SplitArgs) <= 112, "see above");
 
