@@ -122,6 +122,16 @@ static_assert(sizeof(MoveArgs<kTile>) <= 112 && sizeof(MoveArgs<kCrop>) <= 112 &
                   sizeof(MoveArgs<kPadConst>) <= 112 && sizeof(MoveArgs<kSwap>) <= 112 && sizeof(MoveArgs<kDilate>) <= 112,
               "see MovePlan");
 
+// 4 x 4 bytes: byte k of row i becomes byte i of t[k]
+__device__ __forceinline__ void transpose_bytes(const uint32_t (&r)[4], uint32_t (&t)[4]) {
+  const uint32_t lo0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u), hi0 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
+  const uint32_t lo1 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u), hi1 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+  t[0] = __builtin_amdgcn_perm(lo1, lo0, 0x05040100u);
+  t[1] = __builtin_amdgcn_perm(lo1, lo0, 0x07060302u);
+  t[2] = __builtin_amdgcn_perm(hi1, hi0, 0x05040100u);
+  t[3] = __builtin_amdgcn_perm(hi1, hi0, 0x07060302u);
+}
+
 // where output channel c of pixel (n, h, w) comes from, and how many channels from it on, c included, lie one after the other
 // in the source as well (p null: without a source, that many take a.fill).  A source row that ends with the output's ends in
 // zero pad bytes up to a multiple of 16: `left` is then 16.
@@ -245,6 +255,24 @@ __device__ __forceinline__ v4i group_of_bytes(const MoveArgs<F> &a, int n, int h
     if constexpr (F == kShuffle) {
       g = (uint32_t)c0;
       col = a.by_a.split(g);
+      // Two and four groups, 16 channels that exist: runs of 8 or 4 bytes of each group, at any alignment, woven in registers.
+      // Replayed from a graph, byte by byte and now: four groups of 4 x 96 x 78 x 66 3.72 -> 2.33 us, 16 x 320 x 100 x 90 43 -> 15.
+      if (a.by_a.d == 4 && live == 16) {
+        uint32_t r[4], t[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) __builtin_memcpy(&r[k], row + (int64_t)k * a.p[1] + col, 4);
+        transpose_bytes(r, t);
+        return v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
+      }
+      if (a.by_a.d == 2 && live == 16) {
+        uint32_t r[2][2];
+        __builtin_memcpy(r[0], row + col, 8);
+        __builtin_memcpy(r[1], row + a.p[1] + col, 8);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          out[q] = (int)__builtin_amdgcn_perm(r[1][q >> 1], r[0][q >> 1], q & 1 ? 0x07030602u : 0x05010400u);
+        return out;
+      }
     }
   }
   uint32_t bytes[16];
@@ -303,15 +331,11 @@ __global__ __launch_bounds__(kThreads) void depth_by_two_kernel(MoveWith<MoveTai
       // channels past the last are the zero pad bytes of the input's row, or lie beyond its stride
       v4i v = {0, 0, 0, 0};
       if (c0 * 4 + q * 16 < a.ics) v = *reinterpret_cast<const v4i *>(a.x + (int64_t)pix * a.ics + c0 * 4 + q * 16);
-      // 4 x 4 bytes transposed
-      const uint32_t lo0 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x05010400u),
-                     hi0 = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x07030602u),
-                     lo1 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x05010400u),
-                     hi1 = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x07030602u);
-      out[0][q] = __builtin_amdgcn_perm(lo1, lo0, 0x05040100u);
-      out[1][q] = __builtin_amdgcn_perm(lo1, lo0, 0x07060302u);
-      out[2][q] = __builtin_amdgcn_perm(hi1, hi0, 0x05040100u);
-      out[3][q] = __builtin_amdgcn_perm(hi1, hi0, 0x07060302u);
+      const uint32_t r[4] = {(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+      uint32_t t[4];
+      transpose_bytes(r, t);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) out[k][q] = t[k];
     }
   }
   int8_t *to = a.y + ((int64_t)row * 2 * a.ow + 2 * w) * a.ocs() + c0;
@@ -545,35 +569,44 @@ struct PermTileArgs {
 };
 static_assert(sizeof(PermRowsArgs) <= 112 && sizeof(PermTileArgs) <= 112, "see MovePlan");
 
-// the channels change places with dimension j: 64 x 64 byte tiles through LDS, dword loads along
-// the input's channels, dword stores along the output's (pad channels of the output written as
-// zero: tile rows past the end of dimension j are zero)
+// The channels change places with dimension j: tiles of 64 (Q 16) or 128 channels (32) x 64 of j, 4 x 4 bytes of a lane transposed
+// in registers, dwords through LDS, so that the input is read in runs of 64 or 128 bytes and the output written in runs of 64 (its
+// pad channels as zero: rows past the end of dimension j are zeros).  More than 64 channels take the wider tile: with the other
+// the second half of a line is fetched again by another XCD.  NCHW -> NHWC order, replayed from a graph, with bytes read from
+// LDS before / 64 channels / now: 4 x 96 x 78 x 66 3.43 / 3.04 / 3.07 us, 16 x 320 x 100 x 90 30.6 / 30.3 / 27.9.  Bound by the reads
+// of 128 bytes, a row of the map apart each (97 MB are 15 us as a copy).
+template <int Q>
 __global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermTileArgs q) {
-  __shared__ __attribute__((aligned(4))) int8_t tile[64][68];
-  const int c0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
+  __shared__ uint32_t tile[Q * 4 * 17];   // [channel][four of j]
+  const int c0 = blockIdx.y * (Q * 4), j0 = blockIdx.x * 64;
   uint32_t ib = q.plane0 + blockIdx.z;   // below 2^31, as all pixels are
   const int64_t ia = q.by_b.split(ib);
   const int8_t *src = q.x + ia * q.Sa + ib * q.Sb;
   int8_t *dst = q.y + ia * q.Ta + ib * q.Tb;
-  const int tq = threadIdx.x & 15, tr = threadIdx.x >> 4;   // 16 dwords per row, 16 rows per pass
+  constexpr int kPasses = 16 * Q / kThreads;
+  const int cq = threadIdx.x % Q, cc = c0 + cq * 4;
+  uint32_t r[kPasses][4];
+  // the input's pad channels are zero and its channel stride is a multiple of 16, so a dword that starts inside the row may be
+  // read whole
 #pragma unroll
-  for (int r = tr; r < 64; r += 16) {
-    const int jj = j0 + r, cc = c0 + tq * 4;
-    uint32_t v = 0;
-    // the input's pad channels are zero and its channel stride is a multiple of 16, so a dword
-    // that starts inside the row may be read whole
-    if (jj < q.dim_j && cc < q.dim_c) v = *reinterpret_cast<const uint32_t *>(src + jj * q.Sj + cc);
-    *reinterpret_cast<uint32_t *>(&tile[r][tq * 4]) = v;
+  for (int u = 0; u < kPasses; ++u)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int jj = j0 + (threadIdx.x / Q + u * (kThreads / Q)) * 4 + k;
+      r[u][k] = jj < q.dim_j && cc < q.dim_c ? *reinterpret_cast<const uint32_t *>(src + jj * q.Sj + cc) : 0u;
+    }
+#pragma unroll
+  for (int u = 0; u < kPasses; ++u) {
+    uint32_t t[4];
+    transpose_bytes(r[u], t);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tile[(cq * 4 + k) * 17 + threadIdx.x / Q + u * (kThreads / Q)] = t[k];
   }
   __syncthreads();
 #pragma unroll
-  for (int r = tr; r < 64; r += 16) {
-    const int cc = c0 + r, jj = j0 + tq * 4;
-    if (cc < q.dim_c && jj < q.ocs) {
-      const uint32_t v = (uint32_t)(uint8_t)tile[tq * 4][r] | ((uint32_t)(uint8_t)tile[tq * 4 + 1][r] << 8) |
-                         ((uint32_t)(uint8_t)tile[tq * 4 + 2][r] << 16) | ((uint32_t)(uint8_t)tile[tq * 4 + 3][r] << 24);
-      *reinterpret_cast<uint32_t *>(dst + cc * q.Tc + jj) = v;
-    }
+  for (int k = 0; k < Q / 4; ++k) {
+    const int row = threadIdx.x / 16 + k * 16, c = c0 + row, j = j0 + (threadIdx.x & 15) * 4;
+    if (c < q.dim_c && j < q.ocs) *reinterpret_cast<uint32_t *>(dst + c * q.Tc + j) = tile[row * 17 + (threadIdx.x & 15)];
   }
 }
 
@@ -628,9 +661,10 @@ int run_permute(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const void *x, void 
     PermTileArgs q{(const int8_t *)x, (int8_t *)y, S[j], S[a], S[b], T[1], T[a], T[b], FastDiv(dim[b]), dim[j], dim[1], d->y_cs, 0};
     const int64_t batch = (int64_t)dim[a] * dim[b];
     for (int64_t p0 = 0; p0 < batch; p0 += 65535) {   // as many planes as a grid holds
-      const dim3 grid((unsigned)((d->y_cs + 63) / 64), (unsigned)((d->ic + 63) / 64), (unsigned)std::min<int64_t>(batch - p0, 65535));
+      const int tile = d->ic > 64 ? 128 : 64;
+      const dim3 grid((unsigned)((d->y_cs + 63) / 64), (unsigned)((d->ic + tile - 1) / tile), (unsigned)std::min<int64_t>(batch - p0, 65535));
       q.plane0 = (uint32_t)p0;
-      launch(ctx, permute_tile_kernel, grid, dim3(kThreads), q);
+      launch(ctx, tile == 128 ? permute_tile_kernel<32> : permute_tile_kernel<16>, grid, dim3(kThreads), q);
     }
   }
   TPUHIP_CHECK_HIP(hipGetLastError());
