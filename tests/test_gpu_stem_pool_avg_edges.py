@@ -20,9 +20,11 @@ def ctx():
 
 
 # one tile's patch: 11 rows of 2 * (conv columns - 1) + 8 dwords, rounded to 4: 5632 = 11 loads, then 12, then 5 and 1
-@pytest.mark.parametrize("h,w", [(22, 505), (22, 507), (13, 503), (30, 224), (9, 11)])
-def test_stem_with_pool_patch_ends(h, w):
-    b = Builder("stem", BASE_SEED + w, 2, (6, 16))
+# -- and batches whose tiles are of two, three (the last of two rows) and more pooled rows
+@pytest.mark.parametrize("n,h,w", [(2, 22, 505), (2, 22, 507), (2, 13, 503), (2, 30, 224), (2, 9, 11),
+                                   (40, 33, 20), (70, 33, 20), (100, 41, 12), (257, 13, 9)])
+def test_stem_with_pool_tiles(n, h, w):
+    b = Builder("stem", BASE_SEED + w, n, (6, 16))
     x = b.input("input", 3, h, w)
     c = b.conv("conv", x, 64, 7, stride=2, pad=3, relu=True)
     p = b.pool_max("pool", c, 3, 2, (0, 1, 0, 1))
