@@ -5016,28 +5016,38 @@ bool stem_pool_plan(const tpuhip_conv_weights *w, const tpuhip_pool_desc &p, int
   };
   auto fits = [&](int rows) { return fits_crows(2 * rows + 1); };
   if (!fits(1)) return false;
+  // an image's tiles of r pooled rows, evened out, and the conv rows of the last, which holds those that no window reaches as well
+  struct Tiles { int per_image, rows, crows_last; };
+  auto tiles_of = [&](int r) {
+    const int per_image = (p.oh + r - 1) / r, rows = (p.oh + per_image - 1) / per_image, before = (per_image - 1) * rows;
+    return Tiles{per_image, rows, std::max(2 * (p.oh - before) + 1, d.oh - (2 * before - p.pt))};
+  };
+  auto all_fit = [&](const Tiles &t) { return fits_crows(std::max(2 * t.rows + 1, t.crows_last)); };
+  int widest = 1;   // one tile per CU: what is taken at all
+  while (widest < p.oh && fits(widest + 1)) ++widest;
+  while (widest > 1 && (int64_t)d.n * ((p.oh + widest - 1) / widest) < num_cu) --widest;
+  Tiles tiles = tiles_of(widest);
+  if (!all_fit(tiles)) return false;
   // Rounds of a tile per CU, times what a tile takes: of 25 batches and sizes timed with 1 to 8 rows a round is 4.0 + 1.45 a row
-  // us, whether or not two workgroups share a CU, and this names the fastest in all.  The largest tiles that still are one per CU
-  // (a line before) meet a second, nearly empty round: 8 x 224 x 224 10.5 us with 448 tiles of a row, 7.3 with 224 of two; 16
-  // images 16.7 (three rows) and 10.1 (four), 32 the same (seven).
-  int rows = 1;
+  // us, whether or not two workgroups share a CU, and this names the fastest in all.  The widest meet a second, nearly empty
+  // round: 8 x 224 x 224 10.5 us with 448 tiles of a row, 7.4 with 224 of two; 16 images 16.7 (three rows) and 10.2 (four), 32 the
+  // same (seven).
   int64_t best = INT64_MAX;
   for (int r = 1; r <= p.oh && fits(r); ++r) {
-    const int64_t tiles = (int64_t)d.n * ((p.oh + r - 1) / r), cost = (tiles + num_cu - 1) / num_cu * (8 + 3 * r);
-    if (cost >= best) continue;
+    const Tiles t = tiles_of(r);
+    const int64_t cost = ((int64_t)d.n * t.per_image + num_cu - 1) / num_cu * (8 + 3 * t.rows);
+    if (cost >= best || !all_fit(t)) continue;
     best = cost;
-    rows = r;
+    tiles = t;
   }
-  const int per_image = (p.oh + rows - 1) / rows;
-  rows = (p.oh + per_image - 1) / per_image;
+  const int rows = tiles.rows, per_image = tiles.per_image;
   StemPoolArgs s{};
   s.poh = p.oh; s.pow = p.ow; s.ppt = p.pt; s.ppl = p.pl; s.p_cs = p.y_cs;
   s.rows = rows;
   s.tiles_per_image = per_image;
   s.n_tiles = d.n * per_image;
   s.crows = 2 * rows + 1;
-  s.crows_last = std::max(2 * (p.oh - (per_image - 1) * rows) + 1, d.oh - (2 * (per_image - 1) * rows - p.pt));
-  if (!fits_crows(std::max(s.crows, s.crows_last))) return false;
+  s.crows_last = tiles.crows_last;
   s.prows = (std::max(s.crows, s.crows_last) - 1) * d.sh + d.kh;
   s.pw = pw;
   s.magic_pw = (uint32_t)(((1ull << 32) + pw - 1) / (uint64_t)pw);
