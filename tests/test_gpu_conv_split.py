@@ -112,3 +112,39 @@ def test_shifts_of_zero_and_a_relu_in_front(ctx, tile, case, relu_first):
     ctx.conv_weights_destroy(wh)
     xt.free()
     yt.free()
+
+
+@pytest.mark.parametrize("tile", SPLIT_TILES, ids=_name)
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[12]], ids=lambda c: "x".join(map(str, c[:5])))
+@pytest.mark.parametrize("stride", [65520, 65536, 65552])
+def test_an_input_stride_given_behind_the_choice(ctx, tile, case, stride):
+    """strides on both sides of 16 bits, set once the layer is packed: a part of a wide tensor's channels"""
+    n, ic, ih, iw, oc, k, s, pads, dil, relu = case
+    rng, x, w, bias, mult, rsh = _layer(case, ic + stride)
+    d = conv_desc(x.shape, w.shape, stride=s, pads=pads, dil=dil, do_relu=relu, algo=16 + tile)
+    want = O.conv2d_i8(x, w, bias, rsh, mult, O.make_conv_desc(x.shape, w.shape, 1, s, pads, dil, (0, 0), relu, True, None))
+    wh = ctx.conv_prepack(d, w, f2i32(bias), f2i32(mult), f2i32(rsh))
+    ctx.conv_set_input_stride(wh, stride)
+    xt, yt = ctx.from_nchw(x, stride), ctx.tensor(want.shape)
+    ctx.conv(wh, xt, yt)
+    assert np.array_equal(ctx.to_nchw(yt), want) and not ctx.raw(yt)[..., oc:].any()
+    ctx.conv_weights_destroy(wh)
+    xt.free()
+    yt.free()
+
+
+def test_a_timed_layer_takes_any_input_stride(ctx):
+    case = CASES[0]
+    n, ic, ih, iw, oc, k, s, pads, dil, relu = case
+    rng, x, w, bias, mult, rsh = _layer(case, 3)
+    want = O.conv2d_i8(x, w, bias, rsh, mult, O.make_conv_desc(x.shape, w.shape, 1, s, pads, dil, (0, 0), relu, True, None))
+    wh = ctx.conv_prepack(conv_desc(x.shape, w.shape, stride=s, pads=pads, dil=dil, do_relu=relu), w, f2i32(bias), f2i32(mult), f2i32(rsh))
+    yt = ctx.tensor(want.shape)
+    for stride in (64, 1 << 16, 1 << 21):
+        ctx.conv_set_input_stride(wh, stride)
+        xt = ctx.from_nchw(x, stride)
+        ctx.conv(wh, xt, yt)
+        assert np.array_equal(ctx.to_nchw(yt), want), stride
+        xt.free()
+    ctx.conv_weights_destroy(wh)
+    yt.free()

@@ -126,6 +126,8 @@ struct DenseItem {
   int n, c, h, w, cs;
 };
 int lay_out_dense(tpuhip_ctx *ctx, const DenseItem *items, size_t n);
+// entries of a conv's plane of biases, multipliers, ...: they cover every tile's padding
+__host__ __device__ constexpr int param_entries(int oc) { return ((oc + 255) & ~255) + 16; }
 // conv.hip: packs n filters; the list is in memory the device reads
 int pack_filters(tpuhip_ctx *ctx, const FilterPack *list, size_t n, int64_t largest);
 // conv.hip: makes the requantisation parameters of n layers; the list likewise

@@ -4675,7 +4675,7 @@ void split_ready(tpuhip_conv_weights *cw) {
   if (cw->algo != ALGO_MFMA || kTiles[cw->tile].reg != 10 || !cw->nparam) return;
   const SplitVariant &v = kTiles[cw->tile].split;
   cw->split_plan = split_plan(cw->d, v, cw->fast);
-  cw->split_fits = split_args(cw->d, v, cw->split_plan, cw->nparam, &cw->split);
+  cw->split_fits = split_args(cw->d, v, cw->split_plan, &cw->split);
 }
 
 int pack_mfma_weights(tpuhip_ctx *ctx, tpuhip_conv_weights *cw, int tile) {
@@ -5130,7 +5130,7 @@ bool tile_usable(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, int t, con
   if (kTiles[t].reg == 5 && (!w->fast || w->split_oc % kTiles[t].bm)) return false;
   if (kTiles[t].reg == 9 && (!w->qnarrow || w->split_oc)) return false;
   SplitArgs args;
-  if (kTiles[t].reg == 10 && !split_args(w->d, kTiles[t].split, split_plan(w->d, kTiles[t].split, w->fast), w->nparam, &args)) return false;
+  if (kTiles[t].reg == 10 && !split_args(w->d, kTiles[t].split, split_plan(w->d, kTiles[t].split, w->fast), &args)) return false;
   return !((kTiles[t].reg == 6 || kTiles[t].reg == 7) && (!w->fast || w->split_oc));
 }
 
@@ -5461,7 +5461,7 @@ int tpuhip_conv2d_prepack(tpuhip_ctx *ctx, const tpuhip_conv_desc *desc, const i
   // epilogue parameters, indexed by the true output channel.  `fast` holds when,
   // for every channel, 1 <= rshift and |acc + bias| + 1 + 2^(rshift-1) cannot reach
   // 2^31: |acc| <= 128 * sum|w|, and |x| <= |v| + 1 after the doubling high multiply.
-  const size_t nparam = (size_t)round_up(d.oc, 256) + 16;   // covers every tile's padding
+  const size_t nparam = (size_t)param_entries(d.oc);
   std::vector<int32_t> raw(3 * (size_t)d.oc);
   bool fast = true, narrow = !d.relu_first;
   for (int i = 0; i < d.oc; ++i) {
@@ -5664,7 +5664,7 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
                  "channels on a map narrow enough for its row patch, right shifts of at least 1 and sums that cannot "
                  "overflow the rounding", kTiles[w->tile].name);
   TPUHIP_REQUIRE(!(w->algo == ALGO_MFMA && kTiles[w->tile].reg == 10) || w->split_fits,
-                 "conv: tile variant %s takes sides, strides, paddings and channels below 65536 and fewer outputs",
+                 "conv: tile variant %s takes sides, output strides, paddings and channels below 65536 and fewer outputs",
                  kTiles[w->tile].name);
   TPUHIP_REQUIRE((w->split_oc != 0) == (post.y2 != nullptr),
                  "conv: weights packed as a pair run through tpuhip_conv2d_pair_i8 (and only they do)");

@@ -47,7 +47,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   // named here, the arguments leave the scalar cache together instead of one by one where they are first needed
   asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.x_bytes), "s"(a.n_tiles), "s"(a.n_pix), "s"(a.shape), "s"(a.magic_tile),
                "s"(a.magic_img), "s"(a.magic_row), "s"(a.magic_c16), "s"(a.magic_kw), "s"(a.magic_pw), "s"((int)a.per_img), "s"((int)a.ih),
-               "s"((int)a.x_cs), "s"((int)a.sh), "s"((int)a.dh), "s"((int)a.slices_pad_relu), "s"((int)a.nparam16));
+               "s"(a.x_cs), "s"((int)a.sh), "s"((int)a.dh), "s"((int)a.slices_pad_relu), "s"((int)a.oc));
   extern __shared__ v4i lds[];   // the patch, [group][wave of K][block][lane] sums, the table's 256 bytes
   constexpr int T = KW * PW * 64, B = NB * OB, FIN = (B + KW - 1) / KW;   // FIN: blocks that a wave finishes
   const int tid = threadIdx.x, lane = tid & 63;
@@ -123,7 +123,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
     const uint32_t kg = (uint32_t)(4 * s + (UNI ? 0 : chunk));
     const uint32_t tap = div_by(kg, a.magic_c16), cgrp = kg - tap * a.c16, tkh = div_by(tap, a.magic_kw), tkw = tap - tkh * a.kw;
     const int dh_off = in_k ? (int)(tkh * a.dh) : 1 << 28, dw_off = (int)(tkw * a.dw);
-    const int tap_off = ((int)(tkh * a.dh) * a.iw + dw_off) * a.x_cs + (int)cgrp * 16;
+    const int tap_off = ((int)(tkh * a.dh) * a.iw + dw_off) * (int)a.x_cs + (int)cgrp * 16;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       const int ih = ih0[j] + dh_off, iw = iw0[j] + dw_off;
@@ -170,7 +170,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   v4i bias[FIN], mult[FIN], shift[FIN], hpot[FIN];
   uint32_t src[FIN];
   int64_t off[FIN];
-  const int nparam = a.nparam16 * 16;
+  const int nparam = param_entries(a.oc);
 #pragma unroll
   for (int f = 0; f < FIN; ++f) {
     const int b = wk + f * KW, oc = oc0 + (b / NB) * 16 + chunk * 4;   // block b: channels b / NB, pixels b % NB
@@ -469,15 +469,15 @@ int64_t tpuhip::split_tiles(const tpuhip_conv_desc &d, const SplitVariant &v, co
   return pix * ceil_div64(d.oc, 16 * v.ob);
 }
 
-bool tpuhip::split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const SplitPlan &pl, int nparam, SplitArgs *out) {
+bool tpuhip::split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const SplitPlan &pl, SplitArgs *out) {
   SplitArgs a{};
   const int c16 = (d.ic + 15) / 16, slices = (d.kh * d.kw * c16 + 3) / 4;
   const int64_t n_oc = ceil_div64(d.oc, 16 * v.ob), tiles = split_tiles(d, v, pl), n_pix = tiles / n_oc;
   const int64_t npix = (int64_t)d.n * d.oh * d.ow, in_bytes = (int64_t)d.n * d.ih * d.iw * d.x_cs;
-  for (int64_t u16 : {d.ih, d.iw, d.oh, d.ow, d.x_cs, d.y_cs, d.oc, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw, d.kw, 16 * slices + 15, nparam / 16})
+  for (int64_t u16 : {d.ih, d.iw, d.oh, d.ow, d.y_cs, d.oc, d.sh, d.sw, d.pt, d.pl, d.dh, d.dw, d.kw, 16 * slices + 15})
     if (u16 < 0 || u16 > 65535) return false;
   // the divisions by multiplying are exact where number * divisor stays below 2^32
-  if (nparam % 16 || in_bytes >= 1ll << 31 || n_oc * v.ob * slices * 1024 >= 1ll << 31) return false;
+  if (in_bytes >= 1ll << 31 || n_oc * v.ob * slices * 1024 >= 1ll << 31) return false;
   if ((tiles + 8) * std::max(n_pix, n_oc) >= 1ll << 32 || (npix + 256) * std::max(d.oh, d.ow) >= 1ll << 32) return false;
   a.x_bytes = (uint32_t)in_bytes;
   a.n_tiles = (uint32_t)tiles;
@@ -502,10 +502,9 @@ bool tpuhip::split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const 
   a.magic_c16 = magic_of(c16);
   a.magic_kw = magic_of(d.kw);
   a.ih = (uint16_t)d.ih; a.iw = (uint16_t)d.iw; a.oh = (uint16_t)d.oh; a.ow = (uint16_t)d.ow;
-  a.x_cs = (uint16_t)d.x_cs; a.y_cs = (uint16_t)d.y_cs; a.oc = (uint16_t)d.oc; a.c16 = (uint16_t)c16;
+  a.x_cs = (uint32_t)d.x_cs; a.y_cs = (uint16_t)d.y_cs; a.oc = (uint16_t)d.oc; a.c16 = (uint16_t)c16;
   a.sh = (uint16_t)d.sh; a.sw = (uint16_t)d.sw; a.pt = (uint16_t)d.pt; a.pl = (uint16_t)d.pl;
   a.dh = (uint16_t)d.dh; a.dw = (uint16_t)d.dw; a.kw = (uint16_t)d.kw;
-  a.nparam16 = (uint16_t)(nparam / 16);
   a.slices_pad_relu = (uint16_t)(slices * 16 + (4 * slices - d.kh * d.kw * c16) * 4 + (!d.do_relu ? 0 : d.relu_first ? 2 : 1));
   *out = a;
   return true;

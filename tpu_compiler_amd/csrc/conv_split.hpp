@@ -18,11 +18,11 @@ struct SplitArgs {
   uint32_t magic_tile;         // n_pix, or the channel tiles
   uint32_t magic_img, magic_row;   // patch form: pixel tiles of an image, of a row of them; gather form: output rows, columns
   uint32_t magic_c16, magic_kw, magic_pw;   // pw: columns of the patch
+  uint32_t x_cs;               // any that a layer may be given after its variant is chosen: 32 bits
   uint16_t per_img, per_row;   // patch form: what magic_img and magic_row divide by
   uint16_t by_tw;              // patch form: floor((2^16 - 1) / columns of a tile)
-  uint16_t ih, iw, oh, ow, x_cs, y_cs, oc, c16;
+  uint16_t ih, iw, oh, ow, y_cs, oc, c16;
   uint16_t sh, sw, pt, pl, dh, dw, kw;
-  uint16_t nparam16;           // entries of a plane, by 16
   uint16_t slices_pad_relu;    // slices of 64 bytes of K << 4 | groups of 16 bytes past its end << 2 | 1: ReLU behind the
                                // requantisation, 2: in front of it
 };
@@ -51,7 +51,7 @@ struct SplitPlan {
 SplitPlan split_plan(const tpuhip_conv_desc &d, const SplitVariant &v, bool fast);
 int64_t split_tiles(const tpuhip_conv_desc &d, const SplitVariant &v, const SplitPlan &pl);
 // What a launch of the layer takes but its pointers and what is fused behind it; false: a number is beyond the arguments' fields.
-bool split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const SplitPlan &pl, int nparam, SplitArgs *out);
+bool split_args(const tpuhip_conv_desc &d, const SplitVariant &v, const SplitPlan &pl, SplitArgs *out);
 // post: NULL, nothing is fused
 void split_launch(tpuhip_ctx *ctx, const SplitVariant &v, const SplitPlan &pl, bool fast, bool uni, const SplitArgs &a,
                   const SplitPost *post);
