@@ -20,14 +20,15 @@ int set_error(int status, const char *fmt, ...) {
   return status;
 }
 
-bool raise_lds_limit(const void *kernel, unsigned bytes) {
+bool raise_lds_limit(int device, const void *kernel, unsigned bytes) {
   static std::mutex mu;
-  static std::map<const void *, unsigned> raised;
+  static std::map<std::pair<int, const void *>, unsigned> raised;
   std::lock_guard<std::mutex> lock(mu);
-  auto it = raised.find(kernel);
+  auto it = raised.find({device, kernel});
   if (it != raised.end() && it->second >= bytes) return true;
+  if (hipSetDevice(device) != hipSuccess) return false;
   if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
-  raised[kernel] = bytes;
+  raised[{device, kernel}] = bytes;
   return true;
 }
 

@@ -139,9 +139,10 @@ int prepack_done(tpuhip_ctx *ctx);
 // is none, and the call may do without
 int grow_workspace(tpuhip_ctx *ctx, size_t bytes);
 
-// api.hip: raises a kernel's dynamic LDS limit, once per kernel and size (kernels of one signature share their function-pointer
-// type, so the record is keyed by the kernel's address); on failure the runtime's last error stays set for the caller to report
-bool raise_lds_limit(const void *kernel, unsigned bytes);
+// api.hip: raises a kernel's dynamic LDS limit, once per device, kernel and size: the limit is a setting of the device that is
+// current, and the context's becomes it (kernels of one signature share their function-pointer type, so the record is keyed by the
+// kernel's address); on failure the runtime's last error stays set for the caller to report
+bool raise_lds_limit(int device, const void *kernel, unsigned bytes);
 
 int set_error(int status, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 

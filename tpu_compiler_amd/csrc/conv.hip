@@ -4157,7 +4157,7 @@ void launch_reg(tpuhip_ctx *ctx, dim3 grid, const ConvArgs &a) {
 // the patch kernel's LDS patch is dynamic: (rows + 2) x (W + 2) x C bytes of this layer
 template <typename F>
 void launch_patch(tpuhip_ctx *ctx, F kernel, dim3 grid, const ConvArgs &a, bool dynamic, unsigned stage_bytes) {
-  if (dynamic) (void)raise_lds_limit((const void *)kernel, kPatchBytesDyn);
+  if (dynamic) (void)raise_lds_limit(ctx->device, (const void *)kernel, kPatchBytesDyn);
   // the patch, or the staged output tile that takes its place in the epilogue if that is larger
   const unsigned smem = dynamic ? std::max((unsigned)((a.pstep_pix + 2) * a.stem_pw * (a.c16 * 16)), stage_bytes) : 0u;
   if (ctx->prof_start)
@@ -4172,18 +4172,13 @@ constexpr unsigned pw_lds_bytes(int bm, int bn, int kp, int sd) {
   return (unsigned)(bm * kp + 2 * bn * kp + sd * bn * (bm + 16) + 5 * bm * 4 + 256);
 }
 
-template <typename F>
-bool pw_prepare(F kernel, unsigned lds) {
-  return raise_lds_limit((const void *)kernel, lds);
-}
-
 void launch_pw(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
   switch (tile) {
 #define W(i, name, BM, BN, WM, WN, KP, SD, O)                                                           \
   case i: {                                                                                             \
     auto kernel = a.narrow ? conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, true> : conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, false>; \
     constexpr unsigned lds = pw_lds_bytes(BM, BN, KP, SD);                                              \
-    if (!pw_prepare(kernel, lds)) break;                                                                \
+    if (!raise_lds_limit(ctx->device, (const void *)kernel, lds)) break;                                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(WM * WN * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                \
@@ -4196,13 +4191,13 @@ void launch_pw(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
 
 // workgroups of pointwise tile variant `tile` that fit on one CU at once
 template <bool NARROW>
-int pw_occupancy(int tile) {
+int pw_occupancy(int device, int tile) {
   int n = 0;
   hipError_t e = hipErrorInvalidValue;
   switch (tile) {
 #define W(i, name, BM, BN, WM, WN, KP, SD, O)                                                           \
   case i:                                                                                               \
-    if (pw_prepare(conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, NARROW>, pw_lds_bytes(BM, BN, KP, SD)))     \
+    if (raise_lds_limit(device, (const void *)conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, NARROW>, pw_lds_bytes(BM, BN, KP, SD))) \
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, conv_pw_kernel<BM, BN, WM, WN, KP, SD, O, NARROW>, WM * WN * 64, \
                                                        pw_lds_bytes(BM, BN, KP, SD));                   \
     break;
@@ -4242,7 +4237,7 @@ void launch_patch2(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
 #define V(i, name, BM, BN, WM, WN, BK, O)                                                               \
   case i: {                                                                                             \
     auto kernel = a.narrow ? conv_patch2_kernel<BM, BN, WM, WN, BK, O, true> : conv_patch2_kernel<BM, BN, WM, WN, BK, O, false>; \
-    if (!pw_prepare(kernel, (unsigned)kLdsBytes)) break;                                                \
+    if (!raise_lds_limit(ctx->device, (const void *)kernel, (unsigned)kLdsBytes)) break;                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(WM * WN * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                \
@@ -4330,7 +4325,7 @@ void launch_rows(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsign
 #define U4(i, name, WOC, WPX, OB, NB, G, U, O)                                                                \
   case i: {                                                                                             \
     auto kernel = conv_rows_kernel<WOC, WPX, OB, NB, G, U, O>;                                                \
-    if (!pw_prepare(kernel, (unsigned)kLdsBytes)) break;                                                \
+    if (!raise_lds_limit(ctx->device, (const void *)kernel, (unsigned)kLdsBytes)) break;                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(WOC * WPX * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                \
@@ -4346,7 +4341,7 @@ void launch_patch3(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a, unsi
 #define U3(i, name, NB2, PW, OB)                                                                        \
   case i: {                                                                                             \
     auto kernel = a.narrow ? conv_patch3_kernel<NB2, PW, OB, true> : conv_patch3_kernel<NB2, PW, OB, false>; \
-    if (!pw_prepare(kernel, (unsigned)kLdsBytes)) break;                                                \
+    if (!raise_lds_limit(ctx->device, (const void *)kernel, (unsigned)kLdsBytes)) break;                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(256 * PW), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                \
@@ -4387,7 +4382,7 @@ void launch_ksplit(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
     LeanArgs l;                                                                                         \
     if (lean_args(a, &l)) {                                                                             \
       auto lean = conv_mfma_ksplit_lean_kernel<W, TN, FAST, UNI>;                                       \
-      if (!pw_prepare(lean, lds)) break;                                                                \
+      if (!raise_lds_limit(ctx->device, (const void *)lean, lds)) break;                                \
       if (ctx->prof_start)                                                                              \
         hipExtLaunchKernelGGL(lean, grid, dim3(W * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, l); \
       else                                                                                              \
@@ -4395,7 +4390,7 @@ void launch_ksplit(tpuhip_ctx *ctx, int tile, dim3 grid, const ConvArgs &a) {
       break;                                                                                            \
     }                                                                                                   \
     auto kernel = conv_mfma_ksplit_kernel<W, TN, FAST, UNI>;                                            \
-    if (!pw_prepare(kernel, lds)) break;                                                                \
+    if (!raise_lds_limit(ctx->device, (const void *)kernel, lds)) break;                                \
     if (ctx->prof_start)                                                                                \
       hipExtLaunchKernelGGL(kernel, grid, dim3(W * 64), lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                \
@@ -4457,7 +4452,7 @@ int conv_mode(const tpuhip_conv_weights *w) {
   return w->smallc ? kModeSmallC : uni ? kModeUniform : kModeGeneral;
 }
 
-int persist_wgs_per_cu(const tpuhip_conv_weights *w) {
+int persist_wgs_per_cu(int device, const tpuhip_conv_weights *w) {
   // 0 = not asked yet.  Contexts on several host threads may ask at once: every writer
   // stores the same value, so relaxed atomics are all that is needed.
   static std::atomic<int> cache[kMaxTiles][3][3];
@@ -4473,7 +4468,7 @@ int persist_wgs_per_cu(const tpuhip_conv_weights *w) {
                                     : persist_occupancy<F, kModeGeneral>(w->tile);
     };
     if (kTiles[w->tile].reg == 5)
-      c = form == kNarrow ? pw_occupancy<true>(w->tile) : pw_occupancy<false>(w->tile);
+      c = form == kNarrow ? pw_occupancy<true>(device, w->tile) : pw_occupancy<false>(device, w->tile);
     else
       c = form == kNarrow ? ask(std::integral_constant<int, kNarrow>())
           : form == kFast ? ask(std::integral_constant<int, kFast>())
@@ -4907,7 +4902,7 @@ void fill_args(const tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *
       // every XCD owns a run of whole pixel tiles; a workgroup keeps its channel tile
       const int n_pix_tiles = a.n_tiles / a.n_oc_tiles;
       a.tiles_per_xcd = (n_pix_tiles + 7) / 8 * a.n_oc_tiles;
-      const int slots = std::max(1, ctx->num_cu / 8) * persist_wgs_per_cu(w);
+      const int slots = std::max(1, ctx->num_cu / 8) * persist_wgs_per_cu(ctx->device, w);
       a.wgs_per_xcd = std::min(a.tiles_per_xcd, std::max(1, slots / a.n_oc_tiles) * a.n_oc_tiles);
       a.pstep_pix = a.wgs_per_xcd / a.n_oc_tiles * t.bn;
       a.pstep_ow = a.pstep_pix % d.ow;
@@ -5721,7 +5716,8 @@ static int run_conv(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const void *x
     sp.py = (int8_t *)post.pool_out;
     take_narrow(w, &a);
     a.magic_ow = (uint32_t)(((1ull << 32) + a.ow - 1) / (uint64_t)a.ow);
-    TPUHIP_REQUIRE(pw_prepare(conv_stem_pool_kernel, 160u * 1024), "conv: raising the stem + pool kernel's LDS limit failed");
+    TPUHIP_REQUIRE(raise_lds_limit(ctx->device, (const void *)conv_stem_pool_kernel, 160u * 1024),
+                   "conv: raising the stem + pool kernel's LDS limit failed");
     const int per_cu = std::max(1, std::min(4, (int)(160u * 1024 / lds)));
     const dim3 grid((unsigned)std::min<int64_t>(sp.n_tiles, (int64_t)ctx->num_cu * per_cu)), block(512);
     if (ctx->prof_start)

@@ -539,7 +539,7 @@ int tpuhip_conv2d_chain_i8(tpuhip_ctx *ctx, const tpuhip_conv_chain *ch, const v
   case i: {                                                                                                \
     auto kernel = conv_chain_kernel<OC1, KP1, OC2, BN, O, L>;                                              \
     constexpr unsigned lds = chain_lds_bytes<OC1, KP1, OC2, BN, L>();                                      \
-    TPUHIP_REQUIRE(raise_dynamic_lds((const void *)kernel, lds), "conv chain: raising the LDS limit failed"); \
+    TPUHIP_REQUIRE(raise_lds_limit(ctx->device, (const void *)kernel, lds), "conv chain: raising the LDS limit failed"); \
     const int per_cu = std::max(1, std::min((int)(160u * 1024 / lds), O / 2));                             \
     const int slots = ctx->num_cu * per_cu;                                                                \
     /* whole rounds of BN-pixel tiles over the resident workgroups; what is left runs as 32-pixel */       \

@@ -8,8 +8,6 @@
 #include "conv_epilogue.hpp"
 
 #include <cstdlib>
-#include <map>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -93,18 +91,6 @@ inline std::vector<int8_t> mfma_a_fragments(const int8_t *filter, int oc, int nb
         }
       }
   return out;
-}
-
-// raises a kernel's dynamic LDS limit once per kernel and size
-inline bool raise_dynamic_lds(const void *kernel, unsigned bytes) {
-  static std::mutex mu;
-  static std::map<const void *, unsigned> raised;
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = raised.find(kernel);
-  if (it != raised.end() && it->second >= bytes) return true;
-  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
-  raised[kernel] = bytes;
-  return true;
 }
 
 template <typename T>

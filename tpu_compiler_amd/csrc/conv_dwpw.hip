@@ -504,7 +504,7 @@ int dwpw_run(tpuhip_ctx *ctx, const tpuhip_conv_chain *ch, const void *x, void *
 #define TPUHIP_DWPW_LAUNCH(SH, NTV)                                                                       \
   {                                                                                                       \
     auto kernel = conv_dwpw_kernel<SH, NTV>;                                                              \
-    TPUHIP_REQUIRE(raise_dynamic_lds((const void *)kernel, lds), "conv chain: raising the LDS limit failed"); \
+    TPUHIP_REQUIRE(raise_lds_limit(ctx->device, (const void *)kernel, lds), "conv chain: raising the LDS limit failed"); \
     if (ctx->prof_start)                                                                                  \
       hipExtLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                  \

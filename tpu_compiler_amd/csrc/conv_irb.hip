@@ -514,7 +514,7 @@ int irb_run(tpuhip_ctx *ctx, const tpuhip_conv_chain *ch, const void *x, void *y
 #define TPUHIP_IRB_LAUNCH(NWV, NTV)                                                                       \
   if (plan.nw == NWV && plan.nt == NTV) {                                                                 \
     auto kernel = conv_irb_kernel<NWV, NTV>;                                                              \
-    TPUHIP_REQUIRE(raise_dynamic_lds((const void *)kernel, lds), "conv chain: raising the LDS limit failed"); \
+    TPUHIP_REQUIRE(raise_lds_limit(ctx->device, (const void *)kernel, lds), "conv chain: raising the LDS limit failed"); \
     if (ctx->prof_start)                                                                                  \
       hipExtLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a); \
     else                                                                                                  \

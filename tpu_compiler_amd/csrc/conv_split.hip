@@ -403,7 +403,7 @@ template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, int N
 void launch_form(tpuhip_ctx *ctx, unsigned lds, const SplitArgs &a, const SplitPost *post) {
   const dim3 grid((a.n_tiles + 7) / 8 * 8), block(KW * PW * 64);
   auto go = [&](auto kernel, const auto &args) {
-    if (lds > 65536 && !raise_lds_limit((const void *)kernel, kLdsBytes)) return;
+    if (lds > 65536 && !raise_lds_limit(ctx->device, (const void *)kernel, kLdsBytes)) return;
     if (ctx->prof_start)
       hipExtLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, args);
     else
