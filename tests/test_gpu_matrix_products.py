@@ -19,9 +19,11 @@ def ctx():
 
 
 # rows, K, columns: blocks of 16 x 16, 16 channels x 32 rows, 32 x 32 and 32 x 64, rows and channels over, pad channels in a block
-# of their own, fewer and more slices than the waves hold at once
+# of their own, fewer and more slices than the waves hold at once; K on both sides of what four waves hold; few channels of many rows
 @pytest.mark.parametrize("m,k,n,relu", [(16, 64, 24, False), (17, 130, 1000, True), (100, 2100, 1000, False), (129, 70, 2070, True),
-                                        (250, 192, 4090, False), (256, 2050, 90, True), (1, 5000, 40, False), (300, 4200, 17, True)])
+                                        (250, 192, 4090, False), (256, 2050, 90, True), (1, 5000, 40, False), (300, 4200, 17, True),
+                                        (5, 1024, 33, True), (16, 1025, 24, False), (100, 1024, 1000, False), (32, 960, 4090, True),
+                                        (250, 1024, 4090, True), (129, 1030, 2070, False), (1111, 4150, 10, True), (261, 4200, 300, False)])
 def test_fully_connected_blocks(ctx, m, k, n, relu):
     ops.test_fully_connected(ctx, m, k, n, relu)
 

@@ -306,14 +306,14 @@ __global__ __launch_bounds__(KW * PW * 64) void conv_split_post_kernel(SplitPost
 
 // FullyConnected of few rows (a classifier) the same way, from the filter in fragments of 32 channels that fc_prepack() makes: 16
 // rows of a fragment are 256 contiguous bytes of it, channels 0-7 and 16-23 of the block of 32, or the others.  A workgroup of
-// eight waves per 16 * OB channels x 16 * NB rows; K split over the waves, four slices of 64 bytes in flight each.
+// four or eight waves per 16 * OB channels x 16 * NB rows; K split over the waves, four slices of 64 bytes in flight each.
 // Bound: launch, one trip to memory, one meeting in LDS; from 64 rows on the operands' way into a CU (98 KB each at 100 x 2048 x
 // 1000).  Replayed from a graph, against sixteen waves per block of 32 x 32, two barriers and one wave that finished 16 channels a
 // lane: 1 x 2048 x 1000 3.63 -> 2.35 us, 32 rows 4.92 -> 3.18, 100 rows 5.11 -> 4.25, 16 x 8192 x 4096 10.2 -> 6.9, 256 x 1024 x
-// 4096 8.14 -> 8.25.
-template <int NB, int OB, bool FAST>
-__global__ __launch_bounds__(512) void fc_split_kernel(FcArgs a) {
-  constexpr int KW = 8, B = NB * OB, D = kDepth;
+// 4096 8.11 -> 7.1.
+template <int KW, int NB, int OB, bool FAST>
+__global__ __launch_bounds__(KW * 64) void fc_split_kernel(FcArgs a) {
+  constexpr int B = NB * OB, D = kDepth;
   static_assert(B <= KW, "a wave finishes one block");
   __shared__ v4i sums[KW * B * 64];
   asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.x_bytes), "s"(a.w_bytes), "s"(a.rows), "s"(a.oc), "s"(a.x_cs), "s"(a.slices),
@@ -518,14 +518,18 @@ void tpuhip::split_launch(tpuhip_ctx *ctx, const SplitVariant &v, const SplitPla
 #undef TPUHIP_FORM
 }
 
-// The blocks of a workgroup: those with which the busiest CU fetches the least, a workgroup fetching as many rows of operands as
-// it has channels and rows.  Of nine shapes timed with all four it names the fastest in seven (100 x 2048 x 1000: 4.33, 4.21, 4.36,
-// 6.29 us in the order below; 32 rows: 3.15, 4.05, 4.26, 4.93), 4 % from it in the others.
+// The blocks of a workgroup: those with which the busiest CU fetches the least, a workgroup fetching as many rows of operands as it
+// has channels and rows.  Of nine shapes timed with all four it names the fastest in seven (100 x 2048 x 1000: 4.33, 4.21, 4.36,
+// 6.29 us in the order below; 32 rows: 3.15, 4.05, 4.26, 4.93), 4 % from it in the others.  Beyond 256 rows, which only a K of more
+// than 4096 brings, blocks of 32 channels alone: their rows are HBM's (4000 x 5000 x 16: 7.9 us with two workgroups of eight channels
+// for every block of rows, 6.6).
+// Waves: four where they hold all of K at once, up to four slices each; 4 x 2 blocks, which are more than four waves finish, become
+// 2 x 2.  Eight: 256 x 64 x 4096 4.1 us, four 3.0; 256 x 1024 x 4096 7.9 and 7.1, 100 x 512 x 4096 3.6 and 3.5.
 void tpuhip::fc_split(tpuhip_ctx *ctx, const FcArgs &a, bool fast) {
   const int kinds[][2] = {{1, 1}, {2, 1}, {2, 2}, {4, 2}};
   int best = 0;
   int64_t least = INT64_MAX;
-  for (int k = 0; k < 4; ++k) {
+  for (int k = a.rows > 256 ? 2 : 0; k < 4; ++k) {
     const int nb = kinds[k][0], ob = kinds[k][1];
     const int64_t tiles = ceil_div64(a.oc, 16 * ob) * ceil_div64(a.rows, 16 * nb);
     const int64_t cost = ceil_div64(tiles, ctx->num_cu) * (std::min(a.rows, 16 * nb) + 16 * ob);
@@ -534,19 +538,29 @@ void tpuhip::fc_split(tpuhip_ctx *ctx, const FcArgs &a, bool fast) {
       best = k;
     }
   }
+  const bool four = a.slices <= 4 * kDepth;
+  if (four) best = std::min(best, 2);
   const int nb = kinds[best][0], ob = kinds[best][1];
-  // channel tiles in whole rounds of the XCDs: those of one tile of channels meet its filter in one L2
-  const dim3 grid((unsigned)ceil_div64(ob == 2 ? ceil_div64(a.oc, 32) : 2 * ceil_div64(a.oc, 32), 8) * 8, (unsigned)ceil_div64(a.rows, 16 * nb));
+  // Channel tiles in whole rounds of the XCDs, where that is an eighth more at most: those of one tile of channels meet its filter in
+  // one L2 (2048 x 9216 x 4096: 316 us, 350 with an equal share of all tiles for each XCD).  Few tiles of channels would leave all
+  // rows to as few XCDs (4000 x 5000 x 16 on one of the eight: 24 us).
+  const int64_t across = (ob == 2 ? 1 : 2) * ceil_div64(a.oc, 32), rounds = ceil_div64(across, 8) * 8;
+  const dim3 grid((unsigned)(rounds * 8 <= across * 9 ? rounds : across), (unsigned)ceil_div64(a.rows, 16 * nb)), block(four ? 256 : 512);
   auto go = [&](auto kernel) {
     if (ctx->prof_start || ctx->prof_stop)
-      hipExtLaunchKernelGGL(kernel, grid, dim3(512), 0, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
+      hipExtLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, ctx->prof_start, ctx->prof_stop, 0, a);
     else
-      hipLaunchKernelGGL(kernel, grid, dim3(512), 0, ctx->stream, a);
+      hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, a);
   };
-  switch (best) {
-    case 0: return fast ? go(fc_split_kernel<1, 1, true>) : go(fc_split_kernel<1, 1, false>);
-    case 1: return fast ? go(fc_split_kernel<2, 1, true>) : go(fc_split_kernel<2, 1, false>);
-    case 2: return fast ? go(fc_split_kernel<2, 2, true>) : go(fc_split_kernel<2, 2, false>);
-    default: return fast ? go(fc_split_kernel<4, 2, true>) : go(fc_split_kernel<4, 2, false>);
+#define TPUHIP_FC(KW, NB, OB) return fast ? go(fc_split_kernel<KW, NB, OB, true>) : go(fc_split_kernel<KW, NB, OB, false>)
+  switch (four ? best + 4 : best) {
+    case 0: TPUHIP_FC(8, 1, 1);
+    case 1: TPUHIP_FC(8, 2, 1);
+    case 2: TPUHIP_FC(8, 2, 2);
+    case 3: TPUHIP_FC(8, 4, 2);
+    case 4: TPUHIP_FC(4, 1, 1);
+    case 5: TPUHIP_FC(4, 2, 1);
+    default: TPUHIP_FC(4, 2, 2);
   }
+#undef TPUHIP_FC
 }
