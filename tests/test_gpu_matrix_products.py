@@ -44,9 +44,12 @@ def test_fully_connected_of_a_shift_of_zero(ctx, shift):
 
 
 # batch_high, batch_low, rows, K, columns, transposes: one to five blocks of columns in one and two workgroups, K steps around
-# those in flight and around a pass through LDS, rows left over; enough products for two blocks a wave (the last)
+# those in flight and around a pass through LDS, rows left over; enough products for two blocks a wave, which differs with the views
+# and with one or several pairs (300 and 600 workgroups of one block)
 @pytest.mark.parametrize("bh,bl,m,k,n,lt,ot", [(2, 3, 40, 128, 97, 1, 1), (1, 3, 33, 129, 129, 0, 0), (2, 2, 31, 33, 160, 1, 0),
-                                               (2, 2, 64, 545, 20, 0, 1), (8, 40, 70, 40, 150, 1, 1)])
+                                               (2, 2, 64, 545, 20, 0, 1), (8, 40, 70, 40, 150, 1, 1),
+                                               (1, 3, 33, 20, 70, 0, 0), (2, 2, 40, 96, 100, 1, 1), (4, 25, 90, 70, 161, 0, 1),
+                                               (4, 25, 90, 70, 161, 1, 0)])
 @pytest.mark.parametrize("form", ["one pair", "pairs", "shift of zero"])
 def test_batched_products(ctx, bh, bl, m, k, n, lt, ot, form):
     rng = np.random.default_rng(m + k + n)

@@ -96,14 +96,17 @@ __global__ __launch_bounds__(256) void fc_batched_kernel(FcbArgs a) {
 // with four consecutive m per lane and register, is stored 16 bytes at a time (YM).  Any other view (m between, as in a
 // [batch_high, batch_low, m, k] tensor) is read and written byte by byte at the places that its index gives.
 //
-// Four steps of the filter, the bias and the pair (multiplier, shift) are requested before the rows are waited for; a block of 16
+// Two steps of the filter, the bias and the pair (multiplier, shift) are requested before the rows are waited for; a block of 16
 // outputs a lane is requantised with that pair in scalars where one serves all of it.
 // Bound: launch and one trip to memory.  Replayed from a graph, before (a trip each for the rows, the second step and the
-// parameters; one WG of five blocks; pairs looked up per output) and now: 32 products of 160 x 64 x 160 5.33 -> 3.75 us, 12 of 384 x
-// 64 x 384 6.41 -> 4.21, 96 of 128 x 128 x 128 5.43 -> 4.31, 96 of 384 x 128 x 384 25.8 -> 16.0.
+// parameters; one WG of five blocks; pairs looked up per output) and now: 32 products of 160 x 64 x 160 5.33 -> 3.56 us, 12 of 384 x
+// 64 x 384 6.41 -> 4.18, 96 of 128 x 128 x 128 5.43 -> 4.22, 96 of 384 x 128 x 384 25.8 -> 16.3.
 // ---------------------------------------------------------------------------
 constexpr int kChunkSteps = 16;                  // K steps of 32 per pass through LDS
-constexpr int kAhead = 4;                        // filter fragments in flight, before the rows are waited for
+// Filter fragments in flight, before the rows are waited for.  Of one, two and four, two are within 3 % of the fastest in all of 22
+// shapes: 32 products of 160 x 64 x 160 3.79, 3.75, 3.93 us, 96 of 384 x 128 x 384 18.1, 16.3, 15.9, 32 of 512 x 512 x 512 with rows
+// and results byte by byte 59.7, 59.1, 64.6.
+constexpr int kAhead = 2;
 constexpr int kRowBytes = kChunkSteps * 32 + 16;  // 16 bytes apart from the next bank cycle: 16-byte reads by row do not collide
 
 struct View {
@@ -126,9 +129,11 @@ struct FcbMfmaArgs {
   FastDiv by_mtiles, by_nblocks, by_low, by_mn;
 };
 
-// SIMPLE: one multiplier and shift for all that a workgroup writes, and sums that cannot overflow the rounding
+// SIMPLE: one multiplier and shift for all that a workgroup writes, and sums that cannot overflow the rounding.  The other form
+// looks pairs up per output and is held to the registers that leave three waves on a SIMD (96 products of 200 x 33 x 70, a pair
+// each: two 10.4 us, three 7.4, four, which spill, 8.9).
 template <bool XM, bool YM, bool SIMPLE>
-__global__ __launch_bounds__(256) void fc_batched_mfma_kernel(FcbMfmaArgs a) {
+__global__ __launch_bounds__(256, SIMPLE ? 1 : 3) void fc_batched_mfma_kernel(FcbMfmaArgs a) {
   __shared__ __attribute__((aligned(16))) int8_t rows[32 * kRowBytes];
   __shared__ uint32_t base[32], stride[32];
   asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.mult), "s"(a.rshift), "s"(a.y), "s"(a.xv.cs), "s"(a.yv.cs), "s"(a.m), "s"(a.k),
@@ -397,13 +402,6 @@ int tpuhip_fc_batched_i8(tpuhip_ctx *ctx, const tpuhip_fc_batched_weights *w, co
     a.tiles = (d.n + 31) / 32;
     a.relu = d.do_relu; a.uniform = w->uniform;
     a.in_t = d.input_transpose; a.out_t = d.output_transpose;
-    // a wave takes two blocks of columns only where there are workgroups enough without that: 32 products of 160 x 64 x 160 are 160
-    // of them so, one wave in four with two blocks, and 320 of three and two blocks without
-    const int mtiles = (d.m + 31) / 32;
-    const bool wide = batch * mtiles * ((a.tiles + 3) / 4) > 4 * (int64_t)ctx->num_cu;
-    const int nblocks = wide ? (a.tiles + 7) / 8 : (a.tiles + 3) / 4;
-    a.per_wg = (a.tiles + nblocks - 1) / nblocks;
-    a.by_mtiles = FastDiv(mtiles); a.by_nblocks = FastDiv(nblocks); a.by_low = FastDiv(d.batch_low);
     a.by_mn = FastDiv((int64_t)d.m * d.n);
     // m contiguous: the view's channels are the rows and the rest is one product's (or one batch_high's) columns
     const bool xm = d.x_c == d.m && (int64_t)d.x_h * d.x_w == (d.input_transpose ? (int64_t)d.batch_low * d.k : d.k) && d.x_cs % 4 == 0 &&
@@ -411,6 +409,16 @@ int tpuhip_fc_batched_i8(tpuhip_ctx *ctx, const tpuhip_fc_batched_weights *w, co
     const bool ym = d.y_c == d.m && (int64_t)d.y_h * d.y_w == (d.output_transpose ? (int64_t)d.batch_low * d.n : d.n) && d.y_cs % 16 == 0 &&
                     (uintptr_t)y % 16 == 0;
     const bool simple = w->fast && (w->uniform || !d.output_transpose);
+    // A wave takes two blocks of columns only where there are workgroups enough without that: 32 products of 160 x 64 x 160 are 160
+    // of them so, one wave in four with two blocks, and 320 of three and two blocks without (3.83 and 3.75 us).  Enough are those
+    // that a CU holds, two to four: with one block a wave and two, 96 of 160 x 64 x 160, 960 workgroups, 4.85 and 4.83 us where rows
+    // come in dwords, 10.2 and 9.4 with pairs looked up, 23.6 and 20.2 byte by byte, where every workgroup gathers the rows anew;
+    // 48 of 256 x 128 x 256 (768) 5.68 and 5.83, 8.7 and 10.8, 21.1 and 19.6.
+    const int mtiles = (d.m + 31) / 32;
+    const bool wide = batch * mtiles * ((a.tiles + 3) / 4) > (!xm ? 2 : simple ? 4 : 3) * (int64_t)ctx->num_cu;
+    const int nblocks = wide ? (a.tiles + 7) / 8 : (a.tiles + 3) / 4;
+    a.per_wg = (a.tiles + nblocks - 1) / nblocks;
+    a.by_mtiles = FastDiv(mtiles); a.by_nblocks = FastDiv(nblocks); a.by_low = FastDiv(d.batch_low);
     auto *kernel = xm   ? ym ? simple ? fc_batched_mfma_kernel<true, true, true> : fc_batched_mfma_kernel<true, true, false>
                              : simple ? fc_batched_mfma_kernel<true, false, true> : fc_batched_mfma_kernel<true, false, false>
                    : ym ? simple ? fc_batched_mfma_kernel<false, true, true> : fc_batched_mfma_kernel<false, true, false>
