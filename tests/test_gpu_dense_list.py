@@ -33,3 +33,20 @@ def test_every_tensor_of_a_graph(shapes, i8):
         for i, x in enumerate(xs):
             assert np.array_equal(every["x%d" % i], x) and np.array_equal(every["y%d" % i], np.maximum(x, 0)), i
     m.close()
+
+
+# one tensor of a list of one, as floats of more than one thread's turn (192 KB): straight into the staging buffer, by way of the device
+@pytest.mark.parametrize("shape", [(1, 65, 31, 33), (2, 130, 61, 67)])
+def test_one_tensor_alone(shape):
+    g = graphs.Graph("alone", 1)
+    g.add(graphs.Op("tpu.input", "x", [], shape))
+    g.add(graphs.Op("tpu.relu", "y", ["x"], shape))
+    g.outputs = ["y"]
+    m = module()
+    m.load(g)
+    for k in range(2):
+        x = np.random.default_rng(k).integers(-128, 128, shape).astype(np.int8)
+        m.set_tensor_i8("x", x)
+        m.invoke()
+        assert np.array_equal(m.get_tensor("y"), np.maximum(x, 0)) and np.array_equal(m.get_tensor("x"), x)
+    m.close()
