@@ -37,3 +37,14 @@ def test_channel_shuffle(ctx, c, groups):
 @pytest.mark.parametrize("order", [[0, 2, 3, 1], [0, 3, 1, 2], [1, 0, 2, 3]])
 def test_permute(ctx, c, order):
     _check(ctx, "permute", (3, c, 66, 61), order)
+
+
+# dimensions that end within tiles of j and of channels, in the runs of tiles that an XCD takes and in a grid; few of j (up to 16 and
+# 32 after padding) with planes enough for wide tiles, and just not; channels in whole rounds of the XCDs
+@pytest.mark.parametrize("shape,order", [((1, 66, 40, 37), [1, 0, 2, 3]), ((2, 200, 23, 31), [1, 0, 2, 3]), ((17, 130, 22, 21), [1, 0, 2, 3]),
+                                         ((33, 130, 22, 21), [1, 0, 2, 3]), ((1, 1000, 9, 13), [1, 0, 2, 3]), ((3, 1030, 7, 15), [1, 0, 2, 3]),
+                                         ((1, 66, 31, 16), [1, 0, 2, 3]), ((5, 192, 3, 70), [0, 2, 3, 1]), ((2, 129, 67, 5), [0, 3, 2, 1]),
+                                         ((1, 65, 9, 200), [0, 3, 1, 2]), ((2, 64, 5, 130), [0, 3, 1, 2]), ((60000, 65, 1, 1), [1, 0, 2, 3]),
+                                         ((1, 3, 300, 280), [1, 0, 2, 3])])
+def test_permute_tiles(ctx, shape, order):
+    _check(ctx, "permute", shape, order)

@@ -566,20 +566,41 @@ struct PermTileArgs {
   int dim_j, dim_c;
   int ocs;           // channel stride of the output
   uint32_t plane0;   // first of this launch's (a, b) pairs
+  // RUNS: all tiles; narrow: FastDivs by the tiles of the channels and of j, wide: by the planes of this launch, which mul_j is
+  uint32_t n_tiles, mul_c, shift_c, mul_j, shift_j;
 };
 static_assert(sizeof(PermRowsArgs) <= 112 && sizeof(PermTileArgs) <= 112, "see MovePlan");
 
 // The channels change places with dimension j: tiles of 64 (Q 16) or 128 channels (32) x 64 of j, 4 x 4 bytes of a lane transposed
 // in registers, dwords through LDS, so that the input is read in runs of 64 or 128 bytes and the output written in runs of 64 (its
-// pad channels as zero: rows past the end of dimension j are zeros).  More than 64 channels take the wider tile: with the other
-// the second half of a line is fetched again by another XCD.  NCHW -> NHWC order, replayed from a graph, with bytes read from
-// LDS before / 64 channels / now: 4 x 96 x 78 x 66 3.43 / 3.04 / 3.07 us, 16 x 320 x 100 x 90 30.6 / 30.3 / 27.9.  Bound by the reads
-// of 128 bytes, a row of the map apart each (97 MB are 15 us as a copy).
-template <int Q>
+// pad channels as zero: rows past the end of dimension j are zeros).
+// RUNS: an XCD takes tiles that follow each other, since the parts of a line that lie in several tiles are fetched, and written,
+// once for every L2 they meet in.  Narrow tiles: the channels of the same rows, then the next of j, then the next plane.  Wide ones,
+// where j is one tile: the planes, then the next channels; the output's 16 to 32 bytes of a plane lie beside the next plane's.
+// Else the grid is (j, channels, planes).
+// Bound: by memory at size, where it reaches what a copy does (6.5 TB/s), by launch and one trip below.  To NHWC order, replayed from
+// a graph, with bytes read from LDS and tiles of 64 in a grid / tiles of 128 in a grid / now: 4 x 80 x 96 x 96 4.31 / 3.42 / 3.46 us,
+// 64 x 192 x 90 x 90 (205 MB) 56.8 / 68.2 / 29.7, 32 x 256 x 110 x 110 59.2 / 45.4 / 29.4, 1 x 256 x 62 x 62 2.87 / 2.77 / 2.45.
+template <int Q, bool RUNS>
 __global__ __launch_bounds__(kThreads) void permute_tile_kernel(PermTileArgs q) {
   __shared__ uint32_t tile[Q * 4 * 17];   // [channel][four of j]
-  const int c0 = blockIdx.y * (Q * 4), j0 = blockIdx.x * 64;
+  int c0 = blockIdx.y * (Q * 4), j0 = blockIdx.x * 64;
   uint32_t ib = q.plane0 + blockIdx.z;   // below 2^31, as all pixels are
+  if constexpr (RUNS) {
+    const uint32_t wt = (blockIdx.x & 7) * ((q.n_tiles + 7) >> 3) + (blockIdx.x >> 3);
+    if (wt >= q.n_tiles) return;   // uniform over the workgroup
+    if constexpr (Q == 16) {
+      const uint32_t at_j = (__umulhi(wt, q.mul_c) + wt) >> q.shift_c, plane = (__umulhi(at_j, q.mul_j) + at_j) >> q.shift_j;
+      c0 = (int)(wt - at_j * (uint32_t)((q.dim_c + 63) / 64)) * 64;
+      j0 = (int)(at_j - plane * (uint32_t)((q.ocs + 63) / 64)) * 64;
+      ib = q.plane0 + plane;
+    } else {
+      const uint32_t ct = (__umulhi(wt, q.mul_c) + wt) >> q.shift_c;
+      c0 = (int)ct * 128;
+      j0 = 0;
+      ib = q.plane0 + wt - ct * q.mul_j;
+    }
+  }
   const int64_t ia = q.by_b.split(ib);
   const int8_t *src = q.x + ia * q.Sa + ib * q.Sb;
   int8_t *dst = q.y + ia * q.Ta + ib * q.Tb;
@@ -659,12 +680,28 @@ int run_permute(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const void *x, void 
       if (k != 1 && k != j) rest[nr++] = k;
     const int a = rest[0], b = rest[1];
     PermTileArgs q{(const int8_t *)x, (int8_t *)y, S[j], S[a], S[b], T[1], T[a], T[b], FastDiv(dim[b]), dim[j], dim[1], d->y_cs, 0};
-    const int64_t batch = (int64_t)dim[a] * dim[b];
-    for (int64_t p0 = 0; p0 < batch; p0 += 65535) {   // as many planes as a grid holds
-      const int tile = d->ic > 64 ? 128 : 64;
-      const dim3 grid((unsigned)((d->y_cs + 63) / 64), (unsigned)((d->ic + tile - 1) / tile), (unsigned)std::min<int64_t>(batch - p0, 65535));
+    const int64_t planes = (int64_t)dim[a] * dim[b];
+    const int tiles_j = (d->y_cs + 63) / 64;
+    // Wide tiles where j is so short that a narrow one is half empty at least, and there are four a CU: from a graph, narrow and
+    // wide, order (1, 0, 2, 3), 1 x 80 x 111 x 111 17.6 and 12.9 us, 1 x 256 x 108 x 108 34.2 and 24, 1 x 100 x 14 x 14 2.43 and 2.70;
+    // 64 x 128 x 110 x 110 30.7 and 32.5.
+    const bool wide = d->ic > 64 && d->y_cs <= 32 && planes * ((d->ic + 63) / 64) >= 4 * (int64_t)ctx->num_cu;
+    const int tiles_c = (d->ic + (wide ? 127 : 63)) / (wide ? 128 : 64);
+    // In a grid as it is: a single tile of channels, whose lines end with it, for fewer instructions (512 x 16 x 110 x 110, order
+    // (0, 3, 1, 2): 61 us, 73 in runs); wide tiles that come in whole rounds of the XCDs, which share the channels so by themselves
+    // (8 x 1024 x 110 x 110, order (1, 0, 2, 3): 97 and 130).
+    const bool runs = wide ? tiles_c % 8 != 0 : d->ic > 64;
+    const int64_t most = runs ? std::max<int64_t>(1, (1ll << 30) / ((int64_t)tiles_j * tiles_c)) : 65535;   // planes of a launch
+    for (int64_t p0 = 0; p0 < planes; p0 += most) {
+      const uint32_t now = (uint32_t)std::min(most, planes - p0);
       q.plane0 = (uint32_t)p0;
-      launch(ctx, tile == 128 ? permute_tile_kernel<32> : permute_tile_kernel<16>, grid, dim3(kThreads), q);
+      q.n_tiles = now * tiles_j * tiles_c;
+      const FastDiv by_c(wide ? now : tiles_c), by_j(tiles_j);
+      q.mul_c = by_c.mul; q.shift_c = by_c.shift;
+      q.mul_j = wide ? now : by_j.mul; q.shift_j = by_j.shift;
+      const dim3 grid = runs ? dim3((q.n_tiles + 7) / 8 * 8) : dim3((unsigned)tiles_j, (unsigned)tiles_c, now);
+      launch(ctx, wide ? runs ? permute_tile_kernel<32, true> : permute_tile_kernel<32, false>
+                       : runs ? permute_tile_kernel<16, true> : permute_tile_kernel<16, false>, grid, dim3(kThreads), q);
     }
   }
   TPUHIP_CHECK_HIP(hipGetLastError());
