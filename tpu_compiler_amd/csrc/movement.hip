@@ -18,7 +18,7 @@ constexpr int kThreads = 256;
 // the index maps; the three that move single channels are at the end
 enum Form {
   kPadConst, kPadCut, kPadEdge, kCrop, kReorg, kTile, kTileChannel, kReverse, kDilate, kReflectionPad, kDepthDcr,
-  kReverseChannel, kShuffle, kSwap, kStrided
+  kReverseChannel, kShuffle, kWeave, kSwap, kStrided
 };
 
 // What a kernel reads of it is in the MoveArgs of its form: up to 112 bytes of arguments a launch costs the host 3.1 us
@@ -111,6 +111,7 @@ template <> struct TailOf<kReverse> { using type = MoveTailReverse; };
 template <> struct TailOf<kDilate> { using type = MoveTailDilate; };
 template <> struct TailOf<kDepthDcr> { using type = MoveTail<1, true>; };
 template <> struct TailOf<kShuffle> { using type = MoveTail<2, true>; };
+template <> struct TailOf<kWeave> { using type = MoveTail<2, true>; };               // kShuffle of two or four groups
 template <> struct TailOf<kSwap> { using type = MoveTail<8>; };
 template <> struct TailOf<kStrided> { using type = MoveTail<9, true>; };
 
@@ -237,7 +238,7 @@ __device__ __forceinline__ v4i group_of_bytes(const MoveArgs<F> &a, int n, int h
   }
   const int8_t *row;
   int64_t at, step = 1;       // kStrided: bytes from one channel's source to the next one's
-  uint32_t g = 0, col = 0;    // kShuffle: group (by_a) and column (p[1] of them) of the channel
+  uint32_t g = 0, col = 0;    // kShuffle, kWeave: group (by_a) and column (p[1] of them) of the channel
   if constexpr (F == kStrided) {
     if (a.p[8]) {             // depth to space, CRD; by_a = the factor p[0]
       uint32_t dw = (uint32_t)w, dh = (uint32_t)h;
@@ -252,19 +253,22 @@ __device__ __forceinline__ v4i group_of_bytes(const MoveArgs<F> &a, int n, int h
     }
   } else {
     row = a.x + ((int64_t)(n * a.ih + h) * a.iw + w) * a.ics;
-    if constexpr (F == kShuffle) {
+    if constexpr (F == kShuffle || F == kWeave) {
       g = (uint32_t)c0;
       col = a.by_a.split(g);
-      // Two and four groups, 16 channels that exist: runs of 8 or 4 bytes of each group, at any alignment, woven in registers.
-      // Replayed from a graph, byte by byte and now: four groups of 4 x 96 x 78 x 66 3.72 -> 2.33 us, 16 x 320 x 100 x 90 43 -> 15.
-      if (a.by_a.d == 4 && live == 16) {
+    }
+    // 16 channels that exist: runs of 8 or 4 bytes of each group, at any alignment, woven in registers.  Replayed from a graph, byte
+    // by byte and now: four groups of 4 x 96 x 78 x 66 3.72 -> 2.33 us, 16 x 320 x 100 x 90 43 -> 15.  A form of its own: asking for it
+    // cost the other numbers of groups 2 to 3 % (three of 1 x 24 x 7 x 7: 2.65 and 2.74; eight of 16 x 320 x 100 x 90: 31.1 and 31.7).
+    if constexpr (F == kWeave) {
+      if (live == 16 && a.by_a.d == 4) {
         uint32_t r[4], t[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) __builtin_memcpy(&r[k], row + (int64_t)k * a.p[1] + col, 4);
         transpose_bytes(r, t);
         return v4i{(int)t[0], (int)t[1], (int)t[2], (int)t[3]};
       }
-      if (a.by_a.d == 2 && live == 16) {
+      if (live == 16) {
         uint32_t r[2][2];
         __builtin_memcpy(r[0], row + col, 8);
         __builtin_memcpy(r[1], row + a.p[1] + col, 8);
@@ -283,7 +287,7 @@ __device__ __forceinline__ v4i group_of_bytes(const MoveArgs<F> &a, int n, int h
 #pragma unroll
       for (int k = 0; k < 8; ++k)
         if (b == k) at = a.p[k];
-    } else if constexpr (F == kShuffle) {
+    } else if constexpr (F == kShuffle || F == kWeave) {
       at = (int64_t)g * a.p[1] + col;
       if (++g == a.by_a.d) g = 0, ++col;
     }
@@ -804,7 +808,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
       for (int k = 0; k < 4; ++k) TPUHIP_REQUIRE(os[k] == is[k], "shuffle_channel: shapes differ");
       a.p[1] = is[1] / p[0];
       a.by_a = FastDiv(p[0]);
-      form = kShuffle;
+      form = p[0] == 2 || p[0] == 4 ? kWeave : kShuffle;
       break;
     case TPUHIP_MOVE_SWAP_CHANNEL:
       TPUHIP_REQUIRE(is[1] <= 8, "swap_channel: at most 8 channels (%d)", is[1]);
@@ -886,6 +890,7 @@ extern "C" int tpuhip_move_i8(tpuhip_ctx *ctx, const tpuhip_move_desc *d, const 
       TPUHIP_MOVE_FORM(kDepthDcr);
       TPUHIP_MOVE_FORM(kReverseChannel);
       TPUHIP_MOVE_FORM(kShuffle);
+      TPUHIP_MOVE_FORM(kWeave);
       TPUHIP_MOVE_FORM(kSwap);
       TPUHIP_MOVE_FORM(kStrided);
 #undef TPUHIP_MOVE_FORM
