@@ -4077,9 +4077,9 @@ struct TileCfg {
 // K split over the waves of a workgroup, blocks of 16 x 16 (conv_split.hip):
 // SP(index, name, waves along K, along the pixels, blocks of 16 pixels and of 16 channels per wave).  Of 114 layers (the networks of
 // one image, and layers drawn of 1 to 8 images of 5 to 107 pixels a side, 16 to 1024 channels, 1x1 to 5x5, stride 1 and 2, dilation)
-// one of them is the fastest of all in 91, by 1 % to 2.8 times (profiles/conv_split_tiles.txt): 16x16_w4 in 32 (by up to 12 % over
-// the next of them), 32x32 in 16 (52 %), 16x32 in 15 (16 %), 32x64 in 13 (32 %), 16x16 in 12 (17 %), 32x128 in 2 (5 %), 16x64 in one
-// (25 %).
+// one of them is the fastest of all in 97, by up to 2.8 times (profiles/conv_split_tiles.txt): 16x16_w4 in 26 (by up to 10 % over
+// the next variant), 16x32 in 20 (12 %), 32x32 in 19 (47 %), 32x64 in 15 (9 %), 16x16 in 12 (22 %), 32x128 in 4 (19 %), 16x64 in one
+// (19 %).
 #define TPUHIP_SPLIT_TILES(SP)               \
   SP(75, "mfma_split_16x16_w4", 4, 1, 1, 1)  \
   SP(76, "mfma_split_16x16", 8, 1, 1, 1)     \
@@ -4761,8 +4761,8 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t, int num_cu) {
   // fastest of all in 10 at 256 tiles (256 -> 256 channels 3x3: 5.3 us against 7.4), in 3 at 512, in none at 1024 (14.3
   // against 8.2) and 2048 (27.0 against 13.2): the line is four times where they were last seen to win
   if (c.reg == 8 && ceil_div64((int64_t)d.n * d.oh * d.ow, 32) * ceil_div64(d.oc, 32) > 2048) return false;
-  // likewise: of 114 layers the most tiles with which a variant was the fastest were 752 (64 -> 255 channels 1x1 on 44 x 17: 2.66 us
-  // against 2.88 of the blocks of 32 x 32).  The line lies at nearly three times that
+  // likewise: of 114 layers the most tiles with which a variant was the fastest were 512 (512 -> 2048 channels 1x1 on 7 x 7: 2.66 us
+  // against 2.95 of the blocks of 32 x 32).  The line lies at four times that
   if (c.reg == 10 && split_tiles(d, c.split, split_plan(d, c.split, true)) > 2048) return false;
   if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8 || c.reg == 10)) return false;   // prefer the 4-channel K packing of the LDS kernels
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle

@@ -9,14 +9,14 @@
 // fetches 313.
 //
 // A workgroup of KW x PW waves owns 16 * OB channels of PW * NB blocks of pixels; wave (k, g) multiplies slices k, k + KW, ... of
-// 64 bytes of K for the NB blocks of pixel group g.  The filter is packed fragment by fragment (1 KB loads), all of a wave's up to
-// NS in flight before anything is waited for.  The partial sums meet in LDS behind one barrier; every block is finished by one
+// 64 bytes of K for the NB blocks of pixel group g.  The filter is packed fragment by fragment (1 KB loads), kPatchDepth or
+// kDepth slices of a wave in flight before anything is waited for.  The partial sums meet in LDS behind one barrier; every block is finished by one
 // wave, four channels of a pixel per lane.
 //
 // Replayed from a graph (a launch of nothing is 1.7 us there), against the best of the other forms: 3x3 of 512 channels on 7 x 7
-// 6.7 -> 4.0 us, 256 on 14 x 14 4.84 -> 3.37, 64 on 56 x 56 3.21 -> 2.84, 256 -> 512 on 26 x 26 6.87 -> 5.5, 512 -> 1024 on 13 x 13
-// 7.1 -> 5.2, at stride 2 from 26 x 26 7.2 -> 6.0; 1x1 2048 -> 512 on 7 x 7 4.5 -> 3.2, 1024 -> 256 on 14 x 14 3.5 -> 2.65; 5x5 at
-// stride 2, 128 channels on 4 x 45 x 53, 9.0 -> 6.9.  What is left of the large ones is the same link: 112 KB per CU at 26 x 26 are
+// 6.7 -> 3.9 us, 256 on 14 x 14 4.8 -> 3.35, 64 on 56 x 56 3.2 -> 2.8, 256 -> 512 on 26 x 26 6.8 -> 5.3, 512 -> 1024 on 13 x 13
+// 7.1 -> 4.8, at stride 2 from 26 x 26 7.1 -> 5.6; 1x1 2048 -> 512 on 7 x 7 4.5 -> 3.1, 1024 -> 256 on 14 x 14 3.4 -> 2.6; 5x5 at
+// stride 2, 128 channels on 4 x 45 x 53, 8.9 -> 5.7.  What is left of the large ones is the same link: 112 KB per CU at 26 x 26 are
 // 1.9 us.
 #include "conv_split.hpp"
 
@@ -28,6 +28,12 @@ namespace {
 
 constexpr int kLdsBytes = 160 * 1024;
 constexpr int kDepth = 4;        // gather form: slices in flight
+// Patch form: slices of the filter in flight.  All of a wave's at once, up to nine, take the registers of another workgroup and are
+// waited for together.  Of 56 layers the fastest variant with three is 5.5 % faster in the mean than with all of up to three, five
+// and nine, with two 6 % (512 -> 1024 on 13 x 13: 4.93, 4.85 and 5.22 us with two, three and nine; 512 on 7 x 7 4.05, 3.91, 3.95;
+// 256 -> 512 at stride 2 from 52 x 52 5.66, 5.95 and 6.24 with two, three and five); with two 10 layers lose, up to 3 %, with three
+// two, up to 1.6 %.
+constexpr int kPatchDepth = 3;
 constexpr int kPatchLoads = 8;   // patch form: 16-byte loads of a thread in flight
 
 // x / d for x * d < 2^32, d = 1 too, without a branch: magic = floor((2^32 - 1) / d)
@@ -41,8 +47,8 @@ __device__ __forceinline__ int32_t requant_one(int32_t v, int32_t mult, int32_t 
   return rdbp(x, shift, mask, mask >> 1);
 }
 
-// UNI: the channels are a multiple of 64, a slice lies within one tap.  NS: slices of a wave held at once.
-template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, int NS, bool POST>
+// UNI: the channels are a multiple of 64, a slice lies within one tap.
+template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, bool POST>
 __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *post) {
   // named here, the arguments leave the scalar cache together instead of one by one where they are first needed
   asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.bias), "s"(a.x_bytes), "s"(a.n_tiles), "s"(a.n_pix), "s"(a.shape), "s"(a.magic_tile),
@@ -111,7 +117,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   }
   const uint32_t woff = (uint32_t)lane * 16u;
   const uint32_t wbase = (uint32_t)(oc_tile * OB * slices) * 1024u;
-  constexpr int D = PATCH ? NS : kDepth;
+  constexpr int D = PATCH ? kPatchDepth : kDepth;
   v4i af[D][OB], bf[PATCH ? 1 : D][NB];
   auto load_filter = [&](int slot, int s) {
 #pragma unroll
@@ -295,13 +301,13 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   }
 }
 
-template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, int NS>
+template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH>
 __global__ __launch_bounds__(KW * PW * 64) void conv_split_kernel(SplitArgs a) {
-  split_body<KW, PW, NB, OB, FAST, UNI, PATCH, NS, false>(a, nullptr);
+  split_body<KW, PW, NB, OB, FAST, UNI, PATCH, false>(a, nullptr);
 }
-template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, int NS>
+template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH>
 __global__ __launch_bounds__(KW * PW * 64) void conv_split_post_kernel(SplitPost p) {
-  split_body<KW, PW, NB, OB, FAST, UNI, PATCH, NS, true>(p.a, &p);
+  split_body<KW, PW, NB, OB, FAST, UNI, PATCH, true>(p.a, &p);
 }
 
 // FullyConnected of few rows (a classifier) the same way, from the filter in fragments of 32 channels that fc_prepack() makes: 16
@@ -399,7 +405,7 @@ __global__ __launch_bounds__(KW * 64) void fc_split_kernel(FcArgs a) {
 
 uint32_t magic_of(int64_t d) { return (uint32_t)(0xffffffffull / (uint64_t)d); }
 
-template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH, int NS>
+template <int KW, int PW, int NB, int OB, bool FAST, bool UNI, bool PATCH>
 void launch_form(tpuhip_ctx *ctx, unsigned lds, const SplitArgs &a, const SplitPost *post) {
   const dim3 grid((a.n_tiles + 7) / 8 * 8), block(KW * PW * 64);
   auto go = [&](auto kernel, const auto &args) {
@@ -410,25 +416,20 @@ void launch_form(tpuhip_ctx *ctx, unsigned lds, const SplitArgs &a, const SplitP
       hipLaunchKernelGGL(kernel, grid, block, lds, ctx->stream, args);
   };
   if (post) {
-    go(conv_split_post_kernel<KW, PW, NB, OB, FAST, UNI, PATCH, NS>, *post);
+    go(conv_split_post_kernel<KW, PW, NB, OB, FAST, UNI, PATCH>, *post);
   } else {
-    go(conv_split_kernel<KW, PW, NB, OB, FAST, UNI, PATCH, NS>, a);
+    go(conv_split_kernel<KW, PW, NB, OB, FAST, UNI, PATCH>, a);
   }
 }
 
 template <int KW, int PW, int NB, int OB>
 void launch_variant(tpuhip_ctx *ctx, const SplitPlan &pl, bool fast, bool uni, const SplitArgs &a, const SplitPost *post) {
   if (pl.th) {
-    const int mine = ((a.slices_pad_relu >> 4) + KW - 1) / KW;
-    if (!uni) mine <= 3 ? launch_form<KW, PW, NB, OB, true, false, true, 3>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, true, false, true, 6>(ctx, pl.lds, a, post);
-    else if (mine <= 2) launch_form<KW, PW, NB, OB, true, true, true, 2>(ctx, pl.lds, a, post);
-    else if (mine <= 3) launch_form<KW, PW, NB, OB, true, true, true, 3>(ctx, pl.lds, a, post);
-    else if (mine <= 5) launch_form<KW, PW, NB, OB, true, true, true, 5>(ctx, pl.lds, a, post);
-    else launch_form<KW, PW, NB, OB, true, true, true, 9>(ctx, pl.lds, a, post);
+    uni ? launch_form<KW, PW, NB, OB, true, true, true>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, true, false, true>(ctx, pl.lds, a, post);
     return;
   }
-  if (fast) uni ? launch_form<KW, PW, NB, OB, true, true, false, 0>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, true, false, false, 0>(ctx, pl.lds, a, post);
-  else uni ? launch_form<KW, PW, NB, OB, false, true, false, 0>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, false, false, false, 0>(ctx, pl.lds, a, post);
+  if (fast) uni ? launch_form<KW, PW, NB, OB, true, true, false>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, true, false, false>(ctx, pl.lds, a, post);
+  else uni ? launch_form<KW, PW, NB, OB, false, true, false>(ctx, pl.lds, a, post) : launch_form<KW, PW, NB, OB, false, false, false>(ctx, pl.lds, a, post);
 }
 
 }  // namespace
@@ -436,9 +437,9 @@ void launch_variant(tpuhip_ctx *ctx, const SplitPlan &pl, bool fast, bool uni, c
 // The patch form: a window of more than one tap, a patch that fits; as many whole rows as the slots hold, or the part of a row
 // that they hold, evened out over the image.  It saves what the taps of a block's pixels share and costs a trip through LDS and a
 // barrier, so the line lies by the K that is fetched and the pixels of a wave.  Straight from memory / as a patch, from a graph:
-//   16 pixels and 32: 64 -> 512 on 2 x 6 x 40 at stride 2 (9 slices) 2.43 / 3.05 us, 192 -> 96 on 35 x 19 (27) 2.97 / 3.86, 256 ->
-//     256 on 14 x 14 (36) 3.5 / 3.37, 512 -> 512 on 7 x 7 (72) 4.54 / 4.03, 512 -> 1024 on 13 x 13 (72) 7.89 / 5.23;
-//   64 and 128: 64 -> 64 on 56 x 56 (9) 3.07 / 3.7, 128 -> 256 on 52 x 52 (18) 6.5 / 5.87, 256 -> 512 on 26 x 26 (36) 7.56 / 5.54.
+//   16 pixels and 32: 64 -> 512 on 2 x 6 x 40 at stride 2 (9 slices) 2.40 / 3.02 us, 192 -> 96 on 35 x 19 (27) 2.88 / 3.70, 256 ->
+//     256 on 14 x 14 (36) 3.44 / 3.38, 512 -> 512 on 7 x 7 (72) 4.52 / 3.95, 512 -> 1024 on 13 x 13 (72) 7.72 / 4.85;
+//   64 and 128: 64 -> 64 on 56 x 56 (9) 3.02 / 3.84, 128 -> 256 on 52 x 52 (18) 8.19 / 5.85, 256 -> 512 on 26 x 26 (36) 7.50 / 5.37.
 SplitPlan tpuhip::split_plan(const tpuhip_conv_desc &d, const SplitVariant &v, bool fast) {
   SplitPlan pl;
   const int slots = v.pw * v.nb * 16;
