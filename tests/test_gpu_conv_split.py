@@ -114,6 +114,35 @@ def test_shifts_of_zero_and_a_relu_in_front(ctx, tile, case, relu_first):
     yt.free()
 
 
+# n, ic, ih, iw, oc_a, oc_b, stride, dilation: 36 to 72 slices, which all variants take as a patch; the second result's channels end
+# within a block of 16, at its end, in a block of 32 whose second half is past them, and after several blocks
+@pytest.mark.parametrize("tile", SPLIT_TILES, ids=_name)
+@pytest.mark.parametrize("pair", [(1, 256, 13, 11, 128, 40, 1, 1), (2, 256, 9, 15, 256, 16, 2, 1), (1, 512, 7, 7, 128, 24, 1, 1),
+                                  (1, 256, 14, 14, 128, 130, 1, 2)], ids=lambda c: "x".join(map(str, c[:6])))
+@pytest.mark.parametrize("relus", [(True, False), (False, True)])
+def test_a_pair_of_which_the_input_lies_in_a_patch(ctx, tile, pair, relus):
+    n, ic, ih, iw, oca, ocb, stride, dil = pair
+    parts, refs = [], []
+    for oc, relu in zip((oca, ocb), relus):
+        case = (n, ic, ih, iw, oc, (3, 3), (stride, stride), (dil,) * 4, (dil, dil), relu)
+        rng, x, w, bias, mult, rsh = _layer(case, oca + ocb)
+        if parts:
+            w, bias, mult = w[::-1].copy(), -bias, mult[::-1].copy()
+        d = conv_desc(x.shape, w.shape, stride=case[6], pads=case[7], dil=case[8], do_relu=relu, algo=16 + tile)
+        parts.append((d, (w, f2i32(bias), f2i32(mult), f2i32(rsh))))
+        refs.append(O.conv2d_i8(x, w, bias, rsh, mult, O.make_conv_desc(x.shape, w.shape, 1, case[6], case[7], case[8], (0, 0), relu, True, None)))
+    wh = ctx.conv_prepack_pair(parts[0][0], parts[1][0], parts[0][1], parts[1][1])
+    xt, ys = ctx.from_nchw(x), [ctx.tensor(r.shape) for r in refs]
+    for t in ys:
+        ctx._ck(ctx.lib.tpuhip_memset(ctx.h, t.ptr, 0x55, t.nbytes))
+    ctx.conv_pair(wh, xt, ys[0], ys[1])
+    for t, ref in zip(ys, refs):
+        assert np.array_equal(ctx.to_nchw(t), ref) and not ctx.raw(t)[..., ref.shape[1]:].any()
+    ctx.conv_weights_destroy(wh)
+    for t in [xt] + ys:
+        t.free()
+
+
 @pytest.mark.parametrize("tile", SPLIT_TILES, ids=_name)
 @pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[12]], ids=lambda c: "x".join(map(str, c[:5])))
 @pytest.mark.parametrize("stride", [65520, 65536, 65552])

@@ -1,5 +1,6 @@
 """Several tensors laid out for the host by one launch: more of them than one list holds, vectors among them, up to what goes
-straight into the staging buffer and beyond it."""
+straight into the staging buffer and beyond it, and more than it holds.  Bytes (i8) are asked for one tensor at a time: the same
+values by the launch of one."""
 import numpy as np
 import pytest
 
@@ -32,6 +33,34 @@ def test_every_tensor_of_a_graph(shapes, i8):
             every = m.get_all_tensor()
         for i, x in enumerate(xs):
             assert np.array_equal(every["x%d" % i], x) and np.array_equal(every["y%d" % i], np.maximum(x, 0)), i
+    m.close()
+
+
+# 56 MB that fit the staging buffer (32 MB) one by one: it is filled twice, a filling ends in the middle of the list, and the second
+# read finds the buffers of the first
+FILLINGS = [(1, 129, 300, 301), (1, 3, 5, 7), (2, 70, 251, 257), (3, 13, 1, 1), (1, 64, 331, 333)]
+
+
+@pytest.mark.parametrize("order", [1, -1])
+def test_more_than_the_staging_buffer_holds(order):
+    shapes = FILLINGS[::order]
+    g = graphs.Graph("fillings", 1)
+    for i, s in enumerate(shapes):
+        g.add(graphs.Op("tpu.input", "x%d" % i, [], s))
+        g.add(graphs.Op("tpu.relu", "y%d" % i, ["x%d" % i], s))
+    g.outputs = ["y%d" % i for i in range(len(shapes))]
+    sizes = [int(np.prod(s)) for s in shapes for _ in range(2)]
+    assert max(sizes) <= 32 << 20 < sum(sizes)
+    m = module()
+    m.load(g)
+    for k in range(2):
+        xs = [np.random.default_rng(k + i).integers(-128, 128, s).astype(np.int8) for i, s in enumerate(shapes)]
+        for i, x in enumerate(xs):
+            m.set_tensor_i8("x%d" % i, x)
+        m.invoke()
+        for every in (m.get_all_tensor(), m.get_all_tensor()):
+            for i, x in enumerate(xs):
+                assert np.array_equal(every["x%d" % i], x) and np.array_equal(every["y%d" % i], np.maximum(x, 0)), i
     m.close()
 
 

@@ -98,7 +98,8 @@ def test_round_trip_of_fp32_edges(shape):
     m.close()
 
 
-# together in one round of the staging buffer; several rounds; a tensor larger than the buffer among small ones
+# together straight into the staging buffer; several spans of one filling (test_gpu_dense_list.py has several fillings); a tensor
+# larger than the buffer among small ones
 @pytest.mark.parametrize("shapes", [[(1, 3, 20, 31), (2, 1000, 1, 1)], [(4, 70, 61, 67), (1, 255, 13, 13), (3, 129, 130, 131)],
                                     [(2, 17, 9, 9), (5, 64, 331, 333), (1, 5, 300, 1)]])
 def test_all_tensors_at_once(shapes):
