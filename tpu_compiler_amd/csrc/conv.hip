@@ -4664,8 +4664,8 @@ int pack_filter(tpuhip_ctx *ctx, const FilterPack &a) {
   return TPUHIP_OK;
 }
 
-// (re)builds the device filter of an MFMA conv for tile variant `tile`
-// whenever the tile, the parameters or a stride have changed
+// what a launch of a K-split tile in blocks of 16 x 16 takes but its pointers: called whenever the tile, the parameters or a stride
+// have changed
 void split_ready(tpuhip_conv_weights *cw) {
   if (cw->algo != ALGO_MFMA || kTiles[cw->tile].reg != 10 || !cw->nparam) return;
   const SplitVariant &v = kTiles[cw->tile].split;
@@ -4673,6 +4673,7 @@ void split_ready(tpuhip_conv_weights *cw) {
   cw->split_fits = split_args(cw->d, v, cw->split_plan, &cw->split);
 }
 
+// (re)builds the device filter of an MFMA conv for tile variant `tile`
 int pack_mfma_weights(tpuhip_ctx *ctx, tpuhip_conv_weights *cw, int tile) {
   const tpuhip_conv_desc &d = cw->d;
   const TileCfg &t = kTiles[tile];
@@ -4973,8 +4974,6 @@ void launch_conv_mfma(tpuhip_ctx *ctx, const tpuhip_conv_weights *w, const ConvA
   }
 }
 
-// Times every candidate tile on the layer's real buffers (the kernels are
-// idempotent and bit-identical across tiles) and keeps the fastest.
 // what runs behind the requantisation in the epilogue
 struct PostOps {
   const int8_t *lut = nullptr;   // host table, 256 entries
@@ -4990,9 +4989,9 @@ struct PostOps {
   bool any() const { return lut || has_add() || y2 || pool; }
 };
 
-// The stem + max pool launch: whether it applies, and its tiling.  rows = pooled rows per
-// workgroup: as many as LDS holds (patch + conv tile), fewer while the launch would leave
-// compute units without a tile, then evened out over the image.
+// The stem + max pool launch: whether it applies, and its tiling.  It applies where the widest tiles -- as many pooled rows as LDS
+// holds (patch + conv tile), fewer while the launch would leave compute units without one, evened out over the image -- fit with the
+// conv rows that no window reaches; the rows of a tile are then those with which its rounds over the compute units take the least.
 bool stem_pool_plan(const tpuhip_conv_weights *w, const tpuhip_pool_desc &p, int num_cu, StemPoolArgs *out,
                     unsigned *lds_bytes) {
   const tpuhip_conv_desc &d = w->d;
@@ -5136,7 +5135,8 @@ __global__ __launch_bounds__(64) void delay_kernel(int rounds) {
   for (int i = 0; i < rounds; ++i) __builtin_amdgcn_s_sleep(100);   // 6400 clocks
 }
 
-// The fused add (if any) is part of what is timed: it shifts the balance between
+// Times every candidate tile on the layer's real buffers (the kernels are idempotent and bit-identical across tiles) and keeps the
+// fastest.  The fused add (if any) is part of what is timed: it shifts the balance between
 // the tile shapes.  Every launch recomputes the same bytes, so repeating it is safe
 // as long as the sum is not written over its own input.
 // Every candidate runs five times; those within a fifth of the fastest then run twice fifteen times, and the smaller of
