@@ -4077,8 +4077,8 @@ struct TileCfg {
 // K split over the waves of a workgroup, blocks of 16 x 16 (conv_split.hip):
 // SP(index, name, waves along K, along the pixels, blocks of 16 pixels and of 16 channels per wave).  Of 114 layers (the networks of
 // one image, and layers drawn of 1 to 8 images of 5 to 107 pixels a side, 16 to 1024 channels, 1x1 to 5x5, stride 1 and 2, dilation)
-// one of them is the fastest of all in 97, by up to 2.8 times (profiles/conv_split_tiles.txt): 16x16_w4 in 26 (by up to 10 % over
-// the next variant), 16x32 in 20 (12 %), 32x32 in 19 (47 %), 32x64 in 15 (9 %), 16x16 in 12 (22 %), 32x128 in 4 (19 %), 16x64 in one
+// one of them is the fastest of all in 96, by up to 2.8 times (profiles/conv_split_tiles.txt): 16x16_w4 in 26 (by up to 10 % over
+// the next variant), 16x32 in 20 (11 %), 32x32 in 19 (48 %), 32x64 in 15 (9 %), 16x16 in 12 (19 %), 32x128 in 3 (20 %), 16x64 in one
 // (19 %).
 #define TPUHIP_SPLIT_TILES(SP)               \
   SP(75, "mfma_split_16x16_w4", 4, 1, 1, 1)  \
@@ -4763,7 +4763,7 @@ bool tile_is_candidate(const tpuhip_conv_desc &d, int t, int num_cu) {
   // against 8.2) and 2048 (27.0 against 13.2): the line is four times where they were last seen to win
   if (c.reg == 8 && ceil_div64((int64_t)d.n * d.oh * d.ow, 32) * ceil_div64(d.oc, 32) > 2048) return false;
   // likewise: of 114 layers the most tiles with which a variant was the fastest were 512 (512 -> 2048 channels 1x1 on 7 x 7: 2.66 us
-  // against 2.95 of the blocks of 32 x 32).  The line lies at four times that
+  // against 2.97 of the blocks of 32 x 32).  The line lies at four times that
   if (c.reg == 10 && split_tiles(d, c.split, split_plan(d, c.split, true)) > 2048) return false;
   if (d.ic <= 4 && (c.reg == 1 || c.reg == 2 || c.reg == 8 || c.reg == 10)) return false;   // prefer the 4-channel K packing of the LDS kernels
   return !(c.bm > 32 && c.bm / 2 >= round_up(d.oc, 32));   // more than half the rows idle

@@ -9,7 +9,7 @@
 // fetches 313.
 //
 // A workgroup of KW x PW waves owns 16 * OB channels of PW * NB blocks of pixels; wave (k, g) multiplies slices k, k + KW, ... of
-// 64 bytes of K for the NB blocks of pixel group g.  The filter is packed fragment by fragment (1 KB loads), kPatchDepth or
+// 64 bytes of K for the NB blocks of pixel group g.  The filter is packed fragment by fragment (1 KB loads), patch_depth() or
 // kDepth slices of a wave in flight before anything is waited for.  The partial sums meet in LDS behind one barrier; every block is finished by one
 // wave, four channels of a pixel per lane.
 //
@@ -28,13 +28,15 @@ namespace {
 
 constexpr int kLdsBytes = 160 * 1024;
 constexpr int kDepth = 4;        // gather form: slices in flight
-// Patch form: slices of the filter in flight.  All of a wave's at once, up to nine, take the registers of another workgroup and are
-// waited for together.  Of 56 layers the fastest variant with three is 5.5 % faster in the mean than with all of up to three, five
-// and nine, with two 6 % (512 -> 1024 on 13 x 13: 4.93, 4.85 and 5.22 us with two, three and nine; 512 on 7 x 7 4.05, 3.91, 3.95;
-// 256 -> 512 at stride 2 from 52 x 52 5.66, 5.95 and 6.24 with two, three and five); with two 10 layers lose, up to 3 %, with three
-// two, up to 1.6 %.
-constexpr int kPatchDepth = 3;
 constexpr int kPatchLoads = 8;   // patch form: 16-byte loads of a thread in flight
+// Patch form: slices of the filter in flight per wave.  Eight waves: three.  All of a wave's at once, up to nine, take the registers
+// of another workgroup and are waited for together: of 56 layers, over all variants, three are 9 % faster in the mean than all of
+// up to three, five and nine, the fastest variants 5.5 % (512 -> 1024 on 13 x 13: 4.93, 4.85 and 5.22 us with two, three and nine,
+// and where the filter comes from beyond the L2s 5.37 and 6.14 with three and nine; 512 on 7 x 7 4.05, 3.91, 3.95, 4.72 and 4.85);
+// four are 3 % slower than three.  Four waves have half as much in flight with as many, which is too little where the filter comes
+// from afar: 512 on 7 x 7 5.68, 4.79 and 4.80 us with three, six and nine, 256 on 14 x 14 3.62, 3.62 and 3.51.  Six where a slice
+// straddles taps (337 channels on 17 x 36: nine 8 % slower).
+constexpr int patch_depth(int waves, bool uni) { return waves > 4 ? 3 : uni ? 9 : 6; }
 
 // x / d for x * d < 2^32, d = 1 too, without a branch: magic = floor((2^32 - 1) / d)
 __device__ __forceinline__ uint32_t div_by(uint32_t x, uint32_t magic) { return __umulhi(x + 1, magic); }
@@ -117,7 +119,7 @@ __device__ __forceinline__ void split_body(const SplitArgs &a, const SplitPost *
   }
   const uint32_t woff = (uint32_t)lane * 16u;
   const uint32_t wbase = (uint32_t)(oc_tile * OB * slices) * 1024u;
-  constexpr int D = PATCH ? kPatchDepth : kDepth;
+  constexpr int D = PATCH ? patch_depth(KW * PW, UNI) : kDepth;
   v4i af[D][OB], bf[PATCH ? 1 : D][NB];
   auto load_filter = [&](int slot, int s) {
 #pragma unroll
